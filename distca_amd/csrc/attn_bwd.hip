@@ -265,7 +265,7 @@ int DISTCA_FN(run_bwd)(const BwdQuerySide &qs, const void *k, const void *v, voi
   // ---- dQ: one workgroup per (task, block of query rows, kv head).  It runs first: it also leaves the row
   // statistics (lse in the log2 domain, -delta) in the workspace, which the dK/dV kernel reads.
   {
-    const SchedGeom geom = dq_geom(p);
+    const SchedGeom geom = launched_geom(dq_geom(p), p);
     a.merge_tiles = geom.merge_tiles;
     const int64_t max_items = dq_max_items(p);
     rc = launch_build_schedule(0, cu_q, cu_k, p->num_tasks, geom, (int32_t *)(ws + w.sched_q), max_items, s);

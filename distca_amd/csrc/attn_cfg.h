@@ -63,6 +63,16 @@ constexpr int32_t kMergeTilesDq = DISTCA_MERGE_TILES_DQ;    // the same for a me
 inline bool merge_short_tasks(const distca_ca_params *p) {
   return p->num_tasks > 0 && (int64_t)p->total_q < (int64_t)kMergeMeanTokens * p->num_tasks;
 }
+// The lists as they are launched: merging trades workgroups for the fixed part of a block, which pays only where the blocks
+// fill the device many times over.  A batch with fewer than kMergeMinBlocksPerCU blocks of query rows per compute unit keeps
+// one block per item (forward + backward without / with merging: 389 tokens at 4/1 heads 179 / 261 us, three documents of
+// 4096 tokens in all, forward only, 86 / 187 us; 8.7 blocks per unit -1.4 %, 7.3 blocks -2.2 %; at 32 blocks per unit merging
+// is 2.8 % ahead).  num_heads_q / num_heads_kv cancel: blocks x kv heads = total_q * Hq / rows.
+constexpr int32_t kMergeMinBlocksPerCU = 12;
+inline SchedGeom launched_geom(SchedGeom g, const distca_ca_params *p) {
+  if ((int64_t)p->total_q * p->num_heads_q < (int64_t)kMergeMinBlocksPerCU * g.rows_per_block * num_compute_units()) g.merge_tiles = 0;
+  return g;
+}
 inline SchedGeom fwd_geom(const distca_ca_params *p) {
   SchedGeom g;
   g.split_target = 0;

@@ -650,7 +650,7 @@ int DISTCA_FN(run_fwd_tokens)(const void *q_base, const int64_t *q_task_off, int
   if (!workspace || workspace_bytes < need) return fail(DISTCA_E_WORKSPACE, "ca_fwd: workspace %lld B < required %lld B", (long long)workspace_bytes, (long long)need);
   if (!aligned16(workspace)) return fail(DISTCA_E_INVALID, "ca_fwd: workspace must be 16-byte aligned");
   hipStream_t s = (hipStream_t)stream;
-  const SchedGeom geom = fwd_geom(p);
+  const SchedGeom geom = launched_geom(fwd_geom(p), p);
   const int64_t max_items = fwd_max_items(p);
   rc = launch_build_schedule(0, cu_q, cu_k, p->num_tasks, geom, (int32_t *)workspace, max_items, s);
   if (rc) return rc;

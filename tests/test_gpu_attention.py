@@ -137,6 +137,30 @@ def test_short_tasks_as_merged_work_items(cuda, hq, hkv):
     _run([1024, 300, 700], [1024, 1324, 764], hq, hkv, 52, cuda)
 
 
+@pytest.mark.parametrize("n", [12, 11])
+def test_short_tasks_either_side_of_the_merging_rule(cuda, n):
+    """Blocks of short tasks are merged into larger work items from 12 blocks of query rows per compute unit on (n of them
+    here, on 256 units), and not below that: the first and the last document of a batch on either side against the oracle."""
+    from distca_amd.fused_comm_attn import ca_varlen_bwd, ca_varlen_fwd
+    lens = [1000, 1048] * (n // 2) + [1024] * (n % 2)      # n * 1024 tokens x 64 heads = n blocks per unit
+    q, k, v, do = make_qkv(sum(lens), sum(lens), 64, 16, 128, 53)
+    c = cu(lens)
+    dev = [t.to(cuda) for t in (q, k, v, do)]
+    dc = torch.tensor(c, device=cuda)
+    out, lse = ca_varlen_fwd(*dev[:3], dc, dc, max(lens), max(lens))
+    grads = ca_varlen_bwd(dev[3], *dev[:3], out, lse, dc, dc, max(lens), max(lens))
+    torch.cuda.synchronize()
+    for b in (0, len(lens) - 1):
+        r = slice(int(c[b]), int(c[b + 1]))
+        one = cu([lens[b]])
+        ref_out, ref_lse = ca_reference_fwd(q[r], k[r], v[r], one, one)
+        assert_close_bf16(out[r], ref_out, "out")
+        assert (lse[:, r].cpu() - ref_lse).abs().max().item() < 2e-3
+        ref = ca_reference_bwd(do[r], q[r], k[r], v[r], one, one, out=out[r].cpu(), softmax_lse=lse[:, r].cpu())
+        for name, got, want in zip(("dq", "dk", "dv"), grads, ref):
+            assert_close_bf16(got[r], want, name)
+
+
 def test_non_causal(cuda):
     _run([100, 260], [100, 260], 4, 2, 6, cuda, causal=False)
 
