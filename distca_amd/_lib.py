@@ -45,12 +45,19 @@ class KvShards(Structure):
 
 PACK_MAX_JOBS = 4
 
+# struct distca_exchange_job is 25 words of 64 bits: kind, dtype, num_parts, num_seq, num_tokens, token_bytes, max_cp, max_copies,
+# seq_offset, seq_tokens, mask, num_copies, copy_start, then (data, pitch, bytes) for four parts
+EXCHANGE_MAX_JOBS, TOKEN_MAX_PARTS, EXCHANGE_JOB_WORDS = 4, 4, 25
+JOB_PLAIN, JOB_REPLICAS, JOB_REPLICA_SUM, JOB_COPY_SUM = range(4)
+ExchangeJobs = [c_int64 * (EXCHANGE_JOB_WORDS * n) for n in range(EXCHANGE_MAX_JOBS + 1)]   # arrays of n jobs
+
 # name -> (restype, argtypes); every symbol include/distca_ca.h declares
 SYMBOLS = {
     "distca_last_error": (c_char_p, []),
     "distca_abi_version": (c_int, []),
     "distca_memcpy_non_cp": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p]),
     "distca_memcpy_non_cp_multi": (c_int, [POINTER(PackJob), c_int32, c_void_p, c_int, c_void_p]),
+    "distca_exchange": (c_int, [c_void_p, c_int32, c_void_p, c_int, c_void_p]),
     "distca_memcpy_cp": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int32, c_int64, c_int, c_void_p]),
     "distca_grad_sum": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p]),
     "distca_ca_fwd_workspace_bytes": (c_int64, [POINTER(CaParams)]),

@@ -5,10 +5,15 @@
 // :158-236); the decomposition does not.  A shard is contiguous on both sides (rows
 // start_s.. of the tensor, bytes offset_s.. of the buffer), so the job is a list of
 // contiguous segment copies.  The logical token range is cut into one equal slice per
-// workgroup; a workgroup locates the shard holding its first token with a block-wide
-// prefix scan of the shard lengths, then walks shards, streaming 16-byte vectors with
-// non-temporal loads and stores (the data is touched once, keeping it out of L2 leaves
-// the cache to whoever runs next).
+// workgroup; every wave locates the shard holding its slice's first token with a scan of
+// the shard lengths in registers (no barrier), then the workgroup walks shards, streaming
+// 16-byte vectors with non-temporal loads and stores (the data is touched once, keeping it
+// out of L2 leaves the cache to whoever runs next).
+//
+// What a rank does around an all-to-all is several such copies at once, and each is a job of one
+// launch (distca_exchange): q, k and v; a transport token made of several tensors' rows, put
+// together or taken apart on the way instead of in a pass of its own; a row that goes to several
+// replicas, read once; the rows of several replicas, or of several copies, added up on the way.
 #include "api_util.h"
 #include "common.h"
 
@@ -26,206 +31,129 @@ namespace {
 // (160 KiB slices) 75.4 / 75.3 % packing / unpacking, 16 (256 KiB) 75.0 / 75.5 %, 8 in three rounds 70.7 / 71.7 %,
 // 20 or 24 in one round 73 %, 32 in one round 65 %.
 constexpr int kPackThreads = 1024;
-constexpr int kPackWaves = kPackThreads / 64;
 #ifndef DISTCA_PACK_UNROLL
 #define DISTCA_PACK_UNROLL 10
 #endif
-#ifndef DISTCA_PACK_SLICE_ROUNDS
-#define DISTCA_PACK_SLICE_ROUNDS 1
-#endif
 constexpr int kUnroll = DISTCA_PACK_UNROLL;
-constexpr int64_t kRoundBytes = (int64_t)kUnroll * kPackThreads * 16;  // bytes a workgroup moves per loop round
+constexpr int64_t kVecRound = (int64_t)kPackThreads * 16;      // bytes of one vector per thread
+constexpr int64_t kRoundBytes = kUnroll * kVecRound;           // bytes a workgroup moves per loop round
+// Tokens of several parts compute an address per vector: eight in flight keep to the 64 registers of two workgroups per unit.
+constexpr int kUnrollParts = 8;
+// Jobs that add rows up hold fp32 sums beside the loads: six vectors per lane in flight (of two-byte elements: 48 + 24 registers)
+constexpr int kUnrollSum = 6;
 
-// Inclusive block scan of one int64 per thread.
-__device__ __forceinline__ int64_t block_inclusive_scan(int64_t v, int64_t *lds_wave_sums) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    int64_t o = __shfl_up(v, off, 64);
-    if (lane >= off) v += o;
-  }
-  __syncthreads();  // protect lds_wave_sums from the previous round's readers
-  if (lane == 63) lds_wave_sums[wave] = v;
-  __syncthreads();
-  int64_t base = 0;
-  for (int w = 0; w < wave; ++w) base += lds_wave_sums[w];
-  return v + base;
-}
-
-struct Cursor {
-  int64_t seg;        // shard index s in [0, num_seq)
-  int64_t seg_start;  // first token of shard s inside one pass over the shard list
-  int64_t total;      // sum of all shard lengths
+// The shard that holds position `pos` of the concatenated shard list (idx == num_seq: none) and the position of its first
+// token.  Every wave finds it for itself: four loads of 64 lengths at a time, a scan over the lanes, no barrier.  (A block-wide
+// scan did this before: with its barriers 2 to 3 us of a small copy's 7.)
+struct Segment {
+  int idx;
+  int64_t start;
 };
-
-// Finds the shard containing position `pos` (0 <= pos < total) of the concatenated
-// shard list, and the total length.  All threads return the same values.
-__device__ Cursor locate(const int64_t *__restrict__ seq_tokens, int64_t num_seq, int64_t pos, bool need_total,
-                         int64_t *lds_scratch /* >= kPackWaves + 2 int64 */) {
-  int64_t *wave_sums = lds_scratch;               // kPackWaves
-  int64_t *found = lds_scratch + kPackWaves;      // [seg, seg_start]
-  int64_t running = 0;
-  if (threadIdx.x == 0) { found[0] = num_seq; found[1] = 0; }
-  for (int64_t c0 = 0; c0 < num_seq; c0 += kPackThreads) {
-    const int64_t i = c0 + threadIdx.x;
-    const int64_t len = (i < num_seq) ? seq_tokens[i] : 0;
-    const int64_t incl = running + block_inclusive_scan(len, wave_sums);
-    if (len > 0 && incl - len <= pos && pos < incl) { found[0] = i; found[1] = incl - len; }
-    __syncthreads();
-    // the last thread holds the chunk total
-    if (threadIdx.x == kPackThreads - 1) wave_sums[0] = incl;
-    __syncthreads();
-    running = wave_sums[0];
-    __syncthreads();
-    if (!need_total && found[0] < num_seq) break;  // uniform: found[] is in LDS
-  }
-  Cursor c;
-  c.seg = found[0];
-  c.seg_start = found[1];
-  c.total = running;
-  return c;
+__device__ __forceinline__ int64_t lane_value(int64_t v, int lane) {
+  const uint64_t u = (uint64_t)v;
+  const uint64_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(u >> 32), lane), lo = (uint32_t)__builtin_amdgcn_readlane((int)u, lane);
+  return (int64_t)((hi << 32) | lo);
 }
-
-template <bool STORE_NT>
-__device__ __forceinline__ void copy_bytes(uint8_t *__restrict__ dst, const uint8_t *__restrict__ src, int64_t bytes) {
-  const int64_t nvec = bytes >> 4;
-  const u32x4 *s = reinterpret_cast<const u32x4 *>(src);
-  u32x4 *d = reinterpret_cast<u32x4 *>(dst);
-  int64_t i = threadIdx.x;
-  for (; i + (kUnroll - 1) * kPackThreads < nvec; i += kUnroll * kPackThreads) {
-    u32x4 r[kUnroll];
+__device__ __forceinline__ Segment find_segment(const int64_t *__restrict__ seq_tokens, int num_seq, int64_t pos) {
+  constexpr int kAhead = 4;
+  const int lane = threadIdx.x & 63;
+  int64_t before = 0;
+  for (int c0 = 0; c0 < num_seq; c0 += 64 * kAhead) {
+    int64_t len[kAhead];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) r[u] = __builtin_nontemporal_load(s + i + u * kPackThreads);
-#pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      if (STORE_NT) __builtin_nontemporal_store(r[u], d + i + u * kPackThreads);
-      else d[i + u * kPackThreads] = r[u];
+    for (int j = 0; j < kAhead; ++j) {
+      const int i = c0 + 64 * j + lane;
+      len[j] = i < num_seq ? seq_tokens[i] : 0;
     }
-  }
-  if (i < nvec) {
-    // the last, partial round: every load is issued before the first store, as in a whole round
-    u32x4 r[kUnroll];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u)
-      if (i + u * kPackThreads < nvec) r[u] = __builtin_nontemporal_load(s + i + u * kPackThreads);
+    for (int j = 0; j < kAhead; ++j) {
+      int64_t incl = len[j];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u)
-      if (i + u * kPackThreads < nvec) {
-        if (STORE_NT) __builtin_nontemporal_store(r[u], d + i + u * kPackThreads);
-        else d[i + u * kPackThreads] = r[u];
+      for (int off = 1; off < 64; off <<= 1) {
+        const int64_t o = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += o;
       }
-  }
-}
-
-// One kernel for the plain and the replicating ("cp") form.
-//   plain: logical token L in [0, num_tokens) is row L of the tensor; shard list walked once.
-//   cp:    logical token L in [0, num_tokens*max_cp); the shard list is walked max_cp times,
-//          pass c covering replica c.  Packing reads row L % num_tokens, unpacking writes row L.
-template <bool TO_BUF, bool CP>
-__device__ __forceinline__ void pack_slice(uint8_t *__restrict__ tensor, uint8_t *__restrict__ buffer,
-                                           const int64_t *__restrict__ seq_offset, const int64_t *__restrict__ seq_tokens,
-                                           const int8_t *__restrict__ mask, int64_t num_seq, int64_t token_bytes,
-                                           int64_t num_tokens, int32_t max_cp, int64_t t0, int64_t t1, int64_t *lds_scratch) {
-  int64_t cp = 0, pos = t0, total = 0;
-  if (CP) {
-    Cursor c = locate(seq_tokens, num_seq, 0, true, lds_scratch);
-    total = c.total;
-    if (total <= 0) return;
-    cp = t0 / total;
-    if (cp >= max_cp) return;  // a tensor with more rows than the shards add up to: the slices past the last replica own nothing
-    pos = t0 - cp * total;
-    __syncthreads();
-  }
-  Cursor cur = locate(seq_tokens, num_seq, pos, false, lds_scratch);
-  if (cur.seg >= num_seq) return;  // t0 lies beyond the last shard
-  int64_t seg = cur.seg;
-  int64_t seg_start = cp * total + cur.seg_start;  // logical start of (cp, seg)
-
-  while (seg_start < t1) {
-    const int64_t len = seq_tokens[seg];
-    const int64_t seg_end = seg_start + len;
-    bool live;
-    if (CP) live = mask[seg * max_cp + cp] != 0;
-    else live = (!TO_BUF || mask == nullptr) ? true : (mask[seg] != 0);
-    const int64_t a = seg_start > t0 ? seg_start : t0;
-    const int64_t b = seg_end < t1 ? seg_end : t1;
-    if (live && a < b) {
-      const int64_t off = CP ? seq_offset[cp * num_seq + seg] : seq_offset[seg];
-      uint8_t *buf = buffer + off + (a - seg_start) * token_bytes;
-      if (CP && TO_BUF) {
-        // source rows wrap modulo num_tokens
-        int64_t n = b - a, lg = a;
-        while (n > 0) {
-          const int64_t row = lg % num_tokens;
-          int64_t run = num_tokens - row;
-          if (run > n) run = n;
-          copy_bytes<true>(buf, tensor + row * token_bytes, run * token_bytes);
-          buf += run * token_bytes;
-          lg += run;
-          n -= run;
-        }
-      } else {
-        uint8_t *ten = tensor + a * token_bytes;
-        if (TO_BUF) copy_bytes<true>(buf, ten, (b - a) * token_bytes);
-        else copy_bytes<true>(ten, buf, (b - a) * token_bytes);
+      const unsigned long long past = __ballot(before + incl > pos);
+      if (past) {
+        const int l = __builtin_ctzll(past);
+        return Segment{c0 + 64 * j + l, before + lane_value(incl, l) - lane_value(len[j], l)};
       }
-    }
-    seg_start = seg_end;
-    if (++seg == num_seq) {
-      if (!CP) break;
-      seg = 0;
-      if (++cp >= max_cp) break;
+      before += lane_value(incl, 63);
     }
   }
+  return Segment{num_seq, 0};
 }
 
-// One kernel for the plain and the replicating ("cp") form.
-//   plain: logical token L in [0, num_tokens) is row L of the tensor; shard list walked once.
-//   cp:    logical token L in [0, num_tokens*max_cp); the shard list is walked max_cp times,
-//          pass c covering replica c.  Packing reads row L % num_tokens, unpacking writes row L.
-template <bool TO_BUF, bool CP>
-__global__ __launch_bounds__(kPackThreads) void pack_kernel(
-    uint8_t *__restrict__ tensor, uint8_t *__restrict__ buffer, const int64_t *__restrict__ seq_offset,
-    const int64_t *__restrict__ seq_tokens, const int8_t *__restrict__ mask, int64_t num_seq, int64_t token_bytes,
-    int64_t num_tokens, int32_t max_cp, int64_t tokens_per_wg) {
-  __shared__ int64_t lds_scratch[kPackWaves + 2];
-  const int64_t logical_tokens = CP ? num_tokens * max_cp : num_tokens;
-  int64_t t0 = (int64_t)blockIdx.x * tokens_per_wg;
-  int64_t t1 = t0 + tokens_per_wg;
-  if (t1 > logical_tokens) t1 = logical_tokens;
-  if (t0 >= t1) return;
-  pack_slice<TO_BUF, CP>(tensor, buffer, seq_offset, seq_tokens, mask, num_seq, token_bytes, num_tokens, max_cp, t0, t1, lds_scratch);
-}
-
-// Several tensors against one buffer in one launch (the q, k and v of a tick): workgroups [first_wg, first_wg of the
-// next job) serve job j.  One launch has one tail instead of three, and the small tensors' slices fill the gaps
-// the large one leaves.
-constexpr int kMaxPackJobs = DISTCA_PACK_MAX_JOBS;
-struct PackJob {
-  uint8_t *tensor;
+// One copy: `part_vecs` vectors of every token, at `pitch` bytes in the tensor and from vector `part_v0` of the token on in the
+// buffer.  (The parts of a token are jobs of their own.)
+struct Job {
+  uint8_t *data;   // null: the bytes are zeros (the padding of a token)
   const int64_t *seq_offset, *seq_tokens;
   const int8_t *mask;
-  int64_t num_seq, token_bytes, num_tokens, tokens_per_wg;
-  int32_t first_wg;
+  const int32_t *num_copies;
+  const int64_t *copy_start;
+  int64_t num_tokens, token_bytes, pitch;
+  int32_t kind, dtype, num_seq, max_cp, max_copies, tokens_per_wg, first_wg;
+  uint32_t part_v0, part_vecs, magic;  // magic = ceil(2^32 / part_vecs) (0: part_vecs is 1): i / part_vecs == umulhi(i, magic) for i * part_vecs < 2^32
+  __host__ __device__ bool whole() const { return pitch == token_bytes && (int64_t)part_vecs * 16 == token_bytes; }
 };
-struct PackJobs {
-  PackJob job[kMaxPackJobs];
+constexpr int kMaxJobs = 12;
+struct Jobs {
+  Job job[kMaxJobs];
   int32_t n;
 };
-template <bool TO_BUF>
-__global__ __launch_bounds__(kPackThreads) void pack_multi_kernel(PackJobs jobs, uint8_t *__restrict__ buffer) {
-  __shared__ int64_t lds_scratch[kPackWaves + 2];
-  int j = 0;
+
+// A contiguous run of memory as a buffer resource of its exact length: lanes past its end load zeros and store nothing, so a
+// partial round needs no branches and is issued like a whole one.  (With a predicate per vector the compiler could not keep
+// the loop in the 64 registers that let two workgroups share a compute unit.)
+typedef __amdgpu_buffer_rsrc_t run_t;
+__device__ __forceinline__ run_t make_run(const void *p, uint32_t nvec) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(uniform_ptr(p)), 0, uniform_int((int)(nvec << 4)), 0x00020000);
+}
+constexpr int kNonTemporal = 2;
+constexpr int kNowhere = (int)0x80000000u;   // an offset past the end of every run
+__device__ __forceinline__ u32x4 load_nt(run_t r, int i) { return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, i << 4, 0, kNonTemporal)); }
+__device__ __forceinline__ void store_nt(run_t r, int i, u32x4 v) { __builtin_amdgcn_raw_buffer_store_b128(v, r, i << 4, 0, kNonTemporal); }
+__device__ __forceinline__ u32x4 load_at(run_t r, uint32_t byte, bool ok) {
+  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, ok ? (int)byte : kNowhere, 0, kNonTemporal));
+}
+__device__ __forceinline__ void store_at(run_t r, uint32_t byte, bool ok, u32x4 v) { __builtin_amdgcn_raw_buffer_store_b128(v, r, ok ? (int)byte : kNowhere, 0, kNonTemporal); }
+// N vectors per lane at a time, all loads of a round issued before its first store.
+template <int N, class Load, class Use>
+__device__ __forceinline__ void rounds(uint32_t nvec, Load load, Use use) {
+  for (int i = threadIdx.x; i < (int)nvec; i += N * kPackThreads) {
+    u32x4 r[N];
 #pragma unroll
-  for (int i = 1; i < kMaxPackJobs; ++i)
-    if (i < jobs.n && (int)blockIdx.x >= jobs.job[i].first_wg) j = i;
-  const PackJob &jb = jobs.job[j];
-  int64_t t0 = (int64_t)((int)blockIdx.x - jb.first_wg) * jb.tokens_per_wg;
-  int64_t t1 = t0 + jb.tokens_per_wg;
-  if (t1 > jb.num_tokens) t1 = jb.num_tokens;
-  if (t0 >= t1) return;
-  pack_slice<TO_BUF, false>(jb.tensor, buffer, jb.seq_offset, jb.seq_tokens, TO_BUF ? jb.mask : nullptr, jb.num_seq, jb.token_bytes,
-                            jb.num_tokens, 1, t0, t1, lds_scratch);
+    for (int u = 0; u < N; ++u) r[u] = load(i + u * kPackThreads);
+    int j = i;   // (opaque: what the second half derives from it is computed there, not kept in registers across the loads)
+    asm volatile("" : "+v"(j));
+#pragma unroll
+    for (int u = 0; u < N; ++u) use(j + u * kPackThreads, r[u]);
+  }
+}
+__device__ __forceinline__ void copy_run(uint8_t *dst, const uint8_t *src, uint32_t nvec) {
+  const run_t d = make_run(dst, nvec), s = make_run(src, nvec);
+  rounds<kUnroll>(nvec, [&](int i) { return load_nt(s, i); }, [&](int i, u32x4 v) { store_nt(d, i, v); });
+}
+
+// `n` tokens of a job that covers a part of each, from row `row` on, at `buf` in the buffer: both sides are rows at a pitch.
+template <bool TO_BUF>
+__device__ __forceinline__ void copy_part(const Job &jb, uint8_t *buf, int64_t row, uint32_t n) {
+  const uint32_t nvec = n * jb.part_vecs;
+  const uint32_t tp = (uint32_t)jb.pitch, bp = (uint32_t)jb.token_bytes;
+  const uint32_t last = jb.part_vecs;   // the run of a side ends with the part of its last token
+  const run_t ten = make_run(jb.data + row * jb.pitch, jb.data ? (n - 1) * (tp >> 4) + last : 0);
+  const run_t b = make_run(buf + (int64_t)jb.part_v0 * 16, (n - 1) * (bp >> 4) + last);
+  auto token_of = [&](int i) { return jb.magic ? __umulhi((uint32_t)i, jb.magic) : (uint32_t)i; };
+  rounds<kUnrollParts>(nvec,
+                       [&](int i) {
+                         const uint32_t t = token_of(i), c = i - t * jb.part_vecs;
+                         return load_at(TO_BUF ? ten : b, t * (TO_BUF ? tp : bp) + (c << 4), i < (int)nvec);
+                       },
+                       [&](int i, u32x4 v) {
+                         const uint32_t t = token_of(i), c = i - t * jb.part_vecs;
+                         store_at(TO_BUF ? b : ten, t * (TO_BUF ? bp : tp) + (c << 4), i < (int)nvec, v);
+                       });
 }
 
 template <typename T>
@@ -264,22 +192,171 @@ struct Add<__bf16> {
   }
 };
 
+
+// Sums in fp32 of the rows of several replicas, rounded once.
+template <typename T>
+struct Sum {
+  static constexpr int kN = 16 / sizeof(T);
+  float s[kN];
+  typedef T vec __attribute__((ext_vector_type(16 / sizeof(T))));
+  typedef float fvec __attribute__((ext_vector_type(16 / sizeof(T))));
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int i = 0; i < kN; ++i) s[i] = 0.f;
+  }
+  __device__ __forceinline__ void add(u32x4 v) {
+    const fvec f = __builtin_convertvector(__builtin_bit_cast(vec, v), fvec);
+#pragma unroll
+    for (int i = 0; i < kN; ++i) s[i] += f[i];
+  }
+  __device__ __forceinline__ u32x4 value() const {
+    fvec f;
+#pragma unroll
+    for (int i = 0; i < kN; ++i) f[i] = s[i];
+    return __builtin_bit_cast(u32x4, __builtin_convertvector(f, vec));
+  }
+};
+template <typename T>
+__device__ __forceinline__ void sum_replicas(const Job &jb, const uint8_t *buffer, int seg, int64_t skip, uint8_t *dst_p, uint32_t nvec) {
+  const run_t dst = make_run(dst_p, nvec);
+  for (int i = threadIdx.x; i < (int)nvec; i += kUnrollSum * kPackThreads) {
+    Sum<T> acc[kUnrollSum];
+#pragma unroll
+    for (int u = 0; u < kUnrollSum; ++u) acc[u].clear();
+    for (int c = 0; c < jb.max_cp; ++c) {
+      if (!uniform_int(jb.mask[(int64_t)seg * jb.max_cp + c])) continue;
+      const run_t src = make_run(buffer + jb.seq_offset[(int64_t)c * jb.num_seq + seg] + skip, nvec);
+      u32x4 r[kUnrollSum];
+#pragma unroll
+      for (int u = 0; u < kUnrollSum; ++u) r[u] = load_nt(src, i + u * kPackThreads);
+#pragma unroll
+      for (int u = 0; u < kUnrollSum; ++u) acc[u].add(r[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < kUnrollSum; ++u) store_nt(dst, i + u * kPackThreads, acc[u].value());
+  }
+}
+// Rows of a main copy: the rows of its copies added in order, one rounding per addition; the sum stays in the tensor
+// and, when the shard is sent (buf not null), goes to the buffer.
+template <typename T>
+__device__ __forceinline__ void sum_copies(const Job &jb, int seg, int64_t skip_rows, int32_t nc, uint8_t *main_p, uint8_t *buf, uint32_t nvec) {
+  const int64_t *starts = jb.copy_start + (int64_t)seg * jb.max_copies;
+  const run_t rows = make_run(main_p, nvec), sent = make_run(buf, buf ? nvec : 0);
+  for (int i = threadIdx.x; i < (int)nvec; i += kUnrollSum * kPackThreads) {
+    u32x4 m[kUnrollSum];
+#pragma unroll
+    for (int u = 0; u < kUnrollSum; ++u) m[u] = load_nt(rows, i + u * kPackThreads);
+    for (int32_t c = 0; c < nc; ++c) {
+      const run_t src = make_run(jb.data + (starts[c] + skip_rows) * jb.token_bytes, nvec);
+      u32x4 r[kUnrollSum];
+#pragma unroll
+      for (int u = 0; u < kUnrollSum; ++u) r[u] = load_nt(src, i + u * kPackThreads);
+#pragma unroll
+      for (int u = 0; u < kUnrollSum; ++u) m[u] = Add<T>::apply(m[u], r[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < kUnrollSum; ++u) {
+      store_nt(rows, i + u * kPackThreads, m[u]);
+      store_nt(sent, i + u * kPackThreads, m[u]);
+    }
+  }
+}
+
+// The jobs of one call: workgroups [first_wg, first_wg of the next job) serve a job, each a slice of its tokens.  One
+// launch has one tail instead of one per tensor, and the small tensors' slices fill the gaps the large one leaves.
+// PARTS: with jobs whose tokens have several parts; SUMS: with jobs that add rows up.  Launches without either are spared their
+// registers, so that two workgroups fit a compute unit.
+template <bool TO_BUF, bool PARTS, bool SUMS>
+__global__ __launch_bounds__(kPackThreads, SUMS ? 4 : 8) void exchange_kernel(Jobs jobs, uint8_t *buffer) {
+  int j = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxJobs; ++i)
+    if (i < jobs.n && (int)blockIdx.x >= jobs.job[i].first_wg) j = i;
+  const Job &jb = jobs.job[j];
+  const int64_t t0 = (int64_t)((int)blockIdx.x - jb.first_wg) * jb.tokens_per_wg;
+  int64_t t1 = t0 + jb.tokens_per_wg;
+  if (t1 > jb.num_tokens) t1 = jb.num_tokens;
+  if (t0 >= t1) return;
+  Segment sg = find_segment(jb.seq_tokens, jb.num_seq, t0);
+  int seg = sg.idx;
+  int64_t seg_start = sg.start;
+  const int64_t tb = jb.token_bytes;
+  const bool replicas = jb.kind == DISTCA_JOB_REPLICAS || jb.kind == DISTCA_JOB_REPLICA_SUM;
+  for (; seg < jb.num_seq && seg_start < t1; ++seg) {
+    const int64_t seg_end = seg_start + uniform_int64(jb.seq_tokens[seg]);
+    const int64_t a = seg_start > t0 ? seg_start : t0, b = seg_end < t1 ? seg_end : t1;
+    const int64_t skip = (a - seg_start) * tb;
+    seg_start = seg_end;
+    if (a >= b) continue;
+    const uint32_t nvec = (uint32_t)((b - a) * (tb >> 4));
+    if (replicas) {
+      if (SUMS && jb.kind == DISTCA_JOB_REPLICA_SUM) {
+        uint8_t *dst = jb.data + a * tb;
+        if (jb.dtype == DISTCA_DTYPE_BF16) sum_replicas<__bf16>(jb, buffer, seg, skip, dst, nvec);
+        else if (jb.dtype == DISTCA_DTYPE_F16) sum_replicas<_Float16>(jb, buffer, seg, skip, dst, nvec);
+        else sum_replicas<float>(jb, buffer, seg, skip, dst, nvec);
+        continue;
+      }
+      if (TO_BUF) {
+        // every live replica gets the rows, which are read once
+        const run_t src = make_run(jb.data + a * tb, nvec);
+        for (int i = threadIdx.x; i < (int)nvec; i += kUnroll * kPackThreads) {
+          u32x4 r[kUnroll];
+#pragma unroll
+          for (int u = 0; u < kUnroll; ++u) r[u] = load_nt(src, i + u * kPackThreads);
+          for (int c = 0; c < jb.max_cp; ++c) {
+            if (!uniform_int(jb.mask[(int64_t)seg * jb.max_cp + c])) continue;
+            const run_t dst = make_run(buffer + jb.seq_offset[(int64_t)c * jb.num_seq + seg] + skip, nvec);
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u) store_nt(dst, i + u * kPackThreads, r[u]);
+          }
+        }
+      } else {
+        for (int c = 0; c < jb.max_cp; ++c) {
+          if (!uniform_int(jb.mask[(int64_t)seg * jb.max_cp + c])) continue;
+          copy_run(jb.data + (c * jb.num_tokens + a) * tb, buffer + jb.seq_offset[(int64_t)c * jb.num_seq + seg] + skip, nvec);
+        }
+      }
+      continue;
+    }
+    const bool sent = !TO_BUF || !jb.mask || uniform_int(jb.mask[seg]) != 0;
+    uint8_t *buf = buffer + (sent ? jb.seq_offset[seg] + skip : 0);
+    if (SUMS && jb.kind == DISTCA_JOB_COPY_SUM) {
+      const int32_t nc = uniform_int(jb.num_copies[seg]);
+      if (nc > 0) {
+        uint8_t *m = jb.data + a * tb, *dst = sent ? buf : nullptr;
+        if (jb.dtype == DISTCA_DTYPE_BF16) sum_copies<__bf16>(jb, seg, skip / tb, nc, m, dst, nvec);
+        else if (jb.dtype == DISTCA_DTYPE_F16) sum_copies<_Float16>(jb, seg, skip / tb, nc, m, dst, nvec);
+        else sum_copies<float>(jb, seg, skip / tb, nc, m, dst, nvec);
+        continue;
+      }
+    }
+    if (!sent) continue;
+    if (PARTS && !jb.whole()) {
+      copy_part<TO_BUF>(jb, buf, a, (uint32_t)(b - a));
+      continue;
+    }
+    uint8_t *ten = jb.data + a * tb;
+    if (TO_BUF) copy_run(buf, ten, nvec);
+    else copy_run(ten, buf, nvec);
+  }
+}
+
 // data[start_s + t] += data[copy_start_id[s][c] + t] for c = 0..num_copies[s]-1 in order,
-// one rounding per addition.  Rows are cut into per-workgroup slices like pack_kernel.
+// one rounding per addition.  Rows are cut into per-workgroup slices like those of exchange_kernel.
 template <typename T>
 __global__ __launch_bounds__(kPackThreads) void grad_sum_kernel(T *__restrict__ data, const int32_t *__restrict__ num_copies,
                                                               const int64_t *__restrict__ copy_start_id,
                                                               const int64_t *__restrict__ seq_lens, int64_t num_tokens,
                                                               int64_t hidden, int64_t num_seq, int64_t max_copies,
                                                               int64_t tokens_per_wg) {
-  __shared__ int64_t lds_scratch[kPackWaves + 2];
   int64_t t0 = (int64_t)blockIdx.x * tokens_per_wg;
   int64_t t1 = t0 + tokens_per_wg;
   if (t1 > num_tokens) t1 = num_tokens;
   if (t0 >= t1) return;
-  Cursor cur = locate(seq_lens, num_seq, t0, false, lds_scratch);
-  if (cur.seg >= num_seq) return;
-  int64_t seg = cur.seg, seg_start = cur.seg_start;
+  const Segment sg = find_segment(seq_lens, (int)num_seq, t0);
+  if (sg.idx >= num_seq) return;
+  int64_t seg = sg.idx, seg_start = sg.start;
   constexpr int kPerVec = 16 / sizeof(T);
   const int64_t row_vecs = hidden / kPerVec;        // vector part of a row
   const int64_t row_tail = hidden - row_vecs * kPerVec;
@@ -318,18 +395,113 @@ __global__ __launch_bounds__(kPackThreads) void grad_sum_kernel(T *__restrict__ 
   }
 }
 
-// Tokens per workgroup slice: kSliceRounds loop rounds (one: 160 KiB at 10 vectors per lane), rounded to whole
-// tokens; never below one round.
-constexpr int kSliceRounds = DISTCA_PACK_SLICE_ROUNDS;
-int64_t slice_tokens(int64_t logical_tokens, int64_t token_bytes, int *grid) {
-  int64_t bytes = kSliceRounds * kRoundBytes;
-  const int64_t total = logical_tokens * token_bytes, want = (int64_t)num_compute_units() * 4;
-  while (bytes > kRoundBytes && total / bytes < want) bytes -= kRoundBytes;
-  int64_t per = (bytes + token_bytes / 2) / token_bytes;
+// Bytes of a workgroup's slice for a launch of `total` bytes: one loop round (160 KiB at 10 vectors per lane) once the launch
+// has four such slices per compute unit; below that as many whole vectors per thread as give every unit two workgroups, so
+// that a small copy is spread over the device (2.7 MB: 13 workgroups of 160 KiB took 6.8 us).
+int64_t slice_bytes(int64_t total) {
+  const int64_t cus = num_compute_units();
+  if (total >= 4 * cus * kRoundBytes) return kRoundBytes;
+  int64_t b = (total / (2 * cus) + kVecRound - 1) / kVecRound * kVecRound;
+  return b < kVecRound ? kVecRound : (b > kRoundBytes ? kRoundBytes : b);
+}
+int64_t slice_tokens(int64_t slice, int64_t tokens, int64_t token_bytes, int64_t *grid) {
+  int64_t per = (slice + token_bytes / 2) / token_bytes;
   if (per < 1) per = 1;
-  const int64_t g = (logical_tokens + per - 1) / per;
-  *grid = (int)(g < 0x7fffffff ? g : 0x7fffffff);
+  *grid = (tokens + per - 1) / per;
   return per;
+}
+
+// Checks one job and appends it; 0 when it was empty.
+int add_job(Jobs *jobs, const distca_exchange_job &in, int64_t token_bytes, int to_buffer, const void *buffer, const char *what) {
+  const bool replicas = in.kind == DISTCA_JOB_REPLICAS || in.kind == DISTCA_JOB_REPLICA_SUM;
+  if (in.num_seq < 0 || in.num_tokens < 0 || token_bytes < 0 || (replicas && in.max_cp < 0)) return fail(DISTCA_E_INVALID, "%s: negative size", what);
+  if (in.num_tokens == 0 || in.num_seq == 0 || token_bytes == 0 || (replicas && in.max_cp == 0)) return 0;
+  if (!buffer || !in.seq_offset || !in.seq_tokens || (replicas && !in.mask)) return fail(DISTCA_E_INVALID, "%s: null pointer", what);
+  if (token_bytes % 16) return fail(DISTCA_E_INVALID, "%s: token_bytes=%lld is not a multiple of 16", what, (long long)token_bytes);
+  if (in.num_tokens * (replicas ? in.max_cp : 1) >= (1ll << 31) || in.num_seq >= (1ll << 31) || token_bytes >= (1ll << 31))
+    return fail(DISTCA_E_INVALID, "%s: num_tokens%s must be < 2^31", what, replicas ? "*max_cp" : "");
+  if (in.kind == DISTCA_JOB_REPLICA_SUM && to_buffer) return fail(DISTCA_E_INVALID, "%s: a sum over replicas only unpacks", what);
+  if (in.kind == DISTCA_JOB_COPY_SUM && !to_buffer) return fail(DISTCA_E_INVALID, "%s: a sum over copies only packs", what);
+  if (in.kind == DISTCA_JOB_REPLICA_SUM || in.kind == DISTCA_JOB_COPY_SUM) {
+    if (in.dtype != DISTCA_DTYPE_F32 && in.dtype != DISTCA_DTYPE_F16 && in.dtype != DISTCA_DTYPE_BF16)
+      return fail(DISTCA_E_UNSUPPORTED, "%s: dtype %lld (only fp32, fp16, bf16)", what, (long long)in.dtype);
+    if (in.kind == DISTCA_JOB_COPY_SUM && (!in.num_copies || !in.copy_start)) return fail(DISTCA_E_INVALID, "%s: null pointer", what);
+  }
+  const bool whole = in.num_parts == 1 && in.part[0].bytes == token_bytes && in.part[0].pitch == token_bytes;
+  if (!whole && in.kind != DISTCA_JOB_PLAIN) return fail(DISTCA_E_INVALID, "%s: replicas and sums take whole tokens", what);
+  if (!whole && token_bytes > (1 << 19)) return fail(DISTCA_E_UNSUPPORTED, "%s: tokens of several parts hold at most 512 KiB", what);
+  int64_t at = 0;
+  auto append = [&](void *data, int64_t pitch, int64_t bytes) {
+    if (jobs->n == kMaxJobs) return fail(DISTCA_E_INVALID, "%s: more than %d parts in one launch", what, kMaxJobs);
+    Job &o = jobs->job[jobs->n++];
+    o.data = (uint8_t *)data;
+    o.seq_offset = in.seq_offset; o.seq_tokens = in.seq_tokens; o.mask = in.mask;
+    o.num_copies = in.num_copies; o.copy_start = in.copy_start;
+    o.num_tokens = in.num_tokens; o.token_bytes = token_bytes; o.pitch = pitch;
+    o.kind = (int32_t)in.kind; o.dtype = (int32_t)in.dtype;
+    o.num_seq = (int32_t)in.num_seq; o.max_cp = (int32_t)in.max_cp; o.max_copies = (int32_t)in.max_copies;
+    o.part_v0 = (uint32_t)(at / 16); o.part_vecs = (uint32_t)(bytes / 16);
+    o.magic = o.part_vecs == 1 ? 0u : (uint32_t)(((1ull << 32) + o.part_vecs - 1) / o.part_vecs);
+    at += bytes;
+    return 0;
+  };
+  for (int64_t k = 0; k < in.num_parts; ++k) {
+    const distca_token_part &p = in.part[k];
+    if (!p.data) return fail(DISTCA_E_INVALID, "%s: null pointer", what);
+    if (!aligned16(p.data) || !aligned16(buffer)) return fail(DISTCA_E_INVALID, "%s: tensor/buffer must be 16-byte aligned", what);
+    if (p.bytes <= 0 || p.bytes % 16 || p.pitch < p.bytes || p.pitch % 16 || p.pitch >= (1ll << 31) || at + p.bytes > token_bytes)
+      return fail(DISTCA_E_INVALID, "%s: a part of %lld B at a pitch of %lld B in a token of %lld B (multiples of 16)", what, (long long)p.bytes, (long long)p.pitch, (long long)token_bytes);
+    if (const int rc = append(p.data, p.pitch, p.bytes)) return rc;
+  }
+  if (at < token_bytes && to_buffer)
+    if (const int rc = append(nullptr, 0, token_bytes - at)) return rc;
+  return 0;
+}
+
+int launch_exchange(Jobs &jobs, void *buffer, int to_buffer, void *stream, int timer_id, const char *what) {
+  if (jobs.n == 0) return DISTCA_OK;
+  int64_t total = 0, wg = 0;
+  bool sums = false, parts = false;
+  for (int i = 0; i < jobs.n; ++i) {
+    const Job &o = jobs.job[i];
+    total += o.num_tokens * o.part_vecs * 16;
+    sums |= o.kind == DISTCA_JOB_REPLICA_SUM || o.kind == DISTCA_JOB_COPY_SUM;
+    parts |= !o.whole();
+  }
+  const int64_t slice = slice_bytes(total);
+  for (int i = 0; i < jobs.n; ++i) {
+    Job &o = jobs.job[i];
+    const bool sum = o.kind == DISTCA_JOB_REPLICA_SUM || o.kind == DISTCA_JOB_COPY_SUM;
+    const int64_t round = (sum ? kUnrollSum : o.whole() ? kUnroll : kUnrollParts) * kVecRound;   // one round of the job's own loop
+    int64_t grid;
+    int64_t per = slice_tokens(slice < round ? slice : round, o.num_tokens, (int64_t)o.part_vecs * 16, &grid);
+    if (!o.whole()) {   // a slice's rows lie within 2^30 bytes on both sides (32-bit offsets), and its vectors within the range of `magic`
+      const int64_t widest = o.pitch > o.token_bytes ? o.pitch : o.token_bytes;
+      const int64_t most = (1ll << 30) / widest < (1ll << 15) ? (1ll << 30) / widest : (1ll << 15);
+      if (per > most) per = most < 1 ? 1 : most, grid = (o.num_tokens + per - 1) / per;
+    }
+    o.tokens_per_wg = (int32_t)per;
+    o.first_wg = (int32_t)wg;
+    wg += grid;
+    if (wg > 0x7fffffff) return fail(DISTCA_E_INVALID, "%s: grid too large", what);
+  }
+  hipStream_t s = (hipStream_t)stream;
+  ScopedTimer timer(timer_id, s);
+  const dim3 g((unsigned)wg), b(kPackThreads);
+  uint8_t *buf = (uint8_t *)buffer;
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, b, 0, s, jobs, buf); };
+  if (to_buffer) launch(sums ? exchange_kernel<true, true, true> : parts ? exchange_kernel<true, true, false> : exchange_kernel<true, false, false>);
+  else launch(sums ? exchange_kernel<false, true, true> : parts ? exchange_kernel<false, true, false> : exchange_kernel<false, false, false>);
+  return check_launch(what);
+}
+
+distca_exchange_job whole_tokens(int64_t kind, void *tensor, const int64_t *seq_offset, const int64_t *seq_tokens, const int8_t *mask,
+                                 int64_t num_seq, int64_t token_bytes, int64_t num_tokens, int64_t max_cp) {
+  distca_exchange_job j = {};
+  j.kind = kind; j.num_parts = 1; j.max_cp = max_cp; j.num_seq = num_seq; j.num_tokens = num_tokens; j.token_bytes = token_bytes;
+  j.seq_offset = seq_offset; j.seq_tokens = seq_tokens; j.mask = mask;
+  j.part[0].data = tensor; j.part[0].pitch = j.part[0].bytes = token_bytes;
+  return j;
 }
 
 }  // namespace
@@ -337,87 +509,54 @@ int64_t slice_tokens(int64_t logical_tokens, int64_t token_bytes, int *grid) {
 
 using namespace distca;
 
+extern "C" int distca_exchange(const distca_exchange_job *jobs, int32_t num_jobs, void *buffer, int to_buffer, void *stream) {
+  if (num_jobs < 0 || num_jobs > DISTCA_EXCHANGE_MAX_JOBS) return fail(DISTCA_E_INVALID, "exchange: %d jobs (0..%d)", num_jobs, DISTCA_EXCHANGE_MAX_JOBS);
+  if (num_jobs > 0 && !jobs) return fail(DISTCA_E_INVALID, "exchange: null job list");
+  Jobs list;
+  list.n = 0;
+  for (int i = 0; i < num_jobs; ++i) {
+    if (jobs[i].kind < 0 || jobs[i].kind > DISTCA_JOB_COPY_SUM) return fail(DISTCA_E_INVALID, "exchange: unknown kind of job %lld", (long long)jobs[i].kind);
+    if (jobs[i].num_parts < 1 || jobs[i].num_parts > DISTCA_TOKEN_MAX_PARTS) return fail(DISTCA_E_INVALID, "exchange: %lld parts (1..%d)", (long long)jobs[i].num_parts, DISTCA_TOKEN_MAX_PARTS);
+    const int rc = add_job(&list, jobs[i], jobs[i].token_bytes, to_buffer, buffer, "exchange");
+    if (rc) return rc;
+  }
+  return launch_exchange(list, buffer, to_buffer, stream, DISTCA_TIMER_MEMCPY_NON_CP, "exchange");
+}
+
 extern "C" int distca_memcpy_non_cp(void *tensor, void *buffer, const int64_t *seq_offset, const int64_t *seq_tokens,
                                     const int8_t *copy_seq_mask, int64_t num_seq, int64_t token_bytes, int64_t num_tokens,
                                     int to_buffer, void *stream) {
-  if (num_seq < 0 || num_tokens < 0 || token_bytes < 0) return fail(DISTCA_E_INVALID, "memcpy_non_cp: negative size");
-  if (num_tokens == 0 || num_seq == 0 || token_bytes == 0) return DISTCA_OK;
-  if (!tensor || !buffer || !seq_offset || !seq_tokens) return fail(DISTCA_E_INVALID, "memcpy_non_cp: null pointer");
-  if (token_bytes % 16) return fail(DISTCA_E_INVALID, "memcpy_non_cp: token_bytes=%lld is not a multiple of 16", (long long)token_bytes);
-  if (!aligned16(tensor) || !aligned16(buffer)) return fail(DISTCA_E_INVALID, "memcpy_non_cp: tensor/buffer must be 16-byte aligned");
-  if (num_tokens >= (1ll << 31)) return fail(DISTCA_E_INVALID, "memcpy_non_cp: num_tokens must be < 2^31");
-  int grid;
-  int64_t per = slice_tokens(num_tokens, token_bytes, &grid);
-  hipStream_t s = (hipStream_t)stream;
-  uint8_t *t = (uint8_t *)tensor, *b = (uint8_t *)buffer;
-  ScopedTimer timer(DISTCA_TIMER_MEMCPY_NON_CP, s);
-  if (to_buffer)
-    hipLaunchKernelGGL((pack_kernel<true, false>), dim3(grid), dim3(kPackThreads), 0, s, t, b, seq_offset, seq_tokens,
-                       copy_seq_mask, num_seq, token_bytes, num_tokens, 1, per);
-  else
-    hipLaunchKernelGGL((pack_kernel<false, false>), dim3(grid), dim3(kPackThreads), 0, s, t, b, seq_offset, seq_tokens,
-                       (const int8_t *)nullptr, num_seq, token_bytes, num_tokens, 1, per);
-  return check_launch("memcpy_non_cp");
+  Jobs list;
+  list.n = 0;
+  const int rc = add_job(&list, whole_tokens(DISTCA_JOB_PLAIN, tensor, seq_offset, seq_tokens, copy_seq_mask, num_seq, token_bytes, num_tokens, 1),
+                         token_bytes, to_buffer, buffer, "memcpy_non_cp");
+  return rc ? rc : launch_exchange(list, buffer, to_buffer, stream, DISTCA_TIMER_MEMCPY_NON_CP, "memcpy_non_cp");
 }
 
 extern "C" int distca_memcpy_non_cp_multi(const distca_pack_job *jobs, int32_t num_jobs, void *buffer, int to_buffer, void *stream) {
-  if (num_jobs < 0 || num_jobs > kMaxPackJobs) return fail(DISTCA_E_INVALID, "memcpy_non_cp_multi: %d jobs (0..%d)", num_jobs, kMaxPackJobs);
+  static_assert(DISTCA_PACK_MAX_JOBS <= DISTCA_EXCHANGE_MAX_JOBS, "one launch");
+  if (num_jobs < 0 || num_jobs > DISTCA_PACK_MAX_JOBS) return fail(DISTCA_E_INVALID, "memcpy_non_cp_multi: %d jobs (0..%d)", num_jobs, DISTCA_PACK_MAX_JOBS);
   if (num_jobs == 0) return DISTCA_OK;
   if (!jobs) return fail(DISTCA_E_INVALID, "memcpy_non_cp_multi: null job list");
-  PackJobs pj;
-  pj.n = 0;
-  int64_t wg = 0;
+  Jobs list;
+  list.n = 0;
   for (int i = 0; i < num_jobs; ++i) {
     const distca_pack_job &in = jobs[i];
-    if (in.num_seq < 0 || in.num_tokens < 0 || in.token_bytes < 0) return fail(DISTCA_E_INVALID, "memcpy_non_cp_multi: job %d: negative size", i);
-    if (in.num_tokens == 0 || in.num_seq == 0 || in.token_bytes == 0) continue;
-    if (!in.tensor || !buffer || !in.seq_offset || !in.seq_tokens) return fail(DISTCA_E_INVALID, "memcpy_non_cp_multi: job %d: null pointer", i);
-    if (in.token_bytes % 16) return fail(DISTCA_E_INVALID, "memcpy_non_cp_multi: job %d: token_bytes=%lld is not a multiple of 16", i, (long long)in.token_bytes);
-    if (!aligned16(in.tensor) || !aligned16(buffer)) return fail(DISTCA_E_INVALID, "memcpy_non_cp_multi: job %d: tensor/buffer must be 16-byte aligned", i);
-    if (in.num_tokens >= (1ll << 31)) return fail(DISTCA_E_INVALID, "memcpy_non_cp_multi: job %d: num_tokens must be < 2^31", i);
-    PackJob &o = pj.job[pj.n++];
-    int grid;
-    o.tokens_per_wg = slice_tokens(in.num_tokens, in.token_bytes, &grid);
-    o.tensor = (uint8_t *)in.tensor;
-    o.seq_offset = in.seq_offset;
-    o.seq_tokens = in.seq_tokens;
-    o.mask = in.copy_seq_mask;
-    o.num_seq = in.num_seq;
-    o.token_bytes = in.token_bytes;
-    o.num_tokens = in.num_tokens;
-    o.first_wg = (int32_t)wg;
-    wg += grid;
-    if (wg > 0x7fffffff) return fail(DISTCA_E_INVALID, "memcpy_non_cp_multi: grid too large");
+    const int rc = add_job(&list, whole_tokens(DISTCA_JOB_PLAIN, in.tensor, in.seq_offset, in.seq_tokens, in.copy_seq_mask, in.num_seq, in.token_bytes, in.num_tokens, 1),
+                           in.token_bytes, to_buffer, buffer, "memcpy_non_cp_multi");
+    if (rc) return rc;
   }
-  if (pj.n == 0) return DISTCA_OK;
-  hipStream_t s = (hipStream_t)stream;
-  ScopedTimer timer(DISTCA_TIMER_MEMCPY_NON_CP, s);
-  if (to_buffer) hipLaunchKernelGGL((pack_multi_kernel<true>), dim3((unsigned)wg), dim3(kPackThreads), 0, s, pj, (uint8_t *)buffer);
-  else hipLaunchKernelGGL((pack_multi_kernel<false>), dim3((unsigned)wg), dim3(kPackThreads), 0, s, pj, (uint8_t *)buffer);
-  return check_launch("memcpy_non_cp_multi");
+  return launch_exchange(list, buffer, to_buffer, stream, DISTCA_TIMER_MEMCPY_NON_CP, "memcpy_non_cp_multi");
 }
 
 extern "C" int distca_memcpy_cp(void *tensor, void *buffer, const int8_t *do_shard, const int64_t *seq_offset,
                                 const int64_t *seq_tokens, int64_t token_bytes, int64_t num_tokens, int32_t max_cp,
                                 int64_t num_seq, int to_buffer, void *stream) {
-  if (num_seq < 0 || num_tokens < 0 || token_bytes < 0 || max_cp < 0) return fail(DISTCA_E_INVALID, "memcpy_cp: negative size");
-  if (num_tokens == 0 || num_seq == 0 || token_bytes == 0 || max_cp == 0) return DISTCA_OK;
-  if (!tensor || !buffer || !seq_offset || !seq_tokens || !do_shard) return fail(DISTCA_E_INVALID, "memcpy_cp: null pointer");
-  if (token_bytes % 16) return fail(DISTCA_E_INVALID, "memcpy_cp: token_bytes=%lld is not a multiple of 16", (long long)token_bytes);
-  if (!aligned16(tensor) || !aligned16(buffer)) return fail(DISTCA_E_INVALID, "memcpy_cp: tensor/buffer must be 16-byte aligned");
-  if (num_tokens * (int64_t)max_cp >= (1ll << 31)) return fail(DISTCA_E_INVALID, "memcpy_cp: num_tokens*max_cp must be < 2^31");
-  int grid;
-  int64_t per = slice_tokens(num_tokens * max_cp, token_bytes, &grid);
-  hipStream_t s = (hipStream_t)stream;
-  uint8_t *t = (uint8_t *)tensor, *b = (uint8_t *)buffer;
-  ScopedTimer timer(DISTCA_TIMER_MEMCPY_CP, s);
-  if (to_buffer)
-    hipLaunchKernelGGL((pack_kernel<true, true>), dim3(grid), dim3(kPackThreads), 0, s, t, b, seq_offset, seq_tokens, do_shard,
-                       num_seq, token_bytes, num_tokens, max_cp, per);
-  else
-    hipLaunchKernelGGL((pack_kernel<false, true>), dim3(grid), dim3(kPackThreads), 0, s, t, b, seq_offset, seq_tokens, do_shard,
-                       num_seq, token_bytes, num_tokens, max_cp, per);
-  return check_launch("memcpy_cp");
+  Jobs list;
+  list.n = 0;
+  const int rc = add_job(&list, whole_tokens(DISTCA_JOB_REPLICAS, tensor, seq_offset, seq_tokens, do_shard, num_seq, token_bytes, num_tokens, max_cp),
+                         token_bytes, to_buffer, buffer, "memcpy_cp");
+  return rc ? rc : launch_exchange(list, buffer, to_buffer, stream, DISTCA_TIMER_MEMCPY_CP, "memcpy_cp");
 }
 
 extern "C" int distca_grad_sum(void *data, int dtype, const int32_t *num_copies, const int64_t *copy_start_id,
@@ -428,21 +567,23 @@ extern "C" int distca_grad_sum(void *data, int dtype, const int32_t *num_copies,
   if (!data || !num_copies || !copy_start_id || !seq_lens) return fail(DISTCA_E_INVALID, "grad_sum: null pointer");
   if (!aligned16(data)) return fail(DISTCA_E_INVALID, "grad_sum: data must be 16-byte aligned");
   const int64_t esz = dtype == DISTCA_DTYPE_F32 ? 4 : 2;
-  int grid;
-  int64_t per = slice_tokens(num_tokens, hidden * esz, &grid);
+  if (num_seq >= (1ll << 31)) return fail(DISTCA_E_INVALID, "grad_sum: num_seq must be < 2^31");
+  int64_t grid;
+  const int64_t per = slice_tokens(slice_bytes(num_tokens * hidden * esz), num_tokens, hidden * esz, &grid);
+  if (grid > 0x7fffffff) return fail(DISTCA_E_INVALID, "grad_sum: grid too large");
   hipStream_t s = (hipStream_t)stream;
   ScopedTimer timer(DISTCA_TIMER_GRAD_SUM, s);
   switch (dtype) {
     case DISTCA_DTYPE_F32:
-      hipLaunchKernelGGL((grad_sum_kernel<float>), dim3(grid), dim3(kPackThreads), 0, s, (float *)data, num_copies,
+      hipLaunchKernelGGL((grad_sum_kernel<float>), dim3((unsigned)grid), dim3(kPackThreads), 0, s, (float *)data, num_copies,
                          copy_start_id, seq_lens, num_tokens, hidden, num_seq, max_copies, per);
       break;
     case DISTCA_DTYPE_F16:
-      hipLaunchKernelGGL((grad_sum_kernel<_Float16>), dim3(grid), dim3(kPackThreads), 0, s, (_Float16 *)data, num_copies,
+      hipLaunchKernelGGL((grad_sum_kernel<_Float16>), dim3((unsigned)grid), dim3(kPackThreads), 0, s, (_Float16 *)data, num_copies,
                          copy_start_id, seq_lens, num_tokens, hidden, num_seq, max_copies, per);
       break;
     case DISTCA_DTYPE_BF16:
-      hipLaunchKernelGGL((grad_sum_kernel<__bf16>), dim3(grid), dim3(kPackThreads), 0, s, (__bf16 *)data, num_copies,
+      hipLaunchKernelGGL((grad_sum_kernel<__bf16>), dim3((unsigned)grid), dim3(kPackThreads), 0, s, (__bf16 *)data, num_copies,
                          copy_start_id, seq_lens, num_tokens, hidden, num_seq, max_copies, per);
       break;
     default:

@@ -6,10 +6,11 @@ distca/runtime/attn_kernels/dispatch.py:13-221.  The transport buffer is either 
 then `instance_id` / `dispatcher_id` select the instance (None: the current one), and the unpacking
 steps switch the current instance and release the receive buffer the way the reference's do.
 
-How the steps are carried out is this library's own: the q, k and v of a tick go through one launch
-(`a2a_memcpy_non_cp_multi`) where the reference makes three, and the composite transport tokens
-([out | lse | pad], [dO | O | lse | q | pad]) are described by a `TokenLayout` that writes every part
-straight into its byte range of one preallocated matrix, instead of concatenating and then padding.
+How the steps are carried out is this library's own: the q, k and v of a step go through one launch (`ops.exchange`) where the
+reference makes three and more, and the parts of a composite transport token ([out | lse | pad], [dO | O | lse | q | pad])
+are copied straight between their own tensors and the buffer where their rows are whole 16-byte vectors.  Where they are not, or where the
+caller gets the token matrix itself, a `TokenLayout` writes every part into its byte range of one preallocated matrix,
+instead of concatenating and then padding.
 """
 from __future__ import annotations
 
@@ -18,7 +19,8 @@ from typing import List, Sequence, Tuple
 import torch
 from torch import Tensor
 
-from .ops import DispatcherWrapper, a2a_memcpy_cp, a2a_memcpy_non_cp, a2a_memcpy_non_cp_multi, pre_a2a_grad_acc
+from .ops import (DispatcherWrapper, _transport_buffer, a2a_memcpy_cp, a2a_memcpy_non_cp, a2a_memcpy_non_cp_multi, copy_sum_job, exchange,
+                  plain_job, pre_a2a_grad_acc, replicas_job, whole_vectors)
 from .utils import round_up
 
 
@@ -29,7 +31,7 @@ class TokenLayout:
 
     def __init__(self, parts: Sequence[Tuple[int, torch.dtype]]):
         self.dtypes = [dt for _, dt in parts]
-        self.sizes = [n * torch.empty((), dtype=dt).element_size() for n, dt in parts]
+        self.sizes = [n * dt.itemsize for n, dt in parts]
         self.starts = [sum(self.sizes[:i]) for i in range(len(parts))]
         self.payload = sum(self.sizes)
         self.token_bytes = round_up(self.payload)
@@ -79,20 +81,25 @@ def pre_a2a_qkv(
     that needs it.  Backward (:39-56): the gradients of duplicate k / v copies are first summed into their main
     copy, then q and only the main copies go out."""
     q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    buffer = _transport_buffer(buffer, instance_id, True)
     if is_fwd:
-        a2a_memcpy_non_cp(q, q_send_buffer_offset, q_seq_tokens, True, buffer=buffer, instance_id=instance_id)
-        for t, off in ((k, k_send_buffer_offset), (v, v_send_buffer_offset)):
-            a2a_memcpy_cp(t, kv_dispatch_mask, off, k_seq_tokens, True, buffer=buffer, instance_id=instance_id)
+        exchange([plain_job([q], q_send_buffer_offset, q_seq_tokens), replicas_job(k, kv_dispatch_mask, k_send_buffer_offset, k_seq_tokens),
+                  replicas_job(v, kv_dispatch_mask, v_send_buffer_offset, k_seq_tokens)], buffer, True)
         return q, k, v
     if kv_grad_copy_shard_mask is None:
         raise AssertionError("kv grad copy requires a dedup mask.")
-    if pre_a2a_grad_acc_args is not None:
-        for t in (k, v):
-            pre_a2a_grad_acc(t, *pre_a2a_grad_acc_args)
-    a2a_memcpy_non_cp_multi(
-        [q, k, v], [q_send_buffer_offset, k_send_buffer_offset, v_send_buffer_offset],
-        [q_seq_tokens, k_seq_tokens, k_seq_tokens], True,
-        [None, kv_grad_copy_shard_mask, kv_grad_copy_shard_mask], buffer=buffer, instance_id=instance_id)
+    jobs = [plain_job([q], q_send_buffer_offset, q_seq_tokens)]
+    for t, off in ((k, k_send_buffer_offset), (v, v_send_buffer_offset)):
+        if pre_a2a_grad_acc_args is None:
+            jobs.append(plain_job([t], off, k_seq_tokens, kv_grad_copy_shard_mask))
+        else:
+            num_copies, copy_start_id, lens = pre_a2a_grad_acc_args
+            if lens.data_ptr() == k_seq_tokens.data_ptr():
+                jobs.append(copy_sum_job(t, off, k_seq_tokens, kv_grad_copy_shard_mask, num_copies, copy_start_id))
+            else:   # the shards that are summed are not those that are sent
+                pre_a2a_grad_acc(t, num_copies, copy_start_id, lens)
+                jobs.append(plain_job([t], off, k_seq_tokens, kv_grad_copy_shard_mask))
+    exchange(jobs, buffer, True)
     return q, k, v
 
 
@@ -167,6 +174,26 @@ def pre_a2a_attn_out_grad_resend_qkv(
                        is_fwd=True, buffer=buffer, instance_id=instance_id)
 
 
+def send_attn_out_grad_resend_qkv(attn_out_grad: Tensor, attn_out: Tensor, lse_norm: Tensor, q: Tensor, k: Tensor, v: Tensor,
+                                  kv_dispatch_mask: Tensor, q_seq_tokens: Tensor, k_seq_tokens: Tensor, q_send_buffer_offset: Tensor,
+                                  k_send_buffer_offset: Tensor, v_send_buffer_offset: Tensor, instance_id: int = None, *, buffer: Tensor = None) -> None:
+    """pre_a2a_attn_out_grad_resend_qkv for a caller that does not want the request tokens themselves: the four parts go
+    straight into the buffer, where the merged matrix is written and read once more on the way (half the launch's bytes)."""
+    parts = [attn_out_grad, attn_out, lse_norm, q]
+    if not whole_vectors(*(t.shape[1] * t.element_size() for t in parts)):
+        pre_a2a_attn_out_grad_resend_qkv(attn_out_grad, attn_out, lse_norm, q, k, v, kv_dispatch_mask, q_seq_tokens, k_seq_tokens,
+                                         q_send_buffer_offset, k_send_buffer_offset, v_send_buffer_offset, instance_id, buffer=buffer)
+        return
+    _same_tokens("backward request", *parts)
+    if q.dtype != attn_out.dtype or attn_out_grad.shape != attn_out.shape:
+        raise AssertionError("dO, O and q of a backward request share one dtype, and dO has the shape of O")
+    buffer = _transport_buffer(buffer, instance_id, True)
+    parts = [t if t.stride(1) == 1 and (t.stride(0) * t.element_size()) % 16 == 0 and t.data_ptr() % 16 == 0 else t.contiguous() for t in parts]
+    k, v = k.contiguous(), v.contiguous()
+    exchange([plain_job(parts, q_send_buffer_offset, q_seq_tokens), replicas_job(k, kv_dispatch_mask, k_send_buffer_offset, k_seq_tokens),
+              replicas_job(v, kv_dispatch_mask, v_send_buffer_offset, k_seq_tokens)], buffer, True)
+
+
 def post_a2a_attn_out_grad_resend_qkv(
     recv_attn_out_shape: List[int], recv_lse_shape: List[int], recv_q_shape: List[int],
     recv_lse_dtype: torch.dtype,
@@ -185,6 +212,16 @@ def post_a2a_attn_out_grad_resend_qkv(
     act = recv_k.dtype
     layout = TokenLayout([(recv_attn_out_shape[1], act), (recv_attn_out_shape[1], act),
                           (recv_lse_shape[1], recv_lse_dtype), (recv_q_shape[1], act)])
+    if whole_vectors(*layout.sizes) and recv_k.dim() == recv_v.dim() == 2:
+        dev = recv_k.device
+        parts = [torch.empty(tuple(shape), dtype=dt, device=dev)
+                 for shape, dt in zip((recv_attn_out_shape, recv_attn_out_shape, recv_lse_shape, recv_q_shape), layout.dtypes)]
+        source = _transport_buffer(buffer, instance_id, False)
+        exchange([plain_job(parts, q_recv_buffer_offset, q_recv_seq_tokens), plain_job([recv_k], k_recv_buffer_offset, k_recv_seq_tokens),
+                  plain_job([recv_v], v_recv_buffer_offset, k_recv_seq_tokens)], source, False)
+        _unpacked(buffer, switch_buffer, instance_id)
+        d_out, out, lse, q = parts
+        return d_out, out, lse, q, recv_k, recv_v
     request = torch.empty((rows, layout.token_bytes), dtype=torch.uint8, device=recv_k.device)
     post_a2a_qkv(request, recv_k, recv_v, kv_dispatch_mask, q_recv_seq_tokens, k_recv_seq_tokens,
                  q_recv_buffer_offset, k_recv_buffer_offset, v_recv_buffer_offset,

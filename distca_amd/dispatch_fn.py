@@ -13,6 +13,7 @@ from torch import Tensor
 
 from .dispatch import post_a2a_attn_out, post_a2a_qkv, pre_a2a_attn_out, pre_a2a_qkv
 from .metadata import AlltoAllMetadata
+from .ops import exchange, plain_job, replica_sum_job, whole_vectors
 
 
 def pre_all2all_layout_transfer(q: Tensor, k: Tensor, v: Tensor, metadata: AlltoAllMetadata, is_qkv: bool = True, *,
@@ -31,14 +32,23 @@ def pre_all2all_layout_transfer(q: Tensor, k: Tensor, v: Tensor, metadata: Allto
 def pre_all2all_layout_transfer_backward(bwd_metadata: AlltoAllMetadata, dtype: torch.dtype, is_qkv: bool = True, *,
                                          buffer: Tensor):
     """The original sender unpacks the gradients that came back (dispatch_fn.py:72-107): dq
-    plainly; dk and dv land in one plane per replica, planes nobody wrote stay zero, and the sum
-    over planes is the shard's gradient.  Returns (dq, dk, dv) or (d_attn_out,)."""
+    plainly; dk and dv of a shard are the sums over its replicas, added up as they are read (the reference unpacks
+    into zeroed planes, one per replica, and sums those).  Returns (dq, dk, dv) or (d_attn_out,)."""
     dev = buffer.device
     grad_q = torch.empty(tuple(bwd_metadata.tensor_shape[0].recv_shape), dtype=dtype, device=dev)
     if not is_qkv:
         post_a2a_attn_out(grad_q, bwd_metadata.seq_lens[0].recv_seqlens, *bwd_metadata.recv_memcpy_metadata, buffer=buffer)
         return (grad_q,)
-    grad_k = torch.zeros(tuple(bwd_metadata.tensor_shape[1].recv_shape), dtype=dtype, device=dev)
+    planes = tuple(bwd_metadata.tensor_shape[1].recv_shape)
+    if dtype in (torch.bfloat16, torch.float16, torch.float32) and whole_vectors(planes[2] * dtype.itemsize):
+        grad_k = torch.empty(planes[1:], dtype=dtype, device=dev)
+        grad_v = torch.empty_like(grad_k)
+        q_off, k_off, v_off = bwd_metadata.recv_memcpy_metadata
+        q_lens, kv_lens = bwd_metadata.seq_lens[0].recv_seqlens, bwd_metadata.seq_lens[1].recv_seqlens
+        exchange([plain_job([grad_q], q_off, q_lens), replica_sum_job(grad_k, bwd_metadata.kv_replica_mask, k_off, kv_lens),
+                  replica_sum_job(grad_v, bwd_metadata.kv_replica_mask, v_off, kv_lens)], buffer, False)
+        return grad_q, grad_k, grad_v
+    grad_k = torch.zeros(planes, dtype=dtype, device=dev)
     grad_v = torch.zeros_like(grad_k)
     post_a2a_qkv(grad_q, grad_k, grad_v, bwd_metadata.kv_replica_mask, bwd_metadata.seq_lens[0].recv_seqlens,
                  bwd_metadata.seq_lens[1].recv_seqlens, *bwd_metadata.recv_memcpy_metadata, is_fwd=False, buffer=buffer)

@@ -18,10 +18,11 @@ import torch
 from torch import Tensor
 
 from . import _lib
-from .ops import DispatcherWrapper, a2a_memcpy_non_cp, a2a_memcpy_non_cp_multi, pre_a2a_grad_acc
+from .ops import (DispatcherWrapper, _transport_buffer, a2a_memcpy_non_cp, a2a_memcpy_non_cp_multi, exchange, plain_job, pre_a2a_grad_acc,
+                  whole_vectors)
 from .utils import size_pad_by_int4
-from .dispatch import (post_a2a_attn_out, post_a2a_attn_out_grad_resend_qkv, post_a2a_qkv, pre_a2a_attn_out_grad_resend_qkv,
-                       pre_a2a_attn_out_with_lse, pre_a2a_qkv)
+from .dispatch import (_unpacked, post_a2a_attn_out, post_a2a_attn_out_grad_resend_qkv, post_a2a_qkv, pre_a2a_attn_out_with_lse, pre_a2a_qkv,
+                       send_attn_out_grad_resend_qkv)
 
 
 @dataclass
@@ -691,13 +692,23 @@ def post_a2a_attn_out_with_lse(recv_buffer: Optional[Tensor], q: Tensor, num_hea
     Returns (attn_out [T, 1, Hq*D] in q's dtype, softmax_lse_bytes [T, Hq*4] uint8).  `recv_buffer`
     None reads the receive buffer of dispatcher instance `instance_id`."""
     dtype = dtype or q.dtype
-    recv_shape = tuple(metadata.tensor_shape[0].recv_shape)    # in elements of `dtype`, as the reference has it
-    recv = torch.empty(recv_shape, dtype=dtype, device=q.device).view(torch.uint8)
+    rows, cols = metadata.tensor_shape[0].recv_shape           # in elements of `dtype`, as the reference has it
+    itemsize = dtype.itemsize
+    hidden = math.prod(q.shape[1:])
+    hidden_bytes, lse_bytes = hidden * itemsize, num_heads_q * 4
+    token_bytes = cols * itemsize
+    if whole_vectors(hidden_bytes, lse_bytes, token_bytes) and hidden_bytes + lse_bytes <= token_bytes:
+        # both parts straight from the buffer
+        attn_out = torch.empty((rows, hidden), dtype=dtype, device=q.device)
+        softmax_lse_bytes = torch.empty((rows, lse_bytes), dtype=torch.uint8, device=q.device)
+        source = _transport_buffer(recv_buffer, instance_id, False)
+        exchange([plain_job([attn_out, softmax_lse_bytes], metadata.recv_memcpy_metadata[0], metadata.seq_lens[0].recv_seqlens,
+                            token_bytes=token_bytes)], source, False)
+        _unpacked(recv_buffer, switch_buffer, instance_id)
+        return attn_out.unsqueeze(1), softmax_lse_bytes
+    recv = torch.empty((rows, cols), dtype=dtype, device=q.device).view(torch.uint8)
     post_a2a_attn_out(recv, metadata.seq_lens[0].recv_seqlens, *metadata.recv_memcpy_metadata, switch_buffer=switch_buffer,
                       instance_id=instance_id, buffer=recv_buffer)
-    itemsize = torch.empty((), dtype=dtype).element_size()
-    hidden_bytes = math.prod(q.shape[1:]) * itemsize
-    lse_bytes = num_heads_q * 4
     attn_out = recv[:, :hidden_bytes].contiguous().view(dtype).unsqueeze(1)
     softmax_lse_bytes = recv[:, hidden_bytes:hidden_bytes + lse_bytes]
     return attn_out, softmax_lse_bytes
@@ -710,7 +721,7 @@ def post_a2a_attn_out_with_lse_backward(send_buffer: Optional[Tensor], grad_attn
     send buffer of dispatcher instance `instance_id`)."""
     flat = lambda t: t.reshape(t.shape[0], math.prod(t.shape[1:]))   # -1 is ambiguous for a rank that holds no tokens
     md = bwd_attn_out_qkv_metadata
-    pre_a2a_attn_out_grad_resend_qkv(
+    send_attn_out_grad_resend_qkv(
         flat(grad_attn_out), flat(attn_out), softmax_lse_bytes, flat(q), flat(k), flat(v), md.kv_replica_mask,
         md.seq_lens[0].send_seqlens, md.seq_lens[1].send_seqlens, *md.send_memcpy_metadata,
         instance_id=instance_id, buffer=send_buffer)

@@ -35,8 +35,18 @@ def _check_dtype(x: torch.Tensor, dtype: torch.dtype, name: str) -> None:
         raise RuntimeError(f"expected scalar type {dtype} but found {x.dtype} for {name}")
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+_current_device = torch._C._cuda_getDevice
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
+
+def on_stream(fn, device: torch.device, *args) -> int:
+    """fn(*args, stream) with `device` current and its current stream (as a raw handle: the Stream object torch makes for
+    `torch.cuda.current_stream()` and the device guard cost more host time than a launch)."""
+    index = device.index
+    if index is None or index == _current_device():
+        return fn(*args, _raw_stream(_current_device()))
+    with torch.cuda.device(index):
+        return fn(*args, _raw_stream(index))
 
 
 class DispatcherWrapper:
@@ -153,10 +163,8 @@ def a2a_memcpy_non_cp(
     if not buffer.is_cuda:
         raise RuntimeError("tensor buffer must be on CUDA")
     token_bytes = tensor.size(1) * tensor.element_size()
-    with torch.cuda.device(tensor.device):
-        rc = _lib.load().distca_memcpy_non_cp(
-            tensor.data_ptr(), buffer.data_ptr(), nvshmem_offset.data_ptr(), shard_tokens.data_ptr(),
-            mask_ptr, num_seq, token_bytes, tensor.size(0), 1 if to_nvshmem else 0, _stream())
+    rc = on_stream(_lib.load().distca_memcpy_non_cp, tensor.device, tensor.data_ptr(), buffer.data_ptr(), nvshmem_offset.data_ptr(),
+                   shard_tokens.data_ptr(), mask_ptr, num_seq, token_bytes, tensor.size(0), 1 if to_nvshmem else 0)
     _lib.check(rc, "a2a_memcpy_non_cp")
     return None
 
@@ -194,10 +202,27 @@ def a2a_memcpy_non_cp_multi(tensors, nvshmem_offsets, shard_tokens, to_nvshmem: 
                 raise RuntimeError("copy_seq_mask must be of shape (num_sequence,)")
         jobs[i] = _lib.PackJob(t.data_ptr(), off.data_ptr(), tok.data_ptr(), mask.data_ptr() if mask is not None else None,
                                off.size(0), t.size(1) * t.element_size(), t.size(0))
-    with torch.cuda.device(buffer.device):
-        rc = _lib.load().distca_memcpy_non_cp_multi(jobs, n, buffer.data_ptr(), 1 if to_nvshmem else 0, _stream())
+    rc = on_stream(_lib.load().distca_memcpy_non_cp_multi, buffer.device, jobs, n, buffer.data_ptr(), 1 if to_nvshmem else 0)
     _lib.check(rc, "a2a_memcpy_non_cp_multi")
     return None
+
+
+def _check_replicas(do_shard: torch.Tensor, nvshmem_offset: torch.Tensor, shard_tokens: torch.Tensor):
+    if nvshmem_offset.dim() != 2:
+        raise RuntimeError("tensor seq_nvshmem_offset must have 2 dimensions")
+    cp_degree, num_seq = nvshmem_offset.shape
+    _check_tensor(1, shard_tokens, "seq_tokens")
+    if shard_tokens.size(0) != num_seq:
+        raise RuntimeError("seq_tokens must be of dimension (num_sequence)")
+    _check_tensor(2, do_shard, "do_shard")
+    if do_shard.size(0) != num_seq or do_shard.size(1) != cp_degree:
+        raise RuntimeError("do_shard must be of dimension (num_sequence, cp_degree)")
+    _check_dtype(do_shard, torch.int8, "do_shard")
+    _check_dtype(nvshmem_offset, torch.int64, "seq_nvshmem_offset")
+    _check_dtype(shard_tokens, torch.int64, "seq_tokens")
+    if not nvshmem_offset.is_contiguous():
+        raise RuntimeError("tensor seq_nvshmem_offset must be contiguous")
+    return cp_degree, num_seq
 
 
 def a2a_memcpy_cp(
@@ -210,39 +235,17 @@ def a2a_memcpy_cp(
     `buffer`, or unpack into `tensor` [max_cp, T, hidden] (which the caller pre-zeroes)."""
     buffer = _transport_buffer(buffer, instance_id, to_nvshmem)
     _check_tensor(2 if to_nvshmem else 3, tensor, "tensor")
-    if nvshmem_offset.dim() != 2:
-        raise RuntimeError("tensor seq_nvshmem_offset must have 2 dimensions")
-    num_seq = nvshmem_offset.size(1)
-    cp_degree = nvshmem_offset.size(0)
-    _check_tensor(1, shard_tokens, "seq_tokens")
-    if shard_tokens.size(0) != num_seq:
-        raise RuntimeError("seq_tokens must be of dimension (num_sequence)")
-    _check_tensor(2, do_shard, "do_shard")
-    if do_shard.size(0) != num_seq or do_shard.size(1) != cp_degree:
-        raise RuntimeError("do_shard must be of dimension (num_sequence, cp_degree)")
-    _check_dtype(do_shard, torch.int8, "do_shard")
-    _check_dtype(nvshmem_offset, torch.int64, "seq_nvshmem_offset")
-    _check_dtype(shard_tokens, torch.int64, "seq_tokens")
-    if not nvshmem_offset.is_contiguous():
-        raise RuntimeError("tensor seq_nvshmem_offset must be contiguous")
+    cp_degree, num_seq = _check_replicas(do_shard, nvshmem_offset, shard_tokens)
     hidden_dim = 1 if to_nvshmem else 2
     token_bytes = tensor.size(hidden_dim) * tensor.element_size()
     num_tokens = tensor.size(0) if to_nvshmem else tensor.size(1)
-    with torch.cuda.device(tensor.device):
-        rc = _lib.load().distca_memcpy_cp(
-            tensor.data_ptr(), buffer.data_ptr(), do_shard.data_ptr(), nvshmem_offset.data_ptr(),
-            shard_tokens.data_ptr(), token_bytes, num_tokens, cp_degree, num_seq,
-            1 if to_nvshmem else 0, _stream())
+    rc = on_stream(_lib.load().distca_memcpy_cp, tensor.device, tensor.data_ptr(), buffer.data_ptr(), do_shard.data_ptr(),
+                   nvshmem_offset.data_ptr(), shard_tokens.data_ptr(), token_bytes, num_tokens, cp_degree, num_seq, 1 if to_nvshmem else 0)
     _lib.check(rc, "a2a_memcpy_cp")
     return None
 
 
-def pre_a2a_grad_acc(
-    tensor: torch.Tensor, num_copies: torch.Tensor,
-    copy_start_id: torch.Tensor, shard_tokens: torch.Tensor,
-):
-    """Sums the gradient rows of every duplicate KV copy into its main copy, in place, so
-    that only one gradient per shard has to be sent back."""
+def _check_copies(tensor: torch.Tensor, num_copies: torch.Tensor, copy_start_id: torch.Tensor, shard_tokens: torch.Tensor) -> int:
     _check_tensor(2, tensor, "tensor")
     _check_tensor(1, num_copies, "num_copies")
     _check_tensor(1, shard_tokens, "seq_lens")
@@ -257,9 +260,116 @@ def pre_a2a_grad_acc(
     _check_dtype(shard_tokens, torch.int64, "seq_lens")
     if tensor.dtype not in _DTYPE_CODE:
         raise RuntimeError("Only fp32, fp16 and bf16 inputs are supported")
-    with torch.cuda.device(tensor.device):
-        rc = _lib.load().distca_grad_sum(
-            tensor.data_ptr(), _DTYPE_CODE[tensor.dtype], num_copies.data_ptr(), copy_start_id.data_ptr(),
-            shard_tokens.data_ptr(), tensor.size(0), tensor.size(1), num_seqs, copy_start_id.size(1), _stream())
+    return num_seqs
+
+
+def pre_a2a_grad_acc(
+    tensor: torch.Tensor, num_copies: torch.Tensor,
+    copy_start_id: torch.Tensor, shard_tokens: torch.Tensor,
+):
+    """Sums the gradient rows of every duplicate KV copy into its main copy, in place, so
+    that only one gradient per shard has to be sent back."""
+    num_seqs = _check_copies(tensor, num_copies, copy_start_id, shard_tokens)
+    rc = on_stream(_lib.load().distca_grad_sum, tensor.device, tensor.data_ptr(), _DTYPE_CODE[tensor.dtype], num_copies.data_ptr(),
+                   copy_start_id.data_ptr(), shard_tokens.data_ptr(), tensor.size(0), tensor.size(1), num_seqs, copy_start_id.size(1))
     _lib.check(rc, "pre_a2a_grad_acc")
     return tensor
+
+
+# ---------------------------------------------------------------------------------------
+# Several copies of one side of an all-to-all as the jobs of one launch (distca_exchange).  A job is its words and the tensors they
+# point into, which it keeps alive until it is launched.
+# ---------------------------------------------------------------------------------------
+_NO_PARTS = (0, 0, 0)
+
+
+def _check_shards(offset: torch.Tensor, tokens: torch.Tensor, mask: Optional[torch.Tensor]) -> None:
+    _check_tensor(1, offset, "seq_nvshmem_offset")
+    _check_tensor(1, tokens, "seq_tokens")
+    _check_dtype(offset, torch.int64, "seq_nvshmem_offset")
+    _check_dtype(tokens, torch.int64, "seq_tokens")
+    if tokens.size(0) < offset.size(0):
+        raise RuntimeError("seq_tokens must be of shape (num_sequence,)")
+    if mask is not None:
+        _check_tensor(1, mask, "copy_seq_mask")
+        _check_dtype(mask, torch.int8, "copy_seq_mask")
+        if mask.size(0) != offset.size(0):
+            raise RuntimeError("copy_seq_mask must be of shape (num_sequence,)")
+
+
+def _rows(tensor: torch.Tensor):
+    """(pointer, bytes between rows, bytes of a row) of a [tokens, hidden] tensor whose rows are contiguous."""
+    if tensor.dim() != 2:
+        raise RuntimeError("tensor must have 2 dimensions")
+    if not tensor.is_cuda:
+        raise RuntimeError("tensor must be on CUDA")
+    esz = tensor.element_size()
+    if tensor.size(1) > 1 and tensor.stride(1) != 1:
+        raise RuntimeError("tensor must have contiguous rows")
+    row = tensor.size(1) * esz
+    return tensor.data_ptr(), (tensor.stride(0) * esz if tensor.size(0) > 1 else row), row
+
+
+def plain_job(parts, offset: torch.Tensor, tokens: torch.Tensor, mask: Optional[torch.Tensor] = None, token_bytes: Optional[int] = None):
+    """Rows of `parts` ([tokens, hidden] tensors, side by side in a transport token of `token_bytes`, by default exactly
+    their rows) to or from one place per shard."""
+    _check_shards(offset, tokens, mask)
+    words = []
+    for t in parts:
+        words += _rows(t)
+    row = sum(words[2::3])
+    if any(t.size(0) != parts[0].size(0) for t in parts):
+        raise RuntimeError("token parts disagree on the token count")
+    words += _NO_PARTS * (_lib.TOKEN_MAX_PARTS - len(parts))
+    return [_lib.JOB_PLAIN, 0, len(parts), offset.size(0), parts[0].size(0), token_bytes or row, 1, 0, offset.data_ptr(), tokens.data_ptr(),
+            mask.data_ptr() if mask is not None else 0, 0, 0, *words], (parts, offset, tokens, mask)
+
+
+def _whole_job(kind: int, tensor: torch.Tensor, offset, tokens, mask, num_seq: int, max_cp: int = 1, num_copies=None, copy_start=None):
+    row = tensor.size(1) * tensor.element_size()
+    return [kind, _DTYPE_CODE.get(tensor.dtype, 0), 1, num_seq, tensor.size(0), row, max_cp, copy_start.size(1) if copy_start is not None else 0,
+            offset.data_ptr(), tokens.data_ptr(), mask.data_ptr() if mask is not None else 0,
+            num_copies.data_ptr() if num_copies is not None else 0, copy_start.data_ptr() if copy_start is not None else 0,
+            tensor.data_ptr(), row, row, *_NO_PARTS * (_lib.TOKEN_MAX_PARTS - 1)], (tensor, offset, tokens, mask, num_copies, copy_start)
+
+
+def whole_vectors(*row_bytes: int) -> bool:
+    """Whether parts of these sizes can be copied as parts of a token (whole 16-byte vectors each)."""
+    return all(n > 0 and n % 16 == 0 for n in row_bytes)
+
+
+def replicas_job(tensor: torch.Tensor, do_shard: torch.Tensor, offset: torch.Tensor, tokens: torch.Tensor):
+    """a2a_memcpy_cp packing `tensor` [tokens, hidden]."""
+    _check_tensor(2, tensor, "tensor")
+    cp_degree, num_seq = _check_replicas(do_shard, offset, tokens)
+    return _whole_job(_lib.JOB_REPLICAS, tensor, offset, tokens, do_shard, num_seq, cp_degree)
+
+
+def replica_sum_job(tensor: torch.Tensor, do_shard: torch.Tensor, offset: torch.Tensor, tokens: torch.Tensor):
+    """Every row of `tensor` [tokens, hidden] from the sum of its live replicas' rows: a2a_memcpy_cp into zeroed planes
+    [max_cp, tokens, hidden] and their sum over the first dimension, without the planes."""
+    _check_tensor(2, tensor, "tensor")
+    if tensor.dtype not in _DTYPE_CODE:
+        raise RuntimeError("Only fp32, fp16 and bf16 inputs are supported")
+    cp_degree, num_seq = _check_replicas(do_shard, offset, tokens)
+    return _whole_job(_lib.JOB_REPLICA_SUM, tensor, offset, tokens, do_shard, num_seq, cp_degree)
+
+
+def copy_sum_job(tensor: torch.Tensor, offset: torch.Tensor, tokens: torch.Tensor, mask: Optional[torch.Tensor], num_copies: torch.Tensor,
+                 copy_start_id: torch.Tensor):
+    """pre_a2a_grad_acc(tensor, num_copies, copy_start_id, tokens), then the plain pack of the shards `mask` names."""
+    num_seq = _check_copies(tensor, num_copies, copy_start_id, tokens)
+    _check_shards(offset, tokens, mask)
+    return _whole_job(_lib.JOB_COPY_SUM, tensor, offset, tokens, mask, num_seq, 1, num_copies, copy_start_id)
+
+
+def exchange(jobs, buffer: torch.Tensor, to_nvshmem: bool) -> None:
+    """Runs up to four jobs against `buffer` in one launch."""
+    if not buffer.is_cuda:
+        raise RuntimeError("tensor buffer must be on CUDA")
+    words = []
+    for job, _ in jobs:
+        words += job
+    rc = on_stream(_lib.load().distca_exchange, buffer.device, _lib.ExchangeJobs[len(jobs)](*words), len(jobs), buffer.data_ptr(),
+                   1 if to_nvshmem else 0)
+    _lib.check(rc, "exchange")

@@ -114,6 +114,45 @@ int distca_grad_sum(void *data, int dtype, const int32_t *num_copies,
                     int64_t num_tokens, int64_t hidden, int64_t num_seq,
                     int64_t max_copies, void *stream);
 
+/* What a rank does on one side of an all-to-all, as the jobs of one launch.  The reference makes a pass
+ * per tensor and, where a transport token carries several tensors' rows, further passes that concatenate
+ * and pad them or cut them apart (attn_kernels/dispatch.py:129-206); where replicas come back, it
+ * zeroes planes, unpacks into them and adds them up (dispatch_fn.py:72-107).
+ *
+ * Rows and byte ranges of shards as in distca_memcpy_non_cp.  A token's row may be made of up to
+ * DISTCA_TOKEN_MAX_PARTS parts, side by side in the buffer from byte 0 of the token on, each in a tensor of its own:
+ * part i of token t is at data + t * pitch, `bytes` long.  Bytes of the token behind the last part are written as
+ * zeros when packing and skipped when unpacking.  Kinds:
+ *   PLAIN        one copy per shard; mask (packing only, may be NULL) skips shards
+ *   REPLICAS     distca_memcpy_cp with mask = do_shard; one part of token_bytes
+ *   REPLICA_SUM  unpacking: row t becomes the sum of its live replicas' rows (in fp32, rounded once)
+ *   COPY_SUM     packing: distca_grad_sum of the shard (the sum stays in the tensor), then PLAIN
+ * dtype (the two sums) is one of DISTCA_DTYPE_*.  Pointers, pitches, part and token sizes are multiples of 16.
+ * Jobs run at the same time: their byte ranges must be disjoint, and so must a COPY_SUM's main shards and copies. */
+#define DISTCA_EXCHANGE_MAX_JOBS 4
+#define DISTCA_TOKEN_MAX_PARTS 4
+#define DISTCA_JOB_PLAIN 0
+#define DISTCA_JOB_REPLICAS 1
+#define DISTCA_JOB_REPLICA_SUM 2
+#define DISTCA_JOB_COPY_SUM 3
+typedef struct distca_token_part {
+  void *data;
+  int64_t pitch;
+  int64_t bytes;
+} distca_token_part;
+typedef struct distca_exchange_job {
+  int64_t kind, dtype, num_parts, num_seq, num_tokens, token_bytes;
+  int64_t max_cp;               /* replicas: rows of seq_offset [max_cp, num_seq], columns of mask [num_seq, max_cp] */
+  int64_t max_copies;           /* columns of copy_start */
+  const int64_t *seq_offset;    /* device arrays */
+  const int64_t *seq_tokens;
+  const int8_t *mask;
+  const int32_t *num_copies;    /* COPY_SUM: [num_seq] */
+  const int64_t *copy_start;    /* COPY_SUM: [num_seq, max_copies] first rows of a shard's copies */
+  distca_token_part part[DISTCA_TOKEN_MAX_PARTS];
+} distca_exchange_job;
+int distca_exchange(const distca_exchange_job *jobs, int32_t num_jobs, void *buffer, int to_buffer, void *stream);
+
 /* ---------------------------------------------------------------------------
  * Core attention over a batch of CA tasks.
  *

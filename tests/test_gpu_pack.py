@@ -227,3 +227,110 @@ def test_through_torch_ops(cuda):
     torch.ops.distca_amd.fast_a2a_grad_acc(d, torch.from_numpy(nc).to(cuda), torch.from_numpy(cs).to(cuda), torch.tensor(ln, dtype=torch.int64, device=cuda))
     torch.cuda.synchronize()
     assert torch.equal(d.cpu().view(torch.uint8), expd.view(torch.uint8))
+
+
+@pytest.mark.parametrize("scale", [1, 40])
+@pytest.mark.parametrize("sizes,pad", [((8192, 8192, 128, 8192), 0), ((16,), 32), ((1040, 16), 16), ((2048, 24, 2048), None)])
+def test_tokens_of_several_parts(cuda, sizes, pad, scale):
+    """Parts of a transport token copied straight between their tensors and the buffer, next to a replicated tensor in the
+    same launch, against the oracle's copy of the joined rows: one-vector parts, padding behind the last part, a part read at a pitch;
+    `scale` 40 makes slices of several rounds.  Sizes that are no whole vectors are refused on the host."""
+    from distca_amd.ops import exchange, plain_job, replicas_job, whole_vectors
+    rng = np.random.default_rng(len(sizes) * 100 + scale)
+    lens = (rng.integers(0, 12, size=9) * scale).astype(np.int64)
+    lens[4] += 3
+    T = int(lens.sum())
+    parts = [rng.integers(0, 256, size=(T, n), dtype=np.uint8) for n in sizes]
+    dev = lambda a: torch.from_numpy(a).to(cuda)
+    if pad is None:
+        assert not whole_vectors(*sizes)
+        with pytest.raises(RuntimeError, match="multiple"):
+            exchange([plain_job([dev(p) for p in parts], dev(np.zeros(9, np.int64)), dev(lens))], torch.zeros(64, dtype=torch.uint8, device=cuda), True)
+        return
+    tb = sum(sizes) + pad
+    off, nbuf = _layout(rng, lens, tb)
+    joined = np.concatenate(parts + [np.zeros((T, pad), np.uint8)], axis=1)
+    # a second tensor, replicated twice behind the tokens
+    do_shard = np.ones((9, 2), np.int8)
+    do_shard[1::2, 1] = 0
+    src = rng.integers(0, 256, size=(T, 64), dtype=np.uint8)
+    cp_off = np.zeros((2, 9), np.int64)
+    for c in range(2):
+        cp_off[c] = nbuf + np.concatenate([[0], np.cumsum(lens * 64)[:-1]])
+        nbuf += T * 64
+    exp = rng.integers(0, 256, size=nbuf, dtype=np.uint8)
+    dbuf = dev(exp.copy())
+    fa2a.copy_non_cp(joined, exp, off, lens, None, True)
+    fa2a.copy_cp(src, exp, do_shard, cp_off, lens, True)
+    wide = [np.zeros((T, n + 48), np.uint8) for n in sizes]
+    for w, p in zip(wide, parts):
+        w[:, 16:16 + p.shape[1]] = p
+    d_parts = [dev(p) for p in parts]
+    d_parts[-1] = dev(wide[-1])[:, 16:16 + sizes[-1]]
+    print(f"parts {sizes} pad {pad} tokens {T}", flush=True)
+    exchange([plain_job(d_parts, dev(off), dev(lens), token_bytes=tb), replicas_job(dev(src), dev(do_shard), dev(cp_off), dev(lens))], dbuf, True)
+    torch.cuda.synchronize()
+    assert np.array_equal(dbuf.cpu().numpy(), exp)
+    back = [dev(np.full_like(w, 0x5A)) for w in wide]
+    exchange([plain_job([b[:, 16:16 + n] for b, n in zip(back, sizes)], dev(off), dev(lens), token_bytes=tb)], dbuf, False)
+    torch.cuda.synchronize()
+    for b, p in zip(back, parts):
+        want = np.full(b.shape, 0x5A, np.uint8)
+        want[:, 16:16 + p.shape[1]] = p
+        assert np.array_equal(b.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("scale", [1, 60])
+def test_rows_added_up_on_the_way(cuda, dtype, scale):
+    """A sum over replicas is the oracle's planes summed in fp32 and rounded once (three replicas: exact in fp32 for two-byte
+    elements of this range, one rounding of 2^-24 apart in fp32), shards without replicas give zeros; a sum over copies leaves
+    in tensor and buffer what the oracle's sum followed by its masked pack leaves, bit for bit."""
+    from distca_amd.ops import copy_sum_job, exchange, replica_sum_job
+    rng = np.random.default_rng(scale)
+    hidden, S = 72, 7
+    esz = torch.empty((), dtype=dtype).element_size()
+    tb = hidden * esz
+    lens = (rng.integers(1, 20, size=S) * scale).astype(np.int64)
+    T = int(lens.sum())
+    dev = lambda a: torch.from_numpy(a).to(cuda)
+    do_shard = (rng.random((S, 3)) < 0.6).astype(np.int8)
+    do_shard[0], do_shard[1] = 1, 0
+    off = np.zeros((3, S), np.int64)
+    cur = 16
+    for c in range(3):
+        for s in rng.permutation(S):
+            off[c, s] = cur
+            cur += int(lens[s]) * tb
+    g = torch.Generator().manual_seed(scale)
+    buf = torch.randn(cur // esz, generator=g).to(dtype).view(torch.uint8)
+    planes = np.zeros((3, T, tb), np.uint8)
+    fa2a.copy_cp(planes, buf.numpy(), do_shard, off, lens, False)
+    want = torch.from_numpy(planes).view(dtype).reshape(3, T, hidden).double().sum(0)
+    got = torch.full((T, hidden), float("nan"), dtype=dtype, device=cuda)
+    print(f"replica sum {dtype} tokens {T}", flush=True)
+    exchange([replica_sum_job(got, dev(do_shard), dev(off), dev(lens))], buf.to(cuda), False)
+    torch.cuda.synchronize()
+    if dtype == torch.float32:
+        assert (got.cpu().double() - want).abs().max().item() <= 2 ** -22 * want.abs().max().item()
+    else:
+        assert torch.equal(got.cpu(), want.to(dtype))
+
+    # shards 0 and 2 have copies (2 and 1) in shards 3, 4 and 5 of the same lengths
+    lens[[3, 4]] = lens[0]
+    lens[5] = lens[2]
+    start = np.concatenate([[0], np.cumsum(lens)])
+    T = int(start[-1])
+    nc = np.array([2, 0, 1, 0, 0, 0, 0], np.int32)
+    cs = np.zeros((S, 2), np.int64)
+    cs[0], cs[2, 0] = start[[3, 4]], start[5]
+    for mask in (np.array([1, 1, 1, 0, 0, 0, 1], np.int8), np.array([0, 1, 1, 0, 0, 0, 0], np.int8)):
+        data = torch.randn((T, hidden), generator=g).to(dtype)
+        boff, nbuf = _layout(rng, lens, tb)
+        exp_t, exp = data.clone(), np.full(nbuf, 0x11, np.uint8)
+        fa2a.grad_sum(exp_t, nc, cs, lens)
+        fa2a.copy_non_cp(exp_t.view(torch.uint8).numpy(), exp, boff, lens, mask, True)
+        d, dbuf = data.to(cuda), torch.full((nbuf,), 0x11, dtype=torch.uint8, device=cuda)
+        exchange([copy_sum_job(d, dev(boff), dev(lens), dev(mask), dev(nc), dev(cs))], dbuf, True)
+        torch.cuda.synchronize()
+        assert torch.equal(d.cpu().view(torch.uint8), exp_t.view(torch.uint8)) and np.array_equal(dbuf.cpu().numpy(), exp)
