@@ -62,6 +62,8 @@ SYMBOLS = {
     "distca_grad_sum": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p]),
     "distca_ca_fwd_workspace_bytes": (c_int64, [POINTER(CaParams)]),
     "distca_ca_bwd_workspace_bytes": (c_int64, [POINTER(CaParams)]),
+    "distca_ca_fwd_workspace_preferred_bytes": (c_int64, [POINTER(CaParams)]),
+    "distca_ca_bwd_workspace_preferred_bytes": (c_int64, [POINTER(CaParams)]),
     "distca_ca_fwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                               POINTER(CaParams), c_void_p, c_int64, c_void_p]),
     "distca_ca_fwd_noalloc_max_bytes": (c_int64, []),

@@ -19,7 +19,6 @@ struct BwdArgs {
   const uint8_t *lse_tok;
   float *lse2_w, *dscaled_w;
   elem_t *dq, *dk, *dv;
-  float *dk_acc, *dv_acc;  // used instead of dk/dv when tasks may alias KV rows
   const int32_t *cu_q, *cu_k, *kv_off;
   // the dK/dV list over groups of tasks that share stored K/V rows (sched.h, SharedGroups); null otherwise
   const int32_t *grp_first, *grp_tasks, *grp_off, *grp_lmax;
@@ -38,7 +37,11 @@ struct BwdArgs {
   // tensors, off[b] = cu_q[b] * tok_bytes); head h at + h * 256 bytes.  dq likewise.
   const int64_t *qs_task_off, *dq_task_off;
   int64_t qs_tok_bytes, dq_tok_bytes;
+  const int32_t *cut, *slot;  // a list with cut blocks: its tables (sched.h, SplitTables)
+  uint8_t *partial;           // and the slots of the pieces
 };
+// A piece's slot: the accumulators of a dQ block (256 rows) or of a key block (dK and dV of 256 keys) as they lie
+constexpr int64_t kDqSlotBytes = (int64_t)256 * 128 * 4, kDkdvSlotBytes = 2 * (int64_t)256 * 128 * 4;
 
 
 // The query side of a backward call: where dO, O, lse, q are read and dq is written.
@@ -74,11 +77,11 @@ int make_kv_shards(const distca_kv_shards *in, const int32_t *kv_off, bool backw
 
 // The dK/dV kernel with 64 keys per wave (attn_bwd_dkdv64.hip): LDS bytes it needs, and its launch.
 int dkdv64_lds_bytes();
-// atomic_sums: items add to the fp32 accumulators (pieces of key blocks); shared: items are (group of tasks, key block)
-int launch_dkdv64(const BwdArgs &a, int64_t grid, bool atomic_sums, bool shared, hipStream_t stream);       // bf16 elements
-int launch_dkdv64_f16(const BwdArgs &a, int64_t grid, bool atomic_sums, bool shared, hipStream_t stream);   // fp16 elements
-// The dQ kernel with 64 query rows per wave (attn_bwd_dq64.hip).
-int launch_dq64(const BwdArgs &a, int64_t grid, hipStream_t stream);
-int launch_dq64_f16(const BwdArgs &a, int64_t grid, hipStream_t stream);
+// few: the kernels for few items (sched.h, take_item); max_cut > 0 (only then): items may be pieces of key blocks, of which at most that many are cut; shared: items are (group of tasks, key block)
+int launch_dkdv64(const BwdArgs &a, int64_t grid, bool few, int64_t max_cut, bool shared, hipStream_t stream);       // bf16 elements
+int launch_dkdv64_f16(const BwdArgs &a, int64_t grid, bool few, int64_t max_cut, bool shared, hipStream_t stream);   // fp16 elements
+// The dQ kernel with 64 query rows per wave (attn_bwd_dq64.hip).  max_cut as above, for blocks of query rows.
+int launch_dq64(const BwdArgs &a, int64_t grid, bool few, int64_t max_cut, hipStream_t stream);
+int launch_dq64_f16(const BwdArgs &a, int64_t grid, bool few, int64_t max_cut, hipStream_t stream);
 
 }  // namespace distca

@@ -16,8 +16,6 @@
 //      the workspace.
 //   2. ca_bwd_dkdv64_kernel (attn_bwd_dkdv64.hip): dK and dV, one workgroup of 4 waves per (task, block of
 //      256 keys, kv head), in the order of the backward tile schedule.
-#include <hip/amd_detail/amd_hip_unsafe_atomics.h>
-
 #include "api_util.h"
 #include "attn_bwd.h"
 #include "attn_cfg.h"
@@ -28,94 +26,40 @@
 namespace distca {
 namespace {
 
-// Zeroes the dk / dv rows that no workgroup of the dK/dV kernel writes when every task owns its K/V rows: the
-// rows of tasks without queries (they get no work item) and the rows past the last task.  Workgroup (b, y):
-// part y of task b's rows, b == num_tasks standing for the tail.
-__global__ __launch_bounds__(256) void fill_unowned_rows_kernel(u32x4 *__restrict__ dk, u32x4 *__restrict__ dv,
-                                                               const int32_t *__restrict__ cu_q, const int32_t *__restrict__ cu_k,
-                                                               int32_t num_tasks, int32_t total_k, int64_t row_vecs) {
-  const int b = blockIdx.x;
-  int64_t r0, r1;
-  if (b < num_tasks) {
-    if (cu_q[b + 1] > cu_q[b]) return;
-    r0 = cu_k[b];
-    r1 = cu_k[b + 1];
-  } else {
-    r0 = cu_k[num_tasks];
-    r1 = total_k;
-  }
-  if (r0 < 0) r0 = 0;
-  if (r1 > total_k) r1 = total_k;
-  const int64_t v0 = r0 * row_vecs, v1 = r1 * row_vecs;
-  for (int64_t i = v0 + (int64_t)blockIdx.y * 256 + threadIdx.x; i < v1; i += (int64_t)gridDim.y * 256) {
-    dk[i] = u32x4{0, 0, 0, 0};
-    dv[i] = u32x4{0, 0, 0, 0};
-  }
-}
-
-// The same for tasks over shared stored rows: zeroes the stored rows no group of tasks covers (sched.h, SharedGroups:
-// gap u, u <= num_tasks; those past the number of groups are empty).  Workgroup (u, y): part y of gap u.
-__global__ __launch_bounds__(256) void fill_gap_rows_kernel(u32x4 *__restrict__ dk, u32x4 *__restrict__ dv,
-                                                           const int32_t *__restrict__ gap_lo, const int32_t *__restrict__ gap_hi,
-                                                           int32_t total_k, int64_t row_vecs) {
-  int64_t r0 = gap_lo[blockIdx.x], r1 = gap_hi[blockIdx.x];
-  if (r0 < 0) r0 = 0;
-  if (r1 > total_k) r1 = total_k;
-  const int64_t v0 = r0 * row_vecs, v1 = r1 * row_vecs;
-  for (int64_t i = v0 + (int64_t)blockIdx.y * 256 + threadIdx.x; i < v1; i += (int64_t)gridDim.y * 256) {
-    dk[i] = u32x4{0, 0, 0, 0};
-    dv[i] = u32x4{0, 0, 0, 0};
-  }
-}
-
-// The same with the dK/dV rows addressed through a table of shards (kv_shards.h): one row per 128-thread slice.
-__global__ __launch_bounds__(256) void fill_gap_rows_shards_kernel(uint8_t *__restrict__ dk, uint8_t *__restrict__ dv,
-                                                                  const int32_t *__restrict__ gap_lo, const int32_t *__restrict__ gap_hi,
-                                                                  int32_t total_k, int64_t row_bytes, KvShards sh) {
-  int64_t r0 = gap_lo[blockIdx.x], r1 = gap_hi[blockIdx.x];
-  if (r0 < 0) r0 = 0;
-  if (r1 > total_k) r1 = total_k;
-  for (int64_t r = r0 + blockIdx.y; r < r1; r += gridDim.y) {
-    const int s = find_shard(sh.row_start, sh.num_shards, (int)r);
-    const int64_t in_shard = (r - sh.row_start[s]) * row_bytes;
-    u32x4 *pk = reinterpret_cast<u32x4 *>(dk + sh.dk_off[s] + in_shard), *pv = reinterpret_cast<u32x4 *>(dv + sh.dv_off[s] + in_shard);
-    for (int64_t i = threadIdx.x; i < row_bytes / 16; i += 256) {
-      pk[i] = u32x4{0, 0, 0, 0};
-      pv[i] = u32x4{0, 0, 0, 0};
-    }
-  }
-}
-
 __global__ __launch_bounds__(256) void fill_zero_kernel(u32x4 *__restrict__ p, int64_t nvec) {
   int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t stride = (int64_t)gridDim.x * 256;
   for (; i < nvec; i += stride) p[i] = u32x4{0, 0, 0, 0};
 }
 
-// fp32 accumulator -> bf16, 8 elements per thread
-__global__ __launch_bounds__(256) void cvt_elem_kernel(const float *__restrict__ src, elem_t *__restrict__ dst, int64_t n8) {
-  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t stride = (int64_t)gridDim.x * 256;
-  for (; i < n8; i += stride) {
-    const f32x4 x = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(src) + 2 * i);
-    const f32x4 y = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(src) + 2 * i + 1);
-    reinterpret_cast<elemx8 *>(dst)[i] = cvt8(x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]);
-  }
-}
-
-struct BwdWorkspace {
-  int64_t sched_kv, sched_q, delta, lse2, dk_acc, dv_acc, total;
+// How a backward is laid out in its workspace: the two lists, the row statistics, and, where blocks are cut into pieces, the lists'
+// tables and one place for the slots of both (dQ's pieces are added up before the first of dK / dV is written).
+struct BwdLayout {
+  int64_t sched_kv, sched_q, delta, lse2, tables_kv, tables_q, slots, total;
+  int64_t blocks_kv, blocks_q, items_kv, items_q;   // bounds on blocks, and room of the lists
+  int32_t target_kv, target_q;                      // pieces aimed for per kv head, 0: whole blocks
 };
-// acc: with the fp32 dK/dV accumulators (needed only when key blocks are cut into pieces); max_items_kv: room of the dK/dV list
-BwdWorkspace bwd_layout(const distca_ca_params *p, bool alias, int64_t max_items_kv) {
-  BwdWorkspace w;
+// shared: tasks over shared stored rows (items are then over groups of tasks).  preferred: cut blocks of query rows as well, and
+// key blocks whatever `deterministic` says.
+BwdLayout bwd_layout(const distca_ca_params *p, bool shared, bool preferred) {
+  BwdLayout w;
+  w.blocks_kv = shared ? bwd_key_blocks_own_rows(p) : bwd_max_items(p) - bwd_split_target(p);
+  w.blocks_q = dq_max_items(p);
+  w.target_kv = preferred ? bwd_split_pieces(p, kSplitPreferredPerCU) : bwd_split_target(p);
+  w.target_q = preferred ? row_split_target(p, w.blocks_q) : 0;
+  w.items_kv = w.blocks_kv + w.target_kv;
+  w.items_q = w.blocks_q + w.target_q;
   int64_t o = 0;
-  w.sched_kv = o; o += sched_shared_region_bytes(p->num_tasks, max_items_kv);
-  w.sched_q = o; o += sched_region_bytes(p->num_tasks, dq_max_items(p));
-  w.delta = o; o += align_up((int64_t)p->num_heads_q * p->total_q * 4, 256);
-  w.lse2 = o; o += align_up((int64_t)p->num_heads_q * p->total_q * 4, 256);
-  w.dk_acc = o; if (alias) o += align_up((int64_t)p->total_k * p->num_heads_kv * kHeadDim * 4, 256);
-  w.dv_acc = o; if (alias) o += align_up((int64_t)p->total_k * p->num_heads_kv * kHeadDim * 4, 256);
+  auto take = [&](int64_t bytes) { const int64_t at = o; o = align_up(o + bytes, 256); return at; };
+  w.sched_kv = take(sched_shared_region_bytes(p->num_tasks, w.items_kv));
+  w.sched_q = take(sched_region_bytes(p->num_tasks, w.items_q));
+  w.delta = take((int64_t)p->num_heads_q * p->total_q * 4);
+  w.lse2 = take((int64_t)p->num_heads_q * p->total_q * 4);
+  w.tables_kv = take(split_tables_bytes(w.blocks_kv, w.target_kv, w.items_kv));
+  w.tables_q = take(split_tables_bytes(w.blocks_q, w.target_q, w.items_q));
+  const int64_t kv = split_max_slots(w.blocks_kv, w.target_kv) * kDkdvSlotBytes, q = split_max_slots(w.blocks_q, w.target_q) * kDqSlotBytes;
+  w.slots = take((kv > q ? kv : q) * p->num_heads_kv);
+  if (preferred && o > w.slots) take(256);   // (so that no call that brought the smallest workspace is taken for one that brought this)
   w.total = o;
   return w;
 }
@@ -137,9 +81,17 @@ extern "C" int64_t distca_ca_bwd_workspace_bytes(const distca_ca_params *p) {
   if (!p) return fail(DISTCA_E_INVALID, "bwd_workspace_bytes: null params");
   int rc = validate_params(p);
   if (rc) return rc;
-  // the work lists and row statistics, and, only when key blocks are cut into pieces (small batches whose caller
-  // allows float atomics), the fp32 dK/dV accumulators
-  return bwd_layout(p, bwd_split_target(p) > 0, bwd_max_items(p)).total;
+  // the work lists and row statistics, and, when key blocks are cut into pieces (small batches whose caller does not ask for
+  // a deterministic backward), the slots of the pieces
+  return bwd_layout(p, false, false).total;
+}
+
+extern "C" int64_t distca_ca_bwd_workspace_preferred_bytes(const distca_ca_params *p) {
+  if (!p) return fail(DISTCA_E_INVALID, "bwd_workspace_preferred_bytes: null params");
+  int rc = validate_params(p);
+  if (rc) return rc;
+  const int64_t own = bwd_layout(p, false, true).total, shared = bwd_layout(p, true, true).total;
+  return own > shared ? own : shared;
 }
 
 extern "C" int distca_ca_bwd(const void *dout, const void *q, const void *k, const void *v, const void *out, const float *lse,
@@ -202,46 +154,31 @@ int DISTCA_FN(run_bwd)(const BwdQuerySide &qs, const void *k, const void *v, voi
   }
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out) || !aligned16(dout) || !aligned16(dq) || !aligned16(dk) || !aligned16(dv))
     return fail(DISTCA_E_INVALID, "ca_bwd: tensors must be 16-byte aligned");
-  // dK/dV go through fp32 accumulators (float atomics) only when key blocks are cut into pieces.  Tasks over shared
-  // K/V rows otherwise have one work item per (group of tasks, key block), which sums in registers like any other.
-  // With K/V shards read in place nothing is cut (the accumulators are dense tensors over stored rows).
+  // Tasks over shared K/V rows have one work item per (group of tasks, key block), or pieces of it.
   KvShards shards{};
   if (kv_shards) {
     rc = make_kv_shards(kv_shards, kv_off, true, &shards);
     if (rc) return rc;
   }
-  const int32_t split = kv_shards ? 0 : bwd_split_target(p);
-  const bool use_acc = split > 0;
-  const bool shared = alias && !use_acc;
-  const int64_t max_items_kv = split > 0 ? bwd_key_blocks_bound(p) + split : bwd_key_blocks_own_rows(p);
-  const BwdWorkspace w = bwd_layout(p, use_acc, max_items_kv);
+  const bool shared = alias;
+  const bool preferred = workspace_bytes >= bwd_layout(p, shared, true).total;   // room for everything the call can use
+  const BwdLayout w = bwd_layout(p, shared, preferred);
   if (!workspace || workspace_bytes < w.total)
     return fail(DISTCA_E_WORKSPACE, "ca_bwd: workspace %lld B < required %lld B", (long long)workspace_bytes, (long long)w.total);
   if (!aligned16(workspace)) return fail(DISTCA_E_INVALID, "ca_bwd: workspace must be 16-byte aligned");
   hipStream_t s = (hipStream_t)stream;
   uint8_t *ws = (uint8_t *)workspace;
   const int64_t kv_elems = (int64_t)p->total_k * p->num_heads_kv * kHeadDim;
-  const int64_t q_elems = (int64_t)p->total_q * p->num_heads_q * kHeadDim;
 
-  // rows no task touches must come back as zero
-  if (kv_elems > 0) {
-    if (use_acc) {
-      hipLaunchKernelGGL(fill_zero_kernel, dim3(grid_for(kv_elems / 2)), dim3(256), 0, s, (u32x4 *)(ws + w.dk_acc),
-                         (w.total - w.dk_acc) / 16);
-    } else if ((p->num_tasks == 0 || p->total_q == 0) && kv_shards) {
+  if (p->num_tasks == 0 || p->total_q == 0) {   // nothing to do but to clear dk and dv
+    if (kv_elems > 0 && kv_shards)
       return fail(DISTCA_E_UNSUPPORTED, "ca_bwd_buffers: a batch without tasks or queries (there is nothing to tell which rows to clear)");
-    } else if (p->num_tasks == 0 || p->total_q == 0) {
+    if (kv_elems > 0) {
       hipLaunchKernelGGL(fill_zero_kernel, dim3(grid_for(kv_elems / 8)), dim3(256), 0, s, (u32x4 *)dk, kv_elems / 8);
       hipLaunchKernelGGL(fill_zero_kernel, dim3(grid_for(kv_elems / 8)), dim3(256), 0, s, (u32x4 *)dv, kv_elems / 8);
-    } else if (!shared) {
-      // every task owns its rows and the dK/dV kernel writes each row of a task that has queries exactly once:
-      // only the others need the fill (at 131 072 tokens that is 0.5 GB of writes not made); with shared rows the
-      // fill follows the list builder below, which finds the rows no group of tasks covers
-      hipLaunchKernelGGL(fill_unowned_rows_kernel, dim3((unsigned)p->num_tasks + 1, 16), dim3(256), 0, s, (u32x4 *)dk, (u32x4 *)dv,
-                         cu_q, cu_k, p->num_tasks, p->total_k, (int64_t)p->num_heads_kv * kHeadDim / 8);
     }
+    return check_launch("ca_bwd(clear)");
   }
-  if (p->num_tasks == 0 || p->total_q == 0) return check_launch("ca_bwd(clear)");
 
   BwdArgs a;
   a.q = (const elem_t *)q; a.k = (const elem_t *)k; a.v = (const elem_t *)v; a.dout = (const elem_t *)dout;
@@ -250,8 +187,7 @@ int DISTCA_FN(run_bwd)(const BwdQuerySide &qs, const void *k, const void *v, voi
   a.out = (const elem_t *)out; a.lse = qs.lse; a.lse_tok = (const uint8_t *)qs.lse_tok;
   a.dq = (elem_t *)dq; a.dk = (elem_t *)dk; a.dv = (elem_t *)dv;
   a.qs_task_off = qs.task_off; a.qs_tok_bytes = qs.tok_bytes; a.dq_task_off = qs.dq_task_off; a.dq_tok_bytes = qs.dq_tok_bytes;
-  a.dk_acc = use_acc ? (float *)(ws + w.dk_acc) : nullptr;
-  a.dv_acc = use_acc ? (float *)(ws + w.dv_acc) : nullptr;
+  a.partial = ws + w.slots;
   a.cu_q = cu_q; a.cu_k = cu_k; a.kv_off = kv_off;
   a.grp_first = a.grp_tasks = a.grp_off = a.grp_lmax = nullptr;
   a.shards = shards;
@@ -262,60 +198,49 @@ int DISTCA_FN(run_bwd)(const BwdQuerySide &qs, const void *k, const void *v, voi
   if ((uint64_t)p->max_seqlen_q * a.group * a.group >= (1ull << 32))
     return fail(DISTCA_E_UNSUPPORTED, "ca_bwd: max_seqlen_q * (Hq/Hkv)^2 must stay below 2^32");
 
+  // ---- both work lists, and zeros where no work item writes dk / dv
+  const bool few_q = few_row_blocks(p), few_kv = few_key_blocks(p, kSplitFewPerCU) || w.target_kv > 0;
+  auto tables_of = [&](int64_t at, int64_t blocks, int32_t target) { return target > 0 ? split_tables(ws + at, blocks, target) : SplitTables{}; };
+  ListJob q_list{cu_q, cu_k, launched_geom(dq_geom(p), p), (int32_t *)(ws + w.sched_q), w.items_q, tables_of(w.tables_q, w.blocks_q, w.target_q)};
+  if (w.target_q > 0) cut_where_worth(&q_list.geom, p, w.target_q, 6, 3);
+  ListJob kv_list{cu_q, cu_k, shared ? bwd_shared_geom(p) : bwd_geom(p), (int32_t *)(ws + w.sched_kv), w.items_kv, tables_of(w.tables_kv, w.blocks_kv, w.target_kv)};
+  kv_list.geom.split_target = w.target_kv;
+  if (w.target_kv > 0 && preferred) cut_where_worth(&kv_list.geom, p, w.target_kv, 9, 14);
+  if (shared && w.target_kv > 0) kv_list.geom.walk_round = 0;   // pieces count a group's visits downwards
+  rc = launch_build_backward(kv_list, q_list, kv_off, p->num_tasks, BwdFill{(uint8_t *)dk, (uint8_t *)dv, (int64_t)p->num_heads_kv * kHeadDim * 2, p->total_k, shards}, s);
+  if (rc) return rc;
+
   // ---- dQ: one workgroup per (task, block of query rows, kv head).  It runs first: it also leaves the row
   // statistics (lse in the log2 domain, -delta) in the workspace, which the dK/dV kernel reads.
   {
-    const SchedGeom geom = launched_geom(dq_geom(p), p);
-    a.merge_tiles = geom.merge_tiles;
-    const int64_t max_items = dq_max_items(p);
-    rc = launch_build_schedule(0, cu_q, cu_k, p->num_tasks, geom, (int32_t *)(ws + w.sched_q), max_items, s);
-    if (rc) return rc;
-    const int64_t grid = max_items * p->num_heads_kv * kSchedOversubNum / kSchedOversubDen;
+    const int64_t grid = list_grid(p, w.items_q, few_q);
     if (grid > 0x7fffffff) return fail(DISTCA_E_INVALID, "ca_bwd: grid too large");
-    a.sched = (const int32_t *)(ws + w.sched_q);
-    a.zero_row = ws + w.sched_q + sched_zero_row_off(p->num_tasks, max_items);
-    a.tickets = (int32_t *)(ws + w.sched_q + sched_ticket_off(p->num_tasks, max_items));
+    a.merge_tiles = q_list.geom.merge_tiles;
+    a.sched = q_list.ws;
+    a.zero_row = ws + w.sched_q + sched_zero_row_off(p->num_tasks, w.items_q);
+    a.tickets = (int32_t *)(ws + w.sched_q + sched_ticket_off(p->num_tasks, w.items_q));
+    a.cut = q_list.split.cut; a.slot = q_list.split.slot;
     ScopedTimer timer(DISTCA_TIMER_CA_BWD_DQ, s);
-    rc = DISTCA_FN(launch_dq64)(a, grid, s);
+    rc = DISTCA_FN(launch_dq64)(a, grid, few_q, w.target_q > 0 ? split_max_cut(w.blocks_q, w.target_q) : 0, s);
     if (rc) return rc;
   }
   // ---- dK, dV: one workgroup per (task, 256-key block, kv head)
   {
-    const int64_t max_items = max_items_kv;
-    int32_t *list = (int32_t *)(ws + w.sched_kv);
-    if (shared) {
-      rc = launch_build_shared_schedule(cu_q, cu_k, kv_off, p->num_tasks, p->total_k, bwd_shared_geom(p), list, max_items, s);
-      if (rc) return rc;
-      const SharedGroups sg = shared_groups(list, p->num_tasks, max_items);
-      a.grp_first = sg.first; a.grp_tasks = sg.tasks; a.grp_off = sg.off; a.grp_lmax = sg.lmax;
-      if (kv_shards)
-        hipLaunchKernelGGL(fill_gap_rows_shards_kernel, dim3((unsigned)p->num_tasks + 1, 64), dim3(256), 0, s, (uint8_t *)dk,
-                           (uint8_t *)dv, sg.gap_lo, sg.gap_hi, p->total_k, (int64_t)p->num_heads_kv * kHeadDim * 2, shards);
-      else
-        hipLaunchKernelGGL(fill_gap_rows_kernel, dim3((unsigned)p->num_tasks + 1, 16), dim3(256), 0, s, (u32x4 *)dk, (u32x4 *)dv,
-                           sg.gap_lo, sg.gap_hi, p->total_k, (int64_t)p->num_heads_kv * kHeadDim / 8);
-    } else {
-      rc = launch_build_schedule(1, cu_q, cu_k, p->num_tasks, bwd_geom(p), list, max_items, s);
-      if (rc) return rc;
-    }
-    // when the list is sized for pieces of tasks over shared K/V rows but the tasks own their rows, the tighter bound
-    // sizes the grid (a batch of many short documents and one long one would otherwise launch mostly workgroups
-    // that find nothing to do)
-    const int64_t grid_items = alias ? max_items : bwd_key_blocks_own_rows(p) + split;
-    const int64_t grid = grid_items * p->num_heads_kv * kSchedOversubNum / kSchedOversubDen;
+    // items tile stored rows (tasks that own their rows, or groups of tasks that share them); the list may have more room
+    const int64_t grid = list_grid(p, bwd_key_blocks_own_rows(p) + w.target_kv, few_kv);
     if (grid > 0x7fffffff) return fail(DISTCA_E_INVALID, "ca_bwd: grid too large");
-    a.sched = (const int32_t *)(ws + w.sched_kv);
-    a.zero_row = ws + w.sched_kv + sched_zero_row_off(p->num_tasks, max_items);
-    a.tickets = (int32_t *)(ws + w.sched_kv + sched_ticket_off(p->num_tasks, max_items));
+    if (shared) {
+      const SharedGroups sg = shared_groups(kv_list.ws, p->num_tasks, w.items_kv);
+      a.grp_first = sg.first; a.grp_tasks = sg.tasks; a.grp_off = sg.off; a.grp_lmax = sg.lmax;
+    }
+    a.sched = kv_list.ws;
+    a.zero_row = ws + w.sched_kv + sched_zero_row_off(p->num_tasks, w.items_kv);
+    a.tickets = (int32_t *)(ws + w.sched_kv + sched_ticket_off(p->num_tasks, w.items_kv));
+    a.cut = kv_list.split.cut; a.slot = kv_list.split.slot;
     ScopedTimer timer(DISTCA_TIMER_CA_BWD, s);
-    rc = DISTCA_FN(launch_dkdv64)(a, grid, use_acc, shared, s);
+    rc = DISTCA_FN(launch_dkdv64)(a, grid, few_kv, w.target_kv > 0 ? split_max_cut(w.blocks_kv, w.target_kv) : 0, shared, s);
     if (rc) return rc;
   }
-  if (use_acc) {
-    hipLaunchKernelGGL(cvt_elem_kernel, dim3(grid_for(kv_elems / 8)), dim3(256), 0, s, (const float *)(ws + w.dk_acc), (elem_t *)dk, kv_elems / 8);
-    hipLaunchKernelGGL(cvt_elem_kernel, dim3(grid_for(kv_elems / 8)), dim3(256), 0, s, (const float *)(ws + w.dv_acc), (elem_t *)dv, kv_elems / 8);
-  }
-  (void)q_elems;
   return check_launch("ca_bwd");
 }
 }  // namespace distca

@@ -19,8 +19,6 @@
 //
 // Every LDS fragment a wave reads feeds two MFMAs (one per key block of the wave): half the LDS traffic per MFMA of
 // a 32-key wave: with eight waves of 32 keys, two per SIMD, the LDS reads bounded the kernel.
-#include <hip/amd_detail/amd_hip_unsafe_atomics.h>
-
 #include "api_util.h"
 #include "attn_bwd.h"
 #include "attn_cfg.h"
@@ -89,15 +87,80 @@ __device__ __forceinline__ void mfma32_vc(f32x16 &acc, elemx8 a, elemx8 b, const
 
 #define DKDV_SHARED 0
 #define DKDV_SEG 0
+#define DKDV_SPLIT 0
+#define DKDV_NAME ca_bwd_dkdv64_kernel
+#include "attn_bwd_dkdv64_kernel.inc"
+#undef DKDV_SPLIT
+#undef DKDV_NAME
+#define DKDV_SPLIT 1
+#define DKDV_NAME ca_bwd_dkdv64_split_kernel
 #include "attn_bwd_dkdv64_kernel.inc"
 #undef DKDV_SHARED
+#undef DKDV_NAME
 #define DKDV_SHARED 1
+#define DKDV_NAME ca_bwd_dkdv64_shared_split_kernel
 #include "attn_bwd_dkdv64_kernel.inc"
 #undef DKDV_SEG
+#undef DKDV_NAME
 #define DKDV_SEG 1
+#define DKDV_NAME ca_bwd_dkdv64_shards_split_kernel
+#include "attn_bwd_dkdv64_kernel.inc"
+#undef DKDV_SPLIT
+#undef DKDV_NAME
+#define DKDV_SPLIT 0
+#define DKDV_NAME ca_bwd_dkdv64_shards_kernel
+#include "attn_bwd_dkdv64_kernel.inc"
+#undef DKDV_SEG
+#undef DKDV_NAME
+#define DKDV_SEG 0
+#define DKDV_NAME ca_bwd_dkdv64_shared_kernel
 #include "attn_bwd_dkdv64_kernel.inc"
 #undef DKDV_SHARED
 #undef DKDV_SEG
+#undef DKDV_SPLIT
+#undef DKDV_NAME
+
+// Adds up the pieces of the key blocks that were cut, in their order: workgroup (cut block, kv head, an eighth of the
+// accumulators: dK or dV, key half, half of d), a lane holding what it held in the kernels above.  Bound by reading the slots
+// (256 KB a piece).
+__global__ __launch_bounds__(kThreads) void ca_bwd_dkdv64_combine_kernel(BwdArgs a) {
+  if ((int)blockIdx.x >= a.cut[0]) return;
+  const int4 e = reinterpret_cast<const int4 *>(a.cut + 4)[blockIdx.x];
+  const int unit = e.x, pieces = e.z, kvh = blockIdx.y, part = blockIdx.z;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, g = lane >> 5;
+  const f32x4 *first = reinterpret_cast<const f32x4 *>(a.partial + ((int64_t)e.w * a.hkv + kvh) * kDkdvSlotBytes) + part * 8 * kThreads + tid;
+  const int64_t step = a.hkv * (kDkdvSlotBytes / 16);
+  f32x4 o[8] = {};
+  for (int j = 0; j < pieces; ++j) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const f32x4 v = first[j * step + i * kThreads];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[i][r] += v[r];
+    }
+  }
+  const bool is_dv = part >= 4;
+  const int kb = (part >> 1) & 1, db0 = 2 * (part & 1);
+  const int ks = a.grp_off ? a.grp_off[unit] : (a.kv_off ? a.kv_off[unit] : a.cu_k[unit]);
+  const int kmax = a.grp_lmax ? a.grp_lmax[unit] : a.cu_k[unit + 1] - a.cu_k[unit];
+  const int key = e.y * kBN + wave * 64 + 32 * kb + l32;
+  if (key >= kmax) return;
+  elem_t *out = is_dv ? a.dv : a.dk;
+  const int64_t kv_stride = (int64_t)a.hkv * kHeadDim;
+  int64_t row = ks + key;
+  if (a.shards.num_shards > 0) {
+    const int sh = find_shard(a.shards.row_start, a.shards.num_shards, ks + key);
+    out += (is_dv ? a.shards.dv_off[sh] : a.shards.dk_off[sh]) / 2;
+    row -= a.shards.row_start[sh];
+  }
+  out += row * kv_stride + kvh * kHeadDim;
+  const float f = is_dv ? 1.f : a.scale;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int db = db0 + (i >> 2), cq = i & 3;
+    *reinterpret_cast<elemx4 *>(out + 16 * db + 64 * (cq >> 1) + 8 * (cq & 1) + 4 * g) = cvt4(o[i][0] * f, o[i][1] * f, o[i][2] * f, o[i][3] * f);
+  }
+}
 
 }  // namespace
 
@@ -105,25 +168,20 @@ __device__ __forceinline__ void mfma32_vc(f32x16 &acc, elemx8 a, elemx8 b, const
 int dkdv64_lds_bytes() { return kLds; }
 #endif
 
-int DISTCA_FN(launch_dkdv64)(const BwdArgs &a, int64_t grid, bool atomic_sums, bool shared, hipStream_t stream) {
+int DISTCA_FN(launch_dkdv64)(const BwdArgs &a, int64_t grid, bool few, int64_t max_cut, bool shared, hipStream_t stream) {
   if (device_setup_pending(kSlotBwdLds64)) {
-    hipError_t e1 = hipFuncSetAttribute((const void *)ca_bwd_dkdv64_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
-    hipError_t e2 = hipFuncSetAttribute((const void *)ca_bwd_dkdv64_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
-    hipError_t e3 = hipFuncSetAttribute((const void *)ca_bwd_dkdv64_shared_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
-    if (e3 == hipSuccess) e3 = hipFuncSetAttribute((const void *)ca_bwd_dkdv64_shards_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
-    if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess) return fail(DISTCA_E_LAUNCH, "ca_bwd: cannot reserve %d B of LDS", kLds);
+    const void *kernels[] = {(const void *)ca_bwd_dkdv64_kernel,        (const void *)ca_bwd_dkdv64_shared_kernel,       (const void *)ca_bwd_dkdv64_shards_kernel,
+                             (const void *)ca_bwd_dkdv64_split_kernel,  (const void *)ca_bwd_dkdv64_shared_split_kernel, (const void *)ca_bwd_dkdv64_shards_split_kernel};
+    for (const void *kf : kernels)
+      if (hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess) return fail(DISTCA_E_LAUNCH, "ca_bwd: cannot reserve %d B of LDS", kLds);
     device_setup_done(kSlotBwdLds64);
   }
-  if (shared && atomic_sums) return fail(DISTCA_E_INVALID, "ca_bwd: items over groups of tasks are never cut into pieces");
   if (a.shards.num_shards > 0 && !shared) return fail(DISTCA_E_INVALID, "ca_bwd: K/V shards in place need tasks over shared stored rows");
-  if (shared && a.shards.num_shards > 0)
-    hipLaunchKernelGGL(ca_bwd_dkdv64_shards_kernel, dim3((unsigned)grid), dim3(kThreads), kLds, stream, a);
-  else if (shared)
-    hipLaunchKernelGGL(ca_bwd_dkdv64_shared_kernel, dim3((unsigned)grid), dim3(kThreads), kLds, stream, a);
-  else if (atomic_sums)
-    hipLaunchKernelGGL((ca_bwd_dkdv64_kernel<true>), dim3((unsigned)grid), dim3(kThreads), kLds, stream, a);
-  else
-    hipLaunchKernelGGL((ca_bwd_dkdv64_kernel<false>), dim3((unsigned)grid), dim3(kThreads), kLds, stream, a);
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kThreads), kLds, stream, a); };
+  if (a.shards.num_shards > 0) launch(few ? ca_bwd_dkdv64_shards_split_kernel : ca_bwd_dkdv64_shards_kernel);
+  else if (shared) launch(few ? ca_bwd_dkdv64_shared_split_kernel : ca_bwd_dkdv64_shared_kernel);
+  else launch(few ? ca_bwd_dkdv64_split_kernel : ca_bwd_dkdv64_kernel);
+  if (max_cut > 0) hipLaunchKernelGGL(ca_bwd_dkdv64_combine_kernel, dim3((unsigned)max_cut, a.hkv, 8), dim3(kThreads), 0, stream, a);
   return DISTCA_OK;
 }
 

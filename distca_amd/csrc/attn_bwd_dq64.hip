@@ -78,12 +78,14 @@ __device__ __forceinline__ void mfma32_va0(f32x16 &acc, elemx8 a, accop_t b) {
 // SEG: K/V rows are addressed through a table of shards (kv_shards.h) instead of as one dense tensor.
 // MERGE: a work item is several consecutive blocks of a task's query rows (sched.h, fwd_merge), worked off one after the
 // other; otherwise it is one block.
-template <bool SEG, bool MERGE>
+// SPLIT (batches of few blocks): a work item may be a piece of a block, a range of its K/V tiles (sched.h, piece_count), whose dQ
+// goes to a slot; items are taken by workgroup id.
+template <bool SEG, bool MERGE, bool SPLIT>
 __global__ __launch_bounds__(kThreads, 1) void ca_bwd_dq64_kernel(BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int nitems = a.sched[0];
   int item, kvh;
-  if (!take_item(a.tickets, nitems, a.hkv, reinterpret_cast<int32_t *>(lds), item, kvh)) return;
+  if (!take_item<SPLIT>(a.tickets, nitems, a.hkv, reinterpret_cast<int32_t *>(lds), item, kvh)) return;
   int4 it4 = reinterpret_cast<const int4 *>(a.sched + a.sched_items_off)[item];
   it4.x = uniform_int(it4.x);
   it4.y = uniform_int(it4.y);
@@ -99,14 +101,15 @@ __global__ __launch_bounds__(kThreads, 1) void ca_bwd_dq64_kernel(BwdArgs a) {
   const int q0_ = cq[0], q1_ = cq[1], k0_ = ck[0], k1_ = ck[1], ks_ = *kvp;
   const int64_t qs_given_ = *qsp, dq_given_ = *dqp;
   fence();
-  const int q0 = uniform_int(q0_), q1 = uniform_int(q1_), k0 = uniform_int(k0_), k1 = uniform_int(k1_), ks = uniform_int(ks_);
+  const int q0 = uniform_int(q0_), q1 = uniform_int(q1_), k0 = uniform_int(k0_), k1 = uniform_int(k1_);
+  int ks = uniform_int(ks_);
   const int64_t qs_given = uniform_int64(qs_given_), dq_given = uniform_int64(dq_given_);
   const int64_t qs_task = a.qs_task_off ? qs_given : (int64_t)q0 * a.qs_tok_bytes;
   const int64_t dq_task = a.dq_task_off ? dq_given : (int64_t)q0 * a.dq_tok_bytes;
   const int lq = q1 - q0;
-  const int lk = k1 - k0;
+  int lk = k1 - k0;
   const int G = a.group;
-  const int shift = lk - lq;
+  int shift = lk - lq;
 
   const int nrows = lq * G;
   // the blocks of this item
@@ -136,7 +139,19 @@ next_block:
   if (tok_end > lq) tok_end = lq;
   int nvis = a.causal ? tok_end + shift : lk;
   if (nvis > lk) nvis = lk;
-  const int ntiles = nvis > 0 ? (nvis + kKeys - 1) / kKeys : 0;
+  int ntiles = nvis > 0 ? (nvis + kKeys - 1) / kKeys : 0;
+  if constexpr (SPLIT) {
+    // A piece is what a whole block over the keys from its first tile on would be: what counts keys from the start of the prefix is
+    // moved by the tiles before it.  (The list counts keys in units of kFwdKV.)
+    const int w = uniform_int(it4.w);
+    int lo, hi;
+    piece_range((ntiles * kKeys + kFwdKV - 1) / kFwdKV, item_piece(w), item_pieces(w), a.cut ? uniform_int(a.cut[2]) : 0, &lo, &hi);
+    const int end = hi * (kFwdKV / kKeys);
+    ntiles = (end < ntiles ? end : ntiles) - lo * (kFwdKV / kKeys);
+    ks += lo * kFwdKV;
+    lk -= lo * kFwdKV;
+    shift -= lo * kFwdKV;
+  }
 
   const uint32_t lds0 = (uint32_t)(uintptr_t)(DISTCA_LDS uint8_t *)lds;
   auto div_group = [&](int n) { return a.group_magic ? (int)__umulhi((uint32_t)n, a.group_magic) : n; };
@@ -148,7 +163,8 @@ next_block:
   const elem_t *kbase = a.k + (SEG ? 0 : (int64_t)ks * kv_stride) + kvh * kHeadDim;
   const elem_t *vbase = a.v + (SEG ? 0 : (int64_t)ks * kv_stride) + kvh * kHeadDim;
   ShardCursor cur;  // SEG: the shard that holds the rows of the tile requested next
-  if constexpr (SEG) cur.open(a.shards, a.shards.task_shard[task]);
+  if constexpr (SEG)
+    cur.open(a.shards, SPLIT ? find_shard_wave(a.shards.row_start, a.shards.num_shards, ks) : a.shards.task_shard[task]);
   uint32_t voff[2];
 #pragma unroll
   for (int ii = 0; ii < 2; ++ii) {
@@ -532,6 +548,21 @@ next_block:
       a.dscaled_w[so] = ndl[m][0];  // -delta: the start value of the dP accumulators in the dK/dV kernel
     }
   }
+  if constexpr (SPLIT) {
+    // a piece's dQ as its accumulators lie, 16 bytes of a lane beside those of the next
+    const int slot = a.slot ? uniform_int(a.slot[2 * item]) : -1;
+    if (slot >= 0) {
+      f32x4 *op = reinterpret_cast<f32x4 *>(a.partial + ((int64_t)slot * a.hkv + kvh) * kDqSlotBytes) + wave * 32 * 64 + lane;
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+#pragma unroll
+          for (int cq = 0; cq < 4; ++cq)
+            op[(16 * m + 4 * db + cq) * 64] = f32x4{dqacc[m][db][4 * cq], dqacc[m][db][4 * cq + 1], dqacc[m][db][4 * cq + 2], dqacc[m][db][4 * cq + 3]};
+      return;
+    }
+  }
   {
     const uint32_t out_b = MERGE ? lds0 + wave * kStageBytes : stg;
 #pragma unroll
@@ -566,12 +597,48 @@ next_block:
   }
 }
 
+// Adds up the pieces of the blocks that were cut, in their order: workgroup (cut block, kv head, quarter of d), a lane holding
+// what it held in the kernel above.
+__global__ __launch_bounds__(kThreads) void ca_bwd_dq64_combine_kernel(BwdArgs a) {
+  if ((int)blockIdx.x >= a.cut[0]) return;
+  const int4 e = reinterpret_cast<const int4 *>(a.cut + 4)[blockIdx.x];
+  const int task = e.x, pieces = e.z, kvh = blockIdx.y, db = blockIdx.z, G = a.group;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, g = lane >> 5;
+  const int q0 = a.cu_q[task], nrows = (a.cu_q[task + 1] - q0) * G;
+  const uint8_t *first = a.partial + ((int64_t)e.w * a.hkv + kvh) * kDqSlotBytes;
+  f32x4 o[2][4] = {};
+  for (int j = 0; j < pieces; ++j) {
+    const f32x4 *op = reinterpret_cast<const f32x4 *>(first + (int64_t)j * a.hkv * kDqSlotBytes) + (wave * 32 + 4 * db) * 64 + lane;
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int cq = 0; cq < 4; ++cq) {
+        const f32x4 v = op[(16 * m + cq) * 64];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[m][cq][r] += v[r];
+      }
+  }
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const int row = e.y * kRowsWg + (wave * 2 + m) * 32 + l32;
+    if (row >= nrows) continue;
+    const int tok = row / G, hg = row - tok * G;
+    elem_t *op = reinterpret_cast<elem_t *>(reinterpret_cast<uint8_t *>(a.dq) + (a.dq_task_off ? a.dq_task_off[task] : (int64_t)q0 * a.dq_tok_bytes) +
+                                            (int64_t)tok * a.dq_tok_bytes) + (kvh * G + hg) * kHeadDim;
+#pragma unroll
+    for (int cq = 0; cq < 4; ++cq)
+      *reinterpret_cast<elemx4 *>(op + 16 * db + 64 * (cq >> 1) + 8 * (cq & 1) + 4 * g) =
+          cvt4(o[m][cq][0] * a.scale, o[m][cq][1] * a.scale, o[m][cq][2] * a.scale, o[m][cq][3] * a.scale);
+  }
+}
+
 }  // namespace
 
-int DISTCA_FN(launch_dq64)(const BwdArgs &a, int64_t grid, hipStream_t stream) {
+int DISTCA_FN(launch_dq64)(const BwdArgs &a, int64_t grid, bool few, int64_t max_cut, hipStream_t stream) {
   if (device_setup_pending(kSlotBwdDq64)) {
-    const void *kernels[] = {(const void *)ca_bwd_dq64_kernel<false, false>, (const void *)ca_bwd_dq64_kernel<true, false>,
-                             (const void *)ca_bwd_dq64_kernel<false, true>, (const void *)ca_bwd_dq64_kernel<true, true>};
+    const void *kernels[] = {(const void *)ca_bwd_dq64_kernel<false, false, false>, (const void *)ca_bwd_dq64_kernel<true, false, false>,
+                             (const void *)ca_bwd_dq64_kernel<false, true, false>,  (const void *)ca_bwd_dq64_kernel<true, true, false>,
+                             (const void *)ca_bwd_dq64_kernel<false, false, true>,  (const void *)ca_bwd_dq64_kernel<true, false, true>};
     for (const void *kf : kernels) {
       hipError_t e = hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
       if (e != hipSuccess) return fail(DISTCA_E_LAUNCH, "ca_bwd: cannot reserve %d B of LDS: %s", kLds, hipGetErrorString(e));
@@ -579,11 +646,12 @@ int DISTCA_FN(launch_dq64)(const BwdArgs &a, int64_t grid, hipStream_t stream) {
     device_setup_done(kSlotBwdDq64);
   }
   const dim3 g((unsigned)grid), b(kThreads);
-  const bool seg = a.shards.num_shards > 0, merge = a.merge_tiles > 0;
-  if (seg && merge) hipLaunchKernelGGL((ca_bwd_dq64_kernel<true, true>), g, b, kLds, stream, a);
-  else if (seg) hipLaunchKernelGGL((ca_bwd_dq64_kernel<true, false>), g, b, kLds, stream, a);
-  else if (merge) hipLaunchKernelGGL((ca_bwd_dq64_kernel<false, true>), g, b, kLds, stream, a);
-  else hipLaunchKernelGGL((ca_bwd_dq64_kernel<false, false>), g, b, kLds, stream, a);
+  const bool seg = a.shards.num_shards > 0;
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, b, kLds, stream, a); };
+  if (few) launch(seg ? ca_bwd_dq64_kernel<true, false, true> : ca_bwd_dq64_kernel<false, false, true>);
+  else if (a.merge_tiles > 0) launch(seg ? ca_bwd_dq64_kernel<true, true, false> : ca_bwd_dq64_kernel<false, true, false>);
+  else launch(seg ? ca_bwd_dq64_kernel<true, false, false> : ca_bwd_dq64_kernel<false, false, false>);
+  if (max_cut > 0) hipLaunchKernelGGL(ca_bwd_dq64_combine_kernel, dim3((unsigned)max_cut, a.hkv, 4), b, 0, stream, a);
   return DISTCA_OK;
 }
 

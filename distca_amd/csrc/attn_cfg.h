@@ -4,6 +4,7 @@
 #include <stdlib.h>
 
 #include "api_util.h"
+#include "kv_shards.h"
 #include "sched.h"
 
 namespace distca {
@@ -76,6 +77,8 @@ inline SchedGeom launched_geom(SchedGeom g, const distca_ca_params *p) {
 inline SchedGeom fwd_geom(const distca_ca_params *p) {
   SchedGeom g;
   g.split_target = 0;
+  g.min_piece = kMinPiece;
+  g.units_per_head = g.item_cost = g.piece_extra = 0;
   g.walk_round = 0;
   g.merge_tiles = merge_short_tasks(p) ? kMergeTilesFwd : 0;
   g.rows_per_block = kFwdRows;
@@ -87,8 +90,9 @@ inline SchedGeom fwd_geom(const distca_ca_params *p) {
   return g;
 }
 // Key blocks are cut into pieces (sched.h) when the batch has so few of them that they could not occupy the
-// device twice over, unless the caller asked for a deterministic backward (the pieces' dK/dV are added up with
-// float atomics).  Returns the number of pieces to aim for per kv head, 0 = no cutting.
+// device twice over.  Returns the number of pieces to aim for per kv head, 0 = no cutting.  A caller that asks for a
+// deterministic backward and brings the smallest workspace gets whole blocks (the same bits either way: pieces are added up in
+// their order).
 constexpr int kSplitPiecesPerCU = 2;
 // Upper bounds, from host-known sizes, of the number of key blocks = sum over tasks of ceil(Lk / kBwdKV).
 // When every task has its own K/V rows the Lk add up to total_k at most; when tasks read shared rows
@@ -99,12 +103,53 @@ inline int64_t bwd_key_blocks_bound(const distca_ca_params *p) {
   const int64_t by_max = ((int64_t)p->max_seqlen_k / kBwdKV + 1) * p->num_tasks + 1;
   return by_total > by_max ? by_total : by_max;
 }
-inline int32_t bwd_split_target(const distca_ca_params *p) {
-  if (p->deterministic) return 0;
-  const int cus = num_compute_units();  // of the current device; 256 when there is none (the host mirror on a CPU box)
-  if (bwd_key_blocks_own_rows(p) * p->num_heads_kv >= 2 * cus) return 0;
-  const int32_t t = kSplitPiecesPerCU * cus / p->num_heads_kv;
-  return t > 0 ? t : 1;
+inline bool few_key_blocks(const distca_ca_params *p, int per_cu) {
+  // (compute units of the current device; 256 when there is none, the host mirror on a CPU box)
+  return bwd_key_blocks_own_rows(p) * p->num_heads_kv < (int64_t)per_cu * num_compute_units();
+}
+constexpr int kSplitFewPerCU = 2, kSplitPreferredPerCU = 8;
+// (`per_cu`: below how many blocks per compute unit)
+inline int32_t bwd_split_pieces(const distca_ca_params *p, int per_cu) {
+  const int cus = num_compute_units();
+  if (!few_key_blocks(p, per_cu)) return 0;
+  const int64_t t = kSplitPiecesPerCU * cus / p->num_heads_kv;
+  // (no more than there can be: every block in pieces of kMinPiece)
+  const int64_t rows = (int64_t)p->total_q * (p->num_heads_q / p->num_heads_kv);
+  const int64_t all = bwd_key_blocks_bound(p) * ((rows / kBwdRows + p->num_tasks + kMinPiece) / kMinPiece);
+  return (int32_t)(t < 1 ? 1 : (t < all ? t : all));
+}
+inline int32_t bwd_split_target(const distca_ca_params *p) { return p->deterministic ? 0 : bwd_split_pieces(p, kSplitFewPerCU); }
+// Blocks of query rows are cut into pieces of consecutive KV tiles when the batch has so few of them that the longest one
+// could bound the launch: fewer than kSplitMaxBlocksPerCU blocks per compute unit (above that longest-first dispatch evens
+// them out), and a prefix long enough for two pieces.  Returns the number of pieces to aim for per kv head, 0 = no cutting.
+// It depends only on sizes that do not change with how K/V are stored, so that a tick gives the same bits in every form.
+constexpr int kSplitRowPiecesPerCU = 2;
+constexpr int kSplitMaxBlocksPerCU = 8;
+inline bool few_row_blocks(const distca_ca_params *p) {
+  return (int64_t)p->total_q * p->num_heads_q < (int64_t)kSplitMaxBlocksPerCU * kFwdRows * num_compute_units();
+}
+inline int32_t row_split_target(const distca_ca_params *p, int64_t max_blocks) {
+  const int64_t cus = num_compute_units();
+  if (!few_row_blocks(p)) return 0;
+  const int64_t most = ((int64_t)p->max_seqlen_k / kFwdKV + 1 + kMinPiece - 1) / kMinPiece;   // pieces of the longest block
+  if (most < 2) return 0;
+  const int64_t t = kSplitRowPiecesPerCU * cus / p->num_heads_kv, all = max_blocks * most;
+  return (int32_t)(t < 1 ? 1 : (t < all ? t : all));
+}
+// Workgroups for a list: 5/4 of its places, drawing tickets (sched.h, take_item), or, where the items are few, one each.
+inline int64_t list_grid(const distca_ca_params *p, int64_t items, bool few) {
+  return few ? items * p->num_heads_kv : items * p->num_heads_kv * kSchedOversubNum / kSchedOversubDen;
+}
+// A list of which only what is worth it is cut (sched.h, worth_cutting).  item_cost and piece_extra in the list's cost unit: an
+// item's ticket, first loads and last stores take 11 us against 1.7 us per forward tile (dQ 15 against 2.4, dK/dV 14 against 1.5
+// per query block), and a piece's fp32 result written and read again about as long as its bytes take at the unit's share of the memory rate.
+inline void cut_where_worth(SchedGeom *g, const distca_ca_params *p, int32_t target, int32_t item_cost, int32_t piece_extra) {
+  const int32_t units = num_compute_units() / p->num_heads_kv;
+  g->split_target = target;
+  g->merge_tiles = 0;
+  g->units_per_head = units > 0 ? units : 1;
+  g->item_cost = item_cost;
+  g->piece_extra = piece_extra;
 }
 inline SchedGeom dq_geom(const distca_ca_params *p) {
   SchedGeom g = fwd_geom(p);
@@ -121,6 +166,8 @@ inline SchedGeom bwd_geom(const distca_ca_params *p) {
   g.causal = p->causal != 0;
   g.cost_shift = pick_cost_shift((int64_t)p->max_seqlen_q * g.group / kBwdRows + 1);
   g.split_target = bwd_split_target(p);
+  g.min_piece = kMinPiece;
+  g.units_per_head = g.item_cost = g.piece_extra = 0;
   // one round of the dK/dV list per kv head: as many items as compute units serve that head (sched.h, kWalkUp)
   g.walk_round = num_compute_units() / p->num_heads_kv > 0 ? num_compute_units() / p->num_heads_kv : 1;
   return g;
@@ -149,12 +196,25 @@ inline SchedGeom bwd_shared_geom(const distca_ca_params *p) {
   return g;
 }
 
-int launch_build_schedule(int kind, const int32_t *cu_q, const int32_t *cu_k, int32_t num_tasks, const SchedGeom &g,
-                          int32_t *ws, int64_t max_items, hipStream_t stream);
-// The dK/dV list over groups of tasks that share stored K/V rows (sched.h, SharedGroups); the region behind `ws` is
-// sched_shared_region_bytes long.
-int launch_build_shared_schedule(const int32_t *cu_q, const int32_t *cu_k, const int32_t *kv_off, int32_t num_tasks, int32_t total_k,
-                                 const SchedGeom &g, int32_t *ws, int64_t max_items, hipStream_t stream);
+// One list to build: for a batch with these bounds, into region `ws`.
+struct ListJob {
+  const int32_t *cu_q, *cu_k;
+  SchedGeom geom;
+  int32_t *ws;
+  int64_t max_items;
+  SplitTables split;
+};
+// The dk / dv rows a backward clears: rows that no task reads.
+struct BwdFill {
+  uint8_t *dk, *dv;
+  int64_t row_bytes;
+  int32_t total_k;
+  KvShards shards;
+};
+int launch_build_forward(const ListJob &j, int32_t num_tasks, hipStream_t stream);
+// kv_off: null, or the tasks share stored K/V rows and the dK/dV list is made over groups of them (sched.h, SharedGroups; its region
+// is sched_shared_region_bytes long)
+int launch_build_backward(const ListJob &kv, const ListJob &q, const int32_t *kv_off, int32_t num_tasks, const BwdFill &fill, hipStream_t stream);
 
 inline int64_t align_up(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 

@@ -61,17 +61,39 @@ struct FwdArgs {
   int32_t merge_tiles;   // MERGE kernels: the list's merge_tiles (sched.h)
   int32_t lse_in_token;  // 1: lse of (token, head) as fp32 at token + hq * 256 + h * 4 (the [out | lse] reply), 0: lse[h][token]
   KvShards shards;       // SEG kernels: k and v are the bases of a buffer that holds the stored rows shard by shard
+  const int32_t *cut, *slot;  // SPLIT kernels: the tables of a list with cut blocks (sched.h, SplitTables)
+  uint8_t *partial;           // and the slots
 };
+
+// A piece's slot: O before normalisation as the accumulators lie, 16 bytes of a lane beside those of the next (a store of 1 KB
+// per instruction), then (m, l) per row.
+constexpr int64_t kFwdSlotStats = (int64_t)kFwdRows * kHeadDim * 4;
+constexpr int64_t kFwdSlotBytes = kFwdSlotStats + kFwdRows * 8;
+
+// Where lse of (token, head) goes, and, in the [out | lse] reply, the zeros behind the last head's.
+__device__ __forceinline__ void store_lse(const FwdArgs &a, uint8_t *otok, int head, int64_t row, float lse) {
+  if (a.lse_in_token) {
+    float *lp = reinterpret_cast<float *>(otok + (int64_t)a.hq * kHeadDim * 2);
+    lp[head] = lse;
+    if (head == a.hq - 1) {  // zero the padding that rounds the token up to 16 bytes
+      for (int64_t b = (int64_t)a.hq * (kHeadDim * 2 + 4); b < (((int64_t)a.hq * (kHeadDim * 2 + 4) + 15) & ~(int64_t)15); b += 4) *reinterpret_cast<float *>(otok + b) = 0.f;
+    }
+  } else {
+    a.lse[(int64_t)head * a.total_q + row] = lse;
+  }
+}
 
 // SEG: K/V rows are addressed through a table of shards (kv_shards.h) instead of as one dense tensor.
 // MERGE: a work item is several consecutive blocks of a task's query rows (sched.h, fwd_merge), worked off one after the
 // other; otherwise it is one block.
-template <int MSUB, bool SEG, bool MERGE>
+// SPLIT (batches of few blocks): a work item may be a piece of a block, a range of its KV tiles (sched.h, piece_count), whose result
+// goes to a slot; items are taken by workgroup id.
+template <int MSUB, bool SEG, bool MERGE, bool SPLIT>
 __global__ __launch_bounds__(kFwdWaves * 64, (MSUB == 1 && kFwdWaves == 4 ? 2 : 1)) void ca_fwd_kernel(FwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int nitems = a.sched[0];
   int item, kvh;
-  if (!take_item(a.tickets, nitems, a.hkv, reinterpret_cast<int32_t *>(lds), item, kvh)) return;
+  if (!take_item<SPLIT>(a.tickets, nitems, a.hkv, reinterpret_cast<int32_t *>(lds), item, kvh)) return;
   // (the item's fields and the task's bounds are moved to scalar registers as they are read: what derives from them,
   // base pointers, loop limits and tile addresses, is then scalar arithmetic)
   int4 it = reinterpret_cast<const int4 *>(a.sched + a.sched_items_off)[item];
@@ -81,10 +103,10 @@ __global__ __launch_bounds__(kFwdWaves * 64, (MSUB == 1 && kFwdWaves == 4 ? 2 : 
 
   const int q0 = uniform_int(a.cu_q[task]);
   const int lq = uniform_int(a.cu_q[task + 1]) - q0;
-  const int lk = uniform_int(a.cu_k[task + 1]) - uniform_int(a.cu_k[task]);
-  const int ks = uniform_int(a.kv_off ? a.kv_off[task] : a.cu_k[task]);
+  int lk = uniform_int(a.cu_k[task + 1]) - uniform_int(a.cu_k[task]);
+  int ks = uniform_int(a.kv_off ? a.kv_off[task] : a.cu_k[task]);
   const int G = a.group;
-  const int shift = lk - lq;
+  int shift = lk - lq;
 
   constexpr int kRows = kFwdWaves * 32 * MSUB;
   const int nrows = lq * G;
@@ -119,7 +141,18 @@ next_block:
   if (tok_end > lq) tok_end = lq;
   int nvis = a.causal ? tok_end + shift : lk;
   if (nvis > lk) nvis = lk;
-  const int ntiles = nvis > 0 ? (nvis + kFwdKV - 1) / kFwdKV : 0;
+  int ntiles = nvis > 0 ? (nvis + kFwdKV - 1) / kFwdKV : 0;
+  if constexpr (SPLIT) {
+    // A piece is what a whole block over the keys from its first tile on would be: what counts keys from the start of the prefix is
+    // moved by the tiles before it, and below nothing knows of it.  (Carrying the first tile into the loops cost 5 % of a block's time.)
+    const int w = uniform_int(it.w);
+    int tile0, tile1;
+    piece_range(ntiles, item_piece(w), item_pieces(w), a.cut ? uniform_int(a.cut[2]) : 0, &tile0, &tile1);
+    ntiles = tile1 - tile0;
+    ks += tile0 * kFwdKV;
+    lk -= tile0 * kFwdKV;
+    shift -= tile0 * kFwdKV;
+  }
 
   // ---- per-lane rows
   const uint8_t *qbytes = reinterpret_cast<const uint8_t *>(a.q) + uniform_int64(a.q_task_off ? a.q_task_off[task] : (int64_t)q0 * a.q_tok_bytes);
@@ -174,7 +207,7 @@ next_block:
   // SEG: the shards that hold the rows of the K tile and of the V tile requested next (the K requests run a tile ahead)
   ShardCursor kcur, vcur;
   if constexpr (SEG) {
-    kcur.open(a.shards, a.shards.task_shard[task]);
+    kcur.open(a.shards, SPLIT ? find_shard_wave(a.shards.row_start, a.shards.num_shards, ks) : a.shards.task_shard[task]);
     vcur = kcur;
   }
   // a wave brings kRowsW rows of a K tile or of a V tile, four rows per instruction
@@ -481,6 +514,22 @@ next_block:
     if (more) request_next_block();
   }
 
+  if constexpr (SPLIT) {
+    static_assert(MSUB == 1, "layout of a slot");
+    const int slot = a.slot ? uniform_int(a.slot[2 * item]) : -1;
+    if (slot >= 0) {
+      uint8_t *at = a.partial + ((int64_t)slot * a.hkv + kvh) * kFwdSlotBytes;
+      f32x4 *op = reinterpret_cast<f32x4 *>(at) + wave * 16 * 64 + lane;
+#pragma unroll
+      for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int cq = 0; cq < 4; ++cq) op[(4 * db + cq) * 64] = f32x4{oacc[0][db][4 * cq], oacc[0][db][4 * cq + 1], oacc[0][db][4 * cq + 2], oacc[0][db][4 * cq + 3]};
+      const float l = pair_sum(l_run[0]);
+      if (g == 0) reinterpret_cast<f32x2 *>(at + kFwdSlotStats)[wave * 32 + l32] = f32x2{m_run[0], l};
+      return;
+    }
+  }
+
   // ---- epilogue: normalise, write O (bf16) and LSE (fp32, natural log)
 #pragma unroll
   for (int m = 0; m < MSUB; ++m) {
@@ -502,22 +551,70 @@ next_block:
         }
       if (g == 0) {
         const float lse = l_tot > 0.f ? (m_run[m] * c + fast_log2(l_tot)) * kLn2 : -INFINITY;
-        const int head = kvh * G + hg;
-        if (a.lse_in_token) {
-          float *lp = reinterpret_cast<float *>(otok + (int64_t)a.hq * kHeadDim * 2);
-          lp[head] = lse;
-          if (head == a.hq - 1) {  // zero the padding that rounds the token up to 16 bytes
-            for (int64_t b = (int64_t)a.hq * (kHeadDim * 2 + 4); b < (((int64_t)a.hq * (kHeadDim * 2 + 4) + 15) & ~(int64_t)15); b += 4) *reinterpret_cast<float *>(otok + b) = 0.f;
-          }
-        } else {
-          a.lse[(int64_t)head * a.total_q + q0 + tok[m]] = lse;
-        }
+        store_lse(a, otok, kvh * G + hg, q0 + tok[m], lse);
       }
     }
   }
   if constexpr (MERGE) {
     if (++mblk < mb_end) goto next_block;
   }
+}
+
+// Adds up the pieces of the blocks that were cut: workgroup (cut block, kv head, quarter of d), a lane holding what it held in
+// the kernel above.  Pieces are taken in their order.  Bound by reading the slots (128 KB a piece), which the quarters
+// spread over four times as many compute units.
+__global__ __launch_bounds__(kFwdWaves * 64) void ca_fwd_combine_kernel(FwdArgs a) {
+  if ((int)blockIdx.x >= a.cut[0]) return;
+  const int4 e = reinterpret_cast<const int4 *>(a.cut + 4)[blockIdx.x];
+  const int task = e.x, pieces = e.z, kvh = blockIdx.y, db = blockIdx.z, G = a.group;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, g = lane >> 5;
+  const int q0 = a.cu_q[task], nrows = (a.cu_q[task + 1] - q0) * G;
+  const int row = e.y * kFwdRows + wave * 32 + l32;
+  const float c = a.scale * kLog2e;
+  const uint8_t *first = a.partial + ((int64_t)e.w * a.hkv + kvh) * kFwdSlotBytes;
+  const int64_t step = a.hkv * kFwdSlotBytes;
+  auto stat = [&](int j) { return reinterpret_cast<const f32x2 *>(first + j * step + kFwdSlotStats)[wave * 32 + l32]; };
+  float m = -INFINITY;
+  for (int j = 0; j < pieces; ++j) m = __builtin_fmaxf(m, stat(j)[0]);
+  f32x4 o[4] = {};
+  float l = 0.f;
+  for (int j = 0; j < pieces; ++j) {
+    const f32x2 s = stat(j);
+    const float w = s[0] == -INFINITY ? 0.f : fast_exp2((s[0] - m) * c);
+    l += w * s[1];
+    const f32x4 *op = reinterpret_cast<const f32x4 *>(first + j * step) + (wave * 16 + 4 * db) * 64 + lane;
+#pragma unroll
+    for (int cq = 0; cq < 4; ++cq) {
+      const f32x4 v = op[cq * 64];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[cq][r] = __builtin_fmaf(w, v[r], o[cq][r]);
+    }
+  }
+  if (row >= nrows) return;
+  const int tok = row / G, hg = row - tok * G;
+  uint8_t *otok = reinterpret_cast<uint8_t *>(a.out) + (a.out_task_off ? a.out_task_off[task] : (int64_t)q0 * a.out_tok_bytes) + (int64_t)tok * a.out_tok_bytes;
+  elem_t *op = reinterpret_cast<elem_t *>(otok) + (kvh * G + hg) * kHeadDim;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+  for (int cq = 0; cq < 4; ++cq)
+    *reinterpret_cast<elemx4 *>(op + 16 * db + 64 * (cq >> 1) + 8 * (cq & 1) + 4 * g) = cvt4(o[cq][0] * inv, o[cq][1] * inv, o[cq][2] * inv, o[cq][3] * inv);
+  if (db == 0 && g == 0) store_lse(a, otok, kvh * G + hg, q0 + tok, l > 0.f ? (m * c + fast_log2(l)) * kLn2 : -INFINITY);
+}
+
+// How a forward is laid out in its workspace: the list, and, when blocks are cut, the tables and slots of the pieces.
+struct FwdLayout {
+  int64_t max_blocks, max_items, tables, slots, total;
+  int32_t target;
+};
+FwdLayout fwd_layout(const distca_ca_params *p, bool split) {
+  FwdLayout w;
+  w.max_blocks = fwd_max_items(p);
+  w.target = split ? row_split_target(p, w.max_blocks) : 0;
+  w.max_items = w.max_blocks + w.target;
+  w.tables = align_up(sched_region_bytes(p->num_tasks, w.max_items), 256);
+  w.slots = w.tables + split_tables_bytes(w.max_blocks, w.target, w.max_items);
+  w.total = w.target > 0 ? w.slots + split_max_slots(w.max_blocks, w.target) * p->num_heads_kv * kFwdSlotBytes : sched_region_bytes(p->num_tasks, w.max_items);
+  return w;
 }
 
 }  // namespace
@@ -559,7 +656,13 @@ extern "C" int64_t distca_ca_fwd_workspace_bytes(const distca_ca_params *p) {
   if (!p) return fail(DISTCA_E_INVALID, "fwd_workspace_bytes: null params");
   int rc = validate_params(p);
   if (rc) return rc;
-  return sched_region_bytes(p->num_tasks, fwd_max_items(p));
+  return fwd_layout(p, false).total;
+}
+extern "C" int64_t distca_ca_fwd_workspace_preferred_bytes(const distca_ca_params *p) {
+  if (!p) return fail(DISTCA_E_INVALID, "fwd_workspace_preferred_bytes: null params");
+  int rc = validate_params(p);
+  if (rc) return rc;
+  return fwd_layout(p, true).total;
 }
 
 extern "C" int distca_ca_fwd_tokens(const void *q_base, const int64_t *q_task_off, int64_t q_tok_bytes, const void *k,
@@ -621,7 +724,7 @@ extern "C" int distca_ca_fwd_noalloc(const void *q, const void *k, const void *v
   void *ws = nullptr;
   const int rc = noalloc_scratch(&ws);
   if (rc) return rc;
-  return distca_ca_fwd(q, k, v, out, lse, cu_q, cu_k, kv_off, p, ws, kNoAllocScratchBytes, stream);
+  return distca_ca_fwd(q, k, v, out, lse, cu_q, cu_k, kv_off, p, ws, need, stream);
 }
 
 #endif  // !DISTCA_F16
@@ -650,9 +753,14 @@ int DISTCA_FN(run_fwd_tokens)(const void *q_base, const int64_t *q_task_off, int
   if (!workspace || workspace_bytes < need) return fail(DISTCA_E_WORKSPACE, "ca_fwd: workspace %lld B < required %lld B", (long long)workspace_bytes, (long long)need);
   if (!aligned16(workspace)) return fail(DISTCA_E_INVALID, "ca_fwd: workspace must be 16-byte aligned");
   hipStream_t s = (hipStream_t)stream;
-  const SchedGeom geom = launched_geom(fwd_geom(p), p);
-  const int64_t max_items = fwd_max_items(p);
-  rc = launch_build_schedule(0, cu_q, cu_k, p->num_tasks, geom, (int32_t *)workspace, max_items, s);
+  SchedGeom geom = launched_geom(fwd_geom(p), p);
+  FwdLayout lay = fwd_layout(p, true);
+  if (lay.target > 0 && workspace_bytes < lay.total) lay = fwd_layout(p, false);   // no room for pieces
+  const int64_t max_items = lay.max_items;
+  const bool split = lay.target > 0, few = few_row_blocks(p);
+  if (split) cut_where_worth(&geom, p, lay.target, 6, 4);
+  const SplitTables tables = split ? split_tables((uint8_t *)workspace + lay.tables, lay.max_blocks, lay.target) : SplitTables{};
+  rc = launch_build_forward(ListJob{cu_q, cu_k, geom, (int32_t *)workspace, max_items, tables}, p->num_tasks, s);
   if (rc) return rc;
 
   FwdArgs a;
@@ -668,16 +776,18 @@ int DISTCA_FN(run_fwd_tokens)(const void *q_base, const int64_t *q_task_off, int
   a.q_task_off = q_task_off; a.out_task_off = out_task_off; a.q_tok_bytes = q_tok_bytes; a.out_tok_bytes = out_tok_bytes;
   a.lse_in_token = lse ? 0 : 1;
   a.merge_tiles = geom.merge_tiles;
+  a.cut = tables.cut; a.slot = tables.slot; a.partial = (uint8_t *)workspace + lay.slots;
   a.shards = KvShards{};
   if (kv_shards) {
     rc = make_kv_shards(kv_shards, kv_off, false, &a.shards);
     if (rc) return rc;
   }
-  const int64_t grid = max_items * p->num_heads_kv * kSchedOversubNum / kSchedOversubDen;
+  const int64_t grid = list_grid(p, max_items, few);
   if (grid > 0x7fffffff) return fail(DISTCA_E_INVALID, "ca_fwd: grid too large");
   if (device_setup_pending(kSlotFwdLds)) {
-    const void *kernels[] = {(const void *)ca_fwd_kernel<kFwdMsub, false, false>, (const void *)ca_fwd_kernel<kFwdMsub, true, false>,
-                             (const void *)ca_fwd_kernel<kFwdMsub, false, true>, (const void *)ca_fwd_kernel<kFwdMsub, true, true>};
+    const void *kernels[] = {(const void *)ca_fwd_kernel<kFwdMsub, false, false, false>, (const void *)ca_fwd_kernel<kFwdMsub, true, false, false>,
+                             (const void *)ca_fwd_kernel<kFwdMsub, false, true, false>,  (const void *)ca_fwd_kernel<kFwdMsub, true, true, false>,
+                             (const void *)ca_fwd_kernel<kFwdMsub, false, false, true>,  (const void *)ca_fwd_kernel<kFwdMsub, true, false, true>};
     for (const void *kf : kernels) {
       hipError_t e = hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, kFwdLds);
       if (e != hipSuccess) return fail(DISTCA_E_LAUNCH, "ca_fwd: cannot reserve %d B of LDS: %s", kFwdLds, hipGetErrorString(e));
@@ -687,11 +797,11 @@ int DISTCA_FN(run_fwd_tokens)(const void *q_base, const int64_t *q_task_off, int
   {
     ScopedTimer timer(DISTCA_TIMER_CA_FWD, s);
     const dim3 g((unsigned)grid), b(kFwdWaves * 64);
-    const bool merge = geom.merge_tiles > 0;
-    if (kv_shards && merge) hipLaunchKernelGGL((ca_fwd_kernel<kFwdMsub, true, true>), g, b, kFwdLds, s, a);
-    else if (kv_shards) hipLaunchKernelGGL((ca_fwd_kernel<kFwdMsub, true, false>), g, b, kFwdLds, s, a);
-    else if (merge) hipLaunchKernelGGL((ca_fwd_kernel<kFwdMsub, false, true>), g, b, kFwdLds, s, a);
-    else hipLaunchKernelGGL((ca_fwd_kernel<kFwdMsub, false, false>), g, b, kFwdLds, s, a);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, b, kFwdLds, s, a); };
+    if (few) launch(kv_shards ? ca_fwd_kernel<kFwdMsub, true, false, true> : ca_fwd_kernel<kFwdMsub, false, false, true>);
+    else if (geom.merge_tiles > 0) launch(kv_shards ? ca_fwd_kernel<kFwdMsub, true, true, false> : ca_fwd_kernel<kFwdMsub, false, true, false>);
+    else launch(kv_shards ? ca_fwd_kernel<kFwdMsub, true, false, false> : ca_fwd_kernel<kFwdMsub, false, false, false>);
+    if (split) hipLaunchKernelGGL(ca_fwd_combine_kernel, dim3((unsigned)split_max_cut(lay.max_blocks, lay.target), p->num_heads_kv, 4), b, 0, s, a);
   }
   return check_launch("ca_fwd");
 }

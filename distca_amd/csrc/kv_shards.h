@@ -31,6 +31,16 @@ __device__ __forceinline__ int find_shard(const int32_t *row_start, int n, int r
   return lo;
 }
 
+// The same by a whole wave, for a row that is the same in every lane: 64 shards per look instead of a chain of loads.
+__device__ __forceinline__ int find_shard_wave(const int32_t *row_start, int n, int r) {
+  int before = 0;
+  for (int base = 0; base < n; base += 64) {
+    const int i = base + (int)(threadIdx.x & 63);
+    before += __popcll(__ballot(i < n && row_start[i] <= r));
+  }
+  return before > 0 ? before - 1 : 0;
+}
+
 // The shard that holds the rows a wave is about to request, carried along a walk over ascending rows (all of it
 // wave-uniform: scalar registers and scalar loads).
 // The values are forced into scalar registers as they are loaded (the loads are vector loads from a uniform address): the

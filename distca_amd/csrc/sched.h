@@ -11,6 +11,7 @@
 // The reference itself has no such component on the GPU: flash-attn launches a static
 // (m-block, batch, head) grid sized by max_seqlen_q.
 #pragma once
+#include <math.h>
 #include <stdint.h>
 
 #if defined(__HIPCC__)
@@ -22,13 +23,16 @@
 namespace distca {
 
 struct SchedGeom {
-  int32_t rows_per_block;  // flattened (token, head-in-group) query rows per m-block
-  int32_t kv_per_block;    // keys per KV block
+  int32_t rows_per_block;  // flattened (token, head-in-group) query rows per m-block, a power of two
+  int32_t kv_per_block;    // keys per KV block, a power of two
   int32_t group;           // Hq / Hkv
   int32_t causal;
   int32_t cost_shift;      // bin = min(kSchedBins-1, cost >> cost_shift)
-  int32_t split_target;    // backward only, 0 = off: cut expensive key blocks into pieces so that about this
-                           // many pieces exist per kv head (see piece_count)
+  int32_t split_target;    // 0 = off: cut expensive blocks into pieces so that about this many pieces exist per kv head
+                           // (see piece_count)
+  int32_t min_piece;       // the least cost of a piece
+  int32_t units_per_head;  // > 0: cut only where it is worth it (worth_cutting), for so many compute units per kv head
+  int32_t item_cost, piece_extra;  // with units_per_head: what an item costs beside its blocks' cost, and what a piece adds to that
   int32_t walk_round;      // backward only, 0 = off: items whose rank in the list is in an odd group of this many
                            // carry kWalkUp (below)
   int32_t merge_tiles;     // lists over blocks of query rows only, 0 = off: consecutive blocks of a short task form
@@ -55,20 +59,21 @@ constexpr int32_t kWalkUp = (int32_t)0x80000000u;  // flag in an item's fourth w
 DISTCA_HD int32_t item_piece(int32_t w) { return w & 0xffff; }
 DISTCA_HD int32_t item_pieces(int32_t w) { return (w >> 16) & 0x7fff; }
 
-// Cutting key blocks: a batch of few tokens has fewer key blocks than the device has compute units, and
-// the block at the start of a long document streams every query row below it, so without cuts the launch
-// lasts as long as that one workgroup.  A block of cost c (query blocks to stream) is cut into
-// ceil(c / piece) pieces of consecutive query blocks, piece = max(kMinPiece, ceil(total cost / split_target));
-// the pieces are independent work items whose dK/dV are added up in fp32.
+// Cutting blocks: a batch of few tokens has fewer blocks than the device has compute units, and the block at the start of
+// a long document (key blocks: it streams every query row below it; query blocks: the last ones stream every key above
+// them) lasts as long as the launch.  A block of cost c (query blocks, or KV tiles, to stream) is cut into ceil(c / piece)
+// pieces of consecutive ones, piece = max(min_piece, ceil(total cost / split_target)); the pieces are independent work
+// items that leave their fp32 results in slots of the workspace (SplitTables), and a second kernel adds the pieces of a block
+// up in their order, so that the result is the same in every run.
 constexpr int32_t kMinPiece = 16;
 constexpr int32_t kMaxPieces = 64;
 // Piece size for a batch of `total_cost` query-block visits: the ceiling of total / target, so that the pieces
 // of all blocks together number at most target + (number of blocks) -- the bound the work list is sized by
 // (sum of ceil(c / piece) <= total / piece + blocks, and total / piece <= target only when piece is rounded up).
-DISTCA_HD int32_t piece_size(unsigned long long total_cost, int32_t split_target) {
+DISTCA_HD int32_t piece_size(unsigned long long total_cost, int32_t split_target, int32_t min_piece) {
   if (split_target <= 0) return 0;
   const unsigned long long per = (total_cost + (unsigned long long)split_target - 1) / (unsigned long long)split_target;
-  if (per <= (unsigned long long)kMinPiece) return kMinPiece;
+  if (per <= (unsigned long long)min_piece) return min_piece;
   return per < 0x7fffffffull ? (int32_t)per : 0x7fffffff;
 }
 DISTCA_HD int32_t piece_count(int32_t cost, int32_t piece) {
@@ -79,12 +84,66 @@ DISTCA_HD int32_t piece_count(int32_t cost, int32_t piece) {
 // query blocks [lo, hi) of piece j of k over n blocks, counted from the last block downwards
 DISTCA_HD int32_t piece_begin(int32_t n, int32_t j, int32_t k) { return (int32_t)(((int64_t)n * j) / k); }
 
+// Pieces of one size, for lists of which only what is worth it is cut (units_per_head > 0): piece j of a block is its visits
+// j * size .. (j + 1) * size - 1, the last one taking what is left, up to an eighth more than `size`.  Equal parts of every block
+// (piece_begin) pack badly: four pieces of 53 for a load of 128 a unit.
+DISTCA_HD int32_t fixed_piece_count(int32_t cost, int32_t size) {
+  if (size <= 0 || cost <= size) return 1;
+  const int32_t k = (int32_t)(((uint32_t)cost - (uint32_t)size / 8 + (uint32_t)size - 1) / (uint32_t)size);
+  return k > kMaxPieces ? kMaxPieces : k;
+}
+// Visits [lo, hi) of piece j of k of a block of cost n; size: that of fixed pieces, 0 for equal parts.
+DISTCA_HD void piece_range(int32_t n, int32_t j, int32_t k, int32_t size, int32_t *lo, int32_t *hi) {
+  if (k <= 1) {
+    *lo = 0;
+    *hi = n;
+  } else if (size > 0) {
+    *lo = j * size;
+    *hi = j == k - 1 ? n : (j + 1) * size;
+  } else {
+    *lo = piece_begin(n, j, k);
+    *hi = piece_begin(n, j + 1, k);
+  }
+}
+// The size of fixed pieces for a batch of n blocks whose costs, from the most expensive down, are c[k] at rank k * units
+// (k = 0 .. 3, 0 where there is no such block); blocks stay whole when they do as well.
+// Whole blocks: units work through the list longest first, and last at least as long as the average load, as the longest block,
+// and, since of the first k * units + 1 blocks some unit gets k + 1, as k + 1 blocks of that rank's cost; longest-first
+// dispatch comes close to the largest of these.  Pieces of load / m: m of them a unit, each with its own cost on top of the load;
+// what is left over of the blocks fills the gaps, to about a quarter of a piece.
+// (8192 tokens in two documents, 32/8 heads: the forward's four blocks per unit even out, 287 us of 276 possible, and are left whole;
+// the dK/dV list's 34 key blocks for 32 units are cut, 939 -> 600 us with the adding up.)
+constexpr int kPieceTries = 8;
+// The longest a unit works when blocks stay whole, and with pieces of load / m (whose size goes to *size).
+DISTCA_HD float whole_time(const SchedGeom &g, float total_cost, int32_t n, const int32_t c[4]) {
+  const float per_unit = 1.f / (float)g.units_per_head, item = (float)g.item_cost;
+  float t = (total_cost + item * (float)n) * per_unit;
+  for (int k = 0; k < 4; ++k) {
+    const float w = c[k] > 0 ? (float)(k + 1) * ((float)c[k] + item) : 0.f;
+    t = w > t ? w : t;
+  }
+  return t;
+}
+DISTCA_HD float pieces_time(const SchedGeom &g, float total_cost, int32_t n, int32_t longest, int32_t least, int m, int32_t *size) {
+  const float per_unit = 1.f / (float)g.units_per_head, piece = (float)(g.item_cost + g.piece_extra);
+  const float load = total_cost * per_unit + 0.5f * piece * (float)n * per_unit;
+  int32_t s = (int32_t)(load / (float)m) + 1;
+  s = s < least ? least : s;
+  s = s < longest / (kMaxPieces - 8) ? longest / (kMaxPieces - 8) : s;
+  *size = s;
+  return load + piece * (total_cost * per_unit / (float)s) + 0.25f * (float)s + (float)g.piece_extra;
+}
+constexpr float kWorthCutting = 0.93f;   // cut when the pieces' time is below this share of the whole blocks'
+
 constexpr int kSchedBins = 4096;
 
 DISTCA_HD int32_t ceil_div(int32_t a, int32_t b) { return (a + b - 1) / b; }
+// The same for a power of two (the builder evaluates costs by the thousand, and a division is some thirty instructions).
+DISTCA_HD int32_t log2_of(int32_t b) { return 31 - __builtin_clz((unsigned)b); }
+DISTCA_HD int32_t ceil_div_pow2(int32_t a, int32_t b) { return (a + b - 1) >> log2_of(b); }
 
 // forward: blocks of query rows
-DISTCA_HD int32_t fwd_num_blocks(const SchedGeom &g, int32_t lq) { return ceil_div(lq * g.group, g.rows_per_block); }
+DISTCA_HD int32_t fwd_num_blocks(const SchedGeom &g, int32_t lq) { return ceil_div_pow2(lq * g.group, g.rows_per_block); }
 
 // Keys visible to the last token of m-block i (0 when none): the KV extent the block streams.
 DISTCA_HD int32_t fwd_visible_keys(const SchedGeom &g, int32_t lq, int32_t lk, int32_t i) {
@@ -95,7 +154,7 @@ DISTCA_HD int32_t fwd_visible_keys(const SchedGeom &g, int32_t lq, int32_t lk, i
   return nvis > 0 ? nvis : 0;
 }
 DISTCA_HD int32_t fwd_cost(const SchedGeom &g, int32_t lq, int32_t lk, int32_t i) {
-  return ceil_div(fwd_visible_keys(g, lq, lk, i), g.kv_per_block);
+  return ceil_div_pow2(fwd_visible_keys(g, lq, lk, i), g.kv_per_block);
 }
 
 // Short tasks: a block of query rows that sees a handful of KV tiles spends a third of its workgroup's time outside the
@@ -125,14 +184,14 @@ DISTCA_HD int32_t fwd_item_cost(const SchedGeom &g, int32_t lq, int32_t lk, int3
 
 // backward: blocks of keys
 DISTCA_HD int32_t bwd_num_blocks(const SchedGeom &g, int32_t lq, int32_t lk) {
-  return lq > 0 ? ceil_div(lk, g.kv_per_block) : 0;
+  return lq > 0 ? ceil_div_pow2(lk, g.kv_per_block) : 0;
 }
 // First m-block that sees any key of KV block n.
 DISTCA_HD int32_t bwd_first_mblock(const SchedGeom &g, int32_t lq, int32_t lk, int32_t n) {
   if (!g.causal) return 0;
   int32_t t_first = n * g.kv_per_block - (lk - lq);
   if (t_first < 0) t_first = 0;
-  return (int32_t)(((int64_t)t_first * g.group) / g.rows_per_block);
+  return (int32_t)(((int64_t)t_first * g.group) >> log2_of(g.rows_per_block));
 }
 DISTCA_HD int32_t bwd_cost(const SchedGeom &g, int32_t lq, int32_t lk, int32_t n) {
   int32_t c = fwd_num_blocks(g, lq) - bwd_first_mblock(g, lq, lk, n);
@@ -218,10 +277,39 @@ DISTCA_HD SharedGroups shared_groups(int32_t *ws, int32_t num_tasks, int64_t max
   return g;
 }
 
+// Where the pieces of cut blocks leave their results, and what the kernel that adds them up reads.  A block is cut only when it
+// costs more than total / target, so fewer than `target` blocks are, and their pieces number fewer than target + blocks cut:
+// both arrays and the slots are sized by these bounds, whatever the sequence lengths are.
+//   cut   [0] blocks that are cut   [1] slots in use   [2] size of fixed pieces (0: equal parts)   [3] unused, then (unit, block, pieces, first slot) quadruples
+//   slot  per item of the list two words: its slot, -1 for an item that is a whole block; the cost of the whole block
+struct SplitTables {
+  int32_t *cut, *slot;
+};
+DISTCA_HD int64_t split_max_cut(int64_t max_blocks, int32_t target) { return max_blocks < target ? max_blocks : target; }
+DISTCA_HD int64_t split_max_slots(int64_t max_blocks, int32_t target) { return target > 0 ? target + split_max_cut(max_blocks, target) : 0; }
+DISTCA_HD int64_t split_tables_bytes(int64_t max_blocks, int32_t target, int64_t max_items) {
+  return target > 0 ? ((4 + 4 * split_max_cut(max_blocks, target) + 2 * max_items) * 4 + 255) / 256 * 256 : 0;
+}
+DISTCA_HD SplitTables split_tables(void *at, int64_t max_blocks, int32_t target) {
+  int32_t *p = (int32_t *)at;
+  return SplitTables{p, p + 4 + 4 * split_max_cut(max_blocks, target)};
+}
+
 #if defined(__HIPCC__)
 // Draws this workgroup's (item rank, kv head); false when every list is used up.  `slot` is two ints
 // of LDS that the caller may reuse afterwards.  All threads of the workgroup must call it.
+// BY_ID (the kernels for few items): no counters, the workgroup's id names the item, id / hkv of the list for head id % hkv.
+// Workgroups start in the order of their ids, so that the list is still worked through longest first, and neither an item nor the
+// end of the list costs the 3 us of a draw.  By id / drawn: 4127 tokens at 32/8 heads, forward, 74 / 97 us; 60148 tokens of short
+// documents at 8/2 heads, both directions, 539 / 590 us; 4096 query rows over 32768 keys, forward, 264 / 274 us; dK/dV of a tick of 17846
+// query rows, 2742 / 2863 us.
+template <bool BY_ID = false>
 __device__ __forceinline__ bool take_item(int32_t *tickets, int32_t nitems, int32_t hkv, int32_t *slot, int &item, int &kvh) {
+  if constexpr (BY_ID) {
+    item = (int)(blockIdx.x / (unsigned)hkv);
+    kvh = (int)(blockIdx.x - (unsigned)item * (unsigned)hkv);
+    return item < nitems;
+  }
   if (threadIdx.x < 64) {  // the first wave
     // One look at all the counters at once (a lane per head): a workgroup that comes when every list is used
     // up -- half of the launch's workgroups -- leaves after a single round trip to memory.  Counters only

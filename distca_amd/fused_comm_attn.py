@@ -133,7 +133,7 @@ def ca_varlen_fwd(q: Tensor, k: Tensor, v: Tensor, cu_seqlens_q: Tensor, cu_seql
     tk, hkv, _ = k.shape
     lib = _lib.load()
     p = _params(cu_seqlens_q.shape[0] - 1, tq, tk, hq, hkv, d, max_seqlen_q, max_seqlen_k, scale, causal, False, q.dtype)
-    need = lib.distca_ca_fwd_workspace_bytes(ctypes.byref(p))
+    need = (lib.distca_ca_fwd_workspace_preferred_bytes if workspace is None else lib.distca_ca_fwd_workspace_bytes)(ctypes.byref(p))
     if need < 0:
         _lib.check(int(need), "ca_varlen_fwd")
     out = torch.empty_like(q)
@@ -180,7 +180,10 @@ def ca_varlen_bwd(dout: Tensor, q: Tensor, k: Tensor, v: Tensor, out: Tensor, so
     scale = softmax_scale if softmax_scale is not None else d ** (-0.5)
     lib = _lib.load()
     p = _params(cu_seqlens_q.shape[0] - 1, tq, tk, hq, hkv, d, max_seqlen_q, max_seqlen_k, scale, causal, deterministic, q.dtype)
-    need = lib.distca_ca_bwd_workspace_bytes(ctypes.byref(p))
+    # (a call over shared K/V rows brings what distca_ca_bwd_workspace_bytes asks for: the same bits as the C ABI's other forms give
+    # with it; the server's tick takes the preferred size)
+    whole = workspace is not None or kv_task_offsets is not None
+    need = (lib.distca_ca_bwd_workspace_bytes if whole else lib.distca_ca_bwd_workspace_preferred_bytes)(ctypes.byref(p))
     if need < 0:
         _lib.check(int(need), "ca_varlen_bwd")
     dq = torch.empty_like(q) if dq is None else dq
@@ -369,7 +372,7 @@ def ca_server_forward(recv_buffer: Tensor, send_buffer: Tensor, meta: ServerFwdM
         assert fa_args.causal and fa_args.window_size == (-1, -1) and fa_args.dropout_p == 0.0
         p = _params(cu_q.shape[0] - 1, tq, tk, hq, hkv, d, fa_params.max_seqlen_q, fa_params.max_seqlen_kv, scale,
                     fa_args.causal, False, dtype)
-        need = lib.distca_ca_fwd_workspace_bytes(ctypes.byref(p))
+        need = lib.distca_ca_fwd_workspace_preferred_bytes(ctypes.byref(p))
         if need < 0:
             _lib.check(int(need), "ca_server_forward")
         ws = _workspace(None, int(need), dev)
@@ -456,7 +459,7 @@ With that layout and `kv_shards_in_place` (the default) the kernels also read th
         lib = _lib.load()
         p = _params(cu_seqlens_q.shape[0] - 1, tq, int(k_rows), hq, hkv, d, max_seqlen_q, max_seqlen_kv, scale, fa_args.causal,
                     fa_args.deterministic, dtype)
-        need = lib.distca_ca_bwd_workspace_bytes(ctypes.byref(p))
+        need = lib.distca_ca_bwd_workspace_preferred_bytes(ctypes.byref(p))
         if need < 0:
             _lib.check(int(need), "ca_server_backward")
         ws = _workspace(None, int(need), dev)
@@ -488,7 +491,7 @@ With that layout and `kv_shards_in_place` (the default) the kernels also read th
         lib = _lib.load()
         p = _params(cu_seqlens_q.shape[0] - 1, tq, tk, hq, hkv, d, max_seqlen_q, max_seqlen_kv, scale, fa_args.causal,
                     fa_args.deterministic, dtype)
-        need = lib.distca_ca_bwd_workspace_bytes(ctypes.byref(p))
+        need = lib.distca_ca_bwd_workspace_preferred_bytes(ctypes.byref(p))
         if need < 0:
             _lib.check(int(need), "ca_server_backward")
         ws = _workspace(None, int(need), dev)

@@ -193,12 +193,12 @@ typedef struct distca_ca_params {
   int32_t max_seqlen_k; /* upper bound of any task's Lk                       */
   float softmax_scale;  /* multiplies q.k before softmax                      */
   int32_t causal;       /* 0 / 1                                              */
-  int32_t deterministic;/* backward only: 1 = use no float atomics, so that two
-                           runs give the same bits (the reference's server
-                           default, fused_comm_attn.py:95-104).  0 allows them
-                           where they pay: a batch too small to occupy the
-                           device has its key blocks cut into pieces whose
-                           dK/dV are added up with atomics                    */
+  int32_t deterministic;/* backward only (the reference's server default,
+                           fused_comm_attn.py:95-104).  Two runs give the same
+                           bits either way: there are no float atomics.  1 asks
+                           for the smallest workspace: a batch too small to
+                           occupy the device keeps whole key blocks unless
+                           the caller brings the preferred workspace          */
   int32_t dtype;        /* element type of q, k, v, out and the gradients:
                            DISTCA_DTYPE_BF16 or DISTCA_DTYPE_F16; 0 (callers
                            written before the field existed) means bf16      */
@@ -213,6 +213,12 @@ typedef struct distca_ca_params {
  * a workspace of their own, while calls ordered on one stream can share one.           */
 int64_t distca_ca_fwd_workspace_bytes(const distca_ca_params *p);
 int64_t distca_ca_bwd_workspace_bytes(const distca_ca_params *p);
+/* The size from which a call has room for everything it can use: a batch with fewer blocks of
+ * work than the device has room for then has its longest blocks cut into pieces, whose fp32
+ * results pass through the workspace and are added up in a fixed order.  Never less than the sizes above, and equal to
+ * them for batches that fill the device.  A call decides by the workspace_bytes it is given. */
+int64_t distca_ca_fwd_workspace_preferred_bytes(const distca_ca_params *p);
+int64_t distca_ca_bwd_workspace_preferred_bytes(const distca_ca_params *p);
 
 int distca_ca_fwd(const void *q, const void *k, const void *v, void *out,
                   float *lse, const int32_t *cu_seqlens_q,

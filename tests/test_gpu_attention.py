@@ -137,6 +137,51 @@ def test_short_tasks_as_merged_work_items(cuda, hq, hkv):
     _run([1024, 300, 700], [1024, 1324, 764], hq, hkv, 52, cuda)
 
 
+@pytest.mark.parametrize("q_lens,k_lens,hq,hkv", [
+    ([64, 1, 300, 0, 37], [5000, 4097, 2348, 300, 2600], 8, 2),     # few query rows over long prefixes, none of a tile's length
+    ([33, 70], [4100, 70], 6, 2),                                   # three heads per kv head: blocks end inside a token
+    ([3000, 129], [3000, 129], 4, 4),                               # one document longer than the rest together
+    ([200], [9000], 16, 1)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_blocks_cut_into_pieces(cuda, q_lens, k_lens, hq, hkv, causal):
+    """Batches of so few blocks that the longest are cut into pieces, whose fp32 results a second kernel adds up: forward (pieces of
+    KV tiles, some of which no row of a wave sees), dQ, and dK/dV (pieces of query blocks), with the workspace that has room
+    for them, the same bits in a second run, and within rounding of whole blocks (the smallest workspace)."""
+    import ctypes
+    from distca_amd._lib import CaParams, load
+    from distca_amd.fused_comm_attn import ca_varlen_bwd, ca_varlen_fwd
+    lib = load()
+    tq, tk = sum(q_lens), sum(k_lens)
+    p = CaParams(len(q_lens), tq, tk, hq, hkv, 128, max(q_lens), max(k_lens), 128 ** -0.5, int(causal), 1, 0)
+    assert lib.distca_ca_fwd_workspace_preferred_bytes(ctypes.byref(p)) > lib.distca_ca_fwd_workspace_bytes(ctypes.byref(p))
+    small = int(lib.distca_ca_bwd_workspace_bytes(ctypes.byref(p)))
+    assert lib.distca_ca_bwd_workspace_preferred_bytes(ctypes.byref(p)) > small
+    _run(q_lens, k_lens, hq, hkv, 71, cuda, causal=causal, deterministic=True)
+    q, k, v, do = (t.to(cuda) for t in make_qkv(tq, tk, hq, hkv, 128, 72))
+    cq, ck = torch.tensor(cu(q_lens), device=cuda), torch.tensor(cu(k_lens), device=cuda)
+    fwd = lambda x, ws=None: ca_varlen_fwd(q, k, x, cq, ck, max(q_lens), max(k_lens), None, causal, None, ws)
+    bwd = lambda ws=None: ca_varlen_bwd(do, q, k, v, *first, cq, ck, max(q_lens), max(k_lens), None, causal, True, workspace=ws)
+    first, again = fwd(v), fwd(v)
+    whole = fwd(v, torch.empty(int(lib.distca_ca_fwd_workspace_bytes(ctypes.byref(p))), dtype=torch.uint8, device=cuda))
+    sizes = fwd(v.abs())[0].float()
+    grads, grads_again, grads_whole = bwd(), bwd(), bwd(torch.empty(small, dtype=torch.uint8, device=cuda))
+    torch.cuda.synchronize()
+    assert all(torch.equal(x, y) for x, y in zip(first + grads, again + grads_again))
+    # Forward: each P is rounded to bf16 under another running maximum, at most 2^-9 of it on either side, so that the sums differ by at
+    # most 2^-8 sum P |V|, which the call with |V| gives (itself to 2^-8); then both results are rounded, 2^-9 each.
+    x, y = first[0].float(), whole[0].float()
+    assert ((x - y).abs() <= 2.0 ** -8 * (1.01 * sizes + torch.maximum(x.abs(), y.abs()))).all()
+    # the sums of the unrounded P: fp32 roundings of some hundred additions and of the exponents
+    live = torch.isfinite(whole[1])
+    assert torch.equal(torch.isfinite(first[1]), live)
+    assert ((first[1] - whole[1])[live].abs() <= 256 * 2.0 ** -24 * whole[1][live].abs().clamp(min=1)).all()
+    # Backward, from the same out and lse: the same P and dS, added up in fp32 in another order, then rounded to bf16: one unit in the last
+    # place (2^-7 at most), and for what nearly cancels, n / 16 additions of 2^-24 of terms that sum to no more than sqrt(n) times the largest result
+    for x, y in zip(grads, grads_whole):
+        x, y = x.float(), y.float()
+        assert ((x - y).abs() <= 2.0 ** -7 * y.abs() + max(k_lens) ** 1.5 / 16 * 2.0 ** -24 * y.abs().max()).all()
+
+
 @pytest.mark.parametrize("n", [12, 11])
 def test_short_tasks_either_side_of_the_merging_rule(cuda, n):
     """Blocks of short tasks are merged into larger work items from 12 blocks of query rows per compute unit on (n of them

@@ -72,6 +72,16 @@ def test_layer_step_of_a_planned_batch_whose_documents_span_ranks(cuda):
     _layer_step(cuda, 4, plan, 16, replicas=True)
 
 
+@pytest.mark.parametrize("last", [100, 1])
+def test_layer_step_of_a_lightly_loaded_server(cuda, last):
+    """Rank 0 serves one short query shard at the end of a document of many shards, so that its blocks are cut into pieces that begin in
+    the middle of the document's K/V shards; rank 1 serves the rest."""
+    from distca_amd.compute_metadata import ShardInfo
+    lens = [700, 333, 64, 1000, 1, 900, 650]
+    plan = [[ShardInfo(i % 2, 1, i, n) for i, n in enumerate(lens)] + [ShardInfo(1, 0, len(lens), last)]]
+    _layer_step(cuda, 2, plan, 17, replicas=False)
+
+
 def test_layer_step_with_an_idle_server_and_an_empty_owner(cuda):
     """Rank 2 holds tokens but serves no attention; rank 3 serves attention but holds no tokens."""
     from distca_amd.compute_metadata import ShardInfo
