@@ -1,4 +1,5 @@
-"""Compiles the HIP sources under csrc/ into distca_amd/libdistca_ca.so for gfx950.
+"""Compiles the HIP sources under csrc/ into distca_amd/libdistca_ca.so for gfx950, and the native host side of the Python
+calls (csrc/host.cpp) into distca_amd/_host.so.
 
 Run on a machine with hipcc (no GPU needed: hipcc cross-compiles).  The library is
 loaded by distca_amd._lib; tests, smoke and bench only load what is already built.
@@ -14,6 +15,7 @@ from concurrent.futures import ThreadPoolExecutor
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_PATH = os.path.join(PKG_DIR, "libdistca_ca.so")
+HOST_PATH = os.path.join(PKG_DIR, "_host.so")
 SOURCES = ["api.cpp", "pack.hip", "sched.hip", "attn_fwd.hip", "attn_bwd.hip", "attn_bwd_dkdv64.hip", "attn_bwd_dq64.hip", "probe.hip"]
 # The attention kernels exist once per element type: the same sources compiled again with -DDISTCA_F16 give the fp16
 # kernels and their launchers under names of their own; the entry points (compiled once) pick by distca_ca_params.dtype.
@@ -61,6 +63,23 @@ def _compile(src: str, obj: str, extra: list[str]) -> None:
         sys.stderr.write(err + "\n")
 
 
+def build_host() -> str:
+    """csrc/host.cpp against the C ABI's header and torch's C++ API: host code only, linked with the library beside it."""
+    import sysconfig
+    from torch.utils.cpp_extension import include_paths, library_paths
+    tmp = HOST_PATH + ".tmp"
+    cxx = shutil.which("g++") or shutil.which("c++") or "g++"
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           "-I" + sysconfig.get_paths()["include"], *("-isystem" + p for p in include_paths("cuda")), os.path.join(CSRC, "host.cpp"), "-o", tmp,
+           "-L" + PKG_DIR, *("-L" + p for p in library_paths("cuda")), "-ldistca_ca", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip",
+           "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("building _host.so failed:\n" + r.stderr)
+    os.replace(tmp, HOST_PATH)
+    return HOST_PATH
+
+
 def build_library(extra_flags: list[str] | None = None, verbose: bool = False, out_path: str | None = None) -> str:
     """Compiles and links into `out_path` (default distca_amd/libdistca_ca.so, the only path
     the loader reads)."""
@@ -81,6 +100,10 @@ def build_library(extra_flags: list[str] | None = None, verbose: bool = False, o
     os.replace(tmp, lib_path)
     if verbose:
         print("built", lib_path)
+    if lib_path == LIB_PATH:
+        build_host()
+        if verbose:
+            print("built", HOST_PATH)
     return lib_path
 
 

@@ -12,6 +12,7 @@ from ctypes import POINTER, Structure, c_char_p, c_float, c_int, c_int32, c_int6
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdistca_ca.so")
+HOST_PATH = os.path.join(_HERE, "_host.so")
 
 ABI_VERSION = 4
 
@@ -45,11 +46,8 @@ class KvShards(Structure):
 
 PACK_MAX_JOBS = 4
 
-# struct distca_exchange_job is 25 words of 64 bits: kind, dtype, num_parts, num_seq, num_tokens, token_bytes, max_cp, max_copies,
-# seq_offset, seq_tokens, mask, num_copies, copy_start, then (data, pitch, bytes) for four parts
-EXCHANGE_MAX_JOBS, TOKEN_MAX_PARTS, EXCHANGE_JOB_WORDS = 4, 4, 25
+EXCHANGE_MAX_JOBS, TOKEN_MAX_PARTS = 4, 4
 JOB_PLAIN, JOB_REPLICAS, JOB_REPLICA_SUM, JOB_COPY_SUM = range(4)
-ExchangeJobs = [c_int64 * (EXCHANGE_JOB_WORDS * n) for n in range(EXCHANGE_MAX_JOBS + 1)]   # arrays of n jobs
 
 # name -> (restype, argtypes); every symbol include/distca_ca.h declares
 SYMBOLS = {
@@ -108,6 +106,21 @@ def load() -> ctypes.CDLL:
         raise RuntimeError(f"libdistca_ca.so ABI {lib.distca_abi_version()} != binding ABI {ABI_VERSION}: rebuild")
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def host():
+    """The native host side of the calls on a step's critical path (csrc/host.cpp), loaded once."""
+    global _host
+    if _host is None:
+        load()
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(f"{HOST_PATH} is missing: build it with `python -m distca_amd._build`")
+        from . import _host as module
+        _host = module
+    return _host
 
 
 TIMER_CA_FWD, TIMER_CA_BWD, TIMER_MEMCPY_NON_CP, TIMER_MEMCPY_CP, TIMER_GRAD_SUM, TIMER_CA_BWD_DQ = range(6)

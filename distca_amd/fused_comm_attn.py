@@ -63,49 +63,14 @@ class FlashAttnArgs:
 
 # element types of the attention kernels -> DISTCA_DTYPE_* of include/distca_ca.h
 _ELEM_CODE = {torch.float16: 1, torch.bfloat16: 2}
-HEAD_DIM = 128   # what the kernels are built for; smaller head dimensions are zero-padded to it on the way in
+HEAD_DIM = 128   # what the kernels are built for; ca_varlen_* zero-pad smaller head dimensions to it on the way in (the reference pads to a
+                 # multiple of 8, fused_comm_attn.py:125-129, and leaves the rest to flash-attn)
 
 
 def _params(num_tasks, total_q, total_k, hq, hkv, d, max_q, max_k, scale, causal, deterministic,
             dtype: torch.dtype = torch.bfloat16) -> _lib.CaParams:
     return _lib.CaParams(num_tasks, total_q, total_k, hq, hkv, d, int(max_q), int(max_k), float(scale),
                          1 if causal else 0, 1 if deterministic else 0, _ELEM_CODE[dtype])
-
-
-def _pad_head_dim(t: Tensor) -> Tensor:
-    """[T, H, d] -> [T, H, 128] with zeros behind the d values of every head (the reference pads to a multiple of 8,
-    fused_comm_attn.py:125-129, and leaves the rest to flash-attn; here the kernels have one head dimension).
-    Zero dimensions add nothing to q.k, and the output's and the gradients' padded dimensions come back as zeros."""
-    d = t.shape[-1]
-    if d == HEAD_DIM:
-        return t
-    if d > HEAD_DIM or d % 8:
-        raise RuntimeError(f"head_dim={d}: must be a multiple of 8 and at most {HEAD_DIM}")
-    return torch.nn.functional.pad(t, (0, HEAD_DIM - d))
-
-
-def _check_qkv(q: Tensor, k: Tensor, v: Tensor, cu_q: Tensor, cu_k: Tensor, kv_off: Optional[Tensor]):
-    for name, t in (("q", q), ("k", k), ("v", v)):
-        if t.dim() != 3:
-            raise RuntimeError(f"{name} must have shape [tokens, heads, head_dim]")
-        if not t.is_cuda:
-            raise RuntimeError(f"{name} must be on CUDA")
-        if t.dtype not in _ELEM_CODE or t.dtype != q.dtype:
-            raise RuntimeError(f"{name} must be bfloat16 or float16, the same for q, k and v (got {t.dtype})")
-        if not t.is_contiguous():
-            raise RuntimeError(f"{name} must be contiguous")
-    if k.shape != v.shape:
-        raise RuntimeError("k and v must have the same shape")
-    if q.shape[2] != k.shape[2]:
-        raise RuntimeError("q and k must have the same head_dim")
-    for name, t in (("cu_seqlens_q", cu_q), ("cu_seqlens_k", cu_k)):
-        if t.dtype != torch.int32 or not t.is_cuda or t.dim() != 1 or not t.is_contiguous():
-            raise RuntimeError(f"{name} must be a contiguous 1-D int32 CUDA tensor")
-    if cu_q.shape != cu_k.shape:
-        raise RuntimeError("cu_seqlens_q and cu_seqlens_k must have the same shape")
-    if kv_off is not None:
-        if kv_off.dtype != torch.int32 or not kv_off.is_cuda or kv_off.shape[0] != cu_q.shape[0] - 1:
-            raise RuntimeError("kv_task_offsets must be an int32 CUDA tensor of shape [num_tasks]")
 
 
 def _workspace(given: Optional[Tensor], need: int, device) -> Tensor:
@@ -122,30 +87,8 @@ def ca_varlen_fwd(q: Tensor, k: Tensor, v: Tensor, cu_seqlens_q: Tensor, cu_seql
     """q [Tq,Hq,D], k,v [Tk,Hkv,D] bf16 or fp16 -> (out [Tq,Hq,D] in the same type, softmax_lse [Hq,Tq] fp32).
     `workspace` (uint8 CUDA tensor of at least distca_ca_fwd_workspace_bytes) is allocated
     per call when omitted.  A head dimension below 128 (multiple of 8) goes through zero-padded copies."""
-    _check_qkv(q, k, v, cu_seqlens_q, cu_seqlens_k, kv_task_offsets)
-    scale = softmax_scale if softmax_scale is not None else q.shape[2] ** (-0.5)
-    if q.shape[2] != HEAD_DIM:
-        d = q.shape[2]
-        out, lse = ca_varlen_fwd(_pad_head_dim(q), _pad_head_dim(k), _pad_head_dim(v), cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
-                                 max_seqlen_k, scale, causal, kv_task_offsets, workspace)
-        return out[..., :d].contiguous(), lse
-    tq, hq, d = q.shape
-    tk, hkv, _ = k.shape
-    lib = _lib.load()
-    p = _params(cu_seqlens_q.shape[0] - 1, tq, tk, hq, hkv, d, max_seqlen_q, max_seqlen_k, scale, causal, False, q.dtype)
-    need = (lib.distca_ca_fwd_workspace_preferred_bytes if workspace is None else lib.distca_ca_fwd_workspace_bytes)(ctypes.byref(p))
-    if need < 0:
-        _lib.check(int(need), "ca_varlen_fwd")
-    out = torch.empty_like(q)
-    lse = torch.empty((hq, tq), dtype=torch.float32, device=q.device)
-    ws = _workspace(workspace, int(need), q.device)
-    with torch.cuda.device(q.device):
-        rc = lib.distca_ca_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
-                               cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(),
-                               kv_task_offsets.data_ptr() if kv_task_offsets is not None else None,
-                               ctypes.byref(p), ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
-    _lib.check(rc, "ca_varlen_fwd")
-    return out, lse
+    return _lib.host().varlen_fwd(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale, causal,
+                                  kv_task_offsets, workspace)
 
 
 def ca_varlen_bwd(dout: Tensor, q: Tensor, k: Tensor, v: Tensor, out: Tensor, softmax_lse: Tensor,
@@ -156,51 +99,8 @@ def ca_varlen_bwd(dout: Tensor, q: Tensor, k: Tensor, v: Tensor, out: Tensor, so
                   workspace: Optional[Tensor] = None):
     """Gradients (dq, dk, dv) in the type of q; written into dq/dk/dv when given (the reference's
     flash-attn backward fills caller-allocated tensors, fused_comm_attn.py:236,259-272)."""
-    _check_qkv(q, k, v, cu_seqlens_q, cu_seqlens_k, kv_task_offsets)
-    tq, hq, d = q.shape
-    tk, hkv, _ = k.shape
-    for name, t in (("dout", dout), ("out", out)):
-        if t.shape != q.shape or t.dtype != q.dtype or not t.is_cuda:
-            raise RuntimeError(f"{name} must be a CUDA tensor with the shape and type of q")
-    if d != HEAD_DIM:
-        scale = softmax_scale if softmax_scale is not None else d ** (-0.5)
-        grads = ca_varlen_bwd(_pad_head_dim(dout), _pad_head_dim(q), _pad_head_dim(k), _pad_head_dim(v), _pad_head_dim(out),
-                              softmax_lse, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, scale, causal, deterministic,
-                              kv_task_offsets, workspace=workspace)
-        res = []
-        for g, given in zip(grads, (dq, dk, dv)):
-            g = g[..., :d]
-            res.append(g.contiguous() if given is None else given.copy_(g))
-        return tuple(res)
-    dout = dout.contiguous()
-    out = out.contiguous()
-    if softmax_lse.shape != (hq, tq) or softmax_lse.dtype != torch.float32:
-        raise RuntimeError(f"softmax_lse must be fp32 of shape [Hq, Tq] = {(hq, tq)}, got {tuple(softmax_lse.shape)}")
-    softmax_lse = softmax_lse.contiguous()
-    scale = softmax_scale if softmax_scale is not None else d ** (-0.5)
-    lib = _lib.load()
-    p = _params(cu_seqlens_q.shape[0] - 1, tq, tk, hq, hkv, d, max_seqlen_q, max_seqlen_k, scale, causal, deterministic, q.dtype)
-    # (a call over shared K/V rows brings what distca_ca_bwd_workspace_bytes asks for: the same bits as the C ABI's other forms give
-    # with it; the server's tick takes the preferred size)
-    whole = workspace is not None or kv_task_offsets is not None
-    need = (lib.distca_ca_bwd_workspace_bytes if whole else lib.distca_ca_bwd_workspace_preferred_bytes)(ctypes.byref(p))
-    if need < 0:
-        _lib.check(int(need), "ca_varlen_bwd")
-    dq = torch.empty_like(q) if dq is None else dq
-    dk = torch.empty_like(k) if dk is None else dk
-    dv = torch.empty_like(v) if dv is None else dv
-    for name, t, ref in (("dq", dq, q), ("dk", dk, k), ("dv", dv, v)):
-        if t.shape != ref.shape or t.dtype != q.dtype or not t.is_contiguous() or not t.is_cuda:
-            raise RuntimeError(f"{name} must be a contiguous CUDA tensor with the shape and type of its input")
-    ws = _workspace(workspace, int(need), q.device)
-    with torch.cuda.device(q.device):
-        rc = lib.distca_ca_bwd(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                               softmax_lse.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-                               cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(),
-                               kv_task_offsets.data_ptr() if kv_task_offsets is not None else None,
-                               ctypes.byref(p), ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
-    _lib.check(rc, "ca_varlen_bwd")
-    return dq, dk, dv
+    return _lib.host().varlen_bwd(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale, causal,
+                                  kv_task_offsets, dout, out, softmax_lse, deterministic, dq, dk, dv, workspace)
 
 
 def _qkv_to_attn_out_fwd(q: Tensor, k: Tensor, v: Tensor, fa_params: PackedSeqParams, fa_args: FlashAttnArgs):
@@ -247,33 +147,17 @@ def _qkv_to_attn_out_bwd(
     return (dq.reshape(dq.shape[0], hq * d), dk.reshape(dk.shape[0], hkv * d), dv.reshape(dv.shape[0], hkv * d))
 
 
-class CoreAttention(torch.autograd.Function):
-    """Differentiable varlen core attention on [T, H, D] tensors (drop-in for
-    flash_attn_varlen_func(..., causal=True) on the reference's call pattern)."""
-
-    @staticmethod
-    def forward(ctx, q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale, causal,
-                deterministic, kv_task_offsets):
-        out, lse = ca_varlen_fwd(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale, causal,
-                                 kv_task_offsets)
-        ctx.save_for_backward(q, k, v, out, lse, cu_seqlens_q, cu_seqlens_k)
-        ctx.kv_task_offsets = kv_task_offsets
-        ctx.args = (max_seqlen_q, max_seqlen_k, softmax_scale, causal, deterministic)
-        return out
-
-    @staticmethod
-    def backward(ctx, dout):
-        q, k, v, out, lse, cu_q, cu_k = ctx.saved_tensors
-        max_q, max_k, scale, causal, det = ctx.args
-        dq, dk, dv = ca_varlen_bwd(dout.contiguous(), q, k, v, out, lse, cu_q, cu_k, max_q, max_k, scale, causal, det,
-                                   ctx.kv_task_offsets)
-        return dq, dk, dv, None, None, None, None, None, None, None, None
-
-
 def core_attention(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale=None, causal=True,
                    deterministic=False, kv_task_offsets=None):
-    return CoreAttention.apply(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale, causal,
-                               deterministic, kv_task_offsets)
+    """Differentiable varlen core attention on [T, H, D] tensors (drop-in for
+    flash_attn_varlen_func(..., causal=True) on the reference's call pattern)."""
+    return _lib.host().core_attention(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale, causal,
+                                      kv_task_offsets, deterministic)
+
+
+class CoreAttention:
+    """core_attention by the call form of an autograd function."""
+    apply = staticmethod(core_attention)
 
 
 # ---------------------------------------------------------------------------------------

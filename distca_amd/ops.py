@@ -277,60 +277,13 @@ def pre_a2a_grad_acc(
 
 
 # ---------------------------------------------------------------------------------------
-# Several copies of one side of an all-to-all as the jobs of one launch (distca_exchange).  A job is its words and the tensors they
-# point into, which it keeps alive until it is launched.
+# Several copies of one side of an all-to-all as the jobs of one launch (distca_exchange).  A job is a tuple (kind, parts, offsets, lengths,
+# mask, token bytes, copies, first rows of copies), which keeps the tensors alive until the launch that reads and checks it.
 # ---------------------------------------------------------------------------------------
-_NO_PARTS = (0, 0, 0)
-
-
-def _check_shards(offset: torch.Tensor, tokens: torch.Tensor, mask: Optional[torch.Tensor]) -> None:
-    _check_tensor(1, offset, "seq_nvshmem_offset")
-    _check_tensor(1, tokens, "seq_tokens")
-    _check_dtype(offset, torch.int64, "seq_nvshmem_offset")
-    _check_dtype(tokens, torch.int64, "seq_tokens")
-    if tokens.size(0) < offset.size(0):
-        raise RuntimeError("seq_tokens must be of shape (num_sequence,)")
-    if mask is not None:
-        _check_tensor(1, mask, "copy_seq_mask")
-        _check_dtype(mask, torch.int8, "copy_seq_mask")
-        if mask.size(0) != offset.size(0):
-            raise RuntimeError("copy_seq_mask must be of shape (num_sequence,)")
-
-
-def _rows(tensor: torch.Tensor):
-    """(pointer, bytes between rows, bytes of a row) of a [tokens, hidden] tensor whose rows are contiguous."""
-    if tensor.dim() != 2:
-        raise RuntimeError("tensor must have 2 dimensions")
-    if not tensor.is_cuda:
-        raise RuntimeError("tensor must be on CUDA")
-    esz = tensor.element_size()
-    if tensor.size(1) > 1 and tensor.stride(1) != 1:
-        raise RuntimeError("tensor must have contiguous rows")
-    row = tensor.size(1) * esz
-    return tensor.data_ptr(), (tensor.stride(0) * esz if tensor.size(0) > 1 else row), row
-
-
 def plain_job(parts, offset: torch.Tensor, tokens: torch.Tensor, mask: Optional[torch.Tensor] = None, token_bytes: Optional[int] = None):
     """Rows of `parts` ([tokens, hidden] tensors, side by side in a transport token of `token_bytes`, by default exactly
     their rows) to or from one place per shard."""
-    _check_shards(offset, tokens, mask)
-    words = []
-    for t in parts:
-        words += _rows(t)
-    row = sum(words[2::3])
-    if any(t.size(0) != parts[0].size(0) for t in parts):
-        raise RuntimeError("token parts disagree on the token count")
-    words += _NO_PARTS * (_lib.TOKEN_MAX_PARTS - len(parts))
-    return [_lib.JOB_PLAIN, 0, len(parts), offset.size(0), parts[0].size(0), token_bytes or row, 1, 0, offset.data_ptr(), tokens.data_ptr(),
-            mask.data_ptr() if mask is not None else 0, 0, 0, *words], (parts, offset, tokens, mask)
-
-
-def _whole_job(kind: int, tensor: torch.Tensor, offset, tokens, mask, num_seq: int, max_cp: int = 1, num_copies=None, copy_start=None):
-    row = tensor.size(1) * tensor.element_size()
-    return [kind, _DTYPE_CODE.get(tensor.dtype, 0), 1, num_seq, tensor.size(0), row, max_cp, copy_start.size(1) if copy_start is not None else 0,
-            offset.data_ptr(), tokens.data_ptr(), mask.data_ptr() if mask is not None else 0,
-            num_copies.data_ptr() if num_copies is not None else 0, copy_start.data_ptr() if copy_start is not None else 0,
-            tensor.data_ptr(), row, row, *_NO_PARTS * (_lib.TOKEN_MAX_PARTS - 1)], (tensor, offset, tokens, mask, num_copies, copy_start)
+    return _lib.JOB_PLAIN, parts, offset, tokens, mask, token_bytes, None, None
 
 
 def whole_vectors(*row_bytes: int) -> bool:
@@ -340,36 +293,21 @@ def whole_vectors(*row_bytes: int) -> bool:
 
 def replicas_job(tensor: torch.Tensor, do_shard: torch.Tensor, offset: torch.Tensor, tokens: torch.Tensor):
     """a2a_memcpy_cp packing `tensor` [tokens, hidden]."""
-    _check_tensor(2, tensor, "tensor")
-    cp_degree, num_seq = _check_replicas(do_shard, offset, tokens)
-    return _whole_job(_lib.JOB_REPLICAS, tensor, offset, tokens, do_shard, num_seq, cp_degree)
+    return _lib.JOB_REPLICAS, (tensor,), offset, tokens, do_shard, None, None, None
 
 
 def replica_sum_job(tensor: torch.Tensor, do_shard: torch.Tensor, offset: torch.Tensor, tokens: torch.Tensor):
     """Every row of `tensor` [tokens, hidden] from the sum of its live replicas' rows: a2a_memcpy_cp into zeroed planes
     [max_cp, tokens, hidden] and their sum over the first dimension, without the planes."""
-    _check_tensor(2, tensor, "tensor")
-    if tensor.dtype not in _DTYPE_CODE:
-        raise RuntimeError("Only fp32, fp16 and bf16 inputs are supported")
-    cp_degree, num_seq = _check_replicas(do_shard, offset, tokens)
-    return _whole_job(_lib.JOB_REPLICA_SUM, tensor, offset, tokens, do_shard, num_seq, cp_degree)
+    return _lib.JOB_REPLICA_SUM, (tensor,), offset, tokens, do_shard, None, None, None
 
 
 def copy_sum_job(tensor: torch.Tensor, offset: torch.Tensor, tokens: torch.Tensor, mask: Optional[torch.Tensor], num_copies: torch.Tensor,
                  copy_start_id: torch.Tensor):
     """pre_a2a_grad_acc(tensor, num_copies, copy_start_id, tokens), then the plain pack of the shards `mask` names."""
-    num_seq = _check_copies(tensor, num_copies, copy_start_id, tokens)
-    _check_shards(offset, tokens, mask)
-    return _whole_job(_lib.JOB_COPY_SUM, tensor, offset, tokens, mask, num_seq, 1, num_copies, copy_start_id)
+    return _lib.JOB_COPY_SUM, (tensor,), offset, tokens, mask, None, num_copies, copy_start_id
 
 
 def exchange(jobs, buffer: torch.Tensor, to_nvshmem: bool) -> None:
     """Runs up to four jobs against `buffer` in one launch."""
-    if not buffer.is_cuda:
-        raise RuntimeError("tensor buffer must be on CUDA")
-    words = []
-    for job, _ in jobs:
-        words += job
-    rc = on_stream(_lib.load().distca_exchange, buffer.device, _lib.ExchangeJobs[len(jobs)](*words), len(jobs), buffer.data_ptr(),
-                   1 if to_nvshmem else 0)
-    _lib.check(rc, "exchange")
+    _lib.host().exchange(jobs, buffer, to_nvshmem)
