@@ -85,6 +85,15 @@ __device__ __forceinline__ void mfma32_vc(f32x16 &acc, elemx8 a, elemx8 b, const
   asm volatile(DISTCA_MFMA32_ASM " %0, %1, %2, %3" : "=&v"(acc) : "v"(a), "v"(b), "v"(c0));
 }
 
+// First key, in the workgroup's block of 256, of a wave's first or second half of 32: the halves from the block's start go to waves
+// 0, 1, 2, 3, 3, 2, 1, 0.  Every wave passes the same barrier per query block, so a block on the diagonal takes as long as the wave that
+// sees most of it: with 64 keys in a row wave 0 has a whole block's work as soon as the first key is seen.  Dealt this way no wave has more
+// than half a block's until the rows see 128 keys, nor ever where a task ends in a block of at most 128 keys.
+// The kernel over 131072 tokens in documents of 64 / 128 / 256 / 512 / 2048, 32/8 heads, in us: 64 keys in a row 1523 / 1228 / 1152 /
+// 1554 / 4346, in halves 1299 / 1075 / 1121 / 1530 / 4275 (a visit of half the work still takes 1.7 us of 2.0: requests, barrier and
+// the chain from S to dK do not shrink with it).
+__device__ __forceinline__ int dkdv_half_key(int wave, int half) { return half ? kBN - 32 - 32 * wave : 32 * wave; }
+
 #define DKDV_SHARED 0
 #define DKDV_SEG 0
 #define DKDV_SPLIT 0
@@ -143,7 +152,7 @@ __global__ __launch_bounds__(kThreads) void ca_bwd_dkdv64_combine_kernel(BwdArgs
   const int kb = (part >> 1) & 1, db0 = 2 * (part & 1);
   const int ks = a.grp_off ? a.grp_off[unit] : (a.kv_off ? a.kv_off[unit] : a.cu_k[unit]);
   const int kmax = a.grp_lmax ? a.grp_lmax[unit] : a.cu_k[unit + 1] - a.cu_k[unit];
-  const int key = e.y * kBN + wave * 64 + 32 * kb + l32;
+  const int key = e.y * kBN + dkdv_half_key(wave, kb) + l32;
   if (key >= kmax) return;
   elem_t *out = is_dv ? a.dv : a.dk;
   const int64_t kv_stride = (int64_t)a.hkv * kHeadDim;

@@ -365,6 +365,21 @@ def test_fp16_inputs(cuda, case):
         _run([4096], [4096], 8, 2, 65, cuda, dtype=f16)
 
 
+@pytest.mark.parametrize("form", ["own", "shared", "whole"])
+@pytest.mark.parametrize("group", [(4, 4), (12, 4), (8, 2)])
+def test_key_blocks_that_end_anywhere(cuda, form, group):
+    """Tasks that end at every edge of the 32-key halves that the dK/dV kernel's waves own in a block of 256 keys, seen whole or
+    through a prefix, own or shared, causal (some halves are never seen by a query block) and not."""
+    ends = [1, 32, 33, 96, 97, 128, 129, 160, 223, 225, 256 + 31, 512 + 127]
+    if form == "shared":
+        _run([32] * 5, [32, 96, 128, 160, 287], *group, 71, cuda, kv_offsets=[0] * 5, total_k=287)
+    elif form == "whole":
+        _run(ends, ends, *group, 72, cuda, causal=False)
+    else:
+        _run(ends, ends, *group, 73, cuda)
+        _run([e - e // 3 for e in ends], ends, *group, 74, cuda)
+
+
 def test_fp16_and_bf16_agree_on_the_same_values(cuda):
     """Inputs that are exact in both types give outputs that differ by the types' rounding only: the fp16 build is
     the bf16 build with another element type, not another algorithm."""
