@@ -89,8 +89,8 @@ __device__ __forceinline__ void mfma32_vc(f32x16 &acc, elemx8 a, elemx8 b, const
 // 0, 1, 2, 3, 3, 2, 1, 0.  Every wave passes the same barrier per query block, so a block on the diagonal takes as long as the wave that
 // sees most of it: with 64 keys in a row wave 0 has a whole block's work as soon as the first key is seen.  Dealt this way no wave has more
 // than half a block's until the rows see 128 keys, nor ever where a task ends in a block of at most 128 keys.
-// The kernel over 131072 tokens in documents of 64 / 128 / 256 / 512 / 2048, 32/8 heads, in us: 64 keys in a row 1523 / 1228 / 1152 /
-// 1554 / 4346, in halves 1299 / 1075 / 1121 / 1530 / 4275 (a visit of half the work still takes 1.7 us of 2.0: requests, barrier and
+// The kernel over 131072 tokens in documents of 64 / 128 / 256 / 512 / 2048, 32/8 heads, in us: 64 keys in a row 1526 / 1225 / 1168 /
+// 1599 / 4426, in halves 1326 / 1115 / 1092 / 1536 / 4321 (a visit of half the work still takes 1.7 us of 2.0: requests, barrier and
 // the chain from S to dK do not shrink with it).
 __device__ __forceinline__ int dkdv_half_key(int wave, int half) { return half ? kBN - 32 - 32 * wave : 32 * wave; }
 
