@@ -38,9 +38,23 @@ constexpr int kRowB = 256;    // bytes per K or V row in LDS (unpadded; chunk c 
 constexpr int kKTile = kFwdKV * kRowB;
 constexpr int kVTile = kFwdKV * kRowB;
 constexpr int kKOff = 0, kVOff = 2 * kKTile;  // two K stages, then two V stages
-constexpr int kFwdLds = 2 * kKTile + 2 * kVTile;
+// Behind the tiles the rows of O on their way out, 8 KB of a wave's own (see the epilogue); at 256 registers a wave the workgroup has
+// its compute unit, and its LDS, to itself anyway.
+constexpr int kOutOff = 2 * kKTile + 2 * kVTile, kOutWave = 32 * kRowB;
+constexpr int kFwdLds = kOutOff + kFwdWaves * kFwdMsub * kOutWave;
+constexpr int kOutStores = 32 / 4;   // store instructions of a sub-block's rows
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
+
+// The wait in the form that the compiler takes into account: it then knows that Q is there (by its own count it would wait for it
+// before every S, and with it for the tiles requested meanwhile).
+template <int N>
+__device__ __forceinline__ void wait_vm_known() {
+  static_assert(N < 16, "the low four bits of the count");
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0f70 | N);  // vmcnt(N), nothing of the other counters
+  asm volatile("" ::: "memory");
+}
 
 struct FwdArgs {
   const elem_t *q, *k, *v;
@@ -53,6 +67,7 @@ struct FwdArgs {
   int32_t hq, hkv, group, total_q;
   int32_t causal;
   float scale;
+  uint32_t group_magic;  // as in BwdArgs
   // Where the query and output tokens live.  Token t of task b starts at base + off[b] + t * tok_bytes
   // (off == nullptr: the packed tensor, off[b] = cu_q[b] * tok_bytes); head h at + h * 256 bytes.
   int32_t *tickets;  // one counter per kv head (sched.h)
@@ -124,7 +139,7 @@ __global__ __launch_bounds__(kFwdWaves * 64, (MSUB == 1 && kFwdWaves == 4 ? 2 : 
   int mblk = mb_first;
   // MERGE: the Q rows and the first K tile of a block are requested while the block before it finishes (below)
   elemx8 qf[MSUB][8];
-  bool requested = false;
+  bool requested = false, first_made = true;
 next_block:
   // MERGE: the thread index is made opaque once per block, so that what derives from it (the lanes' LDS and global
   // offsets, a few dozen registers) is computed afresh for every block instead of being carried, and partly spilled,
@@ -135,6 +150,7 @@ next_block:
   const int tid = tid_, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, g = lane >> 5;
   const int row_wg = mblk * kRows;
+  auto div_group = [&](int n) { return a.group_magic ? (int)__umulhi((uint32_t)n, a.group_magic) : n; };
 
   // ---- KV extent of this workgroup
   int tok_end = (row_wg + kRows + G - 1) / G;
@@ -186,7 +202,7 @@ next_block:
   }
 
   // ---- Q fragments (B operand of S^T = K Q^T): lane holds row l32, d = 16*s + 8*g .. +7
-  if (!MERGE || !requested) {
+  auto load_q = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int m = 0; m < MSUB; ++m) {
 #pragma unroll
@@ -195,7 +211,8 @@ next_block:
         else qf[m][s] = elemx8{0, 0, 0, 0, 0, 0, 0, 0};
       }
     }
-  }
+  };
+  if constexpr (!MERGE) load_q();
 
   // ---- K/V tile fetch: wave w brings rows 16w .. 16w+15 of the K tile and of the V tile, four
   // rows per instruction; lane p fetches the chunk that belongs at chunk position p%16 of row p/16
@@ -427,18 +444,27 @@ next_block:
   //   [b(2p),   b(2p+1)):  group 0: PV(p-1), S(p)     group 1: softmax(p-1)
   //   [b(2p+1), b(2p+2)):  group 0: softmax(p)        group 1: PV(p-1), S(p)
   // Tile p of K is read between b(2p) and b(2p+2), tile p of V between b(2p+2) and b(2p+4); every
-  // wave requests K(p+1) and V(p) at the start of its softmax half of period p (group 1 right after
-  // b(2p), group 0 right after b(2p+1)), into the stages whose last readers finished before b(2p), and
+  // wave requests K(p+1) and V(p) (those of period 0 ahead of the loop: below) at the start of its softmax half of period p (group 1
+  // right after b(2p), group 0 right after b(2p+1)), into the stages whose last readers finished before b(2p), and
   // waits for its own requests before b(2p+2).  The MFMA halves are the critical path of a period (one
   // group's, then the other's); a request holds its wave for a hundred cycles or so, and in front of
   // group 0's MFMA half that time showed in the period (-3 % with the requests behind it).
+  // The first two K tiles and the first V tile are requested together ahead of the loop, so that a block waits for memory once: with
+  // K(1) and V(0) requested in period 0, as the loop has it, that period (one tile's S to cover them) lasted as long as a second trip.
+  // (Together with the rows of O leaving through LDS and Q known to be there, 131072 tokens in documents of 128 / 256 / 512 / 2048, 32/8
+  // heads: 958 / 1010 / 1151 / 2798 -> 854 / 857 / 1014 / 2725 us; 131072 packed tokens 12.86 -> 12.72 ms.)
   // MERGE: what the item's next block starts with is requested when this block's tile loop is over, so that it
   // arrives while the results are normalised and stored: its Q rows (the Q registers are free: every S of this block
-  // is done) and its first K tile (no wave reads a K stage any more: the last barrier of the loop lies behind every S
-  // phase; tile 0 is the same for every block of a task).  The run and cursor objects the request goes through are
-  // set up afresh by the next block, which also finds its tile 0 request made.  (Made from inside the loop's last
+  // is done) and those tiles (no wave reads a stage any more: the last barrier of the loop lies behind every
+  // phase; they are the same for every block of a task).  The run and cursor objects the request goes through are
+  // set up afresh by the next block.  (Made from inside the loop's last
   // period instead, the requests cost the loop its register allocation: six hundred spills.)
   const bool more = MERGE && mblk + 1 < mb_end;
+  auto request_first = [&](int n) __attribute__((always_inline)) {
+    issue_k(0);
+    issue_v(0);
+    if (n > 1) issue_k(1);
+  };
   auto request_next_block = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int m = 0; m < MSUB; ++m) {
@@ -451,13 +477,30 @@ next_block:
         else qf[m][s] = elemx8{0, 0, 0, 0, 0, 0, 0, 0};
       }
     }
-    krun = Run{kbase, SEG ? 0 : lk};
-    if constexpr (SEG) kcur.open(a.shards, a.shards.task_shard[task]);
-    issue_k(0);  // (the next block has rows, hence at least one tile)
+    krun = vrun = Run{kbase, SEG ? 0 : lk};
+    vrun.virt = vbase;
+    if constexpr (SEG) {
+      kcur.open(a.shards, a.shards.task_shard[task]);
+      vcur = kcur;
+    }
+    request_first(ntiles);  // (of the next block's tiles, which are as many or more)
   };
   const int grp = uwave >> 2;
-  if (ntiles > 0 && (!MERGE || !requested)) issue_k(0);
-  wait_vm0();
+  // first_made: nothing is left of period 0's requests (else it repeats V(0), to the same place)
+  if (!MERGE || !requested) {
+    if constexpr (MERGE) load_q();  // (here, so that no path leads from these loads past the wait for them)
+    if (ntiles > 0) request_first(ntiles);
+    wait_vm_known<0>();
+  } else {
+    // what came after the requests are the stores of the block before this one, whose rows all exist (others follow): they need not
+    // have arrived
+    wait_vm_known<kOutStores * MSUB>();
+    first_made = first_made || ntiles == 1;
+  }
+  // the first period that makes requests of its own (opaque: known to the compiler, it becomes a first iteration of its own, and the
+  // registers of the two spill)
+  int requests_from = uniform_int(!MERGE || first_made ? 1 : 0);
+  asm volatile("" : "+s"(requests_from));
   __syncthreads();  // b0
   // The period loop is unrolled by two so that the LDS stage of every operand read is a constant folded into
   // the instruction's offset field instead of an addition per read between the MFMAs.
@@ -470,23 +513,27 @@ next_block:
     const bool act = p < ntiles && tile_active(p);
     if (act) phase_s(p, Same{});
     __syncthreads();
-    if (p + 1 < ntiles) issue_k(p + 1);
-    if (p < ntiles) issue_v(p);
+    if (p >= requests_from) {
+      if (p + 1 < ntiles) issue_k(p + 1);
+      if (p < ntiles) issue_v(p);
+    }
     if (act) phase_x(p);
-    wait_vm0();
+    if (p >= requests_from) wait_vm0();
     __syncthreads();
   };
   auto period1 = [&](int p, auto par) __attribute__((always_inline)) {
     using Same = std::integral_constant<int, decltype(par)::value>;
     using Other = std::integral_constant<int, 1 - decltype(par)::value>;
-    if (p + 1 < ntiles) issue_k(p + 1);
-    if (p < ntiles) issue_v(p);
+    if (p >= requests_from) {
+      if (p + 1 < ntiles) issue_k(p + 1);
+      if (p < ntiles) issue_v(p);
+    }
     const bool act_prev = p > 0 && tile_active(p - 1);
     if (act_prev) phase_x(p - 1);
     __syncthreads();
     if (act_prev) phase_pv(p - 1, Other{});
     if (p < ntiles && tile_active(p)) phase_s(p, Same{});
-    wait_vm0();
+    if (p >= requests_from) wait_vm0();
     __syncthreads();
   };
   if (grp == 0) {
@@ -511,7 +558,7 @@ next_block:
   }
   if constexpr (MERGE) {
     requested = more;
-    if (more) request_next_block();
+    first_made = ntiles > 1;
   }
 
   if constexpr (SPLIT) {
@@ -530,30 +577,48 @@ next_block:
     }
   }
 
-  // ---- epilogue: normalise, write O (bf16) and LSE (fp32, natural log)
+  // ---- epilogue: normalise, write O (bf16) and LSE (fp32, natural log).  A lane holds half of its row in pieces of 8 bytes (registers
+  // 4*cq .. 4*cq+3 of block db hold d0 .. d0+3); stored from there, an instruction touched 32 rows.  The pieces go to the wave's
+  // 8 KB behind the tiles, in the tiles' swizzled row layout, and leave from there four whole rows per instruction.
+  auto store_rows = [&](auto all) __attribute__((always_inline)) {  // all: every row of the block exists
 #pragma unroll
-  for (int m = 0; m < MSUB; ++m) {
-    const float l_tot = pair_sum(l_run[m]);
-    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    if (valid[m]) {
-      const int hg = row[m] - tok[m] * G;
-      uint8_t *otok = otok_m[m];
-      elem_t *op = reinterpret_cast<elem_t *>(otok) + (kvh * G + hg) * kHeadDim;
+    for (int m = 0; m < MSUB; ++m) {
+      const float l_tot = pair_sum(l_run[m]);
+      const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+      const uint32_t out_w = lds0 + kOutOff + (uwave * MSUB + m) * kOutWave;
+      const uint32_t wr = out_w + l32 * kRowB + 8 * g;
 #pragma unroll
       for (int db = 0; db < 4; ++db)
 #pragma unroll
         for (int cq = 0; cq < 4; ++cq) {
-          // registers 4*cq .. 4*cq+3 of block db hold d0 .. d0+3
-          const int d0 = 16 * db + 64 * (cq >> 1) + 8 * (cq & 1) + 4 * g;
-          const elemx4 o4 = cvt4(oacc[m][db][4 * cq] * inv, oacc[m][db][4 * cq + 1] * inv, oacc[m][db][4 * cq + 2] * inv,
-                                 oacc[m][db][4 * cq + 3] * inv);
-          *reinterpret_cast<elemx4 *>(op + d0) = o4;
+          // d0 = 16 db + 64 (cq >> 1) + 8 (cq & 1) + 4 g: chunk 2 db + 8 (cq >> 1) + (cq & 1), half g
+          const int chunk = 2 * db + 8 * (cq >> 1) + (cq & 1);
+          *static_cast<DISTCA_LDS elemx4 *>(const_cast<DISTCA_LDS void *>(lds_ptr(wr + ((chunk ^ tile_swz(l32)) << 4)))) =
+              cvt4(oacc[m][db][4 * cq] * inv, oacc[m][db][4 * cq + 1] * inv, oacc[m][db][4 * cq + 2] * inv, oacc[m][db][4 * cq + 3] * inv);
         }
-      if (g == 0) {
+      // (LDS operations of one wave complete in order: the reads below see the writes above)
+#pragma unroll
+      for (int i = 0; i < kOutStores; ++i) {
+        const int rl = 4 * i + (lane >> 4);
+        const int r = row_wg + (wave * MSUB + m) * 32 + rl;
+        const elemx8 o8 = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(out_w + rl * kRowB + (((lane & 15) ^ tile_swz(rl)) << 4)));
+        if (decltype(all)::value || r < nrows) {
+          const int t = div_group(r);
+          *reinterpret_cast<elemx8 *>(reinterpret_cast<elem_t *>(obytes + (int64_t)t * a.out_tok_bytes) + (kvh * G + (r - t * G)) * kHeadDim + 8 * (lane & 15)) = o8;
+        }
+      }
+      if (valid[m] && g == 0) {
+        const int hg = row[m] - tok[m] * G;
         const float lse = l_tot > 0.f ? (m_run[m] * c + fast_log2(l_tot)) * kLn2 : -INFINITY;
-        store_lse(a, otok, kvh * G + hg, q0 + tok[m], lse);
+        store_lse(a, otok_m[m], kvh * G + hg, q0 + tok[m], lse);
       }
     }
+  };
+  if (MERGE && more) {
+    request_next_block();
+    store_rows(std::true_type{});
+  } else {
+    store_rows(std::false_type{});
   }
   if constexpr (MERGE) {
     if (++mblk < mb_end) goto next_block;
@@ -773,6 +838,7 @@ int DISTCA_FN(run_fwd_tokens)(const void *q_base, const int64_t *q_task_off, int
   a.tickets = (int32_t *)((uint8_t *)workspace + sched_ticket_off(p->num_tasks, max_items));
   a.hq = p->num_heads_q; a.hkv = p->num_heads_kv; a.group = p->num_heads_q / p->num_heads_kv;
   a.total_q = p->total_q; a.causal = p->causal != 0; a.scale = p->softmax_scale;
+  a.group_magic = a.group == 1 ? 0u : (uint32_t)(((1ull << 32) + a.group - 1) / a.group);
   a.q_task_off = q_task_off; a.out_task_off = out_task_off; a.q_tok_bytes = q_tok_bytes; a.out_tok_bytes = out_tok_bytes;
   a.lse_in_token = lse ? 0 : 1;
   a.merge_tiles = geom.merge_tiles;

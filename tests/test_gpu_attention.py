@@ -206,6 +206,17 @@ def test_short_tasks_either_side_of_the_merging_rule(cuda, n):
             assert_close_bf16(got[r], want, name)
 
 
+@pytest.mark.parametrize("hq,hkv", [(64, 16), (64, 64)])
+def test_merged_items_whose_blocks_start_alike_and_not(cuda, hq, hkv):
+    """A merged item requests the first tiles of its next block before it stores the present one: blocks of no tile, one tile and
+    several after one another (prefixes shorter than, equal to and longer than the queries, ends on either side of a tile), items of
+    one block, a last block that is not full; enough of them for the merging rule (12 blocks of query rows per compute unit)."""
+    q_lens = [1, 63, 64, 65, 100, 128, 129, 200, 257, 300, 31]
+    k_lens = [1, 63, 64, 70, 100, 128, 193, 100, 257, 40, 95]
+    n = -(-12 * 256 * 256 // (hq * sum(q_lens)))
+    _run(q_lens * n, k_lens * n, hq, hkv, 54, cuda)
+
+
 def test_non_causal(cuda):
     _run([100, 260], [100, 260], 4, 2, 6, cuda, causal=False)
 
