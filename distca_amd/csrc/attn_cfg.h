@@ -78,7 +78,7 @@ inline SchedGeom fwd_geom(const distca_ca_params *p) {
   SchedGeom g;
   g.split_target = 0;
   g.min_piece = kMinPiece;
-  g.units_per_head = g.item_cost = g.piece_extra = 0;
+  g.units_per_head = g.item_cost = g.piece_extra = g.add_cost = 0;
   g.walk_round = 0;
   g.merge_tiles = merge_short_tasks(p) ? kMergeTilesFwd : 0;
   g.rows_per_block = kFwdRows;
@@ -109,30 +109,33 @@ inline bool few_key_blocks(const distca_ca_params *p, int per_cu) {
 }
 constexpr int kSplitFewPerCU = 2, kSplitPreferredPerCU = 8;
 // (`per_cu`: below how many blocks per compute unit)
-inline int32_t bwd_split_pieces(const distca_ca_params *p, int per_cu) {
+inline int32_t bwd_split_pieces(const distca_ca_params *p, int per_cu, int min_piece) {
   const int cus = num_compute_units();
   if (!few_key_blocks(p, per_cu)) return 0;
   const int64_t t = kSplitPiecesPerCU * cus / p->num_heads_kv;
-  // (no more than there can be: every block in pieces of kMinPiece)
+  // (no more than there can be: every block in pieces of min_piece)
   const int64_t rows = (int64_t)p->total_q * (p->num_heads_q / p->num_heads_kv);
-  const int64_t all = bwd_key_blocks_bound(p) * ((rows / kBwdRows + p->num_tasks + kMinPiece) / kMinPiece);
+  const int64_t all = bwd_key_blocks_bound(p) * ((rows / kBwdRows + p->num_tasks + min_piece) / min_piece);
   return (int32_t)(t < 1 ? 1 : (t < all ? t : all));
 }
-inline int32_t bwd_split_target(const distca_ca_params *p) { return p->deterministic ? 0 : bwd_split_pieces(p, kSplitFewPerCU); }
+inline int32_t bwd_split_target(const distca_ca_params *p) { return p->deterministic ? 0 : bwd_split_pieces(p, kSplitFewPerCU, kMinPiece); }
 // Blocks of query rows are cut into pieces of consecutive KV tiles when the batch has so few of them that the longest one
 // could bound the launch: fewer than kSplitMaxBlocksPerCU blocks per compute unit (above that longest-first dispatch evens
-// them out), and a prefix long enough for two pieces.  Returns the number of pieces to aim for per kv head, 0 = no cutting.
+// them out), and a prefix of more than kCutFromTiles KV tiles (the second launch takes 4.5 us though nothing be cut: 1000 tokens at
+// 32/8 heads, forward, 32.0 / 36.4 us).  Returns the number of pieces to aim for per kv head, 0 = no cutting.
 // It depends only on sizes that do not change with how K/V are stored, so that a tick gives the same bits in every form.
 constexpr int kSplitRowPiecesPerCU = 2;
 constexpr int kSplitMaxBlocksPerCU = 8;
+constexpr int kCutFromTiles = 16;
 inline bool few_row_blocks(const distca_ca_params *p) {
   return (int64_t)p->total_q * p->num_heads_q < (int64_t)kSplitMaxBlocksPerCU * kFwdRows * num_compute_units();
 }
 inline int32_t row_split_target(const distca_ca_params *p, int64_t max_blocks) {
   const int64_t cus = num_compute_units();
   if (!few_row_blocks(p)) return 0;
-  const int64_t most = ((int64_t)p->max_seqlen_k / kFwdKV + 1 + kMinPiece - 1) / kMinPiece;   // pieces of the longest block
-  if (most < 2) return 0;
+  const int64_t tiles = (int64_t)p->max_seqlen_k / kFwdKV + 1;
+  if (tiles <= kCutFromTiles) return 0;
+  const int64_t most = (tiles + kMinPieceWorth - 1) / kMinPieceWorth;   // pieces of the longest block
   const int64_t t = kSplitRowPiecesPerCU * cus / p->num_heads_kv, all = max_blocks * most;
   return (int32_t)(t < 1 ? 1 : (t < all ? t : all));
 }
@@ -142,14 +145,18 @@ inline int64_t list_grid(const distca_ca_params *p, int64_t items, bool few) {
 }
 // A list of which only what is worth it is cut (sched.h, worth_cutting).  item_cost and piece_extra in the list's cost unit: an
 // item's ticket, first loads and last stores take 11 us against 1.7 us per forward tile (dQ 15 against 2.4, dK/dV 14 against 1.5
-// per query block), and a piece's fp32 result written and read again about as long as its bytes take at the unit's share of the memory rate.
-inline void cut_where_worth(SchedGeom *g, const distca_ca_params *p, int32_t target, int32_t item_cost, int32_t piece_extra) {
+// per query block), a piece's fp32 result written and read again about as long as its bytes take at the unit's share of the memory rate, and
+// add_cost is the second launch.  us with pieces of 16 at least and no add_cost / of 8 with it, both directions: 256 tokens at 8/2 heads 86.6 / 74.6
+// (left whole), 389 tokens at 4/1 93.6 / 84.1, 2048 tokens at 4/1 160 / 143, a tick of 2048 query rows at 8/2 206 / 190.
+inline void cut_where_worth(SchedGeom *g, const distca_ca_params *p, int32_t target, int32_t item_cost, int32_t piece_extra, int32_t add_cost) {
   const int32_t units = num_compute_units() / p->num_heads_kv;
   g->split_target = target;
   g->merge_tiles = 0;
   g->units_per_head = units > 0 ? units : 1;
   g->item_cost = item_cost;
   g->piece_extra = piece_extra;
+  g->add_cost = add_cost;
+  g->min_piece = kMinPieceWorth;
 }
 inline SchedGeom dq_geom(const distca_ca_params *p) {
   SchedGeom g = fwd_geom(p);
@@ -167,7 +174,7 @@ inline SchedGeom bwd_geom(const distca_ca_params *p) {
   g.cost_shift = pick_cost_shift((int64_t)p->max_seqlen_q * g.group / kBwdRows + 1);
   g.split_target = bwd_split_target(p);
   g.min_piece = kMinPiece;
-  g.units_per_head = g.item_cost = g.piece_extra = 0;
+  g.units_per_head = g.item_cost = g.piece_extra = g.add_cost = 0;
   // one round of the dK/dV list per kv head: as many items as compute units serve that head (sched.h, kWalkUp)
   g.walk_round = num_compute_units() / p->num_heads_kv > 0 ? num_compute_units() / p->num_heads_kv : 1;
   return g;

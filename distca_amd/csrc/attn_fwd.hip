@@ -823,7 +823,7 @@ int DISTCA_FN(run_fwd_tokens)(const void *q_base, const int64_t *q_task_off, int
   if (lay.target > 0 && workspace_bytes < lay.total) lay = fwd_layout(p, false);   // no room for pieces
   const int64_t max_items = lay.max_items;
   const bool split = lay.target > 0, few = few_row_blocks(p);
-  if (split) cut_where_worth(&geom, p, lay.target, 6, 4);
+  if (split) cut_where_worth(&geom, p, lay.target, 6, 4, 8);
   const SplitTables tables = split ? split_tables((uint8_t *)workspace + lay.tables, lay.max_blocks, lay.target) : SplitTables{};
   rc = launch_build_forward(ListJob{cu_q, cu_k, geom, (int32_t *)workspace, max_items, tables}, p->num_tasks, s);
   if (rc) return rc;

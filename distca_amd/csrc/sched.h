@@ -32,7 +32,8 @@ struct SchedGeom {
                            // (see piece_count)
   int32_t min_piece;       // the least cost of a piece
   int32_t units_per_head;  // > 0: cut only where it is worth it (worth_cutting), for so many compute units per kv head
-  int32_t item_cost, piece_extra;  // with units_per_head: what an item costs beside its blocks' cost, and what a piece adds to that
+  int32_t item_cost, piece_extra, add_cost;  // with units_per_head: what an item costs beside its blocks' cost, what a piece adds to
+                                             // that, and what adding the pieces up takes when there are any
   int32_t walk_round;      // backward only, 0 = off: items whose rank in the list is in an odd group of this many
                            // carry kWalkUp (below)
   int32_t merge_tiles;     // lists over blocks of query rows only, 0 = off: consecutive blocks of a short task form
@@ -65,7 +66,7 @@ DISTCA_HD int32_t item_pieces(int32_t w) { return (w >> 16) & 0x7fff; }
 // pieces of consecutive ones, piece = max(min_piece, ceil(total cost / split_target)); the pieces are independent work
 // items that leave their fp32 results in slots of the workspace (SplitTables), and a second kernel adds the pieces of a block
 // up in their order, so that the result is the same in every run.
-constexpr int32_t kMinPiece = 16;
+constexpr int32_t kMinPiece = 16, kMinPieceWorth = 8;   // the latter where only what is worth it is cut
 constexpr int32_t kMaxPieces = 64;
 // Piece size for a batch of `total_cost` query-block visits: the ceiling of total / target, so that the pieces
 // of all blocks together number at most target + (number of blocks) -- the bound the work list is sized by
@@ -131,7 +132,7 @@ DISTCA_HD float pieces_time(const SchedGeom &g, float total_cost, int32_t n, int
   s = s < least ? least : s;
   s = s < longest / (kMaxPieces - 8) ? longest / (kMaxPieces - 8) : s;
   *size = s;
-  return load + piece * (total_cost * per_unit / (float)s) + 0.25f * (float)s + (float)g.piece_extra;
+  return load + piece * (total_cost * per_unit / (float)s) + 0.25f * (float)s + (float)(g.piece_extra + g.add_cost);
 }
 constexpr float kWorthCutting = 0.93f;   // cut when the pieces' time is below this share of the whole blocks'
 

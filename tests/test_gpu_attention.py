@@ -217,6 +217,13 @@ def test_merged_items_whose_blocks_start_alike_and_not(cuda, hq, hkv):
     _run(q_lens * n, k_lens * n, hq, hkv, 54, cuda)
 
 
+@pytest.mark.parametrize("lens", [[255], [300], [1023], [1024, 65], [2048], [40, 1500, 8]])
+@pytest.mark.parametrize("hq,hkv", [(4, 1), (8, 2)])
+def test_small_batches_either_side_of_the_cutting_rules(cuda, lens, hq, hkv):
+    """Blocks left whole, key blocks in pieces of eight query blocks and more, blocks of query rows from 1024 keys on; the same bits twice."""
+    _run(lens, lens, hq, hkv, 55, cuda, deterministic=True)
+
+
 def test_non_causal(cuda):
     _run([100, 260], [100, 260], 4, 2, 6, cuda, causal=False)
 
