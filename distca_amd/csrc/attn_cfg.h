@@ -65,13 +65,19 @@ inline bool merge_short_tasks(const distca_ca_params *p) {
   return p->num_tasks > 0 && (int64_t)p->total_q < (int64_t)kMergeMeanTokens * p->num_tasks;
 }
 // The lists as they are launched: merging trades workgroups for the fixed part of a block, which pays only where the blocks
-// fill the device many times over.  A batch with fewer than kMergeMinBlocksPerCU blocks of query rows per compute unit keeps
-// one block per item (forward + backward without / with merging: 389 tokens at 4/1 heads 179 / 261 us, three documents of
-// 4096 tokens in all, forward only, 86 / 187 us; 8.7 blocks per unit -1.4 %, 7.3 blocks -2.2 %; at 32 blocks per unit merging
-// is 2.8 % ahead).  num_heads_q / num_heads_kv cancel: blocks x kv heads = total_q * Hq / rows.
-constexpr int32_t kMergeMinBlocksPerCU = 12;
+// fill the device many times over, the more so the longer the tasks: from 8 blocks of query rows per compute unit on where they average
+// fewer than kMergeShortMeanTokens, else from 12 on.  The former's items aim for 64 tiles, and for 32 below 16 blocks per unit.  us,
+// forward and backward of documents of 64 to n tokens, 32/8 heads, with no merging / 32 / 64 / 128 tiles an item: n = 1024, 9 blocks per
+// unit 766 / 726 / 746 / 805, 16 blocks 1325 / 1266 / 1260 / 1352, 32 blocks 2624 / 2514 / 2446 / 2578, 64 blocks 5364 / 4974 / 4835 /
+// 4920; n = 512, 32 blocks 2194 / 2045 / 1992 / 2016.  At n = 2048 (1056 tokens in the mean) 64 tiles lose to 128 by 1 % from 24
+// blocks per unit on, and at n = 3500 all are within 1 %.  Below 8 blocks the kernels are those for few items (few_row_blocks), which
+// do not merge.  num_heads_q / num_heads_kv cancel: blocks x kv heads = total_q * Hq / rows.
+constexpr int32_t kMergeShortMeanTokens = 768;
 inline SchedGeom launched_geom(SchedGeom g, const distca_ca_params *p) {
-  if ((int64_t)p->total_q * p->num_heads_q < (int64_t)kMergeMinBlocksPerCU * g.rows_per_block * num_compute_units()) g.merge_tiles = 0;
+  const int64_t blocks = (int64_t)p->total_q * p->num_heads_q, per_cu = (int64_t)g.rows_per_block * num_compute_units();
+  const bool very_short = (int64_t)p->total_q < (int64_t)kMergeShortMeanTokens * p->num_tasks;
+  if (blocks < (very_short ? 8 : 12) * per_cu) g.merge_tiles = 0;
+  else if (very_short) g.merge_tiles = blocks < 16 * per_cu ? 32 : 64;   // (these average below kMergeMeanTokens: merge_tiles was set)
   return g;
 }
 inline SchedGeom fwd_geom(const distca_ca_params *p) {

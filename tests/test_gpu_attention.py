@@ -182,6 +182,14 @@ def test_blocks_cut_into_pieces(cuda, q_lens, k_lens, hq, hkv, causal):
         assert ((x - y).abs() <= 2.0 ** -7 * y.abs() + max(k_lens) ** 1.5 / 16 * 2.0 ** -24 * y.abs().max()).all()
 
 
+@pytest.mark.parametrize("n", [8, 7, 16, 15])
+def test_very_short_tasks_either_side_of_their_merging_rule(cuda, n):
+    """Tasks of fewer than 768 tokens in the mean are merged from 8 blocks of query rows per compute unit on, and into items twice
+    as long from 16 on: n of them here, on 256 units."""
+    lens = [1000, 17, 512, 519] * (n // 2) + [700, 324] * (n % 2)      # n * 1024 tokens x 64 heads = n blocks per unit
+    _run(lens, lens, 64, 16, 56, cuda, bwd=n < 9)
+
+
 @pytest.mark.parametrize("n", [12, 11])
 def test_short_tasks_either_side_of_the_merging_rule(cuda, n):
     """Blocks of short tasks are merged into larger work items from 12 blocks of query rows per compute unit on (n of them
