@@ -42,6 +42,7 @@ constexpr int kKOff = 0, kVOff = 2 * kKTile;  // two K stages, then two V stages
 // its compute unit, and its LDS, to itself anyway.
 constexpr int kOutOff = 2 * kKTile + 2 * kVTile, kOutWave = 32 * kRowB;
 constexpr int kFwdLds = kOutOff + kFwdWaves * kFwdMsub * kOutWave;
+constexpr int kDirectTasks = 256;    // batches without a list: at most so many tasks to look through
 constexpr int kOutStores = 32 / 4;   // store instructions of a sub-block's rows
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
@@ -61,7 +62,8 @@ struct FwdArgs {
   elem_t *out;
   float *lse;
   const int32_t *cu_q, *cu_k, *kv_off;
-  const int32_t *sched;  // schedule workspace
+  const int32_t *sched;  // schedule workspace; null (SPLIT kernels): there is no list, num_tasks tasks' blocks are taken as they come
+  int32_t num_tasks;
   const void *zero_row;  // 256 zero bytes: source of tile rows past the end of the prefix
   int32_t sched_items_off;  // int32 offset of the item array
   int32_t hq, hkv, group, total_q;
@@ -98,6 +100,33 @@ __device__ __forceinline__ void store_lse(const FwdArgs &a, uint8_t *otok, int h
   }
 }
 
+__device__ __align__(256) unsigned char zero_row_static[256];   // the zero row of a call without a list; nothing writes it
+
+// Block `e` of the batch's blocks of query rows, counted task after task, as a list's item: (task, block, -, one piece); task -1: none.
+// Every wave finds it by a scan over 64 tasks at a time.
+__device__ __forceinline__ int4 block_of_batch(const int32_t *cu_q, int num_tasks, int group, int e) {
+  const int lane = threadIdx.x & 63;
+  int before = 0;
+  for (int b0 = 0; b0 < num_tasks; b0 += 64) {
+    const int b = b0 + lane;
+    const int lq = b < num_tasks ? cu_q[b + 1] - cu_q[b] : 0;
+    const int n = lq > 0 ? (lq * group + kFwdRows - 1) / kFwdRows : 0;
+    int incl = n;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int o = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += o;
+    }
+    const unsigned long long past = __ballot(before + incl > e);
+    if (past) {
+      const int l = __builtin_ctzll(past);
+      return make_int4(b0 + l, e - before - __shfl(incl - n, l, 64), 0, 1 << 16);
+    }
+    before += __shfl(incl, 63, 64);
+  }
+  return make_int4(-1, 0, 0, 0);
+}
+
 // SEG: K/V rows are addressed through a table of shards (kv_shards.h) instead of as one dense tensor.
 // MERGE: a work item is several consecutive blocks of a task's query rows (sched.h, fwd_merge), worked off one after the
 // other; otherwise it is one block.
@@ -106,12 +135,21 @@ __device__ __forceinline__ void store_lse(const FwdArgs &a, uint8_t *otok, int h
 template <int MSUB, bool SEG, bool MERGE, bool SPLIT>
 __global__ __launch_bounds__(kFwdWaves * 64, (MSUB == 1 && kFwdWaves == 4 ? 2 : 1)) void ca_fwd_kernel(FwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  const int nitems = a.sched[0];
   int item, kvh;
-  if (!take_item<SPLIT>(a.tickets, nitems, a.hkv, reinterpret_cast<int32_t *>(lds), item, kvh)) return;
+  int4 it;
+  if (SPLIT && !a.sched) {
+    // no list (see run_fwd_tokens): the workgroup's id counts the batch's blocks
+    item = (int)(blockIdx.x / (unsigned)a.hkv);
+    kvh = (int)(blockIdx.x - (unsigned)item * (unsigned)a.hkv);
+    it = block_of_batch(a.cu_q, a.num_tasks, a.group, item);
+    if (it.x < 0) return;
+  } else {
+    const int nitems = a.sched[0];
+    if (!take_item<SPLIT>(a.tickets, nitems, a.hkv, reinterpret_cast<int32_t *>(lds), item, kvh)) return;
+    it = reinterpret_cast<const int4 *>(a.sched + a.sched_items_off)[item];
+  }
   // (the item's fields and the task's bounds are moved to scalar registers as they are read: what derives from them,
   // base pointers, loop limits and tile addresses, is then scalar arithmetic)
-  int4 it = reinterpret_cast<const int4 *>(a.sched + a.sched_items_off)[item];
   it.x = uniform_int(it.x);
   it.y = uniform_int(it.y);
   const int task = it.x;
@@ -242,7 +280,7 @@ next_block:
       } else {
         src = base + (int64_t)key * kv_stride;
       }
-      if (key >= lk) src = reinterpret_cast<const elem_t *>(a.zero_row);
+      if (key >= lk) src = reinterpret_cast<const elem_t *>(SPLIT && !a.sched ? zero_row_static : a.zero_row);
       lds_direct_load16_ptr(src + chunk * 8, lds0 + tile_off + (kRowsW * uwave + 4 * i) * kRowB);
     }
   };
@@ -825,14 +863,21 @@ int DISTCA_FN(run_fwd_tokens)(const void *q_base, const int64_t *q_task_off, int
   const bool split = lay.target > 0, few = few_row_blocks(p);
   if (split) cut_where_worth(&geom, p, lay.target, 6, 4, 8);
   const SplitTables tables = split ? split_tables((uint8_t *)workspace + lay.tables, lay.max_blocks, lay.target) : SplitTables{};
-  rc = launch_build_forward(ListJob{cu_q, cu_k, geom, (int32_t *)workspace, max_items, tables}, p->num_tasks, s);
-  if (rc) return rc;
+  // A batch whose blocks all run at once (one workgroup a compute unit) and stay whole needs no list: which workgroup has which block
+  // does not matter then, and finding one by a scan of the task bounds takes one trip to memory where the list takes a launch of 5 us.
+  // us with a list / without: 256 tokens at 4/1 heads 17.3 / 12.4, 389 at 8/2 20.0 / 15.1, 1000 at 32/8 31.9 / 26.9.
+  const bool direct = few && !split && max_items * p->num_heads_kv <= num_compute_units() && p->num_tasks <= kDirectTasks;
+  if (!direct) {
+    rc = launch_build_forward(ListJob{cu_q, cu_k, geom, (int32_t *)workspace, max_items, tables}, p->num_tasks, s);
+    if (rc) return rc;
+  }
 
   FwdArgs a;
   a.q = (const elem_t *)q; a.k = (const elem_t *)k; a.v = (const elem_t *)v;
   a.out = (elem_t *)out; a.lse = lse;
   a.cu_q = cu_q; a.cu_k = cu_k; a.kv_off = kv_off;
-  a.sched = (const int32_t *)workspace;
+  a.sched = direct ? nullptr : (const int32_t *)workspace;
+  a.num_tasks = p->num_tasks;
   a.zero_row = (const uint8_t *)workspace + sched_zero_row_off(p->num_tasks, max_items);
   a.sched_items_off = (int32_t)sched_header_ints(p->num_tasks);
   a.tickets = (int32_t *)((uint8_t *)workspace + sched_ticket_off(p->num_tasks, max_items));

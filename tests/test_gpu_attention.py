@@ -232,6 +232,15 @@ def test_small_batches_either_side_of_the_cutting_rules(cuda, lens, hq, hkv):
     _run(lens, lens, hq, hkv, 55, cuda, deterministic=True)
 
 
+@pytest.mark.parametrize("hq,hkv,lens", [(4, 1, [1]), (4, 1, [389]), (8, 2, [0, 65, 0, 0, 129, 64, 0]), (4, 4, [1, 257, 3] * 5), (32, 8, [1000]),
+                                         (8, 1, [2, 0] * 70 + [33, 31]), (2, 2, [3] * 127), (2, 2, [3] * 128), (32, 8, [1300])])
+def test_few_blocks_without_a_list(cuda, hq, hkv, lens):
+    """Forward batches whose blocks all run at once are taken by a scan of the task bounds: empty tasks, more tasks than a wave has
+    lanes, as many blocks as compute units and more, a longer prefix; the lists of the backward beside them."""
+    _run(lens, lens, hq, hkv, 57, cuda, bwd=len(lens) < 20)
+    _run(lens, [n + 70 if n else 0 for n in lens], hq, hkv, 58, cuda, bwd=False)
+
+
 def test_non_causal(cuda):
     _run([100, 260], [100, 260], 4, 2, 6, cuda, causal=False)
 
