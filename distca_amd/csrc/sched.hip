@@ -15,23 +15,26 @@ constexpr int kSchedThreads = 1024;
 // chains of dependent reads, and at half a microsecond a read from memory they were most of its time.
 constexpr int kLdsTasks = kSchedThreads;
 
+// Inclusive sum over the wave's lanes, by DPP moves: within rows of 16, then from the last lane of a row and of a half on.  (Lane
+// exchanges through LDS, ten of them a scan, were most of a scan's microsecond.)
+__device__ __forceinline__ int32_t wave_inclusive_scan_i32(int32_t v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
 __device__ __forceinline__ int32_t block_inclusive_scan_i32(int32_t v, int32_t *wave_sums) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    int32_t o = __shfl_up(v, off, 64);
-    if (lane >= off) v += o;
-  }
+  v = wave_inclusive_scan_i32(v);
   __syncthreads();
   if (lane == 63) wave_sums[wave] = v;
   __syncthreads();
-  // (the sums of the waves before this one: a read and a few lane exchanges instead of a chain of up to fifteen reads)
-  int32_t sum = lane < kSchedThreads / 64 ? wave_sums[lane] : 0;
-#pragma unroll
-  for (int off = 1; off < kSchedThreads / 64; off <<= 1) {
-    const int32_t o = __shfl_up(sum, off, 64);
-    if (lane >= off) sum += o;
-  }
+  // (the sums of the waves before this one: a read and a scan instead of a chain of up to fifteen reads)
+  const int32_t sum = wave_inclusive_scan_i32(lane < kSchedThreads / 64 ? wave_sums[lane] : 0);
   return v + (wave > 0 ? __builtin_amdgcn_readlane(sum, __builtin_amdgcn_readfirstlane(wave) - 1) : 0);
 }
 
@@ -100,6 +103,7 @@ __device__ __forceinline__ int32_t find_task(const int32_t *base, int32_t num_ta
 
 struct ListScratch {
   int32_t bins[kSchedBins], base[kLdsTasks + 1], wave_sums[kSchedThreads / 64], ranked[4];
+  uint32_t order[kLdsTasks];   // of a dK/dV list's entries: (unit, block, piece), as one number
   int32_t carry, num_cut, num_slots, piece;
   unsigned long long total_cost;
 };
@@ -161,9 +165,10 @@ __device__ __forceinline__ void build_list(ListScratch &s, const Units &u, int32
   if (g.split_target > 0) {
     unsigned long long local = 0;
     each_block([&](int32_t, int32_t, int32_t cost) { local += (unsigned long long)cost; });
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) local += __shfl_xor(local, off, 64);
-    if ((tid & 63) == 0) atomicAdd(&s.total_cost, local);
+    // (three sums that cannot overflow: a thread's costs stay below 2^58)
+    const int32_t lo = wave_inclusive_scan_i32((int32_t)(local & 0xffff)), mid = wave_inclusive_scan_i32((int32_t)((local >> 16) & 0xffff)),
+                  hi = wave_inclusive_scan_i32((int32_t)(local >> 32));
+    if ((tid & 63) == 63) atomicAdd(&s.total_cost, (unsigned long long)(uint32_t)lo + ((unsigned long long)(uint32_t)mid << 16) + ((unsigned long long)(uint32_t)hi << 32));
     if (tid == 0) s.piece = 0;
     __syncthreads();
     if (tid == 0) s.piece = piece_size(s.total_cost, g.split_target, g.min_piece);
@@ -238,6 +243,8 @@ __device__ __forceinline__ void build_list(ListScratch &s, const Units &u, int32
   }
   offsets(starts);
 
+  // (piece numbers are below kMaxPieces)
+  auto order_of = [](int32_t block, int32_t piece) { return ((uint32_t)block << 6) | (uint32_t)piece; };
   // 4. scatter
   each_block([&](int32_t b, int32_t i, int32_t cost) {
     const int32_t k = fixed ? fixed_piece_count(cost, piece) : piece_count(cost, piece);
@@ -259,6 +266,7 @@ __device__ __forceinline__ void build_list(ListScratch &s, const Units &u, int32
       if (pos < max_items) {
         reinterpret_cast<int4 *>(items)[pos] = make_int4(b, i, cj, j | (k << 16));
         if (split.cut) reinterpret_cast<int2 *>(split.slot)[pos] = make_int2(slot < 0 ? -1 : slot + j, cost);
+        if (BWD && pos < kLdsTasks) s.order[pos] = order_of(base[b] + i, j);
       }
     }
   });
@@ -277,9 +285,16 @@ __device__ __forceinline__ void build_list(ListScratch &s, const Units &u, int32
       const int32_t seg1 = s.bins[bin] < total ? s.bins[bin] : total;
       const int64_t key = ((int64_t)(base[it.x] + it.y) << 16) | item_piece(it.w);
       int32_t rank = seg0;
-      for (int32_t o = seg0; o < seg1 && seg1 - seg0 <= kWalkTieLimit; ++o) {
-        const int4 ot = reinterpret_cast<const int4 *>(items)[o];
-        rank += (((int64_t)(base[ot.x] + ot.y) << 16) | item_piece(ot.w)) < key;
+      if (seg1 - seg0 <= kWalkTieLimit) {
+        if (total <= kLdsTasks && nitems <= kLdsTasks) {   // from LDS: 76 items of 8192 tokens, 5.7 us of the launch's 24 otherwise
+          const uint32_t mine = order_of(base[it.x] + it.y, item_piece(it.w));
+          for (int32_t o = seg0; o < seg1; ++o) rank += s.order[o] < mine;
+        } else {
+          for (int32_t o = seg0; o < seg1; ++o) {
+            const int4 ot = reinterpret_cast<const int4 *>(items)[o];
+            rank += (((int64_t)(base[ot.x] + ot.y) << 16) | item_piece(ot.w)) < key;
+          }
+        }
       }
       // only the flag bit changes, and the reads above look at the other bits only
       if ((rank / g.walk_round) & 1) items[4 * pos + 3] = it.w | kWalkUp;
