@@ -19,8 +19,8 @@ from typing import List, Sequence, Tuple
 import torch
 from torch import Tensor
 
-from .ops import (DispatcherWrapper, _transport_buffer, a2a_memcpy_cp, a2a_memcpy_non_cp, a2a_memcpy_non_cp_multi, copy_sum_job, exchange,
-                  plain_job, pre_a2a_grad_acc, replicas_job, whole_vectors)
+from .ops import (DispatcherWrapper, _transport_buffer, a2a_memcpy_cp, a2a_memcpy_non_cp, a2a_memcpy_non_cp_multi,
+                  copy_sum_job, exchange, plain_job, pre_a2a_grad_acc, replicas_job, token_part, whole_vectors)
 from .utils import round_up
 
 
@@ -188,9 +188,8 @@ def send_attn_out_grad_resend_qkv(attn_out_grad: Tensor, attn_out: Tensor, lse_n
     if q.dtype != attn_out.dtype or attn_out_grad.shape != attn_out.shape:
         raise AssertionError("dO, O and q of a backward request share one dtype, and dO has the shape of O")
     buffer = _transport_buffer(buffer, instance_id, True)
-    parts = [t if t.stride(1) == 1 and (t.stride(0) * t.element_size()) % 16 == 0 and t.data_ptr() % 16 == 0 else t.contiguous() for t in parts]
     k, v = k.contiguous(), v.contiguous()
-    exchange([plain_job(parts, q_send_buffer_offset, q_seq_tokens), replicas_job(k, kv_dispatch_mask, k_send_buffer_offset, k_seq_tokens),
+    exchange([plain_job([token_part(t) for t in parts], q_send_buffer_offset, q_seq_tokens), replicas_job(k, kv_dispatch_mask, k_send_buffer_offset, k_seq_tokens),
               replicas_job(v, kv_dispatch_mask, v_send_buffer_offset, k_seq_tokens)], buffer, True)
 
 

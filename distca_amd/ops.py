@@ -291,6 +291,16 @@ def whole_vectors(*row_bytes: int) -> bool:
     return all(n > 0 and n % 16 == 0 for n in row_bytes)
 
 
+def token_part(t: torch.Tensor) -> torch.Tensor:
+    """`t` [tokens, hidden] as a part a token is put together from: itself where the launch can read its rows where they lie (rows of
+    their own, one behind the other at a pitch of whole vectors), else a copy.  Expanded rows, rows that overlap, transposed matrices
+    and rows off 16-byte alignment (which `contiguous` may hand back as they are) are copied."""
+    pitch = t.stride(0) * t.element_size()
+    if t.stride(1) == 1 and t.size(1) <= t.stride(0) and pitch % 16 == 0 and pitch < 1 << 31 and t.data_ptr() % 16 == 0:
+        return t
+    return t.clone(memory_format=torch.contiguous_format)
+
+
 def replicas_job(tensor: torch.Tensor, do_shard: torch.Tensor, offset: torch.Tensor, tokens: torch.Tensor):
     """a2a_memcpy_cp packing `tensor` [tokens, hidden]."""
     return _lib.JOB_REPLICAS, (tensor,), offset, tokens, do_shard, None, None, None

@@ -274,3 +274,22 @@ def test_torch_ops_are_registered_for_device_tensors_only():
         torch.ops.distca_amd.fast_a2a_memcpy_non_cp_debug(t, i64, i64, None, True, torch.zeros(64, dtype=torch.uint8))
     with pytest.raises(NotImplementedError):
         torch.ops.distca_amd.fast_a2a_grad_acc(t, torch.zeros(1, dtype=torch.int32), torch.zeros((1, 1), dtype=torch.int64), i64)
+
+
+def test_parts_of_a_request_token_are_rows_the_launch_can_read():
+    """What goes into a request as it is has a pitch of whole vectors, at least a row long, and a 16-byte aligned start (the launch
+    refuses anything else); every other form a caller may bring is copied, the gradient of a sum over tokens (a pitch of 0) among them."""
+    import torch
+    from distca_amd.ops import token_part
+    T, h = 5, 32
+    base = torch.arange(2 * T * h + 64, dtype=torch.float32).to(torch.bfloat16)
+    rows = base[:T * h].view(T, h)
+    assert token_part(rows) is rows
+    wide = base[:2 * T * h].view(T, 2 * h)[:, h:]
+    assert token_part(wide) is wide
+    forms = [rows[:1].expand(T, h), rows[:, :1].expand(T, h), base[:h * T].view(h, T).t(), base.as_strided((T, h), (8, 1)), base.as_strided((T, h), (h + 1, 1)),
+             base[1:1 + T * h].view(T, h), base.as_strided((T, h), (2 * h, 2)), rows[:1].expand(T, h)[:1], rows[:0]]
+    for t in forms:
+        p = token_part(t)
+        assert torch.equal(p, t) and p.stride(1) == 1 and p.data_ptr() % 16 == 0
+        assert p.size(0) <= 1 or (p.stride(0) >= h and p.stride(0) * 2 % 16 == 0)

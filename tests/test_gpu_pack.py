@@ -334,3 +334,41 @@ def test_rows_added_up_on_the_way(cuda, dtype, scale):
         exchange([copy_sum_job(d, dev(boff), dev(lens), dev(mask), dev(nc), dev(cs))], dbuf, True)
         torch.cuda.synchronize()
         assert torch.equal(d.cpu().view(torch.uint8), exp_t.view(torch.uint8)) and np.array_equal(dbuf.cpu().numpy(), exp)
+
+
+REQUEST_FORMS = {
+    "expanded": lambda t: t[:1].expand_as(t),                                       # what autograd hands on for a sum over tokens
+    "one value": lambda t: t[:1, :1].expand_as(t),
+    "overlapping": lambda t: t.reshape(-1).as_strided(t.shape, (16, 1)),
+    "transposed": lambda t: t.t().contiguous().t(),
+    "every other column": lambda t: t.repeat_interleave(2, dim=1)[:, ::2],
+    "off alignment": lambda t: torch.cat([t.reshape(-1)[:1], t.reshape(-1)])[1:].view(t.shape),
+    "odd pitch": lambda t: torch.cat([t, t[:, :1]], dim=1)[:, :t.shape[1]],
+    "wide pitch": lambda t: torch.cat([t, t], dim=1)[:, :t.shape[1]],
+}
+
+
+@pytest.mark.parametrize("form", list(REQUEST_FORMS))
+@pytest.mark.parametrize("which", range(4))
+def test_request_tokens_from_any_strides(cuda, form, which):
+    """The backward request with one of its parts in a form other than packed rows: the bytes of the token matrix, which takes any."""
+    from distca_amd.dispatch import pre_a2a_attn_out_grad_resend_qkv, send_attn_out_grad_resend_qkv
+    g = torch.Generator().manual_seed(5 + which)
+    lens = [3, 0, 9, 1]
+    T, hq, hkv, d = sum(lens), 4, 1, 128
+    rnd = lambda n, dt=torch.bfloat16: torch.randn((T, n), generator=g).to(dt).to(cuda)
+    parts = [rnd(hq * d), rnd(hq * d), rnd(hq, torch.float32).view(torch.uint8), rnd(hq * d)]
+    parts[which] = REQUEST_FORMS[form](parts[which])
+    k, v = rnd(hkv * d), rnd(hkv * d)
+    i64 = lambda x: torch.tensor(x, dtype=torch.int64, device=cuda)
+    tb, kb = 3 * hq * d * 2 + hq * 4, hkv * d * 2
+    start = np.concatenate([[0], np.cumsum(lens)[:-1]])
+    end = T * tb
+    args = (k, v, torch.ones((len(lens), 1), dtype=torch.int8, device=cuda), i64(lens), i64(lens), i64(start * tb), i64(end + start * kb)[None],
+            i64(end + T * kb + start * kb)[None])
+    print(f"request with part {which} {form}: strides {parts[which].stride()}", flush=True)
+    got, want = (torch.zeros(end + 2 * T * kb, dtype=torch.uint8, device=cuda) for _ in range(2))
+    send_attn_out_grad_resend_qkv(*parts, *args, buffer=got)
+    pre_a2a_attn_out_grad_resend_qkv(*parts, *args, buffer=want)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
