@@ -180,11 +180,11 @@ def send_attn_out_grad_resend_qkv(attn_out_grad: Tensor, attn_out: Tensor, lse_n
     """pre_a2a_attn_out_grad_resend_qkv for a caller that does not want the request tokens themselves: the four parts go
     straight into the buffer, where the merged matrix is written and read once more on the way (half the launch's bytes)."""
     parts = [attn_out_grad, attn_out, lse_norm, q]
+    _same_tokens("backward request", *parts)
     if not whole_vectors(*(t.shape[1] * t.element_size() for t in parts)):
         pre_a2a_attn_out_grad_resend_qkv(attn_out_grad, attn_out, lse_norm, q, k, v, kv_dispatch_mask, q_seq_tokens, k_seq_tokens,
                                          q_send_buffer_offset, k_send_buffer_offset, v_send_buffer_offset, instance_id, buffer=buffer)
         return
-    _same_tokens("backward request", *parts)
     if q.dtype != attn_out.dtype or attn_out_grad.shape != attn_out.shape:
         raise AssertionError("dO, O and q of a backward request share one dtype, and dO has the shape of O")
     buffer = _transport_buffer(buffer, instance_id, True)

@@ -293,3 +293,14 @@ def test_parts_of_a_request_token_are_rows_the_launch_can_read():
         p = token_part(t)
         assert torch.equal(p, t) and p.stride(1) == 1 and p.data_ptr() % 16 == 0
         assert p.size(0) <= 1 or (p.stride(0) >= h and p.stride(0) * 2 % 16 == 0)
+
+
+def test_request_parts_that_are_no_matrices_are_named():
+    """A part of a backward request that is no [tokens, hidden] matrix is an AssertionError that says so, whichever way the token goes."""
+    import torch
+    from distca_amd.dispatch import pre_a2a_attn_out_grad_resend_qkv, send_attn_out_grad_resend_qkv
+    t, lse, none = torch.zeros((3, 64), dtype=torch.bfloat16), torch.zeros((3, 16), dtype=torch.uint8), [None] * 8
+    for bad in (lse.reshape(-1), lse[:2], lse[:, None]):
+        for send in (pre_a2a_attn_out_grad_resend_qkv, send_attn_out_grad_resend_qkv):
+            with pytest.raises(AssertionError, match="every part must be"):
+                send(t, t, bad, t, *none)
