@@ -8,9 +8,9 @@ steps switch the current instance and release the receive buffer the way the ref
 
 How the steps are carried out is this library's own: the q, k and v of a step go through one launch (`ops.exchange`) where the
 reference makes three and more, and the parts of a composite transport token ([out | lse | pad], [dO | O | lse | q | pad])
-are copied straight between their own tensors and the buffer where their rows are whole 16-byte vectors.  Where they are not, or where the
-caller gets the token matrix itself, a `TokenLayout` writes every part into its byte range of one preallocated matrix,
-instead of concatenating and then padding.
+are copied straight between their own tensors and the buffer where their rows are whole 16-byte vectors and the token holds at most
+512 KiB.  Where not, or where the caller gets the token matrix itself, a `TokenLayout` writes every part into its byte range of one
+preallocated matrix, instead of concatenating and then padding.
 """
 from __future__ import annotations
 
@@ -19,7 +19,7 @@ from typing import List, Sequence, Tuple
 import torch
 from torch import Tensor
 
-from .ops import (DispatcherWrapper, _transport_buffer, a2a_memcpy_cp, a2a_memcpy_non_cp, a2a_memcpy_non_cp_multi,
+from .ops import (TOKEN_OF_PARTS_MAX_BYTES, DispatcherWrapper, _transport_buffer, a2a_memcpy_cp, a2a_memcpy_non_cp, a2a_memcpy_non_cp_multi,
                   copy_sum_job, exchange, plain_job, pre_a2a_grad_acc, replicas_job, token_part, whole_vectors)
 from .utils import round_up
 
@@ -35,6 +35,11 @@ class TokenLayout:
         self.starts = [sum(self.sizes[:i]) for i in range(len(parts))]
         self.payload = sum(self.sizes)
         self.token_bytes = round_up(self.payload)
+
+    @property
+    def in_parts(self) -> bool:
+        """Whether one launch can copy the parts straight between their tensors and the buffer."""
+        return whole_vectors(*self.sizes) and self.token_bytes <= TOKEN_OF_PARTS_MAX_BYTES
 
     @classmethod
     def of(cls, tensors: Sequence[Tensor]) -> "TokenLayout":
@@ -181,7 +186,7 @@ def send_attn_out_grad_resend_qkv(attn_out_grad: Tensor, attn_out: Tensor, lse_n
     straight into the buffer, where the merged matrix is written and read once more on the way (half the launch's bytes)."""
     parts = [attn_out_grad, attn_out, lse_norm, q]
     _same_tokens("backward request", *parts)
-    if not whole_vectors(*(t.shape[1] * t.element_size() for t in parts)):
+    if not TokenLayout.of(parts).in_parts:
         pre_a2a_attn_out_grad_resend_qkv(attn_out_grad, attn_out, lse_norm, q, k, v, kv_dispatch_mask, q_seq_tokens, k_seq_tokens,
                                          q_send_buffer_offset, k_send_buffer_offset, v_send_buffer_offset, instance_id, buffer=buffer)
         return
@@ -211,7 +216,7 @@ def post_a2a_attn_out_grad_resend_qkv(
     act = recv_k.dtype
     layout = TokenLayout([(recv_attn_out_shape[1], act), (recv_attn_out_shape[1], act),
                           (recv_lse_shape[1], recv_lse_dtype), (recv_q_shape[1], act)])
-    if whole_vectors(*layout.sizes) and recv_k.dim() == recv_v.dim() == 2:
+    if layout.in_parts and recv_k.dim() == recv_v.dim() == 2:
         dev = recv_k.device
         parts = [torch.empty(tuple(shape), dtype=dt, device=dev)
                  for shape, dt in zip((recv_attn_out_shape, recv_attn_out_shape, recv_lse_shape, recv_q_shape), layout.dtypes)]

@@ -18,8 +18,8 @@ import torch
 from torch import Tensor
 
 from . import _lib
-from .ops import (DispatcherWrapper, _transport_buffer, a2a_memcpy_non_cp, a2a_memcpy_non_cp_multi, exchange, plain_job, pre_a2a_grad_acc,
-                  whole_vectors)
+from .ops import (TOKEN_OF_PARTS_MAX_BYTES, DispatcherWrapper, _transport_buffer, a2a_memcpy_non_cp, a2a_memcpy_non_cp_multi, exchange,
+                  plain_job, pre_a2a_grad_acc, whole_vectors)
 from .utils import size_pad_by_int4
 from .dispatch import (_unpacked, post_a2a_attn_out, post_a2a_attn_out_grad_resend_qkv, post_a2a_qkv, pre_a2a_attn_out_with_lse, pre_a2a_qkv,
                        send_attn_out_grad_resend_qkv)
@@ -584,7 +584,7 @@ def post_a2a_attn_out_with_lse(recv_buffer: Optional[Tensor], q: Tensor, num_hea
     hidden = math.prod(q.shape[1:])
     hidden_bytes, lse_bytes = hidden * itemsize, num_heads_q * 4
     token_bytes = cols * itemsize
-    if whole_vectors(hidden_bytes, lse_bytes, token_bytes) and hidden_bytes + lse_bytes <= token_bytes:
+    if whole_vectors(hidden_bytes, lse_bytes, token_bytes) and hidden_bytes + lse_bytes <= token_bytes <= TOKEN_OF_PARTS_MAX_BYTES:
         # both parts straight from the buffer
         attn_out = torch.empty((rows, hidden), dtype=dtype, device=q.device)
         softmax_lse_bytes = torch.empty((rows, lse_bytes), dtype=torch.uint8, device=q.device)

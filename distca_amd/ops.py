@@ -291,6 +291,9 @@ def whole_vectors(*row_bytes: int) -> bool:
     return all(n > 0 and n % 16 == 0 for n in row_bytes)
 
 
+TOKEN_OF_PARTS_MAX_BYTES = 1 << 19   # of a token that a launch puts together or takes apart (distca_exchange); larger ones pass as whole rows
+
+
 def token_part(t: torch.Tensor) -> torch.Tensor:
     """`t` [tokens, hidden] as a part a token is put together from: itself where the launch can read its rows where they lie (rows of
     their own, one behind the other at a pitch of whole vectors), else a copy.  Expanded rows, rows that overlap, transposed matrices

@@ -122,7 +122,8 @@ int distca_grad_sum(void *data, int dtype, const int32_t *num_copies,
  * Rows and byte ranges of shards as in distca_memcpy_non_cp.  A token's row may be made of up to
  * DISTCA_TOKEN_MAX_PARTS parts, side by side in the buffer from byte 0 of the token on, each in a tensor of its own:
  * part i of token t is at data + t * pitch, `bytes` long.  Bytes of the token behind the last part are written as
- * zeros when packing and skipped when unpacking.  Kinds:
+ * zeros when packing and skipped when unpacking.  A token of several parts, or with bytes behind its one part, holds at
+ * most 512 KiB (DISTCA_E_UNSUPPORTED beyond).  Kinds:
  *   PLAIN        one copy per shard; mask (packing only, may be NULL) skips shards
  *   REPLICAS     distca_memcpy_cp with mask = do_shard; one part of token_bytes
  *   REPLICA_SUM  unpacking: row t becomes the sum of its live replicas' rows (in fp32, rounded once)

@@ -372,3 +372,41 @@ def test_request_tokens_from_any_strides(cuda, form, which):
     pre_a2a_attn_out_grad_resend_qkv(*parts, *args, buffer=want)
     torch.cuda.synchronize()
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("hq", [2016, 2020, 676, 680])
+def test_tokens_either_side_of_what_a_launch_takes_apart(cuda, hq):
+    """A launch puts tokens together from parts, or takes them apart, up to 512 KiB; larger ones pass as whole rows.  A reply holds
+    260 bytes a head (2016: 524 160, 2020: 525 200), a request 772 (676: 521 872, 680: 524 960)."""
+    from distca_amd.dispatch import post_a2a_attn_out_grad_resend_qkv, send_attn_out_grad_resend_qkv
+    from distca_amd.fused_comm_attn import post_a2a_attn_out_with_lse
+    from types import SimpleNamespace as NS
+    g = torch.Generator().manual_seed(hq)
+    lens, row = [1, 0, 2], hq * 256
+    T = sum(lens)
+    i64 = lambda x: torch.tensor(x, dtype=torch.int64, device=cuda)
+    start = np.concatenate([[0], np.cumsum(lens)[:-1]])
+    rows = lambda n: torch.randint(0, 256, (T, n), generator=g, dtype=torch.uint8)
+    print(f"tokens of {hq} heads", flush=True)
+    if hq > 2000:
+        tb = (row + 4 * hq + 15) // 16 * 16
+        reply = rows(tb)
+        md = NS(tensor_shape=[NS(recv_shape=(T, tb // 2))], recv_memcpy_metadata=[i64(start * tb)], seq_lens=[NS(recv_seqlens=i64(lens))])
+        out, lse = post_a2a_attn_out_with_lse(reply.reshape(-1).to(cuda), torch.empty((T, hq * 128), dtype=torch.bfloat16, device=cuda), hq, md)
+        assert torch.equal(out.reshape(T, -1).view(torch.uint8).cpu(), reply[:, :row]) and torch.equal(lse.cpu(), reply[:, row:row + 4 * hq])
+        return
+    tb, kb = 3 * row + 4 * hq, 256
+    parts = [rows(row), rows(row), rows(4 * hq), rows(row)]
+    k, v = rows(kb), rows(kb)
+    bf = lambda t: t.to(cuda).view(torch.bfloat16)
+    ones = torch.ones((len(lens), 1), dtype=torch.int8, device=cuda)
+    offs = [i64(start * tb), i64(T * tb + start * kb), i64(T * (tb + kb) + start * kb)]
+    buf = torch.zeros(T * (tb + 2 * kb), dtype=torch.uint8, device=cuda)
+    send_attn_out_grad_resend_qkv(bf(parts[0]), bf(parts[1]), parts[2].to(cuda), bf(parts[3]), bf(k), bf(v), ones, i64(lens), i64(lens), offs[0],
+                                  offs[1][None], offs[2][None], buffer=buf)
+    assert torch.equal(buf.cpu(), torch.cat([torch.cat(parts, dim=1).reshape(-1), k.reshape(-1), v.reshape(-1)]))
+    rk, rv = (torch.empty((T, kb // 2), dtype=torch.bfloat16, device=cuda) for _ in range(2))
+    got = post_a2a_attn_out_grad_resend_qkv([T, row // 2], [T, hq], [T, row // 2], torch.float32, rk, rv, None, i64(lens), i64(lens), *offs, True,
+                                            buffer=buf)
+    for t, want in zip(got, parts + [k, v]):
+        assert torch.equal(t.view(torch.uint8).cpu(), want)
