@@ -279,7 +279,7 @@ __global__ __launch_bounds__(kPackThreads, SUMS ? 4 : 8) void exchange_kernel(Jo
   if (t0 >= t1) return;
   Segment sg = find_segment(jb.seq_tokens, jb.num_seq, t0);
   int seg = sg.idx;
-  int64_t seg_start = sg.start;
+  int64_t seg_start = seg < jb.num_seq ? sg.start : t0;
   const int64_t tb = jb.token_bytes;
   const bool replicas = jb.kind == DISTCA_JOB_REPLICAS || jb.kind == DISTCA_JOB_REPLICA_SUM;
   for (; seg < jb.num_seq && seg_start < t1; ++seg) {
@@ -339,6 +339,11 @@ __global__ __launch_bounds__(kPackThreads, SUMS ? 4 : 8) void exchange_kernel(Jo
     uint8_t *ten = jb.data + a * tb;
     if (TO_BUF) copy_run(buf, ten, nvec);
     else copy_run(ten, buf, nvec);
+  }
+  if (SUMS && jb.kind == DISTCA_JOB_REPLICA_SUM && seg_start < t1) {   // rows behind the last shard: sums of nothing
+    const uint32_t nvec = (uint32_t)((t1 - seg_start) * (tb >> 4));
+    const run_t dst = make_run(jb.data + seg_start * tb, nvec);
+    for (int i = threadIdx.x; i < (int)nvec; i += kPackThreads) store_nt(dst, i, u32x4{0, 0, 0, 0});
   }
 }
 
@@ -415,10 +420,12 @@ int64_t slice_tokens(int64_t slice, int64_t tokens, int64_t token_bytes, int64_t
 int add_job(Jobs *jobs, const distca_exchange_job &in, int64_t token_bytes, int to_buffer, const void *buffer, const char *what) {
   const bool replicas = in.kind == DISTCA_JOB_REPLICAS || in.kind == DISTCA_JOB_REPLICA_SUM;
   if (in.num_seq < 0 || in.num_tokens < 0 || token_bytes < 0 || (replicas && in.max_cp < 0)) return fail(DISTCA_E_INVALID, "%s: negative size", what);
-  if (in.num_tokens == 0 || in.num_seq == 0 || token_bytes == 0 || (replicas && in.max_cp == 0)) return 0;
-  if (!buffer || !in.seq_offset || !in.seq_tokens || (replicas && !in.mask)) return fail(DISTCA_E_INVALID, "%s: null pointer", what);
+  // (a sum over replicas writes its rows also where there is no shard or no replica: as zeros, and nothing else of the job is read)
+  const int64_t num_seq = replicas && in.max_cp == 0 ? 0 : in.num_seq;
+  if (in.num_tokens == 0 || token_bytes == 0 || (num_seq == 0 && in.kind != DISTCA_JOB_REPLICA_SUM)) return 0;
+  if (num_seq > 0 && (!buffer || !in.seq_offset || !in.seq_tokens || (replicas && !in.mask))) return fail(DISTCA_E_INVALID, "%s: null pointer", what);
   if (token_bytes % 16) return fail(DISTCA_E_INVALID, "%s: token_bytes=%lld is not a multiple of 16", what, (long long)token_bytes);
-  if (in.num_tokens * (replicas ? in.max_cp : 1) >= (1ll << 31) || in.num_seq >= (1ll << 31) || token_bytes >= (1ll << 31))
+  if (in.num_tokens * (replicas && in.max_cp > 0 ? in.max_cp : 1) >= (1ll << 31) || in.num_seq >= (1ll << 31) || token_bytes >= (1ll << 31))
     return fail(DISTCA_E_INVALID, "%s: num_tokens%s must be < 2^31", what, replicas ? "*max_cp" : "");
   if (in.kind == DISTCA_JOB_REPLICA_SUM && to_buffer) return fail(DISTCA_E_INVALID, "%s: a sum over replicas only unpacks", what);
   if (in.kind == DISTCA_JOB_COPY_SUM && !to_buffer) return fail(DISTCA_E_INVALID, "%s: a sum over copies only packs", what);
@@ -439,7 +446,7 @@ int add_job(Jobs *jobs, const distca_exchange_job &in, int64_t token_bytes, int 
     o.num_copies = in.num_copies; o.copy_start = in.copy_start;
     o.num_tokens = in.num_tokens; o.token_bytes = token_bytes; o.pitch = pitch;
     o.kind = (int32_t)in.kind; o.dtype = (int32_t)in.dtype;
-    o.num_seq = (int32_t)in.num_seq; o.max_cp = (int32_t)in.max_cp; o.max_copies = (int32_t)in.max_copies;
+    o.num_seq = (int32_t)num_seq; o.max_cp = (int32_t)in.max_cp; o.max_copies = (int32_t)in.max_copies;
     o.part_v0 = (uint32_t)(at / 16); o.part_vecs = (uint32_t)(bytes / 16);
     o.magic = o.part_vecs == 1 ? 0u : (uint32_t)(((1ull << 32) + o.part_vecs - 1) / o.part_vecs);
     at += bytes;

@@ -126,7 +126,8 @@ int distca_grad_sum(void *data, int dtype, const int32_t *num_copies,
  * most 512 KiB (DISTCA_E_UNSUPPORTED beyond).  Kinds:
  *   PLAIN        one copy per shard; mask (packing only, may be NULL) skips shards
  *   REPLICAS     distca_memcpy_cp with mask = do_shard; one part of token_bytes
- *   REPLICA_SUM  unpacking: row t becomes the sum of its live replicas' rows (in fp32, rounded once)
+ *   REPLICA_SUM  unpacking: row t becomes the sum of its live replicas' rows (in fp32, rounded once); zeros where there
+ *                is none, and behind the last shard
  *   COPY_SUM     packing: distca_grad_sum of the shard (the sum stays in the tensor), then PLAIN
  * dtype (the two sums) is one of DISTCA_DTYPE_*.  Pointers, pitches, part and token sizes are multiples of 16.
  * Jobs run at the same time: their byte ranges must be disjoint, and so must a COPY_SUM's main shards and copies. */

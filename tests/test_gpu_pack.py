@@ -410,3 +410,33 @@ def test_tokens_either_side_of_what_a_launch_takes_apart(cuda, hq):
                                             buffer=buf)
     for t, want in zip(got, parts + [k, v]):
         assert torch.equal(t.view(torch.uint8).cpu(), want)
+
+
+@pytest.mark.parametrize("max_cp,nshard,behind", [(0, 3, 0), (2, 0, 0), (0, 0, 5), (2, 3, 1), (2, 3, 9000), (1, 1, 700)])
+def test_sums_over_no_replicas_are_zeros(cuda, max_cp, nshard, behind):
+    """The gradients a rank gets back are sums over replicas: zeros for rows without a replica, with no shard at all, and behind the last
+    shard (`behind` rows, in slices of their own and in one with shards), as the zeroed planes of a2a_memcpy_cp summed up."""
+    from distca_amd.dispatch_fn import pre_all2all_layout_transfer_backward
+    from distca_amd.ops import a2a_memcpy_cp
+    from types import SimpleNamespace as NS
+    rng = np.random.default_rng(behind + nshard)
+    hidden, lens = 512, rng.integers(1, 40, size=nshard).astype(np.int64)
+    covered = int(lens.sum()) if max_cp else 8
+    T, tb = covered + behind, hidden * 2
+    off = np.array([[c * covered * tb + int(lens[:s].sum()) * tb for s in range(nshard)] for c in range(max_cp)], np.int64).reshape(max_cp, nshard)
+    mask = np.ones((nshard, max_cp), np.int8)
+    mask[1:2] = 0
+    dev = lambda a: torch.from_numpy(a).to(cuda)
+    buf = torch.randn(max_cp * covered * hidden, device=cuda).to(torch.bfloat16).view(torch.uint8)
+    poison = [torch.full((T, hidden), float("nan"), dtype=torch.bfloat16, device=cuda) for _ in range(4)]   # what the allocator hands out next
+    torch.cuda.synchronize()
+    del poison
+    md = NS(tensor_shape=[NS(recv_shape=(0, hidden)), NS(recv_shape=(max_cp, T, hidden))], kv_replica_mask=dev(mask),
+            recv_memcpy_metadata=[torch.zeros(0, dtype=torch.int64, device=cuda), dev(off), dev(off)],
+            seq_lens=[NS(recv_seqlens=torch.zeros(0, dtype=torch.int64, device=cuda)), NS(recv_seqlens=dev(lens))])
+    print(f"replica sums: {max_cp} replicas of {nshard} shards, {behind} rows behind them", flush=True)
+    _, dk, dv = pre_all2all_layout_transfer_backward(md, torch.bfloat16, buffer=buf)
+    planes = torch.zeros((max_cp, T, hidden), dtype=torch.bfloat16, device=cuda)
+    a2a_memcpy_cp(planes, md.kv_replica_mask, dev(off), dev(lens), False, buffer=buf)
+    torch.cuda.synchronize()
+    assert dk.shape == dv.shape == (T, hidden) and torch.equal(dk, planes.sum(0)) and torch.equal(dv, planes.sum(0))
