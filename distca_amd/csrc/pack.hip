@@ -432,8 +432,10 @@ int add_job(Jobs *jobs, const distca_exchange_job &in, int64_t token_bytes, int 
   if (in.kind == DISTCA_JOB_REPLICA_SUM || in.kind == DISTCA_JOB_COPY_SUM) {
     if (in.dtype != DISTCA_DTYPE_F32 && in.dtype != DISTCA_DTYPE_F16 && in.dtype != DISTCA_DTYPE_BF16)
       return fail(DISTCA_E_UNSUPPORTED, "%s: dtype %lld (only fp32, fp16, bf16)", what, (long long)in.dtype);
-    if (in.kind == DISTCA_JOB_COPY_SUM && (!in.num_copies || !in.copy_start)) return fail(DISTCA_E_INVALID, "%s: null pointer", what);
+    if (in.kind == DISTCA_JOB_COPY_SUM && in.max_copies < 0) return fail(DISTCA_E_INVALID, "%s: negative size", what);
+    if (in.kind == DISTCA_JOB_COPY_SUM && in.max_copies > 0 && (!in.num_copies || !in.copy_start)) return fail(DISTCA_E_INVALID, "%s: null pointer", what);
   }
+  const int64_t kind = in.kind == DISTCA_JOB_COPY_SUM && in.max_copies == 0 ? DISTCA_JOB_PLAIN : in.kind;   // no copies to add up
   const bool whole = in.num_parts == 1 && in.part[0].bytes == token_bytes && in.part[0].pitch == token_bytes;
   if (!whole && in.kind != DISTCA_JOB_PLAIN) return fail(DISTCA_E_INVALID, "%s: replicas and sums take whole tokens", what);
   if (!whole && token_bytes > (1 << 19)) return fail(DISTCA_E_UNSUPPORTED, "%s: tokens of several parts hold at most 512 KiB", what);
@@ -445,7 +447,7 @@ int add_job(Jobs *jobs, const distca_exchange_job &in, int64_t token_bytes, int 
     o.seq_offset = in.seq_offset; o.seq_tokens = in.seq_tokens; o.mask = in.mask;
     o.num_copies = in.num_copies; o.copy_start = in.copy_start;
     o.num_tokens = in.num_tokens; o.token_bytes = token_bytes; o.pitch = pitch;
-    o.kind = (int32_t)in.kind; o.dtype = (int32_t)in.dtype;
+    o.kind = (int32_t)kind; o.dtype = (int32_t)in.dtype;
     o.num_seq = (int32_t)num_seq; o.max_cp = (int32_t)in.max_cp; o.max_copies = (int32_t)in.max_copies;
     o.part_v0 = (uint32_t)(at / 16); o.part_vecs = (uint32_t)(bytes / 16);
     o.magic = o.part_vecs == 1 ? 0u : (uint32_t)(((1ull << 32) + o.part_vecs - 1) / o.part_vecs);

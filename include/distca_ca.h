@@ -128,7 +128,7 @@ int distca_grad_sum(void *data, int dtype, const int32_t *num_copies,
  *   REPLICAS     distca_memcpy_cp with mask = do_shard; one part of token_bytes
  *   REPLICA_SUM  unpacking: row t becomes the sum of its live replicas' rows (in fp32, rounded once); zeros where there
  *                is none, and behind the last shard
- *   COPY_SUM     packing: distca_grad_sum of the shard (the sum stays in the tensor), then PLAIN
+ *   COPY_SUM     packing: distca_grad_sum of the shard (the sum stays in the tensor), then PLAIN; max_copies 0: PLAIN
  * dtype (the two sums) is one of DISTCA_DTYPE_*.  Pointers, pitches, part and token sizes are multiples of 16.
  * Jobs run at the same time: their byte ranges must be disjoint, and so must a COPY_SUM's main shards and copies. */
 #define DISTCA_EXCHANGE_MAX_JOBS 4

@@ -440,3 +440,23 @@ def test_sums_over_no_replicas_are_zeros(cuda, max_cp, nshard, behind):
     a2a_memcpy_cp(planes, md.kv_replica_mask, dev(off), dev(lens), False, buffer=buf)
     torch.cuda.synchronize()
     assert dk.shape == dv.shape == (T, hidden) and torch.equal(dk, planes.sum(0)) and torch.equal(dv, planes.sum(0))
+
+
+def test_gradients_without_copies_are_sent_as_they_are(cuda):
+    """A table of copies without a column (no shard of the step has any): the main shards go out unchanged."""
+    from distca_amd.dispatch import pre_a2a_qkv
+    lens, hidden = [3, 2], 64
+    T, tb = sum(lens), hidden * 2
+    i64 = lambda x: torch.tensor(x, dtype=torch.int64, device=cuda)
+    q, k, v = (torch.randn((T, hidden), device=cuda).to(torch.bfloat16) for _ in range(3))
+    start = np.concatenate([[0], np.cumsum(lens)[:-1]]) * tb
+    offs = [i64(start + i * T * tb) for i in range(3)]
+    buf = torch.full((3 * T * tb,), 0x11, dtype=torch.uint8, device=cuda)
+    copies = (torch.zeros(2, dtype=torch.int32, device=cuda), torch.zeros((2, 0), dtype=torch.int64, device=cuda))
+    lens = i64(lens)
+    print("no copies", flush=True)
+    pre_a2a_qkv(q, k, v, None, lens, lens, *offs, is_fwd=False, kv_grad_copy_shard_mask=torch.tensor([1, 0], dtype=torch.int8, device=cuda),
+                pre_a2a_grad_acc_args=(*copies, lens), buffer=buf)
+    for i, (t, rows) in enumerate(((q, T), (k, 3), (v, 3))):
+        part = buf[i * T * tb:(i + 1) * T * tb].view(T, tb)
+        assert torch.equal(part[:rows], t.view(torch.uint8)[:rows]) and (part[rows:] == 0x11).all()
