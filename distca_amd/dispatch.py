@@ -74,6 +74,13 @@ def _unpacked(buffer, switch_buffer: bool, instance_id) -> None:
         DispatcherWrapper.release(instance_id)
 
 
+def _lengths_of(tokens: Tensor, offset: Tensor) -> Tensor:
+    """The lengths of exactly the shards `offset` places (a plain job alone takes longer arrays, as a2a_memcpy_non_cp does)."""
+    if tokens.shape != offset.shape:
+        raise RuntimeError("seq_tokens must be of shape (num_sequence,)")
+    return tokens
+
+
 def pre_a2a_qkv(
     q: Tensor, k: Tensor, v: Tensor, kv_dispatch_mask: Tensor,
     q_seq_tokens: Tensor, k_seq_tokens: Tensor,
@@ -93,8 +100,9 @@ def pre_a2a_qkv(
         return q, k, v
     if kv_grad_copy_shard_mask is None:
         raise AssertionError("kv grad copy requires a dedup mask.")
-    jobs = [plain_job([q], q_send_buffer_offset, q_seq_tokens)]
+    jobs = [plain_job([q], q_send_buffer_offset, _lengths_of(q_seq_tokens, q_send_buffer_offset))]
     for t, off in ((k, k_send_buffer_offset), (v, v_send_buffer_offset)):
+        _lengths_of(k_seq_tokens, off)
         if pre_a2a_grad_acc_args is None:
             jobs.append(plain_job([t], off, k_seq_tokens, kv_grad_copy_shard_mask))
         else:
@@ -221,8 +229,9 @@ def post_a2a_attn_out_grad_resend_qkv(
         parts = [torch.empty(tuple(shape), dtype=dt, device=dev)
                  for shape, dt in zip((recv_attn_out_shape, recv_attn_out_shape, recv_lse_shape, recv_q_shape), layout.dtypes)]
         source = _transport_buffer(buffer, instance_id, False)
-        exchange([plain_job(parts, q_recv_buffer_offset, q_recv_seq_tokens), plain_job([recv_k], k_recv_buffer_offset, k_recv_seq_tokens),
-                  plain_job([recv_v], v_recv_buffer_offset, k_recv_seq_tokens)], source, False)
+        exchange([plain_job(t, off, _lengths_of(tokens, off))
+                  for t, off, tokens in ((parts, q_recv_buffer_offset, q_recv_seq_tokens), ([recv_k], k_recv_buffer_offset, k_recv_seq_tokens),
+                                         ([recv_v], v_recv_buffer_offset, k_recv_seq_tokens))], source, False)
         _unpacked(buffer, switch_buffer, instance_id)
         d_out, out, lse, q = parts
         return d_out, out, lse, q, recv_k, recv_v

@@ -304,3 +304,17 @@ def test_request_parts_that_are_no_matrices_are_named():
         for send in (pre_a2a_attn_out_grad_resend_qkv, send_attn_out_grad_resend_qkv):
             with pytest.raises(AssertionError, match="every part must be"):
                 send(t, t, bad, t, *none)
+
+
+def test_exchange_steps_take_a_length_for_every_shard_they_place():
+    """The gradients' way out and the request's way in refuse lengths that are not one per shard placed, as the launch of several
+    tensors did."""
+    import torch
+    from distca_amd.dispatch import post_a2a_attn_out_grad_resend_qkv, pre_a2a_qkv
+    t, off, long = torch.zeros((4, 8), dtype=torch.bfloat16), torch.zeros(2, dtype=torch.int64), torch.tensor([2, 2, 0])
+    right, mask, buf = long[:2], torch.ones(2, dtype=torch.int8), torch.zeros(64, dtype=torch.uint8)
+    for q_lens, k_lens in ((long, right), (right, long), (right[:1], right), (right, right[:, None])):
+        with pytest.raises(RuntimeError, match="seq_tokens must be of shape"):
+            pre_a2a_qkv(t, t, t, None, q_lens, k_lens, off, off, off, is_fwd=False, kv_grad_copy_shard_mask=mask, buffer=buf)
+        with pytest.raises(RuntimeError, match="seq_tokens must be of shape"):
+            post_a2a_attn_out_grad_resend_qkv([4, 8], [4, 4], [4, 8], torch.float32, t, t, None, q_lens, k_lens, off, off, off, False, buffer=buf)
