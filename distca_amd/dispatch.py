@@ -107,7 +107,7 @@ def pre_a2a_qkv(
             jobs.append(plain_job([t], off, k_seq_tokens, kv_grad_copy_shard_mask))
         else:
             num_copies, copy_start_id, lens = pre_a2a_grad_acc_args
-            if lens.data_ptr() == k_seq_tokens.data_ptr():
+            if lens.data_ptr() == k_seq_tokens.data_ptr() and lens.shape == k_seq_tokens.shape and lens.stride() == k_seq_tokens.stride():
                 jobs.append(copy_sum_job(t, off, k_seq_tokens, kv_grad_copy_shard_mask, num_copies, copy_start_id))
             else:   # the shards that are summed are not those that are sent
                 pre_a2a_grad_acc(t, num_copies, copy_start_id, lens)

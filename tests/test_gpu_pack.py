@@ -460,3 +460,27 @@ def test_gradients_without_copies_are_sent_as_they_are(cuda):
     for i, (t, rows) in enumerate(((q, T), (k, 3), (v, 3))):
         part = buf[i * T * tb:(i + 1) * T * tb].view(T, tb)
         assert torch.equal(part[:rows], t.view(torch.uint8)[:rows]) and (part[rows:] == 0x11).all()
+
+
+def test_copies_of_the_first_shards_alone(cuda):
+    """Sums over copies for a leading part of the shards that are sent: their lengths are a view of the same memory as the sent shards'
+    and must not be taken for them.  Shard 0 has its copy in shard 2; shards 1 and 2 lie behind the summed ones or have no copies."""
+    from distca_amd.dispatch import pre_a2a_qkv
+    lens, hidden = [3, 2, 3], 64
+    T, tb = sum(lens), hidden * 2
+    dev = lambda x, dt=torch.int64: torch.tensor(x, dtype=dt, device=cuda)
+    g = torch.Generator().manual_seed(2)
+    q, k, v = (torch.randn((T, hidden), generator=g).to(torch.bfloat16) for _ in range(3))
+    start = np.concatenate([[0], np.cumsum(lens)[:-1]]) * tb
+    nc, cs, mask = np.array([1, 0], np.int32), np.array([[5], [0]], np.int64), np.array([1, 1, 0], np.int8)
+    want = [q.clone(), k.clone(), v.clone()]
+    for t in want[1:]:
+        fa2a.grad_sum(t, nc, cs, lens[:2])
+    exp = np.full(3 * T * tb, 0x11, np.uint8)
+    for i, t in enumerate(want):
+        fa2a.copy_non_cp(t.view(torch.uint8).numpy(), exp, start + i * T * tb, lens, mask if i else None, True)
+    d_lens, buf = dev(lens), torch.full((3 * T * tb,), 0x11, dtype=torch.uint8, device=cuda)
+    print("copies of the first shards", flush=True)
+    pre_a2a_qkv(q.to(cuda), k.to(cuda), v.to(cuda), None, d_lens, d_lens, *(dev(start + i * T * tb) for i in range(3)), is_fwd=False,
+                kv_grad_copy_shard_mask=dev(mask, torch.int8), pre_a2a_grad_acc_args=(dev(nc, torch.int32), dev(cs), d_lens[:2]), buffer=buf)
+    assert np.array_equal(buf.cpu().numpy(), exp)
