@@ -355,7 +355,8 @@ void read_job(PyObject *o, distca_exchange_job &j) {
   const Tensor &offset = tensor_arg(f[2], "seq_nvshmem_offset"), &tokens = tensor_arg(f[3], "seq_tokens");
 
   PyObject *parts = f[1];
-  const Py_ssize_t n = PySequence_Fast_GET_SIZE(parts);   // (a list or a tuple: made by the functions beside `exchange`)
+  if (!PyList_Check(parts) && !PyTuple_Check(parts)) type_error(std::string("the parts of a token are a list or a tuple of tensors, not ") + Py_TYPE(parts)->tp_name);
+  const Py_ssize_t n = PySequence_Fast_GET_SIZE(parts);
   if (n < 1 || n > DISTCA_TOKEN_MAX_PARTS) fail("a token has one to " + std::to_string(DISTCA_TOKEN_MAX_PARTS) + " parts");
   int64_t row = 0;
   for (Py_ssize_t i = 0; i < n; ++i) {
@@ -421,13 +422,13 @@ PyObject *py_exchange(PyObject *, PyObject *const *a, Py_ssize_t n) {   // jobs,
   HANDLE_TH_ERRORS
   expect(n, 3, "exchange");
   const Tensor &buffer = tensor_arg(a[1], "buffer");
-  if (!buffer.is_cuda()) fail("tensor buffer must be on CUDA");
   const bool to_buffer = bool_arg(a[2]);
   if (!PyList_Check(a[0]) && !PyTuple_Check(a[0])) type_error("jobs must be a list");
   const Py_ssize_t num = PySequence_Fast_GET_SIZE(a[0]);
   if (num > DISTCA_EXCHANGE_MAX_JOBS) fail("at most " + std::to_string(DISTCA_EXCHANGE_MAX_JOBS) + " jobs per launch");
   distca_exchange_job jobs[DISTCA_EXCHANGE_MAX_JOBS];
   for (Py_ssize_t i = 0; i < num; ++i) read_job(PySequence_Fast_GET_ITEM(a[0], i), jobs[i]);
+  if (!buffer.is_cuda()) fail("tensor buffer must be on CUDA");
   {
     const Unlocked u;
     const OnDevice on(buffer.device());

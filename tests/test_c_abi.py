@@ -318,3 +318,14 @@ def test_exchange_steps_take_a_length_for_every_shard_they_place():
             pre_a2a_qkv(t, t, t, None, q_lens, k_lens, off, off, off, is_fwd=False, kv_grad_copy_shard_mask=mask, buffer=buf)
         with pytest.raises(RuntimeError, match="seq_tokens must be of shape"):
             post_a2a_attn_out_grad_resend_qkv([4, 8], [4, 4], [4, 8], torch.float32, t, t, None, q_lens, k_lens, off, off, off, False, buffer=buf)
+
+
+@pytest.mark.parametrize("parts", ["generator", "dict", "tensor", "number", "set", "none"])
+def test_parts_of_a_job_are_a_list_or_a_tuple(parts):
+    """Anything else that a caller may take for a sequence of tensors is a TypeError, whatever lies in its memory."""
+    import torch
+    from distca_amd.ops import exchange, plain_job
+    t, lens = torch.zeros((2, 8), dtype=torch.bfloat16), torch.tensor([2])
+    given = dict(generator=(x for x in [t]), dict={0: t}, tensor=t, number=3, set={1}, none=None)[parts]
+    with pytest.raises(TypeError, match="list or a tuple"):
+        exchange([plain_job(given, torch.zeros(1, dtype=torch.int64), lens)], torch.zeros(64, dtype=torch.uint8), True)
