@@ -438,6 +438,17 @@ PyObject *py_exchange(PyObject *, PyObject *const *a, Py_ssize_t n) {   // jobs,
   END_HANDLE_TH_ERRORS
 }
 
+// (the current device, the current stream of device `index`, or of the current one for -1, as a raw handle)
+PyObject *py_current_stream(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  expect(n, 1, "current_stream");
+  const int here = c10::hip::current_device();
+  const int64_t index = int_arg(a[0]);
+  void *const stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)(index < 0 ? here : index)).stream();
+  return Py_BuildValue("iK", here, (unsigned long long)reinterpret_cast<uintptr_t>(stream));
+  END_HANDLE_TH_ERRORS
+}
+
 template <typename F>
 constexpr PyCFunction fast(F *f) { return reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)); }
 
@@ -446,6 +457,7 @@ PyMethodDef methods[] = {
     {"varlen_bwd", fast(py_varlen_bwd), METH_FASTCALL, nullptr},
     {"core_attention", fast(py_core_attention), METH_FASTCALL, nullptr},
     {"exchange", fast(py_exchange), METH_FASTCALL, nullptr},
+    {"current_stream", fast(py_current_stream), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Native host side of the attention and exchange calls.", -1, methods,

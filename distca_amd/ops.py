@@ -35,18 +35,15 @@ def _check_dtype(x: torch.Tensor, dtype: torch.dtype, name: str) -> None:
         raise RuntimeError(f"expected scalar type {dtype} but found {x.dtype} for {name}")
 
 
-_current_device = torch._C._cuda_getDevice
-_raw_stream = torch._C._cuda_getCurrentRawStream
-
-
 def on_stream(fn, device: torch.device, *args) -> int:
     """fn(*args, stream) with `device` current and its current stream (as a raw handle: the Stream object torch makes for
     `torch.cuda.current_stream()` and the device guard cost more host time than a launch)."""
-    index = device.index
-    if index is None or index == _current_device():
-        return fn(*args, _raw_stream(_current_device()))
+    index = -1 if device.index is None else device.index
+    here, stream = _lib.host().current_stream(index)
+    if index < 0 or index == here:
+        return fn(*args, stream)
     with torch.cuda.device(index):
-        return fn(*args, _raw_stream(index))
+        return fn(*args, stream)
 
 
 class DispatcherWrapper:

@@ -329,3 +329,10 @@ def test_parts_of_a_job_are_a_list_or_a_tuple(parts):
     given = dict(generator=(x for x in [t]), dict={0: t}, tensor=t, number=3, set={1}, none=None)[parts]
     with pytest.raises(TypeError, match="list or a tuple"):
         exchange([plain_job(given, torch.zeros(1, dtype=torch.int64), lens)], torch.zeros(64, dtype=torch.uint8), True)
+
+
+def test_the_package_names_nothing_private_of_torch():
+    """No underscored attribute of torch's modules in the package's Python files: they come and go between releases."""
+    import pathlib
+    for f in pathlib.Path(ROOT, "distca_amd").rglob("*.py"):
+        assert not re.findall(r"\btorch(?:\.\w+)*\._\w+", f.read_text()), f

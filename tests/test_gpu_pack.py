@@ -484,3 +484,14 @@ def test_copies_of_the_first_shards_alone(cuda):
     pre_a2a_qkv(q.to(cuda), k.to(cuda), v.to(cuda), None, d_lens, d_lens, *(dev(start + i * T * tb) for i in range(3)), is_fwd=False,
                 kv_grad_copy_shard_mask=dev(mask, torch.int8), pre_a2a_grad_acc_args=(dev(nc, torch.int32), dev(cs), d_lens[:2]), buffer=buf)
     assert np.array_equal(buf.cpu().numpy(), exp)
+
+
+def test_launches_go_to_the_current_stream(cuda):
+    """The raw stream the pack calls are handed is torch's current one, the default stream's handle among them."""
+    from distca_amd._lib import host
+    from distca_amd.ops import on_stream
+    side = torch.cuda.Stream()
+    for s in (torch.cuda.current_stream(), side):
+        with torch.cuda.stream(s):
+            assert host().current_stream(cuda.index) == host().current_stream(-1) == (cuda.index, s.cuda_stream)
+            assert on_stream(lambda *a: a, cuda, 1) == (1, s.cuda_stream) == on_stream(lambda *a: a, torch.device("cuda"), 1)
