@@ -345,7 +345,8 @@ const T *data_of(const Tensor &t, const char *name) {
   return t.const_data_ptr<T>();
 }
 
-void read_job(PyObject *o, distca_exchange_job &j) {
+// Fills in the job and returns the device of its first tensor.
+c10::Device read_job(PyObject *o, distca_exchange_job &j) {
   if (!PyTuple_Check(o) || PyTuple_GET_SIZE(o) != 8) type_error("a job is a tuple of eight");
   PyObject *const *f = &PyTuple_GET_ITEM(o, 0);
   j = distca_exchange_job{};
@@ -359,6 +360,7 @@ void read_job(PyObject *o, distca_exchange_job &j) {
   const Py_ssize_t n = PySequence_Fast_GET_SIZE(parts);
   if (n < 1 || n > DISTCA_TOKEN_MAX_PARTS) fail("a token has one to " + std::to_string(DISTCA_TOKEN_MAX_PARTS) + " parts");
   int64_t row = 0;
+  const c10::Device device = tensor_arg(PySequence_Fast_GET_ITEM(parts, 0), "tensor").device();
   for (Py_ssize_t i = 0; i < n; ++i) {
     const Tensor &t = tensor_arg(PySequence_Fast_GET_ITEM(parts, i), "tensor");
     if (!plain) check_tensor(t, 2, "tensor");
@@ -416,6 +418,7 @@ void read_job(PyObject *o, distca_exchange_job &j) {
   }
   j.seq_offset = data_of<int64_t>(offset, "seq_nvshmem_offset");
   j.seq_tokens = data_of<int64_t>(tokens, "seq_tokens");
+  return device;
 }
 
 PyObject *py_exchange(PyObject *, PyObject *const *a, Py_ssize_t n) {   // jobs, buffer, to_buffer
@@ -427,11 +430,16 @@ PyObject *py_exchange(PyObject *, PyObject *const *a, Py_ssize_t n) {   // jobs,
   const Py_ssize_t num = PySequence_Fast_GET_SIZE(a[0]);
   if (num > DISTCA_EXCHANGE_MAX_JOBS) fail("at most " + std::to_string(DISTCA_EXCHANGE_MAX_JOBS) + " jobs per launch");
   distca_exchange_job jobs[DISTCA_EXCHANGE_MAX_JOBS];
-  for (Py_ssize_t i = 0; i < num; ++i) read_job(PySequence_Fast_GET_ITEM(a[0], i), jobs[i]);
+  // the launch goes to the device, and its stream, that made the tensors: the buffer may be another device's memory
+  std::optional<c10::Device> device;
+  for (Py_ssize_t i = 0; i < num; ++i) {
+    const c10::Device d = read_job(PySequence_Fast_GET_ITEM(a[0], i), jobs[i]);
+    if (!device) device = d;
+  }
   if (!buffer.is_cuda()) fail("tensor buffer must be on CUDA");
   {
     const Unlocked u;
-    const OnDevice on(buffer.device());
+    const OnDevice on(device ? *device : buffer.device());
     check_rc(distca_exchange(jobs, (int32_t)num, buffer.data_ptr(), to_buffer, on.stream), "exchange");
   }
   Py_RETURN_NONE;

@@ -495,3 +495,23 @@ def test_launches_go_to_the_current_stream(cuda):
         with torch.cuda.stream(s):
             assert host().current_stream(cuda.index) == host().current_stream(-1) == (cuda.index, s.cuda_stream)
             assert on_stream(lambda *a: a, cuda, 1) == (1, s.cuda_stream) == on_stream(lambda *a: a, torch.device("cuda"), 1)
+
+
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="needs a second GPU")
+def test_packing_into_the_memory_of_another_device(cuda):
+    """A buffer that is another device's memory: the launch is one of the tensors' device and comes behind what made them there."""
+    from distca_amd.dispatch import pre_a2a_qkv
+    if not torch.cuda.can_device_access_peer(0, 1):
+        pytest.skip("no peer access")
+    T, hidden = 4096, 512
+    tb = hidden * 2
+    buf = torch.zeros(3 * T * tb, dtype=torch.uint8, device="cuda:1")
+    buf.copy_(torch.zeros_like(buf, device=cuda))   # (makes the two devices peers)
+    torch.cuda.synchronize(1)
+    i64 = lambda x: torch.tensor(x, dtype=torch.int64, device=cuda)
+    lens, ones = i64([T]), torch.ones((1, 1), dtype=torch.int8, device=cuda)
+    torch.cuda._sleep(20_000_000)
+    q, k, v = (torch.full((T, hidden), x, dtype=torch.bfloat16, device=cuda) for x in (1., 2., 3.))
+    pre_a2a_qkv(q, k, v, ones, lens, lens, i64([0]), i64([[T * tb]]), i64([[2 * T * tb]]), is_fwd=True, buffer=buf)
+    torch.cuda.current_stream(cuda).synchronize()
+    assert torch.equal(buf.view(torch.bfloat16).view(3 * T, hidden).cpu(), torch.cat([q, k, v]).cpu())
