@@ -40,9 +40,6 @@ struct BwdArgs {
   const int32_t *cut, *slot;  // a list with cut blocks: its tables (sched.h, SplitTables)
   uint8_t *partial;           // and the slots of the pieces
 };
-// A piece's slot: the accumulators of a dQ block (256 rows) or of a key block (dK and dV of 256 keys) as they lie
-constexpr int64_t kDqSlotBytes = (int64_t)256 * 128 * 4, kDkdvSlotBytes = 2 * (int64_t)256 * 128 * 4;
-
 
 // The query side of a backward call: where dO, O, lse, q are read and dq is written.
 struct BwdQuerySide {

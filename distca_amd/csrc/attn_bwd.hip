@@ -43,7 +43,7 @@ struct BwdLayout {
 // key blocks whatever `deterministic` says.
 BwdLayout bwd_layout(const distca_ca_params *p, bool shared, bool preferred) {
   BwdLayout w;
-  w.blocks_kv = shared ? bwd_key_blocks_own_rows(p) : bwd_max_items(p) - bwd_split_target(p);
+  w.blocks_kv = shared || preferred ? bwd_key_blocks_own_rows(p) : bwd_max_items(p) - bwd_split_target(p);
   w.blocks_q = dq_max_items(p);
   w.target_kv = preferred ? bwd_split_pieces(p, kSplitPreferredPerCU, kMinPieceWorth) : bwd_split_target(p);
   w.target_q = preferred ? row_split_target(p, w.blocks_q) : 0;
@@ -60,6 +60,11 @@ BwdLayout bwd_layout(const distca_ca_params *p, bool shared, bool preferred) {
   const int64_t kv = split_max_slots(w.blocks_kv, w.target_kv) * kDkdvSlotBytes, q = split_max_slots(w.blocks_q, w.target_q) * kDqSlotBytes;
   w.slots = take((kv > q ? kv : q) * p->num_heads_kv);
   if (preferred && o > w.slots) take(256);   // (so that no call that brought the smallest workspace is taken for one that brought this)
+  if (!preferred && bwd_small_pieces(p)) {
+    const int64_t small = sched_shared_region_bytes(p->num_tasks, bwd_key_blocks_bound(p) + bwd_small_list_pieces(p)) +
+                          sched_region_bytes(p->num_tasks, w.blocks_q) + 2 * align_up((int64_t)p->num_heads_q * p->total_q * 4, 256) + bwd_small_pieces_bytes(p);
+    if (o < small) o = small;
+  }
   w.total = o;
   return w;
 }
@@ -81,8 +86,8 @@ extern "C" int64_t distca_ca_bwd_workspace_bytes(const distca_ca_params *p) {
   if (!p) return fail(DISTCA_E_INVALID, "bwd_workspace_bytes: null params");
   int rc = validate_params(p);
   if (rc) return rc;
-  // the work lists and row statistics, and, when key blocks are cut into pieces (small batches whose caller does not ask for
-  // a deterministic backward), the slots of the pieces
+  // the work lists and row statistics, and, for small batches whose caller does not ask for a deterministic backward, room for
+  // the slots of a few pieces of key blocks
   return bwd_layout(p, false, false).total;
 }
 
@@ -90,8 +95,8 @@ extern "C" int64_t distca_ca_bwd_workspace_preferred_bytes(const distca_ca_param
   if (!p) return fail(DISTCA_E_INVALID, "bwd_workspace_preferred_bytes: null params");
   int rc = validate_params(p);
   if (rc) return rc;
-  const int64_t own = bwd_layout(p, false, true).total, shared = bwd_layout(p, true, true).total;
-  return own > shared ? own : shared;
+  const int64_t own = bwd_layout(p, false, true).total, shared = bwd_layout(p, true, true).total, small = bwd_layout(p, false, false).total;
+  return own > shared ? (own > small ? own : small) : (shared > small ? shared : small);
 }
 
 extern "C" int distca_ca_bwd(const void *dout, const void *q, const void *k, const void *v, const void *out, const float *lse,

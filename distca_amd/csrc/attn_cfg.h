@@ -29,6 +29,8 @@ constexpr int kFwdKV = 64;
 // 32 flattened rows.
 constexpr int kBwdRows = 32;
 constexpr int kBwdKV = 256;
+// A piece's slot: the accumulators of a dQ block (256 rows) or of a key block (dK and dV of 256 keys) as they lie
+constexpr int64_t kDqSlotBytes = (int64_t)kDqRows * kHeadDim * 4, kDkdvSlotBytes = 2 * (int64_t)kBwdKV * kHeadDim * 4;
 
 inline int validate_params(const distca_ca_params *p) {
   if (p->head_dim != kHeadDim) return fail(DISTCA_E_UNSUPPORTED, "head_dim=%d: the kernels are built for head_dim 128 (smaller ones can be zero-padded to it)", p->head_dim);
@@ -98,7 +100,7 @@ inline SchedGeom fwd_geom(const distca_ca_params *p) {
 // Key blocks are cut into pieces (sched.h) when the batch has so few of them that they could not occupy the
 // device twice over.  Returns the number of pieces to aim for per kv head, 0 = no cutting.  A caller that asks for a
 // deterministic backward and brings the smallest workspace gets whole blocks (the same bits either way: pieces are added up in
-// their order).
+// their order), one that does not brings room for a few pieces (bwd_small_pieces_bytes).
 constexpr int kSplitPiecesPerCU = 2;
 // Upper bounds, from host-known sizes, of the number of key blocks = sum over tasks of ceil(Lk / kBwdKV).
 // When every task has its own K/V rows the Lk add up to total_k at most; when tasks read shared rows
@@ -124,7 +126,25 @@ inline int32_t bwd_split_pieces(const distca_ca_params *p, int per_cu, int min_p
   const int64_t all = bwd_key_blocks_bound(p) * ((rows / kBwdRows + p->num_tasks + min_piece) / min_piece);
   return (int32_t)(t < 1 ? 1 : (t < all ? t : all));
 }
-inline int32_t bwd_split_target(const distca_ca_params *p) { return p->deterministic ? 0 : bwd_split_pieces(p, kSplitFewPerCU, kMinPiece); }
+// What the smallest workspace of a small batch with deterministic == 0 holds beside the lists and the row statistics: 8 bytes per
+// stored element of K, which callers with a buffer of their own have always brought (they once were fp32 accumulators of dK and dV).
+inline bool bwd_small_pieces(const distca_ca_params *p) { return !p->deterministic && few_key_blocks(p, kSplitFewPerCU); }
+inline int32_t bwd_small_list_pieces(const distca_ca_params *p) {   // ... and the room its dK/dV list has beside the blocks
+  const int32_t t = kSplitPiecesPerCU * num_compute_units() / p->num_heads_kv;
+  return t > 0 ? t : 1;
+}
+inline int64_t bwd_small_pieces_bytes(const distca_ca_params *p) {
+  return 2 * (((int64_t)p->total_k * p->num_heads_kv * kHeadDim * 4 + 255) / 256 * 256);
+}
+// The pieces aimed for there: as many as leave the slots and tables of the worst case room (the longest blocks of a batch of unequal
+// documents; one document alone has no block of twice the average cost, and stays whole).
+inline int32_t bwd_split_target(const distca_ca_params *p) {
+  if (!bwd_small_pieces(p)) return 0;
+  const int64_t blocks = bwd_key_blocks_bound(p);
+  const int32_t list = bwd_small_list_pieces(p), t = bwd_split_pieces(p, kSplitFewPerCU, kMinPiece);
+  const int64_t slots = (bwd_small_pieces_bytes(p) - split_tables_bytes(blocks, list, blocks + list)) / (kDkdvSlotBytes * p->num_heads_kv);
+  return slots < 2 ? 0 : (int32_t)(slots / 2 < t ? slots / 2 : t);
+}
 // Blocks of query rows are cut into pieces of consecutive KV tiles when the batch has so few of them that the longest one
 // could bound the launch: fewer than kSplitMaxBlocksPerCU blocks per compute unit (above that longest-first dispatch evens
 // them out), and a prefix of more than kCutFromTiles KV tiles (the second launch takes 4.5 us though nothing be cut: 1000 tokens at
@@ -198,8 +218,7 @@ inline int64_t bwd_max_items(const distca_ca_params *p) {
   // Without cutting, items are (task, key block) over rows the task owns, or (group of tasks that share rows, key
   // block): either way the blocks tile stored rows.  With cutting (small batches only) tasks over shared rows have an
   // item per task and key block, and cutting adds at most total cost / piece <= split_target pieces (piece_size rounds up).
-  const int32_t split = bwd_split_target(p);
-  return split > 0 ? bwd_key_blocks_bound(p) + split : bwd_key_blocks_own_rows(p);
+  return bwd_small_pieces(p) ? bwd_key_blocks_bound(p) + bwd_split_target(p) : bwd_key_blocks_own_rows(p);
 }
 // The dK/dV list over groups of tasks that share stored K/V rows: an item's cost is the sum over the group's tasks.
 inline SchedGeom bwd_shared_geom(const distca_ca_params *p) {

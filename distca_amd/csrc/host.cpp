@@ -184,9 +184,14 @@ std::array<Tensor, 3> varlen_bwd(const Batch &b, Tensor dout, Tensor out, Tensor
     fail("softmax_lse must be fp32 of shape [Hq, Tq] = (" + std::to_string(b.q.size(1)) + ", " + std::to_string(b.q.size(0)) + ")");
   lse = lse.contiguous();
   const distca_ca_params p = b.params(deterministic);
-  // (a call over shared K/V rows brings what distca_ca_bwd_workspace_bytes asks for: the same bits as the C ABI's other forms give
-  // with it; the server's tick takes the preferred size)
-  const bool whole = workspace || b.kv_off;
+  // (A call over shared K/V rows brings what distca_ca_bwd_workspace_bytes asks for: the same bits as the C ABI's other forms give with
+  // it; the server's tick takes the preferred size.  A small batch, for which more is asked without the deterministic switch than
+  // with it, is cut into pieces either way, and brings room for all of them.)
+  bool whole = workspace || b.kv_off;
+  if (!workspace && b.kv_off && !deterministic) {
+    const distca_ca_params smallest = b.params(true);
+    whole = distca_ca_bwd_workspace_bytes(&p) == distca_ca_bwd_workspace_bytes(&smallest);
+  }
   const Tensor ws = workspace_of(workspace, whole ? distca_ca_bwd_workspace_bytes(&p) : distca_ca_bwd_workspace_preferred_bytes(&p),
                                  b.q.device(), "ca_varlen_bwd");
   std::array<Tensor, 3> grads{given.dq ? *given.dq : at::empty_like(b.q), given.dk ? *given.dk : at::empty_like(b.k),

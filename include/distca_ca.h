@@ -197,10 +197,11 @@ typedef struct distca_ca_params {
   int32_t causal;       /* 0 / 1                                              */
   int32_t deterministic;/* backward only (the reference's server default,
                            fused_comm_attn.py:95-104).  Two runs give the same
-                           bits either way: there are no float atomics.  1 asks
-                           for the smallest workspace: a batch too small to
-                           occupy the device keeps whole key blocks unless
-                           the caller brings the preferred workspace          */
+                           bits either way: there are no float atomics.  With
+                           the workspace of distca_ca_bwd_workspace_bytes, 1
+                           keeps key blocks whole, 0 (which asks for more)
+                           cuts a few of a batch too small to occupy the
+                           device; with the preferred one it changes nothing  */
   int32_t dtype;        /* element type of q, k, v, out and the gradients:
                            DISTCA_DTYPE_BF16 or DISTCA_DTYPE_F16; 0 (callers
                            written before the field existed) means bf16      */
@@ -209,16 +210,19 @@ typedef struct distca_ca_params {
 /* Size of the workspace an attention call needs (no reference counterpart: flash-attn
  * allocates its own).  The workspace holds the work list the call builds on the device
  * and the counters its workgroups draw their work from (and, in the backward, the row
- * statistics: 8 bytes per query row and head; fp32 dK/dV accumulators only for a small
- * batch with deterministic == 0, whose key blocks are cut into pieces); its contents are rewritten
+ * statistics: 8 bytes per query row and head; and for a small batch with deterministic == 0
+ * 8 bytes per stored element of K, in which the fp32 results of a few pieces of key blocks fit); its contents are rewritten
  * by every call, so calls that may run at the same time on different streams each need
  * a workspace of their own, while calls ordered on one stream can share one.           */
 int64_t distca_ca_fwd_workspace_bytes(const distca_ca_params *p);
 int64_t distca_ca_bwd_workspace_bytes(const distca_ca_params *p);
-/* The size from which a call has room for everything it can use: a batch with fewer blocks of
- * work than the device has room for then has its longest blocks cut into pieces, whose fp32
- * results pass through the workspace and are added up in a fixed order.  Never less than the sizes above, and equal to
- * them for batches that fill the device.  A call decides by the workspace_bytes it is given. */
+/* The size from which a call has room for everything it can use: a batch with fewer than eight blocks per
+ * compute unit (256 query rows x heads per kv head in the forward and for dQ, where also a prefix of more than
+ * 1024 keys is needed; 256 keys x kv heads for dK / dV) may then have its longest blocks cut into pieces, whose fp32
+ * results pass through the workspace and are added up in a fixed order.  The room is that of the most pieces such a
+ * batch can have, up to 4 per compute unit whatever its size: at most 140 MB forward and 275 MB backward beyond the
+ * sizes above on 256 units (4096 tokens: 63 and 140 MB at 4/1 heads, 136 and 177 MB at 32/8).  Never less than the
+ * sizes above, and equal to them for batches that fill the device.  A call decides by the workspace_bytes it is given. */
 int64_t distca_ca_fwd_workspace_preferred_bytes(const distca_ca_params *p);
 int64_t distca_ca_bwd_workspace_preferred_bytes(const distca_ca_params *p);
 
@@ -339,8 +343,7 @@ int distca_ca_bwd_tokens(const void *req_base, const int64_t *req_task_off,
  * send buffer (dk_offset[s] / dv_offset[s] from `dk` / `dv`) instead of into
  * contiguous tensors that a pack pass would copy there (pre_a2a_qkv in backward,
  * attn_kernels/dispatch.py:39-56).  Every stored row is written: rows no task reads
- * as zeros.  Key blocks are never cut into pieces in this form (no float atomics:
- * the result is the same in every run). */
+ * as zeros.  The result is the same in every run, whatever `deterministic` says. */
 int distca_ca_bwd_buffers(const void *req_base, const int64_t *req_task_off,
                           int64_t req_tok_bytes, const void *k, const void *v,
                           const distca_kv_shards *kv_shards, void *dq_base,

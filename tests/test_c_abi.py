@@ -156,8 +156,8 @@ def test_attention_argument_errors_are_reported_before_any_launch():
 
 def test_backward_workspace_is_sized_for_what_the_call_needs():
     """The work lists and the two row statistics, and nothing else, for a batch large enough to occupy the device or a
-    deterministic one: 131072 tokens with 32 query heads need 34 MB.  Only a small batch whose caller allows float
-    atomics (its key blocks are then cut into pieces) also brings the fp32 dK/dV accumulators."""
+    deterministic one: 131072 tokens with 32 query heads need 34 MB.  Only a small batch with deterministic == 0 also
+    brings room for a few pieces of key blocks: 8 bytes per stored element of K."""
     lib = _lib.load()
     big = _p(num_tasks=27, total_q=131072, total_k=131072, num_heads_q=32, num_heads_kv=8, max_seqlen_q=65536, max_seqlen_k=65536)
     n = lib.distca_ca_bwd_workspace_bytes(ctypes.byref(big))
@@ -171,8 +171,34 @@ def test_backward_workspace_is_sized_for_what_the_call_needs():
     pieces = lib.distca_ca_bwd_workspace_bytes(ctypes.byref(small))
     small.deterministic = 1
     whole = lib.distca_ca_bwd_workspace_bytes(ctypes.byref(small))
-    assert pieces - whole >= 2 * 4096 * 8 * 128 * 4          # the two accumulators
+    assert pieces - whole >= 2 * 4096 * 8 * 128 * 4          # 8 bytes per element
     assert whole < 2 * 32 * 4096 * 4 + 1e6
+
+
+@pytest.mark.parametrize("deterministic", [0, 1])
+def test_smallest_workspace_stays_what_fixed_buffers_were_sized_for(deterministic):
+    """Over sizes of every magnitude: lists (16 bytes an item, a few words a task), 8 bytes per query row and head, and with
+    deterministic == 0 at most 8 bytes per stored element of K.  A batch of 4096 tokens: 8.7 MB at 8/2 heads, 34.6 at 32/8, 4.3 at 4/1.
+    The preferred size is never less, and beyond that at most 1024 slots (130 KB forward, 256 KB backward) with their tables."""
+    lib = _lib.load()
+    rng = np.random.default_rng(deterministic)
+    for _ in range(5000):
+        hq, hkv = [(4, 1), (8, 2), (32, 8), (64, 8), (8, 8), (128, 8), (16, 16), (1, 1), (6, 2), (256, 256)][rng.integers(10)]
+        n, tq, tk, mq, mk = (int(2 ** rng.uniform(0, top)) for top in (8, 20, 20, 18, 18))
+        p = _p(num_tasks=n, total_q=tq, total_k=tk, num_heads_q=hq, num_heads_kv=hkv, max_seqlen_q=mq, max_seqlen_k=mk, deterministic=deterministic)
+        fwd, bwd, fwd_more, bwd_more = (int(getattr(lib, f"distca_ca_{d}_workspace_{s}bytes")(ctypes.byref(p))) for s in ("", "preferred_") for d in ("fwd", "bwd"))
+        rows = tq * (hq // hkv) // 256 + n + 1
+        keys = max(tk // 256 + n + 1, (mk // 256 + 1) * n + 1) if not deterministic and (tk // 256 + n + 1) * hkv < 512 else tk // 256 + n + 1
+        per_task, fixed = 8 * 4, 4096
+        assert 0 < fwd <= 16 * rows + per_task * n + fixed
+        more = 8 * tk * hkv * 128 + 16 * 512 if not deterministic and (tk // 256 + n + 1) * hkv < 512 else 0
+        assert 0 < bwd <= 16 * (rows + keys) + 2 * (per_task + 32) * n + 8 * hq * tq + more + 2 * fixed
+        tables = 64 * (rows + keys + 512) + 2 * fixed
+        assert fwd <= fwd_more <= fwd + 1024 * (256 * 128 * 4 + 256 * 8) + tables
+        assert bwd <= bwd_more <= bwd + 1024 * 2 * 256 * 128 * 4 + tables
+    for hq, hkv, mb in ((8, 2, 8.7), (32, 8, 34.6), (4, 1, 4.3)):
+        p = _p(num_tasks=3, total_q=4096, total_k=4096, num_heads_q=hq, num_heads_kv=hkv, max_seqlen_q=2560, max_seqlen_k=2560)
+        assert int(lib.distca_ca_bwd_workspace_bytes(ctypes.byref(p))) <= mb * 1e6 + 1e5
 
 
 def test_python_wrappers_reject_wrong_inputs():

@@ -450,3 +450,32 @@ def test_head_dims_that_are_refused(cuda):
         ca_varlen_fwd(q, q.to(torch.bfloat16), q, c, c, 16, 16)
     with pytest.raises(RuntimeError, match="bfloat16 or float16"):
         ca_varlen_fwd(q.float(), q.float(), q.float(), c, c, 16, 16)
+
+
+@pytest.mark.parametrize("q_lens,hq,hkv", [([3000, 129, 40, 33], 8, 2), ([2000] + [64] * 20, 4, 1), ([2600, 900, 600], 32, 8), ([512], 8, 2), ([4100, 17], 2, 2)])
+@pytest.mark.parametrize("shared", [False, True])
+def test_pieces_within_the_smallest_workspace(cuda, q_lens, hq, hkv, shared):
+    """Without the deterministic switch the smallest workspace has room for a few pieces of key blocks (of the longest document; none
+    where all blocks are alike or too few): nothing is written behind it, nothing is dropped, and dK / dV are the preferred workspace's
+    but for the order of their fp32 sums."""
+    import ctypes
+    from distca_amd._lib import CaParams, load
+    from distca_amd.fused_comm_attn import ca_varlen_bwd, ca_varlen_fwd
+    tq = sum(q_lens)
+    q, k, v, do = (t.to(cuda) for t in make_qkv(tq, tq, hq, hkv, 128, 61))
+    c, off = torch.tensor(cu(q_lens), device=cuda), torch.tensor(cu(q_lens)[:-1], device=cuda) if shared else None
+    n = max(q_lens)
+    out, lse = ca_varlen_fwd(q, k, v, c, c, n, n, kv_task_offsets=off)
+    p = CaParams(len(q_lens), tq, tq, hq, hkv, 128, n, n, 128 ** -0.5, 1, 0, 0)
+    need = int(load().distca_ca_bwd_workspace_bytes(ctypes.byref(p)))
+    ws = torch.full((need + 65536,), 0x5A, dtype=torch.uint8, device=cuda)
+    print(f"smallest workspace {need} B, tasks {q_lens} heads {hq}/{hkv} shared={shared}", flush=True)
+    few = ca_varlen_bwd(do, q, k, v, out, lse, c, c, n, n, kv_task_offsets=off, workspace=ws[:need])
+    many = ca_varlen_bwd(do, q, k, v, out, lse, c, c, n, n, kv_task_offsets=off)
+    torch.cuda.synchronize()
+    assert (ws[need:] == 0x5A).all()
+    assert int(ws[:16].view(torch.int32)[2]) == 0
+    for x, y, name in zip(few, many, ("dq", "dk", "dv")):
+        # the bound of test_blocks_cut_into_pieces: the same P and dS, added up in fp32 in another order, then rounded to bf16
+        x, y = x.float(), y.float()
+        assert ((x - y).abs() <= 2.0 ** -7 * y.abs() + n ** 1.5 / 16 * 2.0 ** -24 * y.abs().max()).all(), name
