@@ -124,12 +124,22 @@ struct Batch {
   Batch padded() const { return {pad(q), pad(k), pad(v), cu_q, cu_k, kv_off, max_q, max_k, scale_or_default(), causal}; }
 };
 
-Tensor workspace_of(const OptTensor &given, int64_t need, c10::Device device, const char *what) {
-  if (need < 0) check_rc(need, what);
-  if (!given) return at::empty({need > 16 ? need : 16}, at::TensorOptions().dtype(at::kByte).device(device));
-  if (given->scalar_type() != at::kByte || !given->is_cuda() || !given->is_contiguous() || given->numel() < need)
-    fail("workspace must be a contiguous uint8 CUDA tensor of at least " + std::to_string(need) + " bytes");
-  return *given;
+// The caller's workspace, of at least `least` bytes, or one of `size`, or of `least` where the device has no memory left for that.
+Tensor workspace_of(const OptTensor &given, int64_t least, int64_t size, c10::Device device, const char *what) {
+  if (least < 0) check_rc(least, what);
+  if (given) {
+    if (given->scalar_type() != at::kByte || !given->is_cuda() || !given->is_contiguous() || given->numel() < least)
+      fail("workspace must be a contiguous uint8 CUDA tensor of at least " + std::to_string(least) + " bytes");
+    return *given;
+  }
+  auto empty = [&](int64_t n) { return at::empty({n > 16 ? n : 16}, at::TensorOptions().dtype(at::kByte).device(device)); };
+  if (size > least) {
+    try {
+      return empty(size);
+    } catch (const c10::OutOfMemoryError &) {
+    }
+  }
+  return empty(least);
 }
 
 std::pair<Tensor, Tensor> varlen_fwd(const Batch &b, const OptTensor &workspace) {
@@ -140,8 +150,7 @@ std::pair<Tensor, Tensor> varlen_fwd(const Batch &b, const OptTensor &workspace)
     return {out.narrow(2, 0, d).contiguous(), lse};
   }
   const distca_ca_params p = b.params(false);
-  const int64_t need = workspace ? distca_ca_fwd_workspace_bytes(&p) : distca_ca_fwd_workspace_preferred_bytes(&p);
-  const Tensor ws = workspace_of(workspace, need, b.q.device(), "ca_varlen_fwd");
+  const Tensor ws = workspace_of(workspace, distca_ca_fwd_workspace_bytes(&p), distca_ca_fwd_workspace_preferred_bytes(&p), b.q.device(), "ca_varlen_fwd");
   Tensor out = at::empty_like(b.q);
   Tensor lse = at::empty({b.q.size(1), b.q.size(0)}, b.q.options().dtype(at::kFloat));
   const OnDevice on(b.q.device());
@@ -187,13 +196,13 @@ std::array<Tensor, 3> varlen_bwd(const Batch &b, Tensor dout, Tensor out, Tensor
   // (A call over shared K/V rows brings what distca_ca_bwd_workspace_bytes asks for: the same bits as the C ABI's other forms give with
   // it; the server's tick takes the preferred size.  A small batch, for which more is asked without the deterministic switch than
   // with it, is cut into pieces either way, and brings room for all of them.)
-  bool whole = workspace || b.kv_off;
-  if (!workspace && b.kv_off && !deterministic) {
+  const int64_t least = distca_ca_bwd_workspace_bytes(&p);
+  bool whole = b.kv_off.has_value();
+  if (whole && !deterministic) {
     const distca_ca_params smallest = b.params(true);
-    whole = distca_ca_bwd_workspace_bytes(&p) == distca_ca_bwd_workspace_bytes(&smallest);
+    whole = least == distca_ca_bwd_workspace_bytes(&smallest);
   }
-  const Tensor ws = workspace_of(workspace, whole ? distca_ca_bwd_workspace_bytes(&p) : distca_ca_bwd_workspace_preferred_bytes(&p),
-                                 b.q.device(), "ca_varlen_bwd");
+  const Tensor ws = workspace_of(workspace, least, whole ? least : distca_ca_bwd_workspace_preferred_bytes(&p), b.q.device(), "ca_varlen_bwd");
   std::array<Tensor, 3> grads{given.dq ? *given.dq : at::empty_like(b.q), given.dk ? *given.dk : at::empty_like(b.k),
                               given.dv ? *given.dv : at::empty_like(b.v)};
   const struct { const char *name; const Tensor &of; } like[] = {{"dq", b.q}, {"dk", b.k}, {"dv", b.v}};

@@ -73,12 +73,18 @@ def _params(num_tasks, total_q, total_k, hq, hkv, d, max_q, max_k, scale, causal
                          1 if causal else 0, 1 if deterministic else 0, _ELEM_CODE[dtype])
 
 
-def _workspace(given: Optional[Tensor], need: int, device) -> Tensor:
-    if given is None:
-        return torch.empty((max(need, 16),), dtype=torch.uint8, device=device)
-    if given.dtype != torch.uint8 or not given.is_cuda or not given.is_contiguous() or given.numel() < need:
-        raise RuntimeError(f"workspace must be a contiguous uint8 CUDA tensor of at least {need} bytes")
-    return given
+def _workspace(direction: str, p: _lib.CaParams, device, what: str) -> Tensor:
+    """The workspace a server's tick brings: of the preferred size, or of the smallest where the device has no memory left for that."""
+    lib = _lib.load()
+    for size in ("preferred_", ""):
+        need = getattr(lib, f"distca_ca_{direction}_workspace_{size}bytes")(ctypes.byref(p))
+        if need < 0:
+            _lib.check(int(need), what)
+        try:
+            return torch.empty((max(int(need), 16),), dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            if not size:
+                raise
 
 
 def ca_varlen_fwd(q: Tensor, k: Tensor, v: Tensor, cu_seqlens_q: Tensor, cu_seqlens_k: Tensor,
@@ -256,10 +262,7 @@ def ca_server_forward(recv_buffer: Tensor, send_buffer: Tensor, meta: ServerFwdM
         assert fa_args.causal and fa_args.window_size == (-1, -1) and fa_args.dropout_p == 0.0
         p = _params(cu_q.shape[0] - 1, tq, tk, hq, hkv, d, fa_params.max_seqlen_q, fa_params.max_seqlen_kv, scale,
                     fa_args.causal, False, dtype)
-        need = lib.distca_ca_fwd_workspace_preferred_bytes(ctypes.byref(p))
-        if need < 0:
-            _lib.check(int(need), "ca_server_forward")
-        ws = _workspace(None, int(need), dev)
+        ws = _workspace("fwd", p, dev, "ca_server_forward")
         q_tok = hq * d * 2
         out_tok = size_pad_by_int4(q_tok + hq * 4, 1)[0]
         for name, t in (("q_recv_offset", meta.q_recv_offset), ("out_send_offset", meta.out_send_offset)):
@@ -343,10 +346,7 @@ With that layout and `kv_shards_in_place` (the default) the kernels also read th
         lib = _lib.load()
         p = _params(cu_seqlens_q.shape[0] - 1, tq, int(k_rows), hq, hkv, d, max_seqlen_q, max_seqlen_kv, scale, fa_args.causal,
                     fa_args.deterministic, dtype)
-        need = lib.distca_ca_bwd_workspace_preferred_bytes(ctypes.byref(p))
-        if need < 0:
-            _lib.check(int(need), "ca_server_backward")
-        ws = _workspace(None, int(need), dev)
+        ws = _workspace("bwd", p, dev, "ca_server_backward")
         row = hq * d * 2
         req_tok = size_pad_by_int4(3 * row + hq * 4, 1)[0]
         for name, t in (("q_recv_offset", meta.q_recv_offset), ("q_grad_send_offset", meta.q_grad_send_offset)):
@@ -375,10 +375,7 @@ With that layout and `kv_shards_in_place` (the default) the kernels also read th
         lib = _lib.load()
         p = _params(cu_seqlens_q.shape[0] - 1, tq, tk, hq, hkv, d, max_seqlen_q, max_seqlen_kv, scale, fa_args.causal,
                     fa_args.deterministic, dtype)
-        need = lib.distca_ca_bwd_workspace_preferred_bytes(ctypes.byref(p))
-        if need < 0:
-            _lib.check(int(need), "ca_server_backward")
-        ws = _workspace(None, int(need), dev)
+        ws = _workspace("bwd", p, dev, "ca_server_backward")
         row = hq * d * 2
         req_tok = size_pad_by_int4(3 * row + hq * 4, 1)[0]
         for name, t in (("q_recv_offset", meta.q_recv_offset), ("q_grad_send_offset", meta.q_grad_send_offset)):

@@ -479,3 +479,35 @@ def test_pieces_within_the_smallest_workspace(cuda, q_lens, hq, hkv, shared):
         # the bound of test_blocks_cut_into_pieces: the same P and dS, added up in fp32 in another order, then rounded to bf16
         x, y = x.float(), y.float()
         assert ((x - y).abs() <= 2.0 ** -7 * y.abs() + n ** 1.5 / 16 * 2.0 ** -24 * y.abs().max()).all(), name
+
+
+def test_small_batches_where_memory_is_short(cuda):
+    """A batch whose preferred workspace does not fit any more: the smallest is taken, and the results are those of calls that bring it."""
+    import ctypes
+    from distca_amd._lib import CaParams, load
+    from distca_amd.fused_comm_attn import _workspace, ca_varlen_bwd, ca_varlen_fwd, core_attention
+    n, hq, hkv = 4096, 8, 2
+    q, k, v, do = (t.to(cuda) for t in make_qkv(n, n, hq, hkv, 128, 63))
+    c = torch.tensor(cu([n]), device=cuda)
+    p = CaParams(1, n, n, hq, hkv, 128, n, n, 128 ** -0.5, 1, 1, 0)
+    size = lambda name: int(getattr(load(), name)(ctypes.byref(p)))
+    least = [size(f"distca_ca_{d}_workspace_bytes") for d in ("fwd", "bwd")]
+    assert min(size(f"distca_ca_{d}_workspace_preferred_bytes") for d in ("fwd", "bwd")) > 80e6
+    small = [torch.empty(b, dtype=torch.uint8, device=cuda) for b in least]
+    out, lse = ca_varlen_fwd(q, k, v, c, c, n, n, workspace=small[0])
+    want = (out,) + tuple(ca_varlen_bwd(do, q, k, v, out, lse, c, c, n, n, deterministic=True, workspace=small[1]))
+    for t in (q, k, v):
+        t.requires_grad_(True)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    print("memory capped at 64 MB beyond what is held", flush=True)
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (64 << 20)) / torch.cuda.mem_get_info()[1])
+    try:
+        ticks = [_workspace(d, p, cuda, "tick").numel() for d in ("fwd", "bwd")]
+        got = core_attention(q, k, v, c, c, n, n, deterministic=True)
+        got = (got,) + torch.autograd.grad(got, (q, k, v), do)
+        torch.cuda.synchronize()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert ticks == least
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
