@@ -45,7 +45,7 @@ BwdLayout bwd_layout(const distca_ca_params *p, bool shared, bool preferred) {
   BwdLayout w;
   w.blocks_kv = shared || preferred ? bwd_key_blocks_own_rows(p) : bwd_max_items(p) - bwd_split_target(p);
   w.blocks_q = dq_max_items(p);
-  w.target_kv = preferred ? bwd_split_pieces(p, kSplitPreferredPerCU, kMinPieceWorth) : bwd_split_target(p);
+  w.target_kv = preferred ? preferred_key_pieces(p) : bwd_split_target(p);
   w.target_q = preferred ? row_split_target(p, w.blocks_q) : 0;
   w.items_kv = w.blocks_kv + w.target_kv;
   w.items_q = w.blocks_q + w.target_q;
@@ -206,12 +206,9 @@ int DISTCA_FN(run_bwd)(const BwdQuerySide &qs, const void *k, const void *v, voi
   // ---- both work lists, and zeros where no work item writes dk / dv
   const bool few_q = few_row_blocks(p), few_kv = few_key_blocks(p, kSplitFewPerCU) || w.target_kv > 0;
   auto tables_of = [&](int64_t at, int64_t blocks, int32_t target) { return target > 0 ? split_tables(ws + at, blocks, target) : SplitTables{}; };
-  ListJob q_list{cu_q, cu_k, launched_geom(dq_geom(p), p), (int32_t *)(ws + w.sched_q), w.items_q, tables_of(w.tables_q, w.blocks_q, w.target_q)};
-  if (w.target_q > 0) cut_where_worth(&q_list.geom, p, w.target_q, 6, 3, 6);
-  ListJob kv_list{cu_q, cu_k, shared ? bwd_shared_geom(p) : bwd_geom(p), (int32_t *)(ws + w.sched_kv), w.items_kv, tables_of(w.tables_kv, w.blocks_kv, w.target_kv)};
-  kv_list.geom.split_target = w.target_kv;
-  if (w.target_kv > 0 && preferred) cut_where_worth(&kv_list.geom, p, w.target_kv, 9, 14, 4);
-  if (shared && w.target_kv > 0) kv_list.geom.walk_round = 0;   // pieces count a group's visits downwards
+  const ListJob q_list{cu_q, cu_k, launched_dq_geom(p, w.target_q), (int32_t *)(ws + w.sched_q), w.items_q, tables_of(w.tables_q, w.blocks_q, w.target_q)};
+  const ListJob kv_list{cu_q, cu_k, launched_dkdv_geom(p, w.target_kv, preferred, shared), (int32_t *)(ws + w.sched_kv), w.items_kv,
+                        tables_of(w.tables_kv, w.blocks_kv, w.target_kv)};
   rc = launch_build_backward(kv_list, q_list, kv_off, p->num_tasks, BwdFill{(uint8_t *)dk, (uint8_t *)dv, (int64_t)p->num_heads_kv * kHeadDim * 2, p->total_k, shards}, s);
   if (rc) return rc;
 

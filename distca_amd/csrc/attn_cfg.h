@@ -126,6 +126,7 @@ inline int32_t bwd_split_pieces(const distca_ca_params *p, int per_cu, int min_p
   const int64_t all = bwd_key_blocks_bound(p) * ((rows / kBwdRows + p->num_tasks + min_piece) / min_piece);
   return (int32_t)(t < 1 ? 1 : (t < all ? t : all));
 }
+inline int32_t preferred_key_pieces(const distca_ca_params *p) { return bwd_split_pieces(p, kSplitPreferredPerCU, kMinPieceWorth); }
 // What the smallest workspace of a small batch with deterministic == 0 holds beside the lists and the row statistics: 8 bytes per
 // stored element of K, which callers with a buffer of their own have always brought (they once were fp32 accumulators of dK and dV).
 inline bool bwd_small_pieces(const distca_ca_params *p) { return !p->deterministic && few_key_blocks(p, kSplitFewPerCU); }
@@ -203,6 +204,26 @@ inline SchedGeom bwd_geom(const distca_ca_params *p) {
   g.units_per_head = g.item_cost = g.piece_extra = g.add_cost = 0;
   // one round of the dK/dV list per kv head: as many items as compute units serve that head (sched.h, kWalkUp)
   g.walk_round = num_compute_units() / p->num_heads_kv > 0 ? num_compute_units() / p->num_heads_kv : 1;
+  return g;
+}
+// The lists as the calls launch them.  `target`: pieces aimed for per kv head, 0: whole blocks; for dK/dV also whether they are what
+// the preferred workspace has room for (only what is worth it, at one size) or the smallest (equal parts).
+inline SchedGeom launched_fwd_geom(const distca_ca_params *p, int32_t target) {
+  SchedGeom g = launched_geom(fwd_geom(p), p);
+  if (target > 0) cut_where_worth(&g, p, target, 6, 4, 8);
+  return g;
+}
+inline SchedGeom launched_dq_geom(const distca_ca_params *p, int32_t target) {
+  SchedGeom g = launched_geom(dq_geom(p), p);
+  if (target > 0) cut_where_worth(&g, p, target, 6, 3, 6);
+  return g;
+}
+inline SchedGeom bwd_shared_geom(const distca_ca_params *p);
+inline SchedGeom launched_dkdv_geom(const distca_ca_params *p, int32_t target, bool preferred, bool shared) {
+  SchedGeom g = shared ? bwd_shared_geom(p) : bwd_geom(p);
+  g.split_target = target;
+  if (target > 0 && preferred) cut_where_worth(&g, p, target, 9, 14, 4);
+  if (shared && target > 0) g.walk_round = 0;   // pieces count a group's visits downwards
   return g;
 }
 // Upper bound of the item count that needs only host-known sizes.

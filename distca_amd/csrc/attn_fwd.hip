@@ -859,12 +859,11 @@ int DISTCA_FN(run_fwd_tokens)(const void *q_base, const int64_t *q_task_off, int
   if (!workspace || workspace_bytes < need) return fail(DISTCA_E_WORKSPACE, "ca_fwd: workspace %lld B < required %lld B", (long long)workspace_bytes, (long long)need);
   if (!aligned16(workspace)) return fail(DISTCA_E_INVALID, "ca_fwd: workspace must be 16-byte aligned");
   hipStream_t s = (hipStream_t)stream;
-  SchedGeom geom = launched_geom(fwd_geom(p), p);
   FwdLayout lay = fwd_layout(p, true);
   if (lay.target > 0 && workspace_bytes < lay.total) lay = fwd_layout(p, false);   // no room for pieces
   const int64_t max_items = lay.max_items;
   const bool split = lay.target > 0, few = few_row_blocks(p);
-  if (split) cut_where_worth(&geom, p, lay.target, 6, 4, 8);
+  const SchedGeom geom = launched_fwd_geom(p, lay.target);
   const SplitTables tables = split ? split_tables((uint8_t *)workspace + lay.tables, lay.max_blocks, lay.target) : SplitTables{};
   // A batch whose blocks all run at once (one workgroup a compute unit) and stay whole needs no list: which workgroup has which block
   // does not matter then, and finding one by a scan of the task bounds takes one trip to memory where the list takes a launch of 5 us.

@@ -135,6 +135,17 @@ DISTCA_HD float pieces_time(const SchedGeom &g, float total_cost, int32_t n, int
   return load + piece * (total_cost * per_unit / (float)s) + 0.25f * (float)s + (float)(g.piece_extra + g.add_cost);
 }
 constexpr float kWorthCutting = 0.93f;   // cut when the pieces' time is below this share of the whole blocks'
+// The size chosen, 0: blocks stay whole (the host mirror; the builder tries the sizes in as many lanes).
+inline int32_t fixed_piece_size(const SchedGeom &g, unsigned long long total_cost, int32_t n, const int32_t c[4], int32_t least) {
+  float best = 0.f;
+  int32_t size = 0;
+  for (int m = 1; m <= kPieceTries; ++m) {
+    int32_t s;
+    const float t = pieces_time(g, (float)total_cost, n, c[0], least, m, &s);
+    if (size == 0 || t < best || (t == best && s > size)) best = t, size = s;
+  }
+  return best < kWorthCutting * whole_time(g, (float)total_cost, n, c) ? size : 0;
+}
 
 constexpr int kSchedBins = 4096;
 

@@ -529,6 +529,20 @@ int launch_build_backward(const ListJob &kv, const ListJob &q, const int32_t *kv
 
 using namespace distca;
 
+namespace {
+// The list of kind 0 (forward), 1 (dK/dV) or 2 (dQ) that a call with the preferred workspace launches over rows that tasks own.
+struct LaunchedList {
+  SchedGeom geom;
+  int64_t max_blocks;
+};
+LaunchedList launched_list(int kind, const distca_ca_params *p) {
+  if (kind == 1) return {launched_dkdv_geom(p, preferred_key_pieces(p), true, false), bwd_key_blocks_own_rows(p)};
+  const int64_t blocks = kind == 0 ? fwd_max_items(p) : dq_max_items(p);
+  const int32_t target = row_split_target(p, blocks);
+  return {kind == 0 ? launched_fwd_geom(p, target) : launched_dq_geom(p, target), blocks};
+}
+}  // namespace
+
 extern "C" int distca_ca_tile_shape(int kind, const distca_ca_params *p, int32_t out[2]) {
   if (!p || !out) return fail(DISTCA_E_INVALID, "tile_shape: null pointer");
   int rc = validate_params(p);
@@ -546,7 +560,11 @@ extern "C" int64_t distca_ca_schedule_capacity(int kind, const distca_ca_params 
   if (kind == 0) return fwd_max_items(p);
   if (kind == 1) return bwd_max_items(p);
   if (kind == 2) return dq_max_items(p);
-  return fail(DISTCA_E_INVALID, "schedule_capacity: kind must be 0 (fwd), 1 (bwd dK/dV) or 2 (bwd dQ)");
+  if (kind >= DISTCA_SCHED_LAUNCHED && kind <= DISTCA_SCHED_LAUNCHED + 2) {
+    const LaunchedList l = launched_list(kind - DISTCA_SCHED_LAUNCHED, p);
+    return l.max_blocks + l.geom.split_target;
+  }
+  return fail(DISTCA_E_INVALID, "schedule_capacity: kind must be 0 (fwd), 1 (bwd dK/dV) or 2 (bwd dQ), or one of these + %d", DISTCA_SCHED_LAUNCHED);
 }
 
 extern "C" int64_t distca_ca_schedule_host(int kind, const int32_t *cu_q, const int32_t *cu_k, const distca_ca_params *p,
@@ -554,31 +572,48 @@ extern "C" int64_t distca_ca_schedule_host(int kind, const int32_t *cu_q, const 
   if (!p || !cu_q || !cu_k || (!items && max_items > 0)) return fail(DISTCA_E_INVALID, "schedule_host: null pointer");
   int rc = validate_params(p);
   if (rc) return rc;
-  if (kind != 0 && kind != 1) return fail(DISTCA_E_INVALID, "schedule_host: kind must be 0 (fwd) or 1 (bwd)");
-  const SchedGeom g = kind == 0 ? fwd_geom(p) : bwd_geom(p);
+  const bool launched = kind >= DISTCA_SCHED_LAUNCHED;
+  if (kind != 0 && kind != 1 && !(launched && kind <= DISTCA_SCHED_LAUNCHED + 2))
+    return fail(DISTCA_E_INVALID, "schedule_host: kind must be 0 (fwd) or 1 (bwd), or 0 to 2 + %d", DISTCA_SCHED_LAUNCHED);
+  if (launched) kind -= DISTCA_SCHED_LAUNCHED;
+  const LaunchedList list = launched ? launched_list(kind, p) : LaunchedList{kind == 0 ? fwd_geom(p) : bwd_geom(p), 0};
+  const SchedGeom &g = list.geom;
   struct It { int32_t task, block, cost, bin, piece; };
   std::vector<It> whole, v;
   unsigned long long total_cost = 0;
   for (int32_t b = 0; b < p->num_tasks; ++b) {
     const int32_t lq = cu_q[b + 1] - cu_q[b], lk = cu_k[b + 1] - cu_k[b];
-    const int32_t n = kind == 0 ? fwd_num_items(g, lq, lk) : bwd_num_blocks(g, lq, lk);
+    const int32_t n = kind == 1 ? bwd_num_blocks(g, lq, lk) : fwd_num_items(g, lq, lk);
     for (int32_t i = 0; i < n; ++i) {
-      const int32_t c = kind == 0 ? fwd_item_cost(g, lq, lk, i) : bwd_cost(g, lq, lk, i);
+      const int32_t c = kind == 1 ? bwd_cost(g, lq, lk, i) : fwd_item_cost(g, lq, lk, i);
       whole.push_back({b, i, c, 0, 0});
       total_cost += (unsigned long long)c;
     }
   }
   int32_t piece = 0;
-  if (kind == 1 && g.split_target > 0) {
-    piece = piece_size(total_cost, g.split_target, g.min_piece);
+  if (g.split_target > 0) piece = piece_size(total_cost, g.split_target, g.min_piece);
+  const bool fixed = g.units_per_head > 0;
+  if (fixed) {
+    std::vector<int32_t> bins;
+    for (const It &w : whole) bins.push_back(cost_bin(g, w.cost));
+    std::sort(bins.begin(), bins.end(), [](int32_t a, int32_t b) { return a > b; });
+    int32_t ranked[4];
+    for (int k = 0; k < 4; ++k) ranked[k] = (size_t)k * g.units_per_head < bins.size() ? bins[(size_t)k * g.units_per_head] << g.cost_shift : 0;
+    piece = fixed_piece_size(g, total_cost, (int32_t)whole.size(), ranked, piece);
   }
+  int64_t cut = 0, slots = 0;
   for (const It &w : whole) {
-    const int32_t k = piece_count(w.cost, piece);
+    const int32_t k = fixed ? fixed_piece_count(w.cost, piece) : piece_count(w.cost, piece);
+    if (k > 1) ++cut, slots += k;
     for (int32_t j = 0; j < k; ++j) {
-      const int32_t cj = piece_begin(w.cost, j + 1, k) - piece_begin(w.cost, j, k);
-      v.push_back({w.task, w.block, cj, cost_bin(g, cj), j | (k << 16)});
+      int32_t lo, hi;
+      piece_range(w.cost, j, k, fixed ? piece : 0, &lo, &hi);
+      v.push_back({w.task, w.block, hi - lo, cost_bin(g, hi - lo), j | (k << 16)});
     }
   }
+  if (launched && (cut > split_max_cut(list.max_blocks, g.split_target) || slots > split_max_slots(list.max_blocks, g.split_target)))
+    return fail(DISTCA_E_WORKSPACE, "schedule_host: %lld blocks cut into %lld pieces, room for %lld into %lld", (long long)cut, (long long)slots,
+                (long long)split_max_cut(list.max_blocks, g.split_target), (long long)split_max_slots(list.max_blocks, g.split_target));
   std::stable_sort(v.begin(), v.end(), [](const It &a, const It &b) { return a.bin > b.bin; });
   const int64_t n = (int64_t)v.size();
   if (kind == 1 && g.walk_round > 0)

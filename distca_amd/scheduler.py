@@ -15,6 +15,7 @@ import numpy as np
 from . import _lib
 
 FWD, BWD = 0, 1
+LAUNCHED = 4   # added to FWD, BWD or DQ: the list as a call with the preferred workspace launches it (blocks merged and cut as it does)
 
 
 def _params(cu_q, cu_k, hq, hkv, d, causal, deterministic=False) -> _lib.CaParams:
@@ -34,7 +35,7 @@ def tile_shape(kind: int, hq: int, hkv: int, d: int = 128) -> Tuple[int, int]:
     return int(out[0]), int(out[1])
 
 
-DQ = 2  # a third list kind for capacity queries: the dQ kernel's blocks of query rows
+DQ = 2  # a third list kind, for capacity queries and with LAUNCHED: the dQ kernel's blocks of query rows
 
 
 def schedule_capacity(kind: int, cu_seqlens_q: Sequence[int], cu_seqlens_k: Sequence[int], num_heads_q: int,
@@ -57,8 +58,9 @@ def build_schedule(kind: int, cu_seqlens_q: Sequence[int], cu_seqlens_k: Sequenc
                    total_k: int | None = None) -> np.ndarray:
     """Work items as an int32 array [n, 4] of (task, block, cost, piece | pieces << 16), most expensive
     first; in a backward list bit 31 of the fourth word (WALK_UP) marks items walked upwards from the diagonal
-    (`item_piece`, `item_pieces` take the word apart).  Backward items of a batch too small to occupy the device are cut into pieces of
-    consecutive query blocks unless `deterministic`; everything else has pieces = 1, piece = 0."""
+    (`item_piece`, `item_pieces` take the word apart).  The longest backward items of a batch too small to occupy the device are cut into
+    pieces of consecutive query blocks unless `deterministic`, as the smallest workspace has room for them; with LAUNCHED, blocks of any
+    kind are where that is worth it; everything else has pieces = 1, piece = 0."""
     cu_q = np.ascontiguousarray(cu_seqlens_q, dtype=np.int32)
     cu_k = np.ascontiguousarray(cu_seqlens_k, dtype=np.int32)
     p = _params(cu_q, cu_k, num_heads_q, num_heads_kv, head_dim, causal, deterministic)

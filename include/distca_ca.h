@@ -361,8 +361,14 @@ int distca_ca_bwd_buffers(const void *req_base, const int64_t *req_task_off,
  * kind 0 = forward (one item per (task, block of query rows), cost = KV tiles
  * visible to the block), 1 = backward (one item per (task, KV block), cost =
  * query blocks that see it; when the batch has too few key blocks to occupy
- * the device and p->deterministic is 0, a key block is cut into pieces of
- * consecutive query blocks, whose dK/dV the kernel adds up in fp32).  Writes
+ * the device and p->deterministic is 0, the longest key blocks are cut into pieces of
+ * consecutive query blocks, whose dK/dV are added up in fp32, as many as the workspace
+ * of distca_ca_bwd_workspace_bytes has room for); kind 0 is made without the least batch that
+ * blocks are merged from.  DISTCA_SCHED_LAUNCHED + 0, 1 or 2 (dQ): the list that a call with the
+ * preferred workspace launches over rows that tasks own, with blocks merged and cut as it does
+ * (a forward whose whole blocks all run at once takes these without a list); the time model that
+ * decides on cutting runs in floats on either side.  Fails with DISTCA_E_WORKSPACE should the
+ * pieces outnumber their slots.  Writes
  * up to max_items (task, block, cost, piece | pieces << 16) quadruples sorted
  * by descending cost and returns the item count, or a negative error.  In a
  * backward list bit 31 of the fourth word marks the items whose query blocks
@@ -372,12 +378,13 @@ int distca_ca_bwd_buffers(const void *req_base, const int64_t *req_task_off,
  * 0xffff, pieces = (word >> 16) & 0x7fff.  The reference has no counterpart: flash-attn launches a static
  * (m-block, batch, head) grid sized by max_seqlen_q.
  * ------------------------------------------------------------------------- */
+#define DISTCA_SCHED_LAUNCHED 4
 int64_t distca_ca_schedule_host(int kind, const int32_t *cu_seqlens_q,
                                 const int32_t *cu_seqlens_k,
                                 const distca_ca_params *p, int32_t *items,
                                 int64_t max_items);
-/* Number of work items the list of `kind` (0 forward, 1 backward dK/dV, 2 backward dQ)
- * has room for inside the workspace, computed from the sizes in p alone.  The device
+/* Number of work items the list of `kind` (0 forward, 1 backward dK/dV, 2 backward dQ; the preferred
+ * workspace's with DISTCA_SCHED_LAUNCHED) has room for inside the workspace, computed from the sizes in p alone.  The device
  * builder never writes more; it counts what did not fit in word 2 of the list's header
  * (always 0 when p bounds the sequence lengths as required above).  No reference
  * counterpart. */

@@ -587,3 +587,49 @@ def test_mfma_rate_probe(cuda):
         assert cyc >= 31.9
     with pytest.raises(RuntimeError):
         _lib.probe_mfma_rate(9, 10, scratch.data_ptr())
+
+
+@pytest.mark.parametrize("lens,extra,hq,hkv", [([8192], 0, 32, 8), ([389, 64, 0, 1200], 0, 4, 1), ([300, 40, 700], 9000, 8, 2), ([4096], 0, 8, 2),
+                                               ([5000, 2000, 128, 1064], 0, 32, 8), ([1000, 300, 17, 600] * 12, 0, 64, 8), ([3000, 2100] * 7, 500, 6, 2)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_device_lists_equal_the_mirror_of_launched_lists(cuda, lens, extra, hq, hkv, causal):
+    """With the preferred workspace: the forward's, the dK/dV and the dQ list the builder left, pieces, merged items, walk marks and
+    costs, are those of the host mirror (as sets within a cost bin), and so are the counts of blocks cut and of slots in use."""
+    import ctypes
+    from distca_amd import scheduler
+    from distca_amd._lib import CaParams, load
+    from distca_amd.fused_comm_attn import ca_varlen_bwd, ca_varlen_fwd
+    lq = np.array(lens, dtype=np.int64)
+    lk = lq + extra * (np.arange(len(lq)) % 2 == 0)
+    tq, tk, mq, mk = int(lq.sum()), int(lk.sum()), int(lq.max()), int(lk.max())
+    q, do = (randn_bf16((tq, hq, 128), s).to(cuda) for s in (1, 2))
+    k, v = (randn_bf16((tk, hkv, 128), s).to(cuda) for s in (3, 4))
+    i32 = lambda x: torch.tensor(np.concatenate([[0], np.cumsum(x)]), dtype=torch.int32, device=cuda)
+    p = CaParams(len(lq), tq, tk, hq, hkv, 128, mq, mk, 128 ** -0.5, int(causal), 1, 0)
+    ws = [torch.zeros(int(getattr(load(), f"distca_ca_{d}_workspace_preferred_bytes")(ctypes.byref(p))), dtype=torch.uint8, device=cuda) for d in ("fwd", "bwd")]
+    print(f"launched lists {lens[:5]} + {extra} heads {hq}/{hkv} causal={causal}", flush=True)
+    out, lse = ca_varlen_fwd(q, k, v, i32(lq), i32(lk), mq, mk, None, causal, None, ws[0])
+    ca_varlen_bwd(do, q, k, v, out, lse, i32(lq), i32(lk), mq, mk, None, causal, True, workspace=ws[1])
+    torch.cuda.synchronize()
+    words = [w[:w.numel() // 4 * 4].cpu().view(torch.int32).numpy() for w in ws]
+    header = (4 + len(lq) + 1 + 3) // 4 * 4
+    cap = lambda kind: scheduler.schedule_capacity(kind | scheduler.LAUNCHED, np.cumsum([0, *lq]), np.cumsum([0, *lk]), hq, hkv, causal=causal)
+    region = lambda kind: ((header + 4 * cap(kind)) * 4 + 255) // 256 * 256 + 256 + 1024
+    groups = (8 * (len(lq) + 1) + 63) // 64 * 64 * 4
+    stats = 2 * ((hq * tq * 4 + 255) // 256 * 256)
+    dq_at = region(scheduler.BWD) + groups
+    for kind, w, at in ((scheduler.FWD, words[0], 0), (scheduler.BWD, words[1], 0), (scheduler.DQ, words[1], dq_at // 4)):
+        host = scheduler.build_schedule(kind | scheduler.LAUNCHED, np.cumsum([0, *lq]), np.cumsum([0, *lk]), hq, hkv, causal=causal)
+        n = int(w[at])
+        if kind == scheduler.FWD and n == 0 and len(host) > 0:
+            continue          # (blocks that all run at once: no list was built)
+        assert n == len(host) and int(w[at + 2]) == 0, kind
+        dev = w[at + header:at + header + 4 * n].reshape(n, 4)
+        assert np.array_equal(dev[:, 2], host[:, 2]), kind
+        assert sorted(map(tuple, dev.tolist())) == sorted(map(tuple, host.tolist())), kind
+    # the dK/dV list's table of cut blocks lies behind both lists and the row statistics
+    whole = words[1][(dq_at + region(scheduler.DQ) + stats) // 4:]
+    host = scheduler.build_schedule(scheduler.BWD | scheduler.LAUNCHED, np.cumsum([0, *lq]), np.cumsum([0, *lk]), hq, hkv, causal=causal)
+    pieces = host[scheduler.item_pieces(host[:, 3]) > 1]
+    if len(pieces):
+        assert int(whole[1]) == len(pieces) and int(whole[0]) == len({(t, b) for t, b, _, _ in pieces.tolist()})

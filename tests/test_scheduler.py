@@ -227,3 +227,79 @@ def test_walk_flags_of_a_bin_too_large_to_rank():
     for c in np.unique(costs):
         idx = np.flatnonzero(costs == c)
         assert len(idx) == 100 and (up[idx] == bool((idx[0] // rnd) & 1)).all()
+
+
+KINDS = {scheduler.FWD: "forward", scheduler.BWD: "dK/dV", scheduler.DQ: "dQ"}
+
+
+def _blocks(kind, a, k, g, causal):
+    """What the blocks of one task cost, restated: KV tiles of 64 keys that 256 query rows stream, or blocks of 32 rows that see 256 keys."""
+    if kind == scheduler.BWD:
+        first = lambda n: max(0, n * 256 - (k - a)) * g // 32 if causal else 0
+        return [max(0, -(-a * g // 32) - first(n)) for n in range(-(-k // 256))] if a > 0 else []
+    last = lambda b: min(a, -(-(b + 1) * 256 // g))
+    return [-(-(min(k, max(0, last(b) + k - a)) if causal else k) // 64) for b in range(-(-a * g // 256))]
+
+
+def _launched_batches():
+    rng = np.random.default_rng(11)
+    yield [8192], [8192]
+    yield [389], [389]
+    yield [40, 64, 0, 3], [9000, 20000, 50, 3]                 # few rows over long prefixes
+    yield [1000, 1000], [900, 400]                             # first tokens that see nothing
+    for trial in range(60):
+        n = int(rng.integers(1, 12))
+        lq = np.minimum(np.exp(rng.normal(6.5, 1.6, size=n)).astype(int), 20000)
+        yield lq.tolist(), (lq + rng.integers(0, 12000, size=n) * (rng.random(n) < 0.4)).tolist()
+
+
+@pytest.mark.parametrize("hq,hkv", [(4, 1), (8, 2), (32, 8), (64, 8), (6, 2), (16, 16)])
+@pytest.mark.parametrize("kind", list(KINDS), ids=KINDS.get)
+def test_launched_lists_hold_every_block_whole_or_in_pieces_of_one_size(kind, hq, hkv):
+    """The lists as a call with the preferred workspace launches them: every block once, whole, merged with its neighbours by the rule for
+    batches of many blocks, or in pieces of one size (the last up to an eighth longer); the items, the blocks cut and the pieces'
+    slots within the room the workspace gives them (the mirror fails on the latter two), the most expensive first."""
+    g, cut_lists = hq // hkv, 0
+    for lq, lk in _launched_batches():
+        causal = (sum(lq) + sum(lk)) % 5 > 0
+        items = scheduler.build_schedule(kind | scheduler.LAUNCHED, _cu(lq), _cu(lk), hq, hkv, causal=causal)
+        assert len(items) <= scheduler.schedule_capacity(kind | scheduler.LAUNCHED, _cu(lq), _cu(lk), hq, hkv, causal=causal)
+        per_unit = sum(lq) * hq / (256 * 256)                  # blocks of query rows per compute unit
+        mean = sum(lq) / len(lq)
+        least = 8 if mean < 768 else 12
+        tiles = 0 if kind == scheduler.BWD or mean >= 2048 or per_unit < least else 128 if mean >= 768 else 32 if per_unit < 16 else 64
+        got = {}
+        for t, b, c, w in items.tolist():
+            got.setdefault((t, b), []).append((scheduler.item_piece(w), scheduler.item_pieces(w), c))
+        sizes, want = set(), {}
+        for t, (a, k) in enumerate(zip(lq, lk)):
+            costs = _blocks(kind, a, k, g, causal)
+            m = min(8, max(1, tiles // max(1, costs[-1]))) if tiles and len(costs) > 1 else 1
+            want.update({(t, i): sum(costs[i * m:(i + 1) * m]) for i in range(-(-len(costs) // m))})
+        assert sorted(got) == sorted(want)
+        for key, ps in got.items():
+            n, ps = ps[0][1], sorted(ps)
+            assert [j for j, _, _ in ps] == list(range(n)) and all(k == n for _, k, _ in ps) and n <= 64
+            assert sum(c for _, _, c in ps) == want[key]
+            sizes |= {c for _, _, c in ps[:-1]}
+            assert n == 1 or n == 64 or 0 < ps[-1][2] <= ps[0][2] + ps[0][2] // 8
+        assert len(sizes) <= 1
+        if sizes:
+            cut_lists += 1
+            size = sizes.pop()
+            assert size >= 8 and all(len(got[key]) > 1 or c <= size + size // 8 for key, c in want.items())
+        if kind != scheduler.BWD and (per_unit >= 8 or max(lk) < 1024):
+            assert (scheduler.item_pieces(items[:, 3]) == 1).all()
+        assert (np.diff(items[:, 2] >> max(0, (int(items[:, 2].max()) // 4096).bit_length())) <= 0).all()
+    assert cut_lists > 0
+
+
+@pytest.mark.parametrize("kind", list(KINDS), ids=KINDS.get)
+def test_cutting_follows_what_bounds_the_launch(kind):
+    """Blocks are cut where the longest outlasts the average load of a compute unit, and stay whole where the load bounds the launch:
+    one document alone on a few heads, beside documents that fill the device, and rows of a document whose blocks even out."""
+    pieces = lambda lens, hq, hkv: int(scheduler.item_pieces(scheduler.build_schedule(kind | scheduler.LAUNCHED, _cu(lens), _cu(lens), hq, hkv)[:, 3]).max())
+    assert pieces([4096], 8, 2) > 2
+    assert pieces([16384] * 4, 32, 8) == 1
+    assert pieces([8192], 32, 8) == 1 if kind != scheduler.BWD else pieces([8192], 32, 8) > 1
+    assert pieces([64] * 8, 8, 2) == 1
