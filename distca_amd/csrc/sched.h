@@ -264,9 +264,10 @@ DISTCA_HD int64_t sched_region_bytes(int32_t num_tasks, int64_t max_items) {
 //   first [B + 1]   group u's tasks are tasks[first[u] .. first[u + 1]), by (prefix length, task index)
 //   tasks [B]
 //   off   [B]       first stored row of the group        lmax [B]   its longest prefix
-//   gap_lo, gap_hi [B + 1]   stored rows [gap_lo[u], gap_hi[u]) belong to no group (zeroed by the backward): from the
-//                            end of group u to the start of the next one; entry `number of groups`: the rows before
-//                            the first group
+//   gap_lo, gap_hi [B + 1]   stored rows [gap_lo[u], gap_hi[u]) belong to no group: from the end of group u to the start
+//                            of the next one; entry `number of groups`: the rows before the first group.  Made to count
+//                            the groups that run into the next one; no kernel reads them.  The workgroups that zero dk / dv
+//                            of such rows run beside the builder and find them from the task bounds (fill_rows).
 //   tmp   [2 B]     scratch of the builder
 struct SharedGroups {
   int32_t *first, *tasks, *off, *lmax, *gap_lo, *gap_hi, *tmp;

@@ -401,8 +401,9 @@ __device__ void build_shared(ListScratch &s, TaskCache &cache, GroupScratch &gs,
         }
       sg.tasks[sg.first[gid[l]] + before] = b;
     }
-  // e. the stored rows no group covers: before the first group, and from the end of a group to the start of the next.
-  // Groups must not overlap (tasks that share rows start at the same row); those that do are counted in word 3.
+  // e. Groups must not overlap (tasks that share rows start at the same row); those that do are counted in word 3, from the stored rows
+  // no group covers: before the first group, and from the end of a group to the start of the next.  (They stay in the table for whoever
+  // reads a list back; fill_rows, in the launch's other workgroups, does not wait for it.)
   for (int32_t u = tid; u <= num_tasks; u += kSchedThreads) {
     int32_t lo = 0, hi = 0;
     if (u <= ngroups) {
