@@ -223,8 +223,9 @@ struct CoreAttention : torch::autograd::Function<CoreAttention> {
                         const Tensor &cu_k, const OptTensor &kv_off, int64_t max_q, int64_t max_k, std::optional<double> scale, bool causal,
                         bool deterministic) {
     auto [out, lse] = varlen_fwd({q, k, v, cu_q, cu_k, kv_off, max_q, max_k, scale, causal}, std::nullopt);
-    ctx->save_for_backward({q, k, v, out, lse, cu_q, cu_k, kv_off ? *kv_off : Tensor()});
+    ctx->save_for_backward({q, k, v, out, lse, cu_q, cu_k});
     auto &data = ctx->saved_data;
+    data["kv_off"] = kv_off;   // (beside the saved tensors: a caller may write the offsets of one layer into the buffer of the last)
     data["max_q"] = max_q;
     data["max_k"] = max_k;
     data["scale"] = scale;
@@ -235,7 +236,7 @@ struct CoreAttention : torch::autograd::Function<CoreAttention> {
     const auto s = ctx->get_saved_variables();
     auto &data = ctx->saved_data;
     const int64_t flags = data["flags"].toInt();
-    const Batch b{s[0], s[1], s[2], s[5], s[6], s[7].defined() ? OptTensor(s[7]) : std::nullopt, data["max_q"].toInt(), data["max_k"].toInt(),
+    const Batch b{s[0], s[1], s[2], s[5], s[6], data["kv_off"].toOptional<Tensor>(), data["max_q"].toInt(), data["max_k"].toInt(),
                   data["scale"].toOptional<double>(), (flags & 1) != 0};
     auto g = varlen_bwd(b, grad[0], s[3], s[4], (flags & 2) != 0, {}, std::nullopt);
     torch::autograd::variable_list res(11);

@@ -511,3 +511,19 @@ def test_small_batches_where_memory_is_short(cuda):
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert ticks == least
     assert all(torch.equal(x, y) for x, y in zip(got, want))
+
+
+def test_offsets_may_be_written_again_before_the_backward(cuda):
+    """The first rows of the tasks, in a buffer that every layer's call fills anew with the same values."""
+    from distca_amd.fused_comm_attn import core_attention
+    lens = [100, 200]
+    q, k, v, do = (t.to(cuda) for t in make_qkv(300, 300, 4, 1, 128, 64))
+    c, off = torch.tensor(cu(lens), device=cuda), torch.tensor(cu(lens)[:-1], device=cuda)
+    buf, res = off.clone(), []
+    for again in (False, True):
+        leaf = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        out = core_attention(*leaf, c, c, 200, 200, deterministic=True, kv_task_offsets=buf)
+        if again:
+            buf.copy_(off)
+        res.append(torch.autograd.grad(out, leaf, do))
+    assert all(torch.equal(x, y) for x, y in zip(*res))
