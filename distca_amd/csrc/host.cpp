@@ -268,8 +268,11 @@ int64_t int_arg(PyObject *o) {
 }
 std::optional<double> optional_float(PyObject *o) {
   if (o == Py_None) return std::nullopt;
-  const double x = PyFloat_AsDouble(o);
-  if (x == -1.0 && PyErr_Occurred()) throw python_error();
+  if (PyFloat_Check(o)) return PyFloat_AS_DOUBLE(o);
+  PyObject *as_float = PyNumber_Float(o);   // (what float() takes, strings among them)
+  if (!as_float) throw python_error();
+  const double x = PyFloat_AS_DOUBLE(as_float);
+  Py_DECREF(as_float);
   return x;
 }
 bool bool_arg(PyObject *o) {

@@ -362,3 +362,17 @@ def test_the_package_names_nothing_private_of_torch():
     import pathlib
     for f in pathlib.Path(ROOT, "distca_amd").rglob("*.py"):
         assert not re.findall(r"\btorch(?:\.\w+)*\._\w+", f.read_text()), f
+
+
+def test_numbers_of_an_attention_call_are_what_int_and_float_take():
+    """Sequence lengths and the scale in any form int() and float() take, truncated as int() does; anything else is a TypeError or ValueError."""
+    import torch
+    from distca_amd.fused_comm_attn import ca_varlen_fwd
+    q = torch.zeros((4, 2, 128), dtype=torch.bfloat16)
+    cu = torch.tensor([0, 4], dtype=torch.int32)
+    for n, scale in ((4, None), (4.7, 0.1), ("4", "0.1"), (np.int64(4), np.float32(0.1)), (torch.tensor(4), torch.tensor(0.1)), (True, 1)):
+        with pytest.raises(RuntimeError, match="CUDA"):   # (the first thing that is wrong here)
+            ca_varlen_fwd(q, q, q, cu, cu, n, n, scale)
+    for n, scale in ((None, 0.1), (4, [0.1]), ("x", 0.1), (4, "x"), (float("nan"), 0.1)):
+        with pytest.raises((TypeError, ValueError)):
+            ca_varlen_fwd(q, q, q, cu, cu, n, n, scale)
