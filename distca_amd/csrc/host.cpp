@@ -413,10 +413,10 @@ c10::Device read_job(PyObject *o, distca_exchange_job &j) {
     j.mask = data_of<int8_t>(mask, "do_shard");
   } else {
     check_tensor(offset, 1, "seq_nvshmem_offset");
-    check_tensor(tokens, 1, "seq_tokens");
+    check_tensor(tokens, tokens.dim(), "seq_tokens");   // (of any shape that begins with a length per shard)
     j.max_cp = 1;
     j.num_seq = offset.size(0);
-    if (tokens.size(0) < j.num_seq) fail("seq_tokens must be of shape (num_sequence,)");
+    if (tokens.numel() < j.num_seq) fail("seq_tokens must be of shape (num_sequence,)");
     if (f[4] != Py_None) {
       const Tensor &mask = tensor_arg(f[4], "copy_seq_mask");
       check_tensor(mask, 1, "copy_seq_mask");
@@ -428,7 +428,7 @@ c10::Device read_job(PyObject *o, distca_exchange_job &j) {
     const Tensor &num_copies = tensor_arg(f[6], "num_copies"), &start = tensor_arg(f[7], "copy_start_id");
     check_tensor(num_copies, 1, "num_copies");
     check_tensor(start, 2, "copy_start_id");
-    if (num_copies.size(0) != j.num_seq || tokens.size(0) != j.num_seq) fail("seq_lens must be of shape (num_sequence,)");
+    if (num_copies.size(0) != j.num_seq || tokens.dim() != 1 || tokens.size(0) != j.num_seq) fail("seq_lens must be of shape (num_sequence,)");
     if (start.size(0) != j.num_seq) fail("copy_start_id must be of shape (num_sequence, max_num_copies)");
     j.num_copies = data_of<int32_t>(num_copies, "num_copies");
     j.copy_start = data_of<int64_t>(start, "copy_start_id");

@@ -515,3 +515,20 @@ def test_packing_into_the_memory_of_another_device(cuda):
     pre_a2a_qkv(q, k, v, ones, lens, lens, i64([0]), i64([[T * tb]]), i64([[2 * T * tb]]), is_fwd=True, buffer=buf)
     torch.cuda.current_stream(cuda).synchronize()
     assert torch.equal(buf.view(torch.bfloat16).view(3 * T, hidden).cpu(), torch.cat([q, k, v]).cpu())
+
+
+@pytest.mark.parametrize("form", ["longer", "matrix"])
+def test_lengths_of_a_plain_pack_in_other_shapes(cuda, form):
+    """The queries' lengths on the way out may go on behind the shards that are placed, and be a matrix: a2a_memcpy_non_cp's terms."""
+    from distca_amd.dispatch import pre_a2a_qkv
+    lens, hidden = [3, 2, 4, 1], 64
+    T, tb = sum(lens), hidden * 2
+    i64 = lambda x: torch.tensor(x, dtype=torch.int64, device=cuda)
+    q, k, v = (torch.randn((T, hidden), device=cuda).to(torch.bfloat16) for _ in range(3))
+    start = np.concatenate([[0], np.cumsum(lens)[:-1]]) * tb
+    q_lens = i64(lens + [7, 9]) if form == "longer" else i64(lens).view(2, 2)
+    buf = torch.zeros(3 * T * tb, dtype=torch.uint8, device=cuda)
+    print("lengths", form, flush=True)
+    pre_a2a_qkv(q, k, v, torch.ones((4, 1), dtype=torch.int8, device=cuda), q_lens, i64(lens), i64(start), i64(start + T * tb)[None],
+                i64(start + 2 * T * tb)[None], is_fwd=True, buffer=buf)
+    assert torch.equal(buf, torch.cat([q, k, v]).view(torch.uint8).view(-1))
