@@ -93,15 +93,24 @@ struct Job {
   const int32_t *num_copies;
   const int64_t *copy_start;
   int64_t num_tokens, token_bytes, pitch;
-  int32_t kind, dtype, num_seq, max_cp, max_copies, tokens_per_wg, first_wg;
+  int32_t kind, dtype, num_seq, max_cp, max_copies, tokens_per_wg;
   uint32_t part_v0, part_vecs, magic;  // magic = ceil(2^32 / part_vecs) (0: part_vecs is 1): i / part_vecs == umulhi(i, magic) for i * part_vecs < 2^32
   __host__ __device__ bool whole() const { return pitch == token_bytes && (int64_t)part_vecs * 16 == token_bytes; }
 };
 constexpr int kMaxJobs = 12;
 struct Jobs {
-  Job job[kMaxJobs];
+  int32_t first_wg[kMaxJobs];   // beside each other: a workgroup looks through all of them
   int32_t n;
+  Job job[kMaxJobs];
 };
+
+__device__ __forceinline__ int job_of_workgroup(const Jobs &jobs) {
+  int j = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxJobs; ++i)
+    if (i < jobs.n && (int)blockIdx.x >= jobs.first_wg[i]) j = i;
+  return j;
+}
 
 // A contiguous run of memory as a buffer resource of its exact length: lanes past its end load zeros and store nothing, so a
 // partial round needs no branches and is issued like a whole one.  (With a predicate per vector the compiler could not keep
@@ -268,12 +277,9 @@ __device__ __forceinline__ void sum_copies(const Job &jb, int seg, int64_t skip_
 // registers, so that two workgroups fit a compute unit.
 template <bool TO_BUF, bool PARTS, bool SUMS>
 __global__ __launch_bounds__(kPackThreads, SUMS ? 4 : 8) void exchange_kernel(Jobs jobs, uint8_t *buffer) {
-  int j = 0;
-#pragma unroll
-  for (int i = 1; i < kMaxJobs; ++i)
-    if (i < jobs.n && (int)blockIdx.x >= jobs.job[i].first_wg) j = i;
+  const int j = job_of_workgroup(jobs);
   const Job &jb = jobs.job[j];
-  const int64_t t0 = (int64_t)((int)blockIdx.x - jb.first_wg) * jb.tokens_per_wg;
+  const int64_t t0 = (int64_t)((int)blockIdx.x - jobs.first_wg[j]) * jb.tokens_per_wg;
   int64_t t1 = t0 + jb.tokens_per_wg;
   if (t1 > jb.num_tokens) t1 = jb.num_tokens;
   if (t0 >= t1) return;
@@ -347,6 +353,174 @@ __global__ __launch_bounds__(kPackThreads, SUMS ? 4 : 8) void exchange_kernel(Jo
   }
 }
 
+// ---- Up to some 100 MB: a vector a thread ----
+//
+// A launch of a few MB is a chain of trips to memory, not a matter of bandwidth: a plain copy of 3 MB takes 2.4 us, and the same by
+// exchange_kernel took 6 to 8, because a slice's runs go one after the other (a trip there and a trip back for each shard and replica it
+// touches), behind a shard's length, place and mask and the replicas' masks and places read one by one.  Here a thread moves one vector,
+// whatever shard it lies in: a wave reads the lengths, places and masks of 64 shards at once, a lane a shard, finds by lane moves where its
+// vectors go, and all of them travel together; what is packed is requested before the list is read.
+// us by slices / by vectors, pack, reply, request and gradients of the linear side: 1024 tokens at 8/2 heads (3 / 2 / 7 / 3 MB)
+// 7.7 7.1 11.5 9.0 / 4.3 3.9 6.0 5.0; 2048 at 32/8 (25 / 17 / 59 / 25 MB) 15.2 12.7 27.3 17.5 / 12.7 8.7 23.2 12.6; 4096 (50 / 34 / 117 / 50)
+// 23.0 17.7 48.4 24.8 / 21.6 18.9 43.9 26.9; 8192 (101 / 67 / 235 / 101) 39.8 34.3 88.2 42.9 / 41.2 33.1 90.7 48.6.  The lines below lie
+// where slices, which load ten vectors a thread before they store, begin to gain; adding rows up, a vector has a load in flight at a time, and loses earlier.
+constexpr int kVectorThreads = 256;
+constexpr int64_t kVectorBytes = 128ll << 20, kVectorSumBytes = 32ll << 20;   // of a launch; of one that adds rows up
+constexpr int kVectorSeqs = 256;             // shards of a job: four reads of 64
+
+// 64 shards from c0 on, one a lane.  end: position behind the shard's last token (sums saturate; tensors have fewer than 2^31 tokens).
+struct ShardWindow {
+  uint32_t len, end;
+  int64_t off;
+  int sent;
+};
+__device__ __forceinline__ uint32_t add_tokens(uint32_t a, uint32_t b) { return __builtin_elementwise_add_sat(a, b); }
+__device__ __forceinline__ ShardWindow read_shards(const Job &jb, bool plain, const int8_t *mask, int c0, uint32_t before) {
+  const int i = c0 + (threadIdx.x & 63);
+  ShardWindow w{0, 0, 0, 1};
+  if (i < jb.num_seq) {
+    const int64_t n = jb.seq_tokens[i];
+    if (plain) w.off = jb.seq_offset[i];
+    if (mask) w.sent = mask[i];
+    w.len = n <= 0 ? 0u : (n > 0x7fffffff ? 0x7fffffffu : (uint32_t)n);
+  }
+  uint32_t v = w.len;   // inclusive sums over the lanes, by DPP moves
+  v = add_tokens(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false));  // row_shr:1
+  v = add_tokens(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false));  // row_shr:2
+  v = add_tokens(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false));  // row_shr:4
+  v = add_tokens(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false));  // row_shr:8
+  v = add_tokens(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));  // row_bcast:15 into rows 1 and 3
+  v = add_tokens(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));  // row_bcast:31 into rows 2 and 3
+  w.end = add_tokens(before, v);
+  return w;
+}
+__device__ __forceinline__ u32x4 load_vec(const uint8_t *p) { return *reinterpret_cast<const u32x4 *>(p); }
+__device__ __forceinline__ void store_vec(uint8_t *p, u32x4 v) { *reinterpret_cast<u32x4 *>(p) = v; }
+
+// f(replica, its place) for every live replica of shard `seg`, in their order: masks and places are read a lane a replica.  By whole waves.
+template <class F>
+__device__ __forceinline__ void each_replica(const Job &jb, int seg, F f) {
+  for (int c0 = 0; c0 < jb.max_cp; c0 += 64) {
+    const int c = c0 + (threadIdx.x & 63);
+    int on = 0;
+    int64_t off = 0;
+    if (c < jb.max_cp) {
+      on = jb.mask[(int64_t)seg * jb.max_cp + c];
+      off = jb.seq_offset[(int64_t)c * jb.num_seq + seg];
+    }
+    for (unsigned long long m = __ballot(on != 0); m; m &= m - 1) f(c0 + __builtin_ctzll(m), lane_value(off, __builtin_ctzll(m)));
+  }
+}
+// f(first row of the copy) for the copies of shard `seg`, in their order.  By whole waves.
+template <class F>
+__device__ __forceinline__ int each_copy(const Job &jb, int seg, F f) {
+  const int64_t *starts = jb.copy_start + (int64_t)seg * jb.max_copies;
+  const int lane = threadIdx.x & 63;
+  const int32_t given = jb.num_copies[seg];
+  int64_t start = lane < jb.max_copies ? starts[lane] : 0;
+  const int32_t nc = uniform_int(given);
+  for (int c = 0; c < nc; ++c) {
+    if (c > 0 && (c & 63) == 0) start = c + lane < jb.max_copies ? starts[c + lane] : 0;
+    f(lane_value(start, c & 63));
+  }
+  return nc;
+}
+
+template <bool TO_BUF, typename T>
+__device__ __forceinline__ void vector_sum(const Job &jb, uint8_t *buffer, int seg, const ShardWindow &w, int l, uint32_t row, bool in, uint32_t byte, uint8_t *at) {
+  if (!TO_BUF) {
+    Sum<T> acc;
+    acc.clear();
+    each_replica(jb, seg, [&](int, int64_t off) {
+      if (in) acc.add(load_vec(buffer + off + (int64_t)row * jb.token_bytes + byte));
+    });
+    if (in) store_vec(at, acc.value());
+    return;
+  }
+  u32x4 m = u32x4{0, 0, 0, 0};
+  if (in) m = load_vec(at);
+  const int nc = each_copy(jb, seg, [&](int64_t start) {
+    if (in) m = Add<T>::apply(m, load_vec(jb.data + (start + row) * jb.token_bytes + byte));
+  });
+  const int64_t off = lane_value(w.off, l);
+  const bool sent = __builtin_amdgcn_readlane(w.sent, l) != 0;
+  if (in && nc > 0) store_vec(at, m);
+  if (in && sent) store_vec(buffer + off + (int64_t)row * jb.token_bytes + byte, m);
+}
+
+template <bool TO_BUF>
+__global__ __launch_bounds__(kVectorThreads) void exchange_vectors_kernel(Jobs jobs, uint8_t *buffer) {
+  const int j = job_of_workgroup(jobs);
+  const Job &jb = jobs.job[j];
+  const int lane = threadIdx.x & 63;
+  const uint32_t nvec = (uint32_t)jb.num_tokens * jb.part_vecs, i = (uint32_t)((int)blockIdx.x - jobs.first_wg[j]) * kVectorThreads + threadIdx.x;
+  const uint32_t first = (uint32_t)uniform_int((int)(i - lane));
+  if (first >= nvec) return;
+  const bool live = i < nvec;
+  const uint32_t ic = live ? i : nvec - 1;
+  const uint32_t t = jb.magic ? __umulhi(ic, jb.magic) : ic, byte = (ic - t * jb.part_vecs) << 4;   // token, and place in its part
+  const uint32_t t_first = (uint32_t)uniform_int((int)t), t_last = (uint32_t)__builtin_amdgcn_readlane((int)t, 63);
+  uint8_t *at = jb.data + (int64_t)t * jb.pitch + byte;
+  const int kind = jb.kind;
+  const bool plain = kind == DISTCA_JOB_PLAIN, sums = kind == DISTCA_JOB_REPLICA_SUM || kind == DISTCA_JOB_COPY_SUM;
+  const bool by_shard = plain || kind == DISTCA_JOB_COPY_SUM;   // (else by shard and replica)
+  u32x4 v = u32x4{0, 0, 0, 0};
+  if (TO_BUF && !sums && live && jb.data) v = load_vec(at);
+
+  // the shard of the wave's first token
+  const int8_t *mask = TO_BUF && by_shard ? jb.mask : nullptr;
+  int c0 = 0, seg = jb.num_seq;
+  ShardWindow w{0, 0, 0, 0};
+  uint32_t before = 0;
+  for (; c0 < jb.num_seq; c0 += 64) {
+    w = read_shards(jb, by_shard, mask, c0, before);
+    const unsigned long long past = __ballot(w.end > t_first);
+    if (past) {
+      seg = c0 + __builtin_ctzll(past);
+      break;
+    }
+    before = (uint32_t)__builtin_amdgcn_readlane((int)w.end, 63);
+  }
+  // and, from there on, those of all of its tokens
+  bool found = false;   // this vector has a place
+  uint8_t *place = buffer;
+  for (; seg < jb.num_seq; ++seg) {
+    if (seg - c0 == 64) {
+      before = (uint32_t)__builtin_amdgcn_readlane((int)w.end, 63);
+      c0 += 64;
+      w = read_shards(jb, by_shard, mask, c0, before);
+    }
+    const int l = seg - c0;
+    const uint32_t end = (uint32_t)__builtin_amdgcn_readlane((int)w.end, l), start = end - (uint32_t)__builtin_amdgcn_readlane((int)w.len, l);
+    if (start > t_last) break;
+    const bool in = live && t >= start && t < end;
+    const uint32_t row = t - start;   // (of the shard, where `in`)
+    if (plain) {
+      if (in && __builtin_amdgcn_readlane(w.sent, l) != 0) {
+        found = true;
+        place = buffer + lane_value(w.off, l) + (int64_t)row * jb.token_bytes + (((int64_t)jb.part_v0 << 4) + byte);
+      }
+    } else if (sums) {
+      found = found || in;
+      if (jb.dtype == DISTCA_DTYPE_BF16) vector_sum<TO_BUF, __bf16>(jb, buffer, seg, w, l, row, in, byte, at);
+      else if (jb.dtype == DISTCA_DTYPE_F16) vector_sum<TO_BUF, _Float16>(jb, buffer, seg, w, l, row, in, byte, at);
+      else vector_sum<TO_BUF, float>(jb, buffer, seg, w, l, row, in, byte, at);
+    } else {
+      each_replica(jb, seg, [&](int c, int64_t off) {
+        uint8_t *b = buffer + off + (int64_t)row * jb.token_bytes + byte;
+        if (!in) return;
+        if (TO_BUF) store_vec(b, v);
+        else store_vec(at + (int64_t)c * jb.num_tokens * jb.token_bytes, load_vec(b));
+      });
+    }
+  }
+  if (plain && found) {
+    if (TO_BUF) store_vec(place, v);
+    else store_vec(at, load_vec(place));
+  }
+  if (!TO_BUF && kind == DISTCA_JOB_REPLICA_SUM && live && !found) store_vec(at, v);   // rows behind the last shard: sums of nothing
+}
+
 // data[start_s + t] += data[copy_start_id[s][c] + t] for c = 0..num_copies[s]-1 in order,
 // one rounding per addition.  Rows are cut into per-workgroup slices like those of exchange_kernel.
 template <typename T>
@@ -402,7 +576,7 @@ __global__ __launch_bounds__(kPackThreads) void grad_sum_kernel(T *__restrict__ 
 
 // Bytes of a workgroup's slice for a launch of `total` bytes: one loop round (160 KiB at 10 vectors per lane) once the launch
 // has four such slices per compute unit; below that as many whole vectors per thread as give every unit two workgroups, so
-// that a small copy is spread over the device (2.7 MB: 13 workgroups of 160 KiB took 6.8 us).
+// that a small copy (of more shards than exchange_vectors_kernel takes) is spread over the device.
 int64_t slice_bytes(int64_t total) {
   const int64_t cus = num_compute_units();
   if (total >= 4 * cus * kRoundBytes) return kRoundBytes;
@@ -477,6 +651,23 @@ int launch_exchange(Jobs &jobs, void *buffer, int to_buffer, void *stream, int t
     sums |= o.kind == DISTCA_JOB_REPLICA_SUM || o.kind == DISTCA_JOB_COPY_SUM;
     parts |= !o.whole();
   }
+  hipStream_t s = (hipStream_t)stream;
+  uint8_t *buf = (uint8_t *)buffer;
+  bool by_vectors = total <= (sums ? kVectorSumBytes : kVectorBytes);
+  for (int i = 0; i < jobs.n && by_vectors; ++i) {   // (a vector's number times the vectors of a part stays below 2^32: Job::magic)
+    const Job &o = jobs.job[i];
+    by_vectors = o.num_seq <= kVectorSeqs && o.num_tokens * o.part_vecs * o.part_vecs < (1ll << 32);
+  }
+  if (by_vectors) {
+    for (int i = 0; i < jobs.n; ++i) {
+      jobs.first_wg[i] = (int32_t)wg;
+      wg += (jobs.job[i].num_tokens * jobs.job[i].part_vecs + kVectorThreads - 1) / kVectorThreads;
+    }
+    ScopedTimer timer(timer_id, s);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)wg), dim3(kVectorThreads), 0, s, jobs, buf); };
+    launch(to_buffer ? exchange_vectors_kernel<true> : exchange_vectors_kernel<false>);
+    return check_launch(what);
+  }
   const int64_t slice = slice_bytes(total);
   for (int i = 0; i < jobs.n; ++i) {
     Job &o = jobs.job[i];
@@ -490,14 +681,12 @@ int launch_exchange(Jobs &jobs, void *buffer, int to_buffer, void *stream, int t
       if (per > most) per = most < 1 ? 1 : most, grid = (o.num_tokens + per - 1) / per;
     }
     o.tokens_per_wg = (int32_t)per;
-    o.first_wg = (int32_t)wg;
+    jobs.first_wg[i] = (int32_t)wg;
     wg += grid;
     if (wg > 0x7fffffff) return fail(DISTCA_E_INVALID, "%s: grid too large", what);
   }
-  hipStream_t s = (hipStream_t)stream;
   ScopedTimer timer(timer_id, s);
   const dim3 g((unsigned)wg), b(kPackThreads);
-  uint8_t *buf = (uint8_t *)buffer;
   auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, b, 0, s, jobs, buf); };
   if (to_buffer) launch(sums ? exchange_kernel<true, true, true> : parts ? exchange_kernel<true, true, false> : exchange_kernel<true, false, false>);
   else launch(sums ? exchange_kernel<false, true, true> : parts ? exchange_kernel<false, true, false> : exchange_kernel<false, false, false>);

@@ -134,6 +134,62 @@ def test_cp_pack_unpack(cuda, max_cp):
     assert np.array_equal(planes.view(torch.uint8).reshape(max_cp, T, tb).cpu().numpy(), exp_p)
 
 
+@pytest.mark.parametrize("max_cp,nshard,hidden,longest", [
+    (1, 4, 8, 1), (64, 4, 8, 3), (65, 5, 8, 40), (130, 4, 24, 5), (2, 256, 8, 2), (3, 40, 2048, 140),   # a vector a thread: at most 256 shards
+    (2, 257, 8, 2), (3, 520, 16, 9), (2, 300, 1024, 60)])                                              # by slices: more than that
+def test_many_replicas_and_shards(cuda, max_cp, nshard, hidden, longest):
+    """Replicas and shards are found by lanes of a wave: more of either than a wave has, shards of fewer rows than that, empty ones among
+    them.  Packed, unpacked, summed over replicas and over copies (exact: small whole numbers); plain copies of the same shards."""
+    from distca_amd.ops import a2a_memcpy_cp, a2a_memcpy_non_cp, copy_sum_job, exchange, replica_sum_job
+    rng = np.random.default_rng(max_cp)
+    lens = rng.integers(0, longest + 1, size=nshard).astype(np.int64)
+    lens[[0, 2, 3]] = longest
+    T, tb = int(lens.sum()), hidden * 2
+    do_shard = (rng.random((nshard, max_cp)) < 0.5).astype(np.int8)
+    do_shard[:, max_cp - 1] = 1
+    off = np.zeros((max_cp, nshard), dtype=np.int64)
+    cur = 0
+    for c in range(max_cp):
+        for s in rng.permutation(nshard):
+            off[c, s] = cur
+            cur += int(lens[s]) * tb
+    src = torch.randint(-2, 3, (T, hidden), generator=torch.Generator().manual_seed(nshard)).to(torch.bfloat16)
+    raw = src.view(torch.uint8).numpy()
+    exp = np.zeros(cur, dtype=np.uint8)
+    fa2a.copy_cp(raw, exp, do_shard, off, lens, True)
+    d_do, d_off, d_len = (torch.from_numpy(x).to(cuda) for x in (do_shard, off, lens))
+    print(f"replicas {max_cp} shards {nshard}", flush=True)
+    dbuf = torch.zeros(cur, dtype=torch.uint8, device=cuda)
+    a2a_memcpy_cp(src.to(cuda), d_do, d_off, d_len, True, buffer=dbuf)
+    planes = torch.zeros((max_cp, T, hidden), dtype=torch.bfloat16, device=cuda)
+    a2a_memcpy_cp(planes, d_do, d_off, d_len, False, buffer=dbuf)
+    total = torch.empty((T + 3, hidden), dtype=torch.bfloat16, device=cuda)
+    exchange([replica_sum_job(total, d_do, d_off, d_len)], dbuf, False)
+    torch.cuda.synchronize()
+    assert np.array_equal(dbuf.cpu().numpy(), exp)
+    exp_p = np.zeros((max_cp, T, tb), dtype=np.uint8)
+    fa2a.copy_cp(exp_p, exp, do_shard, off, lens, False)
+    assert np.array_equal(planes.view(torch.uint8).reshape(max_cp, T, tb).cpu().numpy(), exp_p)
+    want = torch.from_numpy(exp_p).view(torch.bfloat16).reshape(max_cp, T, hidden).float().sum(0).to(torch.bfloat16)
+    assert torch.equal(total[:T].cpu(), want) and not total[T:].any()   # (rows behind the last shard: sums of nothing)
+
+    mask = (rng.random(nshard) < 0.7).astype(np.int8)
+    nc, cs = np.zeros(nshard, np.int32), np.zeros((nshard, 70), np.int64)
+    start = np.concatenate([[0], np.cumsum(lens)])
+    nc[0], cs[0, :66] = 66, np.resize(start[[2, 3]], 66)   # (more copies than lanes)
+    exp_t, exp1 = src.clone(), np.zeros(cur, dtype=np.uint8)
+    fa2a.grad_sum(exp_t, nc, cs, lens)
+    fa2a.copy_non_cp(exp_t.view(torch.uint8).numpy(), exp1, off[0], lens, mask, True)
+    d, dbuf1, d_mask = src.to(cuda), torch.zeros(cur, dtype=torch.uint8, device=cuda), torch.from_numpy(mask).to(cuda)
+    exchange([copy_sum_job(d, d_off[0], d_len, d_mask, torch.from_numpy(nc).to(cuda), torch.from_numpy(cs).to(cuda))], dbuf1, True)
+    dbuf2, back = torch.zeros_like(dbuf1), torch.zeros_like(d)
+    a2a_memcpy_non_cp(d, d_off[0], d_len, True, d_mask, buffer=dbuf2)
+    a2a_memcpy_non_cp(back, d_off[max_cp - 1], d_len, False, None, buffer=dbuf)
+    torch.cuda.synchronize()
+    assert torch.equal(d.cpu(), exp_t) and np.array_equal(dbuf1.cpu().numpy(), exp1) and np.array_equal(dbuf2.cpu().numpy(), exp1)
+    assert torch.equal(back.cpu(), src)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("hidden", [128, 1024, 20])
 def test_grad_sum(cuda, dtype, hidden):
