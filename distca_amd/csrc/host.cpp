@@ -14,6 +14,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -363,24 +364,12 @@ const T *data_of(const Tensor &t, const char *name) {
   return t.const_data_ptr<T>();
 }
 
-// Fills in the job and returns the device of its first tensor.
-c10::Device read_job(PyObject *o, distca_exchange_job &j) {
-  if (!PyTuple_Check(o) || PyTuple_GET_SIZE(o) != 8) type_error("a job is a tuple of eight");
-  PyObject *const *f = &PyTuple_GET_ITEM(o, 0);
-  j = distca_exchange_job{};
-  j.kind = int_arg(f[0]);
-  const bool plain = j.kind == DISTCA_JOB_PLAIN, replicas = j.kind == DISTCA_JOB_REPLICAS || j.kind == DISTCA_JOB_REPLICA_SUM;
-  const bool copies = j.kind == DISTCA_JOB_COPY_SUM;
-  const Tensor &offset = tensor_arg(f[2], "seq_nvshmem_offset"), &tokens = tensor_arg(f[3], "seq_tokens");
-
-  PyObject *parts = f[1];
-  if (!PyList_Check(parts) && !PyTuple_Check(parts)) type_error(std::string("the parts of a token are a list or a tuple of tensors, not ") + Py_TYPE(parts)->tp_name);
-  const Py_ssize_t n = PySequence_Fast_GET_SIZE(parts);
-  if (n < 1 || n > DISTCA_TOKEN_MAX_PARTS) fail("a token has one to " + std::to_string(DISTCA_TOKEN_MAX_PARTS) + " parts");
+// The parts a job's token is made of.
+void set_parts(distca_exchange_job &j, const Tensor *const *parts, int64_t n) {
+  const bool plain = j.kind == DISTCA_JOB_PLAIN, sums = j.kind == DISTCA_JOB_COPY_SUM || j.kind == DISTCA_JOB_REPLICA_SUM;
   int64_t row = 0;
-  const c10::Device device = tensor_arg(PySequence_Fast_GET_ITEM(parts, 0), "tensor").device();
-  for (Py_ssize_t i = 0; i < n; ++i) {
-    const Tensor &t = tensor_arg(PySequence_Fast_GET_ITEM(parts, i), "tensor");
+  for (int64_t i = 0; i < n; ++i) {
+    const Tensor &t = *parts[i];
     if (!plain) check_tensor(t, 2, "tensor");
     if (t.dim() != 2) fail("tensor must have 2 dimensions");
     if (!t.is_cuda()) fail("tensor must be on CUDA");
@@ -395,36 +384,66 @@ c10::Device read_job(PyObject *o, distca_exchange_job &j) {
       case at::kHalf: j.dtype = DISTCA_DTYPE_F16; break;
       case at::kBFloat16: j.dtype = DISTCA_DTYPE_BF16; break;
       default:
-        if (copies || j.kind == DISTCA_JOB_REPLICA_SUM) fail("Only fp32, fp16 and bf16 inputs are supported");
+        if (sums) fail("Only fp32, fp16 and bf16 inputs are supported");
     }
   }
   j.num_parts = n;
-  j.token_bytes = f[5] == Py_None ? row : int_arg(f[5]);
-
-  if (replicas) {
-    const Tensor &mask = tensor_arg(f[4], "do_shard");
+  j.token_bytes = row;
+}
+// Its shards: places, lengths, and which are sent (mask, may be null) or which replicas there are.
+void set_shards(distca_exchange_job &j, const Tensor &offset, const Tensor &tokens, const Tensor *mask) {
+  if (j.kind == DISTCA_JOB_REPLICAS || j.kind == DISTCA_JOB_REPLICA_SUM) {
     check_tensor(offset, 2, "seq_nvshmem_offset");
     check_tensor(tokens, 1, "seq_tokens");
-    check_tensor(mask, 2, "do_shard");
+    check_tensor(*mask, 2, "do_shard");
     j.max_cp = offset.size(0);
     j.num_seq = offset.size(1);
     if (tokens.size(0) != j.num_seq) fail("seq_tokens must be of dimension (num_sequence)");
-    if (mask.size(0) != j.num_seq || mask.size(1) != j.max_cp) fail("do_shard must be of dimension (num_sequence, cp_degree)");
-    j.mask = data_of<int8_t>(mask, "do_shard");
+    if (mask->size(0) != j.num_seq || mask->size(1) != j.max_cp) fail("do_shard must be of dimension (num_sequence, cp_degree)");
+    j.mask = data_of<int8_t>(*mask, "do_shard");
   } else {
     check_tensor(offset, 1, "seq_nvshmem_offset");
     check_tensor(tokens, tokens.dim(), "seq_tokens");   // (of any shape that begins with a length per shard)
     j.max_cp = 1;
     j.num_seq = offset.size(0);
     if (tokens.numel() < j.num_seq) fail("seq_tokens must be of shape (num_sequence,)");
-    if (f[4] != Py_None) {
-      const Tensor &mask = tensor_arg(f[4], "copy_seq_mask");
-      check_tensor(mask, 1, "copy_seq_mask");
-      j.mask = data_of<int8_t>(mask, "copy_seq_mask");
-      if (mask.size(0) != j.num_seq) fail("copy_seq_mask must be of shape (num_sequence,)");
+    if (mask) {
+      check_tensor(*mask, 1, "copy_seq_mask");
+      j.mask = data_of<int8_t>(*mask, "copy_seq_mask");
+      if (mask->size(0) != j.num_seq) fail("copy_seq_mask must be of shape (num_sequence,)");
     }
   }
-  if (copies) {
+  j.seq_offset = data_of<int64_t>(offset, "seq_nvshmem_offset");
+  j.seq_tokens = data_of<int64_t>(tokens, "seq_tokens");
+}
+distca_exchange_job make_job(int64_t kind, std::initializer_list<const Tensor *> parts, const Tensor &offset, const Tensor &tokens, const Tensor *mask = nullptr) {
+  distca_exchange_job j{};
+  j.kind = kind;
+  set_parts(j, parts.begin(), (int64_t)parts.size());
+  set_shards(j, offset, tokens, mask);
+  return j;
+}
+
+// Fills in the job and returns the device of its first tensor.
+c10::Device read_job(PyObject *o, distca_exchange_job &j) {
+  if (!PyTuple_Check(o) || PyTuple_GET_SIZE(o) != 8) type_error("a job is a tuple of eight");
+  PyObject *const *f = &PyTuple_GET_ITEM(o, 0);
+  j = distca_exchange_job{};
+  j.kind = int_arg(f[0]);
+  const bool replicas = j.kind == DISTCA_JOB_REPLICAS || j.kind == DISTCA_JOB_REPLICA_SUM;
+  const Tensor &offset = tensor_arg(f[2], "seq_nvshmem_offset"), &tokens = tensor_arg(f[3], "seq_tokens");
+
+  PyObject *list = f[1];
+  if (!PyList_Check(list) && !PyTuple_Check(list)) type_error(std::string("the parts of a token are a list or a tuple of tensors, not ") + Py_TYPE(list)->tp_name);
+  const Py_ssize_t n = PySequence_Fast_GET_SIZE(list);
+  if (n < 1 || n > DISTCA_TOKEN_MAX_PARTS) fail("a token has one to " + std::to_string(DISTCA_TOKEN_MAX_PARTS) + " parts");
+  const Tensor *parts[DISTCA_TOKEN_MAX_PARTS];
+  for (Py_ssize_t i = 0; i < n; ++i) parts[i] = &tensor_arg(PySequence_Fast_GET_ITEM(list, i), "tensor");
+  set_parts(j, parts, n);
+  if (f[5] != Py_None) j.token_bytes = int_arg(f[5]);
+  const Tensor *mask = replicas || f[4] != Py_None ? &tensor_arg(f[4], replicas ? "do_shard" : "copy_seq_mask") : nullptr;
+  set_shards(j, offset, tokens, mask);
+  if (j.kind == DISTCA_JOB_COPY_SUM) {
     const Tensor &num_copies = tensor_arg(f[6], "num_copies"), &start = tensor_arg(f[7], "copy_start_id");
     check_tensor(num_copies, 1, "num_copies");
     check_tensor(start, 2, "copy_start_id");
@@ -434,9 +453,15 @@ c10::Device read_job(PyObject *o, distca_exchange_job &j) {
     j.copy_start = data_of<int64_t>(start, "copy_start_id");
     j.max_copies = start.size(1);
   }
-  j.seq_offset = data_of<int64_t>(offset, "seq_nvshmem_offset");
-  j.seq_tokens = data_of<int64_t>(tokens, "seq_tokens");
-  return device;
+  return parts[0]->device();
+}
+
+// The launch goes to the device, and its stream, that made the tensors: the buffer may be another device's memory
+void run_exchange(const distca_exchange_job *jobs, int32_t n, const Tensor &buffer, bool to_buffer, c10::Device device) {
+  if (!buffer.is_cuda()) fail("tensor buffer must be on CUDA");
+  const Unlocked u;
+  const OnDevice on(device);
+  check_rc(distca_exchange(jobs, n, buffer.data_ptr(), to_buffer, on.stream), "exchange");
 }
 
 PyObject *py_exchange(PyObject *, PyObject *const *a, Py_ssize_t n) {   // jobs, buffer, to_buffer
@@ -448,19 +473,57 @@ PyObject *py_exchange(PyObject *, PyObject *const *a, Py_ssize_t n) {   // jobs,
   const Py_ssize_t num = PySequence_Fast_GET_SIZE(a[0]);
   if (num > DISTCA_EXCHANGE_MAX_JOBS) fail("at most " + std::to_string(DISTCA_EXCHANGE_MAX_JOBS) + " jobs per launch");
   distca_exchange_job jobs[DISTCA_EXCHANGE_MAX_JOBS];
-  // the launch goes to the device, and its stream, that made the tensors: the buffer may be another device's memory
   std::optional<c10::Device> device;
   for (Py_ssize_t i = 0; i < num; ++i) {
     const c10::Device d = read_job(PySequence_Fast_GET_ITEM(a[0], i), jobs[i]);
     if (!device) device = d;
   }
-  if (!buffer.is_cuda()) fail("tensor buffer must be on CUDA");
-  {
-    const Unlocked u;
-    const OnDevice on(device ? *device : buffer.device());
-    check_rc(distca_exchange(jobs, (int32_t)num, buffer.data_ptr(), to_buffer, on.stream), "exchange");
-  }
+  run_exchange(jobs, (int32_t)num, buffer, to_buffer, device ? *device : buffer.device());
   Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
+// The two halves of the linear side's forward in one call each: with the jobs made and the results allocated in Python the host took longer
+// over them than the device (1021 tokens, 8/2 heads, a pass among others: 14.7 us, by these two 11.8; the kernels take 8.5).
+// q shards as they are, every k / v shard once per destination: (q, k, v, do_shard, q_tokens, k_tokens, q_offset, k_offset, v_offset, buffer)
+PyObject *py_pack_qkv(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  expect(n, 10, "pack_qkv");
+  const Tensor q = tensor_arg(a[0], "tensor").contiguous(), k = tensor_arg(a[1], "tensor").contiguous(), v = tensor_arg(a[2], "tensor").contiguous();
+  const Tensor &mask = tensor_arg(a[3], "do_shard"), &q_tokens = tensor_arg(a[4], "seq_tokens"), &k_tokens = tensor_arg(a[5], "seq_tokens");
+  const char *off = "seq_nvshmem_offset";
+  const distca_exchange_job jobs[3] = {make_job(DISTCA_JOB_PLAIN, {&q}, tensor_arg(a[6], off), q_tokens),
+                                       make_job(DISTCA_JOB_REPLICAS, {&k}, tensor_arg(a[7], off), k_tokens, &mask),
+                                       make_job(DISTCA_JOB_REPLICAS, {&v}, tensor_arg(a[8], off), k_tokens, &mask)};
+  run_exchange(jobs, 3, tensor_arg(a[9], "buffer"), true, q.device());
+  PyObject *t = PyTuple_New(3);
+  if (!t) throw python_error();
+  PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(q));
+  PyTuple_SET_ITEM(t, 1, THPVariable_Wrap(k));
+  PyTuple_SET_ITEM(t, 2, THPVariable_Wrap(v));
+  return t;
+  END_HANDLE_TH_ERRORS
+}
+
+// The [out | lse | pad] tokens of a reply taken apart: (buffer, tensor on the device of the results, dtype of out, tokens, elements of out,
+// bytes of lse, bytes of a token, offset, lengths) -> out [tokens, 1, elements], lse [tokens, bytes]
+PyObject *py_unpack_reply(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  expect(n, 9, "unpack_reply");
+  if (!THPDtype_Check(a[2])) type_error(std::string("dtype must be a torch.dtype, not ") + Py_TYPE(a[2])->tp_name);
+  const auto dtype = reinterpret_cast<THPDtype *>(a[2])->scalar_type;
+  const int64_t rows = int_arg(a[3]), elements = int_arg(a[4]), lse_bytes = int_arg(a[5]);
+  const auto on_device = at::TensorOptions().device(tensor_arg(a[1], "q").device());
+  const Tensor out = at::empty({rows, 1, elements}, on_device.dtype(dtype)), lse = at::empty({rows, lse_bytes}, on_device.dtype(at::kByte));
+  const Tensor out_rows = out.view({rows, elements});
+  distca_exchange_job j = make_job(DISTCA_JOB_PLAIN, {&out_rows, &lse}, tensor_arg(a[7], "seq_nvshmem_offset"), tensor_arg(a[8], "seq_tokens"));
+  j.token_bytes = int_arg(a[6]);
+  run_exchange(&j, 1, tensor_arg(a[0], "buffer"), false, out.device());
+  PyObject *t = PyTuple_New(2);
+  if (!t) throw python_error();
+  PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(out));
+  PyTuple_SET_ITEM(t, 1, THPVariable_Wrap(lse));
+  return t;
   END_HANDLE_TH_ERRORS
 }
 
@@ -483,6 +546,8 @@ PyMethodDef methods[] = {
     {"varlen_bwd", fast(py_varlen_bwd), METH_FASTCALL, nullptr},
     {"core_attention", fast(py_core_attention), METH_FASTCALL, nullptr},
     {"exchange", fast(py_exchange), METH_FASTCALL, nullptr},
+    {"pack_qkv", fast(py_pack_qkv), METH_FASTCALL, nullptr},
+    {"unpack_reply", fast(py_unpack_reply), METH_FASTCALL, nullptr},
     {"current_stream", fast(py_current_stream), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };

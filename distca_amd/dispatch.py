@@ -19,6 +19,7 @@ from typing import List, Sequence, Tuple
 import torch
 from torch import Tensor
 
+from . import _lib
 from .ops import (TOKEN_OF_PARTS_MAX_BYTES, DispatcherWrapper, _transport_buffer, a2a_memcpy_cp, a2a_memcpy_non_cp, a2a_memcpy_non_cp_multi,
                   copy_sum_job, exchange, plain_job, pre_a2a_grad_acc, replicas_job, token_part, whole_vectors)
 from .utils import round_up
@@ -92,12 +93,11 @@ def pre_a2a_qkv(
     """Sender side.  Forward (dispatch.py:30-38): q shards as they are, every k / v shard once per destination
     that needs it.  Backward (:39-56): the gradients of duplicate k / v copies are first summed into their main
     copy, then q and only the main copies go out."""
-    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
     buffer = _transport_buffer(buffer, instance_id, True)
     if is_fwd:
-        exchange([plain_job([q], q_send_buffer_offset, q_seq_tokens), replicas_job(k, kv_dispatch_mask, k_send_buffer_offset, k_seq_tokens),
-                  replicas_job(v, kv_dispatch_mask, v_send_buffer_offset, k_seq_tokens)], buffer, True)
-        return q, k, v
+        return _lib.host().pack_qkv(q, k, v, kv_dispatch_mask, q_seq_tokens, k_seq_tokens, q_send_buffer_offset, k_send_buffer_offset,
+                                    v_send_buffer_offset, buffer)
+    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
     if kv_grad_copy_shard_mask is None:
         raise AssertionError("kv grad copy requires a dedup mask.")
     jobs = [plain_job([q], q_send_buffer_offset, _lengths_of(q_seq_tokens, q_send_buffer_offset))]

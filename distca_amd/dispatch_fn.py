@@ -21,9 +21,8 @@ def pre_all2all_layout_transfer(q: Tensor, k: Tensor, v: Tensor, metadata: Allto
     """Sender packs its shards into the send buffer (dispatch_fn.py:31-70): q plainly, k and v
     once per destination replica; an attention output (is_qkv False) like q."""
     if is_qkv:
-        pre_a2a_qkv(q.contiguous(), k.contiguous(), v.contiguous(), metadata.kv_replica_mask,
-                    metadata.seq_lens[0].send_seqlens, metadata.seq_lens[1].send_seqlens, *metadata.send_memcpy_metadata,
-                    is_fwd=True, buffer=buffer)
+        pre_a2a_qkv(q, k, v, metadata.kv_replica_mask, metadata.seq_lens[0].send_seqlens, metadata.seq_lens[1].send_seqlens,
+                    *metadata.send_memcpy_metadata, is_fwd=True, buffer=buffer)
     else:
         assert k is None and v is None
         pre_a2a_attn_out(q.contiguous(), metadata.seq_lens[0].send_seqlens, *metadata.send_memcpy_metadata, buffer=buffer)

@@ -583,13 +583,10 @@ def post_a2a_attn_out_with_lse(recv_buffer: Optional[Tensor], q: Tensor, num_hea
     token_bytes = cols * itemsize
     if whole_vectors(hidden_bytes, lse_bytes, token_bytes) and hidden_bytes + lse_bytes <= token_bytes <= TOKEN_OF_PARTS_MAX_BYTES:
         # both parts straight from the buffer
-        attn_out = torch.empty((rows, hidden), dtype=dtype, device=q.device)
-        softmax_lse_bytes = torch.empty((rows, lse_bytes), dtype=torch.uint8, device=q.device)
-        source = _transport_buffer(recv_buffer, instance_id, False)
-        exchange([plain_job([attn_out, softmax_lse_bytes], metadata.recv_memcpy_metadata[0], metadata.seq_lens[0].recv_seqlens,
-                            token_bytes=token_bytes)], source, False)
+        parts = _lib.host().unpack_reply(_transport_buffer(recv_buffer, instance_id, False), q, dtype, rows, hidden, lse_bytes, token_bytes,
+                                         metadata.recv_memcpy_metadata[0], metadata.seq_lens[0].recv_seqlens)
         _unpacked(recv_buffer, switch_buffer, instance_id)
-        return attn_out.unsqueeze(1), softmax_lse_bytes
+        return parts
     recv = torch.empty((rows, cols), dtype=dtype, device=q.device).view(torch.uint8)
     post_a2a_attn_out(recv, metadata.seq_lens[0].recv_seqlens, *metadata.recv_memcpy_metadata, switch_buffer=switch_buffer,
                       instance_id=instance_id, buffer=recv_buffer)
