@@ -98,10 +98,14 @@ __device__ __forceinline__ T *uniform_ptr(T *p) {
   const uint64_t hi = uniform32((uint32_t)(u >> 32)), lo = uniform32((uint32_t)u);
   return reinterpret_cast<T *>((hi << 32) | lo);
 }
+// The base goes through a scalar move: a load that reads a scalar register which a vector instruction (v_readfirstlane, or the v_readlane
+// that brings a parked scalar register back) wrote fewer than five wait states before reads what it held before, and the compiler, which
+// spaces its own loads, does not look into assembly.  A scalar instruction waits for such a register by itself, and what it writes can be
+// read at once.  The move, of the register to itself, also stands between the write of M0 and the load, which need a wait state.
 __device__ __forceinline__ void lds_direct_load16(const void *gbase, uint32_t voff, uint32_t lds_base) {
   const uint64_t gb = reinterpret_cast<uint64_t>(gbase);
   const uint64_t gbu = ((uint64_t)uniform32((uint32_t)(gb >> 32)) << 32) | uniform32((uint32_t)gb);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(gbu), "s"(uniform32(lds_base)) : "memory");
+  asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 %1, %1\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(gbu), "s"(uniform32(lds_base)) : "memory");
 }
 // 16 bytes per lane from a per-lane pointer; lane L's data lands at lds_base + 16*L.
 __device__ __forceinline__ void lds_direct_load16_ptr(const void *gptr_lane, uint32_t lds_base) {
@@ -110,7 +114,7 @@ __device__ __forceinline__ void lds_direct_load16_ptr(const void *gptr_lane, uin
 __device__ __forceinline__ void lds_direct_load4_base(const void *gbase, uint32_t voff, uint32_t lds_base) {
   const uint64_t gb = reinterpret_cast<uint64_t>(gbase);
   const uint64_t gbu = ((uint64_t)uniform32((uint32_t)(gb >> 32)) << 32) | uniform32((uint32_t)gb);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(gbu), "s"(uniform32(lds_base)) : "memory");
+  asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 %1, %1\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(gbu), "s"(uniform32(lds_base)) : "memory");
 }
 __device__ __forceinline__ void lds_direct_load4(const void *gptr_lane, uint32_t lds_base) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(gptr_lane), "s"(uniform32(lds_base)) : "memory");
