@@ -374,11 +374,26 @@ next_block:
 
 
   // One tile.  MASKED: the tile straddles the diagonal or the end of the prefix, compare and select per element.
-  auto tile = [&](auto stage, int key0, auto masked) __attribute__((always_inline)) {  // stage: an int or a constant
+  // request(i), i = 0 .. 3: the loads of the tile after the next, each between MFMAs of step 1, which has no arithmetic beside it.  (All four behind
+  // the barrier, from all four waves at once, they held the waves up for a seventh of a tile.)  The first two K fragments are there when a tile
+  // begins: in the middle of step 3 the wave waits for the next tile and reads them, so that neither the barrier nor the reads' latency stands
+  // between two tiles' MFMAs.  131072 packed tokens at 32/8 heads, 18 200 us: with the requests between MFMAs 17 750, with both 17 600 (one box); a
+  // conditional jump around each request instead of a loop of its own for tiles that lie whole took 1.7 % back; four K fragments in flight
+  // instead of two, or one M0 write for all four requests, change nothing: the clock gives up what the cycles gain.
+  elemx8 kf[2];
+  auto landed = [&]() {
+    // tile p has landed when at most the loads of tile p + 1 are still on their way
+    wait_vm<kLoadsPerTile>();
+    fence();
+    asm volatile("s_barrier" ::: "memory");
+    fence();
+  };
+  auto first_k = [&](uint32_t so, int s) { kf[s] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(k_ad[s] + so)); };
+  auto tile = [&](auto stage, auto next_stage, int key0, auto masked, auto request) __attribute__((always_inline)) {  // stages: ints or constants
     constexpr bool kMasked = decltype(masked)::value;
-    const uint32_t so = (uint32_t)stage * kStageBytes;
+    const uint32_t so = (uint32_t)stage * kStageBytes, so_next = (uint32_t)next_stage * kStageBytes;
     f32x16 sacc[2], dpacc[2];
-    elemx8 kf[2], vf[2];
+    elemx8 vf[2];
     elemx4 ct[kFrags][2];
     auto load_k = [&](int s, int buf) { kf[buf] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(k_ad[s] + so)); };
     auto load_v = [&](int s, int buf) { vf[buf] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(k_ad[s] + so + kTile)); };
@@ -387,8 +402,6 @@ next_block:
       ct[buf][1] = lds_read_tr(lds_ptr(t_ad[4 + (n & 3)] + so + 16 * (n >> 2) * kRow));
     };
     // ---- step 1: S^T = K Q^T
-    load_k(0, 0);
-    load_k(1, 1);
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
       fence();
@@ -402,6 +415,7 @@ next_block:
       fence();
       if (s + 2 < 8) load_k(s + 2, s & 1);
       if (s >= 6) load_v(s - 6, s - 6);  // the first operands of step 2
+      if (s & 1) request(s >> 1);
     }
     // ---- step 2: dP^T = V dO^T; beside the MFMAs, P = exp2(S c - lse2) of two elements per MFMA
     auto p_elem = [&](int m, int r) {
@@ -485,6 +499,9 @@ next_block:
         dqacc[0][n0 & 3] = mfma32(kt0, dsf[0][n0 >> 2], dqacc[0][n0 & 3]);
         fence();
       }
+      if (n == 3) landed();
+      if (n == 4) first_k(so_next, 0);
+      if (n == 5) first_k(so_next, 1);
     }
   };
 
@@ -492,37 +509,49 @@ next_block:
   // wave sees whole (no masking), then tiles on the diagonal or at the end of the prefix (masked), then, for waves
   // whose rows end below those of the block's last wave, tiles that none of their rows sees.  Each kind has a loop
   // of its own with one body; every wave passes the same barriers and makes the same requests in all of them.
-  auto advance = [&](int p) {
-    wait_vm<kLoadsPerTile>();
-    fence();
-    asm volatile("s_barrier" ::: "memory");
-    fence();
-    issue_tile((p + 2) % kStages, p + 2);
-  };
   int p = 0;
-  // four unmasked tiles per round, one per ring stage, as long as the fourth is still unmasked
+  landed();
+  first_k(0, 0);
+  first_k(0, 1);
+  auto none = [](int) {};
+  const uint32_t dst_w = lds0 + 8 * wave * kRow;
+  // four unmasked tiles per round, one per ring stage, as long as the fourth is still unmasked and the tiles requested meanwhile lie
+  // wholly inside the prefix (SEG: and in the present shard)
   for (; p + 3 < ntiles; p += 4) {
-    if (!wave_live || (p + 3) * kKeys + kKeys - 1 > lim_first) break;
-    advance(p);
-    tile(std::integral_constant<int, 0>{}, p * kKeys, std::false_type{});
-    advance(p + 1);
-    tile(std::integral_constant<int, 1>{}, (p + 1) * kKeys, std::false_type{});
-    advance(p + 2);
-    tile(std::integral_constant<int, 2>{}, (p + 2) * kKeys, std::false_type{});
-    advance(p + 3);
-    tile(std::integral_constant<int, 3>{}, (p + 3) * kKeys, std::false_type{});
+    if (!wave_live || (p + 3) * kKeys + kKeys - 1 > lim_first || (!SEG && (p + 6) * kKeys > lk)) break;
+    auto four = [&](auto st) __attribute__((always_inline)) {
+      constexpr int kSt = decltype(st)::value;
+      using Next = std::integral_constant<int, (kSt + 1) % kStages>;
+      if constexpr (SEG) {
+        issue_tile((kSt + 2) % kStages, p + kSt + 2);
+        tile(st, Next{}, (p + kSt) * kKeys, std::false_type{}, none);
+      } else {
+        const elem_t *kt = kbase + (int64_t)(p + kSt + 2) * kKeys * kv_stride, *vt = vbase + (int64_t)(p + kSt + 2) * kKeys * kv_stride;
+        const uint32_t dst = dst_w + ((kSt + 2) % kStages) * kStageBytes;
+        tile(st, Next{}, (p + kSt) * kKeys, std::false_type{}, [&](int i) __attribute__((always_inline)) {
+          lds_direct_load16(i < 2 ? kt : vt, voff[i & 1], dst + (i >> 1) * kTile + (i & 1) * 4 * kRow);
+        });
+      }
+    };
+    four(std::integral_constant<int, 0>{});
+    four(std::integral_constant<int, 1>{});
+    four(std::integral_constant<int, 2>{});
+    four(std::integral_constant<int, 3>{});
   }
   for (; p < ntiles; ++p) {
     if (!wave_live || p * kKeys + kKeys - 1 > lim_first) break;
-    advance(p);
-    tile(p % kStages, p * kKeys, std::false_type{});
+    issue_tile((p + 2) % kStages, p + 2);
+    tile(p % kStages, (p + 1) % kStages, p * kKeys, std::false_type{}, none);
   }
   for (; p < ntiles; ++p) {
     if (!wave_live || p * kKeys > lim_last) break;
-    advance(p);
-    tile(p % kStages, p * kKeys, std::true_type{});
+    issue_tile((p + 2) % kStages, p + 2);
+    tile(p % kStages, (p + 1) % kStages, p * kKeys, std::true_type{}, none);
   }
-  for (; p < ntiles; ++p) advance(p);
+  for (; p < ntiles; ++p) {
+    issue_tile((p + 2) % kStages, p + 2);
+    landed();
+  }
   wait_vm<0>();  // nothing may still be on its way into LDS when the workgroup ends
 
   // MERGE: the next block's first rows are requested now and arrive while this block's results are stored; the dQ rows
