@@ -65,6 +65,12 @@ __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 __device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
+// The lane's number, made where it is asked for (what the compiler knows how to make it makes once, and parks).
+__device__ __forceinline__ int lane_now() {
+  int l;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+  return l;
+}
 // This file is compiled with the compiler's default choice of MFMA form, which at 512 registers per wave keeps
 // every MFMA result in the accumulation registers: right for the 256 dK / dV accumulators, which only MFMAs touch
 // and which fill that file exactly.  The S and dP accumulators, which the vector ALU reads and overwrites, must

@@ -91,6 +91,17 @@ def test_prefix_lengths_around_tile_and_ring_boundaries(cuda, hq, hkv):
     _run(q_lens, k_lens, hq, hkv, 21, cuda)
 
 
+@pytest.mark.parametrize("hq,hkv", [(8, 8), (16, 8), (32, 8)])
+def test_runs_of_whole_tiles_and_blocks(cuda, hq, hkv):
+    """Documents long enough for the runs of whole tiles (dQ) and whole blocks (dK/dV) whose requests stand between the MFMAs, of lengths that end
+    a key, a row and a block either side of where the runs end, and enough of them that dK/dV items of both walk directions are among them
+    (more key blocks than compute units serve a kv head).  At most four query heads per kv head: a bf16-rounded P of about 1 per head (a
+    document's first rows) puts a deviation of 2^-9 / sqrt(3) * sqrt(1.5 heads) on an entry of dV there, and five of them, the largest of the
+    eighty thousand such entries here, are 1.4e-2 for four heads and, at the bar of 2e-2, 2.0e-2 for eight."""
+    lens = [1031, 769, 770, 768, 767, 991, 1024, 1023, 1025, 640, 832]
+    _run(lens, lens, hq, hkv, 23, cuda)
+
+
 def test_shared_kv_prefix(cuda):
     """Three shards of one 600-token document reading one stored KV copy."""
     _run([200, 150, 250], [200, 350, 600], 8, 2, 5, cuda, kv_offsets=[0, 0, 0], total_k=600)
