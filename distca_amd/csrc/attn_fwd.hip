@@ -361,38 +361,44 @@ next_block:
   f32x16 sacc[MSUB][2];
   elemx8 pf[MSUB][4];
   auto tile_active = [&](int j) { return wave_live && j * kFwdKV <= lim_last; };
+  auto nothing = [](auto...) {};
+  using None = std::integral_constant<int, -1>;
 
   // ---- S^T = K Q^T : [64 keys] x [32*MSUB rows]
-  auto phase_s = [&](int j, auto par) __attribute__((always_inline)) {  // par: parity of j, known at compile time
+  constexpr int kPf = 2;  // K fragments are requested kPf steps before the MFMAs that use them
+  elemx8 kf[kPf][2];
+  auto load_k = [&](auto par, int s) __attribute__((always_inline)) {  // par: parity of the tile, known at compile time
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) kf[s % kPf][kb] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(k_ad[s] + decltype(par)::value * kKTile + kb * 32 * kRowB));
+  };
+  auto first_k = [&](auto par) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < kPf; ++s) load_k(par, s);
+  };
+  // (the first fragments have been asked for; all_read() is called ahead of the last MFMAs, which need the last of them)
+  auto phase_s = [&](auto par, auto all_read) __attribute__((always_inline)) {
 #pragma unroll
     for (int m = 0; m < MSUB; ++m)
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) sacc[m][kb][r] = 0.f;
-    constexpr int kPf = 2;  // K fragments are requested kPf steps before the MFMAs that use them
-    elemx8 kf[kPf][2];
-    auto load_k = [&](int s, int buf) {
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb) kf[buf][kb] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(k_ad[s] + decltype(par)::value * kKTile + kb * 32 * kRowB));
-    };
-#pragma unroll
-    for (int s = 0; s < kPf; ++s) load_k(s, s);
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
       __builtin_amdgcn_sched_barrier(0);
+      if (s == 7) all_read();
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int m = 0; m < MSUB; ++m) sacc[m][kb] = mfma32(kf[s % kPf][kb], qf[m][s], sacc[m][kb]);
       __builtin_amdgcn_sched_barrier(0);
-      if (s + kPf < 8) load_k(s + kPf, s % kPf);
+      if (s + kPf < 8) load_k(par, s + kPf);
     }
   };
   // ---- mask, online softmax (log2 domain, one query row per lane pair), P as bf16 B operand
-  auto phase_x = [&](int j) __attribute__((always_inline)) {
+  auto phase_x = [&](int j, auto whole) __attribute__((always_inline)) {  // whole: every row of the wave sees the whole tile
     const int key0 = j * kFwdKV;
-    if (key0 + kFwdKV - 1 > lim_first) {  // the tile straddles the diagonal or the end of the prefix
+    if (!decltype(whole)::value && key0 + kFwdKV - 1 > lim_first) {  // the tile straddles the diagonal or the end of the prefix
 #pragma unroll
       for (int m = 0; m < MSUB; ++m)
 #pragma unroll
@@ -456,23 +462,29 @@ next_block:
     }
   };
   // ---- O^T += V^T P^T : [128 d] x [32*MSUB rows], contraction over the 64 keys
-  auto phase_pv = [&](int j, auto par) __attribute__((always_inline)) {
-    constexpr int kPfV = 4;  // V^T fragments are requested four MFMAs ahead
-    elemx4 vf[kPfV][2];
-    auto load_v = [&](int u, int buf) {  // u = 4*t + db
-      const uint32_t vo = decltype(par)::value * kVTile + 16 * (u >> 2) * kRowB;
-      vf[buf][0] = lds_read_tr(lds_ptr(v_ad[u & 3] + vo));
-      vf[buf][1] = lds_read_tr(lds_ptr(v_ad[4 + (u & 3)] + vo + 8 * kRowB));
-    };
+  constexpr int kPfV = 4;  // V^T fragments are requested four MFMAs ahead
+  elemx4 vf[kPfV][2];
+  auto load_v = [&](auto par, int u) __attribute__((always_inline)) {  // u = 4*t + db
+    const uint32_t vo = decltype(par)::value * kVTile + 16 * (u >> 2) * kRowB;
+    vf[u % kPfV][0] = lds_read_tr(lds_ptr(v_ad[u & 3] + vo));
+    vf[u % kPfV][1] = lds_read_tr(lds_ptr(v_ad[4 + (u & 3)] + vo + 8 * kRowB));
+  };
+  auto first_v = [&](auto par) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < kPfV; ++u) load_v(u, u);
+    for (int u = 0; u < kPfV; ++u) load_v(par, u);
+  };
+  // (the first fragments have been asked for; next: the parity of the K tile whose first fragments to ask for, or None; beside(u) is
+  // called after MFMA u)
+  auto phase_pv = [&](auto par, auto next, auto beside) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int m = 0; m < MSUB; ++m) oacc[m][u & 3] = mfma32(cat4(vf[u % kPfV][0], vf[u % kPfV][1]), pf[m][u >> 2], oacc[m][u & 3]);
       __builtin_amdgcn_sched_barrier(0);
-      if (u + kPfV < 16) load_v(u + kPfV, u % kPfV);
+      beside(u);
+      if (u + kPfV < 16) load_v(par, u + kPfV);
+      else if (decltype(next)::value >= 0 && u - (16 - kPfV) < kPf) load_k(next, u - (16 - kPfV));
     }
   };
 
@@ -482,11 +494,11 @@ next_block:
   //   [b(2p),   b(2p+1)):  group 0: PV(p-1), S(p)     group 1: softmax(p-1)
   //   [b(2p+1), b(2p+2)):  group 0: softmax(p)        group 1: PV(p-1), S(p)
   // Tile p of K is read between b(2p) and b(2p+2), tile p of V between b(2p+2) and b(2p+4); every
-  // wave requests K(p+1) and V(p) (those of period 0 ahead of the loop: below) at the start of its softmax half of period p (group 1
-  // right after b(2p), group 0 right after b(2p+1)), into the stages whose last readers finished before b(2p), and
-  // waits for its own requests before b(2p+2).  The MFMA halves are the critical path of a period (one
-  // group's, then the other's); a request holds its wave for a hundred cycles or so, and in front of
-  // group 0's MFMA half that time showed in the period (-3 % with the requests behind it).
+  // wave requests K(p+1) and V(p) (those of period 0 ahead of the loop: below) after b(2p), into the stages whose last readers finished
+  // before it, and waits for its own requests before b(2p+2).  The MFMA halves are the critical path of a period (one
+  // group's, then the other's).  A request holds its wave for a hundred cycles or so: group 1 makes its requests right after b(2p), in
+  // its softmax half; group 0 between MFMAs of PV(p-1) where it knows beforehand what to request (fast0), else behind b(2p+1) (in front
+  // of its MFMA half they showed in the period, 3 %).
   // The first two K tiles and the first V tile are requested together ahead of the loop, so that a block waits for memory once: with
   // K(1) and V(0) requested in period 0, as the loop has it, that period (one tile's S to cover them) lasted as long as a second trip.
   // (Together with the rows of O leaving through LDS and Q known to be there, 131072 tokens in documents of 128 / 256 / 512 / 2048, 32/8
@@ -540,26 +552,87 @@ next_block:
   int requests_from = uniform_int(!MERGE || first_made ? 1 : 0);
   asm volatile("" : "+s"(requests_from));
   __syncthreads();  // b0
-  // The period loop is unrolled by two so that the LDS stage of every operand read is a constant folded into
+  // The period loops are unrolled by two so that the LDS stage of every operand read is a constant folded into
   // the instruction's offset field instead of an addition per read between the MFMAs.
   using P0 = std::integral_constant<int, 0>;
   using P1 = std::integral_constant<int, 1>;
-  auto period0 = [&](int p, auto par) __attribute__((always_inline)) {   // par = parity of p
+  auto barrier = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // Between period 0 and fast_end the periods are of one kind for this wave: it sees the tile and the one before whole, and what they
+  // request is whole and there, by scalar base.  They have loops of their own without conditions, in which S's first K fragments are asked for
+  // beside the last MFMAs of PV, and b stands ahead of the last two MFMAs of S, when all reads of K are done.  us before -> after: 131072
+  // packed tokens 13 240 -> 12 670, 8192 tokens 294 -> 282, a tick of 16384 tokens 1 483 -> 1 421, one over a document of 131072 29 390 ->
+  // 27 930, forward of three documents (4096 tokens) 76.7 -> 74.7, lightly loaded server 276 -> 267; documents of 128 to 2048 tokens 980 -> 956.
+  // (Of the 4.3 % the loops without conditions give 2.4, requests by a base that moves on 1.4, group 0's between MFMAs 0.5.  b ahead of the
+  // softmax's last quarter, so that V's first fragments come meanwhile: 13 % slower; V's first fragments ahead of b in group 1: nothing;
+  // K fragments three steps ahead: 2 % slower; group 0's requests three MFMAs earlier: 1.3 % slower.)
+  int fast_end = wave_live ? (lim_first + 1) / kFwdKV : 0;
+  if (fast_end > ntiles - 1) fast_end = ntiles - 1;
+  if (!SEG && fast_end > lk / kFwdKV - 1) fast_end = lk / kFwdKV - 1;
+  fast_end = uniform_int(fast_end);
+  const int64_t tile_bytes = kFwdKV * kv_stride * 2;
+  const uint8_t *k_next = reinterpret_cast<const uint8_t *>(kbase) + 2 * tile_bytes, *v_next = reinterpret_cast<const uint8_t *>(vbase) + tile_bytes;
+  auto request_k = [&](auto par) __attribute__((always_inline)) {  // K(p + 1); par: parity of p
+    issue_rows_fast(reinterpret_cast<const elem_t *>(k_next), kKOff + (1 - decltype(par)::value) * kKTile);
+    k_next += tile_bytes;
+  };
+  auto request_v = [&](auto par) __attribute__((always_inline)) {  // V(p)
+    issue_rows_fast(reinterpret_cast<const elem_t *>(v_next), kVOff + decltype(par)::value * kVTile);
+    v_next += tile_bytes;
+  };
+  // (SEG: there is what lies inside the present shards)
+  auto two_fast = [&](int p) __attribute__((always_inline)) {
+    return p + 1 < fast_end && (!SEG || ((p + 3) * kFwdKV <= krun.lim && (p + 2) * kFwdKV <= vrun.lim));
+  };
+  auto enter_fast = [&](int p) __attribute__((always_inline)) {
+    if constexpr (SEG) {
+      k_next = reinterpret_cast<const uint8_t *>(krun.virt) + (p + 1) * tile_bytes;
+      v_next = reinterpret_cast<const uint8_t *>(vrun.virt) + p * tile_bytes;
+    }
+  };
+  auto fast0 = [&](int p, auto par) __attribute__((always_inline)) {
     using Same = std::integral_constant<int, decltype(par)::value>;
     using Other = std::integral_constant<int, 1 - decltype(par)::value>;
-    if (p > 0 && tile_active(p - 1)) phase_pv(p - 1, Other{});
+    first_v(Other{});
+    phase_pv(Other{}, Same{}, [&](int u) __attribute__((always_inline)) {
+      if (u == 4) request_k(par);
+      if (u == 8) request_v(par);
+    });
+    phase_s(Same{}, barrier);
+    phase_x(p, std::true_type{});
+    wait_vm0();
+    barrier();
+  };
+  auto fast1 = [&](int p, auto par) __attribute__((always_inline)) {
+    using Same = std::integral_constant<int, decltype(par)::value>;
+    using Other = std::integral_constant<int, 1 - decltype(par)::value>;
+    request_k(par);
+    request_v(par);
+    phase_x(p - 1, std::true_type{});
+    barrier();
+    first_v(Other{});
+    phase_pv(Other{}, Same{}, nothing);
+    phase_s(Same{}, [&]() __attribute__((always_inline)) { wait_vm0(); barrier(); });
+  };
+  auto slow0 = [&](int p, auto par) __attribute__((always_inline)) {   // par = parity of p
+    using Same = std::integral_constant<int, decltype(par)::value>;
+    using Other = std::integral_constant<int, 1 - decltype(par)::value>;
+    if (p > 0 && tile_active(p - 1)) { first_v(Other{}); phase_pv(Other{}, None{}, nothing); }
     const bool act = p < ntiles && tile_active(p);
-    if (act) phase_s(p, Same{});
+    if (act) { first_k(Same{}); phase_s(Same{}, nothing); }
     __syncthreads();
     if (p >= requests_from) {
       if (p + 1 < ntiles) issue_k(p + 1);
       if (p < ntiles) issue_v(p);
     }
-    if (act) phase_x(p);
+    if (act) phase_x(p, std::false_type{});
     if (p >= requests_from) wait_vm0();
     __syncthreads();
   };
-  auto period1 = [&](int p, auto par) __attribute__((always_inline)) {
+  auto slow1 = [&](int p, auto par) __attribute__((always_inline)) {
     using Same = std::integral_constant<int, decltype(par)::value>;
     using Other = std::integral_constant<int, 1 - decltype(par)::value>;
     if (p >= requests_from) {
@@ -567,24 +640,31 @@ next_block:
       if (p < ntiles) issue_v(p);
     }
     const bool act_prev = p > 0 && tile_active(p - 1);
-    if (act_prev) phase_x(p - 1);
+    if (act_prev) phase_x(p - 1, std::false_type{});
     __syncthreads();
-    if (act_prev) phase_pv(p - 1, Other{});
-    if (p < ntiles && tile_active(p)) phase_s(p, Same{});
+    if (act_prev) { first_v(Other{}); phase_pv(Other{}, None{}, nothing); }
+    if (p < ntiles && tile_active(p)) { first_k(Same{}); phase_s(Same{}, nothing); }
     if (p >= requests_from) wait_vm0();
     __syncthreads();
   };
-  if (grp == 0) {
-    for (int p = 0; p <= ntiles; p += 2) {
-      period0(p, P0{});
-      if (p + 1 <= ntiles) period0(p + 1, P1{});
+  int p = 1;
+  auto work_off = [&](auto fast, auto slow) __attribute__((always_inline)) {
+    auto fast_periods = [&]() __attribute__((always_inline)) {
+      for (enter_fast(p); two_fast(p); p += 2) {
+        fast(p, P1{});
+        fast(p + 1, P0{});
+      }
+    };
+    slow(0, P0{});
+    if constexpr (!SEG) fast_periods();
+    for (; p <= ntiles; p += 2) {
+      if constexpr (SEG) fast_periods();  // (the period below may have found the next shard)
+      slow(p, P1{});
+      if (p + 1 <= ntiles) slow(p + 1, P0{});
     }
-  } else {
-    for (int p = 0; p <= ntiles; p += 2) {
-      period1(p, P0{});
-      if (p + 1 <= ntiles) period1(p + 1, P1{});
-    }
-  }
+  };
+  if (grp == 0) work_off(fast0, slow0);
+  else work_off(fast1, slow1);
 
   // (Where the results go is worked out ahead of those requests: should the compiler have parked a pointer in scratch
   // memory, fetching it back afterwards would wait for the requests as well.)

@@ -712,3 +712,43 @@ def test_kv_shards_read_in_place_equal_dense_tensors(cuda, hq, hkv):
     assert (g[~touched] == 0x3C).all(), "bytes outside the shards' places were written"
     # rows 500..650 of the second document are read by no task: zeros in the dense result, hence in the shards
     assert (dk[int(doc_start[1]) + 500:int(doc_start[2])] == 0).all() and (dv[int(doc_start[1]) + 500:int(doc_start[2])] == 0).all()
+
+
+@pytest.mark.parametrize("hq,hkv,shard_len", [
+    (4, 1, [64, 128, 192, 193, 191, 256, 1, 320, 383, 129, 448]),     # shards end a key either side of a tile's end, runs of both parities
+    (32, 8, [640, 0, 65, 575, 1024, 63, 1, 449]),                     # long runs, shards shorter than a tile between them
+    (8, 2, [2560]),                                                   # one shard
+    (8, 8, [37] * 60)])                                               # no tile inside one shard
+def test_forward_runs_of_tiles_inside_shards(cuda, hq, hkv, shard_len):
+    """The forward's loops over tiles that lie inside one shard begin and end where shards do: out and lse over shards in a buffer (every other
+    one from its far end, K apart from V) equal bit for bit what dense tensors give, for prefixes that end around tiles' ends."""
+    import ctypes
+    from distca_amd import _lib
+    from distca_amd.fused_comm_attn import _params, ca_varlen_fwd
+    d, rows = 128, sum(shard_len)
+    k_lens = [rows, rows - 1, rows // 2 // 64 * 64, rows // 2 // 64 * 64 + 1, 65, 700]
+    q_lens = [min(n, m) for n, m in zip(k_lens, [300, 64, 129, 257, 65, 700])]
+    q, k, v, _ = (t.to(cuda) for t in make_qkv(sum(q_lens), rows, hq, hkv, d, 5))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=cuda)
+    cu_q, cu_k = i32([0] + list(np.cumsum(q_lens))), i32([0] + list(np.cumsum(k_lens)))
+    off = i32([0] * len(q_lens))
+    out, lse = ca_varlen_fwd(q, k, v, cu_q, cu_k, max(q_lens), max(k_lens), kv_task_offsets=off)
+    start, rb, ns = np.concatenate([[0], np.cumsum(shard_len)]), hkv * d * 2, len(shard_len)
+    places = list(range(0, ns, 2)) + list(range(ns - 1 - ns % 2, 0, -2))
+    buf, k_off, v_off = [], [0] * ns, [0] * ns
+    for offs, x in ((k_off, k), (v_off, v)):
+        for s in places:
+            offs[s] = sum(b.numel() for b in buf)
+            buf.append(x[start[s]:start[s + 1]].reshape(-1).view(torch.uint8))
+    buf = torch.cat(buf)
+    tables = [i32(list(start)), torch.tensor(k_off, device=cuda), torch.tensor(v_off, device=cuda), i32([0] * len(q_lens))]
+    shards = _lib.KvShards(ns, *[t.data_ptr() for t in tables], None, None)
+    p = _params(len(q_lens), sum(q_lens), rows, hq, hkv, d, max(q_lens), max(k_lens), d ** -0.5, True, True)
+    lib = _lib.load()
+    ws = torch.empty((int(lib.distca_ca_fwd_workspace_preferred_bytes(ctypes.byref(p))),), dtype=torch.uint8, device=cuda)
+    out2, lse2 = torch.empty_like(out), torch.empty_like(lse)
+    _lib.check(lib.distca_ca_fwd_buffers(q.data_ptr(), None, 0, buf.data_ptr(), buf.data_ptr(), ctypes.byref(shards), out2.data_ptr(), None, 0,
+                                         lse2.data_ptr(), cu_q.data_ptr(), cu_k.data_ptr(), off.data_ptr(), ctypes.byref(p), ws.data_ptr(),
+                                         ws.numel(), torch.cuda.current_stream().cuda_stream), "fwd_buffers")
+    torch.cuda.synchronize()
+    assert torch.equal(out2, out) and torch.equal(lse2, lse)
