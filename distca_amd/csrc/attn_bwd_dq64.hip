@@ -516,30 +516,36 @@ next_block:
   auto none = [](int) {};
   const uint32_t dst_w = lds0 + 8 * wave * kRow;
   // four unmasked tiles per round, one per ring stage, as long as the fourth is still unmasked and the tiles requested meanwhile lie
-  // wholly inside the prefix (SEG: and in the present shard)
-  for (; p + 3 < ntiles; p += 4) {
-    if (!wave_live || (p + 3) * kKeys + kKeys - 1 > lim_first || (!SEG && (p + 6) * kKeys > lk)) break;
-    auto four = [&](auto st) __attribute__((always_inline)) {
-      constexpr int kSt = decltype(st)::value;
-      using Next = std::integral_constant<int, (kSt + 1) % kStages>;
-      if constexpr (SEG) {
-        issue_tile((kSt + 2) % kStages, p + kSt + 2);
-        tile(st, Next{}, (p + kSt) * kKeys, std::false_type{}, none);
-      } else {
-        const elem_t *kt = kbase + (int64_t)(p + kSt + 2) * kKeys * kv_stride, *vt = vbase + (int64_t)(p + kSt + 2) * kKeys * kv_stride;
+  // wholly inside the prefix (SEG: and in the present shard; the loop of single tiles comes back to this one behind every shard's end: tick of
+  // 16384 tokens 1 864 us -> 1 817, tick over a document of 131072 tokens 36 870 -> 35 940, with requests behind the barrier before)
+  int whole_end = wave_live ? (lim_first + 1) / kKeys : 0;  // the tiles that every row of the wave sees whole
+  whole_end = uniform_int(whole_end < ntiles ? whole_end : ntiles);
+  auto rounds = [&]() __attribute__((always_inline)) {
+    for (; p + 4 <= whole_end && (p + 6) * kKeys <= (SEG ? run_lim : lk); p += 4) {
+      auto four = [&](auto st) __attribute__((always_inline)) {
+        constexpr int kSt = decltype(st)::value;
+        using Next = std::integral_constant<int, (kSt + 1) % kStages>;
+        const int64_t at = (int64_t)(p + kSt + 2) * kKeys * kv_stride;
+        const elem_t *kt = (SEG ? kvirt : kbase) + at, *vt = (SEG ? vvirt : vbase) + at;
         const uint32_t dst = dst_w + ((kSt + 2) % kStages) * kStageBytes;
         tile(st, Next{}, (p + kSt) * kKeys, std::false_type{}, [&](int i) __attribute__((always_inline)) {
           lds_direct_load16(i < 2 ? kt : vt, voff[i & 1], dst + (i >> 1) * kTile + (i & 1) * 4 * kRow);
         });
+      };
+      four(std::integral_constant<int, 0>{});
+      four(std::integral_constant<int, 1>{});
+      four(std::integral_constant<int, 2>{});
+      four(std::integral_constant<int, 3>{});
+    }
+  };
+  if constexpr (!SEG) rounds();
+  for (; p < whole_end; ++p) {
+    if constexpr (SEG) {
+      if (p % kStages == 0) {
+        rounds();
+        if (p >= whole_end) break;
       }
-    };
-    four(std::integral_constant<int, 0>{});
-    four(std::integral_constant<int, 1>{});
-    four(std::integral_constant<int, 2>{});
-    four(std::integral_constant<int, 3>{});
-  }
-  for (; p < ntiles; ++p) {
-    if (!wave_live || p * kKeys + kKeys - 1 > lim_first) break;
+    }
     issue_tile((p + 2) % kStages, p + 2);
     tile(p % kStages, (p + 1) % kStages, p * kKeys, std::false_type{}, none);
   }
