@@ -38,12 +38,14 @@ constexpr int kRowB = 256;    // bytes per K or V row in LDS (unpadded; chunk c 
 constexpr int kKTile = kFwdKV * kRowB;
 constexpr int kVTile = kFwdKV * kRowB;
 constexpr int kKOff = 0, kVOff = 2 * kKTile;  // two K stages, then two V stages
-// Behind the tiles the rows of O on their way out, 8 KB of a wave's own (see the epilogue); at 256 registers a wave the workgroup has
-// its compute unit, and its LDS, to itself anyway.
-constexpr int kOutOff = 2 * kKTile + 2 * kVTile, kOutWave = 32 * kRowB;
+// Behind the tiles the rows of Q on their way in, 8 KB of a wave's own, and half rows of O on their way out, 4 KB (see the epilogue); at 256
+// registers a wave the workgroup has its compute unit, and its LDS, to itself anyway.
+constexpr int kQOff = 2 * kKTile + 2 * kVTile, kQWave = 32 * kRowB;
+constexpr int kOutOff = kQOff + kFwdWaves * kFwdMsub * kQWave, kOutWave = 32 * kRowB / 2;
 constexpr int kFwdLds = kOutOff + kFwdWaves * kFwdMsub * kOutWave;
+static_assert(kFwdLds <= 160 * 1024, "LDS of a compute unit");
 constexpr int kDirectTasks = 256;    // batches without a list: at most so many tasks to look through
-constexpr int kOutStores = 32 / 4;   // store instructions of a sub-block's rows
+constexpr int kOutStores = 2 * 32 / 8;   // store instructions of a sub-block's rows
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
@@ -213,17 +215,14 @@ next_block:
   uint8_t *obytes = reinterpret_cast<uint8_t *>(a.out) + uniform_int64(a.out_task_off ? a.out_task_off[task] : (int64_t)q0 * a.out_tok_bytes);
   int row[MSUB], tok[MSUB], lim[MSUB];
   bool valid[MSUB];
-  const elem_t *qptr[MSUB];
 #pragma unroll
   for (int m = 0; m < MSUB; ++m) {
     row[m] = row_wg + (wave * MSUB + m) * 32 + l32;
     valid[m] = row[m] < nrows;
     tok[m] = row[m] / G;
-    const int hg = row[m] - tok[m] * G;
     int lm = a.causal ? tok[m] + shift : lk - 1;
     if (lm > lk - 1) lm = lk - 1;
     lim[m] = lm;
-    qptr[m] = reinterpret_cast<const elem_t *>(qbytes + (int64_t)tok[m] * a.q_tok_bytes) + (kvh * G + hg) * kHeadDim;
   }
   // wave-uniform limits: first row's limit decides whether a tile needs masking, last row's
   // whether the wave has anything to do in it.
@@ -239,24 +238,37 @@ next_block:
     if (lim_last > lk - 1) lim_last = lk - 1;
   }
 
-  // ---- Q fragments (B operand of S^T = K Q^T): lane holds row l32, d = 16*s + 8*g .. +7
-  auto load_q = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int m = 0; m < MSUB; ++m) {
-#pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        if (valid[m]) qf[m][s] = *reinterpret_cast<const elemx8 *>(qptr[m] + 16 * s + 8 * g);
-        else qf[m][s] = elemx8{0, 0, 0, 0, 0, 0, 0, 0};
-      }
-    }
-  };
-  if constexpr (!MERGE) load_q();
-
   // ---- K/V tile fetch: wave w brings rows 16w .. 16w+15 of the K tile and of the V tile, four
   // rows per instruction; lane p fetches the chunk that belongs at chunk position p%16 of row p/16
   const int64_t kv_stride = (int64_t)a.hkv * kHeadDim;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(DISTCA_LDS uint8_t *)lds;
   const int uwave = __builtin_amdgcn_readfirstlane(wave);
+  // ---- Q: the wave's rows of the block whose first row is row0 come through LDS, four whole rows per instruction (a row past the task: the last
+  // one again; nothing of it is stored), and each lane takes its fragments from there (B operand of S^T = K Q^T: row l32, d = 16*s + 8*g .. +7).
+  // Loaded straight into that layout, an instruction touched 32 rows, and the address unit takes about a cycle for every line: of a 30 us block
+  // of short documents these loads took one and a half.  us before -> after: documents of 128 to 2048 tokens (65536) 924 -> 881, three documents
+  // (4096) 71.4 -> 69.8, 8192 tokens 270 -> 265, 389 tokens at 4/1 heads 15.7 -> 14.8, 131072 packed tokens 11 960 -> 11 920.
+  auto request_q = [&](int row0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int m = 0; m < MSUB; ++m)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int rl = 4 * i + (lane >> 4);
+        int r = row0 + (uwave * MSUB + m) * 32 + rl;
+        if (r > nrows - 1) r = nrows - 1;
+        const int t = div_group(r);
+        const uint8_t *src = qbytes + (int64_t)t * a.q_tok_bytes + (kvh * G + (r - t * G)) * (kHeadDim * 2) + (((lane & 15) ^ tile_swz(rl)) << 4);
+        lds_direct_load16_ptr(src, lds0 + kQOff + (uwave * MSUB + m) * kQWave + 4 * i * kRowB);
+      }
+  };
+  auto take_q = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int m = 0; m < MSUB; ++m)
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+        qf[m][s] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(lds0 + kQOff + (uwave * MSUB + m) * kQWave + l32 * kRowB + (((2 * s + g) ^ tile_swz(l32)) << 4)));
+  };
+  if constexpr (!MERGE) request_q(row_wg);
   const elem_t *kbase = a.k + (SEG ? 0 : (int64_t)ks * kv_stride) + kvh * kHeadDim;
   const elem_t *vbase = a.v + (SEG ? 0 : (int64_t)ks * kv_stride) + kvh * kHeadDim;
   // SEG: the shards that hold the rows of the K tile and of the V tile requested next (the K requests run a tile ahead)
@@ -504,7 +516,7 @@ next_block:
   // (Together with the rows of O leaving through LDS and Q known to be there, 131072 tokens in documents of 128 / 256 / 512 / 2048, 32/8
   // heads: 958 / 1010 / 1151 / 2798 -> 854 / 857 / 1014 / 2725 us; 131072 packed tokens 12.86 -> 12.72 ms.)
   // MERGE: what the item's next block starts with is requested when this block's tile loop is over, so that it
-  // arrives while the results are normalised and stored: its Q rows (the Q registers are free: every S of this block
+  // arrives while the results are normalised and stored: its Q rows (their place is free: every S of this block
   // is done) and those tiles (no wave reads a stage any more: the last barrier of the loop lies behind every
   // phase; they are the same for every block of a task).  The run and cursor objects the request goes through are
   // set up afresh by the next block.  (Made from inside the loop's last
@@ -516,17 +528,7 @@ next_block:
     if (n > 1) issue_k(1);
   };
   auto request_next_block = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int m = 0; m < MSUB; ++m) {
-      const int nrow = row[m] + kRows;
-      const int ntok = nrow / G;
-      const elem_t *np = reinterpret_cast<const elem_t *>(qbytes + (int64_t)ntok * a.q_tok_bytes) + (kvh * G + (nrow - ntok * G)) * kHeadDim;
-#pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        if (nrow < nrows) qf[m][s] = *reinterpret_cast<const elemx8 *>(np + 16 * s + 8 * g);
-        else qf[m][s] = elemx8{0, 0, 0, 0, 0, 0, 0, 0};
-      }
-    }
+    request_q(row_wg + kRows);
     krun = vrun = Run{kbase, SEG ? 0 : lk};
     vrun.virt = vbase;
     if constexpr (SEG) {
@@ -538,7 +540,7 @@ next_block:
   const int grp = uwave >> 2;
   // first_made: nothing is left of period 0's requests (else it repeats V(0), to the same place)
   if (!MERGE || !requested) {
-    if constexpr (MERGE) load_q();  // (here, so that no path leads from these loads past the wait for them)
+    if constexpr (MERGE) request_q(row_wg);
     if (ntiles > 0) request_first(ntiles);
     wait_vm_known<0>();
   } else {
@@ -547,6 +549,7 @@ next_block:
     wait_vm_known<kOutStores * MSUB>();
     first_made = first_made || ntiles == 1;
   }
+  take_q();
   // the first period that makes requests of its own (opaque: known to the compiler, it becomes a first iteration of its own, and the
   // registers of the two spill)
   int requests_from = uniform_int(!MERGE || first_made ? 1 : 0);
@@ -697,32 +700,35 @@ next_block:
 
   // ---- epilogue: normalise, write O (bf16) and LSE (fp32, natural log).  A lane holds half of its row in pieces of 8 bytes (registers
   // 4*cq .. 4*cq+3 of block db hold d0 .. d0+3); stored from there, an instruction touched 32 rows.  The pieces go to the wave's
-  // 8 KB behind the tiles, in the tiles' swizzled row layout, and leave from there four whole rows per instruction.
+  // 4 KB of LDS, half of every row at a time (Q's rows of the next block may be on their way to the other 8 KB), and leave from there in whole
+  // cache lines, eight rows per instruction.
   auto store_rows = [&](auto all) __attribute__((always_inline)) {  // all: every row of the block exists
 #pragma unroll
     for (int m = 0; m < MSUB; ++m) {
       const float l_tot = pair_sum(l_run[m]);
       const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
       const uint32_t out_w = lds0 + kOutOff + (uwave * MSUB + m) * kOutWave;
-      const uint32_t wr = out_w + l32 * kRowB + 8 * g;
 #pragma unroll
-      for (int db = 0; db < 4; ++db)
+      for (int h = 0; h < 2; ++h) {  // half rows: d = 64 h .. 64 h + 63
 #pragma unroll
-        for (int cq = 0; cq < 4; ++cq) {
-          // d0 = 16 db + 64 (cq >> 1) + 8 (cq & 1) + 4 g: chunk 2 db + 8 (cq >> 1) + (cq & 1), half g
-          const int chunk = 2 * db + 8 * (cq >> 1) + (cq & 1);
-          *static_cast<DISTCA_LDS elemx4 *>(const_cast<DISTCA_LDS void *>(lds_ptr(wr + ((chunk ^ tile_swz(l32)) << 4)))) =
-              cvt4(oacc[m][db][4 * cq] * inv, oacc[m][db][4 * cq + 1] * inv, oacc[m][db][4 * cq + 2] * inv, oacc[m][db][4 * cq + 3] * inv);
-        }
-      // (LDS operations of one wave complete in order: the reads below see the writes above)
+        for (int db = 0; db < 4; ++db)
 #pragma unroll
-      for (int i = 0; i < kOutStores; ++i) {
-        const int rl = 4 * i + (lane >> 4);
-        const int r = row_wg + (wave * MSUB + m) * 32 + rl;
-        const elemx8 o8 = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(out_w + rl * kRowB + (((lane & 15) ^ tile_swz(rl)) << 4)));
-        if (decltype(all)::value || r < nrows) {
-          const int t = div_group(r);
-          *reinterpret_cast<elemx8 *>(reinterpret_cast<elem_t *>(obytes + (int64_t)t * a.out_tok_bytes) + (kvh * G + (r - t * G)) * kHeadDim + 8 * (lane & 15)) = o8;
+          for (int cq = 2 * h; cq < 2 * h + 2; ++cq) {
+            // d0 = 16 db + 64 h + 8 (cq & 1) + 4 g: chunk 2 db + (cq & 1), half g
+            const int chunk = 2 * db + (cq & 1);
+            *static_cast<DISTCA_LDS elemx4 *>(const_cast<DISTCA_LDS void *>(lds_ptr(out_w + l32 * (kRowB / 2) + ((chunk ^ (l32 & 7)) << 4) + 8 * g))) =
+                cvt4(oacc[m][db][4 * cq] * inv, oacc[m][db][4 * cq + 1] * inv, oacc[m][db][4 * cq + 2] * inv, oacc[m][db][4 * cq + 3] * inv);
+          }
+        // (LDS operations of one wave complete in order: the reads below see the writes above, and the second half's writes come behind them)
+#pragma unroll
+        for (int i = 0; i < kOutStores / 2; ++i) {
+          const int rl = 8 * i + (lane >> 3);
+          const int r = row_wg + (uwave * MSUB + m) * 32 + rl;
+          const elemx8 o8 = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(out_w + rl * (kRowB / 2) + (((lane & 7) ^ (rl & 7)) << 4)));
+          if (decltype(all)::value || r < nrows) {
+            const int t = div_group(r);
+            *reinterpret_cast<elemx8 *>(reinterpret_cast<elem_t *>(obytes + (int64_t)t * a.out_tok_bytes) + (kvh * G + (r - t * G)) * kHeadDim + 64 * h + 8 * (lane & 7)) = o8;
+          }
         }
       }
       if (valid[m] && g == 0) {
