@@ -23,6 +23,7 @@
 #include "attn_bwd.h"
 #include "attn_cfg.h"
 #include "common.h"
+#include "cut_blocks.h"
 
 #include <type_traits>
 
@@ -135,46 +136,40 @@ __device__ __forceinline__ int dkdv_half_key(int wave, int half) { return half ?
 #undef DKDV_SPLIT
 #undef DKDV_NAME
 
-// Adds up the pieces of the key blocks that were cut, in their order: workgroup (cut block, kv head, an eighth of the
-// accumulators: dK or dV, key half, half of d), a lane holding what it held in the kernels above.  Bound by reading the slots
-// (256 KB a piece).
-__global__ __launch_bounds__(kThreads) void ca_bwd_dkdv64_combine_kernel(BwdArgs a) {
-  if ((int)blockIdx.x >= a.cut[0]) return;
-  const int4 e = reinterpret_cast<const int4 *>(a.cut + 4)[blockIdx.x];
-  const int unit = e.x, pieces = e.z, kvh = blockIdx.y, part = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, g = lane >> 5;
-  const f32x4 *first = reinterpret_cast<const f32x4 *>(a.partial + ((int64_t)e.w * a.hkv + kvh) * kDkdvSlotBytes) + part * 8 * kThreads + tid;
-  const int64_t step = a.hkv * (kDkdvSlotBytes / 16);
-  f32x4 o[8] = {};
-  for (int j = 0; j < pieces; ++j) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const f32x4 v = first[j * step + i * kThreads];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[i][r] += v[r];
-    }
-  }
-  const bool is_dv = part >= 4;
-  const int kb = (part >> 1) & 1, db0 = 2 * (part & 1);
-  const int ks = a.grp_off ? a.grp_off[unit] : (a.kv_off ? a.kv_off[unit] : a.cu_k[unit]);
-  const int kmax = a.grp_lmax ? a.grp_lmax[unit] : a.cu_k[unit + 1] - a.cu_k[unit];
-  const int key = e.y * kBN + dkdv_half_key(wave, kb) + l32;
-  if (key >= kmax) return;
-  elem_t *out = is_dv ? a.dv : a.dk;
+// Adds up the pieces of the key blocks that were cut, in their order (cut_blocks.h, once for dK and once for dV: a workgroup has the keys
+// of one half of one wave).  Bound by reading the slots (256 KB a piece).
+__global__ __launch_bounds__(kCutThreads) void ca_bwd_dkdv64_combine_kernel(BwdArgs a) {
+  const int kvh = blockIdx.y, key_wave = (blockIdx.z >> 1) & 3, kb = blockIdx.z & 1, lane = threadIdx.x & 63, db = threadIdx.x >> 6;
   const int64_t kv_stride = (int64_t)a.hkv * kHeadDim;
-  int64_t row = ks + key;
-  if (a.shards.num_shards > 0) {
-    const int sh = find_shard(a.shards.row_start, a.shards.num_shards, ks + key);
-    out += (is_dv ? a.shards.dv_off[sh] : a.shards.dk_off[sh]) / 2;
-    row -= a.shards.row_start[sh];
-  }
-  out += row * kv_stride + kvh * kHeadDim;
-  const float f = is_dv ? 1.f : a.scale;
+  auto gradient = [&](bool is_dv) {
+    add_up_cut_blocks(
+        a.cut,
+        [&](const int4 &e, f32x4 (&o)[4]) {
+          const f32x4 *first = reinterpret_cast<const f32x4 *>(a.partial + ((int64_t)e.w * a.hkv + kvh) * kDkdvSlotBytes);
+          add_pieces(first + ((is_dv ? 32 : 0) + 16 * kb + 4 * db) * kThreads + key_wave * 64 + lane, a.hkv * (kDkdvSlotBytes / 16), kThreads, e.z, o);
+          if (!is_dv) {
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int db = db0 + (i >> 2), cq = i & 3;
-    *reinterpret_cast<elemx4 *>(out + 16 * db + 64 * (cq >> 1) + 8 * (cq & 1) + 4 * g) = cvt4(o[i][0] * f, o[i][1] * f, o[i][2] * f, o[i][3] * f);
-  }
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) o[k][r] *= a.scale;
+          }
+        },
+        [&](const int4 &e, int r) -> elem_t * {
+          const int ks = a.grp_off ? a.grp_off[e.x] : (a.kv_off ? a.kv_off[e.x] : a.cu_k[e.x]);
+          const int kmax = a.grp_lmax ? a.grp_lmax[e.x] : a.cu_k[e.x + 1] - a.cu_k[e.x];
+          const int key = e.y * kBN + dkdv_half_key(key_wave, kb) + r;
+          if (key >= kmax) return nullptr;
+          elem_t *out = is_dv ? a.dv : a.dk;
+          int64_t row = ks + key;
+          if (a.shards.num_shards > 0) {
+            const int sh = find_shard(a.shards.row_start, a.shards.num_shards, ks + key);
+            out += (is_dv ? a.shards.dv_off[sh] : a.shards.dk_off[sh]) / 2;
+            row -= a.shards.row_start[sh];
+          }
+          return out + row * kv_stride + kvh * kHeadDim;
+        });
+  };
+  gradient(blockIdx.z >= kCutParts);
 }
 
 }  // namespace
@@ -196,7 +191,7 @@ int DISTCA_FN(launch_dkdv64)(const BwdArgs &a, int64_t grid, bool few, int64_t m
   if (a.shards.num_shards > 0) launch(few ? ca_bwd_dkdv64_shards_split_kernel : ca_bwd_dkdv64_shards_kernel);
   else if (shared) launch(few ? ca_bwd_dkdv64_shared_split_kernel : ca_bwd_dkdv64_shared_kernel);
   else launch(few ? ca_bwd_dkdv64_split_kernel : ca_bwd_dkdv64_kernel);
-  if (max_cut > 0) hipLaunchKernelGGL(ca_bwd_dkdv64_combine_kernel, dim3((unsigned)max_cut, a.hkv, 8), dim3(kThreads), 0, stream, a);
+  if (max_cut > 0) hipLaunchKernelGGL(ca_bwd_dkdv64_combine_kernel, cut_grid(max_cut, a.hkv, 2 * kCutParts), dim3(kCutThreads), 0, stream, a);
   return DISTCA_OK;
 }
 

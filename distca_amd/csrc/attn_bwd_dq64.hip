@@ -19,6 +19,7 @@
 #include "attn_bwd.h"
 #include "attn_cfg.h"
 #include "common.h"
+#include "cut_blocks.h"
 
 #include <type_traits>
 
@@ -651,39 +652,26 @@ next_block:
   }
 }
 
-// Adds up the pieces of the blocks that were cut, in their order: workgroup (cut block, kv head, quarter of d), a lane holding
-// what it held in the kernel above.
-__global__ __launch_bounds__(kThreads) void ca_bwd_dq64_combine_kernel(BwdArgs a) {
-  if ((int)blockIdx.x >= a.cut[0]) return;
-  const int4 e = reinterpret_cast<const int4 *>(a.cut + 4)[blockIdx.x];
-  const int task = e.x, pieces = e.z, kvh = blockIdx.y, db = blockIdx.z, G = a.group;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, g = lane >> 5;
-  const int q0 = a.cu_q[task], nrows = (a.cu_q[task + 1] - q0) * G;
-  const uint8_t *first = a.partial + ((int64_t)e.w * a.hkv + kvh) * kDqSlotBytes;
-  f32x4 o[2][4] = {};
-  for (int j = 0; j < pieces; ++j) {
-    const f32x4 *op = reinterpret_cast<const f32x4 *>(first + (int64_t)j * a.hkv * kDqSlotBytes) + (wave * 32 + 4 * db) * 64 + lane;
+// Adds up the pieces of the blocks that were cut, in their order (cut_blocks.h).
+__global__ __launch_bounds__(kCutThreads) void ca_bwd_dq64_combine_kernel(BwdArgs a) {
+  const int kvh = blockIdx.y, sub = blockIdx.z, lane = threadIdx.x & 63, db = threadIdx.x >> 6, G = a.group;   // sub: two of a wave, four waves
+  add_up_cut_blocks(
+      a.cut,
+      [&](const int4 &e, f32x4 (&o)[4]) {
+        const f32x4 *first = reinterpret_cast<const f32x4 *>(a.partial + ((int64_t)e.w * a.hkv + kvh) * kDqSlotBytes);
+        add_pieces(first + (16 * sub + 4 * db) * 64 + lane, a.hkv * (kDqSlotBytes / 16), 64, e.z, o);
 #pragma unroll
-    for (int m = 0; m < 2; ++m)
+        for (int k = 0; k < 4; ++k)
 #pragma unroll
-      for (int cq = 0; cq < 4; ++cq) {
-        const f32x4 v = op[(16 * m + cq) * 64];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[m][cq][r] += v[r];
-      }
-  }
-#pragma unroll
-  for (int m = 0; m < 2; ++m) {
-    const int row = e.y * kRowsWg + (wave * 2 + m) * 32 + l32;
-    if (row >= nrows) continue;
-    const int tok = row / G, hg = row - tok * G;
-    elem_t *op = reinterpret_cast<elem_t *>(reinterpret_cast<uint8_t *>(a.dq) + (a.dq_task_off ? a.dq_task_off[task] : (int64_t)q0 * a.dq_tok_bytes) +
-                                            (int64_t)tok * a.dq_tok_bytes) + (kvh * G + hg) * kHeadDim;
-#pragma unroll
-    for (int cq = 0; cq < 4; ++cq)
-      *reinterpret_cast<elemx4 *>(op + 16 * db + 64 * (cq >> 1) + 8 * (cq & 1) + 4 * g) =
-          cvt4(o[m][cq][0] * a.scale, o[m][cq][1] * a.scale, o[m][cq][2] * a.scale, o[m][cq][3] * a.scale);
-  }
+          for (int r = 0; r < 4; ++r) o[k][r] *= a.scale;
+      },
+      [&](const int4 &e, int r) -> elem_t * {
+        const int q0 = a.cu_q[e.x], nrows = (a.cu_q[e.x + 1] - q0) * G, row = e.y * kRowsWg + 32 * sub + r;
+        if (row >= nrows) return nullptr;
+        const int tok = row / G, hg = row - tok * G;
+        return reinterpret_cast<elem_t *>(reinterpret_cast<uint8_t *>(a.dq) + (a.dq_task_off ? a.dq_task_off[e.x] : (int64_t)q0 * a.dq_tok_bytes) +
+                                          (int64_t)tok * a.dq_tok_bytes) + (kvh * G + hg) * kHeadDim;
+      });
 }
 
 }  // namespace
@@ -705,7 +693,7 @@ int DISTCA_FN(launch_dq64)(const BwdArgs &a, int64_t grid, bool few, int64_t max
   if (few) launch(seg ? ca_bwd_dq64_kernel<true, false, true> : ca_bwd_dq64_kernel<false, false, true>);
   else if (a.merge_tiles > 0) launch(seg ? ca_bwd_dq64_kernel<true, true, false> : ca_bwd_dq64_kernel<false, true, false>);
   else launch(seg ? ca_bwd_dq64_kernel<true, false, false> : ca_bwd_dq64_kernel<false, false, false>);
-  if (max_cut > 0) hipLaunchKernelGGL(ca_bwd_dq64_combine_kernel, dim3((unsigned)max_cut, a.hkv, 4), b, 0, stream, a);
+  if (max_cut > 0) hipLaunchKernelGGL(ca_bwd_dq64_combine_kernel, cut_grid(max_cut, a.hkv, kCutParts), dim3(kCutThreads), 0, stream, a);
   return DISTCA_OK;
 }
 

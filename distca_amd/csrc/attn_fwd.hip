@@ -29,6 +29,7 @@
 #include "attn_bwd.h"
 #include "attn_cfg.h"
 #include "common.h"
+#include "cut_blocks.h"
 #include "kv_shards.h"
 
 namespace distca {
@@ -749,48 +750,75 @@ next_block:
   }
 }
 
-// Adds up the pieces of the blocks that were cut: workgroup (cut block, kv head, quarter of d), a lane holding what it held in
-// the kernel above.  Pieces are taken in their order.  Bound by reading the slots (128 KB a piece), which the quarters
-// spread over four times as many compute units; four pieces' loads in flight at a time (17.3 -> 15.5 us for 4096 query rows at 8/2 heads in
-// pieces of 66 tiles over 32768 keys).
-__global__ __launch_bounds__(kFwdWaves * 64) void ca_fwd_combine_kernel(FwdArgs a) {
-  if ((int)blockIdx.x >= a.cut[0]) return;
-  const int4 e = reinterpret_cast<const int4 *>(a.cut + 4)[blockIdx.x];
-  const int task = e.x, pieces = e.z, kvh = blockIdx.y, db = blockIdx.z, G = a.group;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, g = lane >> 5;
-  const int q0 = a.cu_q[task], nrows = (a.cu_q[task + 1] - q0) * G;
-  const int row = e.y * kFwdRows + wave * 32 + l32;
+// Adds up the pieces of the blocks that were cut, in their order (cut_blocks.h; a workgroup has the rows of one wave, a lane what it held
+// in the kernel above).  Bound by reading the slots (128 KB a piece), four pieces' loads in flight at a time.
+__global__ __launch_bounds__(kCutThreads) void ca_fwd_combine_kernel(FwdArgs a) {
+  static_assert(kFwdMsub == 1 && kFwdWaves == kCutParts, "a part is a wave's rows");
+  const int kvh = blockIdx.y, wave = blockIdx.z, lane = threadIdx.x & 63, db = threadIdx.x >> 6, l32 = lane & 31, g = lane >> 5, G = a.group;
   const float c = a.scale * kLog2e;
-  const uint8_t *first = a.partial + ((int64_t)e.w * a.hkv + kvh) * kFwdSlotBytes;
-  const int64_t step = a.hkv * kFwdSlotBytes;
-  auto stat = [&](int j) { return reinterpret_cast<const f32x2 *>(first + j * step + kFwdSlotStats)[wave * 32 + l32]; };
-  float m = -INFINITY;
+  auto token_at = [&](const int4 &e, int r, int &tok, int &head) -> uint8_t * {  // of the output, null if there is no such row
+    const int q0 = a.cu_q[e.x], nrows = (a.cu_q[e.x + 1] - q0) * G, row = e.y * kFwdRows + wave * 32 + r;
+    tok = row / G;
+    head = kvh * G + row - tok * G;
+    uint8_t *at = reinterpret_cast<uint8_t *>(a.out) + (a.out_task_off ? a.out_task_off[e.x] : (int64_t)q0 * a.out_tok_bytes) + (int64_t)tok * a.out_tok_bytes;
+    tok += q0;
+    return row < nrows ? at : nullptr;
+  };
+  add_up_cut_blocks(
+      a.cut,
+      [&](const int4 &e, f32x4 (&o)[4]) {
+        const int pieces = e.z;
+        const uint8_t *first = a.partial + ((int64_t)e.w * a.hkv + kvh) * kFwdSlotBytes;
+        const int64_t step = a.hkv * kFwdSlotBytes;
+        auto stat = [&](int j) { return reinterpret_cast<const f32x2 *>(first + j * step + kFwdSlotStats)[wave * 32 + l32]; };
+        f32x4 v[4][4];
+        f32x2 s[4];
+        auto load = [&](int j) __attribute__((always_inline)) {  // pieces j .. j + 3, as far as there are
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (j + u < pieces) {
+              s[u] = stat(j + u);
+              const f32x4 *op = reinterpret_cast<const f32x4 *>(first + (j + u) * step) + (wave * 16 + 4 * db) * 64 + lane;
+#pragma unroll
+              for (int cq = 0; cq < 4; ++cq) v[u][cq] = op[cq * 64];
+            }
+        };
+        load(0);
+        float m = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (u < pieces) m = __builtin_fmaxf(m, s[u][0]);
 #pragma unroll 4
-  for (int j = 0; j < pieces; ++j) m = __builtin_fmaxf(m, stat(j)[0]);
-  f32x4 o[4] = {};
-  float l = 0.f;
-#pragma unroll 4
-  for (int j = 0; j < pieces; ++j) {
-    const f32x2 s = stat(j);
-    const float w = s[0] == -INFINITY ? 0.f : fast_exp2((s[0] - m) * c);
-    l += w * s[1];
-    const f32x4 *op = reinterpret_cast<const f32x4 *>(first + j * step) + (wave * 16 + 4 * db) * 64 + lane;
+        for (int j = 4; j < pieces; ++j) m = __builtin_fmaxf(m, stat(j)[0]);
+        float l = 0.f;
+        for (int j = 0; j < pieces; j += 4) {
+          if (j > 0) load(j);
 #pragma unroll
-    for (int cq = 0; cq < 4; ++cq) {
-      const f32x4 v = op[cq * 64];
+          for (int u = 0; u < 4; ++u)
+            if (j + u < pieces) {
+              const float w = s[u][0] == -INFINITY ? 0.f : fast_exp2((s[u][0] - m) * c);
+              l += w * s[u][1];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[cq][r] = __builtin_fmaf(w, v[r], o[cq][r]);
-    }
-  }
-  if (row >= nrows) return;
-  const int tok = row / G, hg = row - tok * G;
-  uint8_t *otok = reinterpret_cast<uint8_t *>(a.out) + (a.out_task_off ? a.out_task_off[task] : (int64_t)q0 * a.out_tok_bytes) + (int64_t)tok * a.out_tok_bytes;
-  elem_t *op = reinterpret_cast<elem_t *>(otok) + (kvh * G + hg) * kHeadDim;
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+              for (int cq = 0; cq < 4; ++cq)
 #pragma unroll
-  for (int cq = 0; cq < 4; ++cq)
-    *reinterpret_cast<elemx4 *>(op + 16 * db + 64 * (cq >> 1) + 8 * (cq & 1) + 4 * g) = cvt4(o[cq][0] * inv, o[cq][1] * inv, o[cq][2] * inv, o[cq][3] * inv);
-  if (db == 0 && g == 0) store_lse(a, otok, kvh * G + hg, q0 + tok, l > 0.f ? (m * c + fast_log2(l)) * kLn2 : -INFINITY);
+                for (int r = 0; r < 4; ++r) o[cq][r] = __builtin_fmaf(w, v[u][cq][r], o[cq][r]);
+            }
+        }
+        const float inv = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+        for (int cq = 0; cq < 4; ++cq)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[cq][r] *= inv;
+        if (db == 0 && g == 0) {
+          int tok, head;
+          if (uint8_t *otok = token_at(e, l32, tok, head)) store_lse(a, otok, head, tok, l > 0.f ? (m * c + fast_log2(l)) * kLn2 : -INFINITY);
+        }
+      },
+      [&](const int4 &e, int r) -> elem_t * {
+        int tok, head;
+        uint8_t *otok = token_at(e, r, tok, head);
+        return otok ? reinterpret_cast<elem_t *>(otok) + head * kHeadDim : nullptr;
+      });
 }
 
 // How a forward is laid out in its workspace: the list, and, when blocks are cut, the tables and slots of the pieces.
@@ -1000,7 +1028,7 @@ int DISTCA_FN(run_fwd_tokens)(const void *q_base, const int64_t *q_task_off, int
     if (few) launch(kv_shards ? ca_fwd_kernel<kFwdMsub, true, false, true> : ca_fwd_kernel<kFwdMsub, false, false, true>);
     else if (geom.merge_tiles > 0) launch(kv_shards ? ca_fwd_kernel<kFwdMsub, true, true, false> : ca_fwd_kernel<kFwdMsub, false, true, false>);
     else launch(kv_shards ? ca_fwd_kernel<kFwdMsub, true, false, false> : ca_fwd_kernel<kFwdMsub, false, false, false>);
-    if (split) hipLaunchKernelGGL(ca_fwd_combine_kernel, dim3((unsigned)split_max_cut(lay.max_blocks, lay.target), p->num_heads_kv, 4), b, 0, s, a);
+    if (split) hipLaunchKernelGGL(ca_fwd_combine_kernel, cut_grid(split_max_cut(lay.max_blocks, lay.target), p->num_heads_kv, kCutParts), dim3(kCutThreads), 0, s, a);
   }
   return check_launch("ca_fwd");
 }
