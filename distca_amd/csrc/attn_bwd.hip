@@ -46,7 +46,7 @@ BwdLayout bwd_layout(const distca_ca_params *p, bool shared, bool preferred) {
   w.blocks_kv = shared || preferred ? bwd_key_blocks_own_rows(p) : bwd_max_items(p) - bwd_split_target(p);
   w.blocks_q = dq_max_items(p);
   w.target_kv = preferred ? preferred_key_pieces(p) : bwd_split_target(p);
-  w.target_q = preferred ? row_split_target(p, w.blocks_q) : 0;
+  w.target_q = preferred ? row_split_target(p, w.blocks_q, kCutFromTilesDq) : 0;
   w.items_kv = w.blocks_kv + w.target_kv;
   w.items_q = w.blocks_q + w.target_q;
   int64_t o = 0;

@@ -148,20 +148,28 @@ inline int32_t bwd_split_target(const distca_ca_params *p) {
 }
 // Blocks of query rows are cut into pieces of consecutive KV tiles when the batch has so few of them that the longest one
 // could bound the launch: fewer than kSplitMaxBlocksPerCU blocks per compute unit (above that longest-first dispatch evens
-// them out), and a prefix of more than kCutFromTiles KV tiles (the second launch takes 4.5 us though nothing be cut: 1000 tokens at
-// 32/8 heads, forward, 32.0 / 36.4 us; just above the line it is dQ that gains, 1024 tokens at 8/2 heads, whole / cut: forward 29 / 34, dQ 41 / 34).  Returns the number of pieces to aim for per kv head, 0 = no cutting.
+// them out), and more than kCutFromTiles* KV tiles that cutting could take off the longest block.  That is all of its tiles but the unit's
+// share of the longest task's, half of them for every block of the task per unit; from two blocks per unit on longest-first evens out a task by
+// itself.  Below the line the second launch, which takes 4.5 us though nothing be cut, and the pieces' own time cost more than they give: us
+// forward, cut / whole: 1100 tokens at 4/1 heads (17 tiles to gain) 29.2 / 24.5, 4 x 1024 at 8/2 (15) 33.7 / 24.8, 1500 at 32/8 (15) 40.9 / 32.5,
+// 2048 at 32/8 (16) 55 / 52, 2560 + 1024 + 512 at 32/8 (15) 75.5 / 71.2, 4096 at 32/8 (0) 129 / 125, 12000 at 32/8 (0) 934 / 926; above it: 2048 at 8/2 (29)
+// 38.1 / 39.5, 2048 at 4/1 (31) 34.2 / 39.0, 3000 at 4/1 (42) 41.5 / 54.2, 8192 at 8/2 (64) 145 / 159.
+// dQ's tiles are longer, its line lower: us backward, cut / whole: 1100 at 32/8 (13) 101.5 / 99, 2560 + 1024 + 512 at 32/8 (15) 248 / 245, 8192 at 32/8 (0) 1566 /
+// 1559; just above it, dQ of 1024 tokens at 8/2 (16) 34 / 41.
+// Returns the number of pieces to aim for per kv head, 0 = no cutting.
 // It depends only on sizes that do not change with how K/V are stored, so that a tick gives the same bits in every form.
 constexpr int kSplitRowPiecesPerCU = 2;
 constexpr int kSplitMaxBlocksPerCU = 8;
-constexpr int kCutFromTiles = 16;
+constexpr int kCutFromTilesFwd = 24, kCutFromTilesDq = 16;
 inline bool few_row_blocks(const distca_ca_params *p) {
   return (int64_t)p->total_q * p->num_heads_q < (int64_t)kSplitMaxBlocksPerCU * kFwdRows * num_compute_units();
 }
-inline int32_t row_split_target(const distca_ca_params *p, int64_t max_blocks) {
+inline int32_t row_split_target(const distca_ca_params *p, int64_t max_blocks, int from_tiles) {
   const int64_t cus = num_compute_units();
   if (!few_row_blocks(p)) return 0;
   const int64_t tiles = (int64_t)p->max_seqlen_k / kFwdKV + 1;
-  if (tiles <= kCutFromTiles) return 0;
+  const int64_t two_each = 2 * (int64_t)kFwdRows * cus, rows = (int64_t)p->max_seqlen_q * p->num_heads_q;   // rows x heads, of two blocks per unit; of the longest task
+  if (rows >= two_each || tiles * (two_each - rows) <= from_tiles * two_each) return 0;
   const int64_t most = (tiles + kMinPieceWorth - 1) / kMinPieceWorth;   // pieces of the longest block
   const int64_t t = kSplitRowPiecesPerCU * cus / p->num_heads_kv, all = max_blocks * most;
   return (int32_t)(t < 1 ? 1 : (t < all ? t : all));

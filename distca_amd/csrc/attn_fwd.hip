@@ -829,7 +829,7 @@ struct FwdLayout {
 FwdLayout fwd_layout(const distca_ca_params *p, bool split) {
   FwdLayout w;
   w.max_blocks = fwd_max_items(p);
-  w.target = split ? row_split_target(p, w.max_blocks) : 0;
+  w.target = split ? row_split_target(p, w.max_blocks, kCutFromTilesFwd) : 0;
   w.max_items = w.max_blocks + w.target;
   w.tables = align_up(sched_region_bytes(p->num_tasks, w.max_items), 256);
   w.slots = w.tables + split_tables_bytes(w.max_blocks, w.target, w.max_items);

@@ -539,7 +539,7 @@ struct LaunchedList {
 LaunchedList launched_list(int kind, const distca_ca_params *p) {
   if (kind == 1) return {launched_dkdv_geom(p, preferred_key_pieces(p), true, false), bwd_key_blocks_own_rows(p)};
   const int64_t blocks = kind == 0 ? fwd_max_items(p) : dq_max_items(p);
-  const int32_t target = row_split_target(p, blocks);
+  const int32_t target = row_split_target(p, blocks, kind == 0 ? kCutFromTilesFwd : kCutFromTilesDq);
   return {kind == 0 ? launched_fwd_geom(p, target) : launched_dq_geom(p, target), blocks};
 }
 }  // namespace

@@ -102,6 +102,13 @@ def test_runs_of_whole_tiles_and_blocks(cuda, hq, hkv):
     _run(lens, lens, hq, hkv, 23, cuda)
 
 
+@pytest.mark.parametrize("hq,hkv,lens", [(4, 1, [1020]), (4, 1, [1030]), (4, 1, [1540]), (4, 1, [1600]), (32, 8, [2048]), (64, 16, [2050]), (16, 4, [1800, 250])])
+def test_either_side_of_the_lines_from_which_blocks_are_cut(cuda, hq, hkv, lens):
+    """Tiles that cutting could take off the longest block, where dQ's line is 16 and the forward's 24: 15.5, 16.5, 23.8, 24.7, 16.5 (half of a longer
+    block's), none (two blocks of the task a unit), 22.6 (with a short task beside)."""
+    _run(lens, lens, hq, hkv, 29, cuda, deterministic=True)
+
+
 def test_shared_kv_prefix(cuda):
     """Three shards of one 600-token document reading one stored KV copy."""
     _run([200, 150, 250], [200, 350, 600], 8, 2, 5, cuda, kv_offsets=[0, 0, 0], total_k=600)
