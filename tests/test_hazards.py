@@ -70,7 +70,7 @@ def violations(lines):
     return out
 
 
-def test_checker_sees_what_it_looks_for():
+def test_hazards_planted_in_a_listing_are_found():
     load = "global_load_lds_dwordx4 v1, s[0:1] offset:2048"
     assert violations(["v_readlane_b32 s1, v252, 18", load])
     assert violations(["v_readfirstlane_b32 s0, v2", "s_nop 1", "s_mov_b32 m0, s3", "s_nop 0", load])
