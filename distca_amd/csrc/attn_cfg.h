@@ -148,9 +148,8 @@ inline int32_t bwd_split_target(const distca_ca_params *p) {
 }
 // Blocks of query rows are cut into pieces of consecutive KV tiles when the batch has so few of them that the longest one
 // could bound the launch: fewer than kSplitMaxBlocksPerCU blocks per compute unit (above that longest-first dispatch evens
-// them out), and more than kCutFromTiles* KV tiles that cutting could take off the longest block.  That is all of its tiles but the unit's
-// share of the longest task's, half of them for every block of the task per unit; from two blocks per unit on longest-first evens out a task by
-// itself.  Below the line the second launch, which takes 4.5 us though nothing be cut, and the pieces' own time cost more than they give: us
+// them out), and more than kCutFromTiles* KV tiles that cutting could take off the longest block (row_tiles_to_gain).
+// Below the line the second launch, which takes 4.5 us though nothing be cut, and the pieces' own time cost more than they give: us
 // forward, cut / whole: 1100 tokens at 4/1 heads (17 tiles to gain) 29.2 / 24.5, 4 x 1024 at 8/2 (15) 33.7 / 24.8, 1500 at 32/8 (15) 40.9 / 32.5,
 // 2048 at 32/8 (16) 55 / 52, 2560 + 1024 + 512 at 32/8 (15) 75.5 / 71.2, 4096 at 32/8 (0) 129 / 125, 12000 at 32/8 (0) 934 / 926; above it: 2048 at 8/2 (29)
 // 38.1 / 39.5, 2048 at 4/1 (31) 34.2 / 39.0, 3000 at 4/1 (42) 41.5 / 54.2, 8192 at 8/2 (64) 145 / 159.
@@ -164,14 +163,35 @@ constexpr int kCutFromTilesFwd = 24, kCutFromTilesDq = 16;
 inline bool few_row_blocks(const distca_ca_params *p) {
   return (int64_t)p->total_q * p->num_heads_q < (int64_t)kSplitMaxBlocksPerCU * kFwdRows * num_compute_units();
 }
+// An upper bound, times *scale, of the KV tiles that cutting could take off the longest block of query rows: all of its tiles but the load of a
+// unit, of which only the part counts that the task of the longest prefix brings along, half of its tiles for every block of that task per unit
+// (from two blocks per unit on longest-first evens a task out by itself).  How many rows that task has is known where it is the only one, and
+// where the tasks are whole documents, which equal bounds within the batch's tokens are taken for: of all lengths up to the bound, which need
+// not be reached, a document of one block per unit has the most to gain.  Otherwise the most rows may be one task's and the longest
+// prefix another's, a new document's and a short shard's at the end of a long one; then all tiles count, and the list builder, which sees
+// the tasks, decides.  us at 32/8 heads with the one task's rows set against the other's prefix / left to the builder, forward, backward:
+// 4096 + 256 rows over 4096 + 131072 keys 2175 / 646, 4915 / 2235; 5000 + 300 + 2000 over 5000 + 60000 + 8000 1104 / 653, 2998 / 2183.
+// And at 8/2 heads, the bound taken for a length / for a bound: 8192 + 16 x 512 tokens, bounds of 16384, 173 / 169, 570 / 534.  What the second launch
+// costs where the bound is reached and longest-first would have done: 16384 + 2000 tokens 481 / 484, 1672 / 1675.
+inline int64_t row_tiles_to_gain(const distca_ca_params *p, int64_t *scale) {
+  const int64_t heads = p->num_heads_q, two_each = 2 * (int64_t)kFwdRows * num_compute_units();   // rows x heads of two blocks per unit
+  const bool alone = p->num_tasks == 1, documents = p->max_seqlen_q == p->max_seqlen_k && p->max_seqlen_k <= p->total_q;
+  int64_t tiles = (int64_t)p->max_seqlen_k / kFwdKV + 1, tokens = 0;
+  if (alone || documents) {
+    tokens = p->max_seqlen_q < p->max_seqlen_k ? p->max_seqlen_q : p->max_seqlen_k;   // (queries beyond the keys see nothing)
+    if (tokens > p->total_q) tokens = p->total_q;
+    if (!alone && 2 * tokens * heads > two_each) tokens = two_each / 2 / heads, tiles = tokens / kFwdKV;
+  }
+  *scale = two_each;
+  return tokens * heads < two_each ? tiles * (two_each - tokens * heads) : 0;
+}
 inline int32_t row_split_target(const distca_ca_params *p, int64_t max_blocks, int from_tiles) {
-  const int64_t cus = num_compute_units();
   if (!few_row_blocks(p)) return 0;
+  int64_t scale;
+  if (row_tiles_to_gain(p, &scale) <= from_tiles * scale) return 0;
   const int64_t tiles = (int64_t)p->max_seqlen_k / kFwdKV + 1;
-  const int64_t two_each = 2 * (int64_t)kFwdRows * cus, rows = (int64_t)p->max_seqlen_q * p->num_heads_q;   // rows x heads, of two blocks per unit; of the longest task
-  if (rows >= two_each || tiles * (two_each - rows) <= from_tiles * two_each) return 0;
   const int64_t most = (tiles + kMinPieceWorth - 1) / kMinPieceWorth;   // pieces of the longest block
-  const int64_t t = kSplitRowPiecesPerCU * cus / p->num_heads_kv, all = max_blocks * most;
+  const int64_t t = kSplitRowPiecesPerCU * num_compute_units() / p->num_heads_kv, all = max_blocks * most;
   return (int32_t)(t < 1 ? 1 : (t < all ? t : all));
 }
 // Workgroups for a list: 5/4 of its places, drawing tickets (sched.h, take_item), or, where the items are few, one each.

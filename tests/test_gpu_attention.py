@@ -109,6 +109,12 @@ def test_either_side_of_the_lines_from_which_blocks_are_cut(cuda, hq, hkv, lens)
     _run(lens, lens, hq, hkv, 29, cuda, deterministic=True)
 
 
+@pytest.mark.parametrize("q_lens,k_lens", [([2048, 40], [2048, 6000]), ([100, 2050], [5003, 2050])])
+def test_new_document_beside_a_short_shard_of_a_long_one(cuda, q_lens, k_lens):
+    """Two blocks of query rows a unit of one task, whose blocks stay whole, beside a block of another over a long prefix, which is cut."""
+    _run(q_lens, k_lens, 64, 16, 37, cuda, deterministic=True)
+
+
 def test_shared_kv_prefix(cuda):
     """Three shards of one 600-token document reading one stored KV copy."""
     _run([200, 150, 250], [200, 350, 600], 8, 2, 5, cuda, kv_offsets=[0, 0, 0], total_k=600)

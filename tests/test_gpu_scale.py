@@ -590,7 +590,8 @@ def test_mfma_rate_probe(cuda):
 
 
 @pytest.mark.parametrize("lens,extra,hq,hkv", [([8192], 0, 32, 8), ([389, 64, 0, 1200], 0, 4, 1), ([300, 40, 700], 9000, 8, 2), ([4096], 0, 8, 2),
-                                               ([5000, 2000, 128, 1064], 0, 32, 8), ([1000, 300, 17, 600] * 12, 0, 64, 8), ([3000, 2100] * 7, 500, 6, 2)])
+                                               ([5000, 2000, 128, 1064], 0, 32, 8), ([1000, 300, 17, 600] * 12, 0, 64, 8), ([3000, 2100] * 7, 500, 6, 2),
+                                               ([256, 4096], 30000, 32, 8)])
 @pytest.mark.parametrize("causal", [True, False])
 def test_device_lists_equal_the_mirror_of_launched_lists(cuda, lens, extra, hq, hkv, causal):
     """With the preferred workspace: the forward's, the dK/dV and the dQ list the builder left, pieces, merged items, walk marks and

@@ -303,3 +303,53 @@ def test_cutting_follows_what_bounds_the_launch(kind):
     assert pieces([16384] * 4, 32, 8) == 1
     assert pieces([8192], 32, 8) == 1 if kind != scheduler.BWD else pieces([8192], 32, 8) > 1
     assert pieces([64] * 8, 8, 2) == 1
+
+
+def _launched_costs(kind, lq, lk, hq, hkv, bounds=None):
+    """(costs of the launched list's items, blocks that are cut); bounds: max_seqlen_q and max_seqlen_k as a caller gives them, not the true ones."""
+    from distca_amd import _lib
+    import ctypes
+    cu_q, cu_k = _cu(lq), _cu(lk)
+    p = scheduler._params(cu_q, cu_k, hq, hkv, 128, True)
+    if bounds:
+        p.max_seqlen_q, p.max_seqlen_k = bounds
+    items = np.zeros((scheduler.schedule_capacity(kind | scheduler.LAUNCHED, cu_q, cu_k, hq, hkv) + 1000, 4), dtype=np.int32)
+    n = _lib.load().distca_ca_schedule_host(kind | scheduler.LAUNCHED, cu_q.ctypes.data, cu_k.ctypes.data, ctypes.byref(p), items.ctypes.data, len(items))
+    assert 0 <= n <= len(items)
+    pieces = scheduler.item_pieces(items[:n, 3])
+    return items[:n, 2], len({(t, b) for (t, b, _, _), k in zip(items[:n].tolist(), pieces.tolist()) if k > 1})
+
+
+def _longest_unit(costs, hkv, item_cost=6):
+    heap = [0] * (256 // hkv)
+    for c in costs.tolist():
+        heapq.heappush(heap, heapq.heappop(heap) + c + item_cost)
+    return max(heap)
+
+
+@pytest.mark.parametrize("kind", [scheduler.FWD, scheduler.DQ], ids=["forward", "dQ"])
+@pytest.mark.parametrize("lq,lk,hq,hkv", [
+    ([4096, 256], [4096, 131072], 32, 8), ([256, 4096], [65536, 4096], 32, 8), ([4096, 1024], [4096, 32768], 32, 8),
+    ([5000, 300, 2000], [5000, 60000, 8000], 32, 8), ([8192, 512, 512], [8192, 32768, 65536], 32, 8), ([16384, 256], [16384, 65536], 8, 2),
+    ([4096, 64, 64], [300, 16384, 90], 32, 8)])
+def test_rows_of_one_task_say_nothing_of_the_prefix_of_another(kind, lq, lk, hq, hkv):
+    """A task of many query rows beside a few rows at the end of a long prefix: the latter's blocks outlast everything else and are cut,
+    so that no unit works much longer than the average one (whole, the longest block alone is the larger part of the launch)."""
+    costs, cut = _launched_costs(kind, lq, lk, hq, hkv)
+    average = (costs.sum() + 6 * len(costs)) / (256 // hkv)
+    assert cut > 0 and _longest_unit(costs, hkv) < 1.25 * average
+
+
+@pytest.mark.parametrize("kind", [scheduler.FWD, scheduler.DQ], ids=["forward", "dQ"])
+def test_cutting_takes_the_bounds_of_lengths_as_bounds(kind):
+    """Whole documents of two blocks per unit stay whole, documents too short to gain by cutting do too, whether the caller gives their longest
+    length or a larger one within the batch's tokens; a document that is worth cutting is cut under either, and so is a short
+    shard's long prefix under a bound common to queries and keys that no document of the batch could have."""
+    for lens in ([4096, 4096], [2560, 1024, 512], [3000, 500, 596], [8192]):
+        assert _launched_costs(kind, lens, lens, 32, 8)[1] == 0
+        assert _launched_costs(kind, lens, lens, 32, 8, (sum(lens),) * 2)[1] == 0
+    for lens in ([4096, 300], [8192] + [512] * 16):
+        assert _launched_costs(kind, lens, lens, 8, 2)[1] > 0
+        assert _launched_costs(kind, lens, lens, 8, 2, (sum(lens),) * 2)[1] > 0
+    assert _launched_costs(kind, [2000], [2000], 8, 2, (32768, 32768))[1] > 0
+    assert _launched_costs(kind, [4096, 256], [4096, 131072], 32, 8, (131072, 131072))[1] > 0
