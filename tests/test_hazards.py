@@ -38,34 +38,59 @@ def scalars(operand):
     return {int(m[1])} if m else ({"m0"} if operand == "m0" else set())
 
 
+def registers(operand):
+    """v0 .. and a0 .. of an operand, s0 .. and vcc as numbers (vcc: 106 and 107)."""
+    operand = operand.strip("-|")
+    m = re.fullmatch(r"([va])\[(\d+):(\d+)\]", operand)
+    if m:
+        return {m[1] + str(i) for i in range(int(m[2]), int(m[3]) + 1)}
+    return {operand} if re.fullmatch(r"[va]\d+", operand) else {106, 107} if operand == "vcc" else scalars(operand)
+
+
+def results(op, ops):
+    """The operands that a vector instruction writes: the first, and of those with a carry or flag the second."""
+    return ops[:2] if re.search(r"_co_|div_scale|mad_[ui]64", op) else ops[:1]
+
+
+def union(operands):
+    return set().union(*map(registers, operands))
+
+
 def operands(line):
     rest = line.split(None, 1)
     return [o.strip().split()[0] for o in rest[1].split(",")] if len(rest) > 1 else []
 
 
 def violations(lines):
-    """(what, wait states between, instruction before, instruction) of straight-line code.  A vector instruction's write of a scalar register
-    and a vector memory instruction that reads it: 5, unless a scalar instruction that uses the register, and waits for it, stands between;
-    a write of M0 and a load to LDS: 1."""
+    """(what, wait states between, instruction before, instruction) of straight-line code.  A vector instruction's write of a scalar register and a
+    vector memory instruction that reads it: 5, a vector instruction that reads it: 2, unless a scalar instruction that uses the register, and waits
+    for it, stands between; of a vector or accumulation register and a matrix instruction that reads it: 2; a write of M0 and a load to LDS: 1."""
     out = []
     for i, line in enumerate(lines):
-        if not re.match(r"(global|buffer|flat|scratch)_(load|store|atomic)", line):
+        op, ops = line.split()[0], operands(line)
+        memory, vector = re.match(r"(global|buffer|flat|scratch)_(load|store|atomic)", line), op.startswith("v_")
+        if not memory and not vector:
             continue
-        reads = set().union(*map(scalars, operands(line)))
-        to_lds = "_lds_" in line or line.endswith(" lds")
+        read = union(ops) if memory else union(ops[len(results(op, ops)):])
+        reads, operand_reads = {r for r in read if isinstance(r, int)}, {r for r in read if op.startswith("v_mfma") and isinstance(r, str)}
+        needed = 5 if memory else 2
+        to_lds = memory and ("_lds_" in line or line.endswith(" lds"))
         waits = 0
-        for before in reversed(lines[max(i - 5, 0):i]):
-            op, ops = before.split()[0], operands(before)
-            if op.startswith("v_") and ops and scalars(ops[0]) & reads:
+        for before in reversed(lines[max(i - needed, 0):i]):
+            bop, bops = before.split()[0], operands(before)
+            written = union(results(bop, bops)) if bop.startswith("v_") else set()
+            if written & reads:
                 out.append(("scalar register", waits, before, line))
-            if to_lds and waits < 1 and ops[:1] == ["m0"]:
+            if written & operand_reads and not bop.startswith("v_mfma"):
+                out.append(("operand of a matrix instruction", waits, before, line))
+            if to_lds and waits < 1 and bops[:1] == ["m0"]:
                 out.append(("M0", waits, before, line))
-            if op in ("s_branch", "s_endpgm", "s_setpc_b64"):   # nothing falls through
+            if bop in ("s_branch", "s_endpgm", "s_setpc_b64"):   # nothing falls through
                 break
-            if op.startswith("s_"):
-                reads -= set().union(*map(scalars, ops)) if ops else set()
-            waits += int(ops[0], 0) + 1 if op == "s_nop" else 1
-            if waits >= 5:
+            if bop.startswith("s_"):
+                reads -= union(bops)
+            waits += int(bops[0], 0) + 1 if bop == "s_nop" else 1
+            if waits >= needed:
                 break
     return out
 
@@ -79,10 +104,26 @@ def test_hazards_planted_in_a_listing_are_found():
     assert not violations(["v_readfirstlane_b32 s0, v2", "s_mov_b64 s[0:1], s[0:1]", load])
     assert not violations(["v_readfirstlane_b32 s2, v2", "s_mov_b32 m0, s3", "s_nop 0", load])
 
+    select = "v_cndmask_b32_e64 v3, 0, -1, s[4:5]"
+    assert violations(["v_readlane_b32 s5, v252, 18", select])
+    assert violations(["v_cmp_gt_i32_e32 vcc, v1, v2", "v_mov_b32_e32 v9, v8", "v_cndmask_b32_e32 v3, 0, v4, vcc"])
+    assert violations(["v_add_co_u32_e64 v1, s[4:5], v2, v3", "s_nop 0", select])
+    assert violations(["v_readfirstlane_b32 s7, v2", "v_add_u32_e32 v3, s7, v4"])
+    assert not violations(["v_readlane_b32 s5, v252, 18", "s_nop 1", select])
+    assert not violations(["v_readlane_b32 s5, v252, 18", "s_mov_b64 s[4:5], s[4:5]", select])
+    assert not violations(["s_mov_b32 s5, 0xff00ff00", select]) and not violations([select, "v_readlane_b32 s5, v252, 18"])
 
-@pytest.mark.skipif(not os.path.exists(LIB_PATH) or not os.path.exists(OBJDUMP), reason="needs the built library and llvm-objdump")
+    product = "v_mfma_f32_32x32x16_bf16 v[0:15], v[16:19], a[20:23], v[0:15]"
+    assert violations(["v_cvt_pk_bf16_f32 v19, v40, v41", "v_mov_b32_e32 v50, v51", product])
+    assert violations(["v_accvgpr_write_b32 a20, v3", product]) and violations(["v_accvgpr_read_b32 v15, a3", "s_nop 0", product])
+    assert not violations(["v_cvt_pk_bf16_f32 v19, v40, v41", "s_nop 1", product])
+    assert not violations(["v_mov_b32_e32 v24, v40", product]) and not violations(["ds_read_b128 v[16:19], v60", product])
+
+
+@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="needs llvm-objdump")
 def test_wait_states_of_the_built_kernels(tmp_path):
-    found, loads = [], 0
+    assert os.path.exists(LIB_PATH), "the library is not built"
+    found, loads, products = [], 0, 0
     for k, obj in enumerate(code_objects(LIB_PATH)):
         f = tmp_path / f"{k}.co"
         f.write_bytes(obj)
@@ -93,11 +134,12 @@ def test_wait_states_of_the_built_kernels(tmp_path):
             if m:
                 found += [(kernel,) + v for v in violations(lines)]
                 loads += sum("global_load_lds" in l for l in lines)
+                products += sum(l.startswith("v_mfma") for l in lines)
                 kernel, lines = m[1], []
                 continue
             t = raw.split("//")[0].strip()
             if t and not t.endswith(":"):
                 lines.append(t)
-    assert loads > 1000, "no loads to LDS found: the disassembly is not what this test reads"
+    assert loads > 1000 and products > 1000, "no loads to LDS, no matrix instructions: the disassembly is not what this test reads"
     assert not found, f"{len(found)} places, among them {found[:3]}"
 
