@@ -354,7 +354,7 @@ __global__ __launch_bounds__(kPackThreads, SUMS ? 4 : 8) void exchange_kernel(Jo
   }
 }
 
-// ---- Up to some 100 MB: a vector a thread ----
+// ---- Up to some 30 to 130 MB: a vector a thread ----
 //
 // A launch of a few MB is a chain of trips to memory, not a matter of bandwidth: a plain copy of 3 MB takes 2.4 us, and the same by
 // exchange_kernel took 6 to 8, because a slice's runs go one after the other (a trip there and a trip back for each shard and replica it
@@ -362,11 +362,8 @@ __global__ __launch_bounds__(kPackThreads, SUMS ? 4 : 8) void exchange_kernel(Jo
 // whatever shard it lies in: a wave reads the lengths, places and masks of 64 shards at once, a lane a shard, finds by lane moves where its
 // vectors go, and all of them travel together; what is packed is requested before the list is read.
 // us by slices / by vectors, pack, reply, request and gradients of the linear side: 1024 tokens at 8/2 heads (3 / 2 / 7 / 3 MB)
-// 7.7 7.1 11.5 9.0 / 4.3 3.9 6.0 5.0; 2048 at 32/8 (25 / 17 / 59 / 25 MB) 15.2 12.7 27.3 17.5 / 12.7 8.7 23.2 12.6; 4096 (50 / 34 / 117 / 50)
-// 23.0 17.7 48.4 24.8 / 21.6 18.9 43.9 26.9; 8192 (101 / 67 / 235 / 101) 39.8 34.3 88.2 42.9 / 41.2 33.1 90.7 48.6.  The lines below lie
-// where slices, which load ten vectors a thread before they store, begin to gain; adding rows up, a vector has a load in flight at a time, and loses earlier.
+// 7.7 7.1 11.5 9.0 / 4.3 3.9 6.0 5.0.  Which of the two a launch takes: launch_by_vectors.
 constexpr int kVectorThreads = 256;
-constexpr int64_t kVectorBytes = 128ll << 20, kVectorSumBytes = 32ll << 20;   // of a launch; of one that adds rows up
 constexpr int kVectorSeqs = 256;             // shards of a job: four reads of 64
 
 // 64 shards from c0 on, one a lane.  end: position behind the shard's last token (sums saturate; tensors have fewer than 2^31 tokens).
@@ -642,9 +639,48 @@ int add_job(Jobs *jobs, const distca_exchange_job &in, int64_t token_bytes, int 
   return 0;
 }
 
+// Whether a launch of `total` bytes goes by vectors.  Slices have many vectors of a thread in flight and gain on bandwidth, the sooner the less there is to
+// be found out on the way: an unpack by vectors cannot ask for anything before the list is read, while a pack has its rows by then; adding rows up, a
+// vector has a load in flight at a time.  What slices lose is a trip there and back for each run they walk, so that every line lies further up
+// the more shards there are to the slice of a job; rows of several replicas and parts of a few bytes a token (lse of 8 heads) cost slices more than the
+// bandwidth gives up to 128 MB.  Of 1134 launches of 16 to 127 MB (4 to 64 heads, 3 to 250 documents) the one chosen is at most 9 % slower than the
+// other, 19 times more than 5 %, where one line of 128 MB, 32 MB with sums, took up to 94 % longer.  us by slices / by vectors around the lines (12 documents at 32/8 heads, every replica's mask set once in four, where nothing else is said):
+//   one tensor unpacked          24 MB 14.1 / 13.6   32 MB 16.1 / 16.6   48 MB 20.6 / 22.7   64 MB 25.0 / 28.9
+//   q, k, v unpacked             32 MB 17.4 / 16.7   48 MB 21.9 / 23.0   120 documents, 40 MB 26.2 / 24.5, 72 MB 35.6 / 39.3
+//   one tensor packed            32 MB 16.1 / 15.4   48 MB 20.7 / 20.7   64 MB 25.2 / 26.1
+//   [out | lse] unpacked         64 MB 30.3 / 29.3   96 MB 39.6 / 42.2   3 documents, 40 MB 18.7 / 19.5   8/2 heads, 100 documents, 128 MB 69.9 / 59.4
+//   gradients, replicas added    48 MB 31.5 / 27.7   64 MB 37.2 / 35.6   72 MB 36.9 / 36.9   96 MB 48.7 / 50.6
+//   gradients, copies added      48 MB 26.2 / 24.7   64 MB 30.0 / 31.5   96 MB 39.8 / 43.5
+//   q, k, v packed to replicas   64 MB 34.6 / 32.6  128 MB 64.7 / 60.0; the request 64 MB 38.0 / 29.9, 128 MB 61.5 / 54.5
+// (One tensor packed, 88 to 127 MB: slices begin a second round of workgroups at 84 MB, and until they fill it vectors gain again, 36.0 / 34.1, 48.6 / 47.1, but
+// not where a wave looks through several reads of shards, 250 of them 38.9 / 44.6.)
+constexpr int64_t kVectorUnpackBytes = 30 * 1000 * 1000, kVectorPackBytes = 40 * 1000 * 1000, kVectorSumBytes = 50 * 1000 * 1000, kVectorMostBytes = 128ll << 20;
+constexpr int64_t kNarrowPartBytes = 128;
+bool launch_by_vectors(const Jobs &jobs, int64_t total, int to_buffer) {
+  if (total > kVectorMostBytes) return false;
+  bool sums = false, replicas = false, parts = false, narrow = false, one_read = true;
+  double walked = 0;   // shards, and their replicas, that a slice walks
+  for (int i = 0; i < jobs.n; ++i) {
+    const Job &o = jobs.job[i];
+    // (a vector's number times the vectors of a part stays below 2^32: Job::magic)
+    if (o.num_seq > kVectorSeqs || o.num_tokens * o.part_vecs * o.part_vecs >= (1ll << 32)) return false;
+    const bool adds_replicas = o.kind == DISTCA_JOB_REPLICA_SUM;
+    sums |= adds_replicas || o.kind == DISTCA_JOB_COPY_SUM;
+    replicas |= o.kind == DISTCA_JOB_REPLICAS;
+    parts |= !o.whole();
+    narrow |= !o.whole() && o.part_vecs * 16 < kNarrowPartBytes;
+    one_read &= o.num_seq <= 64;
+    const double w = (double)o.tokens_per_wg * o.num_seq * (adds_replicas ? o.max_cp : 1) / (double)o.num_tokens;
+    walked = w > walked ? w : walked;
+  }
+  if (!sums && (replicas || narrow || (to_buffer && one_read && total > 2 * num_compute_units() * kRoundBytes))) return true;
+  const int64_t line = sums ? kVectorSumBytes : to_buffer ? kVectorPackBytes : kVectorUnpackBytes;
+  return total <= line * (1 + (parts && !sums ? 1.25 : 0.5) * walked);
+}
+
 int launch_exchange(Jobs &jobs, void *buffer, int to_buffer, void *stream, int timer_id, const char *what) {
   if (jobs.n == 0) return DISTCA_OK;
-  int64_t total = 0, wg = 0;
+  int64_t total = 0;
   bool sums = false, parts = false;
   for (int i = 0; i < jobs.n; ++i) {
     const Job &o = jobs.job[i];
@@ -652,44 +688,35 @@ int launch_exchange(Jobs &jobs, void *buffer, int to_buffer, void *stream, int t
     sums |= o.kind == DISTCA_JOB_REPLICA_SUM || o.kind == DISTCA_JOB_COPY_SUM;
     parts |= !o.whole();
   }
-  hipStream_t s = (hipStream_t)stream;
-  uint8_t *buf = (uint8_t *)buffer;
-  bool by_vectors = total <= (sums ? kVectorSumBytes : kVectorBytes);
-  for (int i = 0; i < jobs.n && by_vectors; ++i) {   // (a vector's number times the vectors of a part stays below 2^32: Job::magic)
-    const Job &o = jobs.job[i];
-    by_vectors = o.num_seq <= kVectorSeqs && o.num_tokens * o.part_vecs * o.part_vecs < (1ll << 32);
-  }
-  if (by_vectors) {
-    for (int i = 0; i < jobs.n; ++i) {
-      jobs.job[i].first_wg = (int32_t)wg;
-      wg += (jobs.job[i].num_tokens * jobs.job[i].part_vecs + kVectorThreads - 1) / kVectorThreads;
-    }
-    ScopedTimer timer(timer_id, s);
-    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)wg), dim3(kVectorThreads), 0, s, jobs, buf); };
-    launch(to_buffer ? exchange_vectors_kernel<true> : exchange_vectors_kernel<false>);
-    return check_launch(what);
-  }
   const int64_t slice = slice_bytes(total);
+  int64_t grid[kMaxJobs];   // slices of each job
   for (int i = 0; i < jobs.n; ++i) {
     Job &o = jobs.job[i];
     const bool sum = o.kind == DISTCA_JOB_REPLICA_SUM || o.kind == DISTCA_JOB_COPY_SUM;
     const int64_t round = (sum ? kUnrollSum : o.whole() ? kUnroll : kUnrollParts) * kVecRound;   // one round of the job's own loop
-    int64_t grid;
-    int64_t per = slice_tokens(slice < round ? slice : round, o.num_tokens, (int64_t)o.part_vecs * 16, &grid);
+    int64_t per = slice_tokens(slice < round ? slice : round, o.num_tokens, (int64_t)o.part_vecs * 16, &grid[i]);
     if (!o.whole()) {   // a slice's rows lie within 2^30 bytes on both sides (32-bit offsets), and its vectors within the range of `magic`
       const int64_t widest = o.pitch > o.token_bytes ? o.pitch : o.token_bytes;
       const int64_t most = (1ll << 30) / widest < (1ll << 15) ? (1ll << 30) / widest : (1ll << 15);
-      if (per > most) per = most < 1 ? 1 : most, grid = (o.num_tokens + per - 1) / per;
+      if (per > most) per = most < 1 ? 1 : most, grid[i] = (o.num_tokens + per - 1) / per;
     }
     o.tokens_per_wg = (int32_t)per;
-    jobs.job[i].first_wg = (int32_t)wg;
-    wg += grid;
+  }
+  const bool by_vectors = launch_by_vectors(jobs, total, to_buffer);
+  int64_t wg = 0;
+  for (int i = 0; i < jobs.n; ++i) {
+    Job &o = jobs.job[i];
+    o.first_wg = (int32_t)wg;
+    wg += by_vectors ? (o.num_tokens * o.part_vecs + kVectorThreads - 1) / kVectorThreads : grid[i];
     if (wg > 0x7fffffff) return fail(DISTCA_E_INVALID, "%s: grid too large", what);
   }
+  hipStream_t s = (hipStream_t)stream;
+  uint8_t *buf = (uint8_t *)buffer;
   ScopedTimer timer(timer_id, s);
-  const dim3 g((unsigned)wg), b(kPackThreads);
+  const dim3 g((unsigned)wg), b(by_vectors ? kVectorThreads : kPackThreads);
   auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, b, 0, s, jobs, buf); };
-  if (to_buffer) launch(sums ? exchange_kernel<true, true, true> : parts ? exchange_kernel<true, true, false> : exchange_kernel<true, false, false>);
+  if (by_vectors) launch(to_buffer ? exchange_vectors_kernel<true> : exchange_vectors_kernel<false>);
+  else if (to_buffer) launch(sums ? exchange_kernel<true, true, true> : parts ? exchange_kernel<true, true, false> : exchange_kernel<true, false, false>);
   else launch(sums ? exchange_kernel<false, true, true> : parts ? exchange_kernel<false, true, false> : exchange_kernel<false, false, false>);
   return check_launch(what);
 }

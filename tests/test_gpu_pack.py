@@ -285,15 +285,15 @@ def test_through_torch_ops(cuda):
     assert torch.equal(d.cpu().view(torch.uint8), expd.view(torch.uint8))
 
 
-@pytest.mark.parametrize("scale", [1, 40])
-@pytest.mark.parametrize("sizes,pad", [((8192, 8192, 128, 8192), 0), ((16,), 32), ((1040, 16), 16), ((2048, 24, 2048), None)])
-def test_tokens_of_several_parts(cuda, sizes, pad, scale):
+@pytest.mark.parametrize("sizes,pad,shards,most", [(*form, *layout) for form in [((8192, 8192, 128, 8192), 0), ((16,), 32), ((1040, 16), 16), ((2048, 24, 2048), None)]
+                                                    for layout in [(9, 12), (9, 480), (300, 12)]] + [((262144, 128, 16), 32, 9, 12), ((262144, 128, 16), 32, 300, 3)])
+def test_tokens_of_several_parts(cuda, sizes, pad, shards, most):
     """Parts of a transport token copied straight between their tensors and the buffer, next to a replicated tensor in the
-    same launch, against the oracle's copy of the joined rows: one-vector parts, padding behind the last part, a part read at a pitch;
-    `scale` 40 makes slices of several rounds.  Sizes that are no whole vectors are refused on the host."""
+    same launch, against the oracle's copy of the joined rows: one-vector parts, padding behind the last part, a part read at a pitch, by vectors
+    and (300 shards) by slices, of many tokens and of a part of which one token is several rounds.  Sizes that are no whole vectors are refused on the host."""
     from distca_amd.ops import exchange, plain_job, replicas_job, whole_vectors
-    rng = np.random.default_rng(len(sizes) * 100 + scale)
-    lens = (rng.integers(0, 12, size=9) * scale).astype(np.int64)
+    rng = np.random.default_rng(len(sizes) * 100 + shards + most)
+    lens = rng.integers(0, most, size=shards).astype(np.int64)
     lens[4] += 3
     T = int(lens.sum())
     parts = [rng.integers(0, 256, size=(T, n), dtype=np.uint8) for n in sizes]
@@ -301,16 +301,16 @@ def test_tokens_of_several_parts(cuda, sizes, pad, scale):
     if pad is None:
         assert not whole_vectors(*sizes)
         with pytest.raises(RuntimeError, match="multiple"):
-            exchange([plain_job([dev(p) for p in parts], dev(np.zeros(9, np.int64)), dev(lens))], torch.zeros(64, dtype=torch.uint8, device=cuda), True)
+            exchange([plain_job([dev(p) for p in parts], dev(np.zeros(shards, np.int64)), dev(lens))], torch.zeros(64, dtype=torch.uint8, device=cuda), True)
         return
     tb = sum(sizes) + pad
     off, nbuf = _layout(rng, lens, tb)
     joined = np.concatenate(parts + [np.zeros((T, pad), np.uint8)], axis=1)
     # a second tensor, replicated twice behind the tokens
-    do_shard = np.ones((9, 2), np.int8)
+    do_shard = np.ones((shards, 2), np.int8)
     do_shard[1::2, 1] = 0
     src = rng.integers(0, 256, size=(T, 64), dtype=np.uint8)
-    cp_off = np.zeros((2, 9), np.int64)
+    cp_off = np.zeros((2, shards), np.int64)
     for c in range(2):
         cp_off[c] = nbuf + np.concatenate([[0], np.cumsum(lens * 64)[:-1]])
         nbuf += T * 64
@@ -323,7 +323,7 @@ def test_tokens_of_several_parts(cuda, sizes, pad, scale):
         w[:, 16:16 + p.shape[1]] = p
     d_parts = [dev(p) for p in parts]
     d_parts[-1] = dev(wide[-1])[:, 16:16 + sizes[-1]]
-    print(f"parts {sizes} pad {pad} tokens {T}", flush=True)
+    print(f"parts {sizes} pad {pad} shards {shards} tokens {T}", flush=True)
     exchange([plain_job(d_parts, dev(off), dev(lens), token_bytes=tb), replicas_job(dev(src), dev(do_shard), dev(cp_off), dev(lens))], dbuf, True)
     torch.cuda.synchronize()
     assert np.array_equal(dbuf.cpu().numpy(), exp)
@@ -334,6 +334,79 @@ def test_tokens_of_several_parts(cuda, sizes, pad, scale):
         want = np.full(b.shape, 0x5A, np.uint8)
         want[:, 16:16 + p.shape[1]] = p
         assert np.array_equal(b.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("what,mb", [(w, mb) for w in ("pack", "unpack", "reply", "sum") for mb in (20, 100)] + [("pack", 60)])
+def test_either_side_of_the_lines_between_vectors_and_slices(cuda, what, mb):
+    """The same shards by either kernel: few and long, so that the lines lie between 30 and 60 MB (and a pack's again above 84)."""
+    from distca_amd.ops import exchange, plain_job, replica_sum_job
+    rng = np.random.default_rng(mb)
+    sizes = [4096, 128] if what == "reply" else [4096]
+    tb = sum(sizes)
+    T = mb * 10 ** 6 // tb
+    lens = np.array([T // 3, 1, 0, T // 2, T - T // 3 - T // 2 - 1], dtype=np.int64)
+    off, nbuf = _layout(rng, lens, tb)
+    dev = lambda a: torch.from_numpy(a).to(cuda)
+    print(f"{what} {T} tokens", flush=True)
+    if what == "pack":
+        rows, exp, dbuf = rng.integers(0, 256, size=(T, tb), dtype=np.uint8), np.zeros(nbuf, np.uint8), torch.zeros(nbuf, dtype=torch.uint8, device=cuda)
+        fa2a.copy_non_cp(rows, exp, off, lens, None, True)
+        exchange([plain_job([dev(rows)], dev(off), dev(lens))], dbuf, True)
+        torch.cuda.synchronize()
+        assert np.array_equal(dbuf.cpu().numpy(), exp)
+        return
+    buf = torch.randint(-9, 10, (nbuf // 2,), generator=torch.Generator().manual_seed(mb)).to(torch.bfloat16).view(torch.uint8)
+    exp = np.zeros((T, tb), np.uint8)
+    fa2a.copy_non_cp(exp, buf.numpy(), off, lens, None, False)
+    if what == "sum":   # two replicas of every row, the second the first one over again
+        got = torch.empty((T, tb // 2), dtype=torch.bfloat16, device=cuda)
+        exchange([replica_sum_job(got, torch.ones((5, 2), dtype=torch.int8, device=cuda), dev(np.stack([off, off])), dev(lens))], buf.to(cuda), False)
+        torch.cuda.synchronize()
+        assert torch.equal(got.cpu(), 2 * torch.from_numpy(exp).view(torch.bfloat16))
+        return
+    got = [torch.empty((T, n), dtype=torch.uint8, device=cuda) for n in sizes]
+    exchange([plain_job(got, dev(off), dev(lens))], buf.to(cuda), False)
+    torch.cuda.synchronize()
+    assert np.array_equal(np.concatenate([x.cpu().numpy() for x in got], axis=1), exp)
+
+
+@pytest.mark.parametrize("shards", [20, 300])
+def test_parts_beside_sums_in_one_launch(cuda, shards):
+    """A token of two parts and a tensor whose copies are added up, in one launch, and the parts taken apart beside a sum over replicas: by vectors,
+    and by slices (300 shards)."""
+    from distca_amd.ops import copy_sum_job, exchange, plain_job, replica_sum_job
+    rng = np.random.default_rng(shards)
+    lens = rng.integers(0, 30, size=shards).astype(np.int64)
+    lens[7] = lens[3]
+    T, start = int(lens.sum()), np.concatenate([[0], np.cumsum(lens)])
+    dev = lambda a: torch.from_numpy(a).to(cuda)
+    parts = [rng.integers(0, 256, size=(T, n), dtype=np.uint8) for n in (1040, 16)]
+    off, at = _layout(rng, lens, 1056)
+    main = torch.randint(-2, 3, (T, 72), generator=torch.Generator().manual_seed(shards)).to(torch.bfloat16)
+    sum_off, nbuf = _layout(rng, lens, 144)
+    sum_off += at
+    nbuf += at
+    nc, cs = np.zeros(shards, np.int32), np.zeros((shards, 1), np.int64)
+    nc[3], cs[3, 0] = 1, start[7]
+    mask = (np.arange(shards) != 7).astype(np.int8)
+    exp, exp_main = np.zeros(nbuf, np.uint8), main.clone()
+    fa2a.copy_non_cp(np.concatenate(parts, axis=1), exp, off, lens, None, True)
+    fa2a.grad_sum(exp_main, nc, cs, lens)
+    fa2a.copy_non_cp(exp_main.view(torch.uint8).numpy(), exp, sum_off, lens, mask, True)
+    d, dbuf = main.to(cuda), torch.zeros(nbuf, dtype=torch.uint8, device=cuda)
+    print(f"parts beside sums, {shards} shards", flush=True)
+    exchange([plain_job([dev(p) for p in parts], dev(off), dev(lens)), copy_sum_job(d, dev(sum_off), dev(lens), dev(mask), dev(nc), dev(cs))], dbuf, True)
+    back = [torch.zeros((T, n), dtype=torch.uint8, device=cuda) for n in (1040, 16)]
+    total = torch.empty((T, 72), dtype=torch.bfloat16, device=cuda)
+    do_shard = np.stack([mask, np.zeros(shards, np.int8), mask], axis=1)
+    exchange([plain_job(back, dev(off), dev(lens)), replica_sum_job(total, dev(np.ascontiguousarray(do_shard)), dev(np.stack([sum_off] * 3)), dev(lens))], dbuf, False)
+    torch.cuda.synchronize()
+    assert np.array_equal(dbuf.cpu().numpy(), exp) and torch.equal(d.cpu(), exp_main)
+    for x, p in zip(back, parts):
+        assert np.array_equal(x.cpu().numpy(), p)
+    want = 2 * exp_main
+    want[int(start[7]):int(start[8])] = 0
+    assert torch.equal(total.cpu(), want)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
