@@ -362,7 +362,7 @@ __global__ __launch_bounds__(kPackThreads, SUMS ? 4 : 8) void exchange_kernel(Jo
 // whatever shard it lies in: a wave reads the lengths, places and masks of 64 shards at once, a lane a shard, finds by lane moves where its
 // vectors go, and all of them travel together; what is packed is requested before the list is read.
 // us by slices / by vectors, pack, reply, request and gradients of the linear side: 1024 tokens at 8/2 heads (3 / 2 / 7 / 3 MB)
-// 7.7 7.1 11.5 9.0 / 4.3 3.9 6.0 5.0.  Which of the two a launch takes: launch_by_vectors.
+// 7.7 7.1 11.5 9.0 / 4.3 3.9 6.0 5.0.  Which of the two a launch takes: vectors_gain.
 constexpr int kVectorThreads = 256;
 constexpr int kVectorSeqs = 256;             // shards of a job: four reads of 64
 
@@ -639,12 +639,12 @@ int add_job(Jobs *jobs, const distca_exchange_job &in, int64_t token_bytes, int 
   return 0;
 }
 
-// Whether a launch of `total` bytes goes by vectors.  Slices have many vectors of a thread in flight and gain on bandwidth, the sooner the less there is to
+// The lines between slices and vectors.  Slices have many vectors of a thread in flight and gain on bandwidth, the sooner the less there is to
 // be found out on the way: an unpack by vectors cannot ask for anything before the list is read, while a pack has its rows by then; adding rows up, a
 // vector has a load in flight at a time.  What slices lose is a trip there and back for each run they walk, so that every line lies further up
 // the more shards there are to the slice of a job; rows of several replicas and parts of a few bytes a token (lse of 8 heads) cost slices more than the
 // bandwidth gives up to 128 MB.  Of 1134 launches of 16 to 127 MB (4 to 64 heads, 3 to 250 documents) the one chosen is at most 9 % slower than the
-// other, 19 times more than 5 %, where one line of 128 MB, 32 MB with sums, took up to 94 % longer.  us by slices / by vectors around the lines (12 documents at 32/8 heads, every replica's mask set once in four, where nothing else is said):
+// other, 19 times more than 5 %, where one line of 128 MB, 32 MB with sums, took up to 93 % longer.  us by slices / by vectors around the lines (12 documents at 32/8 heads, every replica's mask set once in four, where nothing else is said):
 //   one tensor unpacked          24 MB 14.1 / 13.6   32 MB 16.1 / 16.6   48 MB 20.6 / 22.7   64 MB 25.0 / 28.9
 //   q, k, v unpacked             32 MB 17.4 / 16.7   48 MB 21.9 / 23.0   120 documents, 40 MB 26.2 / 24.5, 72 MB 35.6 / 39.3
 //   one tensor packed            32 MB 16.1 / 15.4   48 MB 20.7 / 20.7   64 MB 25.2 / 26.1
@@ -656,14 +656,20 @@ int add_job(Jobs *jobs, const distca_exchange_job &in, int64_t token_bytes, int 
 // not where a wave looks through several reads of shards, 250 of them 38.9 / 44.6.)
 constexpr int64_t kVectorUnpackBytes = 30 * 1000 * 1000, kVectorPackBytes = 40 * 1000 * 1000, kVectorSumBytes = 50 * 1000 * 1000, kVectorMostBytes = 128ll << 20;
 constexpr int64_t kNarrowPartBytes = 128;
-bool launch_by_vectors(const Jobs &jobs, int64_t total, int to_buffer) {
-  if (total > kVectorMostBytes) return false;
+// One vector a thread is possible: a vector's number times the vectors of a part stays below 2^32 (Job::magic).
+bool vectors_can(const Jobs &jobs, int64_t total) {
+  for (int i = 0; i < jobs.n; ++i) {
+    const Job &o = jobs.job[i];
+    if (o.num_seq > kVectorSeqs || o.num_tokens * o.part_vecs * o.part_vecs >= (1ll << 32)) return false;
+  }
+  return total <= kVectorMostBytes;
+}
+// Which of the two for a launch that may take either (tokens_per_wg: of its slices).
+bool vectors_gain(const Jobs &jobs, int64_t total, int to_buffer) {
   bool sums = false, replicas = false, parts = false, narrow = false, one_read = true;
   double walked = 0;   // shards, and their replicas, that a slice walks
   for (int i = 0; i < jobs.n; ++i) {
     const Job &o = jobs.job[i];
-    // (a vector's number times the vectors of a part stays below 2^32: Job::magic)
-    if (o.num_seq > kVectorSeqs || o.num_tokens * o.part_vecs * o.part_vecs >= (1ll << 32)) return false;
     const bool adds_replicas = o.kind == DISTCA_JOB_REPLICA_SUM;
     sums |= adds_replicas || o.kind == DISTCA_JOB_COPY_SUM;
     replicas |= o.kind == DISTCA_JOB_REPLICAS;
@@ -688,21 +694,24 @@ int launch_exchange(Jobs &jobs, void *buffer, int to_buffer, void *stream, int t
     sums |= o.kind == DISTCA_JOB_REPLICA_SUM || o.kind == DISTCA_JOB_COPY_SUM;
     parts |= !o.whole();
   }
-  const int64_t slice = slice_bytes(total);
-  int64_t grid[kMaxJobs];   // slices of each job
-  for (int i = 0; i < jobs.n; ++i) {
-    Job &o = jobs.job[i];
-    const bool sum = o.kind == DISTCA_JOB_REPLICA_SUM || o.kind == DISTCA_JOB_COPY_SUM;
-    const int64_t round = (sum ? kUnrollSum : o.whole() ? kUnroll : kUnrollParts) * kVecRound;   // one round of the job's own loop
-    int64_t per = slice_tokens(slice < round ? slice : round, o.num_tokens, (int64_t)o.part_vecs * 16, &grid[i]);
-    if (!o.whole()) {   // a slice's rows lie within 2^30 bytes on both sides (32-bit offsets), and its vectors within the range of `magic`
-      const int64_t widest = o.pitch > o.token_bytes ? o.pitch : o.token_bytes;
-      const int64_t most = (1ll << 30) / widest < (1ll << 15) ? (1ll << 30) / widest : (1ll << 15);
-      if (per > most) per = most < 1 ? 1 : most, grid[i] = (o.num_tokens + per - 1) / per;
+  bool by_vectors = vectors_can(jobs, total);
+  int64_t grid[kMaxJobs];   // slices of each job (below the lowest of the lines nothing asks for them)
+  if (!by_vectors || total > kVectorUnpackBytes) {
+    const int64_t slice = slice_bytes(total);
+    for (int i = 0; i < jobs.n; ++i) {
+      Job &o = jobs.job[i];
+      const bool sum = o.kind == DISTCA_JOB_REPLICA_SUM || o.kind == DISTCA_JOB_COPY_SUM;
+      const int64_t round = (sum ? kUnrollSum : o.whole() ? kUnroll : kUnrollParts) * kVecRound;   // one round of the job's own loop
+      int64_t per = slice_tokens(slice < round ? slice : round, o.num_tokens, (int64_t)o.part_vecs * 16, &grid[i]);
+      if (!o.whole()) {   // a slice's rows lie within 2^30 bytes on both sides (32-bit offsets), and its vectors within the range of `magic`
+        const int64_t widest = o.pitch > o.token_bytes ? o.pitch : o.token_bytes;
+        const int64_t most = (1ll << 30) / widest < (1ll << 15) ? (1ll << 30) / widest : (1ll << 15);
+        if (per > most) per = most < 1 ? 1 : most, grid[i] = (o.num_tokens + per - 1) / per;
+      }
+      o.tokens_per_wg = (int32_t)per;
     }
-    o.tokens_per_wg = (int32_t)per;
+    by_vectors = by_vectors && vectors_gain(jobs, total, to_buffer);
   }
-  const bool by_vectors = launch_by_vectors(jobs, total, to_buffer);
   int64_t wg = 0;
   for (int i = 0; i < jobs.n; ++i) {
     Job &o = jobs.job[i];
