@@ -91,15 +91,23 @@ def test_prefix_lengths_around_tile_and_ring_boundaries(cuda, hq, hkv):
     _run(q_lens, k_lens, hq, hkv, 21, cuda)
 
 
+@pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("hq,hkv", [(8, 8), (16, 8), (32, 8)])
-def test_runs_of_whole_tiles_and_blocks(cuda, hq, hkv):
+def test_runs_of_whole_tiles_and_blocks(cuda, hq, hkv, causal):
     """Documents long enough for the runs of whole tiles (dQ) and whole blocks (dK/dV) whose requests stand between the MFMAs, of lengths that end
     a key, a row and a block either side of where the runs end, and enough of them that dK/dV items of both walk directions are among them
     (more key blocks than compute units serve a kv head).  At most four query heads per kv head: a bf16-rounded P of about 1 per head (a
     document's first rows) puts a deviation of 2^-9 / sqrt(3) * sqrt(1.5 heads) on an entry of dV there, and five of them, the largest of the
     eighty thousand such entries here, are 1.4e-2 for four heads and, at the bar of 2e-2, 2.0e-2 for eight."""
     lens = [1031, 769, 770, 768, 767, 991, 1024, 1023, 1025, 640, 832]
-    _run(lens, lens, hq, hkv, 23, cuda)
+    _run(lens, lens, hq, hkv, 23, cuda, causal=causal)
+
+
+def test_runs_of_whole_tiles_in_merged_blocks_non_causal(cuda):
+    """Without a diagonal every tile of a document but the last is whole, also for the blocks that one work item takes after another:
+    documents short enough to be merged (below 768 tokens on average, more than 12 blocks of rows per compute unit)."""
+    lens = [577, 640, 575, 576, 704, 321] * 8
+    _run(lens, lens, 32, 8, 25, cuda, causal=False)
 
 
 @pytest.mark.parametrize("hq,hkv,lens", [(4, 1, [1020]), (4, 1, [1030]), (4, 1, [1540]), (4, 1, [1600]), (32, 8, [2048]), (64, 16, [2050]), (16, 4, [1800, 250])])
