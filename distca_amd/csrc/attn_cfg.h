@@ -165,7 +165,7 @@ inline bool few_row_blocks(const distca_ca_params *p) {
 }
 // An upper bound, times *scale, of the KV tiles that cutting could take off the longest block of query rows: all of its tiles but the load of a
 // unit, of which only the part counts that the task of the longest prefix brings along, half of its tiles for every block of that task per unit
-// (from two blocks per unit on longest-first evens a task out by itself).  How many rows that task has is known where it is the only one, and
+// (from two blocks per unit on pieces, of which there are two a unit, are on average no shorter than the task's blocks: asked, the list builder cuts none of such a task).  How many rows that task has is known where it is the only one, and
 // where the tasks are whole documents, which equal bounds within the batch's tokens are taken for: of all lengths up to the bound, which need
 // not be reached, a document of one block per unit has the most to gain.  Otherwise the most rows may be one task's and the longest
 // prefix another's, a new document's and a short shard's at the end of a long one; then all tiles count, and the list builder, which sees
