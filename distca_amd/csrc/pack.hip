@@ -643,7 +643,7 @@ int add_job(Jobs *jobs, const distca_exchange_job &in, int64_t token_bytes, int 
 // be found out on the way: an unpack by vectors cannot ask for anything before the list is read, while a pack has its rows by then; adding rows up, a
 // vector has a load in flight at a time.  What slices lose is a trip there and back for each run they walk, so that every line lies further up
 // the more shards there are to the slice of a job; rows of several replicas and parts of a few bytes a token (lse of 8 heads) cost slices more than the
-// bandwidth gives up to 128 MB.  Of 1134 launches of 16 to 127 MB (4 to 64 heads, 3 to 250 documents) the one chosen is at most 9 % slower than the
+// bandwidth gives up to 128 MB.  Of 1134 launches of 16 to 127 MB (4 to 64 heads, 3 to 250 documents) the one chosen is at most 10 % slower than the
 // other, 19 times more than 5 %, where one line of 128 MB, 32 MB with sums, took up to 93 % longer.  us by slices / by vectors around the lines (12 documents at 32/8 heads, every replica's mask set once in four, where nothing else is said):
 //   one tensor unpacked          24 MB 14.1 / 13.6   32 MB 16.1 / 16.6   48 MB 20.6 / 22.7   64 MB 25.0 / 28.9
 //   q, k, v unpacked             32 MB 17.4 / 16.7   48 MB 21.9 / 23.0   120 documents, 40 MB 26.2 / 24.5, 72 MB 35.6 / 39.3
