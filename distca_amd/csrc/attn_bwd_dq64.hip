@@ -1,17 +1,22 @@
 // dQ of the varlen causal attention backward for gfx950, 64 query rows per wave.
 //
 // One workgroup of 4 waves per (task, block of 256 flattened query rows, kv head), one wave per SIMD with the
-// SIMD's whole register file.  A wave owns two sub-blocks of 32 rows: their Q and dO stay in registers as MFMA B
+// SIMD's whole register file.  A wave owns four sub-blocks of 16 rows: their Q and dO stay in registers as MFMA B
 // operands, their dQ^T accumulators in the accumulation registers.  K/V tiles of 32 keys stream through a ring of
 // four LDS stages by LDS-direct loads, from key 0 up to the last key the block's rows see; every LDS fragment a
-// wave reads (K rows, V rows, transposed K) feeds two MFMAs, one per sub-block: half the LDS bytes per MFMA of
-// a wave that owns 32 rows.  With one wave per SIMD the arithmetic of a tile is written between the MFMAs of the
-// same tile, as in the dK/dV kernel (attn_bwd_dkdv64.hip):
+// wave reads (K rows, V rows, transposed K) feeds four MFMAs, one per sub-block.  With one wave per SIMD the
+// arithmetic of a tile is written between the MFMAs of the same tile:
 //
-//   step 1   S^T  = K Q^T        16 MFMAs   A: rows of the K tile (LDS), B: Q registers
-//   step 2   dP^T = V dO^T       16 MFMAs   A: rows of the V tile, B: dO registers      beside them: P from S
-//   step 3   dQ^T += K^T dS^T    16 MFMAs   A: transposing reads of the K tile, B: dS   beside them: dS = P (dP - delta)
-//                                           of the keys and sub-block whose MFMAs come later in the step
+//   S^T  = K Q^T        32 MFMAs   A: rows of the K tile (LDS), B: Q registers
+//   dP^T = V dO^T       32 MFMAs   A: rows of the V tile, B: dO registers
+//   dQ^T += K^T dS^T    32 MFMAs   A: transposing reads of the K tile, B: dS = P (dP - delta) with P = exp2(S c - lse2)
+//
+// 16x16x32 MFMAs rather than 32x32x16: the kernel is bound by power, and a FLOP of theirs moves half the accumulator
+// bytes (and twice the operand bytes, which cost less where neighbours share one).  A loop of nothing but MFMAs delivers
+// 1 765 TFLOP/s with the latter and 2 044 with the former, with half a KB of LDS reads and 2.3 vector instructions per
+// 32 K FLOP beside them 1 520 and 1 630 to 1 710.  They leave 2 issue slots each for anything else (the larger ones 5), so the side work
+// is spread over the whole tile.  The kernel, before -> after: 131072 packed tokens at 32/8 heads 16 870 us -> 15 510
+// (1.66 -> 1.9 GHz at 78 % of the pipe's cycles), a tick of 16384 tokens 1 837 -> 1 711, documents of 128 to 2048 tokens 1 268 -> 1 251.
 //
 // The prologue also makes the row statistics of the backward (delta = <dO, O>, lse in the log2 domain) and leaves
 // them in the workspace for the dK/dV kernel, which runs after this one.
@@ -29,7 +34,7 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kRowsWg = 256;            // flattened query rows per workgroup (kDqRows)
 constexpr int kKeys = 32;               // keys per tile
-constexpr int kRow = 256;               // bytes per tile row, chunks swizzled by tile_swz
+constexpr int kRow = 256;               // bytes per tile row, chunks swizzled by tile_swz16
 constexpr int kTile = kKeys * kRow;
 constexpr int kStageBytes = 2 * kTile;  // K tile, V tile
 constexpr int kStages = 4;
@@ -39,41 +44,48 @@ constexpr int kLds = kLdsRing + 4 * kRowsLds;
 static_assert(kLds <= 160 * 1024 && kRowsLds >= 64 * kRow, "LDS of a compute unit");
 constexpr int kLoadsPerTile = 4;        // vector-memory instructions a wave issues per tile
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr int kLead = 2;                // fragments by which sub-block 0 leads in the dQ step
-constexpr int kFrags = 4;               // transposed K fragments held at a time
+constexpr int kDoAcc = 2;               // of a wave's four sub-blocks, those whose dO lies in accumulation registers
+constexpr int kAhead = 3;               // tiles by which requests run ahead
 static_assert(kDqRows == kRowsWg, "the dQ work list is built for blocks of 256 rows");
 
 template <int N>
 __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
+// all LDS reads (the compiler knows this form and puts no waits of its own behind it)
+__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xc07f); }
 __device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
 // The S and dP accumulators are read and overwritten by the vector ALU and must live in vector registers; this file
 // is compiled with the compiler's default MFMA form (results in the accumulation registers, right for dQ), so
 // these MFMAs are written as assembly.  The compiler does not space such an instruction from the vector
-// instructions that read its result (an eight-pass MFMA: 11 quad-cycles from its issue): the order of a tile's
-// instructions below, held in place by the scheduling fences, keeps between every such MFMA and the first read of its
-// result either two later MFMAs, or one later MFMA (which cannot start before the pipe has finished the eight passes
-// of the one in question) and at least four vector instructions; a change to the tile body has to keep that.
-__device__ __forceinline__ void mfma32_v(f32x16 &acc, elemx8 a, elemx8 b) {
-  asm volatile(DISTCA_MFMA32_ASM " %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
-}
-__device__ __forceinline__ void mfma32_vc(f32x16 &acc, elemx8 a, elemx8 b, const f32x16 &c0) {  // acc = A B + c0
-  asm volatile(DISTCA_MFMA32_ASM " %0, %1, %2, %3" : "=&v"(acc) : "v"(a), "v"(b), "v"(c0));
-}
-// The same with the B operand in accumulation registers, where Q lives: a wave's 512 registers are 256 of each
-// kind, and the vector half is what the tile arithmetic is short of.
+// instructions that read its result (a four-pass MFMA: 8 wait states): the order of a tile's instructions below,
+// held in place by the scheduling fences, keeps at least three later MFMAs, each of which waits for the four passes
+// of the one before it, between every such MFMA and the first read of its result; a change to the tile body has to keep that.
+// The B operands, Q and dO, are in accumulation registers: a wave's 512 registers are 256 of each kind, and the
+// vector half is what the tile arithmetic is short of.
 typedef float accop_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ accop_t to_acc_regs(elemx8 v) {
   accop_t r;
   asm volatile("; operand to accumulation registers" : "=a"(r) : "0"(__builtin_bit_cast(accop_t, v)));
   return r;
 }
-__device__ __forceinline__ void mfma32_va(f32x16 &acc, elemx8 a, accop_t b) {
-  asm volatile(DISTCA_MFMA32_ASM " %0, %1, %2, %0" : "+v"(acc) : "v"(a), "a"(b));
+__device__ __forceinline__ void mfma16_va(f32x4 &acc, elemx8 a, accop_t b) {  // acc += A B
+  asm volatile(DISTCA_MFMA16_ASM " %0, %1, %2, %0" : "+v"(acc) : "v"(a), "a"(b));
 }
-__device__ __forceinline__ void mfma32_va0(f32x16 &acc, elemx8 a, accop_t b) {
-  asm volatile(DISTCA_MFMA32_ASM " %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "a"(b));
+__device__ __forceinline__ void mfma16_va0(f32x4 &acc, elemx8 a, accop_t b) {  // acc = A B
+  asm volatile(DISTCA_MFMA16_ASM " %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "a"(b));
+}
+__device__ __forceinline__ void mfma16_a(f32x4 &acc, elemx8 a, elemx8 b) {  // acc += A B, in accumulation registers
+  asm volatile(DISTCA_MFMA16_ASM " %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void mfma16_v(f32x4 &acc, elemx8 a, elemx8 b) {
+  asm volatile(DISTCA_MFMA16_ASM " %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void mfma16_vc(f32x4 &acc, elemx8 a, elemx8 b, const f32x4 &c0) {
+  asm volatile(DISTCA_MFMA16_ASM " %0, %1, %2, %3" : "=&v"(acc) : "v"(a), "v"(b), "v"(c0));
+}
+__device__ __forceinline__ void mfma16_vac(f32x4 &acc, elemx8 a, accop_t b, const f32x4 &c0) {  // acc = A B + c0
+  asm volatile(DISTCA_MFMA16_ASM " %0, %1, %2, %3" : "=&v"(acc) : "v"(a), "a"(b), "v"(c0));
 }
 
 // SEG: K/V rows are addressed through a table of shards (kv_shards.h) instead of as one dense tensor.
@@ -133,7 +145,7 @@ next_block:
   if constexpr (MERGE) asm volatile("" : "+v"(tid_));
   const int tid = tid_, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l32 = lane & 31, g = lane >> 5;
+  const int c16 = lane & 15, g4 = lane >> 4;
   const int row_wg = mblk * kRowsWg;
 
   int tok_end = (row_wg + kRowsWg + G - 1) / G;
@@ -170,7 +182,7 @@ next_block:
 #pragma unroll
   for (int ii = 0; ii < 2; ++ii) {
     const int r = 8 * wave + 4 * ii + (lane >> 4);
-    voff[ii] = (uint32_t)((r * kv_stride + (((lane & 15) ^ tile_swz(r)) * 8)) * 2);
+    voff[ii] = (uint32_t)((r * kv_stride + (((lane & 15) ^ tile_swz16(r)) * 8)) * 2);
   }
   // SEG: tiles that end at or before key run_lim lie in the present shard, key x of the prefix at kvirt / vvirt +
   // x * kv_stride; a tile past it looks for its shard first, so that a run of tiles inside one shard is requested
@@ -205,7 +217,7 @@ next_block:
       for (int ii = 0; ii < 2; ++ii) {
         const int r = 8 * wave + 4 * ii + (lane >> 4);
         const int key = j * kKeys + r;
-        const int chunk = (lane & 15) ^ tile_swz(r);
+        const int chunk = (lane & 15) ^ tile_swz16(r);
         const bool ok = key < lk;
         const uint8_t *zero = reinterpret_cast<const uint8_t *>(a.zero_row);
         const uint8_t *kp = ok ? reinterpret_cast<const uint8_t *>(kbase) + shard_row_offset(a.shards, cur, ks + key, 0, kv_stride * 2) : zero;
@@ -226,7 +238,7 @@ next_block:
       for (int ii = 0; ii < 2; ++ii) {
         const int r = 8 * wave + 4 * ii + (lane >> 4);
         const int key = j * kKeys + r;
-        const int chunk = (lane & 15) ^ tile_swz(r);
+        const int chunk = (lane & 15) ^ tile_swz16(r);
         const bool ok = key < lk;
         const elem_t *kp = ok ? kbase + (int64_t)key * kv_stride : reinterpret_cast<const elem_t *>(a.zero_row);
         const elem_t *vp = ok ? vbase + (int64_t)key * kv_stride : reinterpret_cast<const elem_t *>(a.zero_row);
@@ -243,25 +255,25 @@ next_block:
     issue_tile(1, 1);
   }
 
-  // ---- this lane's two rows: Q and dO as B operands (row l32 of a sub-block, d = 16 s + 8 g .. +7), statistics
-  int row[2], tok[2], lim[2];
-  bool valid[2];
-  float lse2[2], delta[2];
-  accop_t qf[2][8];
-  elemx8 dof[2][8];
+  // ---- this lane's four rows: Q and dO as B operands (row c16 of a sub-block of 16, d = 32 s + 8 g4 .. +7), statistics
+  int row[4], tok[4], lim[4];
+  bool valid[4];
+  float lse2[4], delta[4];
+  accop_t qf[4][4], dof[kDoAcc][4];
+  elemx8 dov[4 - kDoAcc][4];
   // The wave's 64 rows of Q, dO and O come through LDS: LDS-direct loads bring four whole rows of 256 bytes per
-  // instruction, and the lanes then read their operand fragments (row l32 of a sub-block, chunk 2 s + g) from there.
+  // instruction, and the lanes then read their operand fragments (row c16 of a sub-block, chunk 4 s + g4) from there.
   // Loaded straight into the operand layout, every load instruction touched 32 rows, 32 bytes of each, and the address
   // unit takes about a cycle per cache line it has to look up: 48 such loads per wave took 7.7 us to *issue*, a third
   // of what a block of a 1024-token document then spent in its tile loop.  The rows use the 24 KB per wave that lie
-  // behind the tile ring (the 32 rows of a sub-block of Q, dO and O at a time), so the ring is free for the first tiles
+  // behind the tile ring (32 rows of Q, dO and O at a time), so the ring is free for the first tiles
   // meanwhile, and each wave reads only what it has loaded itself: no barrier.
-  // Before that, and also in one batch, the lse of the lane's two rows (the opaque statements that move Q into the
+  // Before that, and also in one batch, the lse of the lane's four rows (the opaque statements that move Q into the
   // accumulation registers order memory accesses around themselves: no load may be left between them).
-  float lse_row[2];
+  float lse_row[4];
 #pragma unroll
-  for (int m = 0; m < 2; ++m) {
-    row[m] = row_wg + (wave * 2 + m) * 32 + l32;
+  for (int m = 0; m < 4; ++m) {
+    row[m] = row_wg + wave * 64 + 16 * m + c16;
     valid[m] = row[m] < nrows;
     // A row past the task (the last block of a task only) reads the task's last row instead, without a branch: with
     // lse2 = +inf its P and dS are zero whatever Q and dO hold, as long as they are finite, and nothing of it is stored.
@@ -275,8 +287,8 @@ next_block:
                            : a.lse[(int64_t)(kvh * G + hg) * a.total_q + q0 + tok[m]];
   }
   const int wrow0 = row_wg + wave * 64;
-  const uint32_t stg = lds0 + kLdsRing + wave * kRowsLds;  // [Q | dO | O] of one sub-block, 8 KB each
-  // requests sub-block m of the wave's rows in block `blk` of the task: instruction i brings rows 32 m + 4 i + lane / 16
+  const uint32_t stg = lds0 + kLdsRing + wave * kRowsLds;  // [Q | dO | O] of one half of the wave's rows, 8 KB each
+  // requests half m of the wave's rows in block `blk` of the task: instruction i brings rows 32 m + 4 i + lane / 16
   // of the wave, lane % 16 being the position of the 16-byte chunk in the (swizzled) LDS row
   auto request_rows = [&](int blk, int m) {
     const int rw = blk * kRowsWg;
@@ -291,7 +303,7 @@ next_block:
       int rg = rw + wave * 64 + r;
       if (rg > nrows - 1) rg = nrows - 1;
       const int t = div_group(rg);
-      roff[i] = (uint32_t)((t - tok0) * a.qs_tok_bytes + (rg - t * G) * (kHeadDim * 2) + (((lane & 15) ^ tile_swz(r)) << 4));
+      roff[i] = (uint32_t)((t - tok0) * a.qs_tok_bytes + (rg - t * G) * (kHeadDim * 2) + (((lane & 15) ^ tile_swz16(r)) << 4));
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) lds_direct_load16(qb, roff[i], stg + i * 4 * kRow);
@@ -300,41 +312,101 @@ next_block:
 #pragma unroll
     for (int i = 0; i < 8; ++i) lds_direct_load16(ob, roff[i], stg + 2 * kTile + i * 4 * kRow);
   };
-  {
-    const uint32_t frag = l32 * kRow + ((g ^ tile_swz(l32)) << 4);  // this lane's chunk 0 of row l32; ^ (s << 5)
-    elemx8 qt[2][8], ot[2][8];
+  const float c = a.scale * kLog2e;
+  const int k_rd = c16 * kRow + ((g4 ^ tile_swz16(c16)) << 4);  // A operand rows of a tile, ^ 64*s
+  // transposed K operand: lane points at (key 4 g4 + i4 [+ 16], chunk h1 [+ 2 db], half lane & 1)
+  const int i4 = (lane & 15) >> 2, h1 = (lane & 3) >> 1;
+  const int t_rd = (4 * g4 + i4) * kRow + ((h1 ^ tile_swz16(4 * g4 + i4)) << 4) + 8 * (lane & 1);  // ^ 32*db
+
+  // Absolute LDS addresses of this lane's operand reads in stage 0, the swizzled variants of each read shape,
+  // kept in registers: where the stage is a constant (the unrolled loop below) stage and tile sit in the read
+  // instruction's offset field and no address arithmetic is left between the MFMAs.
+  uint32_t k_ad[4], t_ad[8];
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      // MERGE: the first sub-block's rows were requested before the previous block of the item stored its results
-      if (m == 0 && !(MERGE && requested)) request_rows(mblk, 0);
-      wait_vm<0>();  // (the first tiles, requested before, and lse as well)
-#pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        qt[m][s] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(stg + (frag ^ (s << 5))));
-        dof[m][s] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(stg + kTile + (frag ^ (s << 5))));
-        ot[m][s] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(stg + 2 * kTile + (frag ^ (s << 5))));
-      }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the reads are done before the place is filled again
-      if (m == 0) request_rows(mblk, 1);   // (they arrive while the first sub-block's sums are made: documents of 128 to 2048 tokens 1 316 us -> 1 307)
-      fence();
-      float part = 0.f;
-#pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        qf[m][s] = to_acc_regs(qt[m][s]);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) part += (float)dof[m][s][i] * (float)ot[m][s][i];
-      }
-      delta[m] = pair_sum(part);  // this lane's half of d, then the sum of the lane pair
-      lse2[m] = valid[m] ? lse_row[m] * kLog2e : INFINITY;  // rows past the task: P = exp2(-inf) = 0
+  for (int i = 0; i < 8; ++i) {
+    t_ad[i] = lds0 + (t_rd ^ (i << 5));
+    asm volatile("" : "+v"(t_ad[i]));
+    if (i < 4) {
+      k_ad[i] = lds0 + (k_rd ^ (i << 6));
+      asm volatile("" : "+v"(k_ad[i]));
     }
   }
-  // -delta of the lane's row in all 16 registers of a vector: the C operand of a tile's first dP MFMA, so that
+
+  f32x4 s0[4], s1[4];        // S, then P, of keys 0 .. 15 and 16 .. 31
+  elemx8 fx[4], fy[4];       // K and V fragments of this phase and the next
+  auto frag = [&](uint32_t so, int s) { return *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(k_ad[s] + so)); };
+  auto p_of = [&](float x, int rb) __attribute__((always_inline)) { return fast_exp2(__builtin_fmaf(x, c, -lse2[rb])); };
+  {
+    const uint32_t frag_at = c16 * kRow + ((g4 ^ tile_swz16(c16)) << 4);  // this lane's chunk 0 of row c16; ^ (s << 6)
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      elemx8 qt[2][4], dt[2][4], ot[2][4];
+      // MERGE: the first half's rows were requested before the previous block of the item stored its results
+      if (m == 0 && !(MERGE && requested)) request_rows(mblk, 0);
+      wait_vm<0>();  // (the first tiles, requested before, and lse as well)
+      if (m == 0) {  // the first two tiles are there
+        fence();
+        asm volatile("s_barrier" ::: "memory");
+        fence();
+      }
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const uint32_t at = stg + 16 * b * kRow + (frag_at ^ (s << 6));
+          qt[b][s] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(at));
+          dt[b][s] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(at + kTile));
+          ot[b][s] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(at + 2 * kTile));
+        }
+      if (m == 0) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) fx[s] = frag(0, s);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the reads are done before the place is filled again
+      if (m == 0) request_rows(mblk, 1);   // (they arrive while the first half's sums are made: documents of 128 to 2048 tokens 1 316 us -> 1 307)
+      fence();
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const int rb = 2 * m + b;
+          qf[rb][s] = to_acc_regs(qt[b][s]);
+          if (rb < kDoAcc) dof[rb][s] = to_acc_regs(dt[b][s]);
+          else dov[rb - kDoAcc][s] = dt[b][s];
+        }
+      float part[2] = {0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          // (without a tile, of whatever the ring holds, for nothing)
+          fence();
+          if (s == 0) mfma16_va0(s0[2 * m + b], fx[s], qf[2 * m + b][s]);
+          else mfma16_va(s0[2 * m + b], fx[s], qf[2 * m + b][s]);
+          fence();
+#pragma unroll
+          for (int i = 0; i < 8; ++i) part[b] += (float)dt[b][s][i] * (float)ot[b][s][i];
+        }
+      fence();
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const int rb = 2 * m + b;
+        delta[rb] = quad_sum(part[b]);  // this lane's quarter of d, then the sum of the four lanes of the row
+        lse2[rb] = valid[rb] ? lse_row[rb] * kLog2e : INFINITY;  // rows past the task: P = exp2(-inf) = 0
+      }
+      if (m == 0) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s0[e >> 2][e & 3] = p_of(s0[e >> 2][e & 3], e >> 2);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) fy[s] = frag(16 * kRow, s);
+  }
+  // -delta of the lane's row in all 4 registers of a vector: the C operand of a tile's first dP MFMA, so that
   // dS = P * (what the MFMAs leave) costs one instruction per element
-  f32x16 ndl[2];
+  f32x4 ndl[4];
 #pragma unroll
-  for (int m = 0; m < 2; ++m)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) ndl[m][r] = -delta[m];
+  for (int m = 0; m < 4; ++m) ndl[m] = f32x4{-delta[m], -delta[m], -delta[m], -delta[m]};
   int wrow1 = wrow0 + 63;
   if (wrow1 > nrows - 1) wrow1 = nrows - 1;
   const bool wave_live = wrow0 < nrows;
@@ -346,40 +418,22 @@ next_block:
     if (lim_last > lk - 1) lim_last = lk - 1;
   }
 
-  f32x16 dqacc[2][4];
+  f32x4 dqacc[4][8];
 #pragma unroll
-  for (int m = 0; m < 2; ++m)
+  for (int m = 0; m < 4; ++m)
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) dqacc[m][db][r] = 0.f;
-  const float c = a.scale * kLog2e;
-  const int k_rd = l32 * kRow + ((g ^ tile_swz(l32)) << 4);  // A operand rows of a tile, ^ 32*s
-  // transposed K operand: lane points at (key 4g + i4 [+8 hi +16 t], chunk 8 b4 + h1 [+2 db], half lane&1);
-  // tile_swz of that row is (i4<<1) | (g<<3) | hi
-  const int i4 = (lane & 15) >> 2, b4 = (lane >> 4) & 1, h1 = (lane & 3) >> 1;
-  const int t_rd = (4 * g + i4) * kRow + ((((b4 ^ g) << 3) | (i4 << 1) | h1) << 4) + 8 * (lane & 1);  // ^ 32*db ^ 16*hi
-
-  // Absolute LDS addresses of this lane's operand reads in stage 0, the eight swizzled variants of each read shape,
-  // kept in registers: where the stage is a constant (the unrolled loop below) stage and tile sit in the read
-  // instruction's offset field and no address arithmetic is left between the MFMAs.
-  uint32_t k_ad[8], t_ad[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    k_ad[i] = lds0 + (k_rd ^ (i << 5));
-    t_ad[i] = lds0 + ((t_rd ^ ((i & 3) << 5) ^ ((i >> 2) << 4)) + (i >> 2) * 8 * kRow);
-    asm volatile("" : "+v"(k_ad[i]), "+v"(t_ad[i]));
-  }
-
-
-  // One tile.  MASKED: the tile straddles the diagonal or the end of the prefix, compare and select per element.
-  // request(i), i = 0 .. 3: the loads of the tile after the next, each between MFMAs of step 1, which has no arithmetic beside it.  (All four behind
-  // the barrier, from all four waves at once, they held the waves up for a seventh of a tile.)  The first two K fragments are there when a tile
-  // begins: in the middle of step 3 the wave waits for the next tile and reads them, so that neither the barrier nor the reads' latency stands
-  // between two tiles' MFMAs.  131072 packed tokens at 32/8 heads, 18 200 us: with the requests between MFMAs 17 750, with both 17 600 (one box); a
-  // conditional jump around each request instead of a loop of its own for tiles that lie whole took 1.7 % back; four K fragments in flight
-  // instead of two, or one M0 write for all four requests, change nothing: the clock gives up what the cycles gain.
-  elemx8 kf[2];
+    for (int db = 0; db < 8; ++db) dqacc[m][db] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // One tile, in six phases of 16 MFMAs.  What a tile begins with is there when it begins: S of its first 16 keys, the exponentials of
+  // sub-blocks 0 and 1 of them (kept as they are until the tile is known to be masked), and the K fragments of its other 16 keys.  A MFMA leaves
+  // two slots for other instructions, so the arithmetic is spread over all phases: per phase 16, 24, 24, 16, 16, 16 vector instructions, about two behind a MFMA.
+  //   1  S, keys 16 .. 31       beside it: P of keys 0 .. 15, sub-blocks 2 and 3; V fragments
+  //   2  dP, keys 0 .. 15       P of keys 16 .. 31, sub-blocks 0 to 2; V fragments; then the barrier for the next tile
+  //   3  dP, keys 16 .. 31      the rest of P; dS of keys 0 .. 15; the next tile's K fragments
+  //   4  S, keys 0 .. 15 of the next tile     dS of keys 16 .. 31, sub-blocks 0 and 1; transposed K fragments
+  //   5  dQ, sub-blocks 0 and 1               the rest of dS; transposed K fragments
+  //   6  dQ, sub-blocks 2 and 3               P of the next tile, keys 0 .. 15, sub-blocks 0 and 1; its K fragments; request(0 .. 3), the loads
+  //                                           of the tile kAhead tiles on, whose stage every wave left before the barrier of phase 2
+  // MASKED: the tile straddles the diagonal or the end of the prefix, compare and select per element.
   auto landed = [&]() {
     // tile p has landed when at most the loads of tile p + 1 are still on their way
     wait_vm<kLoadsPerTile>();
@@ -387,139 +441,165 @@ next_block:
     asm volatile("s_barrier" ::: "memory");
     fence();
   };
-  auto first_k = [&](uint32_t so, int s) { kf[s] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(k_ad[s] + so)); };
-  auto tile = [&](auto stage, auto next_stage, int key0, auto masked, auto request) __attribute__((always_inline)) {  // stages: ints or constants
-    constexpr bool kMasked = decltype(masked)::value;
+  // LAST: there is no next tile for this wave, nothing of it is made.
+  auto tile = [&](auto stage, auto next_stage, int key0, auto masked, auto last, auto request) __attribute__((always_inline)) {  // stages: ints or constants
+    constexpr bool kMasked = decltype(masked)::value, kLast = decltype(last)::value;
     const uint32_t so = (uint32_t)stage * kStageBytes, so_next = (uint32_t)next_stage * kStageBytes;
-    f32x16 sacc[2], dpacc[2];
-    elemx8 vf[2];
-    elemx4 ct[kFrags][2];
-    auto load_k = [&](int s, int buf) { kf[buf] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(k_ad[s] + so)); };
-    auto load_v = [&](int s, int buf) { vf[buf] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(k_ad[s] + so + kTile)); };
-    auto load_t = [&](int n, int buf) {  // n = 4 t + db: keys 16 t .. 16 t + 15, d block db
-      ct[buf][0] = lds_read_tr(lds_ptr(t_ad[n & 3] + so + 16 * (n >> 2) * kRow));
-      ct[buf][1] = lds_read_tr(lds_ptr(t_ad[4 + (n & 3)] + so + 16 * (n >> 2) * kRow));
+    f32x4 d0[4], d1[4];  // dP, then dS
+    elemx4 ct[8][2];
+    auto load_t = [&](int db) {
+      ct[db][0] = lds_read_tr(lds_ptr(t_ad[db] + so));
+      ct[db][1] = lds_read_tr(lds_ptr(t_ad[db] + so + 16 * kRow));
     };
-    // masked: which rows do not see the two keys of the next MFMA's exponentials, found a MFMA ahead: a select has to stand two wait states
-    // behind its compare, and with the two side by side a tile held thirty s_nop (65536 tokens in documents of 128 to 2048: 1 299 us -> 1 280)
-    uint64_t hidden[2][2];
-    int last_key[2];  // of this lane's rows, counted from its first key of the tile
+    // masked: which rows do not see the key of an element, found two elements ahead: a select has to stand two wait states
+    // behind its compare (65536 tokens in documents of 128 to 2048, side by side -> ahead: 1 299 us -> 1 280)
+    uint64_t hidden[4];
+    int last_key[4];  // of this lane's rows, counted from its first key of the tile
+    auto find_hidden = [&](int e) __attribute__((always_inline)) {  // element e: keys 16 (e / 16) + e % 4, sub-block e / 4 % 4
+      if (e >= 32) return;
+      hidden[e & 3] = __builtin_amdgcn_ballot_w64(16 * (e >> 4) + (e & 3) > last_key[(e >> 2) & 3]);
+      asm volatile("" : "+s"(hidden[e & 3]));  // here, not where it is used
+    };
+    auto hide = [&](float x, int e) __attribute__((always_inline)) {
+      if (__builtin_amdgcn_inverse_ballot_w64(hidden[e & 3])) x = 0.f;
+      find_hidden(e + 2);
+      return x;
+    };
+    auto p_elem = [&](int e) __attribute__((always_inline)) {
+      const int rb = (e >> 2) & 3, r = e & 3;
+      float x = p_of(e < 16 ? s0[rb][r] : s1[rb][r], rb);
+      if constexpr (kMasked) x = hide(x, e);
+      if (e < 16) s0[rb][r] = x;
+      else s1[rb][r] = x;
+    };
+    auto ds_elem = [&](int e) __attribute__((always_inline)) {  // dP accumulated on top of -delta
+      const int rb = (e >> 2) & 3, r = e & 3;
+      if (e < 16) d0[rb][r] = s0[rb][r] * d0[rb][r];
+      else d1[rb][r] = s1[rb][r] * d1[rb][r];
+    };
+    // dS as B operand: slots 8 g4 .. +3 are keys 4 g4 .. +3, slots 8 g4 + 4 .. +7 the same 16 keys on
+    // (pinned where they are made: joined at their MFMA, the two halves would be converted there, with nothing between a conversion and the MFMA)
+    u32x2 dsl[4], dsh[4];
+    auto pinned = [](f32x4 x) __attribute__((always_inline)) {
+      asm volatile("" : "+v"(x));
+      u32x2 r = __builtin_bit_cast(u32x2, cvt4(x[0], x[1], x[2], x[3]));
+      asm volatile("" : "+v"(r));
+      return r;
+    };
+    auto ds_lo = [&](int rb) __attribute__((always_inline)) { dsl[rb] = pinned(d0[rb]); };
+    auto ds_hi = [&](int rb) __attribute__((always_inline)) { dsh[rb] = pinned(d1[rb]); };
+    auto ds_frag = [&](int rb) __attribute__((always_inline)) { return cat4(__builtin_bit_cast(elemx4, dsl[rb]), __builtin_bit_cast(elemx4, dsh[rb])); };
     if constexpr (kMasked) {
 #pragma unroll
-      for (int m = 0; m < 2; ++m) last_key[m] = lim[m] - key0 - acc_row(0, g);
+      for (int m = 0; m < 4; ++m) last_key[m] = lim[m] - key0 - 4 * g4;
+      find_hidden(0);
+      find_hidden(1);
     }
-    auto find_hidden = [&](int s) __attribute__((always_inline)) {
-#pragma unroll
-      for (int m = 0; m < 2; ++m)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          hidden[m][i] = __builtin_amdgcn_ballot_w64(acc_row(2 * s + i, 0) > last_key[m]);
-          asm volatile("" : "+s"(hidden[m][i]));  // here, not where it is used
-        }
-    };
-    // ---- step 1: S^T = K Q^T
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      fence();
-      if (s == 0) {
-        mfma32_va0(sacc[0], kf[0], qf[0][0]);
-        mfma32_va0(sacc[1], kf[0], qf[1][0]);
+    auto dp_mfma = [&](f32x4 &acc, elemx8 v, int rb, int s) __attribute__((always_inline)) {
+      if (rb < kDoAcc) {
+        if (s == 0) mfma16_vac(acc, v, dof[rb][s], ndl[rb]);
+        else mfma16_va(acc, v, dof[rb][s]);
       } else {
-        mfma32_va(sacc[0], kf[s & 1], qf[0][s]);
-        mfma32_va(sacc[1], kf[s & 1], qf[1][s]);
+        if (s == 0) mfma16_vc(acc, v, dov[rb - kDoAcc][s], ndl[rb]);
+        else mfma16_v(acc, v, dov[rb - kDoAcc][s]);
       }
-      fence();
-      if (s + 2 < 8) load_k(s + 2, s & 1);
-      if (s >= 6) load_v(s - 6, s - 6);  // the first operands of step 2
-      if (s & 1) request(s >> 1);
-      if (kMasked && s == 7) find_hidden(0);
-    }
-    // ---- step 2: dP^T = V dO^T; beside the MFMAs, P = exp2(S c - lse2) of two elements per MFMA
-    auto p_elem = [&](int m, int r) {
-      float p = fast_exp2(__builtin_fmaf(sacc[m][r], c, -lse2[m]));
-      if constexpr (kMasked) {
-        if (__builtin_amdgcn_inverse_ballot_w64(hidden[m][r & 1])) p = 0.f;
-      }
-      sacc[m][r] = p;
     };
-    auto ds_elem = [&](int m, int r) { dpacc[m][r] = sacc[m][r] * dpacc[m][r]; };  // dP accumulated on top of -delta
-    elemx8 dsf[2][2];
-    auto ds_cvt = [&](int m, int t) {
-      const int r0 = 8 * t;
-      dsf[m][t] = cvt8(dpacc[m][r0], dpacc[m][r0 + 1], dpacc[m][r0 + 2], dpacc[m][r0 + 3], dpacc[m][r0 + 4], dpacc[m][r0 + 5],
-                       dpacc[m][r0 + 6], dpacc[m][r0 + 7]);
-    };
+    // Fragments are requested in the first half of the phase before theirs, so that one wait ahead of a phase does for all of them.
+    // ---- phase 1
+    wait_lds();
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
+    for (int n = 0; n < 16; ++n) {
+      const int s = n >> 2, rb = n & 3;
       fence();
-      if (s == 0) mfma32_vc(dpacc[0], vf[0], dof[0][0], ndl[0]);
-      else mfma32_v(dpacc[0], vf[s & 1], dof[0][s]);
+      if (s == 0) mfma16_va0(s1[rb], fy[s], qf[rb][s]);
+      else mfma16_va(s1[rb], fy[s], qf[rb][s]);
       fence();
-      p_elem(0, 2 * s);
-      p_elem(0, 2 * s + 1);
-      fence();
-      if (s == 0) mfma32_vc(dpacc[1], vf[0], dof[1][0], ndl[1]);
-      else mfma32_v(dpacc[1], vf[s & 1], dof[1][s]);
-      fence();
-      p_elem(1, 2 * s);
-      p_elem(1, 2 * s + 1);
-      if (kMasked && s < 7) find_hidden(s + 1);
-      if (s + 2 < 8) load_v(s + 2, s & 1);
-      if (s >= 8 - kFrags) load_t(s - (8 - kFrags), s - (8 - kFrags));  // the first operands of step 3
+      if (kMasked && n < 4) {  // what was made before the tile was known to be masked
+        s0[n >> 1][2 * (n & 1)] = hide(s0[n >> 1][2 * (n & 1)], 2 * n);
+        s0[n >> 1][2 * (n & 1) + 1] = hide(s0[n >> 1][2 * (n & 1) + 1], 2 * n + 1);
+      }
+      if (n < 8 && n % 2 == 0) fx[n / 2] = frag(so + kTile, n / 2);
+      if (n > 4 && n < 11 && n % 2 == 1) p_elem(8 + (n - 5) / 2);
+      if (n > 10) p_elem(n);
     }
-    fence();
-    // dS of the first 16 keys of sub-block 0: dP is complete only now
+    // ---- phase 2
+    wait_lds();
 #pragma unroll
-    for (int r = 0; r < 8; ++r) ds_elem(0, r);
-    ds_cvt(0, 0);
-    // ---- step 3: dQ^T += K^T dS^T.  Sub-block 0 leads by kLead fragments: dS of sub-block 1's first 16 keys stands
-    // behind its first MFMAs, dS of the other 16 keys of both behind the MFMAs that follow
-    static_assert(kLead == 2 && kFrags == 4, "the portions below are laid out for a lead of two fragments");
-#pragma unroll
-    for (int n = 0; n < kLead; ++n) {
-      const elemx8 kt = cat4(ct[n % kFrags][0], ct[n % kFrags][1]);
+    for (int n = 0; n < 16; ++n) {
+      const int s = n >> 2, rb = n & 3;
       fence();
-      dqacc[0][n & 3] = mfma32(kt, dsf[0][0], dqacc[0][n & 3]);
+      dp_mfma(d0[rb], fx[s], rb, s);
       fence();
-#pragma unroll
-      for (int r = 4 * n; r < 4 * n + 4; ++r) ds_elem(1, r);
+      if (n < 8 && n % 2 == 0) fy[n / 2] = frag(so + kTile + 16 * kRow, n / 2);
+      if (n < 8 && n % 2 == 1) p_elem(16 + n / 2);
+      if (n >= 8) p_elem(12 + n);
     }
-    ds_cvt(1, 0);
+    landed();
+    // ---- phase 3
+    wait_lds();
 #pragma unroll
-    for (int n = 0; n < 8; ++n) {
-      const elemx8 kt1 = cat4(ct[n % kFrags][0], ct[n % kFrags][1]);
+    for (int n = 0; n < 16; ++n) {
+      const int s = n >> 2, rb = n & 3;
       fence();
-      dqacc[1][n & 3] = mfma32(kt1, dsf[1][n >> 2], dqacc[1][n & 3]);
+      dp_mfma(d1[rb], fy[s], rb, s);
       fence();
-      if (n + kFrags < 8) load_t(n + kFrags, n % kFrags);
-      if (n == 0) {
+      if (!kLast && n < 8 && n % 2 == 0) fx[n / 2] = frag(so_next, n / 2);
+      if (n < 8 && n % 2 == 1) p_elem(28 + n / 2);
+      if (n >= 8) ds_elem(2 * n - 16), ds_elem(2 * n - 15);
+    }
+    // ---- phase 4
+    wait_lds();
 #pragma unroll
-        for (int r = 8; r < 12; ++r) ds_elem(0, r);
+    for (int n = 0; n < 16; ++n) {
+      const int s = n >> 2, rb = n & 3;
+      fence();
+      if constexpr (!kLast) {
+        if (s == 0) mfma16_va0(s0[rb], fx[s], qf[rb][s]);
+        else mfma16_va(s0[rb], fx[s], qf[rb][s]);
+      } else if (n < 4) {
+        asm volatile("s_nop 3");  // (in the place of four MFMAs between dP's and the first read of it)
       }
-      if (n == 1) {
+      fence();
+      if (n < 11 && n % 2 == 0) load_t(n / 2);
+      if (n == 1 || n == 3) ds_elem(15 + n), ds_elem(16 + n);
+      if (n == 5) ds_lo(0);
+      if (n == 7) ds_hi(0);
+      if (n == 9 || n == 11) ds_elem(11 + n), ds_elem(12 + n);
+      if (n == 12) ds_lo(1);
+      if (n == 13) ds_hi(1);
+      if (n == 14) ds_lo(2);
+      if (n == 15) ds_lo(3);
+    }
+    // ---- phase 5.  Consecutive MFMAs share an operand, here and in phase 6: what an operand costs in power is its change.
+    wait_lds();
 #pragma unroll
-        for (int r = 12; r < 16; ++r) ds_elem(0, r);
-        ds_cvt(0, 1);
-      }
-      if (n == 2) {
+    for (int n = 0; n < 16; ++n) {
+      const int db = n >> 1, rb = (n ^ db) & 1;
+      if (n == 12) wait_lds();
+      const elemx8 kt = cat4(ct[db][0], ct[db][1]);
+      fence();
+      mfma16_a(dqacc[rb][db], kt, ds_frag(rb));
+      fence();
+      if (n < 2) load_t(6 + n);
+      if (n == 2 || n == 4) ds_elem(22 + n), ds_elem(23 + n);
+      if (n == 6) ds_hi(2);
+      if (n == 8 || n == 10) ds_elem(20 + n), ds_elem(21 + n);
+      if (n == 12) ds_hi(3);
+    }
+    // ---- phase 6
 #pragma unroll
-        for (int r = 8; r < 12; ++r) ds_elem(1, r);
+    for (int n = 0; n < 16; ++n) {
+      const int db = 7 - (n >> 1), rb = 2 + ((n ^ (n >> 1)) & 1);
+      const elemx8 kt = cat4(ct[db][0], ct[db][1]);
+      fence();
+      mfma16_a(dqacc[rb][db], kt, ds_frag(rb));
+      fence();
+      if (n % 4 == 0) request(n / 4);
+      if constexpr (!kLast) {
+        if (n < 8 && n % 2 == 1) fy[n / 2] = frag(so_next + 16 * kRow, n / 2);
+        const int e = n == 2 ? 0 : n == 6 ? 1 : n == 9 ? 2 : n == 10 ? 3 : n == 11 ? 4 : n >= 13 ? n - 8 : -1;
+        if (e >= 0) s0[e >> 2][e & 3] = p_of(s0[e >> 2][e & 3], e >> 2);
       }
-      if (n == 3) {
-#pragma unroll
-        for (int r = 12; r < 16; ++r) ds_elem(1, r);
-        ds_cvt(1, 1);
-      }
-      if (n + kLead < 8) {
-        const int n0 = n + kLead;
-        const elemx8 kt0 = cat4(ct[n0 % kFrags][0], ct[n0 % kFrags][1]);
-        fence();
-        dqacc[0][n0 & 3] = mfma32(kt0, dsf[0][n0 >> 2], dqacc[0][n0 & 3]);
-        fence();
-      }
-      if (n == 3) landed();
-      if (n == 4) first_k(so_next, 0);
-      if (n == 5) first_k(so_next, 1);
     }
   };
 
@@ -528,9 +608,8 @@ next_block:
   // whose rows end below those of the block's last wave, tiles that none of their rows sees.  Each kind has a loop
   // of its own with one body; every wave passes the same barriers and makes the same requests in all of them.
   int p = 0;
-  landed();
-  first_k(0, 0);
-  first_k(0, 1);
+  static_assert(kAhead == 3, "two tiles came in with the rows; stage (p + 3) % 4 is the one that tile p - 1 has left");
+  if (ntiles > 0) issue_tile(2, 2);
   auto none = [](int) {};
   const uint32_t dst_w = lds0 + 8 * wave * kRow;
   // four unmasked tiles per round, one per ring stage, as long as the fourth is still unmasked and the tiles requested meanwhile lie
@@ -539,14 +618,14 @@ next_block:
   int whole_end = wave_live ? (lim_first + 1) / kKeys : 0;  // the tiles that every row of the wave sees whole
   whole_end = uniform_int(whole_end < ntiles ? whole_end : ntiles);
   auto rounds = [&]() __attribute__((always_inline)) {
-    for (; p + 4 <= whole_end && (p + 6) * kKeys <= (SEG ? run_lim : lk); p += 4) {
+    for (; p + 4 <= whole_end && (p + 4 + kAhead) * kKeys <= (SEG ? run_lim : lk); p += 4) {
       auto four = [&](auto st) __attribute__((always_inline)) {
         constexpr int kSt = decltype(st)::value;
         using Next = std::integral_constant<int, (kSt + 1) % kStages>;
-        const int64_t at = (int64_t)(p + kSt + 2) * kKeys * kv_stride;
+        const int64_t at = (int64_t)(p + kSt + kAhead) * kKeys * kv_stride;
         const elem_t *kt = (SEG ? kvirt : kbase) + at, *vt = (SEG ? vvirt : vbase) + at;
-        const uint32_t dst = dst_w + ((kSt + 2) % kStages) * kStageBytes;
-        tile(st, Next{}, (p + kSt) * kKeys, std::false_type{}, [&](int i) __attribute__((always_inline)) {
+        const uint32_t dst = dst_w + ((kSt + kAhead) % kStages) * kStageBytes;
+        tile(st, Next{}, (p + kSt) * kKeys, std::false_type{}, std::false_type{}, [&](int i) __attribute__((always_inline)) {
           lds_direct_load16(i < 2 ? kt : vt, voff[i & 1], dst + (i >> 1) * kTile + (i & 1) * 4 * kRow);
         });
       };
@@ -564,17 +643,23 @@ next_block:
         if (p >= whole_end) break;
       }
     }
-    issue_tile((p + 2) % kStages, p + 2);
-    tile(p % kStages, (p + 1) % kStages, p * kKeys, std::false_type{}, none);
+    tile(p % kStages, (p + 1) % kStages, p * kKeys, std::false_type{}, std::false_type{}, none);
+    issue_tile((p + kAhead) % kStages, p + kAhead);
+  }
+  int seen_end = lim_last / kKeys + 1;  // the tiles that some row of the wave sees
+  seen_end = uniform_int(!wave_live || lim_last < 0 ? 0 : seen_end < ntiles ? seen_end : ntiles);
+  for (; p < seen_end - 1; ++p) {
+    tile(p % kStages, (p + 1) % kStages, p * kKeys, std::true_type{}, std::false_type{}, none);
+    issue_tile((p + kAhead) % kStages, p + kAhead);
+  }
+  if (p < seen_end) {
+    tile(p % kStages, (p + 1) % kStages, p * kKeys, std::true_type{}, std::true_type{}, none);
+    issue_tile((p + kAhead) % kStages, p + kAhead);
+    ++p;
   }
   for (; p < ntiles; ++p) {
-    if (!wave_live || p * kKeys > lim_last) break;
-    issue_tile((p + 2) % kStages, p + 2);
-    tile(p % kStages, (p + 1) % kStages, p * kKeys, std::true_type{}, none);
-  }
-  for (; p < ntiles; ++p) {
-    issue_tile((p + 2) % kStages, p + 2);
     landed();
+    issue_tile((p + kAhead) % kStages, p + kAhead);
   }
   wait_vm<0>();  // nothing may still be on its way into LDS when the workgroup ends
 
@@ -589,12 +674,12 @@ next_block:
 
   // ---- epilogue: the row statistics for the dK/dV kernel, which runs after this one (stored here rather than where
   // they are made: the wait that precedes the tile loop would have to see the stores through as well), and the dQ rows.
-  // A lane holds half of each of its two rows in pieces of 8 bytes (registers 4*cq..+3 of block db hold d0..d0+3):
-  // stored from there, an instruction touched 32 rows.  The pieces go to the wave's 16 KB behind the ring instead, in
+  // A lane holds a quarter of each of its four rows in pieces of 8 bytes (block db holds d = 16 db + 4 g4 .. +3):
+  // stored from there, an instruction touched 16 rows.  The pieces go to the wave's 16 KB behind the ring instead, in
   // the tiles' swizzled row layout, and leave from there four whole rows per instruction.
 #pragma unroll
-  for (int m = 0; m < 2; ++m) {
-    if (valid[m] && g == 0) {
+  for (int m = 0; m < 4; ++m) {
+    if (valid[m] && g4 == 0) {
       const int hg = row[m] - tok[m] * G;
       const int64_t so = (int64_t)(kvh * G + hg) * a.total_q + q0 + tok[m];
       a.lse2_w[so] = lse2[m];
@@ -602,33 +687,27 @@ next_block:
     }
   }
   if constexpr (SPLIT) {
-    // a piece's dQ as its accumulators lie, 16 bytes of a lane beside those of the next
+    // a piece's dQ where the kernel that adds up reads it (cut_blocks.h): d0 = 16 db + 4 g4 of row r of the wave at part r / 32,
+    // d block db % 4, quarter 2 (db / 4) + g4 / 2, lane 32 (g4 % 2) + r % 32
     const int slot = a.slot ? uniform_int(a.slot[2 * item]) : -1;
     if (slot >= 0) {
-      f32x4 *op = reinterpret_cast<f32x4 *>(a.partial + ((int64_t)slot * a.hkv + kvh) * kDqSlotBytes) + wave * 32 * 64 + lane;
+      f32x4 *op = reinterpret_cast<f32x4 *>(a.partial + ((int64_t)slot * a.hkv + kvh) * kDqSlotBytes) + wave * 32 * 64 + (g4 >> 1) * 64 + (g4 & 1) * 32 + c16;
 #pragma unroll
-      for (int m = 0; m < 2; ++m)
+      for (int m = 0; m < 4; ++m)
 #pragma unroll
-        for (int db = 0; db < 4; ++db)
-#pragma unroll
-          for (int cq = 0; cq < 4; ++cq)
-            op[(16 * m + 4 * db + cq) * 64] = f32x4{dqacc[m][db][4 * cq], dqacc[m][db][4 * cq + 1], dqacc[m][db][4 * cq + 2], dqacc[m][db][4 * cq + 3]};
+        for (int db = 0; db < 8; ++db) op[(16 * (m >> 1) + 4 * (db & 3) + 2 * (db >> 2)) * 64 + 16 * (m & 1)] = dqacc[m][db];
       return;
     }
   }
   {
     const uint32_t out_b = MERGE ? lds0 + wave * kStageBytes : stg;
 #pragma unroll
-    for (int m = 0; m < 2; ++m)
+    for (int m = 0; m < 4; ++m)
 #pragma unroll
-      for (int db = 0; db < 4; ++db)
-#pragma unroll
-        for (int cq = 0; cq < 4; ++cq) {
-          const int chunk = 2 * db + 8 * (cq >> 1) + (cq & 1);  // d0 / 8 with d0 = 16 db + 64 (cq >> 1) + 8 (cq & 1) + 4 g
-          *static_cast<DISTCA_LDS elemx4 *>(const_cast<DISTCA_LDS void *>(lds_ptr(out_b + (32 * m + l32) * kRow + ((chunk ^ tile_swz(l32)) << 4) + 8 * g))) =
-              cvt4(dqacc[m][db][4 * cq] * a.scale, dqacc[m][db][4 * cq + 1] * a.scale, dqacc[m][db][4 * cq + 2] * a.scale,
-                   dqacc[m][db][4 * cq + 3] * a.scale);
-        }
+      for (int db = 0; db < 8; ++db)
+        *static_cast<DISTCA_LDS elemx4 *>(const_cast<DISTCA_LDS void *>(
+            lds_ptr(out_b + (16 * m + c16) * kRow + (((2 * db + (g4 >> 1)) ^ tile_swz16(c16)) << 4) + 8 * (g4 & 1)))) =
+            cvt4(dqacc[m][db][0] * a.scale, dqacc[m][db][1] * a.scale, dqacc[m][db][2] * a.scale, dqacc[m][db][3] * a.scale);
     // (LDS operations of one wave complete in order: the reads below see the writes above)
     uint8_t *dq_blk = reinterpret_cast<uint8_t *>(a.dq) + dq_task + (int64_t)kvh * G * kHeadDim * 2;
 #pragma unroll
@@ -638,7 +717,7 @@ next_block:
       const elemx8 v = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(out_b + r * kRow + ((lane & 15) << 4)));
       if (rg < nrows) {
         const int t = div_group(rg);
-        *reinterpret_cast<elemx8 *>(dq_blk + (int64_t)t * a.dq_tok_bytes + (rg - t * G) * (kHeadDim * 2) + (((lane & 15) ^ tile_swz(r)) << 4)) = v;
+        *reinterpret_cast<elemx8 *>(dq_blk + (int64_t)t * a.dq_tok_bytes + (rg - t * G) * (kHeadDim * 2) + (((lane & 15) ^ tile_swz16(r)) << 4)) = v;
       }
     }
   }

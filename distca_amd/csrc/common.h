@@ -11,10 +11,12 @@ namespace distca {
 typedef _Float16 elem_t;
 #define DISTCA_FN(name) name##_f16
 #define DISTCA_MFMA32_ASM "v_mfma_f32_32x32x16_f16"
+#define DISTCA_MFMA16_ASM "v_mfma_f32_16x16x32_f16"
 #else
 typedef __bf16 elem_t;
 #define DISTCA_FN(name) name
 #define DISTCA_MFMA32_ASM "v_mfma_f32_32x32x16_bf16"
+#define DISTCA_MFMA16_ASM "v_mfma_f32_16x16x32_bf16"
 #endif
 typedef elem_t elemx8 __attribute__((ext_vector_type(8)));
 typedef elem_t elemx4 __attribute__((ext_vector_type(4)));
@@ -39,6 +41,18 @@ __device__ __forceinline__ f32x16 mfma32(elemx8 a, elemx8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 #else
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+#endif
+}
+
+// D = A(16x32) * B(32x16) + C on one wave64.
+//   A operand: lane l holds row l%16, k = 8*(l/16) .. +7
+//   B operand: lane l holds col l%16, k = 8*(l/16) .. +7
+//   C/D:       lane l holds col l%16, register r holds row 4*(l/16) + r
+__device__ __forceinline__ f32x4 mfma16(elemx8 a, elemx8 b, f32x4 c) {
+#ifdef DISTCA_F16
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+#else
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 #endif
 }
 
@@ -73,6 +87,8 @@ __device__ __forceinline__ elemx4 cvt4(float a0, float a1, float a2, float a3) {
 // max / sum of x over the lane pair (l, l^32).
 __device__ __forceinline__ float pair_max(float x) { return __builtin_fmaxf(x, __shfl_xor(x, 32, 64)); }
 __device__ __forceinline__ float pair_sum(float x) { return x + __shfl_xor(x, 32, 64); }
+// sum of x over the four lanes l % 16 + 16 i.
+__device__ __forceinline__ float quad_sum(float x) { return pair_sum(x + __shfl_xor(x, 16, 64)); }
 
 // LDS-direct global loads.  One piece per active lane goes from global memory straight into
 // LDS at lds_base + piece_bytes * lane, with no staging registers.  The compiler is not told
@@ -127,6 +143,9 @@ __device__ __forceinline__ void wait_vm0() { asm volatile("s_waitcnt vmcnt(0)" :
 // and the transposing 64-bit reads over 4-row x 32-byte patches), and a row keeps its 256
 // contiguous bytes, so LDS-direct loads can fill four rows per instruction.
 __device__ __forceinline__ int tile_swz(int r) { return ((r & 3) << 1) | ((r & 4) << 1) | ((r >> 3) & 1); }
+// The same for the 16x16x32 MFMAs' operand reads, 16 rows by four chunks: a 128-bit read takes lanes 0 .. 3, 12 .. 15 and 20 .. 27 at a time, 4 .. 11,
+// 16 .. 19 and 28 .. 31 at the next (and so on from 32), so that rows 4 .. 11 of one chunk meet the other rows of the chunk beside it.
+__device__ __forceinline__ int tile_swz16(int r) { return ((r & 3) << 1) | ((r & 4) << 1) | ((r >> 2) & 1); }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
