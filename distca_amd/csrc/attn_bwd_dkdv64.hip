@@ -1,10 +1,10 @@
 // dK / dV of the varlen causal attention backward for gfx950, 64 keys per wave.
 //
 // One workgroup of 4 waves per (task, block of 256 keys, kv head), one wave per SIMD, so that a wave may use the
-// SIMD's whole register file: the dK^T / dV^T accumulators of its 64 keys (2 key blocks x 4 blocks over d x 2
-// matrices x 16 registers) fill the 256 accumulation registers, K of its keys stays in 64 vector registers as MFMA
-// B operand, V of the workgroup's keys in LDS (and, as far as registers allow, in registers too: kVRegSlices*).  The query side (Q, dO and the row statistics of every head of the
-// kv group, flattened into rows) streams through LDS in blocks of 32 rows, by LDS-direct loads into a ring of
+// SIMD's whole register file: the dK^T / dV^T accumulators of its 64 keys (4 sub-blocks of 16 keys x 8 blocks over d x 2
+// matrices x 4 registers) fill the 256 accumulation registers, K of its keys stays in 64 vector registers as MFMA
+// B operand, V of the workgroup's keys in LDS and three quarters of it (kVRegSlices) in registers too.  The query side (Q, dO and
+// the row statistics of every head of the kv group, flattened into rows) streams through LDS in blocks of 32 rows, by LDS-direct loads into a ring of
 // four stages, from the last block down to the first one the causal mask lets see these keys, or from that one up.
 //
 // With one wave per SIMD nothing else can use the SIMD's vector ALU while the wave waits for the matrix pipe, and
@@ -12,13 +12,19 @@
 // block (P = exp2(S c - lse2), dS = P (dP - delta), conversions to bf16) is written between the MFMAs of the same
 // block, a few instructions behind each one, where it runs while the pipe works:
 //
-//   step 1   S  = Q K^T        16 MFMAs   A: rows of the Q tile (LDS), B: K registers
-//   step 2   dP = dO V^T       16 MFMAs   A: rows of the dO tile, B: V (LDS)        beside them: P from S
-//   step 3   dV^T += dO^T P    16 MFMAs   A: transposing reads of the dO tile, B: P  beside them: dS from P, dP
-//   step 4   dK^T += Q^T dS    16 MFMAs   A: transposing reads of the Q tile, B: dS
+//   S  = Q K^T       32 MFMAs   A: rows of the Q tile (LDS), B: K registers
+//   dP = dO V^T      32 MFMAs   A: rows of the dO tile, B: V (registers, LDS)            beside them: P from S
+//   dV^T += dO^T P   32 MFMAs   A: transposing reads of the dO tile, B: P                beside them: dS from P, dP
+//   dK^T += Q^T dS   32 MFMAs   A: transposing reads of the Q tile, B: dS
 //
-// Every LDS fragment a wave reads feeds two MFMAs (one per key block of the wave): half the LDS traffic per MFMA of
+// Every LDS fragment a wave reads feeds four MFMAs (one per sub-block of the wave): half the LDS traffic per FLOP of
 // a 32-key wave: with eight waves of 32 keys, two per SIMD, the LDS reads bounded the kernel.
+//
+// 16x16x32 MFMAs rather than 32x32x16, for the dQ kernel's reason (attn_bwd_dq64.hip): bound by power, and a FLOP of theirs moves half the
+// accumulator bytes.  What they leave beside them, two issue slots each, is all used (294 other instructions beside a block's 128), so every address
+// is one exclusive or on a base per block, and the diagonal's compares cover the half of the keys that it can touch.  The kernel, before -> after, on
+// two boxes: 131072 packed tokens at 32/8 heads 22 870 us -> 21 690 and 23 250 -> 22 360, a tick of 16384 tokens 2 560 -> 2 375 and 2 575 -> 2 499;
+// documents of 128 to 2048 tokens 1 466 -> 1 424, of 1024 (65536 tokens) 1 139 -> 1 114, of 256 527 -> 513; 389 tokens at 4/1 heads 28.5 -> 28.9.
 #include "api_util.h"
 #include "attn_bwd.h"
 #include "attn_cfg.h"
@@ -34,26 +40,18 @@ constexpr int kThreads = 256;
 constexpr int kBN = kBwdKV;    // keys per workgroup
 constexpr int kBM = kBwdRows;  // flattened query rows per block
 static_assert(kBN == 256 && kBM == 32, "tile geometry of this kernel");
-constexpr int kRow = 256;      // bytes per tile row, chunks swizzled by tile_swz
+constexpr int kRow = 256;      // bytes per tile row, chunks swizzled by tile_swz16
 constexpr int kStages = 4;
 constexpr int kTileQ = 0, kTileDO = kBM * kRow;
 constexpr int kTileBytes = 2 * kBM * kRow;
 constexpr int kStatBytes = 3 * kBM * 4;  // lse2, -delta, lim per row
 constexpr int kStatOff = kStages * kTileBytes;
-constexpr int kVPitch = 272;             // resident V rows (padded: 128-bit row reads without bank conflicts)
 constexpr int kVOff = kStatOff + kStages * kStatBytes;
-// Of the eight 16-element slices over d of a wave's V rows, the first kVRegSlices* stay in registers as B operands
-// beside K (as many as fit without spills inside the block loops: 12 fewer of a block's 72 LDS reads, -2 %); the
-// rest is read from LDS every block.
-#ifndef DISTCA_VREG_OWN
-#define DISTCA_VREG_OWN 6
-#endif
-constexpr int kVRegSlicesOwn = DISTCA_VREG_OWN;  // the (task, key block) form
-#ifndef DISTCA_VREG_SHARED
-#define DISTCA_VREG_SHARED 4
-#endif
-constexpr int kVRegSlicesShared = DISTCA_VREG_SHARED;  // the form with a loop over a group's tasks, which has more values to hold
-constexpr int kLds = kVOff + kBN * kVPitch;
+constexpr int kVWave = 64 * kRow + 64 * 16;  // a wave's resident V rows, in the tiles' layout, and (shards) where its rows go
+// Of the four 32-element slices over d of a wave's V rows, as many as fit without spills inside the block loops stay in registers as
+// B operands beside K; the rest is read from LDS every block.
+constexpr int kVRegSlices = 3;
+constexpr int kLds = kVOff + 4 * kVWave;
 static_assert(kLds <= 160 * 1024, "LDS budget");
 #ifndef DISTCA_RAWBAR
 #define DISTCA_RAWBAR 1
@@ -77,29 +75,29 @@ __device__ __forceinline__ int lane_now() {
 // and which fill that file exactly.  The S and dP accumulators, which the vector ALU reads and overwrites, must
 // live in the ordinary vector registers instead, and the only way to say so per instruction is to write those
 // MFMAs as assembly with vector-register operands.  The compiler does not know what such a statement executes and
-// so does not space its result from the vector instructions that read it (an eight-pass MFMA: 11 quad-cycles from
-// its issue): the order of a block's instructions below, held in place by the scheduling fences, keeps between every
-// such MFMA and the first read of its result either two later MFMAs, or one later MFMA (which cannot start before
-// the pipe has finished the eight passes of the one in question) and at least four vector instructions.  Nowhere is
-// a single MFMA the only separation; a change to the block body has to keep that.
-__device__ __forceinline__ void mfma32_v(f32x16 &acc, elemx8 a, elemx8 b) {
-  asm volatile(DISTCA_MFMA32_ASM " %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+// so does not space its result from the vector instructions that read it (a four-pass MFMA: 8 wait states): the order of a block's
+// instructions below, held in place by the scheduling fences, keeps at least three later MFMAs, each of which waits for the four passes
+// of the one before it, between every such MFMA and the first read of its result, and spaced() does where a block's second half of keys
+// is left out; a change to the block body has to keep that.
+__device__ __forceinline__ void mfma16_v(f32x4 &acc, elemx8 a, elemx8 b) {
+  asm volatile(DISTCA_MFMA16_ASM " %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
 }
-__device__ __forceinline__ void mfma32_v0(f32x16 &acc, elemx8 a, elemx8 b) {  // acc = A B
-  asm volatile(DISTCA_MFMA32_ASM " %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b));
+__device__ __forceinline__ void mfma16_v0(f32x4 &acc, elemx8 a, elemx8 b) {  // acc = A B
+  asm volatile(DISTCA_MFMA16_ASM " %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b));
 }
-__device__ __forceinline__ void mfma32_vc(f32x16 &acc, elemx8 a, elemx8 b, const f32x16 &c0) {  // acc = A B + c0
-  asm volatile(DISTCA_MFMA32_ASM " %0, %1, %2, %3" : "=&v"(acc) : "v"(a), "v"(b), "v"(c0));
+__device__ __forceinline__ void mfma16_vc(f32x4 &acc, elemx8 a, elemx8 b, const f32x4 &c0) {  // acc = A B + c0
+  asm volatile(DISTCA_MFMA16_ASM " %0, %1, %2, %3" : "=&v"(acc) : "v"(a), "v"(b), "v"(c0));
 }
 
 // First key, in the workgroup's block of 256, of a wave's first or second half of 32: the halves from the block's start go to waves
-// 0, 1, 2, 3, 3, 2, 1, 0.  Every wave passes the same barrier per query block, so a block on the diagonal takes as long as the wave that
+// 0, 1, 2, 3, 0, 1, 2, 3.  Every wave passes the same barrier per query block, so a block on the diagonal takes as long as the wave that
 // sees most of it: with 64 keys in a row wave 0 has a whole block's work as soon as the first key is seen.  Dealt this way no wave has more
 // than half a block's until the rows see 128 keys, nor ever where a task ends in a block of at most 128 keys.
 // The kernel over 131072 tokens in documents of 64 / 128 / 256 / 512 / 2048, 32/8 heads, in us: 64 keys in a row 1526 / 1225 / 1168 /
 // 1599 / 4426, in halves 1326 / 1115 / 1092 / 1536 / 4321 (a visit of half the work still takes 1.7 us of 2.0: requests, barrier and
-// the chain from S to dK do not shrink with it).
-__device__ __forceinline__ int dkdv_half_key(int wave, int half) { return half ? kBN - 32 - 32 * wave : 32 * wave; }
+// the chain from S to dK do not shrink with it).  (With the second halves in the order 3, 2, 1, 0 instead, wave 3's two lay side by side, and
+// both could lie on the diagonal at once; now only one ever does, and only its elements are compared.)
+__device__ __forceinline__ int dkdv_half_key(int wave, int half) { return kBN / 2 * half + 32 * wave; }
 
 #define DKDV_SHARED 0
 #define DKDV_SEG 0
