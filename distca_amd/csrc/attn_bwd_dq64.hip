@@ -335,7 +335,8 @@ next_block:
   f32x4 s0[4], s1[4];        // S, then P, of keys 0 .. 15 and 16 .. 31
   elemx8 fx[4], fy[4];       // K and V fragments of this phase and the next
   auto frag = [&](uint32_t so, int s) { return *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(k_ad[s] + so)); };
-  auto p_of = [&](float x, int rb) __attribute__((always_inline)) { return fast_exp2(__builtin_fmaf(x, c, -lse2[rb])); };
+  auto x_of = [&](float x, int rb) __attribute__((always_inline)) { return __builtin_fmaf(x, c, -lse2[rb]); };
+  auto p_of = [&](float x, int rb) __attribute__((always_inline)) { return fast_exp2(x_of(x, rb)); };
   {
     const uint32_t frag_at = c16 * kRow + ((g4 ^ tile_swz16(c16)) << 4);  // this lane's chunk 0 of row c16; ^ (s << 6)
 #pragma unroll
@@ -434,15 +435,22 @@ next_block:
   //   6  dQ, sub-blocks 2 and 3               P of the next tile, keys 0 .. 15, sub-blocks 0 and 1; its K fragments; request(0 .. 3), the loads
   //                                           of the tile kAhead tiles on, whose stage every wave left before the barrier of phase 2
   // MASKED: the tile straddles the diagonal or the end of the prefix, compare and select per element.
-  auto landed = [&]() {
-    // tile p has landed when at most the loads of tile p + 1 are still on their way
-    wait_vm<kLoadsPerTile>();
+  // Requests are made for tiles below ntiles only (and, in the rounds below, for what lies behind them in the prefix): one past the end, even from
+  // the zero row, was waited for in the open before the block's results could leave.  Documents of 256 tokens (65536) 694 us -> 676,
+  // of 128 to 2048 1 239 -> 1 220, of 1024 1 033 -> 1 017.
+  auto landed = [&](auto two_on) __attribute__((always_inline)) {  // two_on: the tile after the next, or a constant where it is known to be requested
+    // the next tile has landed when at most the loads of the one after it are still on their way
+    if constexpr (std::is_same_v<decltype(two_on), int>)
+      // (the branch is out of the compiler's sight: as one of its own it would end a block of code between the MFMAs)
+      asm volatile("s_cmp_lt_i32 %0, %1\n\ts_cbranch_scc1 .Lrequested%=\n\ts_waitcnt vmcnt(0)\n.Lrequested%=:\n\ts_waitcnt vmcnt(%2)" ::"s"(two_on), "s"(uniform_int(ntiles)), "n"(kLoadsPerTile) : "memory", "scc");
+    else
+      wait_vm<kLoadsPerTile>();
     fence();
     asm volatile("s_barrier" ::: "memory");
     fence();
   };
   // LAST: there is no next tile for this wave, nothing of it is made.
-  auto tile = [&](auto stage, auto next_stage, int key0, auto masked, auto last, auto request) __attribute__((always_inline)) {  // stages: ints or constants
+  auto tile = [&](auto stage, auto next_stage, int key0, auto two_on, auto masked, auto last, auto request) __attribute__((always_inline)) {  // stages: ints or constants
     constexpr bool kMasked = decltype(masked)::value, kLast = decltype(last)::value;
     const uint32_t so = (uint32_t)stage * kStageBytes, so_next = (uint32_t)next_stage * kStageBytes;
     f32x4 d0[4], d1[4];  // dP, then dS
@@ -460,15 +468,17 @@ next_block:
       hidden[e & 3] = __builtin_amdgcn_ballot_w64(16 * (e >> 4) + (e & 3) > last_key[(e >> 2) & 3]);
       asm volatile("" : "+s"(hidden[e & 3]));  // here, not where it is used
     };
-    auto hide = [&](float x, int e) __attribute__((always_inline)) {
-      if (__builtin_amdgcn_inverse_ballot_w64(hidden[e & 3])) x = 0.f;
+    // (ahead of the exponential where there is a choice: what follows that one at once has to wait for it)
+    auto hide = [&](float x, int e, float hidden_x) __attribute__((always_inline)) {
+      if (__builtin_amdgcn_inverse_ballot_w64(hidden[e & 3])) x = hidden_x;
       find_hidden(e + 2);
       return x;
     };
     auto p_elem = [&](int e) __attribute__((always_inline)) {
       const int rb = (e >> 2) & 3, r = e & 3;
-      float x = p_of(e < 16 ? s0[rb][r] : s1[rb][r], rb);
-      if constexpr (kMasked) x = hide(x, e);
+      float x = x_of(e < 16 ? s0[rb][r] : s1[rb][r], rb);
+      if constexpr (kMasked) x = hide(x, e, -INFINITY);
+      x = fast_exp2(x);
       if (e < 16) s0[rb][r] = x;
       else s1[rb][r] = x;
     };
@@ -515,8 +525,8 @@ next_block:
       else mfma16_va(s1[rb], fy[s], qf[rb][s]);
       fence();
       if (kMasked && n < 4) {  // what was made before the tile was known to be masked
-        s0[n >> 1][2 * (n & 1)] = hide(s0[n >> 1][2 * (n & 1)], 2 * n);
-        s0[n >> 1][2 * (n & 1) + 1] = hide(s0[n >> 1][2 * (n & 1) + 1], 2 * n + 1);
+        s0[n >> 1][2 * (n & 1)] = hide(s0[n >> 1][2 * (n & 1)], 2 * n, 0.f);
+        s0[n >> 1][2 * (n & 1) + 1] = hide(s0[n >> 1][2 * (n & 1) + 1], 2 * n + 1, 0.f);
       }
       if (n < 8 && n % 2 == 0) fx[n / 2] = frag(so + kTile, n / 2);
       if (n > 4 && n < 11 && n % 2 == 1) p_elem(8 + (n - 5) / 2);
@@ -534,7 +544,7 @@ next_block:
       if (n < 8 && n % 2 == 1) p_elem(16 + n / 2);
       if (n >= 8) p_elem(12 + n);
     }
-    landed();
+    landed(two_on);
     // ---- phase 3
     wait_lds();
 #pragma unroll
@@ -609,8 +619,11 @@ next_block:
   // of its own with one body; every wave passes the same barriers and makes the same requests in all of them.
   int p = 0;
   static_assert(kAhead == 3, "two tiles came in with the rows; stage (p + 3) % 4 is the one that tile p - 1 has left");
-  if (ntiles > 0) issue_tile(2, 2);
+  if (ntiles > 2) issue_tile(2, 2);
   auto none = [](int) {};
+  auto issue_ahead = [&](int j) __attribute__((always_inline)) {
+    if (j < ntiles) issue_tile(j % kStages, j);
+  };
   const uint32_t dst_w = lds0 + 8 * wave * kRow;
   // four unmasked tiles per round, one per ring stage, as long as the fourth is still unmasked and the tiles requested meanwhile lie
   // wholly inside the prefix (SEG: and in the present shard; the loop of single tiles comes back to this one behind every shard's end: tick of
@@ -625,7 +638,7 @@ next_block:
         const int64_t at = (int64_t)(p + kSt + kAhead) * kKeys * kv_stride;
         const elem_t *kt = (SEG ? kvirt : kbase) + at, *vt = (SEG ? vvirt : vbase) + at;
         const uint32_t dst = dst_w + ((kSt + kAhead) % kStages) * kStageBytes;
-        tile(st, Next{}, (p + kSt) * kKeys, std::false_type{}, std::false_type{}, [&](int i) __attribute__((always_inline)) {
+        tile(st, Next{}, (p + kSt) * kKeys, std::true_type{}, std::false_type{}, std::false_type{}, [&](int i) __attribute__((always_inline)) {
           lds_direct_load16(i < 2 ? kt : vt, voff[i & 1], dst + (i >> 1) * kTile + (i & 1) * 4 * kRow);
         });
       };
@@ -643,23 +656,23 @@ next_block:
         if (p >= whole_end) break;
       }
     }
-    tile(p % kStages, (p + 1) % kStages, p * kKeys, std::false_type{}, std::false_type{}, none);
-    issue_tile((p + kAhead) % kStages, p + kAhead);
+    tile(p % kStages, (p + 1) % kStages, p * kKeys, p + 2, std::false_type{}, std::false_type{}, none);
+    issue_ahead(p + kAhead);
   }
   int seen_end = lim_last / kKeys + 1;  // the tiles that some row of the wave sees
   seen_end = uniform_int(!wave_live || lim_last < 0 ? 0 : seen_end < ntiles ? seen_end : ntiles);
   for (; p < seen_end - 1; ++p) {
-    tile(p % kStages, (p + 1) % kStages, p * kKeys, std::true_type{}, std::false_type{}, none);
-    issue_tile((p + kAhead) % kStages, p + kAhead);
+    tile(p % kStages, (p + 1) % kStages, p * kKeys, p + 2, std::true_type{}, std::false_type{}, none);
+    issue_ahead(p + kAhead);
   }
   if (p < seen_end) {
-    tile(p % kStages, (p + 1) % kStages, p * kKeys, std::true_type{}, std::true_type{}, none);
-    issue_tile((p + kAhead) % kStages, p + kAhead);
+    tile(p % kStages, (p + 1) % kStages, p * kKeys, p + 2, std::true_type{}, std::true_type{}, none);
+    issue_ahead(p + kAhead);
     ++p;
   }
   for (; p < ntiles; ++p) {
-    landed();
-    issue_tile((p + kAhead) % kStages, p + kAhead);
+    landed(p + 2);
+    issue_ahead(p + kAhead);
   }
   wait_vm<0>();  // nothing may still be on its way into LDS when the workgroup ends
 
