@@ -21,10 +21,13 @@
 // a 32-key wave: with eight waves of 32 keys, two per SIMD, the LDS reads bounded the kernel.
 //
 // 16x16x32 MFMAs rather than 32x32x16, for the dQ kernel's reason (attn_bwd_dq64.hip): bound by power, and a FLOP of theirs moves half the
-// accumulator bytes.  What they leave beside them, two issue slots each, is all used (294 other instructions beside a block's 128), so every address
-// is one exclusive or on a base per block, and the diagonal's compares cover the half of the keys that it can touch.  The kernel, before -> after, on
-// two boxes: 131072 packed tokens at 32/8 heads 22 870 us -> 21 690 and 23 250 -> 22 360, a tick of 16384 tokens 2 560 -> 2 375 and 2 575 -> 2 499;
-// documents of 128 to 2048 tokens 1 466 -> 1 424, of 1024 (65536 tokens) 1 139 -> 1 114, of 256 527 -> 513; 389 tokens at 4/1 heads 28.5 -> 28.9.
+// accumulator bytes.  What they leave beside them, two issue slots each, is all used (240 other instructions beside a block's 128): on the way from
+// one end of a document to the other four blocks, one per stage of the ring, make a round whose stages are constants in the reads' offsets, one wait
+// does for the reads of eight MFMAs, and the diagonal's compares cover the half of the keys that it can touch.  The kernel, us, with 32x32x16 MFMAs ->
+// with 16x16x32 -> with rounds and few waits (two boxes): 131072 packed tokens at 32/8 heads 23 250 -> 22 450 -> 21 020, a tick of 16384 tokens 2 575 ->
+// 2 443 -> 2 328; documents of 128 to 2048 tokens 1 466 -> 1 429 -> 1 348, of 1024 (65536 tokens) 1 139 -> 1 098 -> 1 053, of 256 527 -> 506 -> 504;
+// 389 tokens at 4/1 heads 28.5 -> 29.1 -> 28.9.  (With three lane-derived registers parked in scratch memory, reloaded ahead of each loop, where the
+// reload waits for every request in flight: documents of 256 tokens 554, 389 tokens 30.8.)
 #include "api_util.h"
 #include "attn_bwd.h"
 #include "attn_cfg.h"
