@@ -554,6 +554,8 @@ next_block:
       dp_mfma(d1[rb], fy[s], rb, s);
       fence();
       if (!kLast && n < 8 && n % 2 == 0) fx[n / 2] = frag(so_next, n / 2);
+      // (-delta is kept until here: dead behind a row's last tile, its registers were written over while the MFMA read them as its C operand)
+      if (n == 7) asm volatile("" ::"v"(ndl[0]), "v"(ndl[1]), "v"(ndl[2]), "v"(ndl[3]));
       if (n < 8 && n % 2 == 1) p_elem(28 + n / 2);
       if (n >= 8) ds_elem(2 * n - 16), ds_elem(2 * n - 15);
     }

@@ -95,6 +95,29 @@ def violations(lines):
     return out
 
 
+def overwritten(lines):
+    """(wait states between, matrix instruction, instruction): a vector instruction that writes the vector registers of a matrix instruction's C operand
+    while it may still read them, within 3 wait states of one of four passes (16x16x32) or 7 of one of eight (32x32x16).  Such an instruction takes its
+    passes before the next one of its kind can start."""
+    out = []
+    for i, line in enumerate(lines):
+        if not line.startswith("v_mfma"):
+            continue
+        ops = operands(line)
+        c = {r for r in registers(ops[3]) - registers(ops[0]) if str(r).startswith("v")}
+        needed, waits = (7 if "32x32" in line else 3), 0
+        for after in lines[i + 1:i + 1 + needed] if c else []:
+            op, after_ops = after.split()[0], operands(after)
+            if op.startswith("v_") and not op.startswith("v_mfma") and union(results(op, after_ops)) & c:
+                out.append((waits, line, after))
+            if op in ("s_branch", "s_endpgm", "s_setpc_b64"):
+                break
+            waits += int(after_ops[0], 0) + 1 if op == "s_nop" else (8 if "32x32" in op else 4) if op.startswith("v_mfma") else 1
+            if waits >= needed:
+                break
+    return out
+
+
 def test_hazards_planted_in_a_listing_are_found():
     load = "global_load_lds_dwordx4 v1, s[0:1] offset:2048"
     assert violations(["v_readlane_b32 s1, v252, 18", load])
@@ -119,6 +142,12 @@ def test_hazards_planted_in_a_listing_are_found():
     assert not violations(["v_cvt_pk_bf16_f32 v19, v40, v41", "s_nop 1", product])
     assert not violations(["v_mov_b32_e32 v24, v40", product]) and not violations(["ds_read_b128 v[16:19], v60", product])
 
+    start = "v_mfma_f32_16x16x32_bf16 v[78:81], v[104:107], a[32:35], v[10:13]"
+    assert overwritten([start, "v_fma_f32 v11, v74, v128, -v189"]) and overwritten([start, "s_nop 1", "v_mov_b32_e32 v13, v1"])
+    assert not overwritten([start, "s_nop 2", "v_mov_b32_e32 v13, v1"]) and not overwritten([start, "v_mov_b32_e32 v80, v10"])
+    assert not overwritten([start, "v_mfma_f32_16x16x32_bf16 v[82:85], v[104:107], a[36:39], v[14:17]", "v_mov_b32_e32 v13, v1"])
+    assert overwritten([start.replace("16x16x32", "32x32x16"), "s_nop 5", "v_mov_b32_e32 v13, v1"])
+
 
 @pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="needs llvm-objdump")
 def test_wait_states_of_the_built_kernels(tmp_path):
@@ -132,7 +161,7 @@ def test_wait_states_of_the_built_kernels(tmp_path):
         for raw in text.splitlines() + ["<end>:"]:
             m = re.match(r"(?:[0-9a-f]+ )?<(\S+)>:$", raw.strip())
             if m:
-                found += [(kernel,) + v for v in violations(lines)]
+                found += [(kernel,) + v for v in violations(lines) + overwritten(lines)]
                 loads += sum("global_load_lds" in l for l in lines)
                 products += sum(l.startswith("v_mfma") for l in lines)
                 kernel, lines = m[1], []
