@@ -110,6 +110,15 @@ def test_runs_of_whole_tiles_in_merged_blocks_non_causal(cuda):
     _run(lens, lens, 32, 8, 25, cuda, causal=False)
 
 
+@pytest.mark.parametrize("causal,prefix", [(True, 0), (True, 37), (False, 0)])
+def test_rounds_of_one_block_per_ring_stage(cuda, causal, prefix):
+    """Runs of whole blocks (dK/dV) and whole tiles (dQ) that begin and end at every stage of the ring of four: at four heads per kv head a
+    block of query rows is 8 tokens, so lengths 8 apart (and off by up to 7, with ends of tiles between) leave each remainder, from the first stage on
+    and, in dK/dV items that walk upwards, from wherever the diagonal ends; more key blocks than compute units serve a kv head, for both directions."""
+    q_lens = [600 + 8 * i + (5 * i) % 8 for i in range(16)]
+    _run(q_lens, [n + prefix for n in q_lens], 32, 8, 27, cuda, causal=causal)
+
+
 @pytest.mark.parametrize("hq,hkv,lens", [(4, 1, [1020]), (4, 1, [1030]), (4, 1, [1540]), (4, 1, [1600]), (32, 8, [2048]), (64, 16, [2050]), (16, 4, [1800, 250])])
 def test_either_side_of_the_lines_from_which_blocks_are_cut(cuda, hq, hkv, lens):
     """Tiles that cutting could take off the longest block, where dQ's line is 16 and the forward's 24: 15.5, 16.5, 23.8, 24.7, 16.5 (half of a longer
