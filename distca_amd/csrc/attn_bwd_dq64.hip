@@ -16,7 +16,7 @@
 // 1 765 TFLOP/s with the latter and 2 044 with the former, with half a KB of LDS reads and 2.3 vector instructions per
 // 32 K FLOP beside them 1 520 and 1 630 to 1 710.  They leave 2 issue slots each for anything else (the larger ones 5), so the side work
 // is spread over the whole tile.  The kernel, before -> after: 131072 packed tokens at 32/8 heads 16 870 us -> 15 510
-// (1.66 -> 1.9 GHz at 78 % of the pipe's cycles), a tick of 16384 tokens 1 837 -> 1 711, documents of 128 to 2048 tokens 1 268 -> 1 251.
+// (1.66 -> 1.81 GHz at 79 % of the pipe's cycles), a tick of 16384 tokens 1 837 -> 1 711, documents of 128 to 2048 tokens 1 268 -> 1 251.
 //
 // The prologue also makes the row statistics of the backward (delta = <dO, O>, lse in the log2 domain) and leaves
 // them in the workspace for the dK/dV kernel, which runs after this one.
