@@ -10,12 +10,10 @@ namespace distca {
 #ifdef DISTCA_F16
 typedef _Float16 elem_t;
 #define DISTCA_FN(name) name##_f16
-#define DISTCA_MFMA32_ASM "v_mfma_f32_32x32x16_f16"
 #define DISTCA_MFMA16_ASM "v_mfma_f32_16x16x32_f16"
 #else
 typedef __bf16 elem_t;
 #define DISTCA_FN(name) name
-#define DISTCA_MFMA32_ASM "v_mfma_f32_32x32x16_bf16"
 #define DISTCA_MFMA16_ASM "v_mfma_f32_16x16x32_bf16"
 #endif
 typedef elem_t elemx8 __attribute__((ext_vector_type(8)));
