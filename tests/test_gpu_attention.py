@@ -399,6 +399,47 @@ def test_scores_that_drift_along_the_keys(cuda, span):
     assert_close_bf16(dv, ref_dv, "dv")
 
 
+@pytest.mark.parametrize("case", ["one block", "two blocks", "group of 3", "many blocks", "shared", "non-causal"])
+@pytest.mark.parametrize("dtype,level", [(torch.float16, -24.0), (torch.bfloat16, -120.0)])
+def test_missing_rows_of_a_task_whose_scores_are_far_below_zero(cuda, dtype, level, case):
+    """The last block of 32 query rows of a task that is no multiple of it: where every key is seen the dK/dV kernel compares nothing, so that its
+    missing rows have to add nothing by themselves.  With the statistics of the task's last row their P was exp(-lse): infinite in the element type
+    below lse = -11.1 (fp16) and -88.7 (bf16), and 0 * inf put NaN into dV and dK of every key seen.  Scores are shifted by `level`: dimension 0 of q
+    and k holds constants whose product it is.  Gradients of those constants are left out of the comparison (dS rounded to the element type times a
+    constant of tens, in sums whose exact value is near zero), but not of the check for NaN."""
+    from distca_amd.fused_comm_attn import ca_varlen_bwd, ca_varlen_fwd
+    hq, hkv, offs = 32, 8, None
+    k_lens = {"one block": [150], "two blocks": [300, 129, 159], "group of 3": [139, 270], "many blocks": [289, 300, 383, 141, 258] * 16, "shared": [150, 281, 300],
+              "non-causal": [150, 301]}[case]
+    q_lens = [70, 90, 19] if case == "shared" else k_lens
+    if case == "group of 3":
+        hq, hkv = 12, 4
+    if case == "many blocks":   # enough for the kernel of batches that are not cut
+        hq, hkv = 32, 16
+    causal = case != "non-causal"
+    if case == "shared":
+        offs = [0, 0, 0]
+    cu_q, cu_k = cu(q_lens), cu(k_lens)
+    tk = max(k_lens) if offs else int(cu_k[-1])
+    q, k, v, do = (t.to(dtype) for t in make_qkv(int(cu_q[-1]), tk, hq, hkv, 128, 28))
+    a = 16.0 if dtype == torch.float16 else 32.0
+    q[:, :, 0], k[:, :, 0] = a, round(level * 128 ** 0.5 / a * 4) / 4   # (exact in both types)
+    c = (torch.tensor(cu_q, device=cuda), torch.tensor(cu_k, device=cuda), max(q_lens), max(k_lens))
+    dkv = torch.tensor(offs, dtype=torch.int32, device=cuda) if offs else None
+    qd, kd, vd, dod = (t.to(cuda) for t in (q, k, v, do))
+    print(f"case {case} {dtype} level={level}", flush=True)
+    out, lse = ca_varlen_fwd(qd, kd, vd, *c, None, causal, dkv)
+    torch.cuda.synchronize()
+    assert lse.max().item() < (-11.2 if dtype == torch.float16 else -88.8)
+    got = ca_varlen_bwd(dod, qd, kd, vd, out, lse, *c, None, causal, False, dkv)
+    torch.cuda.synchronize()
+    ref = ca_reference_bwd(do, q, k, v, cu_q, cu_k, causal=causal, kv_task_offsets=offs, out=out.cpu(), softmax_lse=lse.cpu())
+    for name, x, r in zip(("dq", "dk", "dv"), got, ref):
+        bad = int((~torch.isfinite(x.float())).sum())
+        assert bad == 0, f"{name}: {bad} values are not finite"
+        assert_close_bf16(x if name == "dv" else x[..., 1:], r if name == "dv" else r[..., 1:], name)
+
+
 @pytest.mark.parametrize("seed", range(12))
 def test_random_task_batches(cuda, seed):
     """Seeded random batches of CA tasks: lengths around the tile edges (32, 64, 128, 256 +- 1), prefixes
