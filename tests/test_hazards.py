@@ -149,26 +149,49 @@ def test_hazards_planted_in_a_listing_are_found():
     assert overwritten([start.replace("16x16x32", "32x32x16"), "s_nop 5", "v_mov_b32_e32 v13, v1"])
 
 
-@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="needs llvm-objdump")
-def test_wait_states_of_the_built_kernels(tmp_path):
+@pytest.fixture(scope="module")
+def listings(tmp_path_factory):
+    """(kernel, its instructions, {branch: where it leads}) of every kernel of the library, both places as indexes of instructions."""
+    if not os.path.exists(OBJDUMP):
+        pytest.skip("needs llvm-objdump")
     assert os.path.exists(LIB_PATH), "the library is not built"
-    found, loads, products = [], 0, 0
+    out = []
     for k, obj in enumerate(code_objects(LIB_PATH)):
-        f = tmp_path / f"{k}.co"
+        f = tmp_path_factory.mktemp("code") / f"{k}.co"
         f.write_bytes(obj)
-        text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", "--no-leading-addr", str(f)], capture_output=True, text=True, check=True).stdout
-        kernel, lines = None, []
-        for raw in text.splitlines() + ["<end>:"]:
-            m = re.match(r"(?:[0-9a-f]+ )?<(\S+)>:$", raw.strip())
-            if m:
-                found += [(kernel,) + v for v in violations(lines) + overwritten(lines)]
-                loads += sum("global_load_lds" in l for l in lines)
-                products += sum(l.startswith("v_mfma") for l in lines)
-                kernel, lines = m[1], []
-                continue
-            t = raw.split("//")[0].strip()
-            if t and not t.endswith(":"):
+        text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", str(f)], capture_output=True, text=True, check=True).stdout
+        for part in re.split(r"^[0-9a-f]+ <(?=\S+>:$)", text, flags=re.M)[1:]:
+            lines, places, leads = [], {}, {}
+            for t, place in re.findall(r"^\s+(\S.*?)\s*// ([0-9A-F]+):", part, flags=re.M):
+                places[int(place, 16)] = len(lines)
+                m = re.match(r"s_c?branch\S* (\d+)", t)
+                if m:   # (a signed number of words from the next instruction on)
+                    leads[len(lines)] = int(place, 16) + 4 + 4 * ((int(m[1]) ^ 0x8000) - 0x8000)
                 lines.append(t)
+            out.append((part[:part.index(">")], lines, {at: places[to] for at, to in leads.items() if to in places}))
+    return out
+
+
+def test_wait_states_of_the_built_kernels(listings):
+    found, loads, products = [], 0, 0
+    for kernel, lines, _ in listings:
+        found += [(kernel,) + v for v in violations(lines) + overwritten(lines)]
+        loads += sum("global_load_lds" in l for l in lines)
+        products += sum(l.startswith("v_mfma") for l in lines)
     assert loads > 1000 and products > 1000, "no loads to LDS, no matrix instructions: the disassembly is not what this test reads"
     assert not found, f"{len(found)} places, among them {found[:3]}"
 
+
+def test_block_loops_of_the_backward_kernels_reload_nothing(listings):
+    """No register parked in scratch memory comes back inside the loops over blocks or tiles: the wait for it is a wait for every load to LDS on its
+    way.  A loop is what lies between a branch back and where it leads; the body of a block has 64 or 128 matrix instructions, a round of four 512, and
+    the loops around those loops, over tasks and items, have more."""
+    loops, found = 0, []
+    for kernel, lines, leads in listings:
+        for at, to in leads.items() if "ca_bwd" in kernel else ():
+            body = lines[to:at + 1]
+            if any("global_load_lds" in l for l in body) and sum(l.startswith("v_mfma") for l in body) <= 512:
+                loops += 1
+                found += [(kernel, len(body), l) for l in body if l.startswith("scratch_load")]
+    assert loops > 100, "the disassembly is not what this test reads"
+    assert not found, f"{len(found)} reloads, among them {found[:3]}"
