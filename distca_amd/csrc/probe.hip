@@ -74,6 +74,8 @@ __global__ __launch_bounds__(256, 1) void mfma_rate_kernel(int iters, unsigned l
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   const unsigned long long c1 = __builtin_readcyclecounter(), r1 = __builtin_amdgcn_s_memrealtime();
   float t = 0.f;
+  // (the wait states that the compiler, which does not see the MFMAs, does not put between the last of them and the first read of its sums)
+  asm volatile("s_nop 15" : "+a"(acc[0]), "+a"(acc[1]), "+a"(acc[2]), "+a"(acc[3]));
 #pragma unroll
   for (int m = 0; m < 4; ++m)
 #pragma unroll

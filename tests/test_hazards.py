@@ -118,6 +118,48 @@ def overwritten(lines):
     return out
 
 
+def too_early(lines, targets=()):
+    """(wait states between, matrix instruction, instruction): an instruction that reads or overwrites what a matrix instruction writes before it is
+    there: within 8 wait states of one of four passes (16x16x32), 12 of one of eight (32x32x16).  A matrix instruction begins when the one before it has
+    taken its passes, whatever stands between the two; it takes a result over by itself as C operand in the same registers, and writes behind the one
+    before it.  `targets`: where
+    branches lead ({line: line}); both ways are followed."""
+    targets, out = dict(targets), []
+
+    def passes(line):
+        return 8 if "32x32" in line else 4
+
+    for i, start in enumerate(lines):
+        if not start.startswith("v_mfma"):
+            continue
+        result = registers(operands(start)[0])
+        needed = passes(start) + 4
+        todo, seen = [(i + 1, 0, passes(start))], set()   # line, wait states so far, wait states from which a matrix instruction can begin
+        while todo:
+            at, waits, free = todo.pop()
+            if at >= len(lines) or (at, waits, free) in seen:
+                continue
+            seen.add((at, waits, free))
+            op, ops = lines[at].split()[0], operands(lines[at])
+            product = op.startswith("v_mfma")
+            if product:
+                waits = max(waits, free - 1)
+            if waits >= needed:
+                continue
+            touched = union(ops[1:3] if product and registers(ops[3]) == result else ops[1:] if product else ops)
+            if touched & result and re.match(r"v_|ds_|global_|scratch_|buffer_|flat_", op):
+                out.append((waits, start, lines[at]))
+                continue
+            if product:
+                free = waits + 1 + passes(lines[at])
+            after = waits + (int(ops[0], 0) + 1 if op == "s_nop" else 1)
+            if op not in ("s_branch", "s_endpgm", "s_setpc_b64"):
+                todo.append((at + 1, after, free))
+            if at in targets:
+                todo.append((targets[at], after, free))
+    return out
+
+
 def test_hazards_planted_in_a_listing_are_found():
     load = "global_load_lds_dwordx4 v1, s[0:1] offset:2048"
     assert violations(["v_readlane_b32 s1, v252, 18", load])
@@ -148,6 +190,19 @@ def test_hazards_planted_in_a_listing_are_found():
     assert not overwritten([start, "v_mfma_f32_16x16x32_bf16 v[82:85], v[104:107], a[36:39], v[14:17]", "v_mov_b32_e32 v13, v1"])
     assert overwritten([start.replace("16x16x32", "32x32x16"), "s_nop 5", "v_mov_b32_e32 v13, v1"])
 
+    other = "v_mfma_f32_16x16x32_bf16 v[82:85], v[104:107], a[36:39], v[14:17]"
+    read, keep, store = "v_fma_f32 v1, v80, v2, v3", "ds_write_b64 v60, v[78:79]", "global_store_dwordx4 v[2:3], v[78:81], off"
+    assert all(too_early([start, x]) and too_early([start, "s_nop 6", x]) and not too_early([start, "s_nop 7", x]) for x in (read, keep, store, "v_mov_b32_e32 v81, v1"))
+    assert too_early([start, other, read]) and not too_early([start, other, other, read]) and not too_early([start, "v_mov_b32_e32 v9, v8"] * 8)
+    assert too_early([start, "v_mov_b32_e32 v9, v8", "v_mov_b32_e32 v9, v8", other, "s_nop 2", read])   # (what stands ahead of the second is not counted twice)
+    assert not too_early([start, "v_mov_b32_e32 v9, v8", "v_mov_b32_e32 v9, v8", other, "s_nop 3", read])
+    assert too_early([start, "v_mfma_f32_16x16x32_bf16 v[82:85], v[78:81], a[36:39], v[14:17]"])         # as an operand
+    assert too_early([start, "v_mfma_f32_16x16x32_bf16 v[82:85], v[104:107], a[36:39], v[80:83]"])       # as C, in part
+    assert not too_early([start, "v_mfma_f32_16x16x32_bf16 v[78:81], v[104:107], a[36:39], v[78:81]"])   # summed up on top
+    eight = start.replace("16x16x32", "32x32x16").replace("v[78:81]", "v[78:93]").replace("v[10:13]", "v[10:25]")
+    assert too_early([eight, "s_nop 10", read]) and not too_early([eight, "s_nop 11", read])
+    assert too_early([read, "s_nop 7", start, "s_cbranch_scc1 65533"], {3: 0}) and not too_early([read, "s_nop 7", start, "s_cbranch_scc1 65534"], {3: 1})
+
 
 @pytest.fixture(scope="module")
 def listings(tmp_path_factory):
@@ -174,8 +229,8 @@ def listings(tmp_path_factory):
 
 def test_wait_states_of_the_built_kernels(listings):
     found, loads, products = [], 0, 0
-    for kernel, lines, _ in listings:
-        found += [(kernel,) + v for v in violations(lines) + overwritten(lines)]
+    for kernel, lines, leads in listings:
+        found += [(kernel,) + v for v in violations(lines) + overwritten(lines) + too_early(lines, leads)]
         loads += sum("global_load_lds" in l for l in lines)
         products += sum(l.startswith("v_mfma") for l in lines)
     assert loads > 1000 and products > 1000, "no loads to LDS, no matrix instructions: the disassembly is not what this test reads"
