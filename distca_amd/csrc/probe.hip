@@ -53,7 +53,9 @@ __global__ __launch_bounds__(256, 1) void mfma_rate_kernel(int iters, unsigned l
 #pragma unroll
     for (int m = 0; m < 8; ++m) {
       asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc[m & 3]) : "v"(av[m]), "v"(bv[(m * 3) & 7]));
-      if (KIND == kProbeLdsRead) asm volatile("ds_read_b128 %0, %1" : "=v"(ld[m & 1]) : "v"(addr));
+      // (read and written: the registers stay the read's own until the wait at the end.  As results alone, which the next read replaces, they
+      // were given to other values while the read was on its way)
+      if (KIND == kProbeLdsRead) asm volatile("ds_read_b128 %0, %1" : "+v"(ld[m & 1]) : "v"(addr));
       if (KIND == kProbeFma4) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) asm volatile("v_fma_f32 %0, %0, %1, %1" : "+v"(x[(m * 4 + j) & 7]) : "v"(y));
@@ -63,7 +65,7 @@ __global__ __launch_bounds__(256, 1) void mfma_rate_kernel(int iters, unsigned l
         for (int j = 0; j < 2; ++j) asm volatile("v_exp_f32 %0, %0" : "+v"(x[(m * 2 + j) & 7]));
       }
       if (KIND == kProbeMix) {
-        if (m & 1) asm volatile("ds_read_b128 %0, %1" : "=v"(ld[(m >> 1) & 1]) : "v"(addr));
+        if (m & 1) asm volatile("ds_read_b128 %0, %1" : "+v"(ld[(m >> 1) & 1]) : "v"(addr));
 #pragma unroll
         for (int j = 0; j < 2; ++j) asm volatile("v_fma_f32 %0, %0, %1, %1" : "+v"(x[(m * 2 + j) & 7]) : "v"(y));
         if (m & 1) asm volatile("v_exp_f32 %0, %0" : "+v"(x[m & 7]));
@@ -71,7 +73,7 @@ __global__ __launch_bounds__(256, 1) void mfma_rate_kernel(int iters, unsigned l
       }
     }
   }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ld[0]), "+v"(ld[1])::"memory");
   const unsigned long long c1 = __builtin_readcyclecounter(), r1 = __builtin_amdgcn_s_memrealtime();
   float t = 0.f;
   // (the wait states that the compiler, which does not see the MFMAs, does not put between the last of them and the first read of its sums)

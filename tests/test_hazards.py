@@ -160,6 +160,26 @@ def too_early(lines, targets=()):
     return out
 
 
+def in_flight(lines):
+    """(read of LDS, instruction): an instruction that touches the registers of an LDS read ahead of a wait for it, in straight-line code.  Reads come back
+    in their order, so that a later one may bring the same registers."""
+    out = []
+    for i, read in enumerate(lines):
+        if not read.startswith("ds_read"):
+            continue
+        result, behind = registers(operands(read)[0]), 0
+        for after in lines[i + 1:]:
+            op, ops = after.split()[0], operands(after)
+            m = re.search(r"lgkmcnt\((\d+)\)", after)
+            if (m and int(m[1]) <= behind) or op in ("s_branch", "s_endpgm", "s_setpc_b64"):
+                break
+            if union(ops[1:] if op.startswith("ds_read") else ops) & result:
+                out.append((read, after))
+                break
+            behind += bool(re.match("ds_|s_load|s_buffer_load", op))
+    return out
+
+
 def test_hazards_planted_in_a_listing_are_found():
     load = "global_load_lds_dwordx4 v1, s[0:1] offset:2048"
     assert violations(["v_readlane_b32 s1, v252, 18", load])
@@ -203,6 +223,10 @@ def test_hazards_planted_in_a_listing_are_found():
     assert too_early([eight, "s_nop 10", read]) and not too_early([eight, "s_nop 11", read])
     assert too_early([read, "s_nop 7", start, "s_cbranch_scc1 65533"], {3: 0}) and not too_early([read, "s_nop 7", start, "s_cbranch_scc1 65534"], {3: 1})
 
+    read = "ds_read_b128 v[64:67], v62"
+    assert in_flight([read, "v_cvt_pk_bf16_f32 v64, v77, v78"]) and in_flight([read, "ds_read_b128 v[68:71], v62", "s_waitcnt lgkmcnt(1)", "ds_write_b64 v1, v[66:67]"]) == []
+    assert in_flight([read, "ds_read_b128 v[68:71], v62", "s_waitcnt lgkmcnt(1)", "v_mov_b32_e32 v1, v70"]) and not in_flight([read, read, "s_waitcnt lgkmcnt(0)", "v_mov_b32_e32 v1, v64"])
+
 
 @pytest.fixture(scope="module")
 def listings(tmp_path_factory):
@@ -230,7 +254,7 @@ def listings(tmp_path_factory):
 def test_wait_states_of_the_built_kernels(listings):
     found, loads, products = [], 0, 0
     for kernel, lines, leads in listings:
-        found += [(kernel,) + v for v in violations(lines) + overwritten(lines) + too_early(lines, leads)]
+        found += [(kernel,) + v for v in violations(lines) + overwritten(lines) + too_early(lines, leads) + in_flight(lines)]
         loads += sum("global_load_lds" in l for l in lines)
         products += sum(l.startswith("v_mfma") for l in lines)
     assert loads > 1000 and products > 1000, "no loads to LDS, no matrix instructions: the disassembly is not what this test reads"
