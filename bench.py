@@ -257,17 +257,19 @@ def server_tick_bench(torch, dev, batch, q, k, v, do, iters: int = 4, shard_cap:
     return res
 
 
-def mfma_probe(torch, _lib, dev, executed_tflops: float, rounds: int = 5, warm_seconds: float = 0.6):
-    """What this device delivers for the MFMA instruction itself, measured right after the attention steps: a loop of
-    MFMAs on every SIMD, alone and with other work in every MFMA's shadow.  The shader clock under such a load takes a
+def mfma_probe(torch, _lib, dev, fwd_tflops: float, bwd_tflops: float, rounds: int = 5, warm_seconds: float = 0.6):
+    """What this device delivers for the MFMA instructions themselves (32x32x16, the forward's, and 16x16x32, the backward's), measured right after
+    the attention steps: a loop of MFMAs on every SIMD, alone and with other work in every MFMA's shadow.  fwd_tflops, bwd_tflops: what the attention
+    kernels execute.  The shader clock under such a load takes a
     few hundred milliseconds to settle at what the power limit allows, so the MFMA-only loop first runs for
-    `warm_seconds`; the four variants are then run interleaved, round after round, and the median and the spread over
+    `warm_seconds`; the variants are then run interleaved, round after round, and the median and the spread over
     the rounds are reported per variant (so that a clock still drifting cannot favour whichever variant runs last)."""
     scratch = torch.zeros(4, dtype=torch.int64, device=dev)
     stream_ptr = torch.cuda.current_stream().cuda_stream
     kinds = (("mfma_only", _lib.PROBE_MFMA_ONLY), ("with_1kb_lds_read_per_mfma", _lib.PROBE_LDS_READ),
              ("with_4_fma_per_mfma", _lib.PROBE_FMA4), ("with_2_exp_per_mfma", _lib.PROBE_EXP2),
-             ("with_attention_side_work", _lib.PROBE_MIX))
+             ("with_attention_side_work", _lib.PROBE_MIX), ("mfma16_only", _lib.PROBE_MFMA16_ONLY),
+             ("mfma16_with_attention_side_work", _lib.PROBE_MFMA16_MIX))
     iters = 20000
     for _, kind in kinds:    # the first launch of a kernel also loads it
         _lib.probe_mfma_rate(kind, 200, scratch.data_ptr(), stream_ptr)
@@ -284,15 +286,18 @@ def mfma_probe(torch, _lib, dev, executed_tflops: float, rounds: int = 5, warm_s
         probe[name] = {"TFLOP/s": round(float(np.median(tf)), 1), "TFLOP/s_min": round(tf[0], 1), "TFLOP/s_max": round(tf[-1], 1),
                        "cycles_per_mfma": round(float(np.median([r[1] for r in runs[name]])), 2),
                        "clock_GHz": round(float(np.median([r[2] for r in runs[name]])), 3)}
-    probe["executed_TFLOP/s_of_the_three_attention_kernels"] = round(executed_tflops, 1)
-    probe["executed_over_mfma_only"] = round(executed_tflops / probe["mfma_only"]["TFLOP/s"], 4)
-    # with_attention_side_work: beside every MFMA half of a 1 KB LDS read, two multiply-adds, half an exponential and half
-    # a conversion, the per-MFMA average of the backward kernels' tile loops (no tile requests, barriers or prologues)
-    probe["executed_over_mfma_with_attention_side_work"] = round(executed_tflops / probe["with_attention_side_work"]["TFLOP/s"], 4)
-    probe["note"] = (f"v_mfma_f32_32x32x16_bf16 on pseudo-random operands, one wave per SIMD on every SIMD, {8 * iters} per wave and run; "
-                     f"{warm_seconds} s of the MFMA-only loop first, then the four variants interleaved for {rounds} rounds: median (min..max) "
+    probe["executed_TFLOP/s_of_the_forward"] = round(fwd_tflops, 1)
+    probe["executed_TFLOP/s_of_the_backward"] = round(bwd_tflops, 1)
+    probe["forward_over_mfma_only"] = round(fwd_tflops / probe["mfma_only"]["TFLOP/s"], 4)
+    probe["backward_over_mfma16_only"] = round(bwd_tflops / probe["mfma16_only"]["TFLOP/s"], 4)
+    # with_attention_side_work: beside every 32 K FLOP half of a 1 KB LDS read, two multiply-adds, half an exponential and half
+    # a conversion, the average of the backward kernels' tile loops (no tile requests, barriers or prologues)
+    probe["backward_over_mfma16_with_attention_side_work"] = round(bwd_tflops / probe["mfma16_with_attention_side_work"]["TFLOP/s"], 4)
+    probe["note"] = (f"v_mfma_f32_32x32x16_bf16 (mfma16: v_mfma_f32_16x16x32_bf16, two for one) on pseudo-random operands, one wave per SIMD on every SIMD, "
+                     f"{8 * iters} (mfma16: {16 * iters}) per wave and run; "
+                     f"{warm_seconds} s of the MFMA-only loop first, then the variants interleaved for {rounds} rounds: median (min..max) "
                      "rate by HIP events, clock by the device's cycle and real-time counters: what the power limit leaves "
-                     "of the published 2.5 PFLOP/s (every pipe busy at 2.4 GHz) on this device for this instruction")
+                     "of the published 2.5 PFLOP/s (every pipe busy at 2.4 GHz) on this device for these instructions")
     return probe
 
 
@@ -425,18 +430,17 @@ def main():
     log(f"  ca_fwd_kernel {fwd_k:.3f} ms -> {fwd_tf:.1f} TFLOP/s ({100 * fwd_tf / PEAK_BF16_TFLOPS:.1f}%)")
     log(f"  ca_bwd kernels {bwd_k:.3f} ms (dkdv {dkdv_k:.3f} + dq {dq_k:.3f}) -> {bwd_tf:.1f} TFLOP/s ({100 * bwd_tf / PEAK_BF16_TFLOPS:.1f}%)")
 
-    # what this device delivers for the MFMA instruction itself, right after the attention steps (the part is warm):
+    # what this device delivers for the MFMA instructions themselves, right after the attention steps (the part is warm):
     # a loop of MFMAs on every SIMD, alone and with other work in every MFMA's shadow
     probe = None
     if not args.no_probe:
-        executed = 1e-12 * (flop_fwd + 1.4 * flop_bwd) / ((fwd_k + bwd_k) * 1e-3)  # S and dP are computed in both backward kernels
-        probe = mfma_probe(torch, _lib, dev, executed)
-        log(f"  MFMA-only loop {probe['mfma_only']['TFLOP/s']} TFLOP/s (median of {probe['rounds']} rounds, {probe['mfma_only']['TFLOP/s_min']}"
-            f"..{probe['mfma_only']['TFLOP/s_max']}) at {probe['mfma_only']['clock_GHz']} GHz; the attention kernels execute "
-            f"{probe['executed_TFLOP/s_of_the_three_attention_kernels']} TFLOP/s = {100 * probe['executed_over_mfma_only']:.1f} % of it, "
-            f"{100 * probe['executed_over_mfma_with_attention_side_work']:.1f} % of the loop with the backward's per-MFMA side work "
-            f"({probe['with_attention_side_work']['TFLOP/s']} TFLOP/s at {probe['with_attention_side_work']['clock_GHz']} GHz, "
-            f"{probe['with_attention_side_work']['cycles_per_mfma']} cycles per MFMA)")
+        probe = mfma_probe(torch, _lib, dev, fwd_tf, 1.4 * bwd_tf)  # S and dP are computed in both backward kernels
+        log(f"  32x32x16 MFMAs alone {probe['mfma_only']['TFLOP/s']} TFLOP/s (median of {probe['rounds']} rounds, {probe['mfma_only']['TFLOP/s_min']}"
+            f"..{probe['mfma_only']['TFLOP/s_max']}) at {probe['mfma_only']['clock_GHz']} GHz: the forward executes {100 * probe['forward_over_mfma_only']:.1f} % of it; "
+            f"16x16x32 alone {probe['mfma16_only']['TFLOP/s']}, with the backward's side work {probe['mfma16_with_attention_side_work']['TFLOP/s']} "
+            f"({probe['mfma16_with_attention_side_work']['clock_GHz']} GHz, {probe['mfma16_with_attention_side_work']['cycles_per_mfma']} cycles per MFMA): the backward executes "
+            f"{probe['executed_TFLOP/s_of_the_backward']} TFLOP/s, {100 * probe['backward_over_mfma16_only']:.1f} % and "
+            f"{100 * probe['backward_over_mfma16_with_attention_side_work']:.1f} % of them")
 
     pack = None
     if not args.no_pack:

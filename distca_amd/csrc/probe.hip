@@ -1,23 +1,27 @@
-// What the part delivers for the MFMA instruction the attention kernels are made of, measured on the spot.
+// What the part delivers for the MFMA instructions the attention kernels are made of, measured on the spot.
 //
 // The published peak is every MFMA pipe busy at the nominal clock; under load the clock is what the power limit
 // leaves, and that depends on what runs beside the MFMAs.  This kernel keeps one wave on every SIMD of the device
 // issuing nothing but v_mfma_f32_32x32x16_bf16 on pseudo-random operands (eight operand pairs in rotation, four
-// accumulators), optionally with other work behind every MFMA that fits into its shadow: the pipe stays fully
-// occupied (33 cycles per MFMA) and the time per MFMA shows what that other work costs in clock.  Registers and
+// accumulators), the forward's instruction, or v_mfma_f32_16x16x32_bf16, the backward kernels', four in a row with one A operand as
+// theirs are (twelve operands, sixteen accumulators); optionally with other work behind every MFMA that fits into its shadow: the pipe stays
+// fully occupied (33 cycles per MFMA, 16 per small one) and the time per MFMA shows what that other work costs in clock.  Registers and
 // LDS only, fixed trip counts, two numbers written at the end: the benchmark prints the result next to the rate of
 // the attention kernels.
 #include "api_util.h"
 #include "common.h"
+
+#include <type_traits>
 
 namespace distca {
 namespace {
 
 typedef __bf16 probe_bf16x8 __attribute__((ext_vector_type(8)));
 
-// kProbeMix: beside every MFMA what the backward kernels have beside theirs, on average: half a kilobyte of LDS operand
-// reads (one 1 KB read per two MFMAs), two multiply-adds, half an exponential and half a conversion to bf16 pairs.
-enum { kProbeMfmaOnly = 0, kProbeLdsRead = 1, kProbeFma4 = 2, kProbeExp2 = 3, kProbeMix = 4, kProbeKinds = 5 };
+// kProbeMix, kProbe16Mix: beside 32 K FLOP, one large MFMA or two small ones, what the backward kernels have beside theirs, on average: half a
+// kilobyte of LDS operand reads (a 1 KB read every other time), two multiply-adds, half an exponential and half a conversion to bf16 pairs.
+enum { kProbeMfmaOnly = 0, kProbeLdsRead = 1, kProbeFma4 = 2, kProbeExp2 = 3, kProbeMix = 4, kProbe16Only = 5, kProbe16Mix = 6, kProbeKinds = 7 };
+constexpr bool is_small(int kind) { return kind >= kProbe16Only; }
 
 template <int KIND>
 __global__ __launch_bounds__(256, 1) void mfma_rate_kernel(int iters, unsigned long long *out) {
@@ -37,11 +41,12 @@ __global__ __launch_bounds__(256, 1) void mfma_rate_kernel(int iters, unsigned l
       av[q][e] = (__bf16)(((int)(h & 0xffff) - 32768) * (1.f / 16384));
       bv[q][e] = (__bf16)(((int)(h >> 16) - 32768) * (1.f / 16384));
     }
-  f32x16 acc[4];
+  constexpr int kAccs = is_small(KIND) ? 16 : 4;
+  std::conditional_t<is_small(KIND), f32x4, f32x16> acc[kAccs];
 #pragma unroll
-  for (int m = 0; m < 4; ++m)
+  for (int m = 0; m < kAccs; ++m)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[m][r] = 0.f;
+    for (int r = 0; r < 64 / kAccs; ++r) acc[m][r] = 0.f;
   float x[8], y = 0.999f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) x[i] = 0.001f * (lane + i);
@@ -49,10 +54,15 @@ __global__ __launch_bounds__(256, 1) void mfma_rate_kernel(int iters, unsigned l
   uint32_t pk = 0;
   const uint32_t addr = (uint32_t)(uintptr_t)(DISTCA_LDS uint32_t *)tile + lane * 16;
   const unsigned long long c0 = __builtin_readcyclecounter(), r0 = __builtin_amdgcn_s_memrealtime();
-  for (int it = 0; it < iters; ++it) {
+  auto round = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int m = 0; m < 8; ++m) {
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc[m & 3]) : "v"(av[m]), "v"(bv[(m * 3) & 7]));
+      auto small = [&](int n) __attribute__((always_inline)) {
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[n % kAccs]) : "v"(av[n >> 2]), "v"(bv[n & 7]));
+      };
+      if constexpr (!is_small(KIND)) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc[m % kAccs]) : "v"(av[m]), "v"(bv[(m * 3) & 7]));
+      if constexpr (is_small(KIND)) small(2 * m);
+      if constexpr (KIND == kProbe16Only) small(2 * m + 1);
       // (read and written: the registers stay the read's own until the wait at the end.  As results alone, which the next read replaces, they
       // were given to other values while the read was on its way)
       if (KIND == kProbeLdsRead) asm volatile("ds_read_b128 %0, %1" : "+v"(ld[m & 1]) : "v"(addr));
@@ -64,24 +74,35 @@ __global__ __launch_bounds__(256, 1) void mfma_rate_kernel(int iters, unsigned l
 #pragma unroll
         for (int j = 0; j < 2; ++j) asm volatile("v_exp_f32 %0, %0" : "+v"(x[(m * 2 + j) & 7]));
       }
-      if (KIND == kProbeMix) {
+      if (KIND == kProbeMix || KIND == kProbe16Mix) {
         if (m & 1) asm volatile("ds_read_b128 %0, %1" : "+v"(ld[(m >> 1) & 1]) : "v"(addr));
 #pragma unroll
-        for (int j = 0; j < 2; ++j) asm volatile("v_fma_f32 %0, %0, %1, %1" : "+v"(x[(m * 2 + j) & 7]) : "v"(y));
-        if (m & 1) asm volatile("v_exp_f32 %0, %0" : "+v"(x[m & 7]));
-        else asm volatile("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(pk) : "v"(x[m & 7]), "v"(x[(m + 1) & 7]));
+        for (int j = 0; j < 2; ++j) {
+          asm volatile("v_fma_f32 %0, %0, %1, %1" : "+v"(x[(m * 2 + j) & 7]) : "v"(y));
+          if constexpr (KIND == kProbe16Mix) if (j == 0) small(2 * m + 1);   // (two instructions behind each)
+        }
+        // (beside small ones, which leave no slot for wait states, of values that no neighbour makes or uses)
+        const int of = !is_small(KIND) ? m & 7 : m & 1 ? (m - 1) & 2 : (2 * m + 4) & 7;
+        if (m & 1) asm volatile("v_exp_f32 %0, %0" : "+v"(x[of]));
+        else asm volatile("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(pk) : "v"(x[of]), "v"(x[(of + 1) & 7]));
       }
     }
+  };
+  int it = 0;
+  if constexpr (is_small(KIND)) {   // (with a jump behind every 16 of them they took 17.5 cycles each)
+    for (; it + 4 <= iters; it += 4) round(), round(), round(), round();
   }
+  for (; it < iters; ++it) round();
   asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ld[0]), "+v"(ld[1])::"memory");
   const unsigned long long c1 = __builtin_readcyclecounter(), r1 = __builtin_amdgcn_s_memrealtime();
   float t = 0.f;
   // (the wait states that the compiler, which does not see the MFMAs, does not put between the last of them and the first read of its sums)
-  asm volatile("s_nop 15" : "+a"(acc[0]), "+a"(acc[1]), "+a"(acc[2]), "+a"(acc[3]));
 #pragma unroll
-  for (int m = 0; m < 4; ++m)
+  for (int m = 0; m < kAccs; m += 4) asm volatile("s_nop 15" : "+a"(acc[m]), "+a"(acc[m + 1]), "+a"(acc[m + 2]), "+a"(acc[m + 3]));
 #pragma unroll
-    for (int r = 0; r < 16; ++r) t += acc[m][r];
+  for (int m = 0; m < kAccs; ++m)
+#pragma unroll
+    for (int r = 0; r < 64 / kAccs; ++r) t += acc[m][r];
 #pragma unroll
   for (int i = 0; i < 8; ++i) t += x[i];
   t += ld[0][0] + ld[1][3] + (float)pk;
@@ -113,6 +134,8 @@ extern "C" int distca_probe_mfma_rate(int kind, int iters, void *scratch32, doub
     case kProbeLdsRead: hipLaunchKernelGGL((mfma_rate_kernel<kProbeLdsRead>), dim3(cus), dim3(256), 0, s, iters, out); break;
     case kProbeFma4: hipLaunchKernelGGL((mfma_rate_kernel<kProbeFma4>), dim3(cus), dim3(256), 0, s, iters, out); break;
     case kProbeExp2: hipLaunchKernelGGL((mfma_rate_kernel<kProbeExp2>), dim3(cus), dim3(256), 0, s, iters, out); break;
+    case kProbe16Only: hipLaunchKernelGGL((mfma_rate_kernel<kProbe16Only>), dim3(cus), dim3(256), 0, s, iters, out); break;
+    case kProbe16Mix: hipLaunchKernelGGL((mfma_rate_kernel<kProbe16Mix>), dim3(cus), dim3(256), 0, s, iters, out); break;
     default: hipLaunchKernelGGL((mfma_rate_kernel<kProbeMix>), dim3(cus), dim3(256), 0, s, iters, out); break;
   }
   (void)hipEventRecord(e1, s);
@@ -125,8 +148,8 @@ extern "C" int distca_probe_mfma_rate(int kind, int iters, void *scratch32, doub
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (rc != DISTCA_OK) return rc;
-  const double mfmas = (double)iters * 8.0;                  // per wave
-  const double flop = mfmas * 32768.0 * 4.0 * (double)cus;   // 2 * 32 * 32 * 16 per MFMA, four waves per compute unit
+  const double mfmas = (double)iters * (is_small(kind) ? 16.0 : 8.0);   // per wave
+  const double flop = (double)iters * 8.0 * 32768.0 * 4.0 * (double)cus;   // 2 * 32 * 32 * 16 per large MFMA, two small ones; four waves per compute unit
   *tflops = ms > 0.f ? flop / ((double)ms * 1e-3) / 1e12 : 0.0;
   *cycles_per_mfma = (double)h[0] / mfmas;
   *clock_ghz = h[1] ? (double)h[0] / ((double)h[1] * 10.0) : 0.0;  // the real-time counter ticks at 100 MHz
