@@ -153,8 +153,9 @@ inline int32_t bwd_split_target(const distca_ca_params *p) {
 // forward, cut / whole: 1100 tokens at 4/1 heads (17 tiles to gain) 29.2 / 24.5, 4 x 1024 at 8/2 (15) 33.7 / 24.8, 1500 at 32/8 (15) 40.9 / 32.5,
 // 2048 at 32/8 (16) 55 / 52, 2560 + 1024 + 512 at 32/8 (15) 75.5 / 71.2, 4096 at 32/8 (0) 129 / 125, 12000 at 32/8 (0) 934 / 926; above it: 2048 at 8/2 (29)
 // 38.1 / 39.5, 2048 at 4/1 (31) 34.2 / 39.0, 3000 at 4/1 (42) 41.5 / 54.2, 8192 at 8/2 (64) 145 / 159.
-// dQ's tiles are longer, its line lower: us backward, cut / whole: 1100 at 32/8 (13) 101.5 / 99, 2560 + 1024 + 512 at 32/8 (15) 248 / 245, 8192 at 32/8 (0) 1566 /
-// 1559; just above it, dQ of 1024 tokens at 8/2 (16) 34 / 41.
+// dQ's tiles are longer, its line lower: us backward, dQ cut / whole: 1100 at 32/8 (13.2) 102.7 / 100.0, 4 x 1024 at 8/2 (15) 102.5 / 98.7, 1500 at 32/8 (15.2)
+// 127.7 / 124.8, 2560 + 1024 + 512 at 32/8 (15) 233.8 / 231.3; at it, by heads: 1024 at 8/2 (15.9) 76.5 / 81.5, 2048 at 32/8 (16.5) 167.7 / 164.6; above it: 1100 at
+// 8/2 (16.8) 79.1 / 87.1, 1100 at 4/1 (17.4) 75.0 / 86.1, 2048 at 8/2 (29) 97.1 / 123.5.
 // Returns the number of pieces to aim for per kv head, 0 = no cutting.
 // It depends only on sizes that do not change with how K/V are stored, so that a tick gives the same bits in every form.
 constexpr int kSplitRowPiecesPerCU = 2;
@@ -200,7 +201,8 @@ inline int64_t list_grid(const distca_ca_params *p, int64_t items, bool few) {
 }
 // A list of which only what is worth it is cut (sched.h, worth_cutting).  item_cost and piece_extra in the list's cost unit: an
 // item's ticket, first loads and last stores take 11 us against 1.7 us per forward tile (dQ 15 against 2.4, dK/dV 14 against 1.5
-// per query block), a piece's fp32 result written and read again about as long as its bytes take at the unit's share of the memory rate, and
+// per query block, with 32x32x16 MFMAs; with 16x16x32 ones, one item a unit, a tile of dQ takes 2.1 us and a block of dK/dV 1.35, 2.3 and 1.55 before: the
+// costs below were left, which makes an item look a tenth cheaper than it is), a piece's fp32 result written and read again about as long as its bytes take at the unit's share of the memory rate, and
 // add_cost is the second launch.  us with pieces of 16 at least and no add_cost / of 8 with it, both directions: 256 tokens at 8/2 heads 86.6 / 74.6
 // (left whole), 389 tokens at 4/1 93.6 / 84.1, 2048 tokens at 4/1 160 / 143, a tick of 2048 query rows at 8/2 206 / 190.
 inline void cut_where_worth(SchedGeom *g, const distca_ca_params *p, int32_t target, int32_t item_cost, int32_t piece_extra, int32_t add_cost) {
