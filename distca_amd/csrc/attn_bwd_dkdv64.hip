@@ -27,7 +27,9 @@
 // with 16x16x32 -> with rounds and few waits (two boxes): 131072 packed tokens at 32/8 heads 23 250 -> 22 450 -> 21 020, a tick of 16384 tokens 2 575 ->
 // 2 443 -> 2 328; documents of 128 to 2048 tokens 1 466 -> 1 429 -> 1 348, of 1024 (65536 tokens) 1 139 -> 1 098 -> 1 053, of 256 527 -> 506 -> 504;
 // 389 tokens at 4/1 heads 28.5 -> 29.1 -> 28.9.  (With three lane-derived registers parked in scratch memory, reloaded ahead of each loop, where the
-// reload waits for every request in flight: documents of 256 tokens 554, 389 tokens 30.8.)
+// reload waits for every request in flight: documents of 256 tokens 554, 389 tokens 30.8.)  The rounds and the bodies of masked and half blocks make
+// 55 to 62 KB of code a form (40 to 45 before), within the 64 KB instruction cache of two compute units: 3 300 misses in 72 million requests of a launch over
+// documents of 128 to 2048 tokens.
 #include "api_util.h"
 #include "attn_bwd.h"
 #include "attn_cfg.h"
@@ -96,7 +98,7 @@ __device__ __forceinline__ void mfma16_vc(f32x4 &acc, elemx8 a, elemx8 b, const 
 // 0, 1, 2, 3, 0, 1, 2, 3.  Every wave passes the same barrier per query block, so a block on the diagonal takes as long as the wave that
 // sees most of it: with 64 keys in a row wave 0 has a whole block's work as soon as the first key is seen.  Dealt this way no wave has more
 // than half a block's until the rows see 128 keys, nor ever where a task ends in a block of at most 128 keys.
-// The kernel over 131072 tokens in documents of 64 / 128 / 256 / 512 / 2048, 32/8 heads, in us: 64 keys in a row 1526 / 1225 / 1168 /
+// The kernel over 131072 tokens in documents of 64 / 128 / 256 / 512 / 2048, 32/8 heads, with 32x32x16 MFMAs, in us: 64 keys in a row 1526 / 1225 / 1168 /
 // 1599 / 4426, in halves 1326 / 1115 / 1092 / 1536 / 4321 (a visit of half the work still takes 1.7 us of 2.0: requests, barrier and
 // the chain from S to dK do not shrink with it).  (With the second halves in the order 3, 2, 1, 0 instead, wave 3's two lay side by side, and
 // both could lie on the diagonal at once; now only one ever does, and only its elements are compared.)

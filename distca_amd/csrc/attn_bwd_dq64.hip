@@ -12,9 +12,9 @@
 //   dQ^T += K^T dS^T    32 MFMAs   A: transposing reads of the K tile, B: dS = P (dP - delta) with P = exp2(S c - lse2)
 //
 // 16x16x32 MFMAs rather than 32x32x16: the kernel is bound by power, and a FLOP of theirs moves half the accumulator
-// bytes (and twice the operand bytes, which cost less where neighbours share one).  A loop of nothing but MFMAs delivers
-// 1 765 TFLOP/s with the latter and 2 044 with the former, with half a KB of LDS reads and 2.3 vector instructions per
-// 32 K FLOP beside them 1 520 and 1 630 to 1 710.  They leave 2 issue slots each for anything else (the larger ones 5), so the side work
+// bytes (and twice the operand bytes, which cost less where neighbours share one).  A loop of nothing but MFMAs (probe.hip)
+// delivers 1 800 to 1 880 TFLOP/s with the latter and 1 960 to 2 080 with the former, with half a KB of LDS reads and three vector instructions per
+// 32 K FLOP beside them 1 570 to 1 640 and 1 700 to 1 780 (by box).  They leave 2 issue slots each for anything else (the larger ones 5), so the side work
 // is spread over the whole tile.  The kernel, before -> after: 131072 packed tokens at 32/8 heads 16 870 us -> 15 510
 // (1.66 -> 1.81 GHz at 79 % of the pipe's cycles), a tick of 16384 tokens 1 837 -> 1 711, documents of 128 to 2048 tokens 1 268 -> 1 251.
 //
