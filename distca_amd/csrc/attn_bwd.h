@@ -77,6 +77,14 @@ int dkdv64_lds_bytes();
 // few: the kernels for few items (sched.h, take_item); max_cut > 0 (only then): items may be pieces of key blocks, of which at most that many are cut; shared: items are (group of tasks, key block)
 int launch_dkdv64(const BwdArgs &a, int64_t grid, bool few, int64_t max_cut, bool shared, hipStream_t stream);       // bf16 elements
 int launch_dkdv64_f16(const BwdArgs &a, int64_t grid, bool few, int64_t max_cut, bool shared, hipStream_t stream);   // fp16 elements
+// ... and of what adds the pieces of at most max_cut key blocks up
+void launch_dkdv64_combine(const BwdArgs &a, int64_t max_cut, hipStream_t stream);
+void launch_dkdv64_combine_f16(const BwdArgs &a, int64_t max_cut, hipStream_t stream);
+void launch_dq64_combine(const BwdArgs &a, int64_t max_cut, hipStream_t stream);   // the same for blocks of query rows
+void launch_dq64_combine_f16(const BwdArgs &a, int64_t max_cut, hipStream_t stream);
+// dQ and dK/dV in one launch, for batches of few items whose row statistics are there already (attn_bwd_pair.hip)
+int launch_pair(const BwdArgs &q, int64_t grid_q, const BwdArgs &kv, int64_t grid_kv, bool shared, hipStream_t stream);
+int launch_pair_f16(const BwdArgs &q, int64_t grid_q, const BwdArgs &kv, int64_t grid_kv, bool shared, hipStream_t stream);
 // The dQ kernel with 64 query rows per wave (attn_bwd_dq64.hip).  max_cut as above, for blocks of query rows.
 int launch_dq64(const BwdArgs &a, int64_t grid, bool few, int64_t max_cut, hipStream_t stream);
 int launch_dq64_f16(const BwdArgs &a, int64_t grid, bool few, int64_t max_cut, hipStream_t stream);

@@ -16,6 +16,8 @@
 //      the workspace.
 //   2. ca_bwd_dkdv64_kernel (attn_bwd_dkdv64.hip): dK and dV, one workgroup of 4 waves per (task, block of
 //      256 keys, kv head), in the order of the backward tile schedule.
+//
+// Batches of few blocks have both in one launch (attn_bwd_pair.hip; the rule: pair_backward).
 #include "api_util.h"
 #include "attn_bwd.h"
 #include "attn_cfg.h"
@@ -33,11 +35,14 @@ __global__ __launch_bounds__(256) void fill_zero_kernel(u32x4 *__restrict__ p, i
 }
 
 // How a backward is laid out in its workspace: the two lists, the row statistics, and, where blocks are cut into pieces, the lists'
-// tables and one place for the slots of both (dQ's pieces are added up before the first of dK / dV is written).
+// tables and the slots of both: side by side where they fit into kSlotsMost together (attn_bwd_pair.hip writes both at a time), else in one place (dQ's
+// pieces are then added up before the first of dK / dV is written).
+constexpr int64_t kSlotsMost = 1024 * kDkdvSlotBytes;   // what a preferred workspace has at most for slots
 struct BwdLayout {
-  int64_t sched_kv, sched_q, delta, lse2, tables_kv, tables_q, slots, total;
+  int64_t sched_kv, sched_q, delta, lse2, tables_kv, tables_q, slots, slots_q, total;
   int64_t blocks_kv, blocks_q, items_kv, items_q;   // bounds on blocks, and room of the lists
   int32_t target_kv, target_q;                      // pieces aimed for per kv head, 0: whole blocks
+  bool slots_apart;
 };
 // shared: tasks over shared stored rows (items are then over groups of tasks).  preferred: cut blocks of query rows as well, and
 // key blocks whatever `deterministic` says.
@@ -58,7 +63,9 @@ BwdLayout bwd_layout(const distca_ca_params *p, bool shared, bool preferred) {
   w.tables_kv = take(split_tables_bytes(w.blocks_kv, w.target_kv, w.items_kv));
   w.tables_q = take(split_tables_bytes(w.blocks_q, w.target_q, w.items_q));
   const int64_t kv = split_max_slots(w.blocks_kv, w.target_kv) * kDkdvSlotBytes, q = split_max_slots(w.blocks_q, w.target_q) * kDqSlotBytes;
-  w.slots = take((kv > q ? kv : q) * p->num_heads_kv);
+  w.slots_apart = (kv + q) * p->num_heads_kv <= kSlotsMost;
+  w.slots = take((w.slots_apart || kv > q ? kv : q) * p->num_heads_kv);
+  w.slots_q = w.slots_apart ? take(q * p->num_heads_kv) : w.slots;
   if (preferred && o > w.slots) take(256);   // (so that no call that brought the smallest workspace is taken for one that brought this)
   if (!preferred && bwd_small_pieces(p)) {
     const int64_t small = sched_shared_region_bytes(p->num_tasks, bwd_key_blocks_bound(p) + bwd_small_list_pieces(p)) +
@@ -192,7 +199,6 @@ int DISTCA_FN(run_bwd)(const BwdQuerySide &qs, const void *k, const void *v, voi
   a.out = (const elem_t *)out; a.lse = qs.lse; a.lse_tok = (const uint8_t *)qs.lse_tok;
   a.dq = (elem_t *)dq; a.dk = (elem_t *)dk; a.dv = (elem_t *)dv;
   a.qs_task_off = qs.task_off; a.qs_tok_bytes = qs.tok_bytes; a.dq_task_off = qs.dq_task_off; a.dq_tok_bytes = qs.dq_tok_bytes;
-  a.partial = ws + w.slots;
   a.cu_q = cu_q; a.cu_k = cu_k; a.kv_off = kv_off;
   a.grp_first = a.grp_tasks = a.grp_off = a.grp_lmax = nullptr;
   a.shards = shards;
@@ -209,22 +215,32 @@ int DISTCA_FN(run_bwd)(const BwdQuerySide &qs, const void *k, const void *v, voi
   const ListJob q_list{cu_q, cu_k, launched_dq_geom(p, w.target_q), (int32_t *)(ws + w.sched_q), w.items_q, tables_of(w.tables_q, w.blocks_q, w.target_q)};
   const ListJob kv_list{cu_q, cu_k, launched_dkdv_geom(p, w.target_kv, preferred, shared), (int32_t *)(ws + w.sched_kv), w.items_kv,
                         tables_of(w.tables_kv, w.blocks_kv, w.target_kv)};
-  rc = launch_build_backward(kv_list, q_list, kv_off, p->num_tasks, BwdFill{(uint8_t *)dk, (uint8_t *)dv, (int64_t)p->num_heads_kv * kHeadDim * 2, p->total_k, shards}, s);
+  const bool pair = pair_backward(p, few_q && few_kv && (w.target_q == 0 || w.slots_apart));
+  RowStats stats{};
+  if (pair) stats = RowStats{(const uint8_t *)dout, (const uint8_t *)out, a.lse_tok, a.lse, a.qs_task_off, a.qs_tok_bytes, a.hq, a.total_q, kElemF16, a.lse2_w, a.dscaled_w};
+  rc = launch_build_backward(kv_list, q_list, kv_off, p->num_tasks, BwdFill{(uint8_t *)dk, (uint8_t *)dv, (int64_t)p->num_heads_kv * kHeadDim * 2, p->total_k, shards}, stats, s);
   if (rc) return rc;
 
   // ---- dQ: one workgroup per (task, block of query rows, kv head).  It runs first: it also leaves the row
-  // statistics (lse in the log2 domain, -delta) in the workspace, which the dK/dV kernel reads.
+  // statistics (lse in the log2 domain, -delta) in the workspace, which the dK/dV kernel reads.  Side by side (attn_bwd_pair.hip) the launch
+  // above has left them.
+  BwdArgs aq;
+  const int64_t grid_q = list_grid(p, w.items_q, few_q);
   {
-    const int64_t grid = list_grid(p, w.items_q, few_q);
+    const int64_t grid = grid_q;
     if (grid > 0x7fffffff) return fail(DISTCA_E_INVALID, "ca_bwd: grid too large");
     a.merge_tiles = q_list.geom.merge_tiles;
     a.sched = q_list.ws;
     a.zero_row = ws + w.sched_q + sched_zero_row_off(p->num_tasks, w.items_q);
     a.tickets = (int32_t *)(ws + w.sched_q + sched_ticket_off(p->num_tasks, w.items_q));
     a.cut = q_list.split.cut; a.slot = q_list.split.slot;
-    ScopedTimer timer(DISTCA_TIMER_CA_BWD_DQ, s);
-    rc = DISTCA_FN(launch_dq64)(a, grid, few_q, w.target_q > 0 ? split_max_cut(w.blocks_q, w.target_q) : 0, s);
-    if (rc) return rc;
+    a.partial = ws + w.slots_q;
+    aq = a;
+    if (!pair) {
+      ScopedTimer timer(DISTCA_TIMER_CA_BWD_DQ, s);
+      rc = DISTCA_FN(launch_dq64)(a, grid, few_q, w.target_q > 0 ? split_max_cut(w.blocks_q, w.target_q) : 0, s);
+      if (rc) return rc;
+    }
   }
   // ---- dK, dV: one workgroup per (task, 256-key block, kv head)
   {
@@ -239,9 +255,18 @@ int DISTCA_FN(run_bwd)(const BwdQuerySide &qs, const void *k, const void *v, voi
     a.zero_row = ws + w.sched_kv + sched_zero_row_off(p->num_tasks, w.items_kv);
     a.tickets = (int32_t *)(ws + w.sched_kv + sched_ticket_off(p->num_tasks, w.items_kv));
     a.cut = kv_list.split.cut; a.slot = kv_list.split.slot;
+    a.partial = ws + w.slots;
     ScopedTimer timer(DISTCA_TIMER_CA_BWD, s);
-    rc = DISTCA_FN(launch_dkdv64)(a, grid, few_kv, w.target_kv > 0 ? split_max_cut(w.blocks_kv, w.target_kv) : 0, shared, s);
-    if (rc) return rc;
+    const int64_t max_cut = w.target_kv > 0 ? split_max_cut(w.blocks_kv, w.target_kv) : 0;
+    if (pair) {
+      rc = DISTCA_FN(launch_pair)(aq, grid_q, a, grid, shared, s);
+      if (rc) return rc;
+      if (w.target_q > 0) DISTCA_FN(launch_dq64_combine)(aq, split_max_cut(w.blocks_q, w.target_q), s);
+      if (max_cut > 0) DISTCA_FN(launch_dkdv64_combine)(a, max_cut, s);
+    } else {
+      rc = DISTCA_FN(launch_dkdv64)(a, grid, few_kv, max_cut, shared, s);
+      if (rc) return rc;
+    }
   }
   return check_launch("ca_bwd");
 }

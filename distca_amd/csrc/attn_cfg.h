@@ -164,6 +164,16 @@ constexpr int kCutFromTilesFwd = 24, kCutFromTilesDq = 16;
 inline bool few_row_blocks(const distca_ca_params *p) {
   return (int64_t)p->total_q * p->num_heads_q < (int64_t)kSplitMaxBlocksPerCU * kFwdRows * num_compute_units();
 }
+// dQ and dK/dV side by side in one launch (attn_bwd_pair.hip) up to kPairBlocksPerCU blocks of query rows per compute unit: each then
+// fills what the other's longest blocks leave idle, and a launch is saved.  Beyond that their last blocks are a small part of the time and the pass over dO
+// and O that makes the row statistics ahead of both shows.  us backward, one after the other / side by side: 256 tokens at 8/2 heads 51 / 34, 389 at 4/1
+// 56 / 36, 1000 at 4/1 79 / 55, 2048 at 4/1 (both cut) 88 / 64, 8 x 1000 at 32/8 299 / 261, 8192 at 8/2 458 / 395, 4 x 2300 at 32/8 593 / 507; at 4 blocks a
+// unit 8192 at 32/8 1404 / 1354, 32768 at 8/2 5276 / 5123, 2 x 4096 at 32/8 764 / 771 (blocks that pack exactly); at 5 10000 at 32/8 2040 / 2010, 40000 at
+// 8/2 7929 / 7718; at 6 12000 at 32/8 2772 / 2821, at 8 4 x 4000 at 32/8 1329 / 1364.
+constexpr int kPairBlocksPerCU = 5;
+inline bool pair_backward(const distca_ca_params *p, bool possible) {
+  return possible && (int64_t)p->total_q * p->num_heads_q <= (int64_t)kPairBlocksPerCU * kDqRows * num_compute_units();
+}
 // An upper bound, times *scale, of the KV tiles that cutting could take off the longest block of query rows: all of its tiles but the load of a
 // unit, of which only the part counts that the task of the longest prefix brings along, half of its tiles for every block of that task per unit
 // (from two blocks per unit on pieces, of which there are two a unit, are on average no shorter than the task's blocks: asked, the list builder cuts none of such a task).  How many rows that task has is known where it is the only one, and
@@ -294,10 +304,19 @@ struct BwdFill {
   int32_t total_k;
   KvShards shards;
 };
+// The row statistics that the backward's kernels read, where a launch of their own makes them (attn_bwd_pair.hip): -<dO, O> and lse log2(e), [Hq][Tq].
+struct RowStats {
+  const uint8_t *dout, *out, *lse_tok;   // rows and lse as in BwdArgs
+  const float *lse;
+  const int64_t *task_off;
+  int64_t tok_bytes;
+  int32_t hq, total_q, f16;
+  float *lse2, *neg_delta;               // null: no statistics
+};
 int launch_build_forward(const ListJob &j, int32_t num_tasks, hipStream_t stream);
 // kv_off: null, or the tasks share stored K/V rows and the dK/dV list is made over groups of them (sched.h, SharedGroups; its region
 // is sched_shared_region_bytes long)
-int launch_build_backward(const ListJob &kv, const ListJob &q, const int32_t *kv_off, int32_t num_tasks, const BwdFill &fill, hipStream_t stream);
+int launch_build_backward(const ListJob &kv, const ListJob &q, const int32_t *kv_off, int32_t num_tasks, const BwdFill &fill, const RowStats &stats, hipStream_t stream);
 
 inline int64_t align_up(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 

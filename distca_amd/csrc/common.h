@@ -10,10 +10,12 @@ namespace distca {
 #ifdef DISTCA_F16
 typedef _Float16 elem_t;
 #define DISTCA_FN(name) name##_f16
+constexpr bool kElemF16 = true;
 #define DISTCA_MFMA16_ASM "v_mfma_f32_16x16x32_f16"
 #else
 typedef __bf16 elem_t;
 #define DISTCA_FN(name) name
+constexpr bool kElemF16 = false;
 #define DISTCA_MFMA16_ASM "v_mfma_f32_16x16x32_bf16"
 #endif
 typedef elem_t elemx8 __attribute__((ext_vector_type(8)));

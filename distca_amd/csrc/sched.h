@@ -309,6 +309,12 @@ DISTCA_HD SplitTables split_tables(void *at, int64_t max_blocks, int32_t target)
 }
 
 #if defined(__HIPCC__)
+// The (item, kv head) of workgroup `wg` of those over a list of few items; false past the list's end.
+__device__ __forceinline__ bool item_of_workgroup(unsigned wg, int32_t nitems, int32_t hkv, int &item, int &kvh) {
+  item = (int)(wg / (unsigned)hkv);
+  kvh = (int)(wg - (unsigned)item * (unsigned)hkv);
+  return item < nitems;
+}
 // Draws this workgroup's (item rank, kv head); false when every list is used up.  `slot` is two ints
 // of LDS that the caller may reuse afterwards.  All threads of the workgroup must call it.
 // BY_ID (the kernels for few items): no counters, the workgroup's id names the item, id / hkv of the list for head id % hkv.
@@ -318,11 +324,7 @@ DISTCA_HD SplitTables split_tables(void *at, int64_t max_blocks, int32_t target)
 // query rows, 2742 / 2863 us.
 template <bool BY_ID = false>
 __device__ __forceinline__ bool take_item(int32_t *tickets, int32_t nitems, int32_t hkv, int32_t *slot, int &item, int &kvh) {
-  if constexpr (BY_ID) {
-    item = (int)(blockIdx.x / (unsigned)hkv);
-    kvh = (int)(blockIdx.x - (unsigned)item * (unsigned)hkv);
-    return item < nitems;
-  }
+  if constexpr (BY_ID) return item_of_workgroup(blockIdx.x, nitems, hkv, item, kvh);
   if (threadIdx.x < 64) {  // the first wave
     // One look at all the counters at once (a lane per head): a workgroup that comes when every list is used
     // up -- half of the launch's workgroups -- leaves after a single round trip to memory.  Counters only

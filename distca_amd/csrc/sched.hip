@@ -491,9 +491,58 @@ __device__ void fill_rows(FillScratch &f, TaskCache &cache, const BwdFill &a, co
   }
 }
 
-// All that a backward needs before its kernels, in one launch: workgroup 0 builds the dK/dV list, workgroup 1 the dQ list, the
-// others clear the dk / dv rows that no work item writes.  (As launches of their own the three took 25 to 45 us of a small batch's backward.)
-__global__ __launch_bounds__(kSchedThreads) void build_backward_kernel(ListJob kv, ListJob q, const int32_t *__restrict__ kv_off, int32_t num_tasks, BwdFill fill) {
+// The row statistics, four lanes to a row, whose products are added up in the dQ kernel's order: the same bits whichever makes them.
+// Bound by reading dO and O, and by one trip to memory where those are few.
+constexpr int kStatsRows = kSchedThreads / 4;
+__device__ void row_stats(const RowStats &a, const int32_t *__restrict__ cu_q, int32_t num_tasks, int part, int parts) {
+  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+  const int quarter = threadIdx.x & 3;
+  const int32_t rows = a.total_q * a.hq;
+  for (int32_t r = part * kStatsRows + (int32_t)(threadIdx.x >> 2); r < rows; r += parts * kStatsRows) {
+    const int32_t t = r / a.hq, h = r - t * a.hq;
+    int64_t at = (int64_t)t * a.tok_bytes;
+    if (a.task_off) {
+      int32_t lo = 0, hi = num_tasks;   // the last task that starts at or before t
+      while (hi - lo > 1) {
+        const int32_t mid = (lo + hi) >> 1;
+        if (cu_q[mid] <= t) lo = mid;
+        else hi = mid;
+      }
+      if (t < cu_q[lo] || t >= cu_q[lo + 1]) continue;   // (no task's token)
+      at = a.task_off[lo] + (int64_t)(t - cu_q[lo]) * a.tok_bytes;
+    }
+    const u32x4 *dop = reinterpret_cast<const u32x4 *>(a.dout + at + h * (kHeadDim * 2)) + quarter, *op = reinterpret_cast<const u32x4 *>(a.out + at + h * (kHeadDim * 2)) + quarter;
+    u32x4 x[4], y[4];   // d = 32 s + 8 quarter .. +7
+#pragma unroll
+    for (int s = 0; s < 4; ++s) x[s] = dop[4 * s], y[s] = op[4 * s];
+    float lse = 0.f, sum = 0.f;
+    if (quarter == 0) lse = a.lse ? a.lse[(int64_t)h * a.total_q + t] : reinterpret_cast<const float *>(a.lse_tok + at)[h];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t u = x[s][i], v = y[s][i];   // (two elements each; a bit cast of x[s][i] itself took x[s][0] for every i)
+        if (a.f16) {
+          const f16x2 uh = __builtin_bit_cast(f16x2, u), vh = __builtin_bit_cast(f16x2, v);
+          sum += (float)uh[0] * (float)vh[0];
+          sum += (float)uh[1] * (float)vh[1];
+        } else {
+          sum += __builtin_bit_cast(float, u << 16) * __builtin_bit_cast(float, v << 16);
+          sum += __builtin_bit_cast(float, u & 0xffff0000u) * __builtin_bit_cast(float, v & 0xffff0000u);
+        }
+      }
+    sum += __shfl_xor(sum, 1, 4);
+    sum += __shfl_xor(sum, 2, 4);
+    if (quarter == 0) {
+      a.lse2[(int64_t)h * a.total_q + t] = lse * 1.4426950408889634f;
+      a.neg_delta[(int64_t)h * a.total_q + t] = -sum;
+    }
+  }
+}
+
+// All that a backward needs before its kernels, in one launch: workgroup 0 builds the dK/dV list, workgroup 1 the dQ list, `fill_parts` others
+// clear the dk / dv rows that no work item writes, and the rest makes the row statistics, where it is asked to.  (As launches of their own the three took 25 to 45 us of a small batch's backward.)
+__global__ __launch_bounds__(kSchedThreads) void build_backward_kernel(ListJob kv, ListJob q, const int32_t *__restrict__ kv_off, int32_t num_tasks, BwdFill fill, int fill_parts, RowStats stats) {
   __shared__ TaskCache cache;
   __shared__ ListScratch s;
   __shared__ union {
@@ -505,8 +554,10 @@ __global__ __launch_bounds__(kSchedThreads) void build_backward_kernel(ListJob k
     else build_own<true>(s, cache, kv, num_tasks);
   } else if (blockIdx.x == 1) {
     build_own<false>(s, cache, q, num_tasks);
+  } else if ((int)blockIdx.x < 2 + fill_parts) {
+    fill_rows(o.fill, cache, fill, q, kv_off, num_tasks, (int)blockIdx.x - 2, fill_parts);
   } else {
-    fill_rows(o.fill, cache, fill, q, kv_off, num_tasks, (int)blockIdx.x - 2, (int)gridDim.x - 2);
+    row_stats(stats, q.cu_q, num_tasks, (int)blockIdx.x - 2 - fill_parts, (int)gridDim.x - 2 - fill_parts);
   }
 }
 
@@ -518,11 +569,16 @@ int launch_build_forward(const ListJob &j, int32_t num_tasks, hipStream_t stream
   return check_launch("build_forward");
 }
 
-int launch_build_backward(const ListJob &kv, const ListJob &q, const int32_t *kv_off, int32_t num_tasks, const BwdFill &fill, hipStream_t stream) {
+int launch_build_backward(const ListJob &kv, const ListJob &q, const int32_t *kv_off, int32_t num_tasks, const BwdFill &fill, const RowStats &stats, hipStream_t stream) {
   if (kv.max_items > 0x7fffffff || q.max_items > 0x7fffffff) return fail(DISTCA_E_INVALID, "schedule: too many work items");
   // (rows to clear are rare: a workgroup per MB of dk and dv, should it be all of them)
   const int64_t mb = (int64_t)fill.total_k * fill.row_bytes >> 19, parts = mb < 14 ? 14 : (mb > 254 ? 254 : mb);
-  hipLaunchKernelGGL(build_backward_kernel, dim3((unsigned)(2 + parts)), dim3(kSchedThreads), 0, stream, kv, q, kv_off, num_tasks, fill);
+  int64_t stat_parts = 0;
+  if (stats.lse2) {
+    stat_parts = ((int64_t)stats.total_q * stats.hq + kStatsRows - 1) / kStatsRows;
+    if (stat_parts > 2 * num_compute_units()) stat_parts = 2 * num_compute_units();
+  }
+  hipLaunchKernelGGL(build_backward_kernel, dim3((unsigned)(2 + parts + stat_parts)), dim3(kSchedThreads), 0, stream, kv, q, kv_off, num_tasks, fill, (int)parts, stats);
   return check_launch("build_backward");
 }
 

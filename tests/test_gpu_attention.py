@@ -512,6 +512,34 @@ def test_fp16_and_bf16_agree_on_the_same_values(cuda):
     assert (outs[0] - outs[1]).abs().max().item() <= 2e-2
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gradients_side_by_side_and_one_after_the_other(cuda, dtype):
+    """40 documents of 256 tokens at 32/8 heads are the most blocks of query rows (five a compute unit) whose dQ and dK/dV share a launch, with the row
+    statistics made ahead of both; with a document of one token more the dQ kernel makes them and runs first.  Documents that are one
+    key block each are never cut, so that every one of their gradients comes from the same sums in the same order: the same bits (fp16's dk: below)."""
+    from distca_amd.fused_comm_attn import ca_varlen_bwd, ca_varlen_fwd
+    n = 5 * 256 * torch.cuda.get_device_properties(0).multi_processor_count // 32 // 256
+    lens = [256] * n + [1]
+    tokens = 256 * n
+    q, k, v, do = (t.to(dtype).to(cuda) for t in make_qkv(tokens + 1, tokens + 1, 32, 8, 128, 81))
+    res = []
+    for part, docs in ((slice(0, tokens), lens[:-1]), (slice(0, tokens + 1), lens)):
+        c = torch.tensor(cu(docs), device=cuda)
+        x = [t[part].contiguous() for t in (q, k, v, do)]
+        out, lse = ca_varlen_fwd(*x[:3], c, c, 256, 256)
+        res.append(ca_varlen_bwd(x[3], *x[:3], out, lse, c, c, 256, 256, None, True, True))
+    for name, a, b in zip(("dq", "dk", "dv"), *res):
+        if name == "dk" and dtype == torch.float16:
+            # the compiler adds some of <dO, O>'s products in pairs there, others in the dQ kernel: delta differs in its 24th bit, which
+            # moves dS by at most a unit of fp16 (2^-11 of it) where it lies next to the middle of two, one in some thousands
+            assert (a.float() - b[:tokens].float()).norm() <= 1e-4 * b[:tokens].float().norm()
+        else:
+            assert torch.equal(a, b[:tokens]), name
+    ref = ca_reference_bwd(*(t[:256].cpu() for t in (do, q, k, v)), cu([256]), cu([256]))
+    for name, a, b in zip(("dq", "dk", "dv"), res[0], ref):
+        assert_close_bf16(a[:256], b, name)
+
+
 @pytest.mark.parametrize("d,dtype", [(64, torch.bfloat16), (96, torch.float16), (40, torch.bfloat16), (8, torch.bfloat16)])
 def test_head_dims_below_128(cuda, d, dtype):
     """Head dimensions that are multiples of 8 below 128 (the reference pads to a multiple of 8 and lets flash-attn
