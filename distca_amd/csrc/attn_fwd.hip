@@ -46,6 +46,7 @@ constexpr int kOutOff = kQOff + kFwdWaves * kFwdMsub * kQWave, kOutWave = 32 * k
 constexpr int kFwdLds = kOutOff + kFwdWaves * kFwdMsub * kOutWave;
 static_assert(kFwdLds <= 160 * 1024, "LDS of a compute unit");
 constexpr int kDirectTasks = 256;    // batches without a list: at most so many tasks to look through
+constexpr int kRankTasks = 64;       // ... or to find the block of a rank among
 constexpr int kOutStores = 2 * 32 / 8;   // store instructions of a sub-block's rows
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
@@ -65,8 +66,8 @@ struct FwdArgs {
   elem_t *out;
   float *lse;
   const int32_t *cu_q, *cu_k, *kv_off;
-  const int32_t *sched;  // schedule workspace; null (SPLIT kernels): there is no list, num_tasks tasks' blocks are taken as they come
-  int32_t num_tasks;
+  const int32_t *sched;  // schedule workspace; null (SPLIT kernels): there is no list, num_tasks tasks' blocks are taken by rank, or, max_tiles == 0, as they come
+  int32_t num_tasks, max_tiles;   // max_tiles: KV tiles of the longest prefix, at most
   const void *zero_row;  // 256 zero bytes: source of tile rows past the end of the prefix
   int32_t sched_items_off;  // int32 offset of the item array
   int32_t hq, hkv, group, total_q;
@@ -130,6 +131,39 @@ __device__ __forceinline__ int4 block_of_batch(const int32_t *cu_q, int num_task
   return make_int4(-1, 0, 0, 0);
 }
 
+// The block of rank `e` among the batch's blocks of query rows, from the one of the most KV tiles down.  Every wave finds it by itself, a lane to a
+// task: a task's blocks cost the more the later they come, so that how many cost at least c is a division, and the cost at rank e a search over c, a
+// sum over the lanes a step.
+__device__ __forceinline__ int4 block_of_rank(const int32_t *cu_q, const int32_t *cu_k, int num_tasks, int group, int causal, int max_tiles, int e) {
+  const int lane = threadIdx.x & 63;
+  int lq = 0, lk = 0;
+  if (lane < num_tasks) {
+    lq = cu_q[lane + 1] - cu_q[lane];
+    lk = cu_k[lane + 1] - cu_k[lane];
+  }
+  const int blocks = lq > 0 ? (lq * group + kFwdRows - 1) / kFwdRows : 0;
+  // the first block of the lane's task that costs c or more: whose last token sees key kFwdKV (c - 1)
+  auto first_of = [&](int c) {
+    const int key = kFwdKV * (c - 1);
+    const int t = causal ? key + 1 - (lk - lq) : 0;   // tokens of the task up to the first that sees it
+    const int first = t > 1 ? ((t - 1) * group) / kFwdRows : 0;
+    return c <= 0 ? 0 : key >= lk || t > lq ? blocks : first;
+  };
+  auto count = [&](int c) { return __builtin_amdgcn_readlane(wave_inclusive_scan_i32(blocks - first_of(c)), 63); };   // blocks of cost c or more
+  int lo = 0, hi = max_tiles + 1, past = 0;   // count(lo) > e >= count(hi) = past
+  if (e >= count(0)) return make_int4(-1, 0, 0, 0);
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1, n = count(mid);
+    if (n > e) lo = mid;
+    else hi = mid, past = n;
+  }
+  // block e - past of those of that cost, task after task
+  // (prefixes longer than they were said to be count as that long)
+  const int first = first_of(lo), n = (lo < max_tiles ? first_of(lo + 1) : blocks) - first, incl = wave_inclusive_scan_i32(n);
+  const int task = __builtin_ctzll(__ballot(incl > e - past));
+  return make_int4(task, e - past + __builtin_amdgcn_readlane(first - (incl - n), task), 0, 1 << 16);
+}
+
 // SEG: K/V rows are addressed through a table of shards (kv_shards.h) instead of as one dense tensor.
 // MERGE: a work item is several consecutive blocks of a task's query rows (sched.h, fwd_merge), worked off one after the
 // other; otherwise it is one block.
@@ -141,10 +175,10 @@ __global__ __launch_bounds__(kFwdWaves * 64, (MSUB == 1 && kFwdWaves == 4 ? 2 : 
   int item, kvh;
   int4 it;
   if (SPLIT && !a.sched) {
-    // no list (see run_fwd_tokens): the workgroup's id counts the batch's blocks
+    // no list (see run_fwd_tokens): the workgroup's id is its block's rank, or counts the batch's blocks
     item = (int)(blockIdx.x / (unsigned)a.hkv);
     kvh = (int)(blockIdx.x - (unsigned)item * (unsigned)a.hkv);
-    it = block_of_batch(a.cu_q, a.num_tasks, a.group, item);
+    it = a.max_tiles ? block_of_rank(a.cu_q, a.cu_k, a.num_tasks, a.group, a.causal, a.max_tiles, item) : block_of_batch(a.cu_q, a.num_tasks, a.group, item);
     if (it.x < 0) return;
   } else {
     const int nitems = a.sched[0];
@@ -982,7 +1016,12 @@ int DISTCA_FN(run_fwd_tokens)(const void *q_base, const int64_t *q_task_off, int
   // A batch whose blocks all run at once (one workgroup a compute unit) and stay whole needs no list: which workgroup has which block
   // does not matter then, and finding one by a scan of the task bounds takes one trip to memory where the list takes a launch of 5 us.
   // us with a list / without: 256 tokens at 4/1 heads 17.3 / 12.4, 389 at 8/2 20.0 / 15.1, 1000 at 32/8 31.9 / 26.9.
-  const bool direct = few && !split && max_items * p->num_heads_kv <= num_compute_units() && p->num_tasks <= kDirectTasks;
+  const bool at_once = max_items * p->num_heads_kv <= num_compute_units() && p->num_tasks <= kDirectTasks;
+  // With several rounds of workgroups, which take their items by id here, the order matters, longest first; up to 64 tasks a workgroup finds the block of
+  // its rank in less than a microsecond a round.  us with a list / without: 2048 tokens at 32/8 heads 50.2 / 45.3, 512 + 1024 + 2560 70.6 / 66.7, 4096 123.0 /
+  // 118.8, 20 x 300 50.8 / 47.4, 16 x 1024 at 8/2 45.4 / 41.0, 6 blocks a unit (12000 at 32/8) 918 / 917.  (Four tasks a lane, up to 256: a microsecond
+  // more a round, most of it for code that is not in the cache yet, and no gain left.)
+  const bool direct = few && !split && (at_once || p->num_tasks <= kRankTasks);
   if (!direct) {
     rc = launch_build_forward(ListJob{cu_q, cu_k, geom, (int32_t *)workspace, max_items, tables}, p->num_tasks, s);
     if (rc) return rc;
@@ -994,6 +1033,7 @@ int DISTCA_FN(run_fwd_tokens)(const void *q_base, const int64_t *q_task_off, int
   a.cu_q = cu_q; a.cu_k = cu_k; a.kv_off = kv_off;
   a.sched = direct ? nullptr : (const int32_t *)workspace;
   a.num_tasks = p->num_tasks;
+  a.max_tiles = at_once ? 0 : p->max_seqlen_k / kFwdKV + 1;
   a.zero_row = (const uint8_t *)workspace + sched_zero_row_off(p->num_tasks, max_items);
   a.sched_items_off = (int32_t)sched_header_ints(p->num_tasks);
   a.tickets = (int32_t *)((uint8_t *)workspace + sched_ticket_off(p->num_tasks, max_items));

@@ -90,6 +90,18 @@ __device__ __forceinline__ float pair_sum(float x) { return x + __shfl_xor(x, 32
 // sum of x over the four lanes l % 16 + 16 i.
 __device__ __forceinline__ float quad_sum(float x) { return pair_sum(x + __shfl_xor(x, 16, 64)); }
 
+// Inclusive sum over the wave's lanes, by DPP moves: within rows of 16, then from the last lane of a row and of a half on.  (Lane
+// exchanges through LDS, ten of them a scan, were most of a scan's microsecond.)
+__device__ __forceinline__ int32_t wave_inclusive_scan_i32(int32_t v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
 // LDS-direct global loads.  One piece per active lane goes from global memory straight into
 // LDS at lds_base + piece_bytes * lane, with no staging registers.  The compiler is not told
 // that these are memory operations: the caller orders them with wait_vm0() followed by a

@@ -4,6 +4,7 @@
 
 #include "api_util.h"
 #include "attn_cfg.h"
+#include "common.h"
 #include "kv_shards.h"
 #include "sched.h"
 
@@ -14,18 +15,6 @@ constexpr int kSchedThreads = 1024;
 // Batches of at most this many tasks (nearly all of them) are worked on in LDS: the builder is one workgroup whose phases are
 // chains of dependent reads, and at half a microsecond a read from memory they were most of its time.
 constexpr int kLdsTasks = kSchedThreads;
-
-// Inclusive sum over the wave's lanes, by DPP moves: within rows of 16, then from the last lane of a row and of a half on.  (Lane
-// exchanges through LDS, ten of them a scan, were most of a scan's microsecond.)
-__device__ __forceinline__ int32_t wave_inclusive_scan_i32(int32_t v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
-  return v;
-}
 
 __device__ __forceinline__ int32_t block_inclusive_scan_i32(int32_t v, int32_t *wave_sums) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;

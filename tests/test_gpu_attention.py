@@ -512,6 +512,38 @@ def test_fp16_and_bf16_agree_on_the_same_values(cuda):
     assert (outs[0] - outs[1]).abs().max().item() <= 2e-2
 
 
+@pytest.mark.parametrize("seed", range(6))
+def test_blocks_by_rank_and_from_a_list(cuda, seed):
+    """A forward of few blocks over at most 64 tasks has no list: workgroups find the block of their rank.  With a 65th task there is one.  Tasks of all
+    sizes, without tokens or keys among them, more queries than keys or fewer, over their own or over shared rows, causal or not: every block is
+    computed exactly once, to the same bits."""
+    from distca_amd.fused_comm_attn import ca_varlen_fwd
+    rng = np.random.default_rng(900 + seed)
+    hq, hkv = [(32, 8), (16, 4), (8, 8), (12, 4), (64, 8), (4, 1)][seed]
+    n = [64, 64, 63, 64, 8, 64][seed]
+    top = [200, 800, 400, 500, 1400, 1400][seed]   # (no blocks long enough to be cut)
+    q_lens = [int(x) for x in rng.integers(0, top, n)]
+    k_lens = [int(q) if rng.random() < 0.5 else int(rng.integers(0, top + 100)) for q in q_lens]
+    if seed == 1:
+        q_lens[:40] = [0] * 40   # ranks past the last task with blocks
+    causal, shared = seed != 3, seed == 2
+    fill = 65 - n
+    tq = sum(q_lens) + fill
+    tk = max(k_lens) if shared else sum(k_lens) + fill
+    assert tq * hq > 256 * torch.cuda.get_device_properties(0).multi_processor_count, "one round of workgroups: blocks as they come"
+    q, k, v, _ = (t.to(cuda) for t in make_qkv(tq, max(tk, 1), hq, hkv, 128, 90 + seed))
+    res = []
+    for ql, kl in ((q_lens, k_lens), (q_lens + [1] * fill, k_lens + [1] * fill)):
+        off = torch.zeros(len(ql), dtype=torch.int32, device=cuda) if shared else None
+        rows = sum(kl) if not shared else tk
+        res.append(ca_varlen_fwd(q[:sum(ql)].contiguous(), k[:rows].contiguous(), v[:rows].contiguous(), torch.tensor(cu(ql), device=cuda),
+                                 torch.tensor(cu(kl), device=cuda), max(ql), max(kl), None, causal, off))
+    tokens = sum(q_lens)
+    assert torch.equal(res[0][0], res[1][0][:tokens])
+    assert torch.equal(res[0][1], res[1][1][:, :tokens])
+    assert bool(torch.isfinite(res[0][0].float()).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_gradients_side_by_side_and_one_after_the_other(cuda, dtype):
     """40 documents of 256 tokens at 32/8 heads are the most blocks of query rows (five a compute unit) whose dQ and dK/dV share a launch, with the row
