@@ -6,6 +6,7 @@
 // (sched.hip, row_stats: a pass over dO and O, which at such sizes is nothing), and one launch takes both lists, dK/dV's, whose
 // items are the longer ones, first.  389 tokens at 4/1 heads: the lists 9 us (statistics included), dQ 20 and dK/dV 23 one after the other; side by
 // side 24.  The whole backward 56 -> 36 us there, 8 x 1000 tokens at 32/8 heads 299 -> 261, 8192 at 8/2 458 -> 395 (more at pair_backward, attn_cfg.h).
+// dQ reads the statistics too, and O no more: 8 x 1000 tokens at 32/8 heads 269 -> 259 us, 20 x 300 134.5 -> 128.7, 2048 at 32/8 150 -> 146.5.
 // Like the _split forms these park 20 to 40 registers in scratch memory, none of which comes back inside a loop over blocks or tiles.
 #include "api_util.h"
 #include "attn_bwd.h"
