@@ -35,9 +35,8 @@ __global__ __launch_bounds__(256) void fill_zero_kernel(u32x4 *__restrict__ p, i
 }
 
 // How a backward is laid out in its workspace: the two lists, the row statistics, and, where blocks are cut into pieces, the lists'
-// tables and the slots of both: side by side where they fit into kSlotsMost together (attn_bwd_pair.hip writes both at a time), else in one place (dQ's
+// tables and the slots of both: side by side where they fit (slots_apart; attn_bwd_pair.hip writes both at a time), else in one place (dQ's
 // pieces are then added up before the first of dK / dV is written).
-constexpr int64_t kSlotsMost = 1024 * kDkdvSlotBytes;   // what a preferred workspace has at most for slots
 struct BwdLayout {
   int64_t sched_kv, sched_q, delta, lse2, tables_kv, tables_q, slots, slots_q, total;
   int64_t blocks_kv, blocks_q, items_kv, items_q;   // bounds on blocks, and room of the lists
@@ -63,7 +62,7 @@ BwdLayout bwd_layout(const distca_ca_params *p, bool shared, bool preferred) {
   w.tables_kv = take(split_tables_bytes(w.blocks_kv, w.target_kv, w.items_kv));
   w.tables_q = take(split_tables_bytes(w.blocks_q, w.target_q, w.items_q));
   const int64_t kv = split_max_slots(w.blocks_kv, w.target_kv) * kDkdvSlotBytes, q = split_max_slots(w.blocks_q, w.target_q) * kDqSlotBytes;
-  w.slots_apart = (kv + q) * p->num_heads_kv <= kSlotsMost;
+  w.slots_apart = slots_apart(p, w.blocks_kv, w.target_kv, w.blocks_q, w.target_q);
   w.slots = take((w.slots_apart || kv > q ? kv : q) * p->num_heads_kv);
   w.slots_q = w.slots_apart ? take(q * p->num_heads_kv) : w.slots;
   if (preferred && o > w.slots) take(256);   // (so that no call that brought the smallest workspace is taken for one that brought this)
@@ -212,10 +211,10 @@ int DISTCA_FN(run_bwd)(const BwdQuerySide &qs, const void *k, const void *v, voi
   // ---- both work lists, and zeros where no work item writes dk / dv
   const bool few_q = few_row_blocks(p), few_kv = few_key_blocks(p, kSplitFewPerCU) || w.target_kv > 0;
   auto tables_of = [&](int64_t at, int64_t blocks, int32_t target) { return target > 0 ? split_tables(ws + at, blocks, target) : SplitTables{}; };
-  const ListJob q_list{cu_q, cu_k, launched_dq_geom(p, w.target_q), (int32_t *)(ws + w.sched_q), w.items_q, tables_of(w.tables_q, w.blocks_q, w.target_q)};
-  const ListJob kv_list{cu_q, cu_k, launched_dkdv_geom(p, w.target_kv, preferred, shared), (int32_t *)(ws + w.sched_kv), w.items_kv,
-                        tables_of(w.tables_kv, w.blocks_kv, w.target_kv)};
   const bool pair = pair_backward(p, few_q && few_kv && (w.target_q == 0 || w.slots_apart));
+  const ListJob q_list{cu_q, cu_k, launched_dq_geom(p, w.target_q, pair), (int32_t *)(ws + w.sched_q), w.items_q, tables_of(w.tables_q, w.blocks_q, w.target_q)};
+  const ListJob kv_list{cu_q, cu_k, launched_dkdv_geom(p, w.target_kv, preferred, shared, pair), (int32_t *)(ws + w.sched_kv), w.items_kv,
+                        tables_of(w.tables_kv, w.blocks_kv, w.target_kv)};
   RowStats stats{};
   if (pair) stats = RowStats{(const uint8_t *)dout, (const uint8_t *)out, a.lse_tok, a.lse, a.qs_task_off, a.qs_tok_bytes, a.hq, a.total_q, kElemF16, a.lse2_w, a.dscaled_w};
   rc = launch_build_backward(kv_list, q_list, kv_off, p->num_tasks, BwdFill{(uint8_t *)dk, (uint8_t *)dv, (int64_t)p->num_heads_kv * kHeadDim * 2, p->total_k, shards}, stats, s);

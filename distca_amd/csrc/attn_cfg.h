@@ -87,6 +87,7 @@ inline SchedGeom fwd_geom(const distca_ca_params *p) {
   g.split_target = 0;
   g.min_piece = kMinPiece;
   g.units_per_head = g.item_cost = g.piece_extra = g.add_cost = 0;
+  g.beside = 0.f;
   g.walk_round = 0;
   g.merge_tiles = merge_short_tasks(p) ? kMergeTilesFwd : 0;
   g.rows_per_block = kFwdRows;
@@ -171,6 +172,16 @@ inline bool few_row_blocks(const distca_ca_params *p) {
 // unit 8192 at 32/8 1404 / 1354, 32768 at 8/2 5276 / 5123, 2 x 4096 at 32/8 764 / 771 (blocks that pack exactly); at 5 10000 at 32/8 2040 / 2010, 40000 at
 // 8/2 7929 / 7718; at 6 12000 at 32/8 2772 / 2821, at 8 4 x 4000 at 32/8 1329 / 1364.
 constexpr int kPairBlocksPerCU = 5;
+// What either list's items take of the other's time: 256 rows by 64 keys of dQ 2.1 us, the same area as two blocks of dK/dV at 1.35, hence 0.78 of
+// dQ's beside dK/dV and 1.28 the other way round; somewhat less packs better (sched.h, pieces_time; dQ's blocks of one document that has few of them in
+// smaller pieces).
+constexpr float kDqBesideDkdv = 0.7f, kDkdvBesideDq = 0.68f;
+constexpr int32_t kMinPieceBeside = 11;   // of dK/dV (8 in its place: 1024 tokens at 8/2 heads 56 us for 54, 14: 1100 56 for 54)
+// Whether the slots of both kernels' pieces lie side by side, as they have to where both are written at a time: within what a preferred workspace has at
+// most for slots.
+inline bool slots_apart(const distca_ca_params *p, int64_t blocks_kv, int32_t target_kv, int64_t blocks_q, int32_t target_q) {
+  return (split_max_slots(blocks_kv, target_kv) * kDkdvSlotBytes + split_max_slots(blocks_q, target_q) * kDqSlotBytes) * p->num_heads_kv <= 1024 * kDkdvSlotBytes;
+}
 inline bool pair_backward(const distca_ca_params *p, bool possible) {
   return possible && (int64_t)p->total_q * p->num_heads_q <= (int64_t)kPairBlocksPerCU * kDqRows * num_compute_units();
 }
@@ -242,6 +253,7 @@ inline SchedGeom bwd_geom(const distca_ca_params *p) {
   g.split_target = bwd_split_target(p);
   g.min_piece = kMinPiece;
   g.units_per_head = g.item_cost = g.piece_extra = g.add_cost = 0;
+  g.beside = 0.f;
   // one round of the dK/dV list per kv head: as many items as compute units serve that head (sched.h, kWalkUp)
   g.walk_round = num_compute_units() / p->num_heads_kv > 0 ? num_compute_units() / p->num_heads_kv : 1;
   return g;
@@ -253,16 +265,19 @@ inline SchedGeom launched_fwd_geom(const distca_ca_params *p, int32_t target) {
   if (target > 0) cut_where_worth(&g, p, target, 6, 4, 8);
   return g;
 }
-inline SchedGeom launched_dq_geom(const distca_ca_params *p, int32_t target) {
+inline SchedGeom launched_dq_geom(const distca_ca_params *p, int32_t target, bool beside) {
   SchedGeom g = launched_geom(dq_geom(p), p);
   if (target > 0) cut_where_worth(&g, p, target, 6, 3, 6);
+  if (beside) g.beside = kDkdvBesideDq;
   return g;
 }
 inline SchedGeom bwd_shared_geom(const distca_ca_params *p);
-inline SchedGeom launched_dkdv_geom(const distca_ca_params *p, int32_t target, bool preferred, bool shared) {
+// beside: dQ's items share the launch (pair_backward)
+inline SchedGeom launched_dkdv_geom(const distca_ca_params *p, int32_t target, bool preferred, bool shared, bool beside) {
   SchedGeom g = shared ? bwd_shared_geom(p) : bwd_geom(p);
   g.split_target = target;
   if (target > 0 && preferred) cut_where_worth(&g, p, target, 9, 14, 4);
+  if (beside) g.beside = kDqBesideDkdv, g.min_piece = kMinPieceBeside;
   if (shared && target > 0) g.walk_round = 0;   // pieces count a group's visits downwards
   return g;
 }

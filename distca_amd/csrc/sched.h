@@ -32,6 +32,7 @@ struct SchedGeom {
                            // (see piece_count)
   int32_t min_piece;       // the least cost of a piece
   int32_t units_per_head;  // > 0: cut only where it is worth it (worth_cutting), for so many compute units per kv head
+  float beside;            // what another list's items, launched together with this one's and behind them, add to a unit's load, as a share of this list's
   int32_t item_cost, piece_extra, add_cost;  // with units_per_head: what an item costs beside its blocks' cost, what a piece adds to
                                              // that, and what adding the pieces up takes when there are any
   int32_t walk_round;      // backward only, 0 = off: items whose rank in the list is in an odd group of this many
@@ -114,11 +115,17 @@ DISTCA_HD void piece_range(int32_t n, int32_t j, int32_t k, int32_t size, int32_
 // what is left over of the blocks fills the gaps, to about a quarter of a piece.
 // (8192 tokens in two documents, 32/8 heads: the forward's four blocks per unit even out, 287 us of 276 possible, and are left whole;
 // the dK/dV list's 34 key blocks for 32 units are cut, 939 -> 600 us with the adding up.)
+// Where another list's items follow in the same launch (`beside`, attn_bwd_pair.hip) the load is both lists', and what a piece leaves of it they fill:
+// blocks are cut only where they outlast both, into larger pieces, sizes of load, load / 1.5, load / 2, ... are tried, and a few per cent are worth
+// it.  us backward, cut as if alone / so: 1000 tokens at 32/8 heads 75 / 61, 2048 at 8/2 90 / 69, at 32/8 149 / 131, 6000 + 2192 at 32/8 906 / 858, 20 x 300
+// at 8/2 76 / 58, 3000 at 64/8 424 / 407; a set of 24 batches 7.6 % in the geometric mean, none slower by more than 0.2 % (with a tail of 0.1 of a piece and
+// a share of 0.6 for what is beside 3.7 %, without a tail and 0.78 up to 4 % slower at 4/1 heads).
 constexpr int kPieceTries = 8;
+constexpr float kTailAlone = 0.25f, kTailBeside = 0.045f;   // of a piece, by which units end apart
 // The longest a unit works when blocks stay whole, and with pieces of load / m (whose size goes to *size).
 DISTCA_HD float whole_time(const SchedGeom &g, float total_cost, int32_t n, const int32_t c[4]) {
   const float per_unit = 1.f / (float)g.units_per_head, item = (float)g.item_cost;
-  float t = (total_cost + item * (float)n) * per_unit;
+  float t = (total_cost * (1.f + g.beside) + item * (float)n) * per_unit;
   for (int k = 0; k < 4; ++k) {
     const float w = c[k] > 0 ? (float)(k + 1) * ((float)c[k] + item) : 0.f;
     t = w > t ? w : t;
@@ -128,13 +135,15 @@ DISTCA_HD float whole_time(const SchedGeom &g, float total_cost, int32_t n, cons
 DISTCA_HD float pieces_time(const SchedGeom &g, float total_cost, int32_t n, int32_t longest, int32_t least, int m, int32_t *size) {
   const float per_unit = 1.f / (float)g.units_per_head, piece = (float)(g.item_cost + g.piece_extra);
   const float load = total_cost * per_unit + 0.5f * piece * (float)n * per_unit;
-  int32_t s = (int32_t)(load / (float)m) + 1;
+  const float all = load + g.beside * total_cost * per_unit;
+  int32_t s = (int32_t)(all / (g.beside > 0.f ? 0.5f * (float)(m + 1) : (float)m)) + 1;
   s = s < least ? least : s;
   s = s < longest / (kMaxPieces - 8) ? longest / (kMaxPieces - 8) : s;
   *size = s;
-  return load + piece * (total_cost * per_unit / (float)s) + 0.25f * (float)s + (float)(g.piece_extra + g.add_cost);
+  return all + piece * (total_cost * per_unit / (float)s) + (g.beside > 0.f ? kTailBeside : kTailAlone) * (float)s + (float)(g.piece_extra + g.add_cost);
 }
-constexpr float kWorthCutting = 0.93f;   // cut when the pieces' time is below this share of the whole blocks'
+// cut when the pieces' time is below this share of the whole blocks'
+DISTCA_HD float worth_cutting(const SchedGeom &g) { return g.beside > 0.f ? 0.98f : 0.93f; }
 // The size chosen, 0: blocks stay whole (the host mirror; the builder tries the sizes in as many lanes).
 inline int32_t fixed_piece_size(const SchedGeom &g, unsigned long long total_cost, int32_t n, const int32_t c[4], int32_t least) {
   float best = 0.f;
@@ -144,7 +153,7 @@ inline int32_t fixed_piece_size(const SchedGeom &g, unsigned long long total_cos
     const float t = pieces_time(g, (float)total_cost, n, c[0], least, m, &s);
     if (size == 0 || t < best || (t == best && s > size)) best = t, size = s;
   }
-  return best < kWorthCutting * whole_time(g, (float)total_cost, n, c) ? size : 0;
+  return best < worth_cutting(g) * whole_time(g, (float)total_cost, n, c) ? size : 0;
 }
 
 constexpr int kSchedBins = 4096;

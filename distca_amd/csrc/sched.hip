@@ -220,7 +220,7 @@ __device__ __forceinline__ void build_list(ListScratch &s, const Units &u, int32
         const int32_t so = __shfl_xor(size, off, 64);
         if (to < t || (to == t && so > size)) t = to, size = so;
       }
-      if (tid == 0) s.piece = t < kWorthCutting * whole_time(g, (float)s.total_cost, nitems, s.ranked) ? size : 0;
+      if (tid == 0) s.piece = t < worth_cutting(g) * whole_time(g, (float)s.total_cost, nitems, s.ranked) ? size : 0;
     }
     __syncthreads();
     piece = s.piece;
@@ -582,10 +582,13 @@ struct LaunchedList {
   int64_t max_blocks;
 };
 LaunchedList launched_list(int kind, const distca_ca_params *p) {
-  if (kind == 1) return {launched_dkdv_geom(p, preferred_key_pieces(p), true, false), bwd_key_blocks_own_rows(p)};
   const int64_t blocks = kind == 0 ? fwd_max_items(p) : dq_max_items(p);
-  const int32_t target = row_split_target(p, blocks, kind == 0 ? kCutFromTilesFwd : kCutFromTilesDq);
-  return {kind == 0 ? launched_fwd_geom(p, target) : launched_dq_geom(p, target), blocks};
+  if (kind == 0) return {launched_fwd_geom(p, row_split_target(p, blocks, kCutFromTilesFwd)), blocks};
+  const int32_t target_kv = preferred_key_pieces(p), target_q = row_split_target(p, dq_max_items(p), kCutFromTilesDq);
+  const bool pair = pair_backward(p, few_row_blocks(p) && (few_key_blocks(p, kSplitFewPerCU) || target_kv > 0) &&
+                                         (target_q == 0 || slots_apart(p, bwd_key_blocks_own_rows(p), target_kv, dq_max_items(p), target_q)));
+  if (kind == 1) return {launched_dkdv_geom(p, target_kv, true, false, pair), bwd_key_blocks_own_rows(p)};
+  return {launched_dq_geom(p, target_q, pair), blocks};
 }
 }  // namespace
 
