@@ -80,8 +80,9 @@ int launch_dkdv64_f16(const BwdArgs &a, int64_t grid, bool few, int64_t max_cut,
 // ... and of what adds the pieces of at most max_cut key blocks up
 void launch_dkdv64_combine(const BwdArgs &a, int64_t max_cut, hipStream_t stream);
 void launch_dkdv64_combine_f16(const BwdArgs &a, int64_t max_cut, hipStream_t stream);
-void launch_dq64_combine(const BwdArgs &a, int64_t max_cut, hipStream_t stream);   // the same for blocks of query rows
-void launch_dq64_combine_f16(const BwdArgs &a, int64_t max_cut, hipStream_t stream);
+// the same for the pieces of both lists
+void launch_pair_combine(const BwdArgs &q, int64_t max_cut_q, const BwdArgs &kv, int64_t max_cut_kv, hipStream_t stream);
+void launch_pair_combine_f16(const BwdArgs &q, int64_t max_cut_q, const BwdArgs &kv, int64_t max_cut_kv, hipStream_t stream);
 // dQ and dK/dV in one launch, for batches of few items whose row statistics are there already (attn_bwd_pair.hip)
 int launch_pair(const BwdArgs &q, int64_t grid_q, const BwdArgs &kv, int64_t grid_kv, bool shared, hipStream_t stream);
 int launch_pair_f16(const BwdArgs &q, int64_t grid_q, const BwdArgs &kv, int64_t grid_kv, bool shared, hipStream_t stream);

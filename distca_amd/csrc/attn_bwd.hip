@@ -211,7 +211,7 @@ int DISTCA_FN(run_bwd)(const BwdQuerySide &qs, const void *k, const void *v, voi
   // ---- both work lists, and zeros where no work item writes dk / dv
   const bool few_q = few_row_blocks(p), few_kv = few_key_blocks(p, kSplitFewPerCU) || w.target_kv > 0;
   auto tables_of = [&](int64_t at, int64_t blocks, int32_t target) { return target > 0 ? split_tables(ws + at, blocks, target) : SplitTables{}; };
-  const bool pair = pair_backward(p, few_q && few_kv && (w.target_q == 0 || w.slots_apart));
+  const bool pair = pair_backward(p, few_q && few_kv && (w.target_q == 0 || (w.slots_apart && w.target_kv > 0)));
   const ListJob q_list{cu_q, cu_k, launched_dq_geom(p, w.target_q, pair), (int32_t *)(ws + w.sched_q), w.items_q, tables_of(w.tables_q, w.blocks_q, w.target_q)};
   const ListJob kv_list{cu_q, cu_k, launched_dkdv_geom(p, w.target_kv, preferred, shared, pair), (int32_t *)(ws + w.sched_kv), w.items_kv,
                         tables_of(w.tables_kv, w.blocks_kv, w.target_kv)};
@@ -260,8 +260,8 @@ int DISTCA_FN(run_bwd)(const BwdQuerySide &qs, const void *k, const void *v, voi
     if (pair) {
       rc = DISTCA_FN(launch_pair)(aq, grid_q, a, grid, shared, s);
       if (rc) return rc;
-      if (w.target_q > 0) DISTCA_FN(launch_dq64_combine)(aq, split_max_cut(w.blocks_q, w.target_q), s);
-      if (max_cut > 0) DISTCA_FN(launch_dkdv64_combine)(a, max_cut, s);
+      if (w.target_q > 0 && max_cut > 0) DISTCA_FN(launch_pair_combine)(aq, split_max_cut(w.blocks_q, w.target_q), a, max_cut, s);
+      else if (max_cut > 0) DISTCA_FN(launch_dkdv64_combine)(a, max_cut, s);
     } else {
       rc = DISTCA_FN(launch_dkdv64)(a, grid, few_kv, max_cut, shared, s);
       if (rc) return rc;

@@ -61,3 +61,39 @@ __device__ __forceinline__ void mfma16_vc(f32x4 &acc, elemx8 a, elemx8 b, const 
 // the chain from S to dK do not shrink with it).  (With the second halves in the order 3, 2, 1, 0 instead, wave 3's two lay side by side, and
 // both could lie on the diagonal at once; now only one ever does, and only its elements are compared.)
 __device__ __forceinline__ int dkdv_half_key(int wave, int half) { return kBN / 2 * half + 32 * wave; }
+
+// Adds up the pieces of the key blocks that were cut, in their order (cut_blocks.h, once for dK and once for dV: a workgroup has the keys
+// of one half of one wave).  Bound by reading the slots (256 KB a piece).
+__device__ __forceinline__ void add_up_dkdv(const BwdArgs &a, int part) {
+  const int kvh = blockIdx.y, key_wave = (part >> 1) & 3, kb = part & 1, lane = threadIdx.x & 63, db = threadIdx.x >> 6;
+  const int64_t kv_stride = (int64_t)a.hkv * kHeadDim;
+  auto gradient = [&](bool is_dv) {
+    add_up_cut_blocks(
+        a.cut,
+        [&](const int4 &e, f32x4 (&o)[4]) {
+          const f32x4 *first = reinterpret_cast<const f32x4 *>(a.partial + ((int64_t)e.w * a.hkv + kvh) * kDkdvSlotBytes);
+          add_pieces(first + ((is_dv ? 32 : 0) + 16 * kb + 4 * db) * kThreads + key_wave * 64 + lane, a.hkv * (kDkdvSlotBytes / 16), kThreads, e.z, o);
+          if (!is_dv) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) o[k][r] *= a.scale;
+          }
+        },
+        [&](const int4 &e, int r) -> elem_t * {
+          const int ks = a.grp_off ? a.grp_off[e.x] : (a.kv_off ? a.kv_off[e.x] : a.cu_k[e.x]);
+          const int kmax = a.grp_lmax ? a.grp_lmax[e.x] : a.cu_k[e.x + 1] - a.cu_k[e.x];
+          const int key = e.y * kBN + dkdv_half_key(key_wave, kb) + r;
+          if (key >= kmax) return nullptr;
+          elem_t *out = is_dv ? a.dv : a.dk;
+          int64_t row = ks + key;
+          if (a.shards.num_shards > 0) {
+            const int sh = find_shard(a.shards.row_start, a.shards.num_shards, ks + key);
+            out += (is_dv ? a.shards.dv_off[sh] : a.shards.dk_off[sh]) / 2;
+            row -= a.shards.row_start[sh];
+          }
+          return out + row * kv_stride + kvh * kHeadDim;
+        });
+  };
+  gradient(part >= kCutParts);
+}

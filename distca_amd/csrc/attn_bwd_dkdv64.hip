@@ -78,41 +78,7 @@ namespace {
 #undef DKDV_SPLIT
 #undef DKDV_NAME
 
-// Adds up the pieces of the key blocks that were cut, in their order (cut_blocks.h, once for dK and once for dV: a workgroup has the keys
-// of one half of one wave).  Bound by reading the slots (256 KB a piece).
-__global__ __launch_bounds__(kCutThreads) void ca_bwd_dkdv64_combine_kernel(BwdArgs a) {
-  const int kvh = blockIdx.y, key_wave = (blockIdx.z >> 1) & 3, kb = blockIdx.z & 1, lane = threadIdx.x & 63, db = threadIdx.x >> 6;
-  const int64_t kv_stride = (int64_t)a.hkv * kHeadDim;
-  auto gradient = [&](bool is_dv) {
-    add_up_cut_blocks(
-        a.cut,
-        [&](const int4 &e, f32x4 (&o)[4]) {
-          const f32x4 *first = reinterpret_cast<const f32x4 *>(a.partial + ((int64_t)e.w * a.hkv + kvh) * kDkdvSlotBytes);
-          add_pieces(first + ((is_dv ? 32 : 0) + 16 * kb + 4 * db) * kThreads + key_wave * 64 + lane, a.hkv * (kDkdvSlotBytes / 16), kThreads, e.z, o);
-          if (!is_dv) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-#pragma unroll
-              for (int r = 0; r < 4; ++r) o[k][r] *= a.scale;
-          }
-        },
-        [&](const int4 &e, int r) -> elem_t * {
-          const int ks = a.grp_off ? a.grp_off[e.x] : (a.kv_off ? a.kv_off[e.x] : a.cu_k[e.x]);
-          const int kmax = a.grp_lmax ? a.grp_lmax[e.x] : a.cu_k[e.x + 1] - a.cu_k[e.x];
-          const int key = e.y * kBN + dkdv_half_key(key_wave, kb) + r;
-          if (key >= kmax) return nullptr;
-          elem_t *out = is_dv ? a.dv : a.dk;
-          int64_t row = ks + key;
-          if (a.shards.num_shards > 0) {
-            const int sh = find_shard(a.shards.row_start, a.shards.num_shards, ks + key);
-            out += (is_dv ? a.shards.dv_off[sh] : a.shards.dk_off[sh]) / 2;
-            row -= a.shards.row_start[sh];
-          }
-          return out + row * kv_stride + kvh * kHeadDim;
-        });
-  };
-  gradient(blockIdx.z >= kCutParts);
-}
+__global__ __launch_bounds__(kCutThreads) void ca_bwd_dkdv64_combine_kernel(BwdArgs a) { add_up_dkdv(a, blockIdx.z); }
 
 }  // namespace
 

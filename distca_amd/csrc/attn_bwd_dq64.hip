@@ -33,27 +33,7 @@ namespace {
 
 #include "attn_bwd_dq64_kernel.inc"
 
-// Adds up the pieces of the blocks that were cut, in their order (cut_blocks.h).
-__global__ __launch_bounds__(kCutThreads) void ca_bwd_dq64_combine_kernel(BwdArgs a) {
-  const int kvh = blockIdx.y, sub = blockIdx.z, lane = threadIdx.x & 63, db = threadIdx.x >> 6, G = a.group;   // sub: two of a wave, four waves
-  add_up_cut_blocks(
-      a.cut,
-      [&](const int4 &e, f32x4 (&o)[4]) {
-        const f32x4 *first = reinterpret_cast<const f32x4 *>(a.partial + ((int64_t)e.w * a.hkv + kvh) * kDqSlotBytes);
-        add_pieces(first + (16 * sub + 4 * db) * 64 + lane, a.hkv * (kDqSlotBytes / 16), 64, e.z, o);
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) o[k][r] *= a.scale;
-      },
-      [&](const int4 &e, int r) -> elem_t * {
-        const int q0 = a.cu_q[e.x], nrows = (a.cu_q[e.x + 1] - q0) * G, row = e.y * kRowsWg + 32 * sub + r;
-        if (row >= nrows) return nullptr;
-        const int tok = row / G, hg = row - tok * G;
-        return reinterpret_cast<elem_t *>(reinterpret_cast<uint8_t *>(a.dq) + (a.dq_task_off ? a.dq_task_off[e.x] : (int64_t)q0 * a.dq_tok_bytes) +
-                                          (int64_t)tok * a.dq_tok_bytes) + (kvh * G + hg) * kHeadDim;
-      });
-}
+__global__ __launch_bounds__(kCutThreads) void ca_bwd_dq64_combine_kernel(BwdArgs a) { add_up_dq(a, blockIdx.z); }
 
 }  // namespace
 

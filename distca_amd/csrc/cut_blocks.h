@@ -24,6 +24,7 @@ __device__ __forceinline__ void add_up_cut_blocks(const int32_t *cut, Add add, R
   const int4 *entries = reinterpret_cast<const int4 *>(cut + 4);
   const int n = cut[0];
   int4 e = entries[blockIdx.x];   // (asked for together with n: it has a place in the table whatever n is)
+  e.x = uniform_int(e.x), e.y = uniform_int(e.y), e.z = uniform_int(e.z), e.w = uniform_int(e.w);
   asm volatile("" : "+s"(e.x), "+s"(e.y), "+s"(e.z), "+s"(e.w));
   for (int c = blockIdx.x; c < n; c += gridDim.x) {
     if (c != (int)blockIdx.x) {
