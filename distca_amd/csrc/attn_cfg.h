@@ -11,18 +11,11 @@ namespace distca {
 
 constexpr int kHeadDim = 128;
 
-// Forward kernel: each wave owns FWD_MSUB sub-tiles of 32 flattened query rows; KV tiles of 64 keys.  One
-// sub-tile keeps a wave under 256 registers, so a compute unit holds eight waves.
-#ifndef DISTCA_FWD_MSUB
-#define DISTCA_FWD_MSUB 1
-#endif
-#ifndef DISTCA_FWD_WAVES
-#define DISTCA_FWD_WAVES 8
-#endif
-constexpr int kFwdMsub = DISTCA_FWD_MSUB;
-constexpr int kFwdWaves = DISTCA_FWD_WAVES;  // waves per workgroup of the forward kernel
-constexpr int kFwdRows = kFwdWaves * 32 * kFwdMsub;
-constexpr int kDqRows = 256;  // the dQ kernel: four waves of two 32-row sub-blocks
+// Forward kernel: each wave owns 32 flattened query rows, two sub-blocks of 16; KV tiles of 64 keys.  That
+// keeps a wave under 256 registers, so a compute unit holds eight waves.
+constexpr int kFwdWaves = 8;  // waves per workgroup of the forward kernel
+constexpr int kFwdRows = kFwdWaves * 32;
+constexpr int kDqRows = 256;  // the dQ kernel: four waves of four 16-row sub-blocks
 constexpr int kFwdKV = 64;
 
 // dK/dV kernel: a workgroup owns 256 keys (four waves of 64, one per SIMD); query rows are streamed in blocks of

@@ -1,4 +1,4 @@
-// Varlen causal flash-attention forward for gfx950 (wave64, bf16 MFMA 32x32x16).
+// Varlen causal flash-attention forward for gfx950 (wave64, MFMA 16x16x32).
 //
 // Stands where the reference calls flash-attn's varlen forward
 // (distca/runtime/megatron/ops/fused_comm_attn.py:151-197).
@@ -12,15 +12,22 @@
 // through the vector memory unit, whose throughput (about 64 bytes per clock per compute unit)
 // is what a 128-row workgroup ran into.
 //
-// Per wave: MSUB sub-tiles of 32 rows.  Scores are produced transposed, S^T = K Q^T, so a
-// lane holds one query row (column lane%32) and 16 keys per 32x32 block: the online-softmax
-// row reductions are in-register plus one lane-pair exchange, and the fp32 accumulator
-// registers are, after conversion to bf16, already laid out as the B operand of
+// Per wave: 32 rows, two sub-blocks of 16, so that every K or V fragment read from LDS feeds two MFMAs.  Scores are produced transposed,
+// S^T = K Q^T, so a lane holds one query row of each sub-block (column lane%16) and 4 keys per 16x16 block: the online-softmax
+// row reductions are in-register plus an exchange among four lanes, and the fp32 accumulator
+// registers of two blocks are, after conversion, already laid out as the B operand of
 // O^T += V^T P^T.  Q stays in registers for the whole KV loop; K is read from LDS row-major
 // (16-byte reads), V through the transposing LDS read.
 //
+// 16x16x32 MFMAs rather than 32x32x16: long prefixes are bound by power, and a FLOP of theirs moves half the accumulator bytes.  They leave fewer issue
+// slots beside them (two vector instructions each, for five beside the larger one), and the softmax of a SIMD's other wave, some 120 vector instructions per 64
+// MFMAs, does not fit: 131072 packed tokens went from 83 % of the pipe's cycles at 1.47 GHz to 70 % at 1.75.  us before -> after: those at 32/8 heads
+// 12 150 -> 11 640, 8192 tokens 264 -> 254, a tick of 16384 tokens 1 339 -> 1 285, a lightly loaded server 261 -> 253, documents of 128 to 2048 tokens
+// 920 -> 907, three documents (4096 tokens) 69.4 -> 68.8.  (Operands six steps ahead instead of four: 1 % slower; either half's waves at a higher
+// priority: 1 to 2 % slower.)
+//
 // K/V tiles go from global memory straight into LDS (LDS-direct loads, four 256-byte rows per
-// instruction, rows unpadded with swizzled 16-byte chunks, see tile_swz), one period ahead of
+// instruction, rows unpadded with swizzled 16-byte chunks, see tile_swz16), one period ahead of
 // their use.
 #include <type_traits>
 #include <mutex>
@@ -35,19 +42,19 @@
 namespace distca {
 namespace {
 
-constexpr int kRowB = 256;    // bytes per K or V row in LDS (unpadded; chunk c of row r sits at c ^ tile_swz(r))
+constexpr int kRowB = 256;    // bytes per K or V row in LDS (unpadded; chunk c of row r sits at c ^ tile_swz16(r))
 constexpr int kKTile = kFwdKV * kRowB;
 constexpr int kVTile = kFwdKV * kRowB;
 constexpr int kKOff = 0, kVOff = 2 * kKTile;  // two K stages, then two V stages
 // Behind the tiles the rows of Q on their way in, 8 KB of a wave's own, and half rows of O on their way out, 4 KB (see the epilogue); at 256
 // registers a wave the workgroup has its compute unit, and its LDS, to itself anyway.
 constexpr int kQOff = 2 * kKTile + 2 * kVTile, kQWave = 32 * kRowB;
-constexpr int kOutOff = kQOff + kFwdWaves * kFwdMsub * kQWave, kOutWave = 32 * kRowB / 2;
-constexpr int kFwdLds = kOutOff + kFwdWaves * kFwdMsub * kOutWave;
+constexpr int kOutOff = kQOff + kFwdWaves * kQWave, kOutWave = 32 * kRowB / 2;
+constexpr int kFwdLds = kOutOff + kFwdWaves * kOutWave;
 static_assert(kFwdLds <= 160 * 1024, "LDS of a compute unit");
 constexpr int kDirectTasks = 256;    // batches without a list: at most so many tasks to look through
 constexpr int kRankTasks = 64;       // ... or to find the block of a rank among
-constexpr int kOutStores = 2 * 32 / 8;   // store instructions of a sub-block's rows
+constexpr int kOutStores = 2 * 32 / 8;   // store instructions of a wave's rows
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
@@ -59,6 +66,20 @@ __device__ __forceinline__ void wait_vm_known() {
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt(0x0f70 | N);  // vmcnt(N), nothing of the other counters
   asm volatile("" ::: "memory");
+}
+
+// The MFMAs as assembly, their sums in place: of the builtin's, whose result need not be where C was, the compiler moves the accumulators round the
+// registers, spills in the MERGE kernels (documents of 128 to 2048 tokens 8 % slower) and spaces LDS reads from MFMAs that still read what they overwrite.  It does not
+// space these from the vector instructions that read their results: settle() does.
+__device__ __forceinline__ void mfma16_in(f32x4 &acc, elemx8 a, elemx8 b) {  // acc += A B
+  asm volatile(DISTCA_MFMA16_ASM " %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void mfma16_in0(f32x4 &acc, elemx8 a, elemx8 b) {  // acc = A B
+  asm volatile(DISTCA_MFMA16_ASM " %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b));
+}
+// What reads these sums stands behind it, eight wait states and more after the MFMA that made them.
+__device__ __forceinline__ void settle(f32x4 (&x)[4][2]) {
+  asm volatile("s_nop 7" : "+v"(x[0][0]), "+v"(x[0][1]), "+v"(x[1][0]), "+v"(x[1][1]), "+v"(x[2][0]), "+v"(x[2][1]), "+v"(x[3][0]), "+v"(x[3][1]));
 }
 
 struct FwdArgs {
@@ -169,8 +190,8 @@ __device__ __forceinline__ int4 block_of_rank(const int32_t *cu_q, const int32_t
 // other; otherwise it is one block.
 // SPLIT (batches of few blocks): a work item may be a piece of a block, a range of its KV tiles (sched.h, piece_count), whose result
 // goes to a slot; items are taken by workgroup id.
-template <int MSUB, bool SEG, bool MERGE, bool SPLIT>
-__global__ __launch_bounds__(kFwdWaves * 64, (MSUB == 1 && kFwdWaves == 4 ? 2 : 1)) void ca_fwd_kernel(FwdArgs a) {
+template <bool SEG, bool MERGE, bool SPLIT>
+__global__ __launch_bounds__(kFwdWaves * 64, 1) void ca_fwd_kernel(FwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   int item, kvh;
   int4 it;
@@ -198,7 +219,7 @@ __global__ __launch_bounds__(kFwdWaves * 64, (MSUB == 1 && kFwdWaves == 4 ? 2 : 
   const int G = a.group;
   int shift = lk - lq;
 
-  constexpr int kRows = kFwdWaves * 32 * MSUB;
+  constexpr int kRows = kFwdRows;
   const int nrows = lq * G;
   // the blocks of this item
   int mb_first = it.y, mb_end = it.y + 1;
@@ -213,7 +234,7 @@ __global__ __launch_bounds__(kFwdWaves * 64, (MSUB == 1 && kFwdWaves == 4 ? 2 : 
   // kernel that takes one block per item)
   int mblk = mb_first;
   // MERGE: the Q rows and the first K tile of a block are requested while the block before it finishes (below)
-  elemx8 qf[MSUB][8];
+  elemx8 qf[2][4];
   bool requested = false, first_made = true;
 next_block:
   // MERGE: the thread index is made opaque once per block, so that what derives from it (the lanes' LDS and global
@@ -223,7 +244,7 @@ next_block:
   int tid_ = threadIdx.x;
   if constexpr (MERGE) asm volatile("" : "+v"(tid_));
   const int tid = tid_, lane = tid & 63, wave = tid >> 6;
-  const int l32 = lane & 31, g = lane >> 5;
+  const int l32 = lane & 31, c16 = lane & 15, g4 = lane >> 4;
   const int row_wg = mblk * kRows;
   auto div_group = [&](int n) { return a.group_magic ? (int)__umulhi((uint32_t)n, a.group_magic) : n; };
 
@@ -245,24 +266,20 @@ next_block:
     shift -= tile0 * kFwdKV;
   }
 
-  // ---- per-lane rows
+  // ---- per-lane rows: row l32 of the wave where the results are stored, rows c16 and 16 + c16 in the MFMAs' operands and accumulators
   const uint8_t *qbytes = reinterpret_cast<const uint8_t *>(a.q) + uniform_int64(a.q_task_off ? a.q_task_off[task] : (int64_t)q0 * a.q_tok_bytes);
   uint8_t *obytes = reinterpret_cast<uint8_t *>(a.out) + uniform_int64(a.out_task_off ? a.out_task_off[task] : (int64_t)q0 * a.out_tok_bytes);
-  int row[MSUB], tok[MSUB], lim[MSUB];
-  bool valid[MSUB];
-#pragma unroll
-  for (int m = 0; m < MSUB; ++m) {
-    row[m] = row_wg + (wave * MSUB + m) * 32 + l32;
-    valid[m] = row[m] < nrows;
-    tok[m] = row[m] / G;
-    int lm = a.causal ? tok[m] + shift : lk - 1;
+  int lim[2];   // the last key that the row sees
+  {
+    int lm = a.causal ? (row_wg + wave * 32 + l32) / G + shift : lk - 1;
     if (lm > lk - 1) lm = lk - 1;
-    lim[m] = lm;
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) lim[rb] = __shfl(lm, 16 * rb + c16, 64);
   }
   // wave-uniform limits: first row's limit decides whether a tile needs masking, last row's
   // whether the wave has anything to do in it.
-  const int wrow0 = row_wg + wave * MSUB * 32;
-  int wrow1 = wrow0 + MSUB * 32 - 1;
+  const int wrow0 = row_wg + wave * 32;
+  int wrow1 = wrow0 + 31;
   if (wrow1 > nrows - 1) wrow1 = nrows - 1;
   const bool wave_live = wrow0 < nrows;
   int lim_first = 0x7fffffff, lim_last = -1;
@@ -279,29 +296,27 @@ next_block:
   const uint32_t lds0 = (uint32_t)(uintptr_t)(DISTCA_LDS uint8_t *)lds;
   const int uwave = __builtin_amdgcn_readfirstlane(wave);
   // ---- Q: the wave's rows of the block whose first row is row0 come through LDS, four whole rows per instruction (a row past the task: the last
-  // one again; nothing of it is stored), and each lane takes its fragments from there (B operand of S^T = K Q^T: row l32, d = 16*s + 8*g .. +7).
+  // one again; nothing of it is stored), and each lane takes its fragments from there (B operand of S^T = K Q^T: row 16*rb + c16, d = 32*s + 8*g4 .. +7).
   // Loaded straight into that layout, an instruction touched 32 rows, and the address unit takes about a cycle for every line: of a 30 us block
   // of short documents these loads took one and a half.  us before -> after: documents of 128 to 2048 tokens (65536) 924 -> 881, three documents
   // (4096) 71.4 -> 69.8, 8192 tokens 270 -> 265, 389 tokens at 4/1 heads 15.7 -> 14.8, 131072 packed tokens 11 960 -> 11 920.
   auto request_q = [&](int row0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int m = 0; m < MSUB; ++m)
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int rl = 4 * i + (lane >> 4);
-        int r = row0 + (uwave * MSUB + m) * 32 + rl;
-        if (r > nrows - 1) r = nrows - 1;
-        const int t = div_group(r);
-        const uint8_t *src = qbytes + (int64_t)t * a.q_tok_bytes + (kvh * G + (r - t * G)) * (kHeadDim * 2) + (((lane & 15) ^ tile_swz(rl)) << 4);
-        lds_direct_load16_ptr(src, lds0 + kQOff + (uwave * MSUB + m) * kQWave + 4 * i * kRowB);
-      }
+    for (int i = 0; i < 8; ++i) {
+      const int rl = 4 * i + (lane >> 4);
+      int r = row0 + uwave * 32 + rl;
+      if (r > nrows - 1) r = nrows - 1;
+      const int t = div_group(r);
+      const uint8_t *src = qbytes + (int64_t)t * a.q_tok_bytes + (kvh * G + (r - t * G)) * (kHeadDim * 2) + (((lane & 15) ^ tile_swz16(rl)) << 4);
+      lds_direct_load16_ptr(src, lds0 + kQOff + uwave * kQWave + 4 * i * kRowB);
+    }
   };
   auto take_q = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int m = 0; m < MSUB; ++m)
+    for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
-      for (int s = 0; s < 8; ++s)
-        qf[m][s] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(lds0 + kQOff + (uwave * MSUB + m) * kQWave + l32 * kRowB + (((2 * s + g) ^ tile_swz(l32)) << 4)));
+      for (int s = 0; s < 4; ++s)
+        qf[rb][s] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(lds0 + kQOff + uwave * kQWave + (16 * rb + c16) * kRowB + (((4 * s + g4) ^ tile_swz16(c16)) << 4)));
   };
   if constexpr (!MERGE) request_q(row_wg);
   const elem_t *kbase = a.k + (SEG ? 0 : (int64_t)ks * kv_stride) + kvh * kHeadDim;
@@ -319,7 +334,7 @@ next_block:
     for (int i = 0; i < kLdW; ++i) {
       const int r = kRowsW * uwave + 4 * i + (lane >> 4);
       const int key = j * kFwdKV + r;
-      const int chunk = (lane & 15) ^ tile_swz(r);
+      const int chunk = (lane & 15) ^ tile_swz16(r);
       const elem_t *src;
       if constexpr (SEG) {
         src = reinterpret_cast<const elem_t *>(reinterpret_cast<const uint8_t *>(base) +
@@ -337,7 +352,7 @@ next_block:
 #pragma unroll
   for (int i = 0; i < kLdW; ++i) {
     const int r = kRowsW * uwave + 4 * i + (lane >> 4);
-    voff[i] = (uint32_t)((r * kv_stride + (((lane & 15) ^ tile_swz(r)) * 8)) * 2);
+    voff[i] = (uint32_t)((r * kv_stride + (((lane & 15) ^ tile_swz16(r)) * 8)) * 2);
   }
   auto issue_rows_fast = [&](const elem_t *tb, uint32_t tile_off) {
 #pragma unroll
@@ -373,165 +388,168 @@ next_block:
   auto issue_k = [&](int j) __attribute__((always_inline)) { issue_kv(kbase, j, kKOff + (j & 1) * kKTile, krun, kcur, 0); };
   auto issue_v = [&](int j) __attribute__((always_inline)) { issue_kv(vbase, j, kVOff + (j & 1) * kVTile, vrun, vcur, 1); };
 
-  // ---- accumulators
-  f32x16 oacc[MSUB][4];
-  float m_run[MSUB], l_run[MSUB];
+  // ---- accumulators: a lane has column c16 of each, O^T: d = 16 db + 4 g4 + r, S^T: key 16 kb + 4 g4 + r
+  f32x4 oacc[2][4][2];   // [db / 4][db % 4][rb]
+  float m_run[2], mc_run[2], l_run[2];   // a row's reference, -c of it (infinity: there is none), and the lane's share of the sum
 #pragma unroll
-  for (int m = 0; m < MSUB; ++m) {
+  for (int rb = 0; rb < 2; ++rb) {
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) oacc[m][db][r] = 0.f;
-    m_run[m] = -INFINITY;
-    l_run[m] = 0.f;
+    for (int db = 0; db < 8; ++db) oacc[db >> 2][db & 3][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    m_run[rb] = -INFINITY;
+    mc_run[rb] = INFINITY;
+    l_run[rb] = 0.f;
   }
   const float c = a.scale * kLog2e;
   constexpr float kLazy = 8.f, kRedo = 32.f * 256.f;
 
   // LDS read offsets (bytes) that do not depend on the tile
-  const int k_rd = l32 * kRowB + ((g ^ tile_swz(l32)) << 4);  // + kb*32*kRowB, ^ 32*s
-  // transposed V operand: lane points at (key 4g + i4 [+8 hi +16 t], chunk 8 b4 + h1 [+2 db], half lane&1);
-  // tile_swz of that row is (i4<<1) | (g<<3) | hi
-  const int i4 = (lane & 15) >> 2, b4 = (lane >> 4) & 1, h1 = (lane & 3) >> 1;
-  const int v_rd = (4 * g + i4) * kRowB + ((((b4 ^ g) << 3) | (i4 << 1) | h1) << 4) + 8 * (lane & 1);  // ^ 32*db ^ 16*hi
+  const int k_rd = c16 * kRowB + ((g4 ^ tile_swz16(c16)) << 4);  // + kb*16*kRowB, ^ 64*s
+  // transposed V operand: lane points at (key 4 g4 + i4 [+ 16], chunk h1 [+ 2 db], half lane & 1)
+  const int i4 = (lane & 15) >> 2, h1 = (lane & 3) >> 1;
+  const int v_rd = (4 * g4 + i4) * kRowB + ((h1 ^ tile_swz16(4 * g4 + i4)) << 4) + 8 * (lane & 1);  // ^ 32*db
 
-  // Absolute LDS addresses of this lane's operand reads in stage 0, the eight swizzled variants of each,
+  // Absolute LDS addresses of this lane's operand reads in stage 0, the swizzled variants of each,
   // kept in registers: with the stage and the row block in the instruction's offset field, no address
   // arithmetic is left between the MFMAs.
-  uint32_t k_ad[8], v_ad[8];
+  uint32_t k_ad[4], v_ad[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    k_ad[i] = lds0 + kKOff + (k_rd ^ (i << 5));
-    v_ad[i] = lds0 + kVOff + (v_rd ^ ((i & 3) << 5) ^ ((i >> 2) << 4));
-    asm volatile("" : "+v"(k_ad[i]), "+v"(v_ad[i]));
+    v_ad[i] = lds0 + kVOff + (v_rd ^ (i << 5));
+    asm volatile("" : "+v"(v_ad[i]));
+    if (i < 4) {
+      k_ad[i] = lds0 + kKOff + (k_rd ^ (i << 6));
+      asm volatile("" : "+v"(k_ad[i]));
+    }
   }
-  f32x16 sacc[MSUB][2];
-  elemx8 pf[MSUB][4];
+  f32x4 sacc[4][2];
+  elemx8 pf[2][2];
   auto tile_active = [&](int j) { return wave_live && j * kFwdKV <= lim_last; };
   auto nothing = [](auto...) {};
   using None = std::integral_constant<int, -1>;
 
-  // ---- S^T = K Q^T : [64 keys] x [32*MSUB rows]
-  constexpr int kPf = 2;  // K fragments are requested kPf steps before the MFMAs that use them
-  elemx8 kf[kPf][2];
-  auto load_k = [&](auto par, int s) __attribute__((always_inline)) {  // par: parity of the tile, known at compile time
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) kf[s % kPf][kb] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(k_ad[s] + decltype(par)::value * kKTile + kb * 32 * kRowB));
+  // ---- S^T = K Q^T : [64 keys] x [32 rows]
+    constexpr int kPf = 4;  // K fragments are requested kPf steps, of two MFMAs each, before the MFMAs that use them
+  elemx8 kf[kPf];
+  auto load_k = [&](auto par, int f) __attribute__((always_inline)) {  // par: parity of the tile, known at compile time; f = 4*s + kb
+    kf[f % kPf] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(k_ad[f >> 2] + decltype(par)::value * kKTile + (f & 3) * 16 * kRowB));
   };
   auto first_k = [&](auto par) __attribute__((always_inline)) {
 #pragma unroll
-    for (int s = 0; s < kPf; ++s) load_k(par, s);
+    for (int f = 0; f < kPf; ++f) load_k(par, f);
   };
   // (the first fragments have been asked for; all_read() is called ahead of the last MFMAs, which need the last of them)
   auto phase_s = [&](auto par, auto all_read) __attribute__((always_inline)) {
 #pragma unroll
-    for (int m = 0; m < MSUB; ++m)
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) sacc[m][kb][r] = 0.f;
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
+    for (int f = 0; f < 16; ++f) {
       __builtin_amdgcn_sched_barrier(0);
-      if (s == 7) all_read();
+      if (f == 14) all_read();
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int m = 0; m < MSUB; ++m) sacc[m][kb] = mfma32(kf[s % kPf][kb], qf[m][s], sacc[m][kb]);
+      for (int rb = 0; rb < 2; ++rb) {
+        if (f < 4) mfma16_in0(sacc[f][rb], kf[f % kPf], qf[rb][0]);
+        else mfma16_in(sacc[f & 3][rb], kf[f % kPf], qf[rb][f >> 2]);
+      }
       __builtin_amdgcn_sched_barrier(0);
-      if (s + kPf < 8) load_k(par, s + kPf);
+      if (f + kPf < 16) load_k(par, f + kPf);
     }
+    settle(sacc);
   };
-  // ---- mask, online softmax (log2 domain, one query row per lane pair), P as bf16 B operand
+  // ---- mask, online softmax (log2 domain, a query row on four lanes), P as B operand
   auto phase_x = [&](int j, auto whole) __attribute__((always_inline)) {  // whole: every row of the wave sees the whole tile
     const int key0 = j * kFwdKV;
     if (!decltype(whole)::value && key0 + kFwdKV - 1 > lim_first) {  // the tile straddles the diagonal or the end of the prefix
 #pragma unroll
-      for (int m = 0; m < MSUB; ++m)
+      for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
+        for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int key = key0 + kb * 32 + acc_row(r, g);
-            if (key > lim[m]) sacc[m][kb][r] = -INFINITY;
+          for (int r = 0; r < 4; ++r) {
+            const int key = key0 + 16 * kb + 4 * g4 + r;
+            if (key > lim[rb]) sacc[kb][rb][r] = -INFINITY;
           }
     }
-#pragma unroll
-    for (int m = 0; m < MSUB; ++m) {
-      // P = 2^(S c + mc) as bf16 B operand; returns this lane's share of the row sums
-      auto exp_tile = [&](float mc) __attribute__((always_inline)) {
-        float sum = 0.f;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const int kb = t >> 1, r0 = 8 * (t & 1);
-          float e[8];
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            e[i] = fast_exp2(__builtin_fmaf(sacc[m][kb][r0 + i], c, mc));
-            sum += e[i];
-          }
-          pf[m][t] = cvt8(e[0], e[1], e[2], e[3], e[4], e[5], e[6], e[7]);
-        }
-        return sum;
-      };
-      // The running reference m_run of a row need not be its maximum: any value within 2^kLazy of
-      // it gives the same O / l.  So first try the tile against the old reference, without looking
-      // for the maximum at all; only when a lane's 32 exponentials add up to more than 32 * 2^kLazy
-      // (or the row has no reference yet) is the maximum taken, the row rescaled if it moved by
-      // more than 2^kLazy, and the tile done again.
-      bool exact = __any(m_run[m] == -INFINITY);
+    // P = 2^(S c + mc) as B operand: slots 0 .. 3 of lane group g4 are keys 4 g4 .. +3 of a block of 16, slots 4 .. 7 those of the next; returns
+    // this lane's share of the row sums
+    auto exp_tile = [&](int rb, float mc) __attribute__((always_inline)) {
       float sum = 0.f;
-      if (!exact) {
-        sum = exp_tile(-m_run[m] * c);
-        exact = __any(sum > kRedo);
-      }
-      if (exact) {
-        float mx = sacc[m][0][0];
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
+      for (int t = 0; t < 2; ++t) {
+        float e[8];
 #pragma unroll
-          for (int r = 0; r < 16; ++r) mx = __builtin_fmaxf(mx, sacc[m][kb][r]);
-        mx = pair_max(mx);
-        const float m_new = __builtin_fmaxf(m_run[m], mx);
-        if (__any((m_new - m_run[m]) * c > kLazy)) {
-          const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-          const float alpha = fast_exp2((m_run[m] - m_use) * c);
-          l_run[m] *= alpha;
-#pragma unroll
-          for (int db = 0; db < 4; ++db)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) oacc[m][db][r] *= alpha;
-          m_run[m] = m_new;
+        for (int i = 0; i < 8; ++i) {
+          e[i] = fast_exp2(__builtin_fmaf(sacc[2 * t + (i >> 2)][rb][i & 3], c, mc));
+          sum = t == 0 && i == 0 ? e[0] : sum + e[i];
         }
-        sum = exp_tile((m_run[m] == -INFINITY) ? 0.f : -m_run[m] * c);
+        pf[rb][t] = cvt8(e[0], e[1], e[2], e[3], e[4], e[5], e[6], e[7]);
       }
-      l_run[m] += sum;
+      return sum;
+    };
+    // The running reference m_run of a row need not be its maximum: any value within 2^kLazy of
+    // it gives the same O / l.  So first try the tile against the old reference, without looking
+    // for the maximum at all; only when a lane's 32 exponentials do not add up to at most 32 * 2^kLazy
+    // (without a reference they add up to infinity or not at all) is the maximum taken, the rows rescaled if one moved by
+    // more than 2^kLazy, and the tile done again.
+    bool exact = !decltype(whole)::value && __any(m_run[0] == -INFINITY || m_run[1] == -INFINITY);
+    float sum[2] = {0.f, 0.f};
+    if (!exact) {
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) sum[rb] = exp_tile(rb, mc_run[rb]);
+      exact = __any(!(sum[0] + sum[1] <= kRedo));
     }
+    if (exact) {
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) {
+        float mx = sacc[0][rb][0];
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) mx = __builtin_fmaxf(mx, sacc[kb][rb][r]);
+        mx = quad_max(mx);
+        const float m_new = __builtin_fmaxf(m_run[rb], mx);
+        if (__any((m_new - m_run[rb]) * c > kLazy)) {
+          const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
+          const float alpha = fast_exp2((m_run[rb] - m_use) * c);
+          l_run[rb] *= alpha;
+#pragma unroll
+          for (int db = 0; db < 8; ++db)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) oacc[db >> 2][db & 3][rb][r] *= alpha;
+          m_run[rb] = m_new;
+          mc_run[rb] = -m_new * c;
+        }
+        sum[rb] = exp_tile(rb, (m_run[rb] == -INFINITY) ? 0.f : mc_run[rb]);
+      }
+    }
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) l_run[rb] += sum[rb];
   };
-  // ---- O^T += V^T P^T : [128 d] x [32*MSUB rows], contraction over the 64 keys
-  constexpr int kPfV = 4;  // V^T fragments are requested four MFMAs ahead
+  // ---- O^T += V^T P^T : [128 d] x [32 rows], contraction over the 64 keys
+  constexpr int kPfV = 4;  // V^T fragments are requested four steps, of two MFMAs each, ahead
   elemx4 vf[kPfV][2];
-  auto load_v = [&](auto par, int u) __attribute__((always_inline)) {  // u = 4*t + db
-    const uint32_t vo = decltype(par)::value * kVTile + 16 * (u >> 2) * kRowB;
-    vf[u % kPfV][0] = lds_read_tr(lds_ptr(v_ad[u & 3] + vo));
-    vf[u % kPfV][1] = lds_read_tr(lds_ptr(v_ad[4 + (u & 3)] + vo + 8 * kRowB));
+  auto load_v = [&](auto par, int u) __attribute__((always_inline)) {  // u = 8*t + db
+    const uint32_t vo = decltype(par)::value * kVTile + 32 * (u >> 3) * kRowB;
+    vf[u % kPfV][0] = lds_read_tr(lds_ptr(v_ad[u & 7] + vo));
+    vf[u % kPfV][1] = lds_read_tr(lds_ptr(v_ad[u & 7] + vo + 16 * kRowB));
   };
   auto first_v = [&](auto par) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < kPfV; ++u) load_v(par, u);
   };
   // (the first fragments have been asked for; next: the parity of the K tile whose first fragments to ask for, or None; beside(u) is
-  // called after MFMA u)
+  // called after the MFMAs of step u)
   auto phase_pv = [&](auto par, auto next, auto beside) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int m = 0; m < MSUB; ++m) oacc[m][u & 3] = mfma32(cat4(vf[u % kPfV][0], vf[u % kPfV][1]), pf[m][u >> 2], oacc[m][u & 3]);
+      for (int rb = 0; rb < 2; ++rb) mfma16_in(oacc[(u >> 2) & 1][u & 3][rb], cat4(vf[u % kPfV][0], vf[u % kPfV][1]), pf[rb][u >> 3]);
       __builtin_amdgcn_sched_barrier(0);
       beside(u);
       if (u + kPfV < 16) load_v(par, u + kPfV);
       else if (decltype(next)::value >= 0 && u - (16 - kPfV) < kPf) load_k(next, u - (16 - kPfV));
+    }
+    if (decltype(next)::value < 0) {
+      settle(oacc[0]);
+      settle(oacc[1]);
     }
   };
 
@@ -581,7 +599,7 @@ next_block:
   } else {
     // what came after the requests are the stores of the block before this one, whose rows all exist (others follow): they need not
     // have arrived
-    wait_vm_known<kOutStores * MSUB>();
+    wait_vm_known<kOutStores>();
     first_made = first_made || ntiles == 1;
   }
   take_q();
@@ -706,71 +724,70 @@ next_block:
 
   // (Where the results go is worked out ahead of those requests: should the compiler have parked a pointer in scratch
   // memory, fetching it back afterwards would wait for the requests as well.)
-  uint8_t *otok_m[MSUB];
-#pragma unroll
-  for (int m = 0; m < MSUB; ++m) {
-    otok_m[m] = obytes + (int64_t)tok[m] * a.out_tok_bytes;
-    if constexpr (MERGE) asm volatile("" : "+v"(otok_m[m]));
-  }
+  const int row = row_wg + wave * 32 + l32, tok = div_group(row);
+  uint8_t *otok = obytes + (int64_t)tok * a.out_tok_bytes;
+  if constexpr (MERGE) asm volatile("" : "+v"(otok));
   if constexpr (MERGE) {
     requested = more;
     first_made = ntiles > 1;
   }
 
   if constexpr (SPLIT) {
-    static_assert(MSUB == 1, "layout of a slot");
     const int slot = a.slot ? uniform_int(a.slot[2 * item]) : -1;
     if (slot >= 0) {
+      // d0 = 16 db + 4 g4 of row r of the wave at d block db % 4, quarter 2 (db / 4) + g4 / 2, lane 32 (g4 % 2) + r (cut_blocks.h)
       uint8_t *at = a.partial + ((int64_t)slot * a.hkv + kvh) * kFwdSlotBytes;
-      f32x4 *op = reinterpret_cast<f32x4 *>(at) + wave * 16 * 64 + lane;
+      f32x4 *op = reinterpret_cast<f32x4 *>(at) + wave * 16 * 64 + (g4 >> 1) * 64 + (g4 & 1) * 32 + c16;
 #pragma unroll
-      for (int db = 0; db < 4; ++db)
+      for (int db = 0; db < 8; ++db)
 #pragma unroll
-        for (int cq = 0; cq < 4; ++cq) op[(4 * db + cq) * 64] = f32x4{oacc[0][db][4 * cq], oacc[0][db][4 * cq + 1], oacc[0][db][4 * cq + 2], oacc[0][db][4 * cq + 3]};
-      const float l = pair_sum(l_run[0]);
-      if (g == 0) reinterpret_cast<f32x2 *>(at + kFwdSlotStats)[wave * 32 + l32] = f32x2{m_run[0], l};
+        for (int rb = 0; rb < 2; ++rb) op[(4 * (db & 3) + 2 * (db >> 2)) * 64 + 16 * rb] = oacc[db >> 2][db & 3][rb];
+      const float l0 = quad_sum(l_run[0]), l1 = quad_sum(l_run[1]);
+      if (lane < 32) reinterpret_cast<f32x2 *>(at + kFwdSlotStats)[wave * 32 + l32] = g4 ? f32x2{m_run[1], l1} : f32x2{m_run[0], l0};
       return;
     }
   }
 
-  // ---- epilogue: normalise, write O (bf16) and LSE (fp32, natural log).  A lane holds half of its row in pieces of 8 bytes (registers
-  // 4*cq .. 4*cq+3 of block db hold d0 .. d0+3); stored from there, an instruction touched 32 rows.  The pieces go to the wave's
+  // ---- epilogue: normalise, write O and LSE (fp32, natural log).  A lane holds a quarter of its two rows in pieces of 8 bytes (block db
+  // holds d = 16 db + 4 g4 .. +3); stored from there, an instruction touched 16 rows.  The pieces go to the wave's
   // 4 KB of LDS, half of every row at a time (Q's rows of the next block may be on their way to the other 8 KB), and leave from there in whole
   // cache lines, eight rows per instruction.
   auto store_rows = [&](auto all) __attribute__((always_inline)) {  // all: every row of the block exists
+    float l_tot[2], inv[2];
 #pragma unroll
-    for (int m = 0; m < MSUB; ++m) {
-      const float l_tot = pair_sum(l_run[m]);
-      const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-      const uint32_t out_w = lds0 + kOutOff + (uwave * MSUB + m) * kOutWave;
+    for (int rb = 0; rb < 2; ++rb) {
+      l_tot[rb] = quad_sum(l_run[rb]);
+      inv[rb] = l_tot[rb] > 0.f ? 1.f / l_tot[rb] : 0.f;
+    }
+    const uint32_t out_w = lds0 + kOutOff + uwave * kOutWave;
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {  // half rows: d = 64 h .. 64 h + 63
+    for (int h = 0; h < 2; ++h) {  // half rows: d = 64 h .. 64 h + 63
 #pragma unroll
-        for (int db = 0; db < 4; ++db)
+      for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
-          for (int cq = 2 * h; cq < 2 * h + 2; ++cq) {
-            // d0 = 16 db + 64 h + 8 (cq & 1) + 4 g: chunk 2 db + (cq & 1), half g
-            const int chunk = 2 * db + (cq & 1);
-            *static_cast<DISTCA_LDS elemx4 *>(const_cast<DISTCA_LDS void *>(lds_ptr(out_w + l32 * (kRowB / 2) + ((chunk ^ (l32 & 7)) << 4) + 8 * g))) =
-                cvt4(oacc[m][db][4 * cq] * inv, oacc[m][db][4 * cq + 1] * inv, oacc[m][db][4 * cq + 2] * inv, oacc[m][db][4 * cq + 3] * inv);
-          }
-        // (LDS operations of one wave complete in order: the reads below see the writes above, and the second half's writes come behind them)
+        for (int db = 4 * h; db < 4 * h + 4; ++db) {
+          const int chunk = 2 * (db & 3) + (g4 >> 1);   // half g4 & 1 of it
+          const f32x4 &o = oacc[h][db & 3][rb];
+          *static_cast<DISTCA_LDS elemx4 *>(const_cast<DISTCA_LDS void *>(lds_ptr(out_w + (16 * rb + c16) * (kRowB / 2) + ((chunk ^ (c16 & 7)) << 4) + 8 * (g4 & 1)))) =
+              cvt4(o[0] * inv[rb], o[1] * inv[rb], o[2] * inv[rb], o[3] * inv[rb]);
+        }
+      // (LDS operations of one wave complete in order: the reads below see the writes above, and the second half's writes come behind them)
 #pragma unroll
-        for (int i = 0; i < kOutStores / 2; ++i) {
-          const int rl = 8 * i + (lane >> 3);
-          const int r = row_wg + (uwave * MSUB + m) * 32 + rl;
-          const elemx8 o8 = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(out_w + rl * (kRowB / 2) + (((lane & 7) ^ (rl & 7)) << 4)));
-          if (decltype(all)::value || r < nrows) {
-            const int t = div_group(r);
-            *reinterpret_cast<elemx8 *>(reinterpret_cast<elem_t *>(obytes + (int64_t)t * a.out_tok_bytes) + (kvh * G + (r - t * G)) * kHeadDim + 64 * h + 8 * (lane & 7)) = o8;
-          }
+      for (int i = 0; i < kOutStores / 2; ++i) {
+        const int rl = 8 * i + (lane >> 3);
+        const int r = row_wg + uwave * 32 + rl;
+        const elemx8 o8 = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(out_w + rl * (kRowB / 2) + (((lane & 7) ^ (rl & 7)) << 4)));
+        if (decltype(all)::value || r < nrows) {
+          const int t = div_group(r);
+          *reinterpret_cast<elemx8 *>(reinterpret_cast<elem_t *>(obytes + (int64_t)t * a.out_tok_bytes) + (kvh * G + (r - t * G)) * kHeadDim + 64 * h + 8 * (lane & 7)) = o8;
         }
       }
-      if (valid[m] && g == 0) {
-        const int hg = row[m] - tok[m] * G;
-        const float lse = l_tot > 0.f ? (m_run[m] * c + fast_log2(l_tot)) * kLn2 : -INFINITY;
-        store_lse(a, otok_m[m], kvh * G + hg, q0 + tok[m], lse);
-      }
+    }
+    if (row < nrows && lane < 32) {   // lane l32 has the sums of its row as those of row g4 of the two
+      const int hg = row - tok * G;
+      const float l = g4 ? l_tot[1] : l_tot[0], m = g4 ? m_run[1] : m_run[0];
+      const float lse = l > 0.f ? (m * c + fast_log2(l)) * kLn2 : -INFINITY;
+      store_lse(a, otok, kvh * G + hg, q0 + tok, lse);
     }
   };
   if (MERGE && more) {
@@ -787,7 +804,7 @@ next_block:
 // Adds up the pieces of the blocks that were cut, in their order (cut_blocks.h; a workgroup has the rows of one wave, a lane what it held
 // in the kernel above).  Bound by reading the slots (128 KB a piece), four pieces' loads in flight at a time.
 __global__ __launch_bounds__(kCutThreads) void ca_fwd_combine_kernel(FwdArgs a) {
-  static_assert(kFwdMsub == 1 && kFwdWaves == kCutParts, "a part is a wave's rows");
+  static_assert(kFwdWaves == kCutParts, "a part is a wave's rows");
   const int kvh = blockIdx.y, wave = blockIdx.z, lane = threadIdx.x & 63, db = threadIdx.x >> 6, l32 = lane & 31, g = lane >> 5, G = a.group;
   const float c = a.scale * kLog2e;
   auto token_at = [&](const int4 &e, int r, int &tok, int &head) -> uint8_t * {  // of the output, null if there is no such row
@@ -1052,9 +1069,9 @@ int DISTCA_FN(run_fwd_tokens)(const void *q_base, const int64_t *q_task_off, int
   const int64_t grid = list_grid(p, max_items, few);
   if (grid > 0x7fffffff) return fail(DISTCA_E_INVALID, "ca_fwd: grid too large");
   if (device_setup_pending(kSlotFwdLds)) {
-    const void *kernels[] = {(const void *)ca_fwd_kernel<kFwdMsub, false, false, false>, (const void *)ca_fwd_kernel<kFwdMsub, true, false, false>,
-                             (const void *)ca_fwd_kernel<kFwdMsub, false, true, false>,  (const void *)ca_fwd_kernel<kFwdMsub, true, true, false>,
-                             (const void *)ca_fwd_kernel<kFwdMsub, false, false, true>,  (const void *)ca_fwd_kernel<kFwdMsub, true, false, true>};
+    const void *kernels[] = {(const void *)ca_fwd_kernel<false, false, false>, (const void *)ca_fwd_kernel<true, false, false>,
+                             (const void *)ca_fwd_kernel<false, true, false>,  (const void *)ca_fwd_kernel<true, true, false>,
+                             (const void *)ca_fwd_kernel<false, false, true>,  (const void *)ca_fwd_kernel<true, false, true>};
     for (const void *kf : kernels) {
       hipError_t e = hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, kFwdLds);
       if (e != hipSuccess) return fail(DISTCA_E_LAUNCH, "ca_fwd: cannot reserve %d B of LDS: %s", kFwdLds, hipGetErrorString(e));
@@ -1065,9 +1082,9 @@ int DISTCA_FN(run_fwd_tokens)(const void *q_base, const int64_t *q_task_off, int
     ScopedTimer timer(DISTCA_TIMER_CA_FWD, s);
     const dim3 g((unsigned)grid), b(kFwdWaves * 64);
     auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, b, kFwdLds, s, a); };
-    if (few) launch(kv_shards ? ca_fwd_kernel<kFwdMsub, true, false, true> : ca_fwd_kernel<kFwdMsub, false, false, true>);
-    else if (geom.merge_tiles > 0) launch(kv_shards ? ca_fwd_kernel<kFwdMsub, true, true, false> : ca_fwd_kernel<kFwdMsub, false, true, false>);
-    else launch(kv_shards ? ca_fwd_kernel<kFwdMsub, true, false, false> : ca_fwd_kernel<kFwdMsub, false, false, false>);
+    if (few) launch(kv_shards ? ca_fwd_kernel<true, false, true> : ca_fwd_kernel<false, false, true>);
+    else if (geom.merge_tiles > 0) launch(kv_shards ? ca_fwd_kernel<true, true, false> : ca_fwd_kernel<false, true, false>);
+    else launch(kv_shards ? ca_fwd_kernel<true, false, false> : ca_fwd_kernel<false, false, false>);
     if (split) hipLaunchKernelGGL(ca_fwd_combine_kernel, cut_grid(split_max_cut(lay.max_blocks, lay.target), p->num_heads_kv, kCutParts), dim3(kCutThreads), 0, s, a);
   }
   return check_launch("ca_fwd");
