@@ -562,8 +562,9 @@ next_block:
   // wave requests K(p+1) and V(p) (those of period 0 ahead of the loop: below) after b(2p), into the stages whose last readers finished
   // before it, and waits for its own requests before b(2p+2).  The MFMA halves are the critical path of a period (one
   // group's, then the other's).  A request holds its wave for a hundred cycles or so: group 1 makes its requests right after b(2p), in
-  // its softmax half; group 0 between MFMAs of PV(p-1) where it knows beforehand what to request (fast0), else behind b(2p+1) (in front
-  // of its MFMA half they showed in the period, 3 %).
+  // its softmax half; group 0 between MFMAs of PV(p-1) where it knows beforehand what to request (fast0), else behind b(2p+1), in items of
+  // short tasks, which are mostly such periods, between PV(p-1) and S(p) (documents of 64 to 512 tokens, 65536 at 32/8 heads, 511 -> 503 us; three
+  // documents, 4096 tokens, of blocks one by one 67.3 -> 67.5; in front of its MFMA half they showed in the period, 3 %).
   // The first two K tiles and the first V tile are requested together ahead of the loop, so that a block waits for memory once: with
   // K(1) and V(0) requested in period 0, as the loop has it, that period (one tile's S to cover them) lasted as long as a second trip.
   // (Together with the rows of O leaving through LDS and Q known to be there, 131072 tokens in documents of 128 / 256 / 512 / 2048, 32/8
@@ -677,13 +678,17 @@ next_block:
     using Same = std::integral_constant<int, decltype(par)::value>;
     using Other = std::integral_constant<int, 1 - decltype(par)::value>;
     if (p > 0 && tile_active(p - 1)) { first_v(Other{}); phase_pv(Other{}, None{}, nothing); }
+    auto request = [&]() __attribute__((always_inline)) {
+      if (p >= requests_from) {
+        if (p + 1 < ntiles) issue_k(p + 1);
+        if (p < ntiles) issue_v(p);
+      }
+    };
+    if constexpr (MERGE) request();
     const bool act = p < ntiles && tile_active(p);
     if (act) { first_k(Same{}); phase_s(Same{}, nothing); }
     __syncthreads();
-    if (p >= requests_from) {
-      if (p + 1 < ntiles) issue_k(p + 1);
-      if (p < ntiles) issue_v(p);
-    }
+    if constexpr (!MERGE) request();
     if (act) phase_x(p, std::false_type{});
     if (p >= requests_from) wait_vm0();
     __syncthreads();
