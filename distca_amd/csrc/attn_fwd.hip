@@ -22,8 +22,7 @@
 // 16x16x32 MFMAs rather than 32x32x16: long prefixes are bound by power, and a FLOP of theirs moves half the accumulator bytes.  They leave fewer issue
 // slots beside them (two vector instructions each, for five beside the larger one), and the softmax of a SIMD's other wave, some 120 vector instructions per 64
 // MFMAs, does not fit: 131072 packed tokens went from 83 % of the pipe's cycles at 1.47 GHz to 70 % at 1.75.  us before -> after: those at 32/8 heads
-// 12 150 -> 11 640, 8192 tokens 264 -> 254, a tick of 16384 tokens 1 339 -> 1 285, a lightly loaded server 261 -> 253, documents of 128 to 2048 tokens
-// 920 -> 907, three documents (4096 tokens) 69.4 -> 68.8.  (Operands six steps ahead instead of four: 1 % slower; either half's waves at a higher
+// 12 150 -> 11 640, 8192 tokens 264 -> 254, a tick of 16384 tokens 1 339 -> 1 285, a lightly loaded server 261 -> 253, three documents (4096 tokens) 69.4 -> 68.8.  (Operands six steps ahead instead of four: 1 % slower; either half's waves at a higher
 // priority: 1 to 2 % slower.)
 //
 // K/V tiles go from global memory straight into LDS (LDS-direct loads, four 256-byte rows per
@@ -69,7 +68,7 @@ __device__ __forceinline__ void wait_vm_known() {
 }
 
 // The MFMAs as assembly, their sums in place: of the builtin's, whose result need not be where C was, the compiler moves the accumulators round the
-// registers, spills in the MERGE kernels (documents of 128 to 2048 tokens 8 % slower) and spaces LDS reads from MFMAs that still read what they overwrite.  It does not
+// registers and spaces LDS reads from MFMAs that still read what they overwrite.  It does not
 // space these from the vector instructions that read their results: settle() does.
 __device__ __forceinline__ void mfma16_in(f32x4 &acc, elemx8 a, elemx8 b) {  // acc += A B
   asm volatile(DISTCA_MFMA16_ASM " %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
@@ -100,7 +99,7 @@ struct FwdArgs {
   int32_t *tickets;  // one counter per kv head (sched.h)
   const int64_t *q_task_off, *out_task_off;
   int64_t q_tok_bytes, out_tok_bytes;
-  int32_t merge_tiles;   // MERGE kernels: the list's merge_tiles (sched.h)
+  int32_t merge_tiles;   // merged items: the list's merge_tiles (sched.h)
   int32_t lse_in_token;  // 1: lse of (token, head) as fp32 at token + hq * 256 + h * 4 (the [out | lse] reply), 0: lse[h][token]
   KvShards shards;       // SEG kernels: k and v are the bases of a buffer that holds the stored rows shard by shard
   const int32_t *cut, *slot;  // SPLIT kernels: the tables of a list with cut blocks (sched.h, SplitTables)
@@ -186,11 +185,9 @@ __device__ __forceinline__ int4 block_of_rank(const int32_t *cu_q, const int32_t
 }
 
 // SEG: K/V rows are addressed through a table of shards (kv_shards.h) instead of as one dense tensor.
-// MERGE: a work item is several consecutive blocks of a task's query rows (sched.h, fwd_merge), worked off one after the
-// other; otherwise it is one block.
 // SPLIT (batches of few blocks): a work item may be a piece of a block, a range of its KV tiles (sched.h, piece_count), whose result
 // goes to a slot; items are taken by workgroup id.
-template <bool SEG, bool MERGE, bool SPLIT>
+template <bool SEG, bool SPLIT>
 __global__ __launch_bounds__(kFwdWaves * 64, 1) void ca_fwd_kernel(FwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   int item, kvh;
@@ -221,29 +218,9 @@ __global__ __launch_bounds__(kFwdWaves * 64, 1) void ca_fwd_kernel(FwdArgs a) {
 
   constexpr int kRows = kFwdRows;
   const int nrows = lq * G;
-  // the blocks of this item
-  int mb_first = it.y, mb_end = it.y + 1;
-  if constexpr (MERGE) {
-    SchedGeom geom;
-    geom.rows_per_block = kRows; geom.kv_per_block = kFwdKV; geom.group = G; geom.causal = a.causal; geom.merge_tiles = a.merge_tiles;
-    const int m = fwd_merge(geom, lq, lk), nblk = (nrows + kRows - 1) / kRows;
-    mb_first = it.y * m;
-    mb_end = mb_first + m < nblk ? mb_first + m : nblk;
-  }
-  // (a jump back rather than a loop statement: without MERGE the body below is then straight-line code, exactly the
-  // kernel that takes one block per item)
-  int mblk = mb_first;
-  // MERGE: the Q rows and the first K tile of a block are requested while the block before it finishes (below)
+  const int mblk = it.y;
   elemx8 qf[2][4];
-  bool requested = false, first_made = true;
-next_block:
-  // MERGE: the thread index is made opaque once per block, so that what derives from it (the lanes' LDS and global
-  // offsets, a few dozen registers) is computed afresh for every block instead of being carried, and partly spilled,
-  // across the whole body: a reload from scratch memory waits for every request in flight, those made for the next
-  // block included.
-  int tid_ = threadIdx.x;
-  if constexpr (MERGE) asm volatile("" : "+v"(tid_));
-  const int tid = tid_, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, c16 = lane & 15, g4 = lane >> 4;
   const int row_wg = mblk * kRows;
   auto div_group = [&](int n) { return a.group_magic ? (int)__umulhi((uint32_t)n, a.group_magic) : n; };
@@ -318,7 +295,7 @@ next_block:
       for (int s = 0; s < 4; ++s)
         qf[rb][s] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(lds0 + kQOff + uwave * kQWave + (16 * rb + c16) * kRowB + (((4 * s + g4) ^ tile_swz16(c16)) << 4)));
   };
-  if constexpr (!MERGE) request_q(row_wg);
+  request_q(row_wg);
   const elem_t *kbase = a.k + (SEG ? 0 : (int64_t)ks * kv_stride) + kvh * kHeadDim;
   const elem_t *vbase = a.v + (SEG ? 0 : (int64_t)ks * kv_stride) + kvh * kHeadDim;
   // SEG: the shards that hold the rows of the K tile and of the V tile requested next (the K requests run a tile ahead)
@@ -562,51 +539,24 @@ next_block:
   // wave requests K(p+1) and V(p) (those of period 0 ahead of the loop: below) after b(2p), into the stages whose last readers finished
   // before it, and waits for its own requests before b(2p+2).  The MFMA halves are the critical path of a period (one
   // group's, then the other's).  A request holds its wave for a hundred cycles or so: group 1 makes its requests right after b(2p), in
-  // its softmax half; group 0 between MFMAs of PV(p-1) where it knows beforehand what to request (fast0), else behind b(2p+1), in items of
-  // short tasks, which are mostly such periods, between PV(p-1) and S(p) (documents of 64 to 512 tokens, 65536 at 32/8 heads, 511 -> 503 us; three
-  // documents, 4096 tokens, of blocks one by one 67.3 -> 67.5; in front of its MFMA half they showed in the period, 3 %).
+  // its softmax half; group 0 between MFMAs of PV(p-1) where it knows beforehand what to request (fast0), else behind b(2p+1) (in front
+  // of its MFMA half they showed in the period, 3 %).
   // The first two K tiles and the first V tile are requested together ahead of the loop, so that a block waits for memory once: with
   // K(1) and V(0) requested in period 0, as the loop has it, that period (one tile's S to cover them) lasted as long as a second trip.
   // (Together with the rows of O leaving through LDS and Q known to be there, 131072 tokens in documents of 128 / 256 / 512 / 2048, 32/8
   // heads: 958 / 1010 / 1151 / 2798 -> 854 / 857 / 1014 / 2725 us; 131072 packed tokens 12.86 -> 12.72 ms.)
-  // MERGE: what the item's next block starts with is requested when this block's tile loop is over, so that it
-  // arrives while the results are normalised and stored: its Q rows (their place is free: every S of this block
-  // is done) and those tiles (no wave reads a stage any more: the last barrier of the loop lies behind every
-  // phase; they are the same for every block of a task).  The run and cursor objects the request goes through are
-  // set up afresh by the next block.  (Made from inside the loop's last
-  // period instead, the requests cost the loop its register allocation: six hundred spills.)
-  const bool more = MERGE && mblk + 1 < mb_end;
   auto request_first = [&](int n) __attribute__((always_inline)) {
     issue_k(0);
     issue_v(0);
     if (n > 1) issue_k(1);
   };
-  auto request_next_block = [&]() __attribute__((always_inline)) {
-    request_q(row_wg + kRows);
-    krun = vrun = Run{kbase, SEG ? 0 : lk};
-    vrun.virt = vbase;
-    if constexpr (SEG) {
-      kcur.open(a.shards, a.shards.task_shard[task]);
-      vcur = kcur;
-    }
-    request_first(ntiles);  // (of the next block's tiles, which are as many or more)
-  };
   const int grp = uwave >> 2;
-  // first_made: nothing is left of period 0's requests (else it repeats V(0), to the same place)
-  if (!MERGE || !requested) {
-    if constexpr (MERGE) request_q(row_wg);
-    if (ntiles > 0) request_first(ntiles);
-    wait_vm_known<0>();
-  } else {
-    // what came after the requests are the stores of the block before this one, whose rows all exist (others follow): they need not
-    // have arrived
-    wait_vm_known<kOutStores>();
-    first_made = first_made || ntiles == 1;
-  }
+  if (ntiles > 0) request_first(ntiles);
+  wait_vm_known<0>();
   take_q();
   // the first period that makes requests of its own (opaque: known to the compiler, it becomes a first iteration of its own, and the
   // registers of the two spill)
-  int requests_from = uniform_int(!MERGE || first_made ? 1 : 0);
+  int requests_from = 1;
   asm volatile("" : "+s"(requests_from));
   __syncthreads();  // b0
   // The period loops are unrolled by two so that the LDS stage of every operand read is a constant folded into
@@ -678,17 +628,13 @@ next_block:
     using Same = std::integral_constant<int, decltype(par)::value>;
     using Other = std::integral_constant<int, 1 - decltype(par)::value>;
     if (p > 0 && tile_active(p - 1)) { first_v(Other{}); phase_pv(Other{}, None{}, nothing); }
-    auto request = [&]() __attribute__((always_inline)) {
-      if (p >= requests_from) {
-        if (p + 1 < ntiles) issue_k(p + 1);
-        if (p < ntiles) issue_v(p);
-      }
-    };
-    if constexpr (MERGE) request();
     const bool act = p < ntiles && tile_active(p);
     if (act) { first_k(Same{}); phase_s(Same{}, nothing); }
     __syncthreads();
-    if constexpr (!MERGE) request();
+    if (p >= requests_from) {
+      if (p + 1 < ntiles) issue_k(p + 1);
+      if (p < ntiles) issue_v(p);
+    }
     if (act) phase_x(p, std::false_type{});
     if (p >= requests_from) wait_vm0();
     __syncthreads();
@@ -727,15 +673,8 @@ next_block:
   if (grp == 0) work_off(fast0, slow0);
   else work_off(fast1, slow1);
 
-  // (Where the results go is worked out ahead of those requests: should the compiler have parked a pointer in scratch
-  // memory, fetching it back afterwards would wait for the requests as well.)
   const int row = row_wg + wave * 32 + l32, tok = div_group(row);
   uint8_t *otok = obytes + (int64_t)tok * a.out_tok_bytes;
-  if constexpr (MERGE) asm volatile("" : "+v"(otok));
-  if constexpr (MERGE) {
-    requested = more;
-    first_made = ntiles > 1;
-  }
 
   if constexpr (SPLIT) {
     const int slot = a.slot ? uniform_int(a.slot[2 * item]) : -1;
@@ -755,9 +694,9 @@ next_block:
 
   // ---- epilogue: normalise, write O and LSE (fp32, natural log).  A lane holds a quarter of its two rows in pieces of 8 bytes (block db
   // holds d = 16 db + 4 g4 .. +3); stored from there, an instruction touched 16 rows.  The pieces go to the wave's
-  // 4 KB of LDS, half of every row at a time (Q's rows of the next block may be on their way to the other 8 KB), and leave from there in whole
+  // 4 KB of LDS, half of every row at a time, and leave from there in whole
   // cache lines, eight rows per instruction.
-  auto store_rows = [&](auto all) __attribute__((always_inline)) {  // all: every row of the block exists
+  {
     float l_tot[2], inv[2];
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
@@ -782,7 +721,7 @@ next_block:
         const int rl = 8 * i + (lane >> 3);
         const int r = row_wg + uwave * 32 + rl;
         const elemx8 o8 = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(out_w + rl * (kRowB / 2) + (((lane & 7) ^ (rl & 7)) << 4)));
-        if (decltype(all)::value || r < nrows) {
+        if (r < nrows) {
           const int t = div_group(r);
           *reinterpret_cast<elemx8 *>(reinterpret_cast<elem_t *>(obytes + (int64_t)t * a.out_tok_bytes) + (kvh * G + (r - t * G)) * kHeadDim + 64 * h + 8 * (lane & 7)) = o8;
         }
@@ -794,17 +733,10 @@ next_block:
       const float lse = l > 0.f ? (m * c + fast_log2(l)) * kLn2 : -INFINITY;
       store_lse(a, otok, kvh * G + hg, q0 + tok, lse);
     }
-  };
-  if (MERGE && more) {
-    request_next_block();
-    store_rows(std::true_type{});
-  } else {
-    store_rows(std::false_type{});
-  }
-  if constexpr (MERGE) {
-    if (++mblk < mb_end) goto next_block;
   }
 }
+
+#include "attn_fwd_merged.inc"
 
 // Adds up the pieces of the blocks that were cut, in their order (cut_blocks.h; a workgroup has the rows of one wave, a lane what it held
 // in the kernel above).  Bound by reading the slots (128 KB a piece), four pieces' loads in flight at a time.
@@ -1074,9 +1006,9 @@ int DISTCA_FN(run_fwd_tokens)(const void *q_base, const int64_t *q_task_off, int
   const int64_t grid = list_grid(p, max_items, few);
   if (grid > 0x7fffffff) return fail(DISTCA_E_INVALID, "ca_fwd: grid too large");
   if (device_setup_pending(kSlotFwdLds)) {
-    const void *kernels[] = {(const void *)ca_fwd_kernel<false, false, false>, (const void *)ca_fwd_kernel<true, false, false>,
-                             (const void *)ca_fwd_kernel<false, true, false>,  (const void *)ca_fwd_kernel<true, true, false>,
-                             (const void *)ca_fwd_kernel<false, false, true>,  (const void *)ca_fwd_kernel<true, false, true>};
+    const void *kernels[] = {(const void *)ca_fwd_kernel<false, false>, (const void *)ca_fwd_kernel<true, false>,
+                             (const void *)ca_fwd_merged_kernel<false>,  (const void *)ca_fwd_merged_kernel<true>,
+                             (const void *)ca_fwd_kernel<false, true>,  (const void *)ca_fwd_kernel<true, true>};
     for (const void *kf : kernels) {
       hipError_t e = hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, kFwdLds);
       if (e != hipSuccess) return fail(DISTCA_E_LAUNCH, "ca_fwd: cannot reserve %d B of LDS: %s", kFwdLds, hipGetErrorString(e));
@@ -1087,9 +1019,9 @@ int DISTCA_FN(run_fwd_tokens)(const void *q_base, const int64_t *q_task_off, int
     ScopedTimer timer(DISTCA_TIMER_CA_FWD, s);
     const dim3 g((unsigned)grid), b(kFwdWaves * 64);
     auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, b, kFwdLds, s, a); };
-    if (few) launch(kv_shards ? ca_fwd_kernel<true, false, true> : ca_fwd_kernel<false, false, true>);
-    else if (geom.merge_tiles > 0) launch(kv_shards ? ca_fwd_kernel<true, true, false> : ca_fwd_kernel<false, true, false>);
-    else launch(kv_shards ? ca_fwd_kernel<true, false, false> : ca_fwd_kernel<false, false, false>);
+    if (few) launch(kv_shards ? ca_fwd_kernel<true, true> : ca_fwd_kernel<false, true>);
+    else if (geom.merge_tiles > 0) launch(kv_shards ? ca_fwd_merged_kernel<true> : ca_fwd_merged_kernel<false>);
+    else launch(kv_shards ? ca_fwd_kernel<true, false> : ca_fwd_kernel<false, false>);
     if (split) hipLaunchKernelGGL(ca_fwd_combine_kernel, cut_grid(split_max_cut(lay.max_blocks, lay.target), p->num_heads_kv, kCutParts), dim3(kCutThreads), 0, s, a);
   }
   return check_launch("ca_fwd");

@@ -32,6 +32,18 @@ typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 
 #define DISTCA_LDS __attribute__((address_space(3)))
 
+// D = A(32x16) * B(16x32) + C on one wave64.
+//   A operand: lane l holds row l%32, k = 8*(l/32) .. +7
+//   B operand: lane l holds col l%32, k = 8*(l/32) .. +7
+//   C/D:       lane l holds col l%32, register r holds row 8*(r/4) + 4*(l/32) + r%4
+__device__ __forceinline__ f32x16 mfma32(elemx8 a, elemx8 b, f32x16 c) {
+#ifdef DISTCA_F16
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+#else
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+#endif
+}
+
 // D = A(16x32) * B(32x16) + C on one wave64.
 //   A operand: lane l holds row l%16, k = 8*(l/16) .. +7
 //   B operand: lane l holds col l%16, k = 8*(l/16) .. +7
@@ -43,6 +55,9 @@ __device__ __forceinline__ f32x4 mfma16(elemx8 a, elemx8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 #endif
 }
+
+// Row index (0..31) inside a 32x32 accumulator block for register r of lane-half g.
+__device__ __forceinline__ constexpr int acc_row(int r, int g) { return 8 * (r >> 2) + 4 * g + (r & 3); }
 
 // Transposing LDS read.  Within each group of 16 lanes, lane j supplies the address of
 // 4 consecutive 16-bit elements; lane L of the group receives element (L%4) of the
@@ -69,6 +84,9 @@ __device__ __forceinline__ elemx4 cvt4(float a0, float a1, float a2, float a3) {
   return __builtin_convertvector(v, elemx4);
 }
 
+// max / sum of x over the lane pair (l, l^32).
+__device__ __forceinline__ float pair_max(float x) { return __builtin_fmaxf(x, __shfl_xor(x, 32, 64)); }
+__device__ __forceinline__ float pair_sum(float x) { return x + __shfl_xor(x, 32, 64); }
 // max / sum of x over the four lanes l % 16 + 16 i.
 __device__ __forceinline__ float quad_max(float x) {
   x = __builtin_fmaxf(x, __shfl_xor(x, 16, 64));
