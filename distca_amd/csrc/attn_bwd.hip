@@ -75,6 +75,15 @@ BwdLayout bwd_layout(const distca_ca_params *p, bool shared, bool preferred) {
   return w;
 }
 
+// Whether dk or dv may lie on k or v: dense rows by their bytes; of shards in place only the buffers are known, which are then one.
+bool gradients_on_inputs(const void *k, const void *v, const void *dk, const void *dv, int64_t bytes, bool shards) {
+  const uintptr_t in[] = {(uintptr_t)k, (uintptr_t)v}, out[] = {(uintptr_t)dk, (uintptr_t)dv};
+  for (uintptr_t i : in)
+    for (uintptr_t o : out)
+      if (shards ? i == o : i < o + (uintptr_t)bytes && o < i + (uintptr_t)bytes) return true;
+  return false;
+}
+
 int grid_for(int64_t work_items) {
   int64_t g = (work_items + 255) / 256;
   const int64_t cap = (int64_t)num_compute_units() * 16;
@@ -211,7 +220,9 @@ int DISTCA_FN(run_bwd)(const BwdQuerySide &qs, const void *k, const void *v, voi
   // ---- both work lists, and zeros where no work item writes dk / dv
   const bool few_q = few_row_blocks(p), few_kv = few_key_blocks(p, kSplitFewPerCU) || w.target_kv > 0;
   auto tables_of = [&](int64_t at, int64_t blocks, int32_t target) { return target > 0 ? split_tables(ws + at, blocks, target) : SplitTables{}; };
-  const bool pair = pair_backward(p, few_q && few_kv && (w.target_q == 0 || (w.slots_apart && w.target_kv > 0)));
+  // (dQ reads all of K and V, dK/dV each block's rows before it writes them: where the gradients take their inputs' place, dQ has to be done first)
+  const bool pair = !gradients_on_inputs(k, v, dk, dv, kv_elems * 2, kv_shards != nullptr) &&
+                    pair_backward(p, few_q && few_kv && (w.target_q == 0 || (w.slots_apart && w.target_kv > 0)));
   const ListJob q_list{cu_q, cu_k, launched_dq_geom(p, w.target_q, pair), (int32_t *)(ws + w.sched_q), w.items_q, tables_of(w.tables_q, w.blocks_q, w.target_q)};
   const ListJob kv_list{cu_q, cu_k, launched_dkdv_geom(p, w.target_kv, preferred, shared, pair), (int32_t *)(ws + w.sched_kv), w.items_kv,
                         tables_of(w.tables_kv, w.blocks_kv, w.target_kv)};

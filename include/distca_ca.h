@@ -310,7 +310,8 @@ int distca_ca_fwd_buffers(const void *q_base, const int64_t *q_task_off,
  * (stored document, block of 256 keys) walks the query rows of every task whose
  * prefix holds the block, sums in registers and writes the rows once, so the
  * result is the same in every run whatever `deterministic` says; rows that no
- * task reads come back as zeros. */
+ * task reads come back as zeros.  dk and dv may be k and v themselves, which
+ * they then replace; apart from that no output may lie on an input. */
 int distca_ca_bwd(const void *dout, const void *q, const void *k, const void *v,
                   const void *out, const float *lse, void *dq, void *dk,
                   void *dv, const int32_t *cu_seqlens_q,

@@ -572,6 +572,29 @@ def test_gradients_side_by_side_and_one_after_the_other(cuda, dtype):
         assert_close_bf16(a[:256], b, name)
 
 
+@pytest.mark.parametrize("shared", [False, True])
+@pytest.mark.parametrize("lens", [[256, 31, 200, 130], [2048], [1500, 257, 300]])
+def test_gradients_in_the_place_of_their_inputs(cuda, lens, shared):
+    """dk and dv written over k and v: dQ, which reads all keys, is then not made beside them.  Small batches, whose gradients otherwise share a launch,
+    whole and in pieces, which may have other ends then: the order of a few fp32 sums, 2^-24 each of their size, ahead of one rounding to 2^-9, which
+    moves about one result in some thousand by a unit."""
+    from distca_amd.fused_comm_attn import ca_varlen_bwd, ca_varlen_fwd
+    hq, hkv = 8, 2
+    q_lens, k_lens = (lens, lens) if not shared else ([n // 2 for n in lens], lens)
+    off = torch.zeros(len(lens), dtype=torch.int32, device=cuda) if shared else None
+    tq, tk = sum(q_lens), max(lens) if shared else sum(lens)
+    cq, ck = torch.tensor(cu(q_lens), device=cuda), torch.tensor(cu(k_lens), device=cuda)
+    q, k, v, do = (t.to(cuda) for t in make_qkv(tq, tk, hq, hkv, 128, 82))
+    out, lse = ca_varlen_fwd(q, k, v, cq, ck, max(q_lens), max(k_lens), None, True, off)
+    args = (cq, ck, max(q_lens), max(k_lens), None, True, False, off)
+    want = ca_varlen_bwd(do, q, k, v, out, lse, *args)
+    ki, vi = k.clone(), v.clone()
+    got = ca_varlen_bwd(do, q, ki, vi, out, lse, *args, dk=ki, dv=vi)
+    assert got[1].data_ptr() == ki.data_ptr()
+    for name, a, b in zip(("dq", "dk", "dv"), got, want):
+        assert (a.float() - b.float()).norm() <= 1e-3 * b.float().norm(), name
+
+
 @pytest.mark.parametrize("d,dtype", [(64, torch.bfloat16), (96, torch.float16), (40, torch.bfloat16), (8, torch.bfloat16)])
 def test_head_dims_below_128(cuda, d, dtype):
     """Head dimensions that are multiples of 8 below 128 (the reference pads to a multiple of 8 and lets flash-attn
