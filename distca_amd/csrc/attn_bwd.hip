@@ -221,9 +221,8 @@ int DISTCA_FN(run_bwd)(const BwdQuerySide &qs, const void *k, const void *v, voi
   const bool few_q = few_row_blocks(p), few_kv = few_key_blocks(p, kSplitFewPerCU) || w.target_kv > 0;
   auto tables_of = [&](int64_t at, int64_t blocks, int32_t target) { return target > 0 ? split_tables(ws + at, blocks, target) : SplitTables{}; };
   // (dQ reads all of K and V, dK/dV each block's rows before it writes them: where the gradients take their inputs' place, dQ has to be done first)
-  const bool pair = !gradients_on_inputs(k, v, dk, dv, kv_elems * 2, kv_shards != nullptr) &&
-                    pair_backward(p, few_q && few_kv && (w.target_q == 0 || (w.slots_apart && w.target_kv > 0)));
-  const ListJob q_list{cu_q, cu_k, launched_dq_geom(p, w.target_q, pair), (int32_t *)(ws + w.sched_q), w.items_q, tables_of(w.tables_q, w.blocks_q, w.target_q)};
+  const bool pair = pair_backward(p, preferred) && !gradients_on_inputs(k, v, dk, dv, kv_elems * 2, kv_shards != nullptr);
+  const ListJob q_list{cu_q, cu_k, launched_dq_geom(p, w.target_q), (int32_t *)(ws + w.sched_q), w.items_q, tables_of(w.tables_q, w.blocks_q, w.target_q)};
   const ListJob kv_list{cu_q, cu_k, launched_dkdv_geom(p, w.target_kv, preferred, shared, pair), (int32_t *)(ws + w.sched_kv), w.items_kv,
                         tables_of(w.tables_kv, w.blocks_kv, w.target_kv)};
   RowStats stats{};

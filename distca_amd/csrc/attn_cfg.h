@@ -175,9 +175,6 @@ constexpr int32_t kMinPieceBeside = 11;   // of dK/dV (8 in its place: 1024 toke
 inline bool slots_apart(const distca_ca_params *p, int64_t blocks_kv, int32_t target_kv, int64_t blocks_q, int32_t target_q) {
   return (split_max_slots(blocks_kv, target_kv) * kDkdvSlotBytes + split_max_slots(blocks_q, target_q) * kDqSlotBytes) * p->num_heads_kv <= 1024 * kDkdvSlotBytes;
 }
-inline bool pair_backward(const distca_ca_params *p, bool possible) {
-  return possible && (int64_t)p->total_q * p->num_heads_q <= (int64_t)kPairBlocksPerCU * kDqRows * num_compute_units();
-}
 // An upper bound, times *scale, of the KV tiles that cutting could take off the longest block of query rows: all of its tiles but the load of a
 // unit, of which only the part counts that the task of the longest prefix brings along, half of its tiles for every block of that task per unit
 // (from two blocks per unit on pieces, of which there are two a unit, are on average no shorter than the task's blocks: asked, the list builder cuts none of such a task).  How many rows that task has is known where it is the only one, and
@@ -251,6 +248,27 @@ inline SchedGeom bwd_geom(const distca_ca_params *p) {
   g.walk_round = num_compute_units() / p->num_heads_kv > 0 ? num_compute_units() / p->num_heads_kv : 1;
   return g;
 }
+// Whether a backward's lists share a launch.  preferred: the call brought that workspace (and may cut both lists).
+inline int64_t dq_max_items(const distca_ca_params *p);
+inline bool pair_backward(const distca_ca_params *p, bool preferred) {
+  if (!few_row_blocks(p) || (int64_t)p->total_q * p->num_heads_q > (int64_t)kPairBlocksPerCU * kDqRows * num_compute_units()) return false;
+  const int32_t target_kv = preferred ? preferred_key_pieces(p) : bwd_split_target(p);
+  const int32_t target_q = preferred ? row_split_target(p, dq_max_items(p), kCutFromTilesDq) : 0;
+  if (target_q == 0) return target_kv > 0 || few_key_blocks(p, kSplitFewPerCU);
+  return target_kv > 0 && slots_apart(p, bwd_key_blocks_own_rows(p), target_kv, dq_max_items(p), target_q);
+}
+// Whether dQ's pieces are those of a list that shares its launch.  As row_split_target it must not know how K/V are stored (it once did: 8 tasks of 256 rows
+// over a document of 16384 at 4/1 heads had 158 pieces over stored rows and 252 over copies, and dq other bits): it asks for the stored rows that one copy
+// of every task's prefix would be, as far as the bounds tell, whole documents' (what row_tiles_to_gain takes for such) or the longest prefix for every task.
+// Where it says no and the launch is shared all the same, pieces cut as if alone do as well or better.  us backward, 256 or 512 rows each, evenly over the
+// prefixes, cut for both lists / as if alone: 8 tasks to 16384 at 4/1 heads 161 / 162, 16 to 16384 at 4/1 258 / 243, 8 to 16384 at 8/2 253 / 246, 2 to 4096
+// at 32/8 142 / 128.
+inline bool dq_pieces_beside(const distca_ca_params *p) {
+  distca_ca_params q = *p;
+  const int64_t copies = p->max_seqlen_q == p->max_seqlen_k && p->max_seqlen_k <= p->total_q ? p->total_q : (int64_t)p->max_seqlen_k * p->num_tasks;
+  q.total_k = (int32_t)(copies < 0x7fffffff ? copies : 0x7fffffff);
+  return pair_backward(&q, true);
+}
 // The lists as the calls launch them.  `target`: pieces aimed for per kv head, 0: whole blocks; for dK/dV also whether they are what
 // the preferred workspace has room for (only what is worth it, at one size) or the smallest (equal parts).
 inline SchedGeom launched_fwd_geom(const distca_ca_params *p, int32_t target) {
@@ -258,10 +276,12 @@ inline SchedGeom launched_fwd_geom(const distca_ca_params *p, int32_t target) {
   if (target > 0) cut_where_worth(&g, p, target, 6, 4, 8);
   return g;
 }
-inline SchedGeom launched_dq_geom(const distca_ca_params *p, int32_t target, bool beside) {
+inline SchedGeom launched_dq_geom(const distca_ca_params *p, int32_t target) {
   SchedGeom g = launched_geom(dq_geom(p), p);
-  if (target > 0) cut_where_worth(&g, p, target, 6, 3, 6);
-  if (beside) g.beside = kDkdvBesideDq;
+  if (target > 0) {
+    cut_where_worth(&g, p, target, 6, 3, 6);
+    if (dq_pieces_beside(p)) g.beside = kDkdvBesideDq;
+  }
   return g;
 }
 inline SchedGeom bwd_shared_geom(const distca_ca_params *p);

@@ -584,11 +584,8 @@ struct LaunchedList {
 LaunchedList launched_list(int kind, const distca_ca_params *p) {
   const int64_t blocks = kind == 0 ? fwd_max_items(p) : dq_max_items(p);
   if (kind == 0) return {launched_fwd_geom(p, row_split_target(p, blocks, kCutFromTilesFwd)), blocks};
-  const int32_t target_kv = preferred_key_pieces(p), target_q = row_split_target(p, dq_max_items(p), kCutFromTilesDq);
-  const bool pair = pair_backward(p, few_row_blocks(p) && (few_key_blocks(p, kSplitFewPerCU) || target_kv > 0) &&
-                                         (target_q == 0 || target_kv > 0 && slots_apart(p, bwd_key_blocks_own_rows(p), target_kv, dq_max_items(p), target_q)));
-  if (kind == 1) return {launched_dkdv_geom(p, target_kv, true, false, pair), bwd_key_blocks_own_rows(p)};
-  return {launched_dq_geom(p, target_q, pair), blocks};
+  if (kind == 1) return {launched_dkdv_geom(p, preferred_key_pieces(p), true, false, pair_backward(p, true)), bwd_key_blocks_own_rows(p)};
+  return {launched_dq_geom(p, row_split_target(p, blocks, kCutFromTilesDq)), blocks};
 }
 }  // namespace
 

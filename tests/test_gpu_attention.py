@@ -572,6 +572,29 @@ def test_gradients_side_by_side_and_one_after_the_other(cuda, dtype):
         assert_close_bf16(a[:256], b, name)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16])
+@pytest.mark.parametrize("hq,hkv,rows,prefixes", [(4, 1, 256, [2048 * (i + 1) for i in range(8)]), (8, 2, 200, [900, 4000, 4100]), (32, 8, 512, [512, 4096])])
+def test_gradients_of_queries_over_shared_rows_and_over_copies(cuda, hq, hkv, rows, prefixes, dtype):
+    """Tasks over prefixes of one stored document, and over a copy of the prefix each: dq has the same bits, whether its kernel shares a launch with
+    dK/dV (which the number of stored rows decides) or not."""
+    import ctypes
+    from distca_amd import _lib
+    from distca_amd.fused_comm_attn import ca_varlen_bwd, ca_varlen_fwd
+    n = len(prefixes)
+    q, k, v, do = (t.to(dtype).to(cuda) for t in make_qkv(n * rows, max(prefixes), hq, hkv, 128, 83))
+    cq, ck = (torch.tensor(cu(x), device=cuda) for x in ([rows] * n, prefixes))
+    res = []
+    for copies in (False, True):
+        kk, vv = (torch.cat([t[:p] for p in prefixes]) if copies else t for t in (k, v))
+        off = None if copies else torch.zeros(n, dtype=torch.int32, device=cuda)
+        p = _lib.CaParams(n, n * rows, kk.shape[0], hq, hkv, 128, rows, max(prefixes), 128 ** -0.5, 1, 1, 1 if dtype == torch.float16 else 2)
+        ws = torch.empty(_lib.load().distca_ca_bwd_workspace_preferred_bytes(ctypes.byref(p)), dtype=torch.uint8, device=cuda)
+        out, lse = ca_varlen_fwd(q, kk, vv, cq, ck, rows, max(prefixes), None, True, off)
+        res.append((out, lse, ca_varlen_bwd(do, q, kk, vv, out, lse, cq, ck, rows, max(prefixes), None, True, True, off, workspace=ws)[0]))
+    for name, a, b in zip(("out", "lse", "dq"), *res):
+        assert torch.equal(a, b), name
+
+
 @pytest.mark.parametrize("shared", [False, True])
 @pytest.mark.parametrize("lens", [[256, 31, 200, 130], [2048], [1500, 257, 300]])
 def test_gradients_in_the_place_of_their_inputs(cuda, lens, shared):

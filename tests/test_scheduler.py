@@ -353,3 +353,22 @@ def test_cutting_takes_the_bounds_of_lengths_as_bounds(kind):
         assert _launched_costs(kind, lens, lens, 8, 2, (sum(lens),) * 2)[1] > 0
     assert _launched_costs(kind, [2000], [2000], 8, 2, (32768, 32768))[1] > 0
     assert _launched_costs(kind, [4096, 256], [4096, 131072], 32, 8, (131072, 131072))[1] > 0
+
+
+def test_pieces_of_query_rows_do_not_depend_on_how_keys_are_stored():
+    """The lists of blocks of query rows, forward and dQ, with tasks over stored rows that they share, over one copy of the prefix each, and with rows that
+    nobody reads: the same items, so that out, lse and dq have the same bits in every form.  (dQ's share of a launch with dK/dV does depend on it.)"""
+    rng = np.random.default_rng(12)
+    batches = [(hq, hkv, [256] * n, [16384 * (i + 1) // n for i in range(n)]) for hq, hkv, n in ((4, 1, 8), (4, 1, 16), (8, 2, 8), (32, 8, 8))]
+    for _ in range(120):
+        hq, hkv = [(4, 1), (8, 2), (32, 8), (16, 16)][rng.integers(4)]
+        n = int(rng.integers(1, 10))
+        lk = np.sort(np.exp(rng.uniform(5, 10.5, n)).astype(int))
+        batches.append((hq, hkv, [int(min(k, r)) for k, r in zip(lk, np.exp(rng.uniform(4, 7.5, n)))], lk.tolist()))
+    cut = 0
+    for hq, hkv, lq, lk in batches:
+        for kind in (scheduler.FWD, scheduler.DQ):
+            lists = [scheduler.build_schedule(kind | scheduler.LAUNCHED, _cu(lq), _cu(lk), hq, hkv, total_k=t) for t in (max(lk), sum(lk), sum(lk) + 100000)]
+            assert all(np.array_equal(lists[0], other) for other in lists[1:]), (hq, hkv, lq, lk)
+            cut += bool((scheduler.item_pieces(lists[0][:, 3]) > 1).any())
+    assert cut > 50
