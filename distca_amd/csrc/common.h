@@ -97,6 +97,30 @@ __device__ __forceinline__ float quad_sum(float x) {
   return x + __shfl_xor(x, 32, 64);
 }
 
+// sum + the products of eight elements of a row of dO and one of O, one after the other; slice: which 32 of the row's 128 they are of.  Two kernels make
+// the row statistics, and gradients must not tell which: the instructions are named here, as the compiler pairs fp16 products (v_dot2) in some places
+// and not in others.  (The last slice's it paired where these sums were first made, and the bits are kept.)
+template <bool F16>
+__device__ __forceinline__ float add_products(u32x4 x, u32x4 y, int slice, float sum) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t u = x[i], v = y[i];   // (a bit cast of x[i] itself took x[0] for every i)
+    if constexpr (F16) {
+      typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+      if (slice == 3) {
+        sum = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, u), __builtin_bit_cast(f16x2, v), sum, false);
+      } else {
+        asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel_hi:[1,1,0]" : "+v"(sum) : "v"(u), "v"(v));
+        asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel:[1,1,0] op_sel_hi:[1,1,0]" : "+v"(sum) : "v"(u), "v"(v));
+      }
+    } else {
+      sum = __builtin_fmaf(__builtin_bit_cast(float, u << 16), __builtin_bit_cast(float, v << 16), sum);
+      sum = __builtin_fmaf(__builtin_bit_cast(float, u & 0xffff0000u), __builtin_bit_cast(float, v & 0xffff0000u), sum);
+    }
+  }
+  return sum;
+}
+
 // Inclusive sum over the wave's lanes, by DPP moves: within rows of 16, then from the last lane of a row and of a half on.  (Lane
 // exchanges through LDS, ten of them a scan, were most of a scan's microsecond.)
 __device__ __forceinline__ int32_t wave_inclusive_scan_i32(int32_t v) {

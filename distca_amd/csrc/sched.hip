@@ -480,11 +480,10 @@ __device__ void fill_rows(FillScratch &f, TaskCache &cache, const BwdFill &a, co
   }
 }
 
-// The row statistics, four lanes to a row, whose products are added up in the dQ kernel's order: the same bits whichever makes them.
+// The row statistics, four lanes to a row, whose products are added up by the dQ kernel's instructions in its order: the same bits whichever makes them.
 // Bound by reading dO and O, and by one trip to memory where those are few.
 constexpr int kStatsRows = kSchedThreads / 4;
 __device__ void row_stats(const RowStats &a, const int32_t *__restrict__ cu_q, int32_t num_tasks, int part, int parts) {
-  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
   const int quarter = threadIdx.x & 3;
   const int32_t rows = a.total_q * a.hq;
   for (int32_t r = part * kStatsRows + (int32_t)(threadIdx.x >> 2); r < rows; r += parts * kStatsRows) {
@@ -507,19 +506,7 @@ __device__ void row_stats(const RowStats &a, const int32_t *__restrict__ cu_q, i
     float lse = 0.f, sum = 0.f;
     if (quarter == 0) lse = a.lse ? a.lse[(int64_t)h * a.total_q + t] : reinterpret_cast<const float *>(a.lse_tok + at)[h];
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t u = x[s][i], v = y[s][i];   // (two elements each; a bit cast of x[s][i] itself took x[s][0] for every i)
-        if (a.f16) {
-          const f16x2 uh = __builtin_bit_cast(f16x2, u), vh = __builtin_bit_cast(f16x2, v);
-          sum += (float)uh[0] * (float)vh[0];
-          sum += (float)uh[1] * (float)vh[1];
-        } else {
-          sum += __builtin_bit_cast(float, u << 16) * __builtin_bit_cast(float, v << 16);
-          sum += __builtin_bit_cast(float, u & 0xffff0000u) * __builtin_bit_cast(float, v & 0xffff0000u);
-        }
-      }
+    for (int s = 0; s < 4; ++s) sum = a.f16 ? add_products<true>(x[s], y[s], s, sum) : add_products<false>(x[s], y[s], s, sum);
     sum += __shfl_xor(sum, 1, 4);
     sum += __shfl_xor(sum, 2, 4);
     if (quarter == 0) {
