@@ -69,7 +69,7 @@ __device__ __forceinline__ void add_up_dkdv(const BwdArgs &a, int part) {
   const int64_t kv_stride = (int64_t)a.hkv * kHeadDim;
   auto gradient = [&](bool is_dv) {
     add_up_cut_blocks(
-        a.cut,
+        a.cut, a.slot,
         [&](const int4 &e, f32x4 (&o)[4]) {
           const f32x4 *first = reinterpret_cast<const f32x4 *>(a.partial + ((int64_t)e.w * a.hkv + kvh) * kDkdvSlotBytes);
           add_pieces(first + ((is_dv ? 32 : 0) + 16 * kb + 4 * db) * kThreads + key_wave * 64 + lane, a.hkv * (kDkdvSlotBytes / 16), kThreads, e.z, o);

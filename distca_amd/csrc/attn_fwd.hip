@@ -753,7 +753,7 @@ __global__ __launch_bounds__(kCutThreads) void ca_fwd_combine_kernel(FwdArgs a) 
     return row < nrows ? at : nullptr;
   };
   add_up_cut_blocks(
-      a.cut,
+      a.cut, a.slot,
       [&](const int4 &e, f32x4 (&o)[4]) {
         const int pieces = e.z;
         const uint8_t *first = a.partial + ((int64_t)e.w * a.hkv + kvh) * kFwdSlotBytes;

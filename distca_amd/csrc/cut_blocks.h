@@ -18,12 +18,12 @@ inline dim3 cut_grid(int64_t max_cut, int hkv, int parts) {
 }
 // add(entry, o): adds the pieces of entry (unit, block, pieces, first slot) to o.  row_at(entry, r): where row r of the 32 goes, null if it does not exist.
 template <class Add, class RowAt>
-__device__ __forceinline__ void add_up_cut_blocks(const int32_t *cut, Add add, RowAt row_at) {
+__device__ __forceinline__ void add_up_cut_blocks(const int32_t *cut, const int32_t *slot, Add add, RowAt row_at) {
   __shared__ __attribute__((aligned(16))) uint8_t rows[32 * 256];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, g = lane >> 5;
   const int4 *entries = reinterpret_cast<const int4 *>(cut + 4);
   const int n = cut[0];
-  int4 e = entries[blockIdx.x];   // (asked for together with n: it has a place in the table whatever n is)
+  int4 e = entries[first_cut_entry(cut, slot, blockIdx.x)];   // (asked for together with n)
   e.x = uniform_int(e.x), e.y = uniform_int(e.y), e.z = uniform_int(e.z), e.w = uniform_int(e.w);
   asm volatile("" : "+s"(e.x), "+s"(e.y), "+s"(e.z), "+s"(e.w));
   for (int c = blockIdx.x; c < n; c += gridDim.x) {

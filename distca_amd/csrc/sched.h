@@ -316,6 +316,11 @@ DISTCA_HD SplitTables split_tables(void *at, int64_t max_blocks, int32_t target)
   int32_t *p = (int32_t *)at;
   return SplitTables{p, p + 4 + 4 * split_max_cut(max_blocks, target)};
 }
+// The entry that workgroup `wg` of the kernels that add pieces up may ask for before it knows how many there are: its own, or, past the table's places (the launch
+// over two lists has workgroups for the larger table), the first.
+DISTCA_HD int32_t first_cut_entry(const int32_t *cut, const int32_t *slot, unsigned wg) {
+  return wg < (unsigned)((slot - cut - 4) / 4) ? (int32_t)wg : 0;
+}
 
 #if defined(__HIPCC__)
 // The (item, kv head) of workgroup `wg` of those over a list of few items; false past the list's end.

@@ -6,6 +6,8 @@ the items must tile every task exactly once, each item's extent must cover exact
 (or query blocks) the causal mask with KV-prefix offset lk - lq makes visible, and the order
 must be longest first."""
 import heapq
+import os
+import subprocess
 
 import numpy as np
 import pytest
@@ -372,3 +374,29 @@ def test_pieces_of_query_rows_do_not_depend_on_how_keys_are_stored():
             assert all(np.array_equal(lists[0], other) for other in lists[1:]), (hq, hkv, lq, lk)
             cut += bool((scheduler.item_pieces(lists[0][:, 3]) > 1).any())
     assert cut > 50
+
+
+def test_no_workgroup_reads_past_the_table_of_cut_blocks(tmp_path):
+    """What the kernels that add pieces up ask for ahead of the count of cut blocks: the entry of every workgroup of a launch, which may have as many as
+    the larger of two tables has places, lies within its own table."""
+    src = tmp_path / "t.cpp"
+    src.write_text("""
+#include <initializer_list>
+#include "sched.h"
+using namespace distca;
+int main() {
+  static int32_t ws[1 << 16];
+  for (int64_t blocks : {1, 2, 18, 66, 300})
+    for (int32_t target : {1, 2, 17, 64, 512}) {
+      const SplitTables t = split_tables(ws, blocks, target);
+      for (unsigned wg = 0; wg < 700; ++wg) {
+        const int64_t places = split_max_cut(blocks, target), at = first_cut_entry(t.cut, t.slot, wg);
+        if (at < 0 || at >= places || (wg < (uint64_t)places && at != wg) || t.cut + 4 + 4 * at + 4 > t.slot) return 1;
+      }
+    }
+  return 0;
+}
+""")
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "distca_amd", "csrc")
+    subprocess.run(["g++", "-std=c++17", "-I", csrc, str(src), "-o", str(tmp_path / "t")], check=True)
+    subprocess.run([str(tmp_path / "t")], check=True)
