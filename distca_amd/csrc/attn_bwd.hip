@@ -36,7 +36,8 @@ __global__ __launch_bounds__(256) void fill_zero_kernel(u32x4 *__restrict__ p, i
 
 // How a backward is laid out in its workspace: the two lists, the row statistics, and, where blocks are cut into pieces, the lists'
 // tables and the slots of both: side by side where they fit (slots_apart; attn_bwd_pair.hip writes both at a time), else in one place (dQ's
-// pieces are then added up before the first of dK / dV is written).
+// pieces are then added up before the first of dK / dV is written).  In one place as well where the workspace has room for no more: what callers that
+// keep a buffer sized it for before the slots lay side by side.
 struct BwdLayout {
   int64_t sched_kv, sched_q, delta, lse2, tables_kv, tables_q, slots, slots_q, total;
   int64_t blocks_kv, blocks_q, items_kv, items_q;   // bounds on blocks, and room of the lists
@@ -44,8 +45,8 @@ struct BwdLayout {
   bool slots_apart;
 };
 // shared: tasks over shared stored rows (items are then over groups of tasks).  preferred: cut blocks of query rows as well, and
-// key blocks whatever `deterministic` says.
-BwdLayout bwd_layout(const distca_ca_params *p, bool shared, bool preferred) {
+// key blocks whatever `deterministic` says.  one_place: the slots in one place.
+BwdLayout bwd_layout(const distca_ca_params *p, bool shared, bool preferred, bool one_place = false) {
   BwdLayout w;
   w.blocks_kv = shared || preferred ? bwd_key_blocks_own_rows(p) : bwd_max_items(p) - bwd_split_target(p);
   w.blocks_q = dq_max_items(p);
@@ -62,7 +63,7 @@ BwdLayout bwd_layout(const distca_ca_params *p, bool shared, bool preferred) {
   w.tables_kv = take(split_tables_bytes(w.blocks_kv, w.target_kv, w.items_kv));
   w.tables_q = take(split_tables_bytes(w.blocks_q, w.target_q, w.items_q));
   const int64_t kv = split_max_slots(w.blocks_kv, w.target_kv) * kDkdvSlotBytes, q = split_max_slots(w.blocks_q, w.target_q) * kDqSlotBytes;
-  w.slots_apart = slots_apart(p, w.blocks_kv, w.target_kv, w.blocks_q, w.target_q);
+  w.slots_apart = !one_place && slots_apart(p, w.blocks_kv, w.target_kv, w.blocks_q, w.target_q);
   w.slots = take((w.slots_apart || kv > q ? kv : q) * p->num_heads_kv);
   w.slots_q = w.slots_apart ? take(q * p->num_heads_kv) : w.slots;
   if (preferred && o > w.slots) take(256);   // (so that no call that brought the smallest workspace is taken for one that brought this)
@@ -181,8 +182,9 @@ int DISTCA_FN(run_bwd)(const BwdQuerySide &qs, const void *k, const void *v, voi
     if (rc) return rc;
   }
   const bool shared = alias;
-  const bool preferred = workspace_bytes >= bwd_layout(p, shared, true).total;   // room for everything the call can use
-  const BwdLayout w = bwd_layout(p, shared, preferred);
+  const bool roomy = workspace_bytes >= bwd_layout(p, shared, true).total;   // room for everything the call can use
+  const bool preferred = roomy || workspace_bytes >= bwd_layout(p, shared, true, true).total;
+  const BwdLayout w = bwd_layout(p, shared, preferred, !roomy);
   if (!workspace || workspace_bytes < w.total)
     return fail(DISTCA_E_WORKSPACE, "ca_bwd: workspace %lld B < required %lld B", (long long)workspace_bytes, (long long)w.total);
   if (!aligned16(workspace)) return fail(DISTCA_E_INVALID, "ca_bwd: workspace must be 16-byte aligned");
@@ -221,7 +223,7 @@ int DISTCA_FN(run_bwd)(const BwdQuerySide &qs, const void *k, const void *v, voi
   const bool few_q = few_row_blocks(p), few_kv = few_key_blocks(p, kSplitFewPerCU) || w.target_kv > 0;
   auto tables_of = [&](int64_t at, int64_t blocks, int32_t target) { return target > 0 ? split_tables(ws + at, blocks, target) : SplitTables{}; };
   // (dQ reads all of K and V, dK/dV each block's rows before it writes them: where the gradients take their inputs' place, dQ has to be done first)
-  const bool pair = pair_backward(p, preferred) && !gradients_on_inputs(k, v, dk, dv, kv_elems * 2, kv_shards != nullptr);
+  const bool pair = pair_backward(p, preferred) && (w.target_q == 0 || w.slots_apart) && !gradients_on_inputs(k, v, dk, dv, kv_elems * 2, kv_shards != nullptr);
   const ListJob q_list{cu_q, cu_k, launched_dq_geom(p, w.target_q), (int32_t *)(ws + w.sched_q), w.items_q, tables_of(w.tables_q, w.blocks_q, w.target_q)};
   const ListJob kv_list{cu_q, cu_k, launched_dkdv_geom(p, w.target_kv, preferred, shared, pair), (int32_t *)(ws + w.sched_kv), w.items_kv,
                         tables_of(w.tables_kv, w.blocks_kv, w.target_kv)};

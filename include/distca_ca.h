@@ -221,8 +221,10 @@ int64_t distca_ca_bwd_workspace_bytes(const distca_ca_params *p);
  * 1024 keys is needed; 256 keys x kv heads for dK / dV) may then have its longest blocks cut into pieces, whose fp32
  * results pass through the workspace and are added up in a fixed order.  The room is that of the most pieces such a
  * batch can have, up to 4 per compute unit whatever its size: at most 140 MB forward and 275 MB backward beyond the
- * sizes above on 256 units (4096 tokens: 63 and 140 MB at 4/1 heads, 136 and 177 MB at 32/8).  Never less than the
- * sizes above, and equal to them for batches that fill the device.  A call decides by the workspace_bytes it is given. */
+ * sizes above on 256 units (one document of 4096 tokens: 77 and 215 MB at 4/1 heads, 0 and 173 MB at 32/8).  Never less than the
+ * sizes above, and equal to them for batches that fill the device.  A call decides by the workspace_bytes it is given.  In
+ * the backward the slots of dQ's pieces lie beside those of dK / dV, which lets one launch make both; a workspace without room for
+ * that (139 MB for the batch named, at 4/1 heads) has them in one place, and its pieces are made one after the other. */
 int64_t distca_ca_fwd_workspace_preferred_bytes(const distca_ca_params *p);
 int64_t distca_ca_bwd_workspace_preferred_bytes(const distca_ca_params *p);
 

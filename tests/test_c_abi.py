@@ -201,6 +201,18 @@ def test_smallest_workspace_stays_what_fixed_buffers_were_sized_for(deterministi
         assert int(lib.distca_ca_bwd_workspace_bytes(ctypes.byref(p))) <= mb * 1e6 + 1e5
 
 
+def test_preferred_sizes_that_the_header_names():
+    """The sizes quoted for one document of 4096 tokens are those that the functions return."""
+    lib = _lib.load()
+    text = re.sub(r"\s*\n \* ", " ", open(HEADER).read())
+    quoted = re.search(r"one document of 4096 tokens: (\d+) and (\d+) MB at 4/1 heads, (\d+) and (\d+) MB at 32/8", text)
+    sizes = []
+    for hq, hkv in ((4, 1), (32, 8)):
+        p = _p(total_q=4096, total_k=4096, num_heads_q=hq, num_heads_kv=hkv, max_seqlen_q=4096, max_seqlen_k=4096)
+        sizes += [int(getattr(lib, f"distca_ca_{d}_workspace_preferred_bytes")(ctypes.byref(p))) for d in ("fwd", "bwd")]
+    assert [int(mb) for mb in quoted.groups()] == [round(b / 1e6) for b in sizes]
+
+
 def test_python_wrappers_reject_wrong_inputs():
     """The host layer raises RuntimeError for what the reference's C++ wrappers check
     (all_to_all.cpp:18-21, 47-99): device, rank, dtype of metadata."""

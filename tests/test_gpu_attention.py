@@ -664,6 +664,32 @@ def test_pieces_within_the_smallest_workspace(cuda, q_lens, hq, hkv, shared):
         assert ((x - y).abs() <= 2.0 ** -7 * y.abs() + n ** 1.5 / 16 * 2.0 ** -24 * y.abs().max()).all(), name
 
 
+@pytest.mark.parametrize("tokens,hq,hkv,mb", [(4096, 4, 1, 139.3), (4096, 8, 2, 144.0), (2048, 4, 1, 89.3)])
+@pytest.mark.parametrize("shared", [False, True])
+def test_workspace_with_one_place_for_pieces(cuda, tokens, hq, hkv, mb, shared):
+    """Workspaces of what the preferred size was when the pieces of dQ and of dK/dV had their slots in one place (the test's figures): blocks are cut as with
+    the present size, the kernels run one after the other, and nothing is written behind the workspace."""
+    import ctypes
+    from distca_amd._lib import CaParams, load
+    from distca_amd.fused_comm_attn import ca_varlen_bwd, ca_varlen_fwd
+    q, k, v, do = (t.to(cuda) for t in make_qkv(tokens, tokens, hq, hkv, 128, 65))
+    c, off = torch.tensor(cu([tokens]), device=cuda), torch.zeros(1, dtype=torch.int32, device=cuda) if shared else None
+    p = CaParams(1, tokens, tokens, hq, hkv, 128, tokens, tokens, 128 ** -0.5, 1, 1, 0)
+    need, room = int(load().distca_ca_bwd_workspace_preferred_bytes(ctypes.byref(p))), int(mb * 1e6)
+    assert int(load().distca_ca_bwd_workspace_bytes(ctypes.byref(p))) < room < need
+    ws = torch.full((room + 65536,), 0x5A, dtype=torch.uint8, device=cuda)
+    out, lse = ca_varlen_fwd(q, k, v, c, c, tokens, tokens, kv_task_offsets=off)
+    args = (do, q, k, v, out, lse, c, c, tokens, tokens, None, True, True, off)
+    res = [ca_varlen_bwd(*args, workspace=ws[:room]), ca_varlen_bwd(*args, workspace=ws[:room]),
+           ca_varlen_bwd(*args, workspace=torch.empty(need, dtype=torch.uint8, device=cuda))]
+    assert int(ws[:4].view(torch.int32)) > tokens // 256, "no key block was cut"
+    assert (ws[room:] == 0x5A).all()
+    for name, x, again, y in zip(("dq", "dk", "dv"), *res):
+        assert torch.equal(x, again), name
+        x, y = x.float(), y.float()   # (the bound of test_pieces_within_the_smallest_workspace; dq's pieces are the same)
+        assert torch.equal(x, y) if name == "dq" else ((x - y).abs() <= 2.0 ** -7 * y.abs() + tokens ** 1.5 / 16 * 2.0 ** -24 * y.abs().max()).all(), name
+
+
 def test_small_batches_where_memory_is_short(cuda):
     """A batch whose preferred workspace does not fit any more: the smallest is taken, and the results are those of calls that bring it."""
     import ctypes
