@@ -158,6 +158,23 @@ constexpr int kCutFromTilesFwd = 24, kCutFromTilesDq = 16;
 inline bool few_row_blocks(const distca_ca_params *p) {
   return (int64_t)p->total_q * p->num_heads_q < (int64_t)kSplitMaxBlocksPerCU * kFwdRows * num_compute_units();
 }
+// Whether a forward of few blocks has 32x32x16 MFMAs (attn_fwd32.inc) rather than 16x16x32 (attn_fwd.hip).  The smaller ones save energy and cost cycles, so
+// they are for what runs long enough at full load to be bound by power.  That is not so up to prefixes of kFwd32Keys, whose blocks are short, up to
+// kFwd32Tiles tiles a compute unit, as far as the bounds tell, nor, up to kFwd32TilesOnce of them and prefixes of kFwd32KeysOnce, where every unit has a block at
+// most: half of them are soon done.  us forward, 16x16x32 / 32x32x16 (tiles a unit): 200 tokens at 4/1 heads 11.3 / 10.3, 600 18.8 / 16.5, 1500 (9) at 4/1 34.4 / 30.1, at 32/8
+// 36.2 / 32.2, 2048 (17) at 32/8 48.8 / 45.9, 2500 (24) 61.2 / 59.9, 256 rows to 8192 at 8/2 40.1 / 37.6, 4096 in pieces (17) at 8/2 60.9 / 59.9, 5000 (24) 73.3 / 73.1,
+// 12 x 1024 (51) at 32/8 127.2 / 125.1, a block a unit, 4096 (33) at 16/4 97.5 / 91.9, 8 x 2048 (17) at 4/1 57.9 / 54.8; on the other side 1800 (25) at 64/8 57.6 / 57.8,
+// 6000 in pieces (34) at 8/2 91.6 / 92.3, 8192 (32) at 4/1 89.1 / 90.0, 3 x 5000 (37) 91.7 / 92.9, 3000 (35) at 32/8 74.2 / 76.2, 2 x 2048 (33) 67.7 / 69.3, 10 x 1500 (91)
+// 208.5 / 208.5, 4096 (66) 119.3 / 124.0, 8192 434 / 454.
+// As row_split_target it must not know how K/V are stored.
+constexpr int kFwd32Keys = 1280, kFwd32Tiles = 24, kFwd32KeysOnce = 4096, kFwd32TilesOnce = 33;
+inline bool fwd_mfma32(const distca_ca_params *p) {
+  const int64_t k = p->max_seqlen_k, q = p->max_seqlen_q < k ? p->max_seqlen_q : k, rows = (int64_t)p->total_q * p->num_heads_q, units = num_compute_units();
+  if (k <= kFwd32Keys) return true;
+  const bool once = rows <= kFwdRows * units && k <= kFwd32KeysOnce;
+  const int64_t keys = p->causal ? k - q / 2 : k;   // that a row sees on average, of a task with the longest prefix
+  return rows * keys <= (int64_t)(once ? kFwd32TilesOnce : kFwd32Tiles) * kFwdRows * kFwdKV * units;
+}
 // dQ and dK/dV side by side in one launch (attn_bwd_pair.hip) up to kPairBlocksPerCU blocks of query rows per compute unit: each then
 // fills what the other's longest blocks leave idle, and a launch is saved.  Beyond that their last blocks are a small part of the time and the pass over dO
 // and O that makes the row statistics ahead of both shows.  us backward, one after the other / side by side: 256 tokens at 8/2 heads 51 / 34, 389 at 4/1

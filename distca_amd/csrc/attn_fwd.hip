@@ -184,6 +184,34 @@ __device__ __forceinline__ int4 block_of_rank(const int32_t *cu_q, const int32_t
   return make_int4(task, e - past + __builtin_amdgcn_readlane(first - (incl - n), task), 0, 1 << 16);
 }
 
+// Draws a workgroup's item and kv head; false where none is left.
+template <bool SPLIT>
+__device__ __forceinline__ bool take_fwd_item(const FwdArgs &a, int32_t *slot, int &item, int &kvh, int4 &it) {
+  if (SPLIT && !a.sched) {
+    // no list (see run_fwd_tokens): the workgroup's id is its block's rank, or counts the batch's blocks
+    item = (int)(blockIdx.x / (unsigned)a.hkv);
+    kvh = (int)(blockIdx.x - (unsigned)item * (unsigned)a.hkv);
+    it = a.max_tiles ? block_of_rank(a.cu_q, a.cu_k, a.num_tasks, a.group, a.causal, a.max_tiles, item) : block_of_batch(a.cu_q, a.num_tasks, a.group, item);
+    return it.x >= 0;
+  }
+  const int nitems = a.sched[0];
+  if (!take_item<SPLIT>(a.tickets, nitems, a.hkv, slot, item, kvh)) return false;
+  it = reinterpret_cast<const int4 *>(a.sched + a.sched_items_off)[item];
+  return true;
+}
+
+// SPLIT kernels: a piece is what a whole block over the keys from its first tile on would be: what counts keys from the start of the prefix is
+// moved by the tiles before it, and below nothing knows of it.  (Carrying the first tile into the loops cost 5 % of a block's time.)
+__device__ __forceinline__ void cut_out_piece(const FwdArgs &a, const int4 &it, int &ntiles, int &ks, int &lk, int &shift) {
+  const int w = uniform_int(it.w);
+  int tile0, tile1;
+  piece_range(ntiles, item_piece(w), item_pieces(w), a.cut ? uniform_int(a.cut[2]) : 0, &tile0, &tile1);
+  ntiles = tile1 - tile0;
+  ks += tile0 * kFwdKV;
+  lk -= tile0 * kFwdKV;
+  shift -= tile0 * kFwdKV;
+}
+
 // SEG: K/V rows are addressed through a table of shards (kv_shards.h) instead of as one dense tensor.
 // SPLIT (batches of few blocks): a work item may be a piece of a block, a range of its KV tiles (sched.h, piece_count), whose result
 // goes to a slot; items are taken by workgroup id.
@@ -192,17 +220,7 @@ __global__ __launch_bounds__(kFwdWaves * 64, 1) void ca_fwd_kernel(FwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   int item, kvh;
   int4 it;
-  if (SPLIT && !a.sched) {
-    // no list (see run_fwd_tokens): the workgroup's id is its block's rank, or counts the batch's blocks
-    item = (int)(blockIdx.x / (unsigned)a.hkv);
-    kvh = (int)(blockIdx.x - (unsigned)item * (unsigned)a.hkv);
-    it = a.max_tiles ? block_of_rank(a.cu_q, a.cu_k, a.num_tasks, a.group, a.causal, a.max_tiles, item) : block_of_batch(a.cu_q, a.num_tasks, a.group, item);
-    if (it.x < 0) return;
-  } else {
-    const int nitems = a.sched[0];
-    if (!take_item<SPLIT>(a.tickets, nitems, a.hkv, reinterpret_cast<int32_t *>(lds), item, kvh)) return;
-    it = reinterpret_cast<const int4 *>(a.sched + a.sched_items_off)[item];
-  }
+  if (!take_fwd_item<SPLIT>(a, reinterpret_cast<int32_t *>(lds), item, kvh, it)) return;
   // (the item's fields and the task's bounds are moved to scalar registers as they are read: what derives from them,
   // base pointers, loop limits and tile addresses, is then scalar arithmetic)
   it.x = uniform_int(it.x);
@@ -231,17 +249,7 @@ __global__ __launch_bounds__(kFwdWaves * 64, 1) void ca_fwd_kernel(FwdArgs a) {
   int nvis = a.causal ? tok_end + shift : lk;
   if (nvis > lk) nvis = lk;
   int ntiles = nvis > 0 ? (nvis + kFwdKV - 1) / kFwdKV : 0;
-  if constexpr (SPLIT) {
-    // A piece is what a whole block over the keys from its first tile on would be: what counts keys from the start of the prefix is
-    // moved by the tiles before it, and below nothing knows of it.  (Carrying the first tile into the loops cost 5 % of a block's time.)
-    const int w = uniform_int(it.w);
-    int tile0, tile1;
-    piece_range(ntiles, item_piece(w), item_pieces(w), a.cut ? uniform_int(a.cut[2]) : 0, &tile0, &tile1);
-    ntiles = tile1 - tile0;
-    ks += tile0 * kFwdKV;
-    lk -= tile0 * kFwdKV;
-    shift -= tile0 * kFwdKV;
-  }
+  if constexpr (SPLIT) cut_out_piece(a, it, ntiles, ks, lk, shift);
 
   // ---- per-lane rows: row l32 of the wave where the results are stored, rows c16 and 16 + c16 in the MFMAs' operands and accumulators
   const uint8_t *qbytes = reinterpret_cast<const uint8_t *>(a.q) + uniform_int64(a.q_task_off ? a.q_task_off[task] : (int64_t)q0 * a.q_tok_bytes);
@@ -736,7 +744,7 @@ __global__ __launch_bounds__(kFwdWaves * 64, 1) void ca_fwd_kernel(FwdArgs a) {
   }
 }
 
-#include "attn_fwd_merged.inc"
+#include "attn_fwd32.inc"
 
 // Adds up the pieces of the blocks that were cut, in their order (cut_blocks.h; a workgroup has the rows of one wave, a lane what it held
 // in the kernel above).  Bound by reading the slots (128 KB a piece), four pieces' loads in flight at a time.
@@ -1007,8 +1015,9 @@ int DISTCA_FN(run_fwd_tokens)(const void *q_base, const int64_t *q_task_off, int
   if (grid > 0x7fffffff) return fail(DISTCA_E_INVALID, "ca_fwd: grid too large");
   if (device_setup_pending(kSlotFwdLds)) {
     const void *kernels[] = {(const void *)ca_fwd_kernel<false, false>, (const void *)ca_fwd_kernel<true, false>,
-                             (const void *)ca_fwd_merged_kernel<false>,  (const void *)ca_fwd_merged_kernel<true>,
-                             (const void *)ca_fwd_kernel<false, true>,  (const void *)ca_fwd_kernel<true, true>};
+                             (const void *)ca_fwd_kernel<false, true>,    (const void *)ca_fwd_kernel<true, true>,
+                             (const void *)ca_fwd32_kernel<false, true>,  (const void *)ca_fwd32_kernel<true, true>,
+                             (const void *)ca_fwd32_kernel<false, false>, (const void *)ca_fwd32_kernel<true, false>};
     for (const void *kf : kernels) {
       hipError_t e = hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, kFwdLds);
       if (e != hipSuccess) return fail(DISTCA_E_LAUNCH, "ca_fwd: cannot reserve %d B of LDS: %s", kFwdLds, hipGetErrorString(e));
@@ -1019,8 +1028,9 @@ int DISTCA_FN(run_fwd_tokens)(const void *q_base, const int64_t *q_task_off, int
     ScopedTimer timer(DISTCA_TIMER_CA_FWD, s);
     const dim3 g((unsigned)grid), b(kFwdWaves * 64);
     auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, b, kFwdLds, s, a); };
-    if (few) launch(kv_shards ? ca_fwd_kernel<true, true> : ca_fwd_kernel<false, true>);
-    else if (geom.merge_tiles > 0) launch(kv_shards ? ca_fwd_merged_kernel<true> : ca_fwd_merged_kernel<false>);
+    if (few && fwd_mfma32(p)) launch(kv_shards ? ca_fwd32_kernel<true, false> : ca_fwd32_kernel<false, false>);
+    else if (few) launch(kv_shards ? ca_fwd_kernel<true, true> : ca_fwd_kernel<false, true>);
+    else if (geom.merge_tiles > 0) launch(kv_shards ? ca_fwd32_kernel<true, true> : ca_fwd32_kernel<false, true>);
     else launch(kv_shards ? ca_fwd_kernel<true, false> : ca_fwd_kernel<false, false>);
     if (split) hipLaunchKernelGGL(ca_fwd_combine_kernel, cut_grid(split_max_cut(lay.max_blocks, lay.target), p->num_heads_kv, kCutParts), dim3(kCutThreads), 0, s, a);
   }

@@ -542,6 +542,30 @@ def test_blocks_by_rank_and_from_a_list(cuda, seed):
     assert torch.equal(res[0][0], res[1][0][:tokens])
     assert torch.equal(res[0][1], res[1][1][:, :tokens])
     assert bool(torch.isfinite(res[0][0].float()).all())
+    # prefixes longer than they were said to be: every block all the same (a bound on the same side of the line between the forward's kernels)
+    low = max(k_lens) // 2 if max(k_lens) <= 1280 else 1300
+    ql, kl, off = q_lens, k_lens, torch.zeros(n, dtype=torch.int32, device=cuda) if shared else None
+    rows = sum(kl) if not shared else tk
+    short = ca_varlen_fwd(q[:sum(ql)].contiguous(), k[:rows].contiguous(), v[:rows].contiguous(), torch.tensor(cu(ql), device=cuda),
+                          torch.tensor(cu(kl), device=cuda), max(ql), low, None, causal, off)
+    assert torch.equal(short[0], res[0][0]) and torch.equal(short[1], res[0][1])
+
+
+@pytest.mark.parametrize("q_lens,k_lens,hq,hkv,causal", [
+    ([5000], [5000], 8, 2, True), ([5100], [5100], 8, 2, True),               # pieces of one document
+    ([300, 150], [12000, 2500], 16, 2, True), ([500, 60], [12000, 2500], 16, 2, True),   # pieces of a few rows over long prefixes
+    ([2400], [2400], 32, 8, True), ([2600], [2600], 32, 8, True),             # blocks by rank
+    ([1700], [1700], 32, 8, False), ([1800], [1800], 32, 8, False),
+    ([1280] * 5, [1280] * 5, 32, 8, True), ([1281] * 5, [1281] * 5, 32, 8, True),
+    ([4096] * 2, [4096] * 2, 8, 2, True), ([4097, 4000], [4097, 4000], 8, 2, True)])   # a block a unit
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_either_side_of_the_lines_between_the_forwards_mfmas(cuda, q_lens, k_lens, hq, hkv, causal, dtype):
+    """Batches of few blocks have 32x32x16 MFMAs up to 24 tiles a compute unit (as far as the bounds tell) or prefixes of 1280 keys, or, where no unit has two blocks, 33
+    tiles and prefixes of 4096, 16x16x32 beyond."""
+    keys = max(k_lens) - min(max(q_lens), max(k_lens)) // 2 if causal else max(k_lens)
+    load = sum(q_lens) * hq * keys / (256 * 64 * torch.cuda.get_device_properties(0).multi_processor_count)
+    assert 20 < load < 34, "sizes near the line"
+    _run(q_lens, k_lens, hq, hkv, 84, cuda, causal=causal, bwd=False, dtype=dtype)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

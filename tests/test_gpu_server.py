@@ -718,6 +718,7 @@ def test_kv_shards_read_in_place_equal_dense_tensors(cuda, hq, hkv):
     (4, 1, [64, 128, 192, 193, 191, 256, 1, 320, 383, 129, 448]),     # shards end a key either side of a tile's end, runs of both parities
     (32, 8, [640, 0, 65, 575, 1024, 63, 1, 449]),                     # long runs, shards shorter than a tile between them
     (8, 2, [2560]),                                                   # one shard
+    (64, 8, [700, 64, 436]), (64, 8, [1900, 1, 659]),                 # blocks by rank, with either of the forward's MFMAs
     (8, 8, [37] * 60)])                                               # no tile inside one shard
 def test_runs_of_tiles_inside_shards(cuda, hq, hkv, shard_len):
     """The loops over tiles that lie inside one shard begin and end where shards do: out, lse and the gradients over shards in a buffer (every
