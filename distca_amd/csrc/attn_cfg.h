@@ -166,12 +166,14 @@ inline bool few_row_blocks(const distca_ca_params *p) {
 // 12 x 1024 (51) at 32/8 127.2 / 125.1, a block a unit, 4096 (33) at 16/4 97.5 / 91.9, 8 x 2048 (17) at 4/1 57.9 / 54.8; on the other side 1800 (25) at 64/8 57.6 / 57.8,
 // 6000 in pieces (34) at 8/2 91.6 / 92.3, 8192 (32) at 4/1 89.1 / 90.0, 3 x 5000 (37) 91.7 / 92.9, 3000 (35) at 32/8 74.2 / 76.2, 2 x 2048 (33) 67.7 / 69.3, 10 x 1500 (91)
 // 208.5 / 208.5, 4096 (66) 119.3 / 124.0, 8192 434 / 454.
+// Where blocks stay whole for want of room for pieces (split: there is) and no unit has two, most units are idle however long they are: 8192 at 4/1 154 / 135, 6000 at 8/2
+// 116 / 105, 8 x 512 rows to 32768 at 4/1 590 / 510, 8192 (a block for every unit) at 8/2 162 / 159.
 // As row_split_target it must not know how K/V are stored.
 constexpr int kFwd32Keys = 1280, kFwd32Tiles = 24, kFwd32KeysOnce = 4096, kFwd32TilesOnce = 33;
-inline bool fwd_mfma32(const distca_ca_params *p) {
+inline bool fwd_mfma32(const distca_ca_params *p, bool split) {
   const int64_t k = p->max_seqlen_k, q = p->max_seqlen_q < k ? p->max_seqlen_q : k, rows = (int64_t)p->total_q * p->num_heads_q, units = num_compute_units();
-  if (k <= kFwd32Keys) return true;
-  const bool once = rows <= kFwdRows * units && k <= kFwd32KeysOnce;
+  const bool one_each = rows <= kFwdRows * units, once = one_each && k <= kFwd32KeysOnce;
+  if (k <= kFwd32Keys || (one_each && !split)) return true;
   const int64_t keys = p->causal ? k - q / 2 : k;   // that a row sees on average, of a task with the longest prefix
   return rows * keys <= (int64_t)(once ? kFwd32TilesOnce : kFwd32Tiles) * kFwdRows * kFwdKV * units;
 }

@@ -1028,7 +1028,7 @@ int DISTCA_FN(run_fwd_tokens)(const void *q_base, const int64_t *q_task_off, int
     ScopedTimer timer(DISTCA_TIMER_CA_FWD, s);
     const dim3 g((unsigned)grid), b(kFwdWaves * 64);
     auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, b, kFwdLds, s, a); };
-    if (few && fwd_mfma32(p)) launch(kv_shards ? ca_fwd32_kernel<true, false> : ca_fwd32_kernel<false, false>);
+    if (few && fwd_mfma32(p, split)) launch(kv_shards ? ca_fwd32_kernel<true, false> : ca_fwd32_kernel<false, false>);
     else if (few) launch(kv_shards ? ca_fwd_kernel<true, true> : ca_fwd_kernel<false, true>);
     else if (geom.merge_tiles > 0) launch(kv_shards ? ca_fwd32_kernel<true, true> : ca_fwd32_kernel<false, true>);
     else launch(kv_shards ? ca_fwd_kernel<true, false> : ca_fwd_kernel<false, false>);

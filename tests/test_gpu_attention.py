@@ -561,11 +561,23 @@ def test_blocks_by_rank_and_from_a_list(cuda, seed):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_either_side_of_the_lines_between_the_forwards_mfmas(cuda, q_lens, k_lens, hq, hkv, causal, dtype):
     """Batches of few blocks have 32x32x16 MFMAs up to 24 tiles a compute unit (as far as the bounds tell) or prefixes of 1280 keys, or, where no unit has two blocks, 33
-    tiles and prefixes of 4096, 16x16x32 beyond."""
+    tiles and prefixes of 4096, 16x16x32 beyond.  The smallest workspace, without room for pieces, leaves blocks whole: 32x32x16 MFMAs wherever no unit has two, and
+    results within rounding of the others."""
     keys = max(k_lens) - min(max(q_lens), max(k_lens)) // 2 if causal else max(k_lens)
     load = sum(q_lens) * hq * keys / (256 * 64 * torch.cuda.get_device_properties(0).multi_processor_count)
     assert 20 < load < 34, "sizes near the line"
     _run(q_lens, k_lens, hq, hkv, 84, cuda, causal=causal, bwd=False, dtype=dtype)
+    import ctypes
+    from distca_amd._lib import CaParams, load
+    from distca_amd.fused_comm_attn import ca_varlen_fwd
+    q, k, v, _ = (t.to(dtype).to(cuda) for t in make_qkv(sum(q_lens), sum(k_lens), hq, hkv, 128, 84))
+    p = CaParams(len(q_lens), sum(q_lens), sum(k_lens), hq, hkv, 128, max(q_lens), max(k_lens), 128 ** -0.5, int(causal), 0, 0)
+    ws = torch.empty(int(load().distca_ca_fwd_workspace_bytes(ctypes.byref(p))), dtype=torch.uint8, device=cuda)
+    args = (torch.tensor(cu(q_lens), device=cuda), torch.tensor(cu(k_lens), device=cuda), max(q_lens), max(k_lens), None, causal, None)
+    few, sizes, (out, lse) = ca_varlen_fwd(q, k, v, *args, ws), ca_varlen_fwd(q, k, v.abs(), *args)[0].float(), ca_varlen_fwd(q, k, v, *args)
+    x, y = few[0].float(), out.float()   # (the bounds of test_blocks_cut_into_pieces)
+    assert ((x - y).abs() <= 2.0 ** -8 * (1.01 * sizes + torch.maximum(x.abs(), y.abs()))).all()
+    assert ((few[1] - lse).abs() <= 256 * 2.0 ** -24 * lse.abs().clamp(min=1)).all()
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
