@@ -276,6 +276,14 @@ inline bool pair_backward(const distca_ca_params *p, bool preferred) {
   if (target_q == 0) return target_kv > 0 || few_key_blocks(p, kSplitFewPerCU);
   return target_kv > 0 && slots_apart(p, bwd_key_blocks_own_rows(p), target_kv, dq_max_items(p), target_q);
 }
+// Whether lists that share a launch are cut for the load of both.  Without a causal mask a task's blocks are all alike: cut as if alone, each list fills the units
+// evenly, and sizes that follow from both lists leave an uneven end, which shows from some kCutForBothTiles tiles of the forward a unit on.  us backward, non-causal, cut for both /
+// as if alone: 600 tokens at 32/8 heads (3 tiles) 51 / 73, 2048 at 4/1 (4) 77 / 88, 2048 at 8/2 (8) 98 / 101, 3000 at 4/1 (9) 101 / 108; 1000 at 64/8 (15) 138 / 131, 4096 at 4/1
+// (16) 152 / 143, 3000 at 8/2 (17) 153 / 159, 4096 at 8/2 (32) 249 / 220, 8192 at 4/1 (64) 446 / 377 (one launch after the other 387), 4096 at 32/8 (128) 700 / 708.
+constexpr int kCutForBothTiles = 12;
+inline bool cut_for_both(const distca_ca_params *p) {
+  return p->causal || (int64_t)p->total_q * p->num_heads_q * p->max_seqlen_k <= (int64_t)kCutForBothTiles * kFwdRows * kFwdKV * num_compute_units();
+}
 // Whether dQ's pieces are those of a list that shares its launch.  As row_split_target it must not know how K/V are stored (it once did: 8 tasks of 256 rows
 // over a document of 16384 at 4/1 heads had 158 pieces over stored rows and 252 over copies, and dq other bits): it asks for the stored rows that one copy
 // of every task's prefix would be, as far as the bounds tell, whole documents' (what row_tiles_to_gain takes for such) or the longest prefix for every task.
@@ -299,7 +307,7 @@ inline SchedGeom launched_dq_geom(const distca_ca_params *p, int32_t target) {
   SchedGeom g = launched_geom(dq_geom(p), p);
   if (target > 0) {
     cut_where_worth(&g, p, target, 6, 3, 6);
-    if (dq_pieces_beside(p)) g.beside = kDkdvBesideDq;
+    if (cut_for_both(p) && dq_pieces_beside(p)) g.beside = kDkdvBesideDq;
   }
   return g;
 }
@@ -309,7 +317,7 @@ inline SchedGeom launched_dkdv_geom(const distca_ca_params *p, int32_t target, b
   SchedGeom g = shared ? bwd_shared_geom(p) : bwd_geom(p);
   g.split_target = target;
   if (target > 0 && preferred) cut_where_worth(&g, p, target, 9, 14, 4);
-  if (beside) g.beside = kDqBesideDkdv, g.min_piece = kMinPieceBeside;
+  if (beside && cut_for_both(p)) g.beside = kDqBesideDkdv, g.min_piece = kMinPieceBeside;
   if (shared && target > 0) g.walk_round = 0;   // pieces count a group's visits downwards
   return g;
 }

@@ -400,3 +400,11 @@ int main() {
     csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "distca_amd", "csrc")
     subprocess.run(["g++", "-std=c++17", "-I", csrc, str(src), "-o", str(tmp_path / "t")], check=True)
     subprocess.run([str(tmp_path / "t")], check=True)
+
+
+@pytest.mark.parametrize("lens,hq,hkv", [([4096], 4, 1), ([8192], 4, 1), ([4096], 8, 2), ([8192], 8, 2), ([4096] * 4, 4, 1), ([4096], 32, 8)])
+def test_blocks_that_are_all_alike_fill_the_units_evenly(lens, hq, hkv):
+    """Without a causal mask a document's blocks are alike; where whole blocks or equal pieces can fill every unit alike, the lists of a backward in one launch do so each."""
+    for kind in (scheduler.BWD, scheduler.DQ):
+        items = scheduler.build_schedule(kind | scheduler.LAUNCHED, _cu(lens), _cu(lens), hq, hkv, causal=False)
+        assert len(items) * hkv % 256 == 0 and items[:, 2].max() == items[:, 2].min(), KINDS[kind]
