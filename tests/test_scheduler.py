@@ -408,5 +408,5 @@ def test_blocks_that_are_all_alike_fill_the_units_evenly(lens, hq, hkv):
     for kind in (scheduler.BWD, scheduler.DQ):
         items = scheduler.build_schedule(kind | scheduler.LAUNCHED, _cu(lens), _cu(lens), hq, hkv, causal=False)
         assert len(items) * hkv % 256 == 0, KINDS[kind]
-        # (the last piece of a block has what is left of it)
-        assert _longest_unit(items[:, 2], hkv, 0) <= 1.05 * items[:, 2].sum() / (256 // hkv), KINDS[kind]
+        # (the last piece of a block has what is left of it: of 64 tiles in pieces of 18, 10)
+        assert _longest_unit(items[:, 2], hkv, 0) <= 1.15 * items[:, 2].sum() / (256 // hkv), KINDS[kind]
