@@ -413,7 +413,7 @@ __global__ __launch_bounds__(kFwdWaves * 64, 1) void ca_fwd_kernel(FwdArgs a) {
   using None = std::integral_constant<int, -1>;
 
   // ---- S^T = K Q^T : [64 keys] x [32 rows]
-    constexpr int kPf = 4;  // K fragments are requested kPf steps, of two MFMAs each, before the MFMAs that use them
+  constexpr int kPf = 4;  // K fragments are requested kPf steps, of two MFMAs each, before the MFMAs that use them
   elemx8 kf[kPf];
   auto load_k = [&](auto par, int f) __attribute__((always_inline)) {  // par: parity of the tile, known at compile time; f = 4*s + kb
     kf[f % kPf] = *static_cast<const DISTCA_LDS elemx8 *>(lds_ptr(k_ad[f >> 2] + decltype(par)::value * kKTile + (f & 3) * 16 * kRowB));
@@ -578,7 +578,7 @@ __global__ __launch_bounds__(kFwdWaves * 64, 1) void ca_fwd_kernel(FwdArgs a) {
   };
   // Between period 0 and fast_end the periods are of one kind for this wave: it sees the tile and the one before whole, and what they
   // request is whole and there, by scalar base.  They have loops of their own without conditions, in which S's first K fragments are asked for
-  // beside the last MFMAs of PV, and b stands ahead of the last two MFMAs of S, when all reads of K are done.  us before -> after: 131072
+  // beside the last MFMAs of PV, and b stands ahead of the last four MFMAs of S, when all reads of K are done.  With 32x32x16 MFMAs, us before -> after: 131072
   // packed tokens 13 240 -> 12 670, 8192 tokens 294 -> 282, a tick of 16384 tokens 1 483 -> 1 421, one over a document of 131072 29 390 ->
   // 27 930, forward of three documents (4096 tokens) 76.7 -> 74.7, lightly loaded server 276 -> 267; documents of 128 to 2048 tokens 980 -> 956.
   // (Of the 4.3 % the loops without conditions give 2.4, requests by a base that moves on 1.4, group 0's between MFMAs 0.5.  b ahead of the
@@ -670,10 +670,24 @@ __global__ __launch_bounds__(kFwdWaves * 64, 1) void ca_fwd_kernel(FwdArgs a) {
         fast(p + 1, P0{});
       }
     };
+    if constexpr (SEG) {
+      // (Period 0 inside the loop, one copy of its code fewer: with one of its own the kernel was 73 to 77 KB, beyond the instruction cache of 64, between whose
+      // halves every end of a shard goes to and fro.  us, in-place ticks with period 0 of its own / so: 8192 tokens of 8 ranks at 64/8 heads 3 343 / 3 288,
+      // one document 6 457 / 6 372, 4096 of 4 at 32/8 147 / 144, 8192 of 8 at 32/8 1 584 / 1 558.)
+      p = -1;   // (opaque: known to the compiler, the first turn becomes one of its own)
+      asm volatile("" : "+s"(p));
+      for (; p <= ntiles; p += 2) {
+        if (p > 0) {
+          fast_periods();  // (the period below may have found the next shard)
+          slow(p, P1{});
+        }
+        if (p + 1 <= ntiles) slow(p + 1, P0{});
+      }
+      return;
+    }
     slow(0, P0{});
-    if constexpr (!SEG) fast_periods();
+    fast_periods();
     for (; p <= ntiles; p += 2) {
-      if constexpr (SEG) fast_periods();  // (the period below may have found the next shard)
       slow(p, P1{});
       if (p + 1 <= ntiles) slow(p + 1, P0{});
     }
