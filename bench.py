@@ -288,10 +288,13 @@ def mfma_probe(torch, _lib, dev, fwd_tflops: float, bwd_tflops: float, rounds: i
                        "clock_GHz": round(float(np.median([r[2] for r in runs[name]])), 3)}
     probe["executed_TFLOP/s_of_the_forward"] = round(fwd_tflops, 1)
     probe["executed_TFLOP/s_of_the_backward"] = round(bwd_tflops, 1)
-    probe["forward_over_mfma_only"] = round(fwd_tflops / probe["mfma_only"]["TFLOP/s"], 4)
+    # (all three kernels of this workload issue the 16x16x32 form)
+    probe["forward_over_mfma16_only"] = round(fwd_tflops / probe["mfma16_only"]["TFLOP/s"], 4)
     probe["backward_over_mfma16_only"] = round(bwd_tflops / probe["mfma16_only"]["TFLOP/s"], 4)
     # with_attention_side_work: beside every 32 K FLOP half of a 1 KB LDS read, two multiply-adds, half an exponential and half
-    # a conversion, the average of the backward kernels' tile loops (no tile requests, barriers or prologues)
+    # a conversion, the average of the backward kernels' tile loops (no tile requests, barriers or prologues); the forward's have a whole LDS read,
+    # an exponential, a multiply-add and a sum, and half a conversion
+    probe["forward_over_mfma16_with_attention_side_work"] = round(fwd_tflops / probe["mfma16_with_attention_side_work"]["TFLOP/s"], 4)
     probe["backward_over_mfma16_with_attention_side_work"] = round(bwd_tflops / probe["mfma16_with_attention_side_work"]["TFLOP/s"], 4)
     probe["note"] = (f"v_mfma_f32_32x32x16_bf16 (mfma16: v_mfma_f32_16x16x32_bf16, two for one) on pseudo-random operands, one wave per SIMD on every SIMD, "
                      f"{8 * iters} (mfma16: {16 * iters}) per wave and run; "
@@ -436,11 +439,12 @@ def main():
     if not args.no_probe:
         probe = mfma_probe(torch, _lib, dev, fwd_tf, 1.4 * bwd_tf)  # S and dP are computed in both backward kernels
         log(f"  32x32x16 MFMAs alone {probe['mfma_only']['TFLOP/s']} TFLOP/s (median of {probe['rounds']} rounds, {probe['mfma_only']['TFLOP/s_min']}"
-            f"..{probe['mfma_only']['TFLOP/s_max']}) at {probe['mfma_only']['clock_GHz']} GHz: the forward executes {100 * probe['forward_over_mfma_only']:.1f} % of it; "
+            f"..{probe['mfma_only']['TFLOP/s_max']}) at {probe['mfma_only']['clock_GHz']} GHz; "
             f"16x16x32 alone {probe['mfma16_only']['TFLOP/s']}, with the backward's side work {probe['mfma16_with_attention_side_work']['TFLOP/s']} "
-            f"({probe['mfma16_with_attention_side_work']['clock_GHz']} GHz, {probe['mfma16_with_attention_side_work']['cycles_per_mfma']} cycles per MFMA): the backward executes "
-            f"{probe['executed_TFLOP/s_of_the_backward']} TFLOP/s, {100 * probe['backward_over_mfma16_only']:.1f} % and "
-            f"{100 * probe['backward_over_mfma16_with_attention_side_work']:.1f} % of them")
+            f"({probe['mfma16_with_attention_side_work']['clock_GHz']} GHz, {probe['mfma16_with_attention_side_work']['cycles_per_mfma']} cycles per MFMA)")
+        for what in ("forward", "backward"):
+            log(f"  the {what} executes {probe[f'executed_TFLOP/s_of_the_{what}']} TFLOP/s, {100 * probe[f'{what}_over_mfma16_only']:.1f} % and "
+                f"{100 * probe[f'{what}_over_mfma16_with_attention_side_work']:.1f} % of the latter two")
 
     pack = None
     if not args.no_pack:

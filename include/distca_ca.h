@@ -405,12 +405,12 @@ int distca_ca_tile_shape(int kind, const distca_ca_params *p, int32_t out[2]);
  * the summed duration and launch count of kernel `which` since the last read
  * and clears them.  Not thread safe; leave disabled outside benchmarks.
  * ------------------------------------------------------------------------- */
-#define DISTCA_TIMER_CA_FWD 0      /* ca_fwd_kernel                          */
+#define DISTCA_TIMER_CA_FWD 0      /* ca_fwd_kernel, ca_fwd32_kernel         */
 #define DISTCA_TIMER_CA_BWD 1      /* ca_bwd_dkdv64_kernel; for batches of few blocks, where one launch makes dQ as well, ca_bwd_pair_kernel */
 #define DISTCA_TIMER_MEMCPY_NON_CP 2
 #define DISTCA_TIMER_MEMCPY_CP 3
 #define DISTCA_TIMER_GRAD_SUM 4
-#define DISTCA_TIMER_CA_BWD_DQ 5   /* ca_bwd_dq64_kernel                     */
+#define DISTCA_TIMER_CA_BWD_DQ 5   /* ca_bwd_dq64_kernel; counts nothing for a batch whose dQ is made in ca_bwd_pair_kernel's launch */
 #define DISTCA_TIMER_COUNT 6
 void distca_timing_enable(int on);
 int distca_timing_read(int which, double *total_ms, int64_t *launches);
