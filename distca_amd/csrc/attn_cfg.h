@@ -180,8 +180,8 @@ inline bool fwd_mfma32(const distca_ca_params *p, bool split) {
 // dQ and dK/dV side by side in one launch (attn_bwd_pair.hip) up to kPairBlocksPerCU blocks of query rows per compute unit: each then
 // fills what the other's longest blocks leave idle, and a launch is saved.  Beyond that their last blocks are a small part of the time and the pass over dO
 // and O that makes the row statistics ahead of both shows.  us backward, one after the other / side by side: 256 tokens at 8/2 heads 51 / 34, 389 at 4/1
-// 56 / 36, 1000 at 4/1 79 / 55, 2048 at 4/1 (both cut) 88 / 64, 8 x 1000 at 32/8 299 / 261, 8192 at 8/2 458 / 395, 4 x 2300 at 32/8 593 / 507; at 4 blocks a
-// unit 8192 at 32/8 1404 / 1354, 32768 at 8/2 5276 / 5123, 2 x 4096 at 32/8 764 / 771 (blocks that pack exactly); at 5 10000 at 32/8 2040 / 2010, 40000 at
+// 56 / 36, 1000 at 4/1 79 / 55, 2048 at 4/1 (both cut) 88 / 64, 8 x 1000 at 32/8 299 / 261, 8192 at 8/2 458 / 395, 4 x 2300 at 32/8 593 / 507, 2 x 4096 at 32/8 775 / 718; at 4 blocks a
+// unit 8192 at 32/8 1404 / 1354, 32768 at 8/2 5276 / 5123; at 5 10000 at 32/8 2040 / 2010, 40000 at
 // 8/2 7929 / 7718; at 6 12000 at 32/8 2772 / 2821, at 8 4 x 4000 at 32/8 1329 / 1364.
 constexpr int kPairBlocksPerCU = 5;
 // What either list's items take of the other's time: 256 rows by 64 keys of dQ 2.1 us, the same area as two blocks of dK/dV at 1.35, hence 0.78 of
