@@ -671,9 +671,10 @@ __global__ __launch_bounds__(kFwdWaves * 64, 1) void ca_fwd_kernel(FwdArgs a) {
       }
     };
     if constexpr (SEG) {
-      // (Period 0 inside the loop, one copy of its code fewer: with one of its own the kernel was 73 to 77 KB, beyond the instruction cache of 64, between whose
-      // halves every end of a shard goes to and fro.  us, in-place ticks with period 0 of its own / so: 8192 tokens of 8 ranks at 64/8 heads 3 343 / 3 288,
-      // one document 6 457 / 6 372, 4096 of 4 at 32/8 147 / 144, 8192 of 8 at 32/8 1 584 / 1 558.)
+      // Period 0 inside the loop, whose periods with conditions come back at every end of a shard: the compiler then makes less of them (a forward over 22 shards, a launch:
+      // 6.33e8 -> 6.27e8 vector instructions, wave-cycles at a wait 6.5e8 -> 6.0e8 units of four; not the size of the code, 77 -> 64 KB: 7e3 and 4e3 misses in 2.2e8
+      // requests).  us, in-place ticks with period 0 of its own / so: 8192 tokens of 8 ranks at 64/8 heads 3 343 / 3 288, one document 6 457 / 6 372, 4096 of 4 at 32/8
+      // 147 / 144, 8192 of 8 at 32/8 1 584 / 1 558.
       p = -1;   // (opaque: known to the compiler, the first turn becomes one of its own)
       asm volatile("" : "+s"(p));
       for (; p <= ntiles; p += 2) {

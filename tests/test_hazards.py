@@ -274,18 +274,3 @@ def test_block_loops_of_the_backward_kernels_reload_nothing(listings):
                 found += [(kernel, len(body), l) for l in body if l.startswith("scratch_load")]
     assert loops > 100, "the disassembly is not what this test reads"
     assert not found, f"{len(found)} reloads, among them {found[:3]}"
-
-
-def test_the_forward_fits_the_instruction_cache(tmp_path):
-    """A wave of the forward over shards goes to and fro between the periods with conditions and those without, at the end of every shard: both kinds, of both groups of
-    waves, lie in the 64 KB that two compute units share."""
-    if not os.path.exists(OBJDUMP):
-        pytest.skip("needs llvm-objdump")
-    sizes = {}
-    for k, obj in enumerate(code_objects(LIB_PATH)):
-        f = tmp_path / f"{k}.co"
-        f.write_bytes(obj)
-        text = subprocess.run([OBJDUMP, "-t", str(f)], capture_output=True, text=True, check=True).stdout
-        sizes.update({(k, name): int(size, 16) for size, name in re.findall(r"\.text\s+([0-9a-f]{8,})\s+(?:\.\w+\s+)?(\S*ca_fwd_kernel\S*)$", text, flags=re.M)})
-    assert len(sizes) == 8, "four forms for each element type"
-    assert max(sizes.values()) <= 64 << 10, sizes
