@@ -722,7 +722,8 @@ def test_kv_shards_read_in_place_equal_dense_tensors(cuda, hq, hkv):
     (8, 8, [37] * 60)])                                               # no tile inside one shard
 def test_runs_of_tiles_inside_shards(cuda, hq, hkv, shard_len):
     """The loops over tiles that lie inside one shard begin and end where shards do: out, lse and the gradients over shards in a buffer (every
-    other one from its far end, K apart from V) equal bit for bit what dense tensors give, for prefixes that end around tiles' ends."""
+    other one from its far end, K apart from V) equal bit for bit what dense tensors give, for prefixes that end around tiles' ends; the gradients with
+    whole blocks, and with the workspace that has room for pieces of both lists in one launch."""
     import ctypes
     from distca_amd import _lib
     from distca_amd.fused_comm_attn import _params, ca_varlen_bwd, ca_varlen_fwd
@@ -734,7 +735,6 @@ def test_runs_of_tiles_inside_shards(cuda, hq, hkv, shard_len):
     cu_q, cu_k = i32([0] + list(np.cumsum(q_lens))), i32([0] + list(np.cumsum(k_lens)))
     off = i32([0] * len(q_lens))
     out, lse = ca_varlen_fwd(q, k, v, cu_q, cu_k, max(q_lens), max(k_lens), kv_task_offsets=off)
-    dq, dk, dv = ca_varlen_bwd(do, q, k, v, out, lse, cu_q, cu_k, max(q_lens), max(k_lens), deterministic=True, kv_task_offsets=off)
     start, ns = np.concatenate([[0], np.cumsum(shard_len)]), len(shard_len)
     places = list(range(0, ns, 2)) + list(range(ns - 1 - ns % 2, 0, -2))
     buf, k_off, v_off = [], [0] * ns, [0] * ns
@@ -748,8 +748,8 @@ def test_runs_of_tiles_inside_shards(cuda, hq, hkv, shard_len):
     p = _params(len(q_lens), sum(q_lens), rows, hq, hkv, d, max(q_lens), max(k_lens), d ** -0.5, True, True)
     lib = _lib.load()
     # (the sizes that the calls over dense tensors take: blocks are cut into as many pieces as there is room for)
-    room = lib.distca_ca_fwd_workspace_preferred_bytes(ctypes.byref(p)), lib.distca_ca_bwd_workspace_bytes(ctypes.byref(p))
-    ws = torch.empty((int(max(room)),), dtype=torch.uint8, device=cuda)
+    room = [int(getattr(lib, f"distca_ca_{n}_bytes")(ctypes.byref(p))) for n in ("fwd_workspace_preferred", "bwd_workspace", "bwd_workspace_preferred")]
+    ws = torch.empty((max(room),), dtype=torch.uint8, device=cuda)
     stream = torch.cuda.current_stream().cuda_stream
     out2, lse2 = torch.empty_like(out), torch.empty_like(lse)
     _lib.check(lib.distca_ca_fwd_buffers(q.data_ptr(), None, 0, buf.data_ptr(), buf.data_ptr(), ctypes.byref(shards), out2.data_ptr(), None, 0,
@@ -762,13 +762,15 @@ def test_runs_of_tiles_inside_shards(cuda, hq, hkv, shard_len):
     req = torch.cat([x.view(torch.uint8).view(tq, -1) for x in parts], dim=1).contiguous()
     first = torch.tensor(np.concatenate([[0], np.cumsum(q_lens)[:-1]]), device=cuda)
     req_off, dq_off = first * req.shape[1], first * row
-    dq2, gbuf = torch.empty_like(dq), torch.empty_like(buf)
-    _lib.check(lib.distca_ca_bwd_buffers(req.data_ptr(), req_off.data_ptr(), req.shape[1], buf.data_ptr(), buf.data_ptr(), ctypes.byref(shards),
-                                         dq2.data_ptr(), dq_off.data_ptr(), row, gbuf.data_ptr(), gbuf.data_ptr(), cu_q.data_ptr(), cu_k.data_ptr(),
-                                         off.data_ptr(), ctypes.byref(p), ws.data_ptr(), room[1], stream), "bwd_buffers")
-    torch.cuda.synchronize()
-    assert torch.equal(dq2, dq)
-    for offs, x in ((k_off, dk), (v_off, dv)):
-        for s in range(ns):
-            want = x[start[s]:start[s + 1]].reshape(-1).view(torch.uint8)
-            assert torch.equal(gbuf[offs[s]:offs[s] + want.numel()], want), f"gradients of shard {s}"
+    for size in room[1:]:
+        dq, dk, dv = ca_varlen_bwd(do, q, k, v, out, lse, cu_q, cu_k, max(q_lens), max(k_lens), deterministic=True, kv_task_offsets=off, workspace=ws[:size])
+        dq2, gbuf = torch.empty_like(q), torch.empty_like(buf)
+        _lib.check(lib.distca_ca_bwd_buffers(req.data_ptr(), req_off.data_ptr(), req.shape[1], buf.data_ptr(), buf.data_ptr(), ctypes.byref(shards),
+                                             dq2.data_ptr(), dq_off.data_ptr(), row, gbuf.data_ptr(), gbuf.data_ptr(), cu_q.data_ptr(), cu_k.data_ptr(),
+                                             off.data_ptr(), ctypes.byref(p), ws.data_ptr(), size, stream), "bwd_buffers")
+        torch.cuda.synchronize()
+        assert torch.equal(dq2, dq)
+        for offs, x in ((k_off, dk), (v_off, dv)):
+            for s in range(ns):
+                want = x[start[s]:start[s + 1]].reshape(-1).view(torch.uint8)
+                assert torch.equal(gbuf[offs[s]:offs[s] + want.numel()], want), f"gradients of shard {s}"
